@@ -99,11 +99,25 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+def load_native():
+    """The host side of the backend in native code (``csrc/kr_host.cpp``): one call per launch that checks the
+    operands, allocates the outputs and launches.  Its functions answer None to a case they do not take, which then
+    goes through this module's general path.  Built with the kernel library; like it, there is no doing without."""
+    try:
+        from .. import _native
+    except ImportError as e:
+        raise RuntimeError("kareus_amd/_native.so is missing or cannot be loaded: build it with `make -C kareus_amd/csrc` "
+                           f"(or __graft_entry__.build()): {e}") from e
+    return _native
+
+
 class HipBackend:
     name = "hip"
+    _n = None   # the native host side
 
     def __init__(self) -> None:
         self.lib = load_library()
+        self._n = load_native()
         self._gemm_ws_bytes: dict = {}  # (layout, m, n, k, split_k) -> workspace bytes
         self._ws_cache: dict = {}       # (stream, device) -> reusable workspace buffer
         self._cu_count: dict = {}       # device index -> compute units
@@ -179,6 +193,10 @@ class HipBackend:
         """``t`` ([..., cols]) as the kernels can address it in place: a [rows, cols] view when its rows have
         one stride, ``t`` itself when it is a [s, r, cols] tensor whose rows come in runs; None when only a
         copy would do."""
+        if self._n is not None:
+            v = self._n.rows_view(t, self.MAX_RUN_ROWS)
+            if v is not None:
+                return v
         cols = t.shape[-1]
         # (whether the leading dimensions merge into one is read off the strides: asking ``view`` and catching
         # its error costs 10 us per nanobatch slice that does not)
@@ -207,6 +225,7 @@ class HipBackend:
     # launch runs beside other streams' kernels (KR_GEMM_BESIDE_OTHER_STREAMS): the workspace is sized with
     # the same weight, so the cuts the dispatcher plans are the cuts the buffer holds
     SHARED_LATENCY_WEIGHT = 0.1
+    _SPLIT_CODE = {None: 0, True: 1, False: 2}   # ``split_k`` as the native side takes it
 
     def _workspace(self, nbytes: int, device) -> Tensor:
         """A workspace of at least ``nbytes`` for the current stream.  One buffer per (stream, size
@@ -232,6 +251,14 @@ class HipBackend:
         ``max_cus``: compute-unit budget of the launch (0 = the whole device).
         ``swiglu_bwd_x`` ([m, 2n], layout NN): the product is the gradient of a SwiGLU output and
         is not stored; ``out`` ([m, 2n]) receives the gradient of the activation's input instead."""
+        if max_cus == 0:
+            reserved = reserved_compute_units()
+            if reserved:
+                max_cus = max(self._num_cus(a.device) - reserved, 8)
+        done = self._n.gemm(layout, a, b, m, n, k, out, accumulate, self._SPLIT_CODE[split_k], residual, swiglu_out,
+                            swiglu_bwd_x, max_cus)
+        if done is not None:
+            return done
         self._dev(a, b)
         self._bf16(a, b)
         if a.stride(-1) != 1 or b.stride(-1) != 1:
@@ -277,10 +304,6 @@ class HipBackend:
                 self._gemm_ws_bytes[key] = ws_bytes
             if ws_bytes:
                 ws_ptr = self._workspace(ws_bytes, a.device).data_ptr()
-        if max_cus == 0:
-            reserved = reserved_compute_units()
-            if reserved:
-                max_cus = max(self._num_cus(a.device) - reserved, 8)
         if split_k is False:
             epi |= 0x100   # KR_GEMM_BESIDE_OTHER_STREAMS
         c_op = self._operand(out)
@@ -314,6 +337,11 @@ class HipBackend:
     @staticmethod
     def _nrows(t: Tensor) -> int:
         return t.shape[0] if t.dim() == 2 else t.shape[0] * t.shape[1]
+
+    def split_qkv(self, mixed: Tensor, ng: int, per: int, hd: int):
+        """The query, key and value views of a dense fused QKV buffer [s, b, features] and the buffer as
+        [s, b, ng, per + 2, hd]; None for any other tensor."""
+        return self._n.split_qkv(mixed, ng, per, hd)
 
     @staticmethod
     def can_fuse_swiglu(two_f: int) -> bool:
@@ -359,6 +387,13 @@ class HipBackend:
                               split_k: bool = True) -> Tensor:
         """``sum_i dys[i]^T . xs[i]`` in one launch: the weight gradient over all nanobatches of a
         microbatch, each pair read where it lies (``wgrad_segments_ok`` says whether the pairs qualify)."""
+        max_cus = 0
+        reserved = reserved_compute_units()
+        if reserved:
+            max_cus = max(self._num_cus(dys[0].device) - reserved, 8)
+        done = self._n.wgrad_segments(dys, xs, out, accumulate, self._SPLIT_CODE[split_k], max_cus)
+        if done is not None:
+            return done
         if not self.wgrad_segments_ok(dys, xs):
             raise RuntimeError("linear_wgrad_segments: operand pairs must be matrices of one shape and row stride "
                                "with a multiple of 64 rows each")
@@ -380,10 +415,6 @@ class HipBackend:
                 self._gemm_ws_bytes[key] = ws_bytes
             if ws_bytes:
                 ws_ptr = self._workspace(ws_bytes, out.device).data_ptr()
-        max_cus = 0
-        reserved = reserved_compute_units()
-        if reserved:
-            max_cus = max(self._num_cus(out.device) - reserved, 8)
         ptrs = ctypes.c_void_p * nseg
         a_ptrs = ptrs(*[t.data_ptr() for t in dys])
         b_ptrs = ptrs(*[t.data_ptr() for t in xs])
@@ -405,6 +436,9 @@ class HipBackend:
     def rmsnorm_fwd(self, x: Tensor, gamma: Tensor, eps: float) -> Tuple[Tensor, Tensor]:
         """``x``: [rows, cols], or a [s, r, cols] nanobatch slice whose rows come in runs (read in place).
         Returns the dense [rows, cols] result and rstd [rows]."""
+        done = self._n.rmsnorm_fwd(x, gamma, eps)
+        if done is not None:
+            return done
         self._dev(x, gamma)
         self._bf16(x, gamma)
         op = self._operand(x)
@@ -443,6 +477,9 @@ class HipBackend:
         [rows, cols] tensor (possibly a row-strided slice) the input gradient is written into.
         ``partials_out`` ([rmsnorm_partial_rows, cols] fp32, contiguous): the weight gradient is
         left there as partial rows for ``rmsnorm_dgamma`` and None is returned in its place."""
+        done = self._n.rmsnorm_bwd(dy, x, rstd, gamma, residual_grad, out, partials_out)
+        if done is not None:
+            return done
         self._dev(dy, x, rstd, gamma)
         self._bf16(dy, x, gamma)
         dy = self._rows(dy)
@@ -534,6 +571,8 @@ class HipBackend:
     def rope_fused_inplace(self, fused: Tensor, per: int, freqs: Tensor, backward: bool) -> None:
         """Rotate the query and key heads of a fused QKV buffer [s, b, ng, per+2, hd] in place
         (one launch); the value heads are left untouched."""
+        if self._n.rope_fused(fused, freqs, backward):
+            return
         s, b, ng, slots, hd = fused.shape
         if slots != per + 2 or not fused.is_contiguous():
             raise RuntimeError("fused QKV buffer must be contiguous [s, b, ng, per+2, hd]")
@@ -602,6 +641,10 @@ class HipBackend:
             raise RuntimeError(f"dropout_add: shapes differ, {tuple(x.shape)} vs {tuple(residual.shape)}")
         if not 0.0 <= p < 1.0:
             raise RuntimeError(f"dropout_add: probability {p} is outside [0, 1)")
+        seed = int(torch.randint(0, 1 << 62, (1,), dtype=torch.int64).item())
+        done = self._n.dropout_add(x, residual, p, out, seed)
+        if done is not None:
+            return done
         x2, r2 = self._rows(self._leading_rows(x)), self._rows(self._leading_rows(residual))
         if out is None:
             out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
@@ -618,7 +661,6 @@ class HipBackend:
             raise RuntimeError("dropout_add: out cannot be addressed with a single row stride")
         rows, cols = x2.shape
         mask = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-        seed = int(torch.randint(0, 1 << 62, (1,), dtype=torch.int64).item())
         self._check(self.lib.kr_dropout_add(x2.data_ptr(), x2.stride(0), r2.data_ptr(), r2.stride(0), o2.data_ptr(),
                                             o2.stride(0), mask.data_ptr(), rows, cols, float(p), seed, 0,
                                             self._stream()), "kr_dropout_add")
@@ -626,6 +668,9 @@ class HipBackend:
 
     def dropout_bwd(self, dy: Tensor, mask: Tensor, scale: float) -> Tensor:
         """``dy * mask * scale``: native_dropout_backward."""
+        done = self._n.dropout_bwd(dy, mask, scale)
+        if done is not None:
+            return done
         self._dev(dy)
         self._bf16(dy)
         if (not mask.is_cuda or mask.dtype != torch.uint8 or mask.shape != dy.shape
@@ -788,13 +833,16 @@ class HipBackend:
         takes the general fp32 kernels instead of being padded into the MFMA ones."""
         if not causal:
             raise RuntimeError("only causal attention is implemented")
+        flags = (KR_ATTN_BESIDE_OTHER_STREAMS if beside_other_streams else 0) | (KR_ATTN_GENERAL_KERNELS if general_kernels else 0)
+        done = self._n.attn_fwd(q, k, v, scale, flags)
+        if done is not None:
+            return done
         self._dev(q, k, v)
         self._bf16(q, k, v)
         s, b, nq, nkv, hd = self._q_dims(q, k)
         per = nq // nkv
         o = torch.empty((s, b, nq, hd), dtype=q.dtype, device=q.device)
         lse = torch.empty((b, nq, s), dtype=torch.float32, device=q.device)
-        flags = (KR_ATTN_BESIDE_OTHER_STREAMS if beside_other_streams else 0) | (KR_ATTN_GENERAL_KERNELS if general_kernels else 0)
         nbytes = 0 if general_kernels else self._attn_fwd_ws_bytes(s, b, nq, nkv, hd)
         ws_ptr = self._workspace(nbytes, q.device).data_ptr() if nbytes else None
         rc = self.lib.kr_attn_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
@@ -820,6 +868,14 @@ class HipBackend:
         carry it as ``_kr_mixed`` so the QKV-split backward can hand it on without a copy."""
         if not causal:
             raise RuntimeError("only causal attention is implemented")
+        flags = (KR_ATTN_BESIDE_OTHER_STREAMS if beside_other_streams else 0) | (KR_ATTN_GENERAL_KERNELS if general_kernels else 0)
+        done = self._n.attn_bwd(do, q, k, v, o, lse, scale, flags)
+        if done is not None:
+            dq, dk, dv, mixed, fused = done
+            for t in (dq, dk, dv):
+                t._kr_mixed = mixed
+                t._kr_fused5 = fused
+            return dq, dk, dv
         self._dev(do, q, k, v, o, lse)
         self._bf16(do, q, k, v, o)
         s, b, nq, nkv, hd = self._q_dims(q, k)
@@ -837,7 +893,6 @@ class HipBackend:
             dv = torch.empty((s, b, nkv, hd), dtype=q.dtype, device=q.device)
         nbytes = self.lib.kr_attn_bwd_workspace_bytes(s, b, nq, nkv, hd)
         ws = self._workspace(max(nbytes, 16), q.device)
-        flags = (KR_ATTN_BESIDE_OTHER_STREAMS if beside_other_streams else 0) | (KR_ATTN_GENERAL_KERNELS if general_kernels else 0)
         rc = self.lib.kr_attn_bwd_flags(do4.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o4.data_ptr(),
                                         lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(),
                                         s, b, nq, nkv, hd, scale,

@@ -72,6 +72,13 @@ class QKVPostProcessOp(BasicOperation, PartitionableOperator):
         width = ng * (per + 2) * hd
         if mixed.shape[-1] != width:
             raise ValueError(f"fused QKV width {mixed.shape[-1]} != ng*(nq/ng+2)*hd = {width}")
+        cut = getattr(get_backend(self._backend_name), "split_qkv", None) if self.grouped_query_view else None
+        views = cut(mixed, ng, per, hd) if cut is not None else None
+        if views is not None:   # the same views from one call
+            q, k, v, fused5 = views
+            for t in (q, k, v):
+                t._kr_fused5 = fused5
+            return q, k, v
         fused5 = mixed.view(*mixed.shape[:-1], ng, per + 2, hd)
         q, k, v = fused5[..., :per, :], fused5[..., per, :], fused5[..., per + 1, :]
         if not self.grouped_query_view:

@@ -1,0 +1,49 @@
+"""The native host side of the hip backend (``csrc/kr_host.cpp``) classifies tensors as the Python side does, and
+leaves what it does not take to it.  No GPU needed."""
+
+import pytest
+import torch
+
+from kareus_amd.backend.hip import HipBackend, load_native
+
+
+def _slices():
+    whole = torch.empty(40, 8, 64, dtype=torch.bfloat16)
+    wide = torch.empty(16, 128, dtype=torch.bfloat16)
+    deep = torch.empty(5, 3, 4, 2, 16, dtype=torch.bfloat16)
+    return [whole, whole[:, 0:1], whole[:, 2:4], whole[:, 4:8], whole[:, 1:4], whole[:1, 2:4], whole[3:4, 5:6], wide,
+            wide[:, :64], wide.t(), wide[:1], deep, deep[:, :, 1], deep[:, :1], deep[..., :8],
+            torch.empty(4, 64, 64, dtype=torch.bfloat16)[:, :32], torch.empty(40, 8, 60, dtype=torch.bfloat16)[:, 0:2],
+            torch.empty(1, 60, dtype=torch.bfloat16)]
+
+
+@pytest.mark.parametrize("i", range(len(_slices())))
+@pytest.mark.parametrize("max_run_rows", [16, 1])
+def test_rows_view_equals_the_python_side(i, max_run_rows):
+    t = _slices()[i]
+    be = HipBackend.__new__(HipBackend)          # without the native side
+    be.MAX_RUN_ROWS = max_run_rows
+    got, want = load_native().rows_view(t, max_run_rows), be.rows_view(t)
+    if want is not None and max_run_rows == 1 and want.dim() == 3:
+        want = None                              # (the Python side reads the class's limit, not the instance's)
+    assert (got is None) == (want is None)
+    if got is not None:
+        assert got.shape == want.shape and got.data_ptr() == want.data_ptr()
+        assert all(n == 1 or a == b for n, a, b in zip(got.shape, got.stride(), want.stride()))
+
+
+def test_split_qkv_is_the_grouped_view():
+    s, b, ng, per, hd = 6, 2, 3, 4, 16
+    mixed = torch.arange(s * b * ng * (per + 2) * hd, dtype=torch.float32).view(s, b, -1)
+    q, k, v, fused = load_native().split_qkv(mixed, ng, per, hd)
+    want = mixed.view(s, b, ng, per + 2, hd)
+    assert torch.equal(fused, want) and torch.equal(q, want[:, :, :, :per])
+    assert torch.equal(k, want[:, :, :, per]) and torch.equal(v, want[:, :, :, per + 1])
+    assert load_native().split_qkv(mixed[:, :1], ng, per, hd) is None and load_native().split_qkv(mixed, ng + 1, per, hd) is None
+
+
+def test_calls_leave_other_tensors_to_the_python_side():
+    n, x = load_native(), torch.zeros(8, 8, dtype=torch.bfloat16)          # on the host: not the device's business
+    assert n.gemm(0, x, x, 8, 8, 8, None, False, 1, None, None, None, 0) is None
+    assert n.rmsnorm_fwd(x, x[0], 1e-5) is None and n.attn_fwd(x, x, x, 1.0, 0) is None
+    assert n.dropout_bwd(x, x, 1.0) is None and n.wgrad_segments([x], [x], None, False, 1, 0) is None
