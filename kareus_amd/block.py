@@ -99,6 +99,31 @@ class LayerConfig:
     kareus_scheduler: Optional[Any] = None
     nanobatch_streams: Optional[List[Any]] = field(default=None, repr=False)
 
+    # the nanobatch streams were made by the block driver (streams that a caller names are always used)
+    streams_are_own: bool = field(default=False, repr=False)
+
+    # Nanobatches on streams of their own cost the host 0.9-1.0 ms per nanobatch and layer, forward and backward
+    # (launches, and above all the event waits of the schedule points), one after the other on one stream 0.6 ms.
+    # Where the device needs less than that for a nanobatch, the streams' overlap hides nothing and the step takes
+    # as long as the host: on one stream it is shorter, and the launches, alone on the device, are planned for
+    # their latency.  Measured, streams against one stream, two / four nanobatches: small layer (512 hidden) 256-2048
+    # tokens 1.5x / 1.5x, 8B shard of four 1024 tokens 1.48x / 1.32x, 2048 tokens 1.13x / 0.98x, 4096 tokens 0.88x / 0.86x,
+    # 3B layer 512 tokens 1.41x / 1.31x, 1024 tokens 1.18x / 1.01x, 8B layer 256 tokens 1.20x / 0.84x.
+    IN_LINE_BELOW_MS = 0.65
+
+    def nanobatches_in_line(self, seq: int, seqs: int) -> bool:
+        """Whether the nanobatches of a pass ([seq, seqs, hidden] each) run one after the other on the caller's stream
+        instead of on their own: where an estimate of one nanobatch's device time per layer, forward and backward,
+        is below what its launches cost the host.  Products at 0.75 PFLOP/s, attention at 0.4, forty passes over
+        the hidden states at 5 TB/s, the weights read twice at 4.5 TB/s."""
+        if not self.streams_are_own or self.backend != "hip":
+            return False
+        t, h, hd, nq = seq * seqs, self.hidden_size, self.kv_channels, self.num_attention_heads
+        weights = h * (self.qkv_width + nq * hd + 3 * self.ffn_hidden_size)
+        ms = (6.0 * t * weights / 0.75e12 + 7.0 * seqs * nq * hd * float(seq) ** 2 / 0.4e12
+              + 80.0 * t * h / 5e9 + 4.0 * weights / 4.5e9)
+        return ms < self.IN_LINE_BELOW_MS
+
     @property
     def qkv_width(self) -> int:
         return (self.num_attention_heads + 2 * self.num_query_groups) * self.kv_channels
@@ -226,15 +251,16 @@ class DecoderLayer(torch.nn.Module):
             row_parallel.fuse_residual = fuse and c.hidden_dropout == 0.0
             row_parallel.forward_accepts_out_sink = fuse and c.hidden_dropout == 0.0
 
+    _ORDER = ("attn_residual_fork", "input_layernorm",
+              "linear_qkv", "qkv_postprocess", "rotary", "core_attention", "linear_proj",
+              "self_attn_bda",
+              "mlp_residual_fork", "pre_mlp_layernorm",
+              "linear_fc1", "activation", "linear_fc2",
+              "mlp_bda")
+
     def get_all_operators(self) -> List:
-        return [
-            self.attn_residual_fork, self.input_layernorm,
-            self.linear_qkv, self.qkv_postprocess, self.rotary, self.core_attention, self.linear_proj,
-            self.self_attn_bda,
-            self.mlp_residual_fork, self.pre_mlp_layernorm,
-            self.linear_fc1, self.activation, self.linear_fc2,
-            self.mlp_bda,
-        ]
+        modules = self._modules
+        return [modules[name] for name in self._ORDER]
 
     def forward(self, *args, **kwargs):
         raise RuntimeError("DecoderLayer is executed by the partition engine, not called directly")
@@ -327,6 +353,7 @@ class LayerStack(torch.nn.Module):
             c.nanobatch_streams = None
             return None
         if c.nanobatch_streams is None:
+            c.streams_are_own = True
             many = getattr(api, "new_streams", None)
             c.nanobatch_streams = (many(c.num_nanobatches) if many is not None
                                    else [api.new_stream() for _ in range(c.num_nanobatches)])

@@ -65,6 +65,9 @@ class PartitionableLinear(BasicOperation, PartitionableOperator):
         # then the contraction is not split, which costs the least CU-time (set by the block driver)
         self.split_k = True
 
+    def _split(self, ctx):
+        return True if (self.split_k is False and ctx.alone) else self.split_k
+
     # -- what the forward may take along in its epilogue ------------------------------------------
     # fuse_residual (set by the block driver on row-parallel layers of a one-GPU shard): the layer
     # also reads the ``residual`` channel and, when the kernels can address the operands, adds it
@@ -111,7 +114,7 @@ class PartitionableLinear(BasicOperation, PartitionableOperator):
             # (kareus/megatron/core/extensions/ops/bias_swiglu.py:14-20 behind basic_linear.py:571-582)
             act_ctx = basic_op_ctxs[1]
             y = x2d.new_empty((x2d.numel() // k, n // 2))
-            x = be.linear_fwd(x2d, w, split_k=self.split_k, swiglu_out=y)
+            x = be.linear_fwd(x2d, w, split_k=self._split(ctx), swiglu_out=y)
             if act_ctx.requires_grad:
                 act_ctx.save_for_backward(x)
                 act_ctx.ori_shape = (*input_.shape[:-1], n)
@@ -125,11 +128,11 @@ class PartitionableLinear(BasicOperation, PartitionableOperator):
             out2d = be.rows_view(sink) if (sink is not None and sink.shape[-1] == n) else None
             if (res2d is not None and res2d.numel() // n == x2d.numel() // k
                     and (sink is None or (out2d is not None and out2d.numel() == res2d.numel()))):
-                y = be.linear_fwd(x2d, w, split_k=self.split_k, residual=res2d, out=out2d)
+                y = be.linear_fwd(x2d, w, split_k=self._split(ctx), residual=res2d, out=out2d)
                 y = sink if sink is not None else y.view(out_shape)
                 y._kr_residual_added = True
                 return y, [()]
-        y = be.linear_fwd(x2d, w, split_k=self.split_k)
+        y = be.linear_fwd(x2d, w, split_k=self._split(ctx))
         return y.view(out_shape), [()]
 
     def op_forward(self, ctx, input_, *, prev_op=None, next_op=None):
@@ -158,8 +161,8 @@ class PartitionableLinear(BasicOperation, PartitionableOperator):
         n, _k = self.weight.shape
         be = get_backend(self._backend_name)
         dy = be.rows_in_place(grad_output)
-        dx = be.linear_dgrad(dy, self.weight.detach(), split_k=self.split_k, swiglu_bwd_x=act_in)
-        dw = self._weight_grad(be, ctx, dy, x2d, self.split_k) if self.weight.requires_grad else None
+        dx = be.linear_dgrad(dy, self.weight.detach(), split_k=self._split(ctx), swiglu_bwd_x=act_in)
+        dw = self._weight_grad(be, ctx, dy, x2d, self._split(ctx)) if self.weight.requires_grad else None
         return dx.view(act_ctx.ori_shape), [(dw,), ()], [extra, ()]
 
     def op_backward(self, ctx, grad_output):
@@ -167,8 +170,8 @@ class PartitionableLinear(BasicOperation, PartitionableOperator):
         n, k = self.weight.shape
         be = get_backend(self._backend_name)
         dy = be.rows_in_place(grad_output)
-        dx = be.linear_dgrad(dy, self.weight.detach(), split_k=self.split_k)
-        dw = self._weight_grad(be, ctx, dy, x2d, self.split_k) if self.weight.requires_grad else None
+        dx = be.linear_dgrad(dy, self.weight.detach(), split_k=self._split(ctx))
+        dw = self._weight_grad(be, ctx, dy, x2d, self._split(ctx)) if self.weight.requires_grad else None
         return dx.view(*grad_output.shape[:-1], k), (dw,)
 
     @staticmethod
@@ -192,7 +195,7 @@ class PartitionableLinear(BasicOperation, PartitionableOperator):
         if sink is None:
             return be.linear_wgrad(dy, x2d, split_k=split_k)
         api = stream_api()
-        here = api.current_stream()
+        here = None if sink.get("in_line") else api.current_stream()
         n = sink.get("n", 0)
         if n > 1 and sink.get("defer", True) and hasattr(be, "linear_wgrad_segments"):
             ev = None

@@ -57,7 +57,7 @@ class RMSNorm(BasicOperation):
         rows = x2d.numel() // cols
         per = be.rmsnorm_partial_rows(rows, cols)
         api = stream_api()
-        here = api.current_stream()
+        here = None if sink.get("in_line") else api.current_stream()
         buf = sink.get("buf")
         if buf is None or buf.shape[0] != n * per:
             buf = sink["buf"] = torch.empty((n * per, cols), dtype=torch.float32, device=x2d.device)

@@ -64,21 +64,36 @@ def _nanobatch_streams(config, n: int) -> List[Optional[object]]:
     return list(streams)
 
 
+def _nanobatches_in_line(config, hs: Sequence[Tensor]) -> bool:
+    """Whether this pass runs its nanobatches one after the other on the caller's stream although they have
+    streams of their own (``LayerConfig.nanobatches_in_line`` says when that is faster)."""
+    rule = getattr(config, "nanobatches_in_line", None)
+    return len(hs) > 1 and rule is not None and rule(hs[0].shape[0], hs[0].shape[1])
+
+
 def _fork(streams: Sequence[Optional[object]]) -> None:
     """Side streams start after everything already enqueued on the caller's stream."""
     if any(s is not None for s in streams):
-        here = stream_api().current_stream()
-        for s in streams:
-            if s is not None and s != here:
+        api = stream_api()
+        here = api.current_stream()
+        others = [s for s in streams if s is not None and s != here]
+        if hasattr(api, "fan_out"):
+            api.fan_out(here, others)
+        else:
+            for s in others:
                 s.wait_stream(here)
 
 
 def _join(streams: Sequence[Optional[object]]) -> None:
     """The caller's stream continues after everything enqueued on the side streams."""
     if any(s is not None for s in streams):
-        here = stream_api().current_stream()
-        for s in streams:
-            if s is not None and s != here:
+        api = stream_api()
+        here = api.current_stream()
+        others = [s for s in streams if s is not None and s != here]
+        if hasattr(api, "fan_in"):
+            api.fan_in(here, others)
+        else:
+            for s in others:
                 here.wait_stream(s)
 
 
@@ -170,8 +185,9 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
             f"got {len(params)} tensors"
         )
 
-        streams = _nanobatch_streams(config, n)
-        ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i]) for i in range(n)]
+        in_line = _nanobatches_in_line(config, hs)
+        streams = [None] * n if in_line else _nanobatch_streams(config, n)
+        ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=in_line) for i in range(n)]
         _seed_forward(ctxs, hs, rotary, mask, seed)
 
         # The nanobatch outputs are written side by side into one [s, b, h] tensor, so the
@@ -202,6 +218,7 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
 
         func_ctx.n = n
         func_ctx.streams = streams
+        func_ctx.in_line = in_line
         func_ctx.backward_partitions = bwd_parts
         func_ctx.backward_tensor_graph = bwd_graph
         func_ctx.scheduler = scheduler
@@ -250,7 +267,7 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
         _fork(streams)
         if func_ctx.checkpoint_activations:
             hs = func_ctx.saved_tensors
-            ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i]) for i in range(n)]
+            ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=func_ctx.in_line) for i in range(n)]
             _seed_forward(ctxs, hs, rotary, mask, seed)
             # with the generators as they were before the forward pass, and put back afterwards
             # (kareus/megatron/core/partitions/autograd_function.py:263-266)
@@ -285,12 +302,12 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
             if at_end is None:
                 at_end = n >= 4
             # ("pending": where such launches are left to be issued behind the last partition of the pass)
-            pending = [] if (at_end and func_ctx.wgrad_over_all_nanobatches) else None
+            pending = [] if (at_end and func_ctx.wgrad_over_all_nanobatches and not func_ctx.in_line) else None
             for c in ctxs:
                 for op_id, op_ctx in c.op_contexts.items():
                     op_ctx.wgrad_sink = sinks.setdefault(
                         op_id, {"n": n, "turn": turn, "defer": func_ctx.wgrad_over_all_nanobatches,
-                                "pending": pending})
+                                "pending": pending, "in_line": func_ctx.in_line})
                     op_ctx.nanobatch_index = c.batch_idx
 
         if func_ctx.join_in_place:

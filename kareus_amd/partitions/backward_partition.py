@@ -16,7 +16,7 @@ from typing import Dict, List, Optional
 
 from .context_manager import NanoBatchContext
 from .op_context import clear_tensor_data
-from .partition_base import PartitionBase, _current_stream
+from .partition_base import PartitionBase
 
 
 @dataclass
@@ -34,49 +34,47 @@ class BackwardPartition(PartitionBase):
         with self._on_stream(ctx), self._timed():
             return self._execute(ctx, pre_ctx, protected_tensor_ids or set())
 
-    def _fusable_follower(self, idx: int, start: int, ctx: NanoBatchContext):
+    def _fusable_follower(self, plans, idx: int, start: int, ctx: NanoBatchContext):
         """The op after ``idx`` when the two can run as one fused backward: the first op offers it
         (``can_fuse_backward_with``), the second consumes the first's only output and needs a
         gradient, and the scheduled launch point does not fall between them."""
-        if not self.fuse_backward_ops or idx + 1 >= len(self.comp_ops) or start == idx + 1:
+        plan = plans[idx]
+        if not plan.backward_pair or not self.fuse_backward_ops or start == idx + 1:
             return None
-        op, nxt = self.comp_ops[idx], self.comp_ops[idx + 1]
-        offer = getattr(op.operator, "can_fuse_backward_with", None)
-        if offer is None or not offer(nxt.operator):
-            return None
-        outs, nxt_ins = op.get_output_tensor_ids(), nxt.get_input_tensor_ids()
-        if not outs or not nxt_ins or nxt_ins[0] != outs[0]:
+        nxt = plans[idx + 1]
+        if not plan.operator.can_fuse_backward_with(nxt.operator):
             return None
         if not ctx.get_op_context(nxt.op_id).requires_grad:
             return None
-        if any(t not in ctx.tensor_store for t in nxt_ins[1:]):
+        if any([t not in ctx.tensor_store for t in nxt.extra_ids]):
             return None
         return nxt
 
     def _execute(self, ctx, pre_ctx, protected: set) -> Dict[int, List]:
-        start, _end, sm_num, block_size = self._setup_comm()
+        start, _end, sm_num, block_size = self._setup_comm(ctx.in_line)
         store = ctx.tensor_store
+        get, put = store.get, store.set
+        timed = PartitionBase.timer is not None
         comm_out, comm_extra = None, []
         launched = False
         grad_params: Dict[int, List] = {}
 
-        idx, num_ops = 0, len(self.comp_ops)
+        plans = self._plans()
+        idx, num_ops = 0, len(plans)
         while idx < num_ops:
-            op = self.comp_ops[idx]
+            op = plans[idx]
             op_ctx = ctx.get_op_context(op.op_id)
             if not op_ctx.requires_grad:
                 break
 
-            in_ids = op.get_input_tensor_ids()
-            dy = store.get(in_ids[0])
+            dy = get(op.first_in)
             group, group_ctxs = [op], [op_ctx]
-            grad_extra_out = [tuple(store.get(t) for t in in_ids[1:])] if len(in_ids) > 1 else []
-            follower = self._fusable_follower(idx, start, ctx)
+            grad_extra_out = [tuple([get(t) for t in op.extra_ids])] if op.extra_ids else []
+            follower = self._fusable_follower(plans, idx, start, ctx)
             if follower is not None:
                 group.append(follower)
                 group_ctxs.append(ctx.get_op_context(follower.op_id))
-                grad_extra_out = [tuple(store.get(t) for t in in_ids[1:]),
-                                  tuple(store.get(t) for t in follower.get_input_tensor_ids()[1:])]
+                grad_extra_out = [tuple([get(t) for t in op.extra_ids]), tuple([get(t) for t in follower.extra_ids])]
             last = idx + len(group) - 1
 
             if start == idx:
@@ -96,20 +94,20 @@ class BackwardPartition(PartitionBase):
                             *[t for t in member_ctx.saved_tensors if t is not None and id(t) not in protected]
                         )
                     member_ctx.saved_tensors = None
-                self._op_done(idx + k)
-            if last == start - 1:
-                self.comm_op.event_record(_current_stream())
+                if timed:
+                    self._op_done(idx + k)
+            if last == start - 1 and not ctx.in_line:
+                self.comm_op.event_record(self._here())
 
-            store.set(group[-1].get_output_tensor_ids()[0], dx)
+            put(group[-1].first_out, dx)
             # gradients of extra inputs: every member of a fused group may have some (a projection
             # that adds the residual in its epilogue hands the residual's gradient on)
             for k, member in enumerate(group):
                 extras_k = grad_extra_in[k] if (grad_extra_in and len(grad_extra_in) == len(group)) else (
                     grad_extra_in[-1] if (grad_extra_in and k == len(group) - 1) else ())
-                for j, tid in enumerate(member.get_output_tensor_ids()[1:]):
-                    g = extras_k[j] if j < len(extras_k) else None
+                for tid, g in zip(member.extra_out_ids, extras_k):
                     if g is not None:
-                        store.set(tid, g)
+                        put(tid, g)
             idx = last + 1
 
         if self.comm_op is not None:

@@ -75,13 +75,16 @@ class NanoBatchContext:
     tensor_store: TensorStore = field(default_factory=TensorStore)
     op_contexts: Dict[int, OperationContext] = field(default_factory=dict)
     stream: Optional[Any] = None  # torch.cuda.Stream this nanobatch runs on (None: caller's)
+    # the nanobatches of this pass run one after the other on the caller's stream, in the order the
+    # partitions are issued: every edge a schedule point would add is already there
+    in_line: bool = False
     # op_id -> tensor that op's forward output is to be written into (consumed when the op runs)
     output_sinks: Dict[int, torch.Tensor] = field(default_factory=dict)
     _saved_tensors: List[Optional[torch.Tensor]] = field(default_factory=list)
     _saved_ranges: Dict[int, Tuple[int, int]] = field(default_factory=dict)
 
     def create_op_context(self, op_id: int) -> OperationContext:
-        ctx = OperationContext()
+        ctx = OperationContext.__new__(OperationContext)  # every field at its class default
         self.op_contexts[op_id] = ctx
         return ctx
 

@@ -14,7 +14,7 @@ from dataclasses import dataclass
 
 from .context_manager import NanoBatchContext
 from .op_context import operator_parameters
-from .partition_base import PartitionBase, _current_stream
+from .partition_base import PartitionBase
 
 
 @dataclass
@@ -27,72 +27,67 @@ class ForwardPartition(PartitionBase):
         with self._on_stream(ctx), self._timed():
             self._execute(ctx, pre_ctx)
 
-    def _fusable_follower(self, idx: int, start: int):
-        """The op after ``idx`` when the two can run as one fused forward: the first op offers it
-        (``can_fuse_forward_with``), the second is a plain one-in/one-out op consuming the
-        first's only output, and the scheduled launch point does not fall between them."""
-        if not self.fuse_forward_ops or idx + 1 >= len(self.comp_ops) or start == idx + 1:
-            return None
-        op, nxt = self.comp_ops[idx], self.comp_ops[idx + 1]
-        offer = getattr(op.operator, "can_fuse_forward_with", None)
-        if offer is None or not offer(nxt.operator):
-            return None
-        outs, nxt_ins = op.get_output_tensor_ids(), nxt.get_input_tensor_ids()
-        if len(outs) != 1 or len(nxt_ins) != 1 or nxt_ins[0] != outs[0] or len(nxt.get_output_tensor_ids()) != 1:
-            return None
-        return nxt
-
     def _execute(self, ctx: NanoBatchContext, pre_ctx: NanoBatchContext) -> None:
-        start, _end, sm_num, block_size = self._setup_comm()
+        start, _end, sm_num, block_size = self._setup_comm(ctx.in_line)
         store = ctx.tensor_store
+        get, put, needs = store.get, store.set, store.needs_grad
+        sinks = ctx.output_sinks
+        timed = PartitionBase.timer is not None
         comm_out, comm_extra = None, []
 
-        idx, num_ops = 0, len(self.comp_ops)
+        plans = self._plans()
+        idx, num_ops = 0, len(plans)
         while idx < num_ops:
-            op = self.comp_ops[idx]
-            in_ids = op.get_input_tensor_ids()
-            x = store.get(in_ids[0])
-            extras = [tuple(store.get(t) for t in in_ids[1:])] if len(in_ids) > 1 else []
-            follower = self._fusable_follower(idx, start)
-            group = [op] if follower is None else [op, follower]
+            plan = plans[idx]
+            x = get(plan.first_in)
+            extras = [tuple([get(t) for t in plan.extra_ids])] if plan.extra_ids else []
+            # the op behind this one runs in the same call when the two offer a fused forward and the
+            # scheduled launch point does not fall between them
+            group = [plan]
+            if (plan.forward_pair and self.fuse_forward_ops and start != idx + 1
+                    and plan.operator.can_fuse_forward_with(plans[idx + 1].operator)):
+                group.append(plans[idx + 1])
 
             needs_grad = self.is_grad_enabled and (
-                any(store.needs_grad(t) for t in in_ids)
+                any([needs(t) for t in plan.in_ids])
                 or any(p.requires_grad for member in group for p in operator_parameters(member.operator))
             )
             group_ctxs = []
             for member in group:
                 op_ctx = ctx.create_op_context(member.op_id)
                 op_ctx.requires_grad = needs_grad
-                if ctx.output_sinks and member.op_id in ctx.output_sinks:
-                    op_ctx.out_sink = ctx.output_sinks.pop(member.op_id)
+                if ctx.in_line:
+                    op_ctx.alone = True
+                if sinks and member.op_id in sinks:
+                    op_ctx.out_sink = sinks.pop(member.op_id)
                 group_ctxs.append(op_ctx)
-            last = idx + len(group) - 1
+            k = len(group)
+            last = idx + k - 1
 
             if start == idx:
                 comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size)
 
-            k = len(group)
-            x, extra_out = op.operator.fuser_forward(
+            x, extra_out = plan.operator.fuser_forward(
                 group_ctxs,
                 x,
                 basic_op_extra_inputs=extras if k == 1 else [extras[0] if extras else (), ()],
                 basic_op_prev_ops=[None] * k,
                 basic_op_next_ops=[None] * k,
-                basic_op_kwargs=[{} for _ in range(k)],
+                basic_op_kwargs=[{}] if k == 1 else [{}, {}],
             )
 
-            for j in range(k):
-                self._op_done(idx + j)
-            if last == start - 1:
-                self.comm_op.event_record(_current_stream())
+            if timed:
+                for j in range(k):
+                    self._op_done(idx + j)
+            if last == start - 1 and not ctx.in_line:
+                self.comm_op.event_record(self._here())
 
-            out_ids = group[-1].get_output_tensor_ids()
-            store.set(out_ids[0], x, needs_grad)
-            for j, tid in enumerate(out_ids[1:]):
-                extra = extra_out[-1][j] if extra_out and extra_out[-1] else None
-                if extra is not None:
-                    store.set(tid, extra, needs_grad)
+            tail = group[-1]
+            put(tail.first_out, x, needs_grad)
+            if tail.extra_out_ids and extra_out and extra_out[-1]:
+                for tid, extra in zip(tail.extra_out_ids, extra_out[-1]):
+                    if extra is not None:
+                        put(tid, extra, needs_grad)
             idx = last + 1
 
         if self.comm_op is not None:

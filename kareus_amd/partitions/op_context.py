@@ -29,9 +29,14 @@ class OperationContext:
     to_save: Optional[Tuple[Optional[torch.Tensor], ...]] = None
     _saved_tensors_range: Optional[Tuple[int, int]] = None
     requires_grad: bool = True
+    # no kernel of another nanobatch's stream runs beside this op's (NanoBatchContext.in_line)
+    alone: bool = False
 
     def save_for_backward(self, *tensors: Optional[torch.Tensor]) -> None:
         self.to_save = tensors
+
+
+_EMPTY: Dict[Tuple[torch.device, torch.dtype], torch.Tensor] = {}  # one empty tensor per (device, dtype)
 
 
 def clear_tensor_data(*tensors: Optional[torch.Tensor]) -> None:
@@ -44,7 +49,11 @@ def clear_tensor_data(*tensors: Optional[torch.Tensor]) -> None:
     """
     for t in tensors:
         if t is not None:
-            t.data = torch.empty(0, device=t.device, dtype=t.dtype)
+            key = (t.device, t.dtype)
+            empty = _EMPTY.get(key)
+            if empty is None:
+                empty = _EMPTY[key] = torch.empty(0, device=t.device, dtype=t.dtype)
+            t.data = empty
 
 
 def operator_parameters(op: torch.nn.Module):

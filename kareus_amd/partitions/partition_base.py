@@ -86,6 +86,32 @@ def _current_stream():
     return stream_api().current_stream()
 
 
+_NOTHING = contextlib.nullcontext()
+
+
+class _OpPlan:
+    """What the graph says about one compute op of a partition, looked up once: the tensor ids of its ports, and
+    whether the op behind it consumes its output (``forward_pair`` / ``backward_pair``: the structural half of
+    "these two can run as one call"; the operators decide the rest when they run)."""
+
+    __slots__ = ("op", "operator", "op_id", "in_ids", "first_in", "extra_ids", "out_ids", "first_out", "extra_out_ids",
+                 "forward_pair", "backward_pair")
+
+    def __init__(self, op: ComputeOp, nxt: Optional[ComputeOp]) -> None:
+        self.op, self.operator, self.op_id = op, op.operator, op.op_id
+        self.in_ids = tuple(op.get_input_tensor_ids())
+        self.out_ids = tuple(op.get_output_tensor_ids())
+        self.first_in, self.extra_ids = self.in_ids[0] if self.in_ids else None, self.in_ids[1:]
+        self.first_out, self.extra_out_ids = self.out_ids[0] if self.out_ids else None, self.out_ids[1:]
+        self.forward_pair = self.backward_pair = False
+        if nxt is not None:
+            nxt_ins, nxt_outs = nxt.get_input_tensor_ids(), nxt.get_output_tensor_ids()
+            meets = bool(self.out_ids) and bool(nxt_ins) and nxt_ins[0] == self.out_ids[0]
+            self.forward_pair = (meets and len(self.out_ids) == 1 and len(nxt_ins) == 1 and len(nxt_outs) == 1
+                                 and hasattr(op.operator, "can_fuse_forward_with"))
+            self.backward_pair = meets and hasattr(op.operator, "can_fuse_backward_with")
+
+
 class _TimerScope:
     def __init__(self, timer, partition) -> None:
         self.timer, self.partition = timer, partition
@@ -119,6 +145,18 @@ class PartitionBase:
     def __post_init__(self) -> None:
         self._overlap_slots: Dict[str, int] = _build_overlap_slots(self.comp_ops)
 
+    def _plans(self) -> List[_OpPlan]:
+        plans = self.__dict__.get("_op_plans")
+        if plans is None or len(plans) != len(self.comp_ops):
+            ops = self.comp_ops
+            plans = self._op_plans = [_OpPlan(op, ops[i + 1] if i + 1 < len(ops) else None) for i, op in enumerate(ops)]
+        return plans
+
+    def _here(self):
+        """The stream the schedule point is told about; None for a slot without a stream of its own (one
+        nanobatch, or nanobatches in line), which ignores it."""
+        return None if getattr(self.comm_op.operator, "comm_stream", self) is None else _current_stream()
+
     # -- schedule ---------------------------------------------------------------
     def load_schedule(self, schedule) -> None:
         config = getattr(schedule, self.partition_key, None) if self.partition_key else None
@@ -135,7 +173,7 @@ class PartitionBase:
             end = _resolve_slot(self._overlap_slots, end)
         return ((start, end), shape)
 
-    def _setup_comm(self) -> Tuple[int, int, Optional[int], Optional[int]]:
+    def _setup_comm(self, in_line: bool = False) -> Tuple[int, int, Optional[int], Optional[int]]:
         if self.comm_op is None:
             return -1, -1, None, None
         (start, end), (sm_num, block_size) = self._get_comm_config()
@@ -150,8 +188,8 @@ class PartitionBase:
             )
         if self.force_no_overlap:
             start = -1
-        if start == 0:
-            self.comm_op.event_record(_current_stream())
+        if start == 0 and not in_line:
+            self.comm_op.event_record(self._here())
         return start, end, sm_num, block_size
 
     # -- the hand-over itself ---------------------------------------------------
@@ -179,17 +217,20 @@ class PartitionBase:
 
     def _launch_comm(self, pre_ctx, sm_num, block_size, *, backward: bool = False):
         """Release point reached earlier (event already recorded): wait on it, run."""
-        self.comm_op.event_wait()
+        if not pre_ctx.in_line:
+            self.comm_op.event_wait()
         return self._run_comm(pre_ctx, sm_num, block_size, backward)
 
     def _launch_comm_no_overlap(self, pre_ctx, sm_num, block_size, *, backward: bool = False):
         """No slot given: release only after all of this partition's compute."""
-        self.comm_op.event_record(_current_stream())
-        self.comm_op.event_wait()
+        if not pre_ctx.in_line:
+            self.comm_op.event_record(self._here())
+            self.comm_op.event_wait()
         return self._run_comm(pre_ctx, sm_num, block_size, backward)
 
     def _sync_comm(self, pre_ctx: NanoBatchContext, comm_output, comm_extra_outputs) -> None:
-        self.comm_op.sync(_current_stream())
+        if not pre_ctx.in_line:
+            self.comm_op.sync(self._here())
         ports = self.comm_op.output_ports
         src = self.comm_op.input_ports
         store = pre_ctx.tensor_store
@@ -208,7 +249,7 @@ class PartitionBase:
     def _timed(self):
         t = PartitionBase.timer
         if t is None:
-            return contextlib.nullcontext()
+            return _NOTHING
         return _TimerScope(t, self)
 
     def _op_done(self, idx: int) -> None:

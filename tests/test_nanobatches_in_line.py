@@ -1,0 +1,44 @@
+"""Small nanobatches run one after the other on the caller's stream (``LayerConfig.nanobatches_in_line``)."""
+
+import pytest
+import torch
+
+from kareus_amd import LayerConfig, LayerStack
+
+gpu = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")]
+
+
+def _cfg(**kw):
+    base = dict(hidden_size=4096, num_attention_heads=8, num_query_groups=2, kv_channels=128, ffn_hidden_size=3584)
+    return LayerConfig(**{**base, **kw})
+
+
+def test_the_rule_follows_the_size_of_a_nanobatch():
+    own = _cfg(streams_are_own=True)
+    assert own.nanobatches_in_line(256, 1) and own.nanobatches_in_line(1024, 1) and own.nanobatches_in_line(512, 2)
+    assert not own.nanobatches_in_line(4096, 1) and not own.nanobatches_in_line(1024, 4)
+    assert not _cfg().nanobatches_in_line(256, 1)                                    # a caller's own streams are used
+    assert not _cfg(streams_are_own=True, backend="eager").nanobatches_in_line(256, 1)
+
+
+@pytest.mark.parametrize("nnb,b,s", [(2, 2, 256), (4, 4, 136), (2, 6, 200), (4, 8, 64)])
+@pytest.mark.parametrize("recompute", [False, True])
+def test_in_line_gives_the_bits_of_a_run_without_streams(nnb, b, s, recompute):
+    g = torch.Generator().manual_seed(7)
+    x, go = (torch.randn(s, b, 512, generator=g).cuda().bfloat16() for _ in range(2))
+    got = []
+    for use_streams in (True, False):
+        cfg = _cfg(hidden_size=512, num_attention_heads=4, ffn_hidden_size=1024, num_layers=2, num_nanobatches=nnb,
+                   use_streams=use_streams, checkpoint_activations=recompute)
+        model = LayerStack(cfg, device="cuda", seed=3)
+        assert cfg.nanobatches_in_line(s, b // nnb) is use_streams
+        xd = x.clone().requires_grad_(True)
+        for _ in range(2):                                                           # a second pass on the same model
+            y = model(xd)
+            y.backward(go)
+        torch.cuda.synchronize()
+        got.append([y.detach(), xd.grad] + [p.grad for p in model.parameters()])
+    assert all(torch.equal(a, c) for a, c in zip(*got))
+
+
+test_in_line_gives_the_bits_of_a_run_without_streams = gpu[0](gpu[1](test_in_line_gives_the_bits_of_a_run_without_streams))
