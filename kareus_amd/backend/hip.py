@@ -829,8 +829,8 @@ class HipBackend:
                  beside_other_streams: bool = False, general_kernels: bool = False):
         """``beside_other_streams``: kernels of other streams use the compute units this launch leaves idle,
         so it is shaped for the least compute-unit time, not for its own latency.
-        ``general_kernels``: a shape outside the MFMA kernels (head dimension below 128, a ragged length)
-        takes the general fp32 kernels instead of being padded into the MFMA ones."""
+        ``general_kernels``: any shape but head dimension 128 with whole 128-row tiles takes the general fp32
+        kernels instead of the MFMA ones."""
         if not causal:
             raise RuntimeError("only causal attention is implemented")
         flags = (KR_ATTN_BESIDE_OTHER_STREAMS if beside_other_streams else 0) | (KR_ATTN_GENERAL_KERNELS if general_kernels else 0)

@@ -1,4 +1,4 @@
-// Causal grouped-query flash attention for head_dim 128 on the gfx950 matrix cores.
+// Causal grouped-query flash attention for head dimensions 128 and 64 on the gfx950 matrix cores.
 //
 // Roofline: MFMA.  Algorithmic work: forward 2*b*nq*s^2*hd FLOP (causal half of 4*s^2*hd),
 // backward 2.5x that.
@@ -25,7 +25,6 @@ namespace {
 
 constexpr int HD = 128;
 constexpr int BQ = 128;       // queries per workgroup (4 waves x 32, twice over)
-constexpr int BKV = 64;       // keys per staged tile
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 // Online softmax of the MFMA forward kernels: a row's exponents are taken against a reference
@@ -103,11 +102,13 @@ struct RowStage {
   }
 };
 
-// 32 rows x 128 channels of fp32 accumulators (scaled) -> bf16 rows at dst + row * row_stride
-__device__ __forceinline__ void store_rows_bf16(const RowStage& st, const f32x16 (&acc)[HD / 32],
-                                                float mul, bf16* dst, int64_t row_stride) {
+// 32 rows x D channels of fp32 accumulators (scaled) -> bf16 rows at dst + row * row_stride; RAGGED: only the
+// first `valid` rows exist
+template <int D, bool RAGGED>
+__device__ __forceinline__ void store_rows_bf16(const RowStage& st, const f32x16 (&acc)[D / 32],
+                                                float mul, bf16* dst, int64_t row_stride, int valid) {
 #pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
+  for (int pass = 0; pass < D / 64; ++pass) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -122,17 +123,18 @@ __device__ __forceinline__ void store_rows_bf16(const RowStage& st, const f32x16
     for (int q = 0; q < 4; ++q) {
       int row, col;
       const bf16x8 v = st.get_bf16(q, row, col);
-      stg8(dst + (int64_t)row * row_stride + pass * 64 + col, v);
+      if (!RAGGED || row < valid) stg8(dst + (int64_t)row * row_stride + pass * 64 + col, v);
     }
     RowStage::sync();
   }
 }
 
 // the same as fp32 rows (partial results for a later reduction)
-__device__ __forceinline__ void store_rows_f32(const RowStage& st, const f32x16 (&acc)[HD / 32],
+template <int D>
+__device__ __forceinline__ void store_rows_f32(const RowStage& st, const f32x16 (&acc)[D / 32],
                                                float mul, float* dst, int64_t row_stride) {
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt) {
+  for (int dt = 0; dt < D / 32; ++dt) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       f32x4 v;
@@ -159,9 +161,26 @@ static int check_attn_common(int s, int b, int nq, int nkv, int hd) {
   if (b > 65535 || nq > 65535) return KR_EUNSUPPORTED;  // grid dimensions of the general kernels
   return KR_OK;
 }
-// The MFMA kernels take head dimension 128 and whole 128-row tiles; everything else that passes
-// check_attn_common goes through the general fp32 kernels.
+// The training workloads' shapes: head dimension 128 and whole 128-row tiles.
 static bool attn_fast_path(int s, int hd) { return hd == HD && s % BQ == 0; }
+// The MFMA kernels also take head dimension 64 and ragged lengths as they lie (template parameters D and
+// RAGGED), provided that a lane's byte offset to any row of a 128-row tile fits 32 bits.  The alternative is to
+// copy into padded buffers of 128 channels and whole tiles and back (nine to eleven small launches, and half
+// of the matrix work on zeros where D = 64).  Measured, padded -> in place, forward / backward in us:
+//   s 256, b 1, 8/8 heads of 64       28 / 57     ->   9 / 22     (launches)
+//   s 2048, b 1, 32/8 heads of 64     75 / 190    ->  37 / 106
+//   s 4096, b 2, 32/8 heads of 64    282 / 909    -> 171 / 556    (0.80 / 0.62 PFLOP/s)
+//   s 776, b 1, 8/2 heads of 128      31 / 78     ->  20 / 53
+//   s 4000, b 4, 8/2 heads of 128    167 / 532    -> 145 / 485    (whole tiles, s 4096: 133 / 470)
+//   s 8184, b 2, 32/8 heads of 128  1121 / 3744   -> 1092 / 3623
+// Other head dimensions, and strides beyond that bound, are still padded.
+static bool attn_in_place(int s, int hd, std::initializer_list<int64_t> seq_strides) {
+  if (attn_fast_path(s, hd)) return true;
+  if (hd != 128 && hd != 64) return false;
+  for (int64_t ss : seq_strides)
+    if (127 * ss + 128 >= ((int64_t)1 << 31)) return false;
+  return true;
+}
 
 static int kr_compute_units() {
   static const int num_cus = [] {
@@ -258,14 +277,54 @@ __device__ __forceinline__ void dma_b32(const void* base, uint32_t byte_off, uin
 // fragment address is one per-lane base plus an instruction immediate.
 constexpr uint32_t BT_BLK = 1024 + 16, BT_BYTES = 16 * BT_BLK;
 
+// Head dimension 64: the same image holds 128 rows of 64 channels.  Image row i is row i of the tile
+// followed by row i + 64 (chunks 0-7 and 8-15), so requests, bank behaviour and the number of MFMAs a
+// tile feeds are those of 64 rows of 128 channels, and only the lane's source address and the fragment
+// immediates differ: 32-row block t of the tile sits in image rows 32 (t % 2) .., column half t / 2.
+// (Figures against padding the heads to 128 channels: at attn_in_place.)
+template <int D>
+constexpr int tile_rows = 64 * 128 / D;
+
+// row of the tile (relative to the request's first row) and channel a lane fetches
+template <int D>
+__device__ __forceinline__ int tile_lane_row(int lane) {
+  return (lane >> 4) * 16 + (D == 64 ? ((lane >> 3) & 1) * 64 : 0);
+}
+template <int D>
+__device__ __forceinline__ int tile_lane_ch(int lane) {
+  return (lane & (D / 8 - 1)) * 8;
+}
+template <int D>
+__device__ __forceinline__ uint32_t tile_lane_off(int lane, int ss) {
+  return (uint32_t)(tile_lane_row<D>(lane) * ss + tile_lane_ch<D>(lane)) * 2u;
+}
+
+// A tile that reaches beyond the sequence (rows row0 .. of `origin`, s rows exist): every lane's row is
+// clamped into the sequence for the request, and once it has landed the wave overwrites the rows
+// beyond s with zeros (zero_tail), before the barrier that publishes the tile.  `r` is the request's first
+// row within the tile.  Only the last tiles of a ragged sequence take this road.
+template <int D>
+__device__ __forceinline__ void request_clamped(const bf16* origin, int64_t ss, int row0, int r, int s, int lane,
+                                                uint32_t lds) {
+  const int base = row0 < s - 1 ? row0 : s - 1;
+  const int key = r + tile_lane_row<D>(lane), last = s - 1 - base;
+  dma_b128(origin + (int64_t)base * ss,
+           (uint32_t)((key < last ? key : last) * (int)ss + tile_lane_ch<D>(lane)) * 2u, lds);
+}
+template <int D>
+__device__ __forceinline__ void zero_block_tail(int row0, int r, int s, int lane, uint32_t lds) {
+  if (row0 + r + tile_lane_row<D>(lane) >= s) *(KR_LDS bf16x8*)(lds + lane * 16) = zero8();
+}
+
 // The four waves (wave = 0..3) of a group bring in one tile; `rows` = its first row in global
 // memory.  Wave w fills blocks w, w + 4, w + 8, w + 12, which hold the tile rows 4 w + 0..3
 // (+ 16, 32, 48): four consecutive rows, so a request costs one pointer increment.
+template <int D>
 __device__ __forceinline__ void bt_request(const bf16* rows, int64_t ss, uint32_t tile, int wave,
                                            int lane) {
   int l2 = lane;
   asm volatile("" : "+v"(l2));  // nothing derived from it is kept alive between requests
-  const uint32_t lane_off = (uint32_t)((l2 >> 4) * 16 * (int)ss + (l2 & 15) * 8) * 2u;
+  const uint32_t lane_off = tile_lane_off<D>(l2, (int)ss);
   const bf16* row = rows + (int64_t)(4 * wave) * ss;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -273,13 +332,27 @@ __device__ __forceinline__ void bt_request(const bf16* rows, int64_t ss, uint32_
     row += ss;
   }
 }
+// the same for a tile that may reach beyond the sequence, and the zeros behind its rows (see request_clamped)
+template <int D>
+__device__ __forceinline__ void bt_request_clamped(const bf16* origin, int64_t ss, int row0, int s, uint32_t tile,
+                                                   int wave, int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    request_clamped<D>(origin, ss, row0, 4 * wave + i, s, lane, tile + (wave + 4 * i) * BT_BLK);
+}
+template <int D>
+__device__ __forceinline__ void bt_zero_tail(int row0, int s, uint32_t tile, int wave, int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) zero_block_tail<D>(row0, 4 * wave + i, s, lane, tile + (wave + 4 * i) * BT_BLK);
+}
 // row-major fragments: lane gets row 32 t + lane % 32, channels 16 kk + 8 (lane / 32) + 0..7
 __device__ __forceinline__ uint32_t bt_rows_lane(int lane) {
   const int r = lane & 31;
   return (uint32_t)((4 * (r & 3) + ((r >> 2) & 3)) * BT_BLK + (r >> 4) * 256 + (lane >> 5) * 16);
 }
+template <int D>
 __device__ __forceinline__ bf16x8 bt_rows(uint32_t base, int t, int kk) {
-  return *(KR_LDS const bf16x8*)(base + t * 512 + kk * 32);
+  return *(KR_LDS const bf16x8*)(base + (t & 1) * 512 + (t >> 1) * 128 + kk * 32);
 }
 // transposed fragments: lane gets channel 32 dt + lane % 32, rows 16 g + {4 h + 0..3, 8 + 4 h + 0..3}
 __device__ __forceinline__ uint32_t bt_cols_lane(int lane) {
@@ -287,12 +360,13 @@ __device__ __forceinline__ uint32_t bt_cols_lane(int lane) {
   return (uint32_t)((4 * (p >> 2) + (lane >> 5)) * BT_BLK + ((lane >> 4) & 1) * 32 +
                     ((p & 3) >> 1) * 16 + (p & 1) * 8);
 }
+template <int D>
 __device__ __forceinline__ bf16x8 bt_cols(uint32_t base, int g, int dt) {
   union {
     struct { s16x4 lo, hi; } s;
     bf16x8 v;
   } u;
-  const uint32_t a = base + g * 256 + dt * 64;
+  const uint32_t a = base + (g & 3) * 256 + (g >> 2) * 128 + dt * 64;
   u.s.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a));
   u.s.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a + 2 * BT_BLK));
   return u.v;
@@ -308,6 +382,7 @@ __device__ __forceinline__ bf16x8 bt_cols(uint32_t base, int g, int dt) {
 // straight from global memory into blocked [64][128] LDS tiles.  A SIMD hosts one wave of each
 // half, so its matrix pipe and its vector ALU are busy at the same time instead of taking
 // turns, which is what happens when co-resident waves are in the same phase.
+template <int D, bool RAGGED>
 __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     bf16* __restrict__ o, float* __restrict__ lse, int s, int nq, int nkv, float scale_log2,
@@ -315,12 +390,15 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
     int64_t k_sh, int64_t v_ss, int64_t v_sb, int64_t v_sh, int64_t o_ss, int64_t o_sb,
     int64_t o_sg, int64_t o_sh) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  constexpr int NB = tile_rows<D> / 32;  // 32-key blocks of a tile
+  constexpr int DT = D / 32, KK = D / 16;
+  constexpr int TK = tile_rows<D>;       // keys of a tile
 
   const int half = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
   const int tid = threadIdx.x & 255;
   const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nqt = s / BQ;
+  const int nqt = (s + BQ - 1) / BQ;
   const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
   const int qt = nqt - 1 - (lid % nqt);  // longest rows first inside each (batch, head)
   const int head = (lid / nqt) % nq;
@@ -331,22 +409,27 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   const int q0 = qt * BQ;
   const int qw0 = q0 + wave * 32;
   const int qrow = qw0 + (lane & 31);
-  const bf16* qp = q + (int64_t)bi * q_sb + kvh * q_sg + hj * q_sh + (int64_t)qrow * q_ss;
+  const bf16* qp = q + (int64_t)bi * q_sb + kvh * q_sg + hj * q_sh +
+                   (int64_t)(RAGGED && qrow >= s ? s - 1 : qrow) * q_ss;
   const bf16* kb = k + (int64_t)bi * k_sb + (int64_t)kvh * k_sh;
   const bf16* vb = v + (int64_t)bi * v_sb + (int64_t)kvh * v_sh;
 
-  bf16x8 qf[HD / 16];
+  bf16x8 qf[KK];
 #pragma unroll
-  for (int kk = 0; kk < HD / 16; ++kk) qf[kk] = ldg8(qp + kk * 16 + h * 8);
+  for (int kk = 0; kk < KK; ++kk) qf[kk] = ldg8(qp + kk * 16 + h * 8);
 
-  f32x16 oacc[HD / 32];
+  f32x16 oacc[DT];
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[dt][e] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
 
-  const int nsteps = (q0 + BQ) / (2 * BKV);  // key tiles per half
+  const int total_tiles = (q0 + BQ) / TK;       // key tiles up to the workgroup's last row
+  const int nsteps = (total_tiles + 1) / 2;     // steps of the workgroup
+  // With 128-key tiles their number can be odd: half 1 then has one tile less (none at all for the first
+  // 128 queries) and idles through the last step.
+  const int nmine = D == 128 ? nsteps : (total_tiles + 1 - half) / 2;
   // LDS tile = 16 blocks; block b holds rows b, b+16, b+32, b+48 of the tile, 256 bytes each, in
   // the order one wave-wide request delivers them (lane p at +16 p: row b + 16 (p / 16), chunk
   // p % 16 — 16 consecutive lanes fetch one contiguous row), followed by a little padding.  With
@@ -356,7 +439,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   constexpr uint32_t KBLK = 1024 + 16, VBLK = 1024 + 64, KTILE = 16 * KBLK, VTILE = 16 * VBLK;
   const uint32_t kbuf = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem + half * 2 * (KTILE + VTILE);
   const uint32_t vbuf = kbuf + 2 * KTILE;
-  auto key_of = [&](int j) { return (2 * j + half) * BKV; };
+  auto key_of = [&](int j) { return (2 * j + half) * TK; };
   // row-major fragment (K): row 32 t + lane%32, chunk 2 kk + h  ->  + 512 t + 32 kk
   const uint32_t kfrag_lane = (uint32_t)((lane & 15) * KBLK + ((lane >> 4) & 1) * 256 + h * 16);
   // transposed fragment (V): rows 16 g + 4 h + p/4 (+8), channels 32 dt + 16 (lane/16 % 2) +
@@ -371,43 +454,57 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   // number of instructions the wave has to issue.
   const bf16* kreq = kb + (int64_t)(key_of(0) + wave) * k_ss;
   const bf16* vreq = vb + (int64_t)(key_of(0) + wave) * v_ss;
-  const int64_t k_tiles2 = (int64_t)2 * BKV * k_ss, v_tiles2 = (int64_t)2 * BKV * v_ss;
+  const int64_t k_tiles2 = (int64_t)2 * TK * k_ss, v_tiles2 = (int64_t)2 * TK * v_ss;
   const int64_t k_rows4 = 4 * k_ss, v_rows4 = 4 * v_ss;
-  const uint32_t k_lane_off = (uint32_t)((lane >> 4) * 16 * (int)k_ss + (lane & 15) * 8) * 2u;
-  const uint32_t v_lane_off = (uint32_t)((lane >> 4) * 16 * (int)v_ss + (lane & 15) * 8) * 2u;
-  auto request = [&](const bf16* row, int64_t rows4, uint32_t lane_off, uint32_t tile, uint32_t blk_bytes) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      dma_b128(row, lane_off, tile + (wave + 4 * i) * blk_bytes);
-      row += rows4;
-    }
-  };
-  auto request_k = [&](uint32_t tile) {
-    request(kreq, k_rows4, k_lane_off, tile, KBLK);
-    kreq += k_tiles2;
-  };
-  auto request_v = [&](uint32_t tile) {
-    request(vreq, v_rows4, v_lane_off, tile, VBLK);
-    vreq += v_tiles2;
-  };
-  // one of a tile's four requests of this wave (i = 0..3); the last one moves on to the next tile
-  auto request_k_part = [&](uint32_t tile, int i) {
-    dma_b128(kreq + i * k_rows4, k_lane_off, tile + (wave + 4 * i) * KBLK);
+  const uint32_t k_lane_off = tile_lane_off<D>(lane, (int)k_ss);
+  const uint32_t v_lane_off = tile_lane_off<D>(lane, (int)v_ss);
+  // one of a tile's four requests of this wave (i = 0..3); the last one moves on to the next tile.  `j` is the
+  // tile's step: only the tile a ragged sequence ends in needs it.
+  auto request_k_part = [&](uint32_t tile, int j, int i) {
+    const uint32_t dst = tile + (wave + 4 * i) * KBLK;
+    if (RAGGED && key_of(j) + TK > s)
+      request_clamped<D>(kb, k_ss, key_of(j), wave + 4 * i, s, lane, dst);
+    else
+      dma_b128(kreq + i * k_rows4, k_lane_off, dst);
     if (i == 3) kreq += k_tiles2;
   };
-  auto request_v_part = [&](uint32_t tile, int i) {
-    dma_b128(vreq + i * v_rows4, v_lane_off, tile + (wave + 4 * i) * VBLK);
+  auto request_v_part = [&](uint32_t tile, int j, int i) {
+    const uint32_t dst = tile + (wave + 4 * i) * VBLK;
+    if (RAGGED && key_of(j) + TK > s)
+      request_clamped<D>(vb, v_ss, key_of(j), wave + 4 * i, s, lane, dst);
+    else
+      dma_b128(vreq + i * v_rows4, v_lane_off, dst);
     if (i == 3) vreq += v_tiles2;
   };
+  auto request_k = [&](uint32_t tile, int j) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) request_k_part(tile, j, i);
+  };
+  auto request_v = [&](uint32_t tile, int j) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) request_v_part(tile, j, i);
+  };
+  // rows of V tile j beyond the sequence: their probabilities are zero, and so must their values be (a copy
+  // of the last row could be infinite).  K needs none: masked scores are replaced, whatever they are.
+  auto zero_v_tail = [&](int j) {
+    if (RAGGED && key_of(j) + TK > s) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        zero_block_tail<D>(key_of(j), wave + 4 * i, s, lane, vbuf + (j & 1) * VTILE + (wave + 4 * i) * VBLK);
+    }
+  };
 
-  request_k(kbuf);
-  if (nsteps > 1) request_k(kbuf + KTILE);
-  request_v(vbuf);
+  if (D == 128 || nmine > 0) {
+    request_k(kbuf, 0);
+    if (nmine > 1) request_k(kbuf + KTILE, 1);
+    request_v(vbuf, 0);
+  }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  if (D == 128 || nmine > 0) zero_v_tail(0);
   __syncthreads();
   if (half == 1) __syncthreads();  // half 1 starts one period late
 
-  bf16x8 pb[2][2];
+  bf16x8 pb[NB][2];
 
   // O^T += V^T . P^T for tile jj of this half (pb holds its probabilities)
   auto pv_step = [&](int jj) {
@@ -418,27 +515,30 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
           struct { s16x4 lo, hi; } s;
           bf16x8 v;
         } u;
-        const uint32_t a = va + g * 256 + dt * 64;
+        const uint32_t a = va + (g & 3) * 256 + (g >> 2) * 128 + dt * 64;
         u.s.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a));
         u.s.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a + 8 * VBLK));
         return u.v;
       };
       // fragments are fetched one group of four MFMAs ahead, by hand: left to itself the
       // scheduler hoists every read of the period to its start and runs out of registers
-      bf16x8 fr[2][HD / 32];
+      // group g: 16-key groups 4 g / DT .., channel blocks 0 .. DT - 1 of each
+      bf16x8 fr[2][4];
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; ++dt) fr[0][dt] = vfrag(0, dt);
+      for (int u = 0; u < 4; ++u) fr[0][u] = vfrag(u / DT, u % DT);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         if (g + 1 < 4) {
 #pragma unroll
-          for (int dt = 0; dt < HD / 32; ++dt) fr[(g + 1) & 1][dt] = vfrag(g + 1, dt);
+          for (int u = 0; u < 4; ++u) fr[(g + 1) & 1][u] = vfrag((g + 1) * 4 / DT + u / DT, u % DT);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int dt = 0; dt < HD / 32; ++dt)
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][dt], pb[g >> 1][g & 1],
-                                                             oacc[dt], 0, 0, 0);
+        for (int u = 0; u < 4; ++u) {
+          const int kg = g * 4 / DT + u / DT;
+          oacc[u % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][u], pb[kg >> 1][kg & 1],
+                                                                 oacc[u % DT], 0, 0, 0);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
       };
@@ -446,31 +546,34 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   settle_scalar_loads();
   for (int j = 0; j < nsteps; ++j) {
     // ---- matrix period: O^T += V^T . P^T of tile j-1, then S^T = K . Q^T of tile j
-    f32x16 sacc[2];
+    f32x16 sacc[NB];
     __builtin_amdgcn_s_setprio(1);
-    if (j > 0) pv_step(j - 1);
-    {
+    const bool mine = D == 128 || j < nmine;
+    if (j > 0 && (D == 128 || j - 1 < nmine)) pv_step(j - 1);
+    if (mine) {
       uint32_t ka = kbuf + (j & 1) * KTILE + kfrag_lane;
       asm volatile("" : "+v"(ka));
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) sacc[t][e] = 0.f;
-      auto kfrag = [&](int t, int kk) { return *(KR_LDS const bf16x8*)(ka + t * 512 + kk * 32); };
+      auto kfrag = [&](int t, int kk) {
+        return *(KR_LDS const bf16x8*)(ka + (t & 1) * 512 + (t >> 1) * 128 + kk * 32);
+      };
       bf16x8 fr[2][4];  // group g: contraction steps 2g, 2g+1 for both 32-key blocks
 #pragma unroll
-      for (int u = 0; u < 4; ++u) fr[0][u] = kfrag(u & 1, u >> 1);
+      for (int u = 0; u < 4; ++u) fr[0][u] = kfrag(u % NB, u / NB);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         if (g + 1 < 4) {
 #pragma unroll
-          for (int u = 0; u < 4; ++u) fr[(g + 1) & 1][u] = kfrag(u & 1, 2 * (g + 1) + (u >> 1));
+          for (int u = 0; u < 4; ++u) fr[(g + 1) & 1][u] = kfrag(u % NB, (g + 1) * (4 / NB) + u / NB);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-          sacc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][u], qf[2 * g + (u >> 1)],
-                                                                sacc[u & 1], 0, 0, 0);
+          sacc[u % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][u], qf[g * (4 / NB) + u / NB],
+                                                                 sacc[u % NB], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -481,22 +584,22 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
     // the eight requests for K(j+2) and V(j+1) (their buffers were last read in the matrix period
     // that just ended).  Issued back to back the requests hold the wave until the address path
     // has taken them, which is as long as the softmax itself.
-    const bool want_k = j + 2 < nsteps, want_v = j + 1 < nsteps;
+    const bool want_k = j + 2 < nmine, want_v = j + 1 < nmine;
     const uint32_t k_dst = kbuf + (j & 1) * KTILE, v_dst = vbuf + ((j + 1) & 1) * VTILE;
-    {
+    if (mine) {
       const int key0 = key_of(j);
-      if (key0 + BKV - 1 > qw0) {
+      if (key0 + TK - 1 > qw0) {
         asm volatile("" ::: "memory");  // keeps this a branch: off the diagonal no mask code runs
         const int lim = qrow - key0 - 4 * h;  // element offsets beyond it are keys after the query
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < NB; ++t)
 #pragma unroll
           for (int e = 0; e < 16; ++e)
             if (t * 32 + 8 * (e >> 2) + (e & 3) > lim) sacc[t][e] = -INFINITY;
       }
       float mx = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[t][e]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, KR_WAVE));
@@ -509,7 +612,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
       const float neg_m = -m_ref * scale_log2;
       float psum = 0.f;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[t][e], scale_log2, neg_m));
@@ -519,33 +622,36 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
           // would be alive together
           if ((e & 7) == 7) {
             __builtin_amdgcn_sched_barrier(0);
-            const int c = t * 2 + (e >> 3);   // 0..3
-            if (want_k) request_k_part(k_dst, c);
-            if (want_v) request_v_part(v_dst, c);
+            const int c = t * 2 + (e >> 3);   // 0 .. 2 NB - 1; four of them carry requests
+            if (c % (NB / 2) == 0) {
+              if (want_k) request_k_part(k_dst, j + 2, c / (NB / 2));
+              if (want_v) request_v_part(v_dst, j + 1, c / (NB / 2));
+            }
             __builtin_amdgcn_sched_barrier(0);
           }
         }
       l_run = l_run * alpha + psum;
       if (__any(moved)) {
 #pragma unroll
-        for (int dt = 0; dt < HD / 32; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
           for (int e = 0; e < 16; ++e) oacc[dt][e] *= alpha;
       }
     }
     // what was requested one step ago (K(j+1), V(j)) is read in the next matrix period; exactly
     // the requests of this period (4 per tile and wave, retired in order) may stay in flight
-    if (j + 2 < nsteps)
+    if (want_k)
       __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): K(j+2) and V(j+1) were requested
-    else if (j + 1 < nsteps)
+    else if (want_v)
       __builtin_amdgcn_s_waitcnt(0x0f74);  // vmcnt(4): only V(j+1)
     else
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): nothing was requested
+    if (RAGGED && j > 0 && mine) zero_v_tail(j);  // (tile 0 was settled before the loop)
     __syncthreads();
   }
   // last matrix period: the product of the final tile
   __builtin_amdgcn_s_setprio(1);
-  pv_step(nsteps - 1);
+  if (D == 128 || nsteps - 1 < nmine) pv_step(nsteps - 1);
   __builtin_amdgcn_s_setprio(0);
   __syncthreads();
   if (half == 0) __syncthreads();  // the period half 1 is behind by
@@ -558,7 +664,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
     xch[slot] = m_run;
     xch[256 + slot] = l_run;
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int e = 0; e < 16; ++e) xch[(2 + dt * 16 + e) * 256 + slot] = oacc[dt][e];
   }
@@ -572,7 +678,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
     m_run = m_new;
     l_run = l_run * a_a + l_b * a_b;
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int e = 0; e < 16; ++e)
         oacc[dt][e] = oacc[dt][e] * a_a + xch[(2 + dt * 16 + e) * 256 + slot] * a_b;
@@ -583,11 +689,11 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   rs.init(reinterpret_cast<char*>(smem) + 68 * 1024 + wave * 4096, lane);
   bf16* op = o + (int64_t)bi * o_sb + kvh * o_sg + hj * o_sh + (int64_t)qw0 * o_ss;
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[dt][e] *= inv_l;
-  store_rows_bf16(rs, oacc, 1.0f, op, o_ss);
-  if (h == 0)
+  store_rows_bf16<D, RAGGED>(rs, oacc, 1.0f, op, o_ss, s - qw0);
+  if (h == 0 && (!RAGGED || qrow < s))
     lse[((int64_t)bi * nq + head) * s + qrow] =
         (m_run * scale_log2 + __builtin_amdgcn_logf(l_tot)) * kLn2;
 }
@@ -602,6 +708,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
 // tiles (V(j+2)).  K(j) is read in periods 2j (half 0) and 2j+1 (half 1), V(j) in 2j+2 and 2j+3;
 // rings of three tiles each give every request three to four periods to land.  Half 0 needs two
 // tiles fewer than half 1 (its rows end 128 earlier) and idles through the last two steps.
+template <int D, bool RAGGED>
 __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     bf16* __restrict__ o, float* __restrict__ lse, int s, int nq, int nkv, float scale_log2,
@@ -609,13 +716,16 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
     int64_t k_sh, int64_t v_ss, int64_t v_sb, int64_t v_sh, int64_t o_ss, int64_t o_sb,
     int64_t o_sg, int64_t o_sh) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  constexpr int NB = tile_rows<D> / 32;  // 32-key blocks of a tile
+  constexpr int DT = D / 32, KK = D / 16;
+  constexpr int TK = tile_rows<D>;       // keys of a tile
   constexpr int BQ2 = 256;
 
   const int half = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
   const int tid = threadIdx.x & 255;
   const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nqt = s / BQ2;
+  const int nqt = (s + BQ2 - 1) / BQ2;
   int qt, pair;
   longest_first(xcd_contiguous_id(blockIdx.x, gridDim.x), nqt, gridDim.x / nqt, qt, pair);
   const int head = pair % nq;
@@ -626,23 +736,24 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
   const int q0 = qt * BQ2;
   const int qw0 = q0 + half * 128 + wave * 32;
   const int qrow = qw0 + (lane & 31);
-  const bf16* qp = q + (int64_t)bi * q_sb + kvh * q_sg + hj * q_sh + (int64_t)qrow * q_ss;
+  const bf16* qp = q + (int64_t)bi * q_sb + kvh * q_sg + hj * q_sh +
+                   (int64_t)(RAGGED && qrow >= s ? s - 1 : qrow) * q_ss;
   const bf16* kb = k + (int64_t)bi * k_sb + (int64_t)kvh * k_sh;
   const bf16* vb = v + (int64_t)bi * v_sb + (int64_t)kvh * v_sh;
 
-  bf16x8 qf[HD / 16];
+  bf16x8 qf[KK];
 #pragma unroll
-  for (int kk = 0; kk < HD / 16; ++kk) qf[kk] = ldg8(qp + kk * 16 + h * 8);
+  for (int kk = 0; kk < KK; ++kk) qf[kk] = ldg8(qp + kk * 16 + h * 8);
 
-  f32x16 oacc[HD / 32];
+  f32x16 oacc[DT];
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[dt][e] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
 
-  const int ntiles = (q0 + BQ2) / BKV;                // tiles the workgroup walks (>= 4)
-  const int nmine = (q0 + half * 128 + 128) / BKV;    // tiles with keys this half's rows see
+  const int ntiles = (q0 + BQ2) / TK;                 // tiles the workgroup walks (>= 2)
+  const int nmine = (q0 + half * 128 + 128) / TK;     // tiles with keys this half's rows see
   constexpr uint32_t KBLK = 1024 + 16, VBLK = 1024 + 64, KTILE = 16 * KBLK, VTILE = 16 * VBLK;
   const uint32_t kring = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem;
   const uint32_t vring = kring + 3 * KTILE;
@@ -657,21 +768,35 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
   const uint32_t r_blk = half ? VBLK : KBLK, r_tile = half ? VTILE : KTILE;
   const uint32_t r_ring = half ? vring : kring;
   const bf16* req = (half ? vb : kb) + (int64_t)wave * r_ss;
-  const int64_t r_next = (int64_t)BKV * r_ss, r_rows4 = 4 * r_ss;
-  const uint32_t r_lane_off = (uint32_t)((lane >> 4) * 16 * (int)r_ss + (lane & 15) * 8) * 2u;
-  auto request_part = [&](uint32_t tile, int i) {
-    dma_b128(req + i * r_rows4, r_lane_off, tile + (wave + 4 * i) * r_blk);
+  const int64_t r_next = (int64_t)TK * r_ss, r_rows4 = 4 * r_ss;
+  const uint32_t r_lane_off = tile_lane_off<D>(lane, (int)r_ss);
+  auto request_part = [&](uint32_t tile, int j, int i) {
+    const uint32_t dst = tile + (wave + 4 * i) * r_blk;
+    if (RAGGED && (j + 1) * TK > s)
+      request_clamped<D>(half ? vb : kb, r_ss, j * TK, wave + 4 * i, s, lane, dst);
+    else
+      dma_b128(req + i * r_rows4, r_lane_off, dst);
     if (i == 3) req += r_next;
+  };
+  // rows of V tile j (ring slot `slot`) beyond the sequence: as in the kernel above
+  auto zero_v_tail = [&](int j, int slot) {
+    if (RAGGED && half == 1 && (j + 1) * TK > s) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        zero_block_tail<D>(j * TK, wave + 4 * i, s, lane, vring + slot * VTILE + (wave + 4 * i) * VBLK);
+    }
   };
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) request_part(r_ring + t * r_tile, i);
+    for (int i = 0; i < 4; ++i) request_part(r_ring + t * r_tile, t, i);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  zero_v_tail(0, 0);
+  zero_v_tail(1, 1);
   __syncthreads();
   if (half == 1) __syncthreads();  // half 1 starts one period late
 
-  bf16x8 pb[2][2];
+  bf16x8 pb[NB][2];
 
   // O^T += V^T . P^T for the tile in ring slot `slot` (pb holds its probabilities)
   auto pv_step = [&](int slot) {
@@ -682,25 +807,27 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
         struct { s16x4 lo, hi; } s;
         bf16x8 v;
       } u;
-      const uint32_t a = va + g * 256 + dt * 64;
+      const uint32_t a = va + (g & 3) * 256 + (g >> 2) * 128 + dt * 64;
       u.s.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a));
       u.s.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a + 8 * VBLK));
       return u.v;
     };
-    bf16x8 fr[2][HD / 32];
+    bf16x8 fr[2][4];
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt) fr[0][dt] = vfrag(0, dt);
+    for (int u = 0; u < 4; ++u) fr[0][u] = vfrag(u / DT, u % DT);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       if (g + 1 < 4) {
 #pragma unroll
-        for (int dt = 0; dt < HD / 32; ++dt) fr[(g + 1) & 1][dt] = vfrag(g + 1, dt);
+        for (int u = 0; u < 4; ++u) fr[(g + 1) & 1][u] = vfrag((g + 1) * 4 / DT + u / DT, u % DT);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; ++dt)
-        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][dt], pb[g >> 1][g & 1],
-                                                           oacc[dt], 0, 0, 0);
+      for (int u = 0; u < 4; ++u) {
+        const int kg = g * 4 / DT + u / DT;
+        oacc[u % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][u], pb[kg >> 1][kg & 1],
+                                                               oacc[u % DT], 0, 0, 0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -709,7 +836,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
   settle_scalar_loads();
   for (int j = 0; j < ntiles; ++j) {
     // ---- matrix period: O^T += V^T . P^T of tile j-1, then S^T = K . Q^T of tile j
-    f32x16 sacc[2];
+    f32x16 sacc[NB];
     const bool mine = j < nmine;
     __builtin_amdgcn_s_setprio(1);
     if (j > 0 && j - 1 < nmine) pv_step(slot_prev);
@@ -717,24 +844,26 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
       uint32_t ka = kring + slot * KTILE + kfrag_lane;
       asm volatile("" : "+v"(ka));
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) sacc[t][e] = 0.f;
-      auto kfrag = [&](int t, int kk) { return *(KR_LDS const bf16x8*)(ka + t * 512 + kk * 32); };
+      auto kfrag = [&](int t, int kk) {
+        return *(KR_LDS const bf16x8*)(ka + (t & 1) * 512 + (t >> 1) * 128 + kk * 32);
+      };
       bf16x8 fr[2][4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) fr[0][u] = kfrag(u & 1, u >> 1);
+      for (int u = 0; u < 4; ++u) fr[0][u] = kfrag(u % NB, u / NB);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         if (g + 1 < 4) {
 #pragma unroll
-          for (int u = 0; u < 4; ++u) fr[(g + 1) & 1][u] = kfrag(u & 1, 2 * (g + 1) + (u >> 1));
+          for (int u = 0; u < 4; ++u) fr[(g + 1) & 1][u] = kfrag(u % NB, (g + 1) * (4 / NB) + u / NB);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-          sacc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][u], qf[2 * g + (u >> 1)],
-                                                                sacc[u & 1], 0, 0, 0);
+          sacc[u % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[g & 1][u], qf[g * (4 / NB) + u / NB],
+                                                                 sacc[u % NB], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -747,19 +876,19 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
     const bool want = j + 2 < ntiles;
     const uint32_t r_dst = r_ring + slot_req * r_tile;
     if (mine) {
-      const int key0 = j * BKV;
-      if (key0 + BKV - 1 > qw0) {
+      const int key0 = j * TK;
+      if (key0 + TK - 1 > qw0) {
         asm volatile("" ::: "memory");  // keeps this a branch: off the diagonal no mask code runs
         const int lim = qrow - key0 - 4 * h;  // element offsets beyond it are keys after the query
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < NB; ++t)
 #pragma unroll
           for (int e = 0; e < 16; ++e)
             if (t * 32 + 8 * (e >> 2) + (e & 3) > lim) sacc[t][e] = -INFINITY;
       }
       float mx = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sacc[t][e]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, KR_WAVE));
@@ -772,7 +901,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
       const float neg_m = -m_ref * scale_log2;
       float psum = 0.f;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[t][e], scale_log2, neg_m));
@@ -780,20 +909,21 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
           pb[t][e >> 3][e & 7] = (bf16)pe;
           if ((e & 7) == 7) {
             __builtin_amdgcn_sched_barrier(0);
-            if (want) request_part(r_dst, t * 2 + (e >> 3));
+            const int c = t * 2 + (e >> 3);
+            if (c % (NB / 2) == 0 && want) request_part(r_dst, j + 2, c / (NB / 2));
             __builtin_amdgcn_sched_barrier(0);
           }
         }
       l_run = l_run * alpha + psum;
       if (__any(moved)) {
 #pragma unroll
-        for (int dt = 0; dt < HD / 32; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
           for (int e = 0; e < 16; ++e) oacc[dt][e] *= alpha;
       }
     } else if (want) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) request_part(r_dst, i);
+      for (int i = 0; i < 4; ++i) request_part(r_dst, j + 2, i);
     }
     // tile j+1 of this half's operand (requested one step ago) is read from the next period on;
     // only this period's four requests may stay in flight
@@ -801,6 +931,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
       __builtin_amdgcn_s_waitcnt(0x0f74);  // vmcnt(4)
     else
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    if (RAGGED && j > 0 && j + 1 < ntiles) zero_v_tail(j + 1, slot == 2 ? 0 : slot + 1);
     __syncthreads();
     slot_prev = slot;
     slot = slot == 2 ? 0 : slot + 1;
@@ -822,41 +953,53 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
   rs.init(reinterpret_cast<char*>(smem) + (half * 4 + wave) * 4096, lane);
   bf16* op = o + (int64_t)bi * o_sb + kvh * o_sg + hj * o_sh + (int64_t)qw0 * o_ss;
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[dt][e] *= inv_l;
-  store_rows_bf16(rs, oacc, 1.0f, op, o_ss);
-  if (h == 0)
+  store_rows_bf16<D, RAGGED>(rs, oacc, 1.0f, op, o_ss, s - qw0);
+  if (h == 0 && (!RAGGED || qrow < s))
     lse[((int64_t)bi * nq + head) * s + qrow] =
         (m_run * scale_log2 + __builtin_amdgcn_logf(l_tot)) * kLn2;
 }
 
+// delta and the log2-domain statistics have rows of sp = s rounded up to 128: positions beyond s get values
+// that make their probabilities exactly zero.
+constexpr float kPadLse = 1e30f;  // exp2(x - 1.4e30) = 0 for every finite score
+
+template <int D>
 __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* __restrict__ dout,
                                                          const bf16* __restrict__ o,
                                                          const float* __restrict__ lse,
                                                          float* __restrict__ delta,
-                                                         float* __restrict__ neg_lse2, int s, int nq,
+                                                         float* __restrict__ neg_lse2, int s, int sp, int nq,
                                                          int per, int64_t total_rows, QLayout dol,
                                                          QLayout ol) {
-  // 16 lanes per (batch, head, position) row of 128 channels
-  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 4;
-  const int sub = threadIdx.x & 15;
+  constexpr int LPR = D / 8;  // lanes per (batch, head, position) row
+  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LPR;
+  const int sub = threadIdx.x & (LPR - 1);
   if (row >= total_rows) return;
-  const int si = (int)(row % s);
-  const int head = (int)((row / s) % nq);
-  const int bi = (int)(row / ((int64_t)s * nq));
+  const int si = (int)(row % sp);
+  const int head = (int)((row / sp) % nq);
+  const int bi = (int)(row / ((int64_t)sp * nq));
+  if (si >= s) {
+    if (sub == 0) {
+      delta[row] = 0.f;
+      neg_lse2[row] = -kPadLse * kLog2e;
+    }
+    return;
+  }
   const bf16x8 a = ldg8(dout + dol.at(bi, head, per) + (int64_t)si * dol.s_ + sub * 8);
   const bf16x8 b = ldg8(o + ol.at(bi, head, per) + (int64_t)si * ol.s_ + sub * 8);
   float acc = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc += (float)a[e] * (float)b[e];
 #pragma unroll
-  for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, KR_WAVE);
+  for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, KR_WAVE);
   if (sub == 0) {
     delta[row] = acc;
     // -lse in the log2 domain, so that the dK/dV kernel's exponent is one multiply-add and its
     // row statistics can go straight from global memory into LDS
-    neg_lse2[row] = -lse[row] * kLog2e;
+    neg_lse2[row] = -lse[((int64_t)bi * nq + head) * s + si] * kLog2e;
   }
 }
 
@@ -879,8 +1022,9 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* __restrict_
 // requested right after that barrier into the same stage and has an iteration and a half to
 // land (it must be complete by the first barrier of iteration it+2: the score waves start on a
 // tile one block ahead).
-// PARTIAL = true: fp32 results for this query head go to part_k / part_v [b, nq, qsplit, s, 128].
-template <bool PARTIAL>
+// PARTIAL = true: fp32 results for this query head go to part_k / part_v [b, nq, qsplit, sp, D].
+// D = 64: a tile is 128 queries, walked as four 32-query blocks with a hand-over each.
+template <int D, bool RAGGED, bool PARTIAL>
 __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const float* __restrict__ neg_lse2, const float* __restrict__ delta,
@@ -888,8 +1032,11 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
     float* __restrict__ part_v, int s, int nq, int nkv, int qsplit, int hpw, float scale, float scale_log2,
     QLayout ql, KLayout kl, KLayout vl, QLayout dol, KLayout dkl, KLayout dvl) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
-  // stage layout: Q tile | dO tile (blocked tiles) | lse[64] fp32 | delta[64] fp32
-  constexpr uint32_t STAGE = 2 * BT_BYTES + 512;  // bytes
+  constexpr int TQ = tile_rows<D>, NSUB = TQ / 32;  // queries of a tile, its 32-query blocks
+  constexpr int DT = D / 32, KK = D / 16;
+  constexpr int NF = 4 * DT;                        // transposed fragments of a block, two channel operands
+  // stage layout: Q tile | dO tile (blocked tiles) | lse[TQ] fp32 | delta[TQ] fp32
+  constexpr uint32_t STAGE = 2 * BT_BYTES + 8 * TQ;  // bytes
   constexpr int NS = 3;
   // hand-over area behind the stages: [block parity][key block][slot 0..3][lane] 16 bytes each
   constexpr uint32_t XCH = NS * STAGE;
@@ -898,7 +1045,8 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int role = wave8 >> 2;  // 0: score wave, 1: accumulate wave
   const int wave = wave8 & 3;   // key block of the tile
-  const int nkt = s / 128;
+  const int sp = RAGGED ? (s + 127) / 128 * 128 : s;  // rows of the statistics and of the partial results
+  const int nkt = sp / 128;
   const int lid_all = xcd_contiguous_id(blockIdx.x, gridDim.x);
   const int part = lid_all % qsplit, lid = lid_all / qsplit;
   // A workgroup takes `hpw` consecutive query heads of one KV group, one after the other: its K / V
@@ -915,19 +1063,20 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const int key0 = kt * 128;
   const int kw0 = key0 + wave * 32;
   const int krow = kw0 + (lane & 31);
-  const int qt_first = key0 / 64;
-  const int niter = (s / 64 - qt_first - part + qsplit - 1) / qsplit;  // this part's query tiles of 64, per head
+  const int qt_first = key0 / TQ;
+  // this part's query tiles, per head (with tiles of 128 the second part of the last key tile has none)
+  const int niter = (sp / TQ - qt_first - part + qsplit - 1) / qsplit;
   const int nit_all = niter * hpw;                                       // ... over all heads of the workgroup
   const uint32_t lds0 = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem;
   const uint32_t xch_lane = lds0 + XCH + wave * 4096 + lane * 16;  // + parity * 16384 + slot * 1024
 
   if (role == 0) {
     // ------------------------------------------------------------------ score waves
-    const bf16* kp = k + kl.at(bi, kvh) + (int64_t)krow * kl.s_;
-    const bf16* vp = v + vl.at(bi, kvh) + (int64_t)krow * vl.s_;
-    bf16x8 kf[HD / 16], vf[HD / 16];
+    const bf16* kp = k + kl.at(bi, kvh) + (int64_t)(RAGGED && krow >= s ? s - 1 : krow) * kl.s_;
+    const bf16* vp = v + vl.at(bi, kvh) + (int64_t)(RAGGED && krow >= s ? s - 1 : krow) * vl.s_;
+    bf16x8 kf[KK], vf[KK];
 #pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) {
+    for (int kk = 0; kk < KK; ++kk) {
       kf[kk] = ldg8(kp + kk * 16 + h * 8);
       vf[kk] = ldg8(vp + kk * 16 + h * 8);
     }
@@ -942,15 +1091,15 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
         sacc[e] = 0.f;
         dpacc[e] = 0.f;
       }
-      bf16x8 qfr[HD / 16], dofr[HD / 16];
+      bf16x8 qfr[KK], dofr[KK];
 #pragma unroll
-      for (int kk = 0; kk < HD / 16; ++kk) {
-        qfr[kk] = bt_rows(q_rows, sub, kk);
-        dofr[kk] = bt_rows(do_rows, sub, kk);
+      for (int kk = 0; kk < KK; ++kk) {
+        qfr[kk] = bt_rows<D>(q_rows, sub, kk);
+        dofr[kk] = bt_rows<D>(do_rows, sub, kk);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = 0; kk < HD / 16; ++kk) {
+      for (int kk = 0; kk < KK; ++kk) {
         sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfr[kk], kf[kk], sacc, 0, 0, 0);
         dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dofr[kk], vf[kk], dpacc, 0, 0, 0);
       }
@@ -968,11 +1117,11 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       uint32_t q_rows = lds0 + nstage * STAGE + bt_rows_lane(lane);
       uint32_t do_rows = q_rows + BT_BYTES;
       asm volatile("" : "+v"(q_rows), "+v"(do_rows));
-      bf16x8 qfr[HD / 16], dofr[HD / 16];
+      bf16x8 qfr[KK], dofr[KK];
 #pragma unroll
-      for (int kk = 0; kk < HD / 16; ++kk) {
-        qfr[kk] = bt_rows(q_rows, nsub, kk);
-        dofr[kk] = bt_rows(do_rows, nsub, kk);
+      for (int kk = 0; kk < KK; ++kk) {
+        qfr[kk] = bt_rows<D>(q_rows, nsub, kk);
+        dofr[kk] = bt_rows<D>(do_rows, nsub, kk);
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -995,9 +1144,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4 l4 = *reinterpret_cast<const f32x4*>(stats + sub * 32 + 8 * g + 4 * h);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(stats + 64 + sub * 32 + 8 * g + 4 * h);
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(stats + TQ + sub * 32 + 8 * g + 4 * h);
 #pragma unroll
-        for (int kk = 2 * g; kk < 2 * g + 2; ++kk) {
+        for (int kk = g * KK / 4; kk < (g + 1) * KK / 4; ++kk) {
           nsacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfr[kk], kf[kk], nsacc, 0, 0, 0);
           ndpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dofr[kk], vf[kk], ndpacc, 0, 0, 0);
         }
@@ -1010,7 +1159,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      const uint32_t xa = xch_lane + sub * 16384;
+      const uint32_t xa = xch_lane + (sub & 1) * 16384;
       *(KR_LDS bf16x8*)(xa) = pb[0];
       *(KR_LDS bf16x8*)(xa + 1024) = pb[1];
       *(KR_LDS bf16x8*)(xa + 2048) = dsb[0];
@@ -1025,12 +1174,16 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
     issue_scores(0, 0, s0, dp0);
     for (int it = 0, itl = 0; it < nit_all; ++it) {
       const int stage = it % NS;
-      const int q0 = (qt_first + itl * qsplit + part) * 64;
+      const int q0 = (qt_first + itl * qsplit + part) * TQ;
       itl = itl + 1 == niter ? 0 : itl + 1;  // the next head starts over at the diagonal
-      step(stage, 0, q0, s0, dp0, stage, 1, s1, dp1);
-      __syncthreads();  // hand-over of block 0
-      step(stage, 1, q0 + 32, s1, dp1, (it + 1) % NS, 0, s0, dp0);
-      __syncthreads();  // hand-over of block 1
+#pragma unroll
+      for (int sub = 0; sub < NSUB; sub += 2) {
+        step(stage, sub, q0 + 32 * sub, s0, dp0, stage, sub + 1, s1, dp1);
+        __syncthreads();  // hand-over of block `sub`
+        const bool more = sub + 2 < NSUB;
+        step(stage, sub + 1, q0 + 32 * sub + 32, s1, dp1, more ? stage : (it + 1) % NS, more ? sub + 2 : 0, s0, dp0);
+        __syncthreads();  // hand-over of block `sub` + 1
+      }
     }
     return;
   }
@@ -1038,9 +1191,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   // -------------------------------------------------------------------- accumulate waves
   const bf16* qb = q + ql.at(bi, head, per);
   const bf16* dob = dout + dol.at(bi, head, per);
-  const int64_t stat0 = ((int64_t)bi * nq + head) * s;
-  // A tile is brought in by nine requests per wave (eight for waves 2 and 3): the 64 + 64 row
-  // statistics, 4 bytes per lane, by waves 0 and 1, then four consecutive rows (+ 16, 32, 48
+  const int64_t stat0 = ((int64_t)bi * nq + head) * sp;
+  // A tile is brought in by nine requests per wave (with D = 128 eight for waves 2 and 3): the TQ + TQ row
+  // statistics, 4 bytes per lane, 64 of them per wave, then four consecutive rows (+ 16, 32, 48
   // through the lanes) of the Q tile and four of the dO tile.  request_begin names the tile,
   // request_piece(i) issues piece i = 0..8, in this order (requests retire in order).
   uint32_t req_tile = 0, req_lane_off = 0;
@@ -1048,32 +1201,41 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const bf16 *req_q = qb, *req_do = dob;
   int64_t req_stat = stat0;
   int req_qt = 0;
+  const bool has_stat = D == 64 || wave < 2;
   auto request_begin = [&](int it) {
     const int hh = it / niter, itl = it - hh * niter;  // head of the workgroup, query tile of that head
     req_qt = qt_first + itl * qsplit + part;
     req_tile = lds0 + (it % NS) * STAGE;
     req_q = qb + hh * ql.h_;    // consecutive heads of one KV group
     req_do = dob + hh * dol.h_;
-    req_stat = stat0 + (int64_t)hh * s;
+    req_stat = stat0 + (int64_t)hh * sp;
   };
   auto request_piece = [&](int i) {
     if (i == 0) {
-      if (wave < 2) {
+      if (has_stat) {
         int l2 = lane;
         asm volatile("" : "+v"(l2));
-        dma_b32((wave == 0 ? neg_lse2 : delta) + req_stat + req_qt * 64, (uint32_t)l2 * 4u,
+        // D = 128: one wave per statistic; D = 64: two, 64 rows each
+        const bool first = D == 128 ? wave == 0 : wave < 2;
+        const int row = D == 128 ? 0 : (wave & 1) * 64;
+        dma_b32((first ? neg_lse2 : delta) + req_stat + req_qt * TQ + row, (uint32_t)l2 * 4u,
                 req_tile + 2 * BT_BYTES + wave * 256);
       }
       return;
     }
     const int j = (i - 1) & 3;
     const bool second = i > 4;
+    if (RAGGED && (req_qt + 1) * TQ > s) {  // the tile the sequence ends in
+      request_clamped<D>(second ? req_do : req_q, second ? dol.s_ : ql.s_, req_qt * TQ, 4 * wave + j, s, lane,
+                         req_tile + (second ? BT_BYTES : 0) + (wave + 4 * j) * BT_BLK);
+      return;
+    }
     if (j == 0) {
       int l2 = lane;
       asm volatile("" : "+v"(l2));  // the lane offset lives only across the four requests of a tile
       const int64_t ss = second ? dol.s_ : ql.s_;
-      req_lane_off = (uint32_t)((l2 >> 4) * 16 * (int)ss + (l2 & 15) * 8) * 2u;
-      req_row = (second ? req_do : req_q) + ((int64_t)req_qt * 64 + 4 * wave) * ss;
+      req_lane_off = tile_lane_off<D>(l2, (int)ss);
+      req_row = (second ? req_do : req_q) + ((int64_t)req_qt * TQ + 4 * wave) * ss;
     }
     dma_b128(req_row, req_lane_off, req_tile + (second ? BT_BYTES : 0) + (wave + 4 * j) * BT_BLK);
     req_row += second ? dol.s_ : ql.s_;
@@ -1085,20 +1247,32 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   };
   // wait until at most the requests of one tile (the newest) are in flight
   auto wait_all_but_newest_tile = [&]() {
-    if (wave < 2)
+    if (has_stat)
       __builtin_amdgcn_s_waitcnt(0x0f79);  // vmcnt(9)
     else
       __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8)
   };
-  f32x16 dkacc[HD / 32], dvacc[HD / 32];
+  // zeros in the rows of iteration it's tile that lie beyond the sequence, once its requests have landed: their
+  // probabilities are zero (see kPadLse), and so must the factors be
+  auto zero_tail = [&](int it) {
+    if (RAGGED && it < nit_all) {
+      const int row0 = (qt_first + (it % niter) * qsplit + part) * TQ;
+      if (row0 + TQ > s) {
+        const uint32_t tile = lds0 + (it % NS) * STAGE;
+        bt_zero_tail<D>(row0, s, tile, wave, lane);
+        bt_zero_tail<D>(row0, s, tile + BT_BYTES, wave, lane);
+      }
+    }
+  };
+  f32x16 dkacc[DT], dvacc[DT];
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       dkacc[dt][e] = 0.f;
       dvacc[dt][e] = 0.f;
     }
-  request_tile(0);
+  if (D == 128 || nit_all > 0) request_tile(0);
   if (nit_all > 1) request_tile(1);
   if (nit_all > 2) {
     request_tile(2);
@@ -1106,8 +1280,10 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   } else {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   }
+  zero_tail(0);
+  zero_tail(1);
   __syncthreads();
-  // The sixteen transposed fragments of a block (fr[8 k2 + 2 dt]: dO^T, fr[8 k2 + 2 dt + 1]: Q^T,
+  // The transposed fragments of a block (fr[2 DT k2 + 2 dt]: dO^T, fr[2 DT k2 + 2 dt + 1]: Q^T,
   // queries 16 k2 .. of the block, channels 32 dt ..) live in registers across blocks: each is
   // refilled for the next block right behind the MFMA that consumed it (one MFMA later), so the
   // LDS reads of the next block ride under this block's matrix work and the wave reaches the
@@ -1115,65 +1291,66 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const uint32_t cols_lane = bt_cols_lane(lane);
   auto frag = [&](uint32_t stage_base, int sub, int f) {
     const uint32_t base = stage_base + ((f & 1) ? 0u : BT_BYTES);  // odd: Q tile, even: dO tile
-    return bt_cols(base, 2 * sub + (f >> 3), (f >> 1) & 3);
+    return bt_cols<D>(base, 2 * sub + f / (2 * DT), (f >> 1) % DT);
   };
-  bf16x8 fr[16];
+  bf16x8 fr[NF];
   {
     uint32_t base = lds0 + cols_lane;
     asm volatile("" : "+v"(base));
 #pragma unroll
-    for (int f = 0; f < 16; ++f) fr[f] = frag(base, 0, f);
+    for (int f = 0; f < NF; ++f) fr[f] = frag(base, 0, f);
   }
   settle_scalar_loads();
   for (int it = 0; it < nit_all; ++it) {
     const int stage = it % NS;
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
+    for (int sub = 0; sub < NSUB; ++sub) {
       // tile it+1 (requested an iteration and a half ago) must have landed before this
       // iteration's first barrier: the score waves start on it right after.  Tile it+2 may still
       // be on its way.
       if (sub == 0 && it > 0) {  // (tiles 0 and 1 were awaited before the loop)
         if (it + 2 < nit_all) {
           // in flight behind tile it+1: the first five pieces of tile it+2
-          if (wave < 2)
+          if (has_stat)
             __builtin_amdgcn_s_waitcnt(0x0f75);  // vmcnt(5)
           else
             __builtin_amdgcn_s_waitcnt(0x0f74);  // vmcnt(4)
         } else {
           __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         }
+        zero_tail(it + 1);
       }
       __syncthreads();
-      // After the second barrier nobody reads tile it any more (this wave fetched its last
-      // fragments of it during the first block, the score waves before the first barrier):
+      // After the last barrier nobody reads tile it any more (this wave fetched its last
+      // fragments of it during the block before, the score waves before the barrier in front of this):
       // tile it+3 goes into its stage, one request behind each of the first MFMAs — pieces 0-4
       // in this block, pieces 5-8 in the first block of the next iteration, so that neither
       // block of the accumulate waves outlasts the score waves' step beside it.
-      const bool first_pieces = sub == 1 && it + 3 < nit_all;
+      const bool first_pieces = sub == NSUB - 1 && it + 3 < nit_all;
       const bool last_pieces = sub == 0 && it > 0 && it + 2 < nit_all;
       if (first_pieces) request_begin(it + 3);
-      const uint32_t xa = xch_lane + sub * 16384;
+      const uint32_t xa = xch_lane + (sub & 1) * 16384;
       bf16x8 hand[4];  // P (queries 0-15, 16-31 of the block), dS (the same)
 #pragma unroll
       for (int c = 0; c < 4; ++c) hand[c] = *(KR_LDS const bf16x8*)(xa + c * 1024);
-      // next block: the second of this tile, or the first of the next tile (complete since this
+      // next block: the next of this tile, or the first of the next tile (complete since this
       // iteration's first barrier; behind the last tile a stale stage, unused)
-      uint32_t next_base = lds0 + (sub == 0 ? stage : (it + 1) % NS) * STAGE + cols_lane;
+      uint32_t next_base = lds0 + (sub < NSUB - 1 ? stage : (it + 1) % NS) * STAGE + cols_lane;
       asm volatile("" : "+v"(next_base));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int f = 0; f < 16; ++f) {
-        const int dt = (f >> 1) & 3;
+      for (int f = 0; f < NF; ++f) {
+        const int dt = (f >> 1) % DT;
         if (f & 1)
-          dkacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], hand[2 + (f >> 3)], dkacc[dt], 0, 0, 0);
+          dkacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], hand[2 + f / (2 * DT)], dkacc[dt], 0, 0, 0);
         else
-          dvacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], hand[f >> 3], dvacc[dt], 0, 0, 0);
-        if (f > 0) fr[f - 1] = frag(next_base, sub ^ 1, f - 1);
+          dvacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], hand[f / (2 * DT)], dvacc[dt], 0, 0, 0);
+        if (f > 0) fr[f - 1] = frag(next_base, (sub + 1) % NSUB, f - 1);
         if (first_pieces && f < 5) request_piece(f);
         if (last_pieces && f < 4) request_piece(5 + f);
         __builtin_amdgcn_sched_barrier(0);
       }
-      fr[15] = frag(next_base, sub ^ 1, 15);
+      fr[NF - 1] = frag(next_base, (sub + 1) % NSUB, NF - 1);
     }
   }
 
@@ -1182,32 +1359,34 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   RowStage rs;
   rs.init(reinterpret_cast<char*>(smem) + XCH + wave * 4096, lane);
   if (PARTIAL) {
-    const int64_t prow = (((int64_t)bi * nhg + hgroup) * qsplit + part) * s + kw0;
-    store_rows_f32(rs, dkacc, scale, part_k + prow * HD, HD);
-    store_rows_f32(rs, dvacc, 1.0f, part_v + prow * HD, HD);
+    const int64_t prow = (((int64_t)bi * nhg + hgroup) * qsplit + part) * sp + kw0;
+    store_rows_f32<D>(rs, dkacc, scale, part_k + prow * D, D);
+    store_rows_f32<D>(rs, dvacc, 1.0f, part_v + prow * D, D);
   } else {
-    store_rows_bf16(rs, dkacc, scale, dk + dkl.at(bi, kvh) + (int64_t)kw0 * dkl.s_, dkl.s_);
-    store_rows_bf16(rs, dvacc, 1.0f, dv + dvl.at(bi, kvh) + (int64_t)kw0 * dvl.s_, dvl.s_);
+    store_rows_bf16<D, RAGGED>(rs, dkacc, scale, dk + dkl.at(bi, kvh) + (int64_t)kw0 * dkl.s_, dkl.s_, s - kw0);
+    store_rows_bf16<D, RAGGED>(rs, dvacc, 1.0f, dv + dvl.at(bi, kvh) + (int64_t)kw0 * dvl.s_, dvl.s_, s - kw0);
   }
 }
 
 // dk/dv[b, kvh, i, :] = sum over the group's query heads of the fp32 partials; one thread per
 // 8 channels (two 16-byte reads per partial, one 16-byte bf16 store).
+template <int D>
 __global__ __launch_bounds__(256) void attn_group_reduce_kernel(
     const float* __restrict__ part_k, const float* __restrict__ part_v, bf16* __restrict__ dk,
-    bf16* __restrict__ dv, int s, int nslots, int nkv, int qsplit, int64_t total, KLayout dkl, KLayout dvl) {
+    bf16* __restrict__ dv, int s, int sp, int nslots, int nkv, int qsplit, int64_t total, KLayout dkl, KLayout dvl) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (bi, kvh, si, chunk of 8)
   if (idx >= total) return;
-  const int c = (int)(idx & 15);
-  const int si = (int)((idx >> 4) % s);
-  const int kvh = (int)((idx >> 4) / s % nkv);
-  const int bi = (int)((idx >> 4) / ((int64_t)s * nkv));
+  constexpr int VEC = D / 8;
+  const int c = (int)(idx % VEC);
+  const int si = (int)((idx / VEC) % s);
+  const int kvh = (int)((idx / VEC) / s % nkv);
+  const int bi = (int)((idx / VEC) / ((int64_t)s * nkv));
   const int per = nslots / nkv;  // partial results per KV head: one per workgroup that served the group
   float ak[8], av[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) ak[e] = av[e] = 0.f;
   for (int j = 0; j < per * qsplit; ++j) {  // (heads' workgroup, query-tile part) pairs are consecutive
-    const int64_t off = (((((int64_t)bi * nslots + kvh * per) * qsplit + j) * s) + si) * HD + c * 8;
+    const int64_t off = (((((int64_t)bi * nslots + kvh * per) * qsplit + j) * sp) + si) * D + c * 8;
     const f32x4 k0 = *reinterpret_cast<const f32x4*>(part_k + off);
     const f32x4 k1 = *reinterpret_cast<const f32x4*>(part_k + off + 4);
     const f32x4 v0 = *reinterpret_cast<const f32x4*>(part_v + off);
@@ -1235,7 +1414,7 @@ __global__ __launch_bounds__(256) void attn_group_reduce_kernel(
 // LDS at the end.  Chosen by the host when there are few workgroups.
 // When there is a 256-query tile for every compute unit (or other streams run beside the launch)
 // the host takes attn_bwd_dq_w64_kernel below instead.
-template <int HALVES>
+template <int D, bool RAGGED, int HALVES>
 __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta,
@@ -1243,12 +1422,14 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
     KLayout kl, KLayout vl, QLayout dol, QLayout dql) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
   constexpr uint32_t STAGE = 2 * BT_BYTES;  // K tile | V tile (blocked tiles), bytes
+  constexpr int TK = tile_rows<D>, NB = TK / 32, DT = D / 32, KK = D / 16;
 
   const int half = HALVES == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
   const int tid = threadIdx.x & 255, lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int ROWS = BQ;  // queries per workgroup
-  const int nqt = s / ROWS;
+  const int sp = RAGGED ? (s + 127) / 128 * 128 : s;
+  const int nqt = sp / ROWS;
   const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
   const int qt = nqt - 1 - (lid % nqt);
   const int pair = lid / nqt;
@@ -1259,40 +1440,55 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
   const int q0 = qt * ROWS;
   const int qw0 = q0 + wave * 32;
   const int qrow = qw0 + (lane & 31);
+  const int qld = RAGGED && qrow >= s ? s - 1 : qrow;  // the row to load (rows beyond s are not stored)
 
-  const bf16* qp = q + ql.at(bi, head, per) + (int64_t)qrow * ql.s_;
-  const bf16* dop = dout + dol.at(bi, head, per) + (int64_t)qrow * dol.s_;
+  const bf16* qp = q + ql.at(bi, head, per) + (int64_t)qld * ql.s_;
+  const bf16* dop = dout + dol.at(bi, head, per) + (int64_t)qld * dol.s_;
   const bf16* kb = k + kl.at(bi, kvh);
   const bf16* vb = v + vl.at(bi, kvh);
-  bf16x8 qf[HD / 16], dof[HD / 16];
+  bf16x8 qf[KK], dof[KK];
 #pragma unroll
-  for (int kk = 0; kk < HD / 16; ++kk) {
+  for (int kk = 0; kk < KK; ++kk) {
     qf[kk] = ldg8(qp + kk * 16 + h * 8);
     dof[kk] = ldg8(dop + kk * 16 + h * 8);
   }
-  const int64_t stat = ((int64_t)bi * nq + head) * s + qrow;
-  const float neg_lse = -lse[stat] * kLog2e;
-  const float my_delta = delta[stat];
+  const int64_t stat = (int64_t)bi * nq + head;
+  const float neg_lse = -lse[stat * s + qld] * kLog2e;
+  const float my_delta = delta[stat * sp + qld];
 
-  f32x16 dqacc[HD / 32];
+  f32x16 dqacc[DT];
 #pragma unroll
-  for (int dt = 0; dt < HD / 32; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) dqacc[dt][e] = 0.f;
 
-  // key tiles per half (the tile count is even), or all tiles up to the workgroup's last row
-  const int ntiles = (q0 + BQ) / (HALVES * BKV);
-  auto key_of = [&](int j) { return (HALVES * j + half) * BKV; };
+  // key tiles per half, up to the workgroup's last row (with 128-key tiles half 1 may have one less: its
+  // last step then neither requests nor computes)
+  const int ntiles = ((q0 + BQ) / TK + HALVES - 1) / HALVES;
+  auto key_of = [&](int j) { return (HALVES * j + half) * TK; };
   // K and V tiles go straight from global memory into two LDS stages: this half's own, or with
   // shared tiles the workgroup's, half 0 bringing in the K tile and half 1 the V tile
   const uint32_t area = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem + half * 2 * STAGE;
   auto stage_request = [&](int j, int buf) {
     const int key0 = key_of(j);
-    bt_request(kb + (int64_t)key0 * kl.s_, kl.s_, area + buf * STAGE, wave, lane);
-    bt_request(vb + (int64_t)key0 * vl.s_, vl.s_, area + buf * STAGE + BT_BYTES, wave, lane);
+    if (D == 64 && HALVES == 2 && key0 >= q0 + BQ) return;
+    if (RAGGED && key0 + TK > s) {
+      bt_request_clamped<D>(kb, kl.s_, key0, s, area + buf * STAGE, wave, lane);
+      bt_request_clamped<D>(vb, vl.s_, key0, s, area + buf * STAGE + BT_BYTES, wave, lane);
+      return;
+    }
+    bt_request<D>(kb + (int64_t)key0 * kl.s_, kl.s_, area + buf * STAGE, wave, lane);
+    bt_request<D>(vb + (int64_t)key0 * vl.s_, vl.s_, area + buf * STAGE + BT_BYTES, wave, lane);
+  };
+  auto zero_tail = [&](int j, int buf) {  // rows of tile j beyond the sequence, once it has landed
+    if (RAGGED && key_of(j) + TK > s) {
+      bt_zero_tail<D>(key_of(j), s, area + buf * STAGE, wave, lane);
+      bt_zero_tail<D>(key_of(j), s, area + buf * STAGE + BT_BYTES, wave, lane);
+    }
   };
   stage_request(0, 0);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  zero_tail(0, 0);
   __syncthreads();
 
   settle_scalar_loads();
@@ -1306,9 +1502,10 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
       uint32_t v_rows = k_rows + BT_BYTES;
       uint32_t k_cols = area + cur * STAGE + bt_cols_lane(lane);
       asm volatile("" : "+v"(k_rows), "+v"(v_rows), "+v"(k_cols));
-      const bool need_mask = key0 + BKV - 1 > qw0;  // wave-uniform: the tile on the diagonal
+      const bool need_mask = key0 + TK - 1 > qw0;  // wave-uniform: the tile on the diagonal
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < NB; ++t) {
+        if (D == 64 && key0 + 32 * t > qw0 + 31) continue;  // wave-uniform: beyond the diagonal
         f32x16 sacc, dpacc;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -1316,9 +1513,9 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
           dpacc[e] = 0.f;
         }
 #pragma unroll
-        for (int kk = 0; kk < HD / 16; ++kk) {
-          sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt_rows(k_rows, t, kk), qf[kk], sacc, 0, 0, 0);
-          dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt_rows(v_rows, t, kk), dof[kk], dpacc, 0, 0, 0);
+        for (int kk = 0; kk < KK; ++kk) {
+          sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt_rows<D>(k_rows, t, kk), qf[kk], sacc, 0, 0, 0);
+          dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt_rows<D>(v_rows, t, kk), dof[kk], dpacc, 0, 0, 0);
         }
         // lane: query row qrow, keys key0 + 32t + 8g + 4h + e
         bf16x8 dsb[2];
@@ -1342,13 +1539,14 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
 #pragma unroll
         for (int k2 = 0; k2 < 2; ++k2)
 #pragma unroll
-          for (int dt = 0; dt < HD / 32; ++dt) {
-            dqacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt_cols(k_cols, 2 * t + k2, dt), dsb[k2],
+          for (int dt = 0; dt < DT; ++dt) {
+            dqacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bt_cols<D>(k_cols, 2 * t + k2, dt), dsb[k2],
                                                                 dqacc[dt], 0, 0, 0);
           }
       }
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's share of the next tiles has landed
+    if (RAGGED && j + 1 < ntiles) zero_tail(j + 1, cur ^ 1);
     __syncthreads();
   }
 
@@ -1357,14 +1555,14 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
     const int slot = wave * 64 + lane;
     if (half == 1) {
 #pragma unroll
-      for (int dt = 0; dt < HD / 32; ++dt)
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) xch[(dt * 16 + e) * 256 + slot] = dqacc[dt][e];
     }
     __syncthreads();
     if (half == 1) return;
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int e = 0; e < 16; ++e) dqacc[dt][e] += xch[(dt * 16 + e) * 256 + slot];
   }
@@ -1372,7 +1570,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
   // output transposition through LDS (behind the 64 KiB hand-over buffer when there are two halves)
   RowStage rs;
   rs.init(reinterpret_cast<char*>(smem) + (HALVES == 2 ? 64 * 1024 : 0) + wave * 4096, lane);
-  store_rows_bf16(rs, dqacc, scale, dq + dql.at(bi, head, per) + (int64_t)qw0 * dql.s_, dql.s_);
+  store_rows_bf16<D, RAGGED>(rs, dqacc, scale, dq + dql.at(bi, head, per) + (int64_t)qw0 * dql.s_, dql.s_, s - qw0);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1431,8 +1629,9 @@ __device__ __forceinline__ void mfma_from_vv(f32x16& c, bf16x8 a, bf16x8 b, cons
 // MFMA m (0..3) of contraction step kk: S^T of block 0, block 1, dP^T of block 0, block 1.  dP^T
 // starts from -delta of the lane's row (sixteen copies per block, set up once), which takes the
 // subtraction out of every score's vector work.
+template <int KK>
 __device__ __forceinline__ void dq_score_mfma(DqScores& x, int kk, int m, bf16x8 kf, bf16x8 vf,
-                                              const bf16x8 (&qf)[2][HD / 16], const bf16x8 (&dof)[2][HD / 16],
+                                              const bf16x8 (&qf)[2][KK], const bf16x8 (&dof)[2][KK],
                                               const f32x16 (&neg_delta)[2]) {
   if (kk == 0) {
     if (m == 0) mfma_set_v(x.s[0], kf, qf[0][kk]);
@@ -1450,12 +1649,13 @@ __device__ __forceinline__ void dq_score_mfma(DqScores& x, int kk, int m, bf16x8
 // One step (32 keys).  NEXT: issue the score MFMAs of the following 32 keys (fragments of sub-tile nt
 // at nk_rows / nv_rows) into `nxt`.  MASK: the step is on the causal diagonal; lim[qb] is the last
 // visible key of the lane's row, relative to the lane's first key of the step.
-template <bool NEXT, bool MASK>
-__device__ __forceinline__ void dq_step(DqScores& nxt, const DqScores& cur, f32x16 (&dq)[2][HD / 32],
+template <int D, bool NEXT, bool MASK>
+__device__ __forceinline__ void dq_step(DqScores& nxt, const DqScores& cur, f32x16 (&dq)[2][D / 32],
                                         uint32_t nk_rows, uint32_t nv_rows, int nt, uint32_t k_cols, int t,
-                                        const bf16x8 (&qf)[2][HD / 16], const bf16x8 (&dof)[2][HD / 16],
+                                        const bf16x8 (&qf)[2][D / 16], const bf16x8 (&dof)[2][D / 16],
                                         float scale_log2, const float (&neg_lse)[2],
                                         const f32x16 (&neg_delta)[2], const int (&lim)[2]) {
+  constexpr int KK = D / 16, DT = D / 32;
   bf16x8 dsb[2][2];
   auto one_score = [&](int g) {  // lane: query row of block g / 16, key 8 (e / 4) + e % 4 (+ 4 h) of the step
     const int qb = g >> 4, e = g & 15;
@@ -1467,24 +1667,25 @@ __device__ __forceinline__ void dq_step(DqScores& nxt, const DqScores& cur, f32x
   // Fragments are requested from LDS well ahead of the MFMA that takes them (two contraction steps
   // = eight MFMAs for the score products, three fragments = six MFMAs for dQ): one wave per SIMD has
   // nobody to cover an LDS round trip for it.
-  constexpr int NKT = 2 * (HD / 32);  // K^T fragments of the step: 2 contraction steps x 4 channel blocks
-  auto kt_frag = [&](int i) { return bt_cols(k_cols, 2 * t + i / (HD / 32), i % (HD / 32)); };
+  constexpr int NKT = 2 * (DT);  // K^T fragments of the step: 2 contraction steps x D / 32 channel blocks
+  auto kt_frag = [&](int i) { return bt_cols<D>(k_cols, 2 * t + i / (DT), i % (DT)); };
   bf16x8 kt[3];
   if (NEXT) {
     bf16x8 kf[3], vf[3];
-    kf[0] = bt_rows(nk_rows, nt, 0);
-    vf[0] = bt_rows(nv_rows, nt, 0);
-    kf[1] = bt_rows(nk_rows, nt, 1);
-    vf[1] = bt_rows(nv_rows, nt, 1);
+    kf[0] = bt_rows<D>(nk_rows, nt, 0);
+    vf[0] = bt_rows<D>(nv_rows, nt, 0);
+    kf[1] = bt_rows<D>(nk_rows, nt, 1);
+    vf[1] = bt_rows<D>(nv_rows, nt, 1);
 #pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) {
+    for (int kk = 0; kk < KK; ++kk) {
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        if (m == 0 && kk + 2 < HD / 16) kf[(kk + 2) % 3] = bt_rows(nk_rows, nt, kk + 2);
-        if (m == 2 && kk + 2 < HD / 16) vf[(kk + 2) % 3] = bt_rows(nv_rows, nt, kk + 2);
-        if (m == 1 && kk >= HD / 16 - 3) kt[kk - (HD / 16 - 3)] = kt_frag(kk - (HD / 16 - 3));
-        dq_score_mfma(nxt, kk, m, kf[kk % 3], vf[kk % 3], qf, dof, neg_delta);
-        one_score(kk * 4 + m);
+        if (m == 0 && kk + 2 < KK) kf[(kk + 2) % 3] = bt_rows<D>(nk_rows, nt, kk + 2);
+        if (m == 2 && kk + 2 < KK) vf[(kk + 2) % 3] = bt_rows<D>(nv_rows, nt, kk + 2);
+        if (m == 1 && kk >= KK - 3) kt[kk - (KK - 3)] = kt_frag(kk - (KK - 3));
+        dq_score_mfma<KK>(nxt, kk, m, kf[kk % 3], vf[kk % 3], qf, dof, neg_delta);
+#pragma unroll
+        for (int c = 0; c < 8 / KK; ++c) one_score((kk * 4 + m) * (8 / KK) + c);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -1498,7 +1699,7 @@ __device__ __forceinline__ void dq_step(DqScores& nxt, const DqScores& cur, f32x
   }
 #pragma unroll
   for (int i = 0; i < NKT; ++i) {
-    const int k2 = i / (HD / 32), dt = i % (HD / 32);
+    const int k2 = i / (DT), dt = i % (DT);
     const bf16x8 frag = kt[i % 3];
     dq[0][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag, dsb[0][k2], dq[0][dt], 0, 0, 0);
     dq[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag, dsb[1][k2], dq[1][dt], 0, 0, 0);
@@ -1510,6 +1711,7 @@ __device__ __forceinline__ void dq_step(DqScores& nxt, const DqScores& cur, f32x
 // The kernel also takes over the pre-pass of the backward: each wave forms delta = sum_d dO . O of its 64
 // rows from the dO fragments it holds anyway, uses it, and writes it (and -lse in the log2 domain) for
 // the dK/dV kernel, which the host launches behind this one.
+template <int D, bool RAGGED>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const bf16* __restrict__ o, const float* __restrict__ lse,
@@ -1517,13 +1719,15 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
     int nkv, float scale, float scale_log2, QLayout ql, KLayout kl, KLayout vl, QLayout dol, QLayout ol,
     QLayout dql) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  constexpr int TK = tile_rows<D>, NSUB = TK / 32, DT = D / 32, KK = D / 16;
   constexpr uint32_t STAGE = 2 * BT_BYTES;  // K tile | V tile
   constexpr int ROWS = 256;                 // queries per workgroup: 64 per wave
   constexpr int NSTAGE = 3;                 // tiles in LDS: the one in use, the next, the one after
 
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nqt = s / ROWS;
+  const int sp = RAGGED ? (s + 127) / 128 * 128 : s;  // rows of the statistics (whole 256-query tiles here)
+  const int nqt = sp / ROWS;
   const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
   int qt, pair;
   longest_first(lid, nqt, gridDim.x / nqt, qt, pair);
@@ -1536,16 +1740,17 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
 
   const bf16* kb = k + kl.at(bi, kvh);
   const bf16* vb = v + vl.at(bi, kvh);
-  bf16x8 qf[2][HD / 16], dof[2][HD / 16];
+  bf16x8 qf[2][KK], dof[2][KK];
   float neg_lse[2];
   f32x16 neg_delta[2];
   int lim[2];
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     const int qrow = qw0 + 32 * qb + (lane & 31);
-    const bf16* qp = q + ql.at(bi, head, per) + (int64_t)qrow * ql.s_;
-    const bf16* dop = dout + dol.at(bi, head, per) + (int64_t)qrow * dol.s_;
-    const bf16* op = o + ol.at(bi, head, per) + (int64_t)qrow * ol.s_;
+    const int qld = RAGGED && qrow >= s ? s - 1 : qrow;  // the row to load
+    const bf16* qp = q + ql.at(bi, head, per) + (int64_t)qld * ql.s_;
+    const bf16* dop = dout + dol.at(bi, head, per) + (int64_t)qld * dol.s_;
+    const bf16* op = o + ol.at(bi, head, per) + (int64_t)qld * ol.s_;
     // delta from a second read of the dO row: the fragments kept for the MFMAs must stay values that
     // only the MFMAs read, or the compiler keeps them in VGPRs and copies them into accumulation
     // registers in front of every MFMA
@@ -1553,7 +1758,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
     asm volatile("" : "+v"(dop2));
     float dsum = 0.f;  // this lane's half of the row (channels 16 kk + 8 h ..)
 #pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) {
+    for (int kk = 0; kk < KK; ++kk) {
       qf[qb][kk] = ldg8(qp + kk * 16 + h * 8);
       dof[qb][kk] = ldg8(dop + kk * 16 + h * 8);
       const bf16x8 dov = ldg8(dop2 + kk * 16 + h * 8), of = ldg8(op + kk * 16 + h * 8);
@@ -1561,8 +1766,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
       for (int e = 0; e < 8; ++e) dsum += (float)dov[e] * (float)of[e];
     }
     dsum += __shfl_xor(dsum, 32, KR_WAVE);
-    const int64_t stat = ((int64_t)bi * nq + head) * s + qrow;
-    neg_lse[qb] = -lse[stat] * kLog2e;
+    const int64_t stat = ((int64_t)bi * nq + head) * sp + qrow;
+    neg_lse[qb] = -lse[((int64_t)bi * nq + head) * s + qld] * kLog2e;
+    if (RAGGED && qrow >= s) {  // rows the dK/dV kernel must not see
+      dsum = 0.f;
+      neg_lse[qb] = -kPadLse * kLog2e;
+    }
     if (h == 0) {
       delta_out[stat] = dsum;
       neg_lse2_out[stat] = neg_lse[qb];
@@ -1571,24 +1780,36 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
     for (int e = 0; e < 16; ++e) neg_delta[qb][e] = -dsum;
   }
 
-  f32x16 dqacc[2][HD / 32];
+  f32x16 dqacc[2][DT];
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int e = 0; e < 16; ++e) dqacc[qb][dt][e] = 0.f;
 
-  const int ntiles = (q0 + ROWS) / BKV;                             // key tiles of the workgroup
-  const int last = __builtin_amdgcn_readfirstlane(qw0 / BKV);       // this wave's tile on the diagonal
+  const int ntiles = (q0 + ROWS) / TK;                              // key tiles of the workgroup
+  const int last = __builtin_amdgcn_readfirstlane(qw0 / TK);        // this wave's tile on the diagonal
   const uint32_t area = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem;
   auto stage_request = [&](int j, int buf) {  // the four waves bring in the K and the V tile together
-    bt_request(kb + (int64_t)(j * BKV) * kl.s_, kl.s_, area + buf * STAGE, wave, lane);
-    bt_request(vb + (int64_t)(j * BKV) * vl.s_, vl.s_, area + buf * STAGE + BT_BYTES, wave, lane);
+    if (RAGGED && (j + 1) * TK > s) {
+      bt_request_clamped<D>(kb, kl.s_, j * TK, s, area + buf * STAGE, wave, lane);
+      bt_request_clamped<D>(vb, vl.s_, j * TK, s, area + buf * STAGE + BT_BYTES, wave, lane);
+      return;
+    }
+    bt_request<D>(kb + (int64_t)(j * TK) * kl.s_, kl.s_, area + buf * STAGE, wave, lane);
+    bt_request<D>(vb + (int64_t)(j * TK) * vl.s_, vl.s_, area + buf * STAGE + BT_BYTES, wave, lane);
+  };
+  auto zero_tail = [&](int j, int buf) {  // rows of tile j beyond the sequence, once it has landed
+    if (RAGGED && (j + 1) * TK > s) {
+      bt_zero_tail<D>(j * TK, s, area + buf * STAGE, wave, lane);
+      bt_zero_tail<D>(j * TK, s, area + buf * STAGE + BT_BYTES, wave, lane);
+    }
   };
   stage_request(0, 0);
-  stage_request(1, 1);  // ntiles >= 4
+  stage_request(1, 1);  // ntiles >= 2
   __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): everything but the second tile's requests has landed
+  zero_tail(0, 0);
   __syncthreads();
   settle_scalar_loads();
 
@@ -1597,10 +1818,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
   {  // scores of the first 32 keys (tile 0 is below every wave's diagonal or on it)
     const uint32_t k_rows = area + rows_lane, v_rows = k_rows + BT_BYTES;
 #pragma unroll
-    for (int kk = 0; kk < HD / 16; ++kk) {
-      const bf16x8 kf = bt_rows(k_rows, 0, kk), vf = bt_rows(v_rows, 0, kk);
+    for (int kk = 0; kk < KK; ++kk) {
+      const bf16x8 kf = bt_rows<D>(k_rows, 0, kk), vf = bt_rows<D>(v_rows, 0, kk);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) dq_score_mfma(a, kk, m, kf, vf, qf, dof, neg_delta);
+      for (int m = 0; m < 4; ++m) dq_score_mfma<KK>(a, kk, m, kf, vf, qf, dof, neg_delta);
     }
     // the scores pass through the wait: no reader can be moved in front of it
     asm volatile("s_nop 15\n\ts_nop 15" : "+v"(a.s[0]), "+v"(a.s[1]), "+v"(a.dp[0]), "+v"(a.dp[1]));
@@ -1612,6 +1833,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
   int buf = 0;  // stage of tile j
   auto arrive = [&](int j) {  // between the two steps of tile j
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's share of tile j + 1 has landed
+    if (RAGGED && j + 1 < ntiles) zero_tail(j + 1, buf == NSTAGE - 1 ? 0 : buf + 1);
     __syncthreads();                     // ... and everyone's; nobody reads tile j - 1 any more
   };
   auto turn = [&](int j) {
@@ -1626,23 +1848,42 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
     uint32_t k_cols = area + buf * STAGE + cols_lane;
     uint32_t nk_rows = area + buf_next * STAGE + rows_lane, nv_rows = nk_rows + BT_BYTES;
     asm volatile("" : "+v"(k_rows), "+v"(v_rows), "+v"(k_cols), "+v"(nk_rows), "+v"(nv_rows));
-    dq_step<true, false>(b, a, dqacc, k_rows, v_rows, 1, k_cols, 0, qf, dof, scale_log2, neg_lse, neg_delta, lim);
-    turn(j);
-    dq_step<true, false>(a, b, dqacc, nk_rows, nv_rows, 0, k_cols, 1, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+#pragma unroll
+    for (int t = 0; t < NSUB; t += 2) {
+      dq_step<D, true, false>(b, a, dqacc, k_rows, v_rows, t + 1, k_cols, t, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+      if (t + 2 < NSUB) {
+        dq_step<D, true, false>(a, b, dqacc, k_rows, v_rows, t + 2, k_cols, t + 1, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+      } else {
+        turn(j);
+        dq_step<D, true, false>(a, b, dqacc, nk_rows, nv_rows, 0, k_cols, t + 1, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+      }
+    }
     buf = buf_next;
   }
-  {  // the diagonal tile (keys qw0 .. qw0 + 63): lim = last visible key of the lane's row, counted
-     // from the lane's first key of the step
+  {  // the tile on the diagonal: lim = last visible key of the lane's row, counted from the lane's first
+     // key of the step (D = 64: the wave's 64 rows meet one half of the 128 keys; steps beyond the
+     // diagonal are masked rather than branched around)
     uint32_t k_rows = area + buf * STAGE + rows_lane, v_rows = k_rows + BT_BYTES;
     uint32_t k_cols = area + buf * STAGE + cols_lane;
     asm volatile("" : "+v"(k_rows), "+v"(v_rows), "+v"(k_cols));
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) lim[qb] = 32 * qb + (lane & 31) - 4 * h;
-    dq_step<true, true>(b, a, dqacc, k_rows, v_rows, 1, k_cols, 0, qf, dof, scale_log2, neg_lse, neg_delta, lim);
-    turn(last);
+    for (int qb = 0; qb < 2; ++qb) lim[qb] = 32 * qb + (lane & 31) - 4 * h + (D == 64 ? qw0 - last * TK : 0);
+    auto next_keys = [&]() {
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) lim[qb] -= 32;
-    dq_step<false, true>(a, b, dqacc, 0, 0, 0, k_cols, 1, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+      for (int qb = 0; qb < 2; ++qb) lim[qb] -= 32;
+    };
+#pragma unroll
+    for (int t = 0; t < NSUB; t += 2) {
+      dq_step<D, true, true>(b, a, dqacc, k_rows, v_rows, t + 1, k_cols, t, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+      next_keys();
+      if (t + 2 < NSUB) {
+        dq_step<D, true, true>(a, b, dqacc, k_rows, v_rows, t + 2, k_cols, t + 1, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+        next_keys();
+      } else {
+        turn(last);
+        dq_step<D, false, true>(a, b, dqacc, 0, 0, 0, k_cols, t + 1, qf, dof, scale_log2, neg_lse, neg_delta, lim);
+      }
+    }
     buf = buf == NSTAGE - 1 ? 0 : buf + 1;
   }
   for (int j = last + 1; j < ntiles; ++j) {
@@ -1654,31 +1895,15 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
   rs.init(reinterpret_cast<char*>(smem) + NSTAGE * STAGE + wave * 4096, lane);
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb)
-    store_rows_bf16(rs, dqacc[qb], scale, dq + dql.at(bi, head, per) + (int64_t)(qw0 + 32 * qb) * dql.s_, dql.s_);
+    store_rows_bf16<D, RAGGED>(rs, dqacc[qb], scale, dq + dql.at(bi, head, per) + (int64_t)(qw0 + 32 * qb) * dql.s_,
+                               dql.s_, s - (qw0 + 32 * qb));
 }
-
-#define KR_ATTN_DQ_ARGS                                                                          \
-  const bf16*, const bf16*, const bf16*, const bf16*, const float*, const float*, bf16*, int, int, \
-      int, float, float, QLayout, KLayout, KLayout, QLayout, QLayout
-template __global__ void attn_bwd_dq_kernel<1>(KR_ATTN_DQ_ARGS);
-template __global__ void attn_bwd_dq_kernel<2>(KR_ATTN_DQ_ARGS);
-#undef KR_ATTN_DQ_ARGS
-
-#define KR_ATTN_DKDV_ARGS                                                                          \
-  const bf16*, const bf16*, const bf16*, const bf16*, const float*, const float*, bf16*, bf16*, \
-      float*, float*, int, int, int, int, int, float, float, QLayout, KLayout, KLayout, QLayout,      \
-      KLayout, KLayout
-template __global__ void attn_bwd_dkdv_kernel<false>(KR_ATTN_DKDV_ARGS);
-template __global__ void attn_bwd_dkdv_kernel<true>(KR_ATTN_DKDV_ARGS);
-#undef KR_ATTN_DKDV_ARGS
-
 
 // =============================================================================================
 // General path: any sequence length, head dimensions that are a multiple of 8 up to 128.
-// The kernels above are built for head dimension 128 and sequences of whole 128-row tiles, the
-// shapes of the training workloads.  Everything else (head dimension 64, ragged lengths; the
-// reference's flash-attention call takes both) runs through these plain fp32 kernels: same
-// interface, same tensor layouts, same results to rounding, no MFMA — they exist so that such a
+// The kernels above are built for head dimensions 128 and 64.  With KR_ATTN_GENERAL_KERNELS, or where
+// there is neither an instance nor a workspace to pad into, a shape runs through these plain fp32 kernels:
+// same interface, same tensor layouts, same results to rounding, no MFMA — they exist so that such a
 // shape is computed on the device at all, not to be fast.  A workgroup of 256 threads owns 32
 // query rows (forward, dQ) or 32 keys (dK/dV) and walks 32-row tiles of the other operand through
 // LDS; a thread is (row r = tid / 8, part p = tid % 8): it computes the scores of row r against
@@ -1936,7 +2161,7 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_dq_kernel(
 }  // namespace general
 
 // ---- shapes outside the MFMA kernels, padded into them -----------------------------------------
-// Head dimensions below 128 and sequence lengths that are not whole 128-row tiles are copied into
+// Head dimensions other than 128 and 64 (and strides that attn_in_place refuses) are copied into
 // dense [s_pad, b, heads, 128] buffers (zeros beyond the data), run through the MFMA kernels and
 // copied back.  Zero channels add nothing to Q.K^T and give zero output channels; with the causal
 // mask a query row below s never sees a key row at or beyond s, and the rows at or beyond s are
@@ -2066,7 +2291,7 @@ struct AttnForms {
   bool shared_fwd, shared_dq;
   int qsplit;
 };
-static AttnForms attn_forms(int s, int b, int nq, int flags) {
+static AttnForms attn_forms(int s, int b, int nq, int flags) {  // s: rounded up to whole 128-row tiles
   const bool beside = (flags & KR_ATTN_BESIDE_OTHER_STREAMS) != 0;
   const int tiles256 = (s / 256) * nq * b;
   AttnForms f;
@@ -2075,6 +2300,122 @@ static AttnForms attn_forms(int s, int b, int nq, int flags) {
   f.qsplit = beside ? 1 : dkdv_query_split(s, b, nq);
   return f;
 }
+
+namespace {
+struct BwdCall {
+  const bf16 *dout, *q, *k, *v, *o;
+  const float* lse;
+  bf16 *dq, *dk, *dv;
+  float* workspace;
+  int s, b, nq, nkv;
+  float scale;
+  QLayout ql, ol, dol, dql;
+  KLayout kl, vl, dkl, dvl;
+  int flags;
+  hipStream_t st;
+};
+
+// The MFMA backward on tensors as they lie.  The forms are chosen by the length rounded up to whole 128-row
+// tiles: the kernels walk those, whatever part of the last one exists.
+template <int D, bool RAGGED>
+int attn_bwd_mfma(const BwdCall& c) {
+  const bf16 *dout = c.dout, *q = c.q, *k = c.k, *v = c.v, *o = c.o;
+  const float* lse = c.lse;
+  bf16 *dq = c.dq, *dk = c.dk, *dv = c.dv;
+  const int s = c.s, b = c.b, nq = c.nq, nkv = c.nkv, sp = attn_padded_len(s);
+  const float scale = c.scale;
+  const QLayout ql = c.ql, ol = c.ol, dol = c.dol, dql = c.dql;
+  const KLayout kl = c.kl, vl = c.vl, dkl = c.dkl, dvl = c.dvl;
+  hipStream_t st = c.st;
+  float* delta = c.workspace;
+  const int64_t rows = (int64_t)b * nq * sp;
+  float* neg_lse2 = delta + rows;
+  float* part_k = neg_lse2 + rows;
+  const AttnForms forms = attn_forms(sp, b, nq, c.flags);
+  const int qsplit = forms.qsplit;
+  float* part_v = part_k + rows * qsplit * D;
+  // query heads of a KV group per dK/dV workgroup: as many as leave two workgroups per compute
+  // unit (KR_DKDV_HPW_MAX: a build-time cap, for measurements)
+  int hpw = 1;
+  {
+    const int per_group = nq / nkv;
+    const int64_t wgs = (int64_t)(sp / 128) * nq * b * qsplit;
+    for (int h2 = per_group < KR_DKDV_HPW_MAX ? per_group : KR_DKDV_HPW_MAX; h2 > 1; --h2)
+      if (per_group % h2 == 0 && wgs / h2 >= 2 * (int64_t)kr_compute_units()) {
+        hpw = h2;
+        break;
+      }
+  }
+  const bool partial = nq / hpw != nkv || qsplit > 1;
+  constexpr size_t lds_dkdv = 3 * (2 * BT_BYTES + 8 * tile_rows<D>) + 32768;  // three stages + the hand-over area
+  constexpr size_t lds_dq = 2 * (2 * BT_BYTES);  // two stages of a K and a V tile
+  constexpr size_t lds_dq_w64 = 3 * (2 * BT_BYTES) + 4 * 4096;  // three stages + a 4 KB output stage per wave
+  static const hipError_t attr_status = [] {
+    hipError_t e = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<D, RAGGED, false>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<D, RAGGED, true>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, RAGGED, 1>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, RAGGED, 2>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * lds_dq));
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute((const void*)attn_bwd_dq_w64_kernel<D, RAGGED>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq_w64);
+    return e;
+  }();
+  if (attr_status != hipSuccess) return KR_ELAUNCH;
+
+  const int per = nq / nkv;
+  const float scale_log2 = scale * kLog2e;
+  const int dq_blocks = (sp / BQ) * nq * b;
+  if (forms.shared_dq) {
+    // 256-query tiles (one for every compute unit, or other streams beside): one wave per SIMD, 64 rows each.
+    // It comes first: it also computes delta and the log2-domain copy of lse that the dK/dV kernel reads.
+    hipLaunchKernelGGL((attn_bwd_dq_w64_kernel<D, RAGGED>), dim3(dq_blocks / 2), dim3(256), lds_dq_w64, st,
+                       q, k, v, dout, o, lse,
+                       delta, neg_lse2, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol, ol, dql);
+  } else {
+    hipLaunchKernelGGL((attn_delta_kernel<D>), dim3((unsigned)((rows * (D / 8) + 255) / 256)), dim3(256), 0, st,
+                       dout, o, lse, delta, neg_lse2, s, sp, nq, per, rows, dol, ol);
+  }
+  if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
+  const dim3 grid_kv((sp / 128) * (nq / hpw) * b * qsplit);
+#define KR_DKDV_LAUNCH(P)                                                                           \
+  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, RAGGED, P>), grid_kv, dim3(512), lds_dkdv, st, q,   \
+                     k, v, dout, neg_lse2,     \
+                     delta, dk, dv, part_k, part_v, s, nq, nkv,         \
+                     partial ? qsplit : 1, hpw, scale, scale_log2, ql, kl, vl, dol, dkl, dvl)
+  if (partial) {
+    KR_DKDV_LAUNCH(true);
+    if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
+    const int64_t total = (int64_t)b * nkv * s * (D / 8);
+    hipLaunchKernelGGL((attn_group_reduce_kernel<D>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       st, part_k, part_v, dk, dv, s, sp,
+                       nq / hpw, nkv, qsplit, total, dkl, dvl);
+  } else {
+    KR_DKDV_LAUNCH(false);
+  }
+#undef KR_DKDV_LAUNCH
+  if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
+  if (forms.shared_dq) return kr_launch_status();  // its dQ kernel ran in front of the dK/dV kernel
+  if (dq_blocks <= 4 * 256) {  // few workgroups: the longest causal rows set the time
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, RAGGED, 2>), dim3(dq_blocks), dim3(512), 2 * lds_dq, st,
+                       q, k, v, dout, lse,
+                       delta, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
+                       dql);
+  } else {
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<D, RAGGED, 1>), dim3(dq_blocks), dim3(256), lds_dq, st,
+                       q, k, v, dout, lse,
+                       delta, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
+                       dql);
+  }
+  return kr_launch_status();
+}
+}  // namespace
 
 static int attn_bwd_impl(const void* dout, const void* q, const void* k, const void* v,
                            const void* o, const float* lse, void* dq, void* dk, void* dv,
@@ -2108,7 +2449,8 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
   const KLayout kl{k_ss, k_sb, k_sh}, vl{v_ss, v_sb, v_sh}, dkl{dk_ss, dk_sb, dk_sh},
       dvl{dv_ss, dv_sb, dv_sh};
   float* delta = (float*)workspace;
-  if (!attn_fast_path(s, hd) && !(flags & KR_ATTN_GENERAL_KERNELS)) {
+  const bool in_place = attn_in_place(s, hd, {q_ss, k_ss, v_ss, o_ss, do_ss, dq_ss, dk_ss, dv_ss});
+  if (!in_place && !(flags & KR_ATTN_GENERAL_KERNELS)) {
     // padded into the MFMA kernels: dO, q, o, k, v and the log-sum-exp go in, dq, dk, dv come back
     const int sp = attn_padded_len(s), per = nq / nkv;
     const size_t qb = attn_padded_bytes(s, b, nq), kb = attn_padded_bytes(s, b, nkv);
@@ -2139,7 +2481,7 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
     if (rc2 == KR_OK) rc2 = launch_unpad(dv_p, dv, s, b, nkv, 1, hd, as_qlayout(dvl), st);
     return rc2;
   }
-  if (!attn_fast_path(s, hd)) {
+  if (!attn_fast_path(s, hd) && (flags & KR_ATTN_GENERAL_KERNELS)) {
     using namespace general;
     const dim3 qgrid((s + GT - 1) / GT, nq, b), kgrid((s + GT - 1) / GT, nkv, b);
     hipLaunchKernelGGL(attn_general_delta_kernel, qgrid, dim3(GTHREADS), 0, st, (const bf16*)dout,
@@ -2154,92 +2496,10 @@ static int attn_bwd_impl(const void* dout, const void* q, const void* k, const v
                        (bf16*)dq, s, nq, nkv, hd, scale, ql, kl, vl, dol, dql);
     return kr_launch_status();
   }
-  const int64_t rows = (int64_t)b * nq * s;
-  float* neg_lse2 = delta + rows;
-  float* part_k = neg_lse2 + rows;
-  const AttnForms forms = attn_forms(s, b, nq, flags);
-  const int qsplit = forms.qsplit;
-  float* part_v = part_k + rows * qsplit * hd;
-  // query heads of a KV group per dK/dV workgroup: as many as leave two workgroups per compute
-  // unit (KR_DKDV_HPW_MAX: a build-time cap, for measurements)
-  int hpw = 1;
-  {
-    const int per_group = nq / nkv;
-    const int64_t wgs = (int64_t)(s / 128) * nq * b * qsplit;
-    for (int h2 = per_group < KR_DKDV_HPW_MAX ? per_group : KR_DKDV_HPW_MAX; h2 > 1; --h2)
-      if (per_group % h2 == 0 && wgs / h2 >= 2 * (int64_t)kr_compute_units()) {
-        hpw = h2;
-        break;
-      }
-  }
-  const bool partial = nq / hpw != nkv || qsplit > 1;
-  constexpr size_t lds_dkdv = 3 * (2 * BT_BYTES + 512) + 32768;  // three stages + the hand-over area
-  constexpr size_t lds_dq = 2 * (2 * BT_BYTES);  // two stages of a K and a V tile
-  constexpr size_t lds_dq_w64 = 3 * (2 * BT_BYTES) + 4 * 4096;  // three stages + a 4 KB output stage per wave
-  static const hipError_t attr_status = [] {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<1>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<2>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * lds_dq));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)attn_bwd_dq_w64_kernel,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq_w64);
-    return e;
-  }();
-  if (attr_status != hipSuccess) return KR_ELAUNCH;
-
-  const int per = nq / nkv;
-  const float scale_log2 = scale * kLog2e;
-  const int dq_blocks = (s / BQ) * nq * b;
-  if (forms.shared_dq) {
-    // 256-query tiles (one for every compute unit, or other streams beside): one wave per SIMD, 64 rows each.
-    // It comes first: it also computes delta and the log2-domain copy of lse that the dK/dV kernel reads.
-    hipLaunchKernelGGL(attn_bwd_dq_w64_kernel, dim3(dq_blocks / 2), dim3(256), lds_dq_w64, st,
-                       (const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)dout, (const bf16*)o, lse,
-                       delta, neg_lse2, (bf16*)dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol, ol, dql);
-  } else {
-    hipLaunchKernelGGL(attn_delta_kernel, dim3((unsigned)((rows * 16 + 255) / 256)), dim3(256), 0, st,
-                       (const bf16*)dout, (const bf16*)o, lse, delta, neg_lse2, s, nq, per, rows, dol, ol);
-  }
-  if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
-  const dim3 grid_kv((s / 128) * (nq / hpw) * b * qsplit);
-#define KR_DKDV_LAUNCH(P)                                                                           \
-  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<P>), grid_kv, dim3(512), lds_dkdv, st, (const bf16*)q,   \
-                     (const bf16*)k, (const bf16*)v, (const bf16*)dout, (const float*)neg_lse2,     \
-                     (const float*)delta, (bf16*)dk, (bf16*)dv, part_k, part_v, s, nq, nkv,         \
-                     partial ? qsplit : 1, hpw, scale, scale_log2, ql, kl, vl, dol, dkl, dvl)
-  if (partial) {
-    KR_DKDV_LAUNCH(true);
-    if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
-    const int64_t total = (int64_t)b * nkv * s * 16;
-    hipLaunchKernelGGL(attn_group_reduce_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                       st, (const float*)part_k, (const float*)part_v, (bf16*)dk, (bf16*)dv, s,
-                       nq / hpw, nkv, qsplit, total, dkl, dvl);
-  } else {
-    KR_DKDV_LAUNCH(false);
-  }
-#undef KR_DKDV_LAUNCH
-  if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
-  if (forms.shared_dq) return kr_launch_status();  // its dQ kernel ran in front of the dK/dV kernel
-  if (dq_blocks <= 4 * 256) {  // few workgroups: the longest causal rows set the time
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<2>), dim3(dq_blocks), dim3(512), 2 * lds_dq, st,
-                       (const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)dout, lse,
-                       (const float*)delta, (bf16*)dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
-                       dql);
-  } else {
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<1>), dim3(dq_blocks), dim3(256), lds_dq, st,
-                       (const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)dout, lse,
-                       (const float*)delta, (bf16*)dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
-                       dql);
-  }
-  return kr_launch_status();
+  const BwdCall c{(const bf16*)dout, (const bf16*)q, (const bf16*)k, (const bf16*)v, (const bf16*)o, lse, (bf16*)dq,
+                  (bf16*)dk, (bf16*)dv, delta, s, b, nq, nkv, scale, ql, ol, dol, dql, kl, vl, dkl, dvl, flags, st};
+  if (hd == 64) return s % BQ ? attn_bwd_mfma<64, true>(c) : attn_bwd_mfma<64, false>(c);
+  return s % BQ ? attn_bwd_mfma<128, true>(c) : attn_bwd_mfma<128, false>(c);
 }
 
 extern "C" int kr_attn_bwd(const void* dout, const void* q, const void* k, const void* v,
@@ -2271,6 +2531,47 @@ extern "C" int kr_attn_bwd_flags(const void* dout, const void* q, const void* k,
                        do_sh, dq_ss, dq_sb, dq_sg, dq_sh, dk_ss, dk_sb, dk_sh, dv_ss, dv_sb, dv_sh, flags, stream);
 }
 
+namespace {
+struct FwdCall {
+  const bf16 *q, *k, *v;
+  bf16* o;
+  float* lse;
+  int s, b, nq, nkv;
+  float scale;
+  QLayout ql, ol;
+  KLayout kl, vl;
+  int flags;
+  hipStream_t st;
+};
+
+template <int D, bool RAGGED>
+int attn_fwd_mfma(const FwdCall& c) {
+  const int s = c.s, b = c.b, nq = c.nq, sp = attn_padded_len(s);
+  if (attn_forms(sp, b, nq, c.flags).shared_fwd) {
+    // 256-query tiles (one for every compute unit, or other streams beside): the halves share their K / V tiles
+    constexpr size_t lds_sh = 3 * 16 * ((1024 + 16) + (1024 + 64));  // 100 KiB
+    static const hipError_t attr_sh = hipFuncSetAttribute(
+        (const void*)attn_fwd_sh_kernel<D, RAGGED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_sh);
+    if (attr_sh != hipSuccess) return KR_ELAUNCH;
+    hipLaunchKernelGGL((attn_fwd_sh_kernel<D, RAGGED>), dim3((sp / 256) * nq * b), dim3(512), lds_sh, c.st,
+                       c.q, c.k, c.v, c.o, c.lse, s, c.nq, c.nkv, c.scale * kLog2e, c.ql.s_, c.ql.b_, c.ql.g_, c.ql.h_, c.kl.s_,
+                       c.kl.b_, c.kl.h_, c.vl.s_, c.vl.b_, c.vl.h_, c.ol.s_, c.ol.b_, c.ol.g_, c.ol.h_);
+    return kr_launch_status();
+  }
+  // two K and two V tiles of 17 KiB (padded blocks) per half; afterwards the same memory holds
+  // the hand-over of half 1 (66 KiB) and, from 68 KiB on, 4 KiB of output staging per wave
+  constexpr size_t lds_pp = 2 * 2 * 16 * ((1024 + 16) + (1024 + 64));  // 133 KiB
+  static_assert(lds_pp >= 84 * 1024, "hand-over and output staging must fit");
+  static const hipError_t attr_status = hipFuncSetAttribute(
+      (const void*)attn_fwd_pp_kernel<D, RAGGED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pp);
+  if (attr_status != hipSuccess) return KR_ELAUNCH;
+  hipLaunchKernelGGL((attn_fwd_pp_kernel<D, RAGGED>), dim3((sp / BQ) * nq * b), dim3(512), lds_pp, c.st,
+                     c.q, c.k, c.v, c.o, c.lse, s, c.nq, c.nkv, c.scale * kLog2e, c.ql.s_, c.ql.b_, c.ql.g_, c.ql.h_, c.kl.s_,
+                     c.kl.b_, c.kl.h_, c.vl.s_, c.vl.b_, c.vl.h_, c.ol.s_, c.ol.b_, c.ol.g_, c.ol.h_);
+  return kr_launch_status();
+}
+}  // namespace
+
 static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, int s,
                            int b, int nq, int nkv, int hd, float scale, int64_t q_ss, int64_t q_sb,
                            int64_t q_sg, int64_t q_sh, int64_t k_ss, int64_t k_sb, int64_t k_sh,
@@ -2291,11 +2592,12 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
     if (!attn_strides_ok(seq, {q_sb, q_sg, q_sh, k_sb, k_sh, v_sb, v_sh, o_sb, o_sg, o_sh}))
       return KR_EUNSUPPORTED;
   }
+  const bool in_place = attn_in_place(s, hd, {q_ss, k_ss, v_ss, o_ss});
   // (a workspace that is there but too small is a caller's mistake, not a request for the general kernels)
   if (!attn_fast_path(s, hd) && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr &&
       workspace_bytes < kr_attn_fwd_workspace_bytes(s, b, nq, nkv, hd))
     return KR_EINVAL;
-  if (!attn_fast_path(s, hd) && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr) {
+  if (!in_place && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr) {
     // padded into the MFMA kernels
     hipStream_t st = (hipStream_t)stream;
     const int sp = attn_padded_len(s), per = nq / nkv;
@@ -2318,7 +2620,7 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
     if (rc2 == KR_OK) rc2 = launch_resize_rows(lse_p, lse, (int64_t)b * nq, sp, s, 0.f, st);
     return rc2;
   }
-  if (!attn_fast_path(s, hd)) {
+  if (!in_place || (!attn_fast_path(s, hd) && (flags & KR_ATTN_GENERAL_KERNELS))) {
     using namespace general;
     const QLayout ql{q_ss, q_sb, q_sg, q_sh}, ol{o_ss, o_sb, o_sg, o_sh};
     const KLayout kl{k_ss, k_sb, k_sh}, vl{v_ss, v_sb, v_sh};
@@ -2327,31 +2629,11 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
                        lse, s, nq, nkv, hd, scale, ql, kl, vl, ol);
     return kr_launch_status();
   }
-  if (attn_forms(s, b, nq, flags).shared_fwd) {
-    // 256-query tiles (one for every compute unit, or other streams beside): the halves share their K / V tiles
-    constexpr size_t lds_sh = 3 * 16 * ((1024 + 16) + (1024 + 64));  // 100 KiB
-    static const hipError_t attr_sh = hipFuncSetAttribute(
-        (const void*)attn_fwd_sh_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_sh);
-    if (attr_sh != hipSuccess) return KR_ELAUNCH;
-    hipLaunchKernelGGL(attn_fwd_sh_kernel, dim3((s / 256) * nq * b), dim3(512), lds_sh,
-                       (hipStream_t)stream, (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o,
-                       lse, s, nq, nkv, scale * kLog2e, q_ss, q_sb, q_sg, q_sh, k_ss, k_sb, k_sh, v_ss,
-                       v_sb, v_sh, o_ss, o_sb, o_sg, o_sh);
-    return kr_launch_status();
-  }
-  // two K and two V tiles of 17 KiB (padded blocks) per half; afterwards the same memory holds
-  // the hand-over of half 1 (66 KiB) and, from 68 KiB on, 4 KiB of output staging per wave
-  constexpr size_t lds_pp = 2 * 2 * 16 * ((1024 + 16) + (1024 + 64));  // 133 KiB
-  static_assert(lds_pp >= 84 * 1024, "hand-over and output staging must fit");
-  static const hipError_t attr_status = hipFuncSetAttribute(
-      (const void*)attn_fwd_pp_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pp);
-  if (attr_status != hipSuccess) return KR_ELAUNCH;
-  const int blocks = (s / BQ) * nq * b;
-  hipLaunchKernelGGL(attn_fwd_pp_kernel, dim3(blocks), dim3(512), lds_pp, (hipStream_t)stream,
-                     (const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o, lse, s, nq, nkv,
-                     scale * kLog2e, q_ss, q_sb, q_sg, q_sh, k_ss, k_sb, k_sh, v_ss, v_sb, v_sh, o_ss,
-                     o_sb, o_sg, o_sh);
-  return kr_launch_status();
+  const FwdCall c{(const bf16*)q, (const bf16*)k, (const bf16*)v, (bf16*)o, lse, s, b, nq, nkv, scale,
+                  QLayout{q_ss, q_sb, q_sg, q_sh}, QLayout{o_ss, o_sb, o_sg, o_sh}, KLayout{k_ss, k_sb, k_sh},
+                  KLayout{v_ss, v_sb, v_sh}, flags, (hipStream_t)stream};
+  if (hd == 64) return s % BQ ? attn_fwd_mfma<64, true>(c) : attn_fwd_mfma<64, false>(c);
+  return s % BQ ? attn_fwd_mfma<128, true>(c) : attn_fwd_mfma<128, false>(c);
 }
 
 extern "C" int kr_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int s,
@@ -2372,9 +2654,8 @@ extern "C" int kr_attn_fwd_flags(const void* q, const void* k, const void* v, vo
                        v_sb, v_sh, o_ss, o_sb, o_sg, o_sh, flags, stream);
 }
 
-// kr_attn_fwd_flags with a workspace of kr_attn_fwd_workspace_bytes(): a shape outside the MFMA kernels (head
-// dimension below 128, a sequence that is not whole 128-row tiles) is padded into them through the
-// workspace instead of taking the general kernels.  A shape they take as it is needs no workspace.
+// kr_attn_fwd_flags with a workspace of kr_attn_fwd_workspace_bytes(): a shape the MFMA kernels do not take as it
+// lies (attn_in_place) is padded into them through the workspace instead of taking the general kernels.
 extern "C" int kr_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, int s, int b,
                               int nq, int nkv, int hd, float scale, int64_t q_ss, int64_t q_sb, int64_t q_sg,
                               int64_t q_sh, int64_t k_ss, int64_t k_sb, int64_t k_sh, int64_t v_ss, int64_t v_sb,

@@ -119,3 +119,20 @@ def test_no_instruction_reads_a_hand_placed_mfma_result_too_early(tmp_path):
     meta = text[text.index("attn_bwd_dq_w64_kernel", text.index("amdhsa.kernels")):]
     spills = re.search(r"\.vgpr_spill_count:\s*(\d+)", meta)
     assert spills and int(spills.group(1)) == 0
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc is not installed")
+def test_every_instance_of_the_kernel_keeps_the_distance(tmp_path):
+    """Head dimensions 128 and 64, whole and ragged lengths: four instances.  With 64 channels a tile has four steps of
+    sixteen score MFMAs: prologue 16 + loop 64 + the diagonal tile's first three steps 48."""
+    out = tmp_path / "kr_attention.s"
+    subprocess.run(["make", "-C", CSRC, f"HIPCC={HIPCC}", f"ASMDIR={tmp_path}", str(out)], check=True,
+                   stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL, timeout=600)
+    text = out.read_text()
+    names = re.findall(r"^_Z\w*(attn_bwd_dq_w64_kernel\w*):", text, re.M)
+    assert len(set(names)) == 4
+    for name in names:
+        n_asm, bad = early_readers(_kernel_body(text, name))
+        assert n_asm == 128 and not bad, (name, n_asm, bad[:5])
+        meta = text[text.index(name, text.index("amdhsa.kernels")):]
+        assert int(re.search(r"\.vgpr_spill_count:\s*(\d+)", meta).group(1)) == 0

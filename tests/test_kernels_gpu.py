@@ -546,6 +546,33 @@ def test_attention_padded_into_the_mfma_kernels_equals_the_whole_tile_call(be):
     assert torch.equal(dq, dq_f[:s]) and torch.equal(dk, dk_f[:s]) and torch.equal(dv, dv_f[:s])
 
 
+@pytest.mark.parametrize("s,b,nq,nkv,hd", [(8, 1, 2, 1, 64), (127, 1, 2, 2, 64), (128, 1, 2, 1, 64), (129, 2, 4, 1, 64),
+                                            (136, 1, 3, 1, 128), (200, 1, 4, 2, 64), (248, 2, 2, 1, 128),
+                                            (320, 1, 4, 4, 64), (520, 1, 3, 1, 128), (1000, 2, 32, 8, 64),
+                                            (1000, 8, 8, 2, 128), (1024, 2, 32, 8, 64)])
+@pytest.mark.parametrize("beside", [False, True])
+def test_attention_in_place_at_head_dimension_64_and_ragged_lengths(be, s, b, nq, nkv, hd, beside):
+    """The MFMA kernels on tensors as they lie: tiles of 128 rows of 64 channels (an odd number of them for the split
+    forms, none at all for a part), last tiles that the sequence ends in, both forms of every kernel
+    (``beside`` takes the unsplit ones; so do the last three shapes).  What lies behind the sequence in memory is
+    infinite: it must not be read into a result.  Tolerances as for every attention shape (bf16 operands, fp32 sums)."""
+    base, q, k, v = _grouped(s + 3, b, nq, nkv, hd, seed=120)
+    base[s:] = float("inf")
+    q, k, v = q[:s], k[:s], v[:s]
+    do_all = rnd(s + 3, b, nq, hd, seed=121)
+    do_all[s:] = float("inf")
+    do = do_all[:s]
+    scale = hd ** -0.5
+    o, lse = be.attn_fwd(q, k, v, scale, beside_other_streams=beside)
+    qf, kf, vf = (t.float().cpu().clone().requires_grad_(True) for t in (q.flatten(2, 3), k, v))
+    ro, rlse = R.causal_gqa_attention(qf, kf, vf, return_lse=True)
+    assert rel(o, ro) <= TOL and rel(lse, rlse) <= 1e-4
+    ro.backward(do.float().cpu())
+    dq, dk, dv = be.attn_bwd(do, q, k, v, o, lse, scale, beside_other_streams=beside)
+    assert all(torch.isfinite(t.float()).all() for t in (o, lse, dq, dk, dv))
+    assert rel(dq.flatten(2, 3), qf.grad) <= TOL and rel(dk, kf.grad) <= TOL and rel(dv, vf.grad) <= TOL
+
+
 # ------------------------------------------------------------------ fused GEMM epilogues
 @pytest.mark.parametrize("m,n,k", [(512, 768, 512), (264, 520, 200), (4096, 4096, 1024), (1000, 3072, 640),
                                    (16384, 640, 72)])
