@@ -38,6 +38,11 @@
 //   * Workgroups are persistent (one per compute unit); ids are remapped so that the tiles
 //     resident on one XCD (ids congruent mod 8) form a compact band of C and share A/B panels
 //     in that XCD's L2.
+//   * Outputs of few tiles (short sequences, thin shards) use 128 x 128 tiles of the same structure:
+//     4 x 4 MFMA tiles per wave, 16 KB slots, two workgroups per compute unit.  Such a launch is
+//     bound by the number of work items and the latency of a K-step, not by LDS traffic (which a
+//     small tile has twice of per FLOP: 128 KB per 512 MFMA cycles with the loads, so it tops out at
+//     about two thirds of the matrix rate and large outputs keep the large tile).
 //   * Split-K: when C has too few tiles to fill 256 CUs (weight gradients: a small N x K
 //     output contracted over all tokens), the contraction is cut into up to 16 ranges, each
 //     workgroup writes an fp32 partial tile into a caller-provided workspace, and a small
@@ -47,12 +52,15 @@
 namespace {
 
 constexpr int BK = 64;
-constexpr int BM = 256, BN = 256;  // BN: the widest tile; a kernel instance covers 32 * WN columns
-constexpr int WT = 8;  // 16x16 MFMA tiles per wave along M: a wave owns 128 rows x 16 * WN columns of C
+constexpr int BM = 256, BN = 256;  // the largest tile; a kernel instance covers 32 * WT rows x 32 * WN columns
+// WT: 16x16 MFMA tiles per wave along M; a wave owns 16 * WT rows x 16 * WN columns of C.  WT = 8: 256-row tiles
+// with 32 KB ring slots.  WT = 4 (with WN = 4): 128 x 128 tiles with 16 KB slots, two workgroups per compute unit
+// (see choose_plan for when they are taken).
+constexpr int WT_LARGE = 8, WT_SMALL = 4;
 constexpr int NTHREADS = 256;
-constexpr int TILE = 256 * BK;  // elements of one operand tile (either layout)
-constexpr uint32_t SLOT_BYTES = TILE * sizeof(bf16);
-constexpr int NSLOTS = 5;          // 5 x 32 KB = the whole 160 KB of LDS
+template <int WT>
+constexpr uint32_t kSlotBytes = 32 * WT * BK * sizeof(bf16);  // one operand tile (either layout)
+constexpr int NSLOTS = 5;          // 5 x 32 KB = the whole 160 KB of LDS (5 x 16 KB: half of it)
 constexpr int kXcds = 8;
 constexpr int KR_GEMM_EPI_TRANSPOSED_OUT = 100;  // internal: not part of the C ABI's epilogue values
 constexpr int kGroupM = 4;
@@ -75,8 +83,11 @@ __device__ __forceinline__ int kmajor_off(int row, int chunk) {
 // k-row bits 0, 1 (the four k-rows one 16-lane group reads together) and bit 3 (the two groups
 // of a 32-lane half read k-rows 8 apart).
 __device__ __forceinline__ int transp_swz(int krow) { return ((krow & 3) << 2) | (((krow >> 3) & 1) << 1); }
+// A small tile has rows of 128 elements, 256 bytes: as many as there are banks, so what a row and the
+// swizzle do to the banks is the same.
+template <int TW>
 __device__ __forceinline__ int transp_off(int krow, int col) {
-  return krow * 256 + (((col >> 3) ^ transp_swz(krow)) << 3) + (col & 7);
+  return krow * TW + (((col >> 3) ^ transp_swz(krow)) << 3) + (col & 7);
 }
 
 // ---- direct global -> LDS loads ---------------------------------------------------------------
@@ -100,9 +111,10 @@ __device__ __forceinline__ uint32_t lds_addr(const bf16* p) {
 }
 
 // ---- which 16-byte chunk a lane fetches ------------------------------------------------------
-// The four waves share every operand tile: wave w issues loads i = 0..7, load i fills the 1-KiB
-// block w + 4 i.  Block b of a K-major tile holds rows 8b..8b+7; block b of a transposed tile
-// holds contraction rows 2b, 2b+1.  The swizzle is applied on the global side: each lane
+// The four waves share every operand tile: wave w issues loads i = 0..7 (0..3 for a small tile), load i
+// fills the 1-KiB block w + 4 i.  Block b of a K-major tile holds rows 8b..8b+7; block b of a transposed
+// tile holds contraction rows 2b, 2b+1 (4b..4b+3 in a small tile, whose rows are half as long; TW is the
+// number of operand rows a tile holds, 256 or 128).  The swizzle is applied on the global side: each lane
 // fetches the chunk that belongs at its LDS position.
 // Returns the element offset from the K-step's base pointer.  Rows beyond the matrix are
 // clamped to the last valid row; a chunk that would start beyond the contraction range
@@ -119,7 +131,11 @@ __device__ __forceinline__ uint32_t lds_addr(const bf16* p) {
 __device__ __forceinline__ int run_off(int r, int ld, int sh, int outer) {
   return (r >> sh) * outer + (r & ((1 << sh) - 1)) * ld;
 }
-template <bool TRANSPOSED>
+template <int TW>
+__device__ __forceinline__ int load_krow(int i, int wave, int lane) {
+  return TW == 256 ? 2 * wave + (lane >> 5) + 8 * i : 4 * wave + (lane >> 4) + 16 * i;
+}
+template <bool TRANSPOSED, int TW>
 __device__ __forceinline__ uint32_t load_offset(int i, int wave, int lane, int ld, int row0,
                                                 int rows_total, int k_left, int gate_up_f = 0,
                                                 int half_rows = 0, int sh = 0, int outer = 0) {
@@ -134,27 +150,27 @@ __device__ __forceinline__ uint32_t load_offset(int i, int wave, int lane, int l
   }
   // (the contraction rows of a K-step start at a multiple of 64, hence of the run length: the
   // position inside the K-step maps like a row of its own)
-  int krow = 2 * wave + (lane >> 5) + 8 * i;
-  int c = row0 + ((lane & 31) ^ transp_swz(krow)) * 8;
+  int krow = load_krow<TW>(i, wave, lane);
+  int c = row0 + ((lane & (TW / 8 - 1)) ^ transp_swz(krow)) * 8;
   c = c + 8 <= rows_total ? c : rows_total - 8;
   krow = krow < k_left ? krow : k_left - 1;
   return (uint32_t)((sh ? run_off(krow, ld, sh, outer) : krow * ld) + c);
 }
 // contraction index (relative to the K-step) of the chunk that load i of this lane fills
-template <bool TRANSPOSED>
+template <bool TRANSPOSED, int TW>
 __device__ __forceinline__ int load_k(int i, int wave, int lane) {
   if (!TRANSPOSED) {
     const int row = 8 * wave + (lane >> 3);  // (row >> 1) & 7 does not depend on i
     return ((lane & 7) ^ ((row >> 1) & 7)) * 8;
   }
-  return 2 * wave + (lane >> 5) + 8 * i;
+  return load_krow<TW>(i, wave, lane);
 }
 
 // ---- LDS -> MFMA operand fragments ----------------------------------------------------------
 // v_mfma_f32_16x16x32_bf16 wants from lane l the 8 contraction elements 8 (l / 16) .. + 7 of
 // operand row l % 16.  Fragment (g, h): operand rows row0 + 16 g .., contraction half h (32
 // elements) of the K-step.
-template <bool TRANSPOSED>
+template <bool TRANSPOSED, int WT>
 struct FragReader {
   // K-major: one base per half (the swizzle XOR depends on the chunk), g is an immediate
   // transposed: one base per g (the XOR depends on the column), the half is an immediate
@@ -171,7 +187,7 @@ struct FragReader {
       const int p = lane & 15;
       const int krow = 8 * (lane >> 4) + (p >> 2);
 #pragma unroll
-      for (int g = 0; g < WT; ++g) base[g] = 2u * (uint32_t)transp_off(krow, row0 + 16 * g + (p & 3) * 4);
+      for (int g = 0; g < WT; ++g) base[g] = 2u * (uint32_t)transp_off<32 * WT>(krow, row0 + 16 * g + (p & 3) * 4);
     }
   }
 };
@@ -179,14 +195,15 @@ struct FragReader {
 __device__ __forceinline__ bf16x8 frag_kmajor(uint32_t a, int g) {
   return *(KR_LDS const bf16x8*)(a + (uint32_t)(g * 16 * BK * 2));
 }
+template <int TW>
 __device__ __forceinline__ bf16x8 frag_transp(uint32_t a, int h) {
-  const uint32_t a0 = a + (uint32_t)(h * 32 * 256 * 2);
+  const uint32_t a0 = a + (uint32_t)(h * 32 * TW * 2);
   union {
     struct { s16x4 lo, hi; } s;
     bf16x8 v;
   } u;
   u.s.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a0));
-  u.s.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a0 + 2u * 4 * 256));
+  u.s.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((KR_LDS s16x4*)(a0 + 2u * 4 * TW));
   return u.v;
 }
 
@@ -222,7 +239,7 @@ struct Segments {
   int n, steps;
 };
 
-template <int WN>
+template <int WT, int WN>
 struct Frags {
   bf16x8 a[WT], b[WN];
 };
@@ -238,8 +255,8 @@ struct Count { static constexpr int value = N; };
 // extra address arithmetic or its registers.
 // SEG (layout NT): A and B are the pieces named by `segs` (the A / B arguments are unused); K is their
 // total length.
-template <bool A_T, bool B_T, int WN, int EPI, bool RUNS = false, bool SEG = false>
-__global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__ A, int lda,
+template <bool A_T, bool B_T, int WN, int EPI, bool RUNS = false, bool SEG = false, int WT = WT_LARGE>
+__global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(const bf16* __restrict__ A, int lda,
                                                         const bf16* __restrict__ B, int ldb,
                                                         bf16* __restrict__ C, int ldc, int M,
                                                         int N, int K, int accumulate, int k_per,
@@ -248,6 +265,9 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
                                                         bf16* __restrict__ out2, int ld_out2,
                                                         RowRuns runs_arg, Segments segs) {
   static_assert(!SEG || (A_T && B_T), "operand pieces: layout NT");
+  static_assert(WT == WT_LARGE || (WT == WT_SMALL && WN == 4 && EPI != KR_GEMM_EPI_TRANSPOSED_OUT), "tile shapes");
+  constexpr int TW = 32 * WT;  // operand rows an LDS tile holds (a B tile may use fewer)
+  constexpr uint32_t SLOT_BYTES = kSlotBytes<WT>;
   // (without RUNS every run length reads as a compile-time 1: the branches below fold away)
   const RowRuns runs = RUNS ? runs_arg : RowRuns{0, 0, 0, 0, 0, 0};
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
@@ -256,8 +276,10 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
   constexpr int BN_ = 32 * WN;
   // loads per wave of a B tile: a K-major tile's unused rows are simply not fetched; in a
   // transposed tile every load spans all 256 columns
-  constexpr int NB_LOADS = B_T ? 8 : WN;
-  const int wm = wave >> 1, wn = wave & 1;  // wave tile: rows wm*128.., columns wn*16*WN..
+  constexpr int NB_LOADS = B_T ? WT : WN;
+  constexpr int NA_LOADS = WT;
+  constexpr int BM_ = 32 * WT;
+  const int wm = wave >> 1, wn = wave & 1;  // wave tile: rows wm*16*WT.., columns wn*16*WN..
   // fused epilogues: ADD: C = bf16(bf16(A.B) + aux), aux [M,N] with row stride ld_aux.
   // SWIGLU: C = x [M, N = 2F] and out2 = silu(x[:, :F]) * x[:, F:] [M, F]; a tile then covers
   // 16 * WN columns of out2: its left half (the waves with wn = 0) computes their gate columns,
@@ -278,7 +300,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
   constexpr bool epi_add = EPI == KR_GEMM_EPI_ADD;
   constexpr bool swiglu = EPI == KR_GEMM_EPI_SWIGLU;
   const int gate_up_f = swiglu ? N / 2 : 0;
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = swiglu ? N / BN_ : (N + BN_ - 1) / BN_;
+  const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = swiglu ? N / BN_ : (N + BN_ - 1) / BN_;
   const int ntiles = tiles_m * tiles_n;
   const bool split_k = partial != nullptr;
   const uint32_t smem_b = lds_addr(smem);
@@ -296,7 +318,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
     const int split = v / ntiles;
     int tile_m, tile_n;
     remap_block(v - split * ntiles, ntiles, tiles_m, tiles_n, tile_m, tile_n);
-    m0 = tile_m * BM;
+    m0 = tile_m * BM_;
     n0 = swiglu ? tile_n * (16 * WN) : tile_n * BN_;
     int k0 = 0;
     if (split_k) {
@@ -355,27 +377,27 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
   // accumulators live in the accumulation registers (the MFMAs are written as inline assembly
   // with that register class, see mfma() below); fragments in ordinary vector registers
   f32x4 acc[WT][WN];
-  Frags<WN> X, Y;
-  uint32_t la[8], lb[8];  // byte offsets of this lane's chunk in the 8 loads of an A / a B tile
+  Frags<WT, WN> X, Y;
+  uint32_t la[WT], lb[WT];  // byte offsets of this lane's chunk in the loads of an A / a B tile
 
   auto set_offsets = [&](int k_left) {
     int l2 = lane;
     asm volatile("" : "+v"(l2));
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      la[i] = 2u * load_offset<A_T>(i, wave, l2, lda, m0, M, k_left, 0, 0, runs.a_sh, runs.a_outer);
-      lb[i] = 2u * load_offset<B_T>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN);
+    for (int i = 0; i < WT; ++i) {
+      la[i] = 2u * load_offset<A_T, TW>(i, wave, l2, lda, m0, M, k_left, 0, 0, runs.a_sh, runs.a_outer);
+      lb[i] = 2u * load_offset<B_T, TW>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN);
     }
   };
-  // the first `count` loads of a tile (8 for A, NB_LOADS for B)
-  auto request = [&](const bf16* base, const uint32_t (&off)[8], uint32_t slot, auto count_tag) {
+  // the first `count` loads of a tile (NA_LOADS for A, NB_LOADS for B)
+  auto request = [&](const bf16* base, const uint32_t (&off)[WT], uint32_t slot, auto count_tag) {
     constexpr int COUNT = decltype(count_tag)::value;
     const uint32_t dst = slot + wave_blk;
     dma_b128<0 * 4096>(base, off[0], dst);
     dma_b128<1 * 4096>(base, off[1], dst);
     dma_b128<2 * 4096>(base, off[2], dst);
     dma_b128<3 * 4096>(base, off[3], dst);
-    dma_b128<4 * 4096>(base, off[4], dst);
+    if constexpr (COUNT > 4) dma_b128<4 * 4096>(base, off[4], dst);
     if constexpr (COUNT > 5) dma_b128<5 * 4096>(base, off[5], dst);
     if constexpr (COUNT > 6) dma_b128<6 * 4096>(base, off[6], dst);
     if constexpr (COUNT > 7) dma_b128<7 * 4096>(base, off[7], dst);
@@ -383,12 +405,12 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
   // K-steps 0 and 1 of the current item into r0..r3
   auto request_first_two = [&]() {
     set_offsets(nk == 1 ? k_tail : BK);
-    request(a_base(0), la, r0, Count<8>{});
+    request(a_base(0), la, r0, Count<NA_LOADS>{});
     request(b_base(0), lb, r1, Count<NB_LOADS>{});
     seg_advance();
     if (nk > 1) {
       if (nk == 2 && k_tail != BK) set_offsets(k_tail);
-      request(a_base(1), la, r2, Count<8>{});
+      request(a_base(1), la, r2, Count<NA_LOADS>{});
       request(b_base(1), lb, r3, Count<NB_LOADS>{});
       seg_advance();
     }
@@ -400,20 +422,20 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
     int l2 = lane;
     asm volatile("" : "+v"(l2));
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < WT; ++i) {
       const uint32_t blk = (uint32_t)(wave + 4 * i) * 1024u + (uint32_t)l2 * 16u;
-      if (load_k<A_T>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sa + blk) = zero8();
-      if (load_k<B_T>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sb + blk) = zero8();
+      if (load_k<A_T, TW>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sa + blk) = zero8();
+      if (load_k<B_T, TW>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sb + blk) = zero8();
     }
   };
 
   // fragment addressing, recomputed per item from an opaque copy of the lane id so that it is
   // not live through the epilogue
-  FragReader<A_T> fa;
-  FragReader<B_T> fb;
+  FragReader<A_T, WT> fa;
+  FragReader<B_T, WT> fb;
   // addresses for reading half h of the tiles in slots sa / sb
-  auto frag_addrs = [&](uint32_t sa, uint32_t sb, int h, uint32_t (&aa)[FragReader<A_T>::NBASE],
-                        uint32_t (&ba)[FragReader<B_T>::NBASE]) {
+  auto frag_addrs = [&](uint32_t sa, uint32_t sb, int h, uint32_t (&aa)[FragReader<A_T, WT>::NBASE],
+                        uint32_t (&ba)[FragReader<B_T, WT>::NBASE]) {
     if (!A_T) {
       aa[0] = sa + fa.base[h];
       asm volatile("" : "+v"(aa[0]));
@@ -435,11 +457,11 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
       }
     }
   };
-  auto read_a = [&](const uint32_t (&aa)[FragReader<A_T>::NBASE], int g, int h) {
-    if constexpr (!A_T) return frag_kmajor(aa[0], g); else return frag_transp(aa[g], h);
+  auto read_a = [&](const uint32_t (&aa)[FragReader<A_T, WT>::NBASE], int g, int h) {
+    if constexpr (!A_T) return frag_kmajor(aa[0], g); else return frag_transp<TW>(aa[g], h);
   };
-  auto read_b = [&](const uint32_t (&ba)[FragReader<B_T>::NBASE], int g, int h) {
-    if constexpr (!B_T) return frag_kmajor(ba[0], g); else return frag_transp(ba[g], h);
+  auto read_b = [&](const uint32_t (&ba)[FragReader<B_T, WT>::NBASE], int g, int h) {
+    if constexpr (!B_T) return frag_kmajor(ba[0], g); else return frag_transp<TW>(ba[g], h);
   };
 
   // One half-step: the 64 MFMAs of one 32-element half of a K-step on `cur`, with the 16
@@ -447,10 +469,10 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
   // if DMA, the 8 requests of one operand tile woven in between in exactly this order.  The
   // operands are swapped (the B fragment feeds the instruction's A port), so a lane ends up
   // with four consecutive columns of one row of C.
-  auto half = [&](Frags<WN>& cur, Frags<WN>& nxt, uint32_t sa, uint32_t sb, int h, auto dma_tag,
-                  const bf16* dbase, const uint32_t (&doff)[8], uint32_t dslot) {
+  auto half = [&](Frags<WT, WN>& cur, Frags<WT, WN>& nxt, uint32_t sa, uint32_t sb, int h, auto dma_tag,
+                  const bf16* dbase, const uint32_t (&doff)[WT], uint32_t dslot) {
     constexpr int DMA = decltype(dma_tag)::value;  // how many loads to weave in (0: none)
-    uint32_t aa[FragReader<A_T>::NBASE], ba[FragReader<B_T>::NBASE];
+    uint32_t aa[FragReader<A_T, WT>::NBASE], ba[FragReader<B_T, WT>::NBASE];
     frag_addrs(sa, sb, h, aa, ba);
     const uint32_t dst = dslot + wave_blk;
 #pragma unroll
@@ -476,10 +498,10 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
             if (g == 1) dma_b128<1 * 4096>(dbase, doff[1], dst);
             if (g == 2) dma_b128<2 * 4096>(dbase, doff[2], dst);
             if (g == 3) dma_b128<3 * 4096>(dbase, doff[3], dst);
-            if (g == 4) dma_b128<4 * 4096>(dbase, doff[4], dst);
-            if (g == 5) dma_b128<5 * 4096>(dbase, doff[5], dst);
-            if (g == 6) dma_b128<6 * 4096>(dbase, doff[6], dst);
-            if (g == 7) dma_b128<7 * 4096>(dbase, doff[7], dst);
+            if constexpr (DMA > 4) if (g == 4) dma_b128<4 * 4096>(dbase, doff[4], dst);
+            if constexpr (DMA > 5) if (g == 5) dma_b128<5 * 4096>(dbase, doff[5], dst);
+            if constexpr (DMA > 6) if (g == 6) dma_b128<6 * 4096>(dbase, doff[6], dst);
+            if constexpr (DMA > 7) if (g == 7) dma_b128<7 * 4096>(dbase, doff[7], dst);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -502,21 +524,21 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
     {
       int lf = lane;
       asm volatile("" : "+v"(lf));
-      fa.init(wm * 128, lf);
+      fa.init(wm * 16 * WT, lf);
       fb.init(wn * 16 * WN, lf);
     }
     // K-step 0 complete in LDS (requested above, or before the previous item's epilogue); the
-    // 16 loads of K-step 1 may still be in flight (loads retire in order)
+    // loads of K-step 1 may still be in flight (loads retire in order)
     if (nk > 1) {
-      // vmcnt(8 + NB_LOADS); lgkmcnt and expcnt untouched
-      __builtin_amdgcn_s_waitcnt(0x0f70 | ((8 + NB_LOADS) & 15) | (((8 + NB_LOADS) >> 4) << 14));
+      // vmcnt(NA_LOADS + NB_LOADS); lgkmcnt and expcnt untouched
+      __builtin_amdgcn_s_waitcnt(0x0f70 | ((NA_LOADS + NB_LOADS) & 15) | (((NA_LOADS + NB_LOADS) >> 4) << 14));
     } else {
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       fix_tail(r0, r1);
     }
     __syncthreads();
     {
-      uint32_t aa[FragReader<A_T>::NBASE], ba[FragReader<B_T>::NBASE];
+      uint32_t aa[FragReader<A_T, WT>::NBASE], ba[FragReader<B_T, WT>::NBASE];
       frag_addrs(r0, r1, 0, aa, ba);
 #pragma unroll
       for (int g = 0; g < WT; ++g) {
@@ -527,14 +549,14 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
 
     // K loop.  In K-step t: first half-step computes on X (half 0) while Y is read from the
     // tiles of t (half 1) and A(t+2) is requested into r4, dead since the barrier of K-step
-    // t-1; then every load but those eight must have landed (that is all of K-step t+1), one
+    // t-1; then every load but those must have landed (that is all of K-step t+1), one
     // barrier publishes them and retires the tiles of t; the second half-step computes on Y
     // while X is read from the tiles of t+1 and B(t+2) is requested where A(t) was.
     int t = 0;
     for (; t + 2 < nk; ++t) {
       if (t + 3 == nk && k_tail != BK) set_offsets(k_tail);
-      half(X, Y, r0, r1, 1, Count<8>{}, a_base(t + 2), la, r4);
-      __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8)
+      half(X, Y, r0, r1, 1, Count<NA_LOADS>{}, a_base(t + 2), la, r4);
+      __builtin_amdgcn_s_waitcnt(0x0f70 | NA_LOADS);  // vmcnt(NA_LOADS)
       __syncthreads();
       half(Y, X, r2, r3, 0, Count<NB_LOADS>{}, b_base(t + 2), lb, r0);
       seg_advance();
@@ -576,78 +598,85 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
     // data: program order of its LDS instructions is all the ordering needed.  The accumulators
     // are read in one place for all three kinds of output.
     {
-      const uint32_t stage = r4 + (uint32_t)wave * 8192u;
+      // staged rows: 256 bytes of bf16 (two buffers of 16 rows) or 512 of fp32 (one buffer), half of that for
+      // a small tile, whose waves are 64 columns wide
+      constexpr bool small = WT == WT_SMALL;
+      constexpr uint32_t STAGE = SLOT_BYTES / 4, SBUF = STAGE / 2, ROW16 = SBUF / 16, ROW32 = STAGE / 16;
+      constexpr int XOR16 = small ? 7 : 15;         // a bf16 row has 8 or 16 chunks
+      constexpr int L16 = small ? 8 : 16, Q16 = L16 / 4;   // lanes per stored row, passes per 16-row block: bf16
+      constexpr int L32 = small ? 16 : 32, Q32 = L32 / 4;  // ... and fp32
+      const uint32_t stage = r4 + (uint32_t)wave * STAGE;
       int le = lane;  // opaque copy: nothing derived from it is kept alive through the K loop
       asm volatile("" : "+v"(le));
       const int row16 = le & 15, quad = le >> 4;
-      const int hrow = le >> 5, ch = le & 31;  // read side: row 2q + hrow, columns 4 ch .. + 3
-      const int m_wave = out_m0 + wm * 128, n_wave = out_n0 + wn * 16 * WN;
+      const int hrow = le / L32, ch = le % L32;  // read side, fp32: row (64 / L32) q + hrow, columns 4 ch .. + 3
+      const int m_wave = out_m0 + wm * 16 * WT, n_wave = out_n0 + wn * 16 * WN;
       auto wave_sync = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
       };
-      const bool rows_in = m_wave + 128 <= M;  // wave-uniform: no row of the wave tile is cut off
+      const bool rows_in = m_wave + 16 * WT <= M;  // wave-uniform: no row of the wave tile is cut off
       const bool cols_in = 4 * ch < 16 * WN && n_wave + 4 * ch < N;
       const bool to_partial = out_partial != nullptr;
       const bool add_old = !to_partial && accumulate;
       const int ldo = to_partial ? N : ldc;
-      uint32_t lo[8];
+      uint32_t lo[Q32];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) lo[q] = (uint32_t)((2 * q + hrow) * ldo + 4 * ch);
+      for (int q = 0; q < Q32; ++q) lo[q] = (uint32_t)((64 / L32 * q + hrow) * ldo + 4 * ch);
       // accumulation into C: the old values of a 16-row block are requested one block ahead of
       // the pass that uses them (zeros otherwise).  Positions beyond the matrix read a valid
       // neighbour instead and are never stored back.
-      bf16x4 oldc[2][8];
+      bf16x4 oldc[2][Q32];
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
+      for (int q = 0; q < Q32; ++q)
 #pragma unroll
         for (int e = 0; e < 4; ++e) oldc[0][q][e] = oldc[1][q][e] = (bf16)0.f;
       auto fetch_old = [&](int mt) {
         const bf16* const cb = C + ((int64_t)(m_wave + mt * 16) * ldc + n_wave);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const bool in = cols_in && (rows_in || m_wave + mt * 16 + 2 * q + hrow < M);
+        for (int q = 0; q < Q32; ++q) {
+          const bool in = cols_in && (rows_in || m_wave + mt * 16 + 64 / L32 * q + hrow < M);
           oldc[mt & 1][q] = *reinterpret_cast<const bf16x4*>(in ? cb + lo[q] : C);
         }
       };
       if (add_old) fetch_old(0);
       // bf16 output without accumulation goes through the same place as bf16: 16 rows x 256 bytes
-      // per block, two buffers (so one wave-level fence per block), read side row 4q + quad,
-      // 16-byte chunk rch = eight consecutive columns, 16 lanes per row
+      // per block, two buffers (so one wave-level fence per block), read side row (64 / L16) q + row_r,
+      // 16-byte chunk rch = eight consecutive columns, L16 lanes per row
       const bool narrow = !to_partial && !add_old;
-      const int rch = le & 15;
+      const int rch = le % L16, row_r = le / L16;
       // first column the wave stores to: n_wave, or with SwiGLU column out_n0 of the gate half
       // (wn = 0) or of the up half (wn = 1) of x
       const int n_store = swiglu ? out_n0 + (wn ? gate_up_f : 0) : n_wave;
       const int ncol = 8 * rch;
       const bool ncols_in = 8 * rch < 16 * WN && (swiglu || n_wave + 8 * rch < N);
-      uint32_t nlo[4];
+      uint32_t nlo[Q16];
 #pragma unroll
-      for (int q = 0; q < 4; ++q)   // (a 16-row block starts at a multiple of the run length: rows map inside it)
-        nlo[q] = (uint32_t)((runs.c_sh ? run_off(4 * q + quad, ldc, runs.c_sh, runs.c_outer) : (4 * q + quad) * ldc) + ncol);
+      for (int q = 0; q < Q16; ++q)   // (a 16-row block starts at a multiple of the run length: rows map inside it)
+        nlo[q] = (uint32_t)((runs.c_sh ? run_off(64 / L16 * q + row_r, ldc, runs.c_sh, runs.c_outer) : (64 / L16 * q + row_r) * ldc) + ncol);
       // fused residual: the values to add to a 16-row block are requested one block ahead
       // SwiGLU backward: gate and up values of a 16-row block, requested one block ahead
-      bf16x8 xg[swiglu_bwd ? 2 : 1][swiglu_bwd ? 4 : 1], xu[swiglu_bwd ? 2 : 1][swiglu_bwd ? 4 : 1];
+      bf16x8 xg[swiglu_bwd ? 2 : 1][swiglu_bwd ? Q16 : 1], xu[swiglu_bwd ? 2 : 1][swiglu_bwd ? Q16 : 1];
       auto fetch_x = [&](int mt) {
         const bf16* const xb = aux + ((int64_t)(m_wave + mt * 16) * ld_aux + n_wave + 8 * rch);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int rr = 4 * q + quad;
+        for (int q = 0; q < Q16; ++q) {
+          const int rr = 64 / L16 * q + row_r;
           const bool in = ncols_in && (rows_in || m_wave + mt * 16 + rr < M);
           xg[mt & 1][q] = in ? ldg8(xb + (int64_t)rr * ld_aux) : zero8();
           xu[mt & 1][q] = in ? ldg8(xb + (int64_t)rr * ld_aux + N) : zero8();
         }
       };
       if constexpr (swiglu_bwd) fetch_x(0);
-      bf16x8 resv[epi_add ? 2 : 1][epi_add ? 4 : 1];
+      bf16x8 resv[epi_add ? 2 : 1][epi_add ? Q16 : 1];
       auto fetch_res = [&](int mt) {
         const int r0 = m_wave + mt * 16;
         const bf16* const rb =
             aux + ((runs.x_sh ? (int64_t)(r0 >> runs.x_sh) * runs.x_outer : (int64_t)r0 * ld_aux) + n_wave + 8 * rch);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int rr = 4 * q + quad;
+        for (int q = 0; q < Q16; ++q) {
+          const int rr = 64 / L16 * q + row_r;
           const bool in = ncols_in && (rows_in || m_wave + mt * 16 + rr < M);
           const int64_t ro = runs.x_sh ? (int64_t)run_off(rr, ld_aux, runs.x_sh, runs.x_outer) : (int64_t)rr * ld_aux;
           resv[mt & 1][q] = in ? ldg8(rb + ro) : zero8();
@@ -707,19 +736,19 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
                                                  : (int64_t)(m_wave + mt * 16) * ldo) +
                             (narrow ? n_store : n_wave);
         if (narrow) {
-          const uint32_t buf = stage + (uint32_t)(mt & 1) * 4096u;
+          const uint32_t buf = stage + (uint32_t)(mt & 1) * SBUF;
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt) {
             bf16x4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = (bf16)vals[nt][e];
-            *(KR_LDS bf16x4*)(buf + row16 * 256 + (((2 * nt + (quad >> 1)) ^ row16) << 4) + (quad & 1) * 8) = o;
+            *(KR_LDS bf16x4*)(buf + row16 * ROW16 + (((2 * nt + (quad >> 1)) ^ (row16 & XOR16)) << 4) + (quad & 1) * 8) = o;
           }
           if constexpr (swiglu) __syncthreads(); else wave_sync();  // SwiGLU reads the neighbour wave's block too
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int rr = 4 * q + quad;
-            bf16x8 v = *(KR_LDS const bf16x8*)(buf + rr * 256 + ((rch ^ rr) << 4));
+          for (int q = 0; q < Q16; ++q) {
+            const int rr = 64 / L16 * q + row_r;
+            bf16x8 v = *(KR_LDS const bf16x8*)(buf + rr * ROW16 + ((rch ^ (rr & XOR16)) << 4));
             const bool in = ncols_in && (rows_in || m_wave + mt * 16 + rr < M);
             if constexpr (epi_add) {
 #pragma unroll
@@ -744,16 +773,16 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
           }
           if constexpr (swiglu) {
             // the wave beside this one (same rows, other half of the tile) has staged the other
-            // operand of the activation for the same 16 rows: this wave takes rows 4 q + quad
-            // for q = 2 wn, 2 wn + 1 of the block, reads the gate chunk from the left wave's
+            // operand of the activation for the same 16 rows: this wave takes the rows of the passes
+            // q = Q16 / 2 * wn .. of the block, reads the gate chunk from the left wave's
             // buffer and the up chunk from the right wave's, and stores out2
-            const uint32_t gbuf = r4 + (uint32_t)(2 * wm) * 8192u + (uint32_t)(mt & 1) * 4096u;
-            const uint32_t ubuf = gbuf + 8192u;
+            const uint32_t gbuf = r4 + (uint32_t)(2 * wm) * STAGE + (uint32_t)(mt & 1) * SBUF;
+            const uint32_t ubuf = gbuf + STAGE;
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-              const int rr = 4 * (2 * wn + qq) + quad;
-              const bf16x8 g = *(KR_LDS const bf16x8*)(gbuf + rr * 256 + ((rch ^ rr) << 4));
-              const bf16x8 u = *(KR_LDS const bf16x8*)(ubuf + rr * 256 + ((rch ^ rr) << 4));
+            for (int qq = 0; qq < Q16 / 2; ++qq) {
+              const int rr = 64 / L16 * (Q16 / 2 * wn + qq) + row_r;
+              const bf16x8 g = *(KR_LDS const bf16x8*)(gbuf + rr * ROW16 + ((rch ^ (rr & XOR16)) << 4));
+              const bf16x8 u = *(KR_LDS const bf16x8*)(ubuf + rr * ROW16 + ((rch ^ (rr & XOR16)) << 4));
               bf16x8 y;
 #pragma unroll
               for (int e = 0; e < 8; ++e) y[e] = (bf16)kr_swiglu_f((float)g[e], (float)u[e]);
@@ -764,12 +793,12 @@ __global__ __launch_bounds__(NTHREADS) void gemm_kernel(const bf16* __restrict__
         } else {
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt)
-            *(KR_LDS f32x4*)(stage + row16 * 512 + (((4 * nt + quad) ^ row16) << 4)) = vals[nt];
+            *(KR_LDS f32x4*)(stage + row16 * ROW32 + (((4 * nt + quad) ^ row16) << 4)) = vals[nt];
           wave_sync();
 #pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const int rr = 2 * q + hrow;
-            const f32x4 v = *(KR_LDS const f32x4*)(stage + rr * 512 + ((ch ^ rr) << 4));
+          for (int q = 0; q < Q32; ++q) {
+            const int rr = 64 / L32 * q + hrow;
+            const f32x4 v = *(KR_LDS const f32x4*)(stage + rr * ROW32 + ((ch ^ rr) << 4));
             const bool in = cols_in && (rows_in || m_wave + mt * 16 + rr < M);
             if (to_partial) {
               if (in) *reinterpret_cast<f32x4*>(out_partial + blk + lo[q]) = v;
@@ -857,12 +886,14 @@ inline int choose_wn(int M, int N, int num_cus) {
 // keep its CU-time small (the dispatcher uses latency_weight 0.1).  `max_splits` is what the caller's workspace holds.
 struct Plan {
   int wn, splits;
+  bool small;  // 128 x 128 tiles (wn is 4)
 };
 inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, int max_splits,
-                        int min_wn = 4) {
+                        bool fused = false, bool allow_small = true) {
   constexpr int kItemOverhead = 4;
+  const int min_wn = fused ? 5 : 4;
   const int tiles_m = (M + BM - 1) / BM;
-  if (tiles_m * ((N + BN - 1) / BN) >= 192) return {choose_wn(M, N, num_cus), 1};
+  if (tiles_m * ((N + BN - 1) / BN) >= 192) return {choose_wn(M, N, num_cus), 1, false};
   const double w = latency_weight < 0.f ? 0.0 : (latency_weight > 1.f ? 1.0 : (double)latency_weight);
   const int nk = (K + BK - 1) / BK;
   const double reduce_per_split = (double)M * N * 8.0 / 5.0e12 / 1.3e-6;
@@ -875,13 +906,13 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
     const double cu_time = items * per_item / num_cus + reduce;
     return w * latency + (1.0 - w) * cu_time;
   };
-  Plan best{8, 1};
+  Plan best{8, 1, false};
   double best_cost = cost(8, 1);
   for (int wn = 7; wn >= min_wn; --wn) {
     const double c = cost(wn, 1);
     if (c < best_cost) {
       best_cost = c;
-      best = {wn, 1};
+      best = {wn, 1, false};
     }
   }
   const double unsplit = best_cost;
@@ -890,9 +921,49 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
       const double c = cost(wn, sp);
       if (c < unsplit * 0.95 && c < best_cost) {  // a split must pay for itself clearly
         best_cost = c;
-        best = {wn, sp};
+        best = {wn, sp, false};
       }
     }
+  if (!allow_small) return best;
+  // 128 x 128 tiles (half the matrix work per byte read, but four times the work items, a quarter of the
+  // epilogue in each, and two workgroups per compute unit to hide each other's waits).  Measured K-steps: 0.5 us
+  // (0.38 units) with a unit to itself, 0.88 us when every unit holds two, in between when some do; 3 units around
+  // the K loop; a split's extra launch 2 units.  Against them the large tiles' measured rates (their
+  // estimate above, which ranks them among themselves, is 20 % high in the K loop; a fused epilogue costs a large
+  // tile 4 units more).  Measured, large -> small tiles, us: 512 tokens of the 8B shard: fc1 with SwiGLU 65.3 ->
+  // 34.8, out-projection with the residual 22.2 -> 11.1, fc2 49.0 -> 31.3, its input gradient with the SwiGLU
+  // backward 62.9 -> 36.1; 256 x 512 x 512 with the residual 17.4 -> 8.2; 4096 x 1024 x 4096 (NN) 44.0 -> 33.8.
+  // On the other side of the line: 4096 x 1536 x 4096 45.1 -> 48.7, 1536 x 4096 x 7168 (NN) 80.2 -> 87.8,
+  // 1536 tokens of fc1 with SwiGLU 73.0 -> 94.6, 16384 x 512 x 2048 29.2 -> 30.4.
+  constexpr double kAlone = 0.38, kPaired = 0.68, kOverhead = 3, kSplit = 2, kLargeRate = 0.8, kFusedLarge = 4;
+  double large;
+  {
+    const int items = tiles_m * ((N + 32 * best.wn - 1) / (32 * best.wn)) * best.splits;
+    const int rounds = (items + num_cus - 1) / num_cus;
+    const double per_item = (double)((nk + best.splits - 1) / best.splits) * (best.wn + 2) / 10.0 * kLargeRate +
+                            kItemOverhead + (fused ? kFusedLarge : 0.0);
+    const double reduce = best.splits > 1 ? best.splits * reduce_per_split + kSplit : 0.0;
+    large = w * rounds * per_item + (1.0 - w) * items * per_item / num_cus + reduce;
+  }
+  const int small_tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  auto small_cost = [&](int sp) {
+    const int items = small_tiles * sp, steps = (nk + sp - 1) / sp;
+    const double paired = steps * kPaired + kOverhead;
+    const double reduce = sp > 1 ? sp * reduce_per_split + kSplit : 0.0;
+    const int full = items / (2 * num_cus), rest = items % (2 * num_cus);
+    double latency = full * paired;
+    if (rest > num_cus) latency += steps * (kAlone + (kPaired - kAlone) * (rest - num_cus) / num_cus) + kOverhead;
+    else if (rest > 0) latency += steps * kAlone + kOverhead;
+    return w * latency + (1.0 - w) * items * paired / (2 * num_cus) + reduce;
+  };
+  double small_best = large * 0.93;  // the change must be clear
+  for (int sp = 1; sp == 1 || (sp <= 16 && sp <= max_splits && nk / sp >= 8); ++sp) {
+    const double c = small_cost(sp);
+    if (c < small_best) {
+      small_best = c;
+      best = {4, sp, true};
+    }
+  }
   return best;
 }
 
@@ -930,20 +1001,21 @@ using GemmKernel = void (*)(const bf16*, int, const bf16*, int, bf16*, int, int,
                             const bf16*, int, bf16*, int, RowRuns, Segments);
 
 // raises the dynamic-LDS limit of one kernel instance, once (thread-safe static initialisation)
-template <GemmKernel FN>
+template <GemmKernel FN, size_t LDS_BYTES>
 hipError_t raise_lds_limit() {
   static const hipError_t status = hipFuncSetAttribute((const void*)FN, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)(NSLOTS * TILE * sizeof(bf16)));
+                                                       (int)LDS_BYTES);
   return status;
 }
 
-template <bool A_T, bool B_T, int WN, int EPI = KR_GEMM_EPI_NONE>
+template <bool A_T, bool B_T, int WN, int EPI = KR_GEMM_EPI_NONE, int WT = WT_LARGE>
 int launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, bf16* C, int64_t ldc, int M,
            int N, int K, int accumulate, float* workspace, size_t workspace_bytes,
            hipStream_t stream, int num_cus, const Fused& fu, int planned_splits = 1) {
-  constexpr size_t lds_bytes = NSLOTS * TILE * sizeof(bf16);
+  constexpr size_t lds_bytes = NSLOTS * kSlotBytes<WT>;
+  if (WT == WT_SMALL && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
   if (fu.max_cus > 0 && fu.max_cus < num_cus) num_cus = fu.max_cus;
-  const int tiles = ((M + BM - 1) / BM) * ((N + 32 * WN - 1) / (32 * WN));
+  const int tiles = ((M + 32 * WT - 1) / (32 * WT)) * ((N + 32 * WN - 1) / (32 * WN));
   // the planned count, which the dispatcher has already capped by what the caller's workspace holds
   int splits = planned_splits;
   const size_t one = (size_t)M * N * sizeof(float);
@@ -953,7 +1025,7 @@ int launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, bf16* C, int6
     splits = (int)(workspace_bytes / one);
   }
   if (splits < 2 || (int64_t)splits * M * N >= ((int64_t)1 << 31)) splits = 1;
-  // at most one persistent workgroup per compute unit (a workgroup owns a whole CU's LDS)
+  // at most one persistent workgroup per compute unit (a workgroup owns a whole CU's LDS; small tiles: half)
   // Items are spread evenly: with r = ceil(items / CUs) rounds, ceil(items / r) workgroups (rounded
   // up to a multiple of 8, which keeps item ids and XCDs aligned) finish at the same time as one
   // workgroup per CU would, and the CUs left over are free for other streams' kernels from the
@@ -976,24 +1048,24 @@ int launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, bf16* C, int6
   constexpr bool kSegsRunsInstance = kSegsInstance && EPI == KR_GEMM_EPI_NONE;
   if ((with_runs && !kRunsInstance) || (with_segs && !kSegsInstance) || (with_segs && with_runs && !kSegsRunsInstance))
     return KR_EUNSUPPORTED;
-  GemmKernel fn = gemm_kernel<A_T, B_T, WN, EPI>;
-  hipError_t attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI>>();
+  GemmKernel fn = gemm_kernel<A_T, B_T, WN, EPI, false, false, WT>;
+  hipError_t attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, false, WT>, lds_bytes>();
   if constexpr (kRunsInstance) {
     if (with_runs) {
-      fn = gemm_kernel<A_T, B_T, WN, EPI, true>;
-      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true>>();
+      fn = gemm_kernel<A_T, B_T, WN, EPI, true, false, WT>;
+      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, false, WT>, lds_bytes>();
     }
   }
   if constexpr (kSegsInstance) {
     if (with_segs && !with_runs) {
-      fn = gemm_kernel<A_T, B_T, WN, EPI, false, true>;
-      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, true>>();
+      fn = gemm_kernel<A_T, B_T, WN, EPI, false, true, WT>;
+      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, true, WT>, lds_bytes>();
     }
   }
   if constexpr (kSegsRunsInstance) {
     if (with_segs && with_runs) {
-      fn = gemm_kernel<A_T, B_T, WN, EPI, true, true>;
-      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, true>>();
+      fn = gemm_kernel<A_T, B_T, WN, EPI, true, true, WT>;
+      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, true, WT>, lds_bytes>();
     }
   }
   if (attr_status != hipSuccess) return KR_ELAUNCH;
@@ -1120,11 +1192,14 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
     if (max_splits < 1) max_splits = 1;
   }
   // beside other streams the compute-unit time of the launch counts, hardly its latency
-  const Plan plan = choose_plan(M, N, K, fu.shared ? 0.1f : 1.f, cus, max_splits, fu.epi == KR_GEMM_EPI_NONE ? 4 : 5);
+  const Plan plan = choose_plan(M, N, K, fu.shared ? 0.1f : 1.f, cus, max_splits, fu.epi != KR_GEMM_EPI_NONE,
+                                fu.epi != KR_GEMM_EPI_SWIGLU || N % 128 == 0);
   const int wn = fu.epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn;
   const int sp = plan.splits;
   if (fu.epi == KR_GEMM_EPI_SWIGLU_BWD) {
     if (lda < K || ldb < N) return KR_EINVAL;
+    if (plan.small)
+      return launch<false, true, 4, KR_GEMM_EPI_SWIGLU_BWD, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu);
 #define KR_GEMM_SWIGLU_BWD(W) \
   return launch<false, true, W, KR_GEMM_EPI_SWIGLU_BWD>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu)
     switch (wn) {
@@ -1140,6 +1215,8 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
 #define KR_GEMM_FUSED(W, E) \
   return launch<false, false, W, E>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu)
     if (fu.epi == KR_GEMM_EPI_SWIGLU) {
+      if (plan.small)
+        return launch<false, false, 4, KR_GEMM_EPI_SWIGLU, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu);
       switch (wn) {
         case 5: KR_GEMM_FUSED(5, KR_GEMM_EPI_SWIGLU);
         case 6: KR_GEMM_FUSED(6, KR_GEMM_EPI_SWIGLU);
@@ -1147,6 +1224,8 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
         default: KR_GEMM_FUSED(8, KR_GEMM_EPI_SWIGLU);
       }
     }
+    if (plan.small)
+      return launch<false, false, 4, KR_GEMM_EPI_ADD, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu);
     switch (wn) {
       case 5: KR_GEMM_FUSED(5, KR_GEMM_EPI_ADD);
       case 6: KR_GEMM_FUSED(6, KR_GEMM_EPI_ADD);
@@ -1156,6 +1235,8 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
 #undef KR_GEMM_FUSED
   }
 #define KR_GEMM_LAUNCH(AT, BT)                                                                           \
+  if (plan.small)                                                                                        \
+    return launch<AT, BT, 4, KR_GEMM_EPI_NONE, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
   switch (wn) {                                                                                          \
     case 4: return launch<AT, BT, 4>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
     case 5: return launch<AT, BT, 5>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \

@@ -276,6 +276,32 @@ def test_gemm_plan_does_not_change_the_sums_much(be):
             assert rel(acc, ref + c0.float()) <= TOL
 
 
+@pytest.mark.parametrize("m,n,k", [(8, 8, 8), (128, 128, 64), (136, 264, 72), (120, 128, 128), (520, 1024, 200),
+                                   (512, 3584, 1024),     # one round of small tiles, more than one per compute unit
+                                   (2048, 3456, 136)])    # 432 small tiles
+def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
+    """Outputs of few tiles are computed in 128 x 128 tiles.  A launch held to one compute unit takes the large
+    tiles; every element is the same chain of matrix instructions in both, so the bits are the same."""
+    x, w, dy = rnd(m, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(m, n, seed=63)
+    for layout, a, b, shape in ((0, x, w, (m, n, k)), (1, dy, w, (m, k, n)), (2, dy, x, (n, k, m))):
+        one = dict(split_k=None, max_cus=1)
+        got = be.gemm(layout, a, b, *shape, split_k=None)
+        assert torch.equal(got, be.gemm(layout, a, b, *shape, **one))
+        base = rnd(shape[0], shape[1], seed=64)
+        assert torch.equal(be.gemm(layout, a, b, *shape, out=base.clone(), accumulate=True, split_k=None),
+                           be.gemm(layout, a, b, *shape, out=base.clone(), accumulate=True, **one))
+        wide = torch.zeros(shape[0], shape[1] + 8, device=DEV, dtype=torch.bfloat16)
+        be.gemm(layout, a, b, *shape, out=wide[:, :shape[1]], split_k=None)
+        assert torch.equal(wide[:, :shape[1]], got) and not wide[:, shape[1]:].any()
+    assert rel(be.linear_fwd(x, w), x.float() @ w.float().t()) <= TOL
+    res = rnd(m, n, seed=65)
+    assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(x, w, residual=res, max_cus=1))
+    if be.can_fuse_swiglu(n):
+        y, y1 = (torch.empty(m, n // 2, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        assert torch.equal(be.linear_fwd(x, w, swiglu_out=y), be.linear_fwd(x, w, swiglu_out=y1, max_cus=1))
+        assert torch.equal(y, y1)
+
+
 def test_gemm_is_reproducible(be):
     """No atomics and a fixed order of accumulation: repeated launches give the same bits (a
     race on an LDS tile between the waves of a workgroup would show up here)."""
