@@ -60,7 +60,11 @@ constexpr int WT_LARGE = 8, WT_SMALL = 4;
 constexpr int NTHREADS = 256;
 template <int WT>
 constexpr uint32_t kSlotBytes = 32 * WT * BK * sizeof(bf16);  // one operand tile (either layout)
-constexpr int NSLOTS = 5;          // 5 x 32 KB = the whole 160 KB of LDS (5 x 16 KB: half of it)
+// DEPTH: how many K-steps ahead a tile is requested; the ring has 2 * DEPTH + 1 slots.  2: 5 x 32 KB = the whole
+// 160 KB of LDS (5 x 16 KB: half of it).  4, for small tiles that have a compute unit to themselves: 9 x 16 KB.
+constexpr int kDepth = 2, kDepthAlone = 4;
+// s_waitcnt immediate for vmcnt(n); lgkmcnt and expcnt untouched
+constexpr int vm_wait(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int kXcds = 8;
 constexpr int KR_GEMM_EPI_TRANSPOSED_OUT = 100;  // internal: not part of the C ABI's epilogue values
 constexpr int kGroupM = 4;
@@ -255,8 +259,9 @@ struct Count { static constexpr int value = N; };
 // extra address arithmetic or its registers.
 // SEG (layout NT): A and B are the pieces named by `segs` (the A / B arguments are unused); K is their
 // total length.
-template <bool A_T, bool B_T, int WN, int EPI, bool RUNS = false, bool SEG = false, int WT = WT_LARGE>
-__global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(const bf16* __restrict__ A, int lda,
+template <bool A_T, bool B_T, int WN, int EPI, bool RUNS = false, bool SEG = false, int WT = WT_LARGE,
+          int DEPTH = kDepth>
+__global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1) void gemm_kernel(const bf16* __restrict__ A, int lda,
                                                         const bf16* __restrict__ B, int ldb,
                                                         bf16* __restrict__ C, int ldc, int M,
                                                         int N, int K, int accumulate, int k_per,
@@ -265,6 +270,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
                                                         bf16* __restrict__ out2, int ld_out2,
                                                         RowRuns runs_arg, Segments segs) {
   static_assert(!SEG || (A_T && B_T), "operand pieces: layout NT");
+  static_assert(DEPTH == kDepth || (DEPTH == kDepthAlone && WT == WT_SMALL), "ring depths");
   static_assert(WT == WT_LARGE || (WT == WT_SMALL && WN == 4 && EPI != KR_GEMM_EPI_TRANSPOSED_OUT), "tile shapes");
   constexpr int TW = 32 * WT;  // operand rows an LDS tile holds (a B tile may use fewer)
   constexpr uint32_t SLOT_BYTES = kSlotBytes<WT>;
@@ -364,14 +370,19 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
     }
   };
 
-  // The ring of five 32 KB slots as LDS byte addresses, in ring order starting at A of the
-  // current K-step t: r0 = A(t), r1 = B(t), r2 = A(t+1), r3 = B(t+1), r4 = A(t+2); B(t+2) goes
+  // The ring slots as LDS byte addresses, in ring order starting at A of the current K-step t:
+  // ring[0] = A(t), ring[1] = B(t), ring[2] = A(t+1), .., ring[2 DEPTH] = A(t+DEPTH); B(t+DEPTH) goes
   // where A(t) was.  Rotated by two positions per K-step.
-  uint32_t r0 = smem_b, r1 = smem_b + SLOT_BYTES, r2 = smem_b + 2 * SLOT_BYTES,
-           r3 = smem_b + 3 * SLOT_BYTES, r4 = smem_b + 4 * SLOT_BYTES;
+  constexpr int NSLOTS = 2 * DEPTH + 1;
+  uint32_t ring[NSLOTS];
+#pragma unroll
+  for (int i = 0; i < NSLOTS; ++i) ring[i] = smem_b + i * SLOT_BYTES;
   auto rotate = [&]() {
-    const uint32_t o0 = r0, o1 = r1;
-    r0 = r2; r1 = r3; r2 = r4; r3 = o0; r4 = o1;
+    const uint32_t o0 = ring[0], o1 = ring[1];
+#pragma unroll
+    for (int i = 0; i + 2 < NSLOTS; ++i) ring[i] = ring[i + 2];
+    ring[NSLOTS - 2] = o0;
+    ring[NSLOTS - 1] = o1;
   };
 
   // accumulators live in the accumulation registers (the MFMAs are written as inline assembly
@@ -402,17 +413,17 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
     if constexpr (COUNT > 6) dma_b128<6 * 4096>(base, off[6], dst);
     if constexpr (COUNT > 7) dma_b128<7 * 4096>(base, off[7], dst);
   };
-  // K-steps 0 and 1 of the current item into r0..r3
-  auto request_first_two = [&]() {
+  // the first DEPTH K-steps of the current item into ring[0 .. 2 DEPTH - 1]
+  auto request_first = [&]() {
     set_offsets(nk == 1 ? k_tail : BK);
-    request(a_base(0), la, r0, Count<NA_LOADS>{});
-    request(b_base(0), lb, r1, Count<NB_LOADS>{});
-    seg_advance();
-    if (nk > 1) {
-      if (nk == 2 && k_tail != BK) set_offsets(k_tail);
-      request(a_base(1), la, r2, Count<NA_LOADS>{});
-      request(b_base(1), lb, r3, Count<NB_LOADS>{});
-      seg_advance();
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      if (d < nk) {
+        if (d > 0 && d + 1 == nk && k_tail != BK) set_offsets(k_tail);
+        request(a_base(d), la, ring[2 * d], Count<NA_LOADS>{});
+        request(b_base(d), lb, ring[2 * d + 1], Count<NB_LOADS>{});
+        seg_advance();
+      }
     }
   };
   // After this wave's loads of the last K-step have landed (A in slot sa, B in slot sb): zero
@@ -512,7 +523,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
   const int total_items = ntiles * (split_k ? splits : 1);
   int item = blockIdx.x;
   select_item(item);
-  request_first_two();
+  request_first();
   // the accumulators start at zero: here for the first item (behind the latency of its first
   // loads), in the epilogue for every later one (behind its LDS round trips)
 #pragma unroll
@@ -528,18 +539,22 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
       fb.init(wn * 16 * WN, lf);
     }
     // K-step 0 complete in LDS (requested above, or before the previous item's epilogue); the
-    // loads of K-step 1 may still be in flight (loads retire in order)
-    if (nk > 1) {
-      // vmcnt(NA_LOADS + NB_LOADS); lgkmcnt and expcnt untouched
-      __builtin_amdgcn_s_waitcnt(0x0f70 | ((NA_LOADS + NB_LOADS) & 15) | (((NA_LOADS + NB_LOADS) >> 4) << 14));
+    // loads of the K-steps behind it may still be in flight (loads retire in order)
+    constexpr int STEP_LOADS = NA_LOADS + NB_LOADS;
+    if (nk >= DEPTH) {
+      __builtin_amdgcn_s_waitcnt(vm_wait((DEPTH - 1) * STEP_LOADS));
+    } else if (DEPTH > 2 && nk == 3) {
+      __builtin_amdgcn_s_waitcnt(vm_wait(2 * STEP_LOADS));
+    } else if (DEPTH > 2 && nk == 2) {
+      __builtin_amdgcn_s_waitcnt(vm_wait(STEP_LOADS));
     } else {
-      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-      fix_tail(r0, r1);
+      __builtin_amdgcn_s_waitcnt(vm_wait(0));
+      fix_tail(ring[0], ring[1]);
     }
     __syncthreads();
     {
       uint32_t aa[FragReader<A_T, WT>::NBASE], ba[FragReader<B_T, WT>::NBASE];
-      frag_addrs(r0, r1, 0, aa, ba);
+      frag_addrs(ring[0], ring[1], 0, aa, ba);
 #pragma unroll
       for (int g = 0; g < WT; ++g) {
         X.a[g] = read_a(aa, g, 0);
@@ -548,32 +563,36 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
     }
 
     // K loop.  In K-step t: first half-step computes on X (half 0) while Y is read from the
-    // tiles of t (half 1) and A(t+2) is requested into r4, dead since the barrier of K-step
-    // t-1; then every load but those must have landed (that is all of K-step t+1), one
-    // barrier publishes them and retires the tiles of t; the second half-step computes on Y
-    // while X is read from the tiles of t+1 and B(t+2) is requested where A(t) was.
+    // tiles of t (half 1) and A(t+DEPTH) is requested into the last slot, dead since the barrier of
+    // K-step t-1; then all of K-step t+1 must have landed (what may be in flight are the K-steps
+    // behind it and that A), one barrier publishes it and retires the tiles of t; the second
+    // half-step computes on Y while X is read from the tiles of t+1 and B(t+DEPTH) is requested
+    // where A(t) was.
     int t = 0;
-    for (; t + 2 < nk; ++t) {
-      if (t + 3 == nk && k_tail != BK) set_offsets(k_tail);
-      half(X, Y, r0, r1, 1, Count<NA_LOADS>{}, a_base(t + 2), la, r4);
-      __builtin_amdgcn_s_waitcnt(0x0f70 | NA_LOADS);  // vmcnt(NA_LOADS)
+    for (; t + DEPTH < nk; ++t) {
+      if (t + DEPTH + 1 == nk && k_tail != BK) set_offsets(k_tail);
+      half(X, Y, ring[0], ring[1], 1, Count<NA_LOADS>{}, a_base(t + DEPTH), la, ring[NSLOTS - 1]);
+      __builtin_amdgcn_s_waitcnt(vm_wait((DEPTH - 2) * STEP_LOADS + NA_LOADS));
       __syncthreads();
-      half(Y, X, r2, r3, 0, Count<NB_LOADS>{}, b_base(t + 2), lb, r0);
+      half(Y, X, ring[2], ring[3], 0, Count<NB_LOADS>{}, b_base(t + DEPTH), lb, ring[0]);
       seg_advance();
       rotate();
     }
     for (; t < nk; ++t) {
-      half(X, Y, r0, r1, 1, Count<0>{}, nullptr, la, 0u);
-      __builtin_amdgcn_s_waitcnt(0x0f70);
-      if (t + 2 == nk) fix_tail(r2, r3);
+      half(X, Y, ring[0], ring[1], 1, Count<0>{}, nullptr, la, 0u);
+      // (at most DEPTH - 1 K-steps are left behind this one)
+      if (DEPTH > 2 && t + 4 == nk) __builtin_amdgcn_s_waitcnt(vm_wait(2 * STEP_LOADS));
+      else if (DEPTH > 2 && t + 3 == nk) __builtin_amdgcn_s_waitcnt(vm_wait(STEP_LOADS));
+      else __builtin_amdgcn_s_waitcnt(vm_wait(0));
+      if (t + 2 == nk) fix_tail(ring[2], ring[3]);
       __syncthreads();
       // (after the last K-step this reads tiles that do not exist: unused)
-      half(Y, X, r2, r3, 0, Count<0>{}, nullptr, lb, 0u);
+      half(Y, X, ring[2], ring[3], 0, Count<0>{}, nullptr, lb, 0u);
       rotate();
     }
 
-    // Every LDS read of this item that matters finished before the last barrier, so slots
-    // r0..r3 are free: request the first two K-steps of the next item now and let them fly
+    // Every LDS read of this item that matters finished before the last barrier, so all
+    // slots are free: request the first K-steps of the next item now and let them fly
     // during the epilogue.
     const int out_m0 = m0, out_n0 = n0;
     float* const out_partial = split_k ? partial + p_off : nullptr;
@@ -581,7 +600,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
     const bool more = next < total_items;
     if (more) {
       select_item(next);
-      request_first_two();
+      request_first();
     }
     // the compiler does not know the MFMAs' latency: let the last ones finish before their
     // results are read
@@ -589,8 +608,8 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
 
     // Epilogue.  A lane holds C[m][n..n+3] for m = 16 mt + lane%16, n = 16 nt + 4 (lane/16):
     // stored from there, every instruction would scatter 64 small pieces over 16 rows.  Instead
-    // each wave transposes through its own 8 KB of slot r4 (idle until K-step 2 of the next
-    // item is requested, after the next workgroup barrier): a block of 16 rows x 128 columns
+    // each wave transposes through its own quarter of the last slot (idle until K-step DEPTH of the
+    // next item is requested, after the next workgroup barrier): a block of 16 rows x 128 columns
     // goes in as fp32 from the MFMA layout and comes out as whole rows (32 lanes per row, four
     // consecutive columns per lane), so a store instruction writes complete row segments of
     // 256 bytes (bf16 output) or 512 bytes (fp32 partial tiles); accumulation into C adds the
@@ -605,7 +624,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
       constexpr int XOR16 = small ? 7 : 15;         // a bf16 row has 8 or 16 chunks
       constexpr int L16 = small ? 8 : 16, Q16 = L16 / 4;   // lanes per stored row, passes per 16-row block: bf16
       constexpr int L32 = small ? 16 : 32, Q32 = L32 / 4;  // ... and fp32
-      const uint32_t stage = r4 + (uint32_t)wave * STAGE;
+      const uint32_t stage = ring[NSLOTS - 1] + (uint32_t)wave * STAGE;
       int le = lane;  // opaque copy: nothing derived from it is kept alive through the K loop
       asm volatile("" : "+v"(le));
       const int row16 = le & 15, quad = le >> 4;
@@ -776,7 +795,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL ? 2 : 1) void gemm_kernel(
             // operand of the activation for the same 16 rows: this wave takes the rows of the passes
             // q = Q16 / 2 * wn .. of the block, reads the gate chunk from the left wave's
             // buffer and the up chunk from the right wave's, and stores out2
-            const uint32_t gbuf = r4 + (uint32_t)(2 * wm) * STAGE + (uint32_t)(mt & 1) * SBUF;
+            const uint32_t gbuf = ring[NSLOTS - 1] + (uint32_t)(2 * wm) * STAGE + (uint32_t)(mt & 1) * SBUF;
             const uint32_t ubuf = gbuf + STAGE;
 #pragma unroll
             for (int qq = 0; qq < Q16 / 2; ++qq) {
@@ -926,23 +945,23 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
     }
   if (!allow_small) return best;
   // 128 x 128 tiles (half the matrix work per byte read, but four times the work items, a quarter of the
-  // epilogue in each, and two workgroups per compute unit to hide each other's waits).  Measured K-steps: 0.5 us
-  // (0.38 units) with a unit to itself, 0.88 us when every unit holds two, in between when some do; 3 units around
-  // the K loop; a split's extra launch 2 units.  Against them the large tiles' measured rates (their
+  // epilogue in each, and two workgroups per compute unit to hide each other's waits).  Measured K-steps: 0.43 us
+  // (0.33 units) with a unit to itself, 0.88 us when every unit holds two, in between when some do; 3 units around
+  // the K loop; a split's extra launch 2 units (5 for a large tile, whose fp32 partials leave in one burst).  Against them the large tiles' measured rates (their
   // estimate above, which ranks them among themselves, is 20 % high in the K loop; a fused epilogue costs a large
   // tile 4 units more).  Measured, large -> small tiles, us: 512 tokens of the 8B shard: fc1 with SwiGLU 65.3 ->
   // 34.8, out-projection with the residual 22.2 -> 11.1, fc2 49.0 -> 31.3, its input gradient with the SwiGLU
   // backward 62.9 -> 36.1; 256 x 512 x 512 with the residual 17.4 -> 8.2; 4096 x 1024 x 4096 (NN) 44.0 -> 33.8.
   // On the other side of the line: 4096 x 1536 x 4096 45.1 -> 48.7, 1536 x 4096 x 7168 (NN) 80.2 -> 87.8,
   // 1536 tokens of fc1 with SwiGLU 73.0 -> 94.6, 16384 x 512 x 2048 29.2 -> 30.4.
-  constexpr double kAlone = 0.38, kPaired = 0.68, kOverhead = 3, kSplit = 2, kLargeRate = 0.8, kFusedLarge = 4;
+  constexpr double kAlone = 0.33, kPaired = 0.68, kOverhead = 3, kSplit = 2, kSplitLarge = 5, kLargeRate = 0.8, kFusedLarge = 4;
   double large;
   {
     const int items = tiles_m * ((N + 32 * best.wn - 1) / (32 * best.wn)) * best.splits;
     const int rounds = (items + num_cus - 1) / num_cus;
     const double per_item = (double)((nk + best.splits - 1) / best.splits) * (best.wn + 2) / 10.0 * kLargeRate +
                             kItemOverhead + (fused ? kFusedLarge : 0.0);
-    const double reduce = best.splits > 1 ? best.splits * reduce_per_split + kSplit : 0.0;
+    const double reduce = best.splits > 1 ? best.splits * reduce_per_split + kSplitLarge : 0.0;
     large = w * rounds * per_item + (1.0 - w) * items * per_item / num_cus + reduce;
   }
   const int small_tiles = ((M + 127) / 128) * ((N + 127) / 128);
@@ -1012,7 +1031,8 @@ template <bool A_T, bool B_T, int WN, int EPI = KR_GEMM_EPI_NONE, int WT = WT_LA
 int launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, bf16* C, int64_t ldc, int M,
            int N, int K, int accumulate, float* workspace, size_t workspace_bytes,
            hipStream_t stream, int num_cus, const Fused& fu, int planned_splits = 1) {
-  constexpr size_t lds_bytes = NSLOTS * kSlotBytes<WT>;
+  size_t lds_bytes = 0;
+  const int one_per_cu = fu.max_cus > 0 && fu.max_cus < num_cus ? fu.max_cus : num_cus;
   if (WT == WT_SMALL && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
   if (fu.max_cus > 0 && fu.max_cus < num_cus) num_cus = fu.max_cus;
   const int tiles = ((M + 32 * WT - 1) / (32 * WT)) * ((N + 32 * WN - 1) / (32 * WN));
@@ -1048,26 +1068,45 @@ int launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, bf16* C, int6
   constexpr bool kSegsRunsInstance = kSegsInstance && EPI == KR_GEMM_EPI_NONE;
   if ((with_runs && !kRunsInstance) || (with_segs && !kSegsInstance) || (with_segs && with_runs && !kSegsRunsInstance))
     return KR_EUNSUPPORTED;
-  GemmKernel fn = gemm_kernel<A_T, B_T, WN, EPI, false, false, WT>;
-  hipError_t attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, false, WT>, lds_bytes>();
-  if constexpr (kRunsInstance) {
-    if (with_runs) {
-      fn = gemm_kernel<A_T, B_T, WN, EPI, true, false, WT>;
-      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, false, WT>, lds_bytes>();
+  GemmKernel fn = nullptr;
+  hipError_t attr_status = hipSuccess;
+  auto pick = [&](auto depth_tag) {
+    constexpr int DEPTH = decltype(depth_tag)::value;
+    constexpr size_t LDS = (2 * DEPTH + 1) * kSlotBytes<WT>;
+    lds_bytes = LDS;
+    fn = gemm_kernel<A_T, B_T, WN, EPI, false, false, WT, DEPTH>;
+    attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, false, WT, DEPTH>, LDS>();
+    if constexpr (kRunsInstance) {
+      if (with_runs) {
+        fn = gemm_kernel<A_T, B_T, WN, EPI, true, false, WT, DEPTH>;
+        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, false, WT, DEPTH>, LDS>();
+      }
     }
-  }
-  if constexpr (kSegsInstance) {
-    if (with_segs && !with_runs) {
-      fn = gemm_kernel<A_T, B_T, WN, EPI, false, true, WT>;
-      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, true, WT>, lds_bytes>();
+    if constexpr (kSegsInstance) {
+      if (with_segs && !with_runs) {
+        fn = gemm_kernel<A_T, B_T, WN, EPI, false, true, WT, DEPTH>;
+        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, true, WT, DEPTH>, LDS>();
+      }
     }
-  }
-  if constexpr (kSegsRunsInstance) {
-    if (with_segs && with_runs) {
-      fn = gemm_kernel<A_T, B_T, WN, EPI, true, true, WT>;
-      attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, true, WT>, lds_bytes>();
+    if constexpr (kSegsRunsInstance) {
+      if (with_segs && with_runs) {
+        fn = gemm_kernel<A_T, B_T, WN, EPI, true, true, WT, DEPTH>;
+        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, true, WT, DEPTH>, LDS>();
+      }
     }
+  };
+  bool deep = false;
+  if constexpr (WT == WT_SMALL) {
+    // A small tile that has its compute unit to itself waits for memory: a K-step lasts 0.5 us there, two of
+    // them are less than a load from HBM takes.  The deep ring asks four ahead.  Operands in HBM, two -> four
+    // ahead, us: 512 tokens of the 8B shard's fc1 51.4 -> 40.2, fc2 46.0 -> 37.9, fc2's input gradient 51.3 ->
+    // 44.3; 4096 x 1024 x 4096 (NT) 49.4 -> 41.1.  Up to 8 K-steps the longer prologue costs more than it
+    // hides (1536 x 512 x 256 6.3 -> 6.9, 4096 x 1024 x 512 8.7 -> 9.0).  Not beside other streams, whose
+    // workgroups can share the unit with a launch that leaves them half of the LDS.
+    deep = tiles * splits <= one_per_cu && !fu.shared && (K / BK) / splits > 8;
+    if (deep) pick(Count<kDepthAlone>{});
   }
+  if (!deep) pick(Count<kDepth>{});
   if (attr_status != hipSuccess) return KR_ELAUNCH;
   const Segments segs = with_segs ? *fu.segs : Segments{};
   if (splits == 1) {

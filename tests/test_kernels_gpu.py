@@ -277,6 +277,7 @@ def test_gemm_plan_does_not_change_the_sums_much(be):
 
 
 @pytest.mark.parametrize("m,n,k", [(8, 8, 8), (128, 128, 64), (136, 264, 72), (120, 128, 128), (520, 1024, 200),
+                                   (264, 136, 584), (136, 640, 720), (256, 1000, 1096),   # the deep ring, contraction tails
                                    (512, 3584, 1024),     # one round of small tiles, more than one per compute unit
                                    (2048, 3456, 136)])    # 432 small tiles
 def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
