@@ -571,7 +571,7 @@ class HipBackend:
     def rope_fused_inplace(self, fused: Tensor, per: int, freqs: Tensor, backward: bool) -> None:
         """Rotate the query and key heads of a fused QKV buffer [s, b, ng, per+2, hd] in place
         (one launch); the value heads are left untouched."""
-        if self._n.rope_fused(fused, freqs, backward):
+        if self._n.rope_fused(fused, per, freqs, backward):
             return
         s, b, ng, slots, hd = fused.shape
         if slots != per + 2 or not fused.is_contiguous():

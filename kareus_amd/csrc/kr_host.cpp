@@ -348,18 +348,20 @@ PyObject* py_rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // ---- rotary embedding on a fused QKV buffer, in place ------------------------------------------------------
-// rope_fused(fused [s, b, ng, per + 2, hd], freqs [.., hd] fp32 (>= s rows), backward) -> True
+// rope_fused(fused [s, b, ng, per + 2, hd], per, freqs [rows >= s, 1.., hd] fp32, backward) -> True
 PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
-    if (n_args != 3 || !bf16_arg(a[0]) || !f32_arg(a[1])) return none();
-    const Tensor &f = tensor(a[0]), &fr = tensor(a[1]);
-    if (f.dim() != 5 || !f.is_contiguous() || !fr.is_contiguous() || fr.size(-1) != f.size(4) ||
-        fr.numel() < f.size(0) * f.size(4))
+    if (n_args != 4 || !bf16_arg(a[0]) || !f32_arg(a[2])) return none();
+    const Tensor &f = tensor(a[0]), &fr = tensor(a[2]);
+    const int64_t per = PyLong_AsLong(a[1]);
+    // (the table is one row per position: a dimension between the rows and the channels has to be a 1)
+    if (f.dim() != 5 || !f.is_contiguous() || f.size(3) != per + 2 || fr.dim() < 2 || !fr.is_contiguous() ||
+        fr.size(-1) != f.size(4) || fr.numel() != fr.size(0) * f.size(4) || fr.size(0) < f.size(0))
       return none();
     const int64_t s = f.size(0), b = f.size(1), slots = f.size(3), heads = f.size(2) * slots, hd = f.size(4);
     if (!fits_int(s) || !fits_int(b) || !fits_int(heads)) return none();
     const int rc = kr_rope(ptr(f), ptr(f), (const float*)ptr(fr), (int)s, (int)b, (int)heads, (int)hd, b * heads * hd,
-                           heads * hd, hd, b * heads * hd, heads * hd, hd, PyObject_IsTrue(a[2]) == 1, (int)slots,
+                           heads * hd, hd, b * heads * hd, heads * hd, hd, PyObject_IsTrue(a[3]) == 1, (int)slots,
                            (int)slots - 1, stream());
     if (rc != KR_OK) return failed("kr_rope", rc);
     Py_RETURN_TRUE;

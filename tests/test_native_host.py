@@ -47,3 +47,31 @@ def test_calls_leave_other_tensors_to_the_python_side():
     assert n.gemm(0, x, x, 8, 8, 8, None, False, 1, None, None, None, 0) is None
     assert n.rmsnorm_fwd(x, x[0], 1e-5) is None and n.attn_fwd(x, x, x, 1.0, 0) is None
     assert n.dropout_bwd(x, x, 1.0) is None and n.wgrad_segments([x], [x], None, False, 1, 0) is None
+
+
+# ------------------------------------------------- what the Python side refuses, the native side leaves to it
+def _on_device(*shape, dtype=torch.bfloat16):
+    """A tensor of the device in all but its memory: a call that takes it ends before any launch."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        return torch.empty(*shape, dtype=dtype, device="cuda")
+
+
+def _backend():
+    be = HipBackend.__new__(HipBackend)          # without the kernel library: nothing here may get as far
+    be._n = load_native()
+    return be
+
+
+def test_a_rotary_call_with_the_wrong_group_size_or_table_is_refused():
+    fused, table = _on_device(6, 2, 3, 6, 16), _on_device(6, 1, 1, 16, dtype=torch.float32)
+    be = _backend()
+    with pytest.raises(RuntimeError, match=r"contiguous \[s, b, ng, per\+2, hd\]"):
+        be.rope_fused_inplace(fused, 3, table, False)
+    with pytest.raises(RuntimeError, match="shape|size"):        # two rows of angles per position
+        be.rope_fused_inplace(fused, 4, _on_device(6, 1, 2, 16, dtype=torch.float32), False)
+    # (the right ones are taken: with no device here, that shows as the runtime's error)
+    if not torch.cuda.is_available():
+        with pytest.raises(RuntimeError, match="HIP"):
+            be._n.rope_fused(fused, 4, table, False)
