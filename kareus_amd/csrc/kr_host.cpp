@@ -58,7 +58,7 @@ PyObject* guarded(F&& f) {
 // ---- operands the kernels address in place ------------------------------------------------------------
 // A matrix [rows, cols] with one row stride, or the [s, r, cols] slice of a [s, b, cols] tensor whose rows
 // come in runs of r (see "Row runs" in kareus_hip.h); tensors of more dimensions count when their leading
-// ones merge.
+// ones merge, which is for the callers that would otherwise copy them: the others take max_dims.
 struct Operand {
   int64_t rows = 0, cols = 0, ld = 0;
   int run_rows = 1;
@@ -67,10 +67,10 @@ struct Operand {
 };
 constexpr int64_t kMaxRunRows = 16;
 
-Operand operand(const Tensor& t, int64_t max_run_rows = kMaxRunRows) {
+Operand operand(const Tensor& t, int64_t max_run_rows = kMaxRunRows, int64_t max_dims = 64) {
   Operand o;
   const int64_t d = t.dim();
-  if (d < 2 || t.stride(d - 1) != 1 || t.numel() == 0) return o;
+  if (d < 2 || d > max_dims || t.stride(d - 1) != 1 || t.numel() == 0) return o;
   o.cols = t.size(d - 1);
   // merge the leading dimensions from the inside out
   int64_t rows = 1, ld = 0;
@@ -86,7 +86,8 @@ Operand operand(const Tensor& t, int64_t max_run_rows = kMaxRunRows) {
     rows *= t.size(i);
   }
   if (merged) {
-    if (rows == 1) ld = (o.cols + 7) / 8 * 8;
+    // (the stride of one row says nothing; a caller that is strict about dimensions passes a matrix's on as it is)
+    if (rows == 1) ld = max_dims <= 3 && d == 2 ? t.stride(0) : (o.cols + 7) / 8 * 8;
     if (ld % 8 || ld < o.cols) return o;
     o.rows = rows;
     o.ld = ld;
@@ -103,6 +104,10 @@ Operand operand(const Tensor& t, int64_t max_run_rows = kMaxRunRows) {
   o.ok = true;
   return o;
 }
+
+// the operand of a call that refuses what is neither a matrix nor a [s, r, cols] tensor / not a matrix
+Operand operand3(const Tensor& t) { return operand(t, kMaxRunRows, 3); }
+Operand operand2(const Tensor& t) { return operand(t, 1, 2); }
 
 Tensor matrix(int64_t rows, int64_t cols, const Tensor& like) { return at::empty({rows, cols}, like.options()); }
 Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
@@ -163,9 +168,9 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       if (!absent(p) && !bf16_arg(p)) return none();
     if (!absent(p_res) + !absent(p_act) + !absent(p_pre) > 1) return none();
     const Tensor &ta = tensor(a[1]), &tb = tensor(a[2]);
-    const Operand oa = operand(ta);
-    const Operand ob = operand(tb);
-    if (!oa.ok || !ob.ok || ob.run_rows > 1) return none();
+    const Operand oa = operand3(ta);
+    const Operand ob = operand2(tb);
+    if (!oa.ok || !ob.ok) return none();
     const bool a_t = layout == KR_GEMM_NT, b_t = layout != KR_GEMM_TN;
     if (layout < KR_GEMM_TN || layout > KR_GEMM_NT || oa.rows != (a_t ? k : m) || oa.cols != (a_t ? m : k) ||
         ob.rows != (b_t ? k : n) || ob.cols != (b_t ? n : k) || !fits_int(m) || !fits_int(n) || !fits_int(k))
@@ -177,7 +182,7 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     int64_t ld_out2 = 0;
     int64_t out_cols = n;
     if (!absent(p_res)) {
-      ox = operand(tensor(p_res));
+      ox = operand3(tensor(p_res));
       if (!ox.ok || ox.rows != m || ox.cols != n) return none();
       epi = KR_GEMM_EPI_ADD;
       aux = ptr(tensor(p_res));
@@ -197,7 +202,7 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     if (accumulate && absent(p_out)) return none();
     Tensor out = absent(p_out) ? matrix(m, out_cols, ta) : tensor(p_out);
-    const Operand oc = operand(out);
+    const Operand oc = operand3(out);
     if (!oc.ok || oc.rows != m || oc.cols != out_cols) return none();
     Tensor ws;
     size_t ws_bytes = 0;
@@ -236,8 +241,10 @@ PyObject* py_wgrad_segments(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     for (Py_ssize_t i = 0; i < nseg; ++i) {
       PyObject *dy = PyList_GET_ITEM(a[0], i), *x = PyList_GET_ITEM(a[1], i);
       if (!bf16_arg(dy) || !bf16_arg(x)) return none();
-      const Operand oa = operand(tensor(dy)), ob = operand(tensor(x));
-      if (!oa.ok || !ob.ok || ob.run_rows > 1 || oa.rows != ob.rows || oa.rows % 64) return none();
+      const Operand oa = operand3(tensor(dy)), ob = operand3(tensor(x));
+      if (!oa.ok || !ob.ok || ob.run_rows > 1 || oa.rows != ob.rows || oa.rows % 64 ||
+          tensor(x).device() != tensor(dy).device())
+        return none();
       if (i == 0) {
         fa = oa, fb = ob;
       } else if (oa.rows != fa.rows || oa.ld != fa.ld || oa.run_rows != fa.run_rows || oa.run_ld != fa.run_ld ||
@@ -254,8 +261,8 @@ PyObject* py_wgrad_segments(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor& like = tensor(PyList_GET_ITEM(a[0], 0));
     if (absent(a[2]) ? accumulate : !bf16_arg(a[2])) return none();
     Tensor out = absent(a[2]) ? matrix(m, n, like) : tensor(a[2]);
-    const Operand oc = operand(out);
-    if (!oc.ok || oc.run_rows > 1 || oc.rows != m || oc.cols != n) return none();
+    const Operand oc = operand2(out);
+    if (!oc.ok || oc.rows != m || oc.cols != n) return none();
     Tensor ws;
     size_t ws_bytes = split ? gemm_workspace(KR_GEMM_NT, (int)m, (int)n, (int)k, split == 1) : 0;
     if (ws_bytes) ws = bytes(ws_bytes, like);
@@ -303,8 +310,8 @@ PyObject* py_rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
     if (n_args != 7 || !bf16_arg(a[0]) || !bf16_arg(a[1]) || !f32_arg(a[2])) return none();
     const Tensor &dy = tensor(a[0]), &x = tensor(a[1]), &rstd = tensor(a[2]);
-    const Operand od = operand(dy), ox = operand(x);
-    if (!od.ok || od.run_rows > 1 || !ox.ok || od.rows != ox.rows || od.cols != ox.cols || !fits_int(ox.rows) ||
+    const Operand od = operand2(dy), ox = operand(x);
+    if (!od.ok || !ox.ok || od.rows != ox.rows || od.cols != ox.cols || !fits_int(ox.rows) ||
         !is_gamma(a[3], ox.cols) || !rstd.is_contiguous() || rstd.numel() != ox.rows)
       return none();
     Operand orr, oc;
@@ -315,7 +322,7 @@ PyObject* py_rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     if (!absent(a[5]) && !bf16_arg(a[5])) return none();
     Tensor dx = absent(a[5]) ? matrix(ox.rows, ox.cols, x) : tensor(a[5]);
-    oc = operand(dx);
+    oc = operand3(dx);
     if (!oc.ok || oc.rows != ox.rows || oc.cols != ox.cols) return none();
     const int rows = (int)ox.rows, cols = (int)ox.cols;
     Tensor dgamma, ws;

@@ -50,12 +50,12 @@ def test_calls_leave_other_tensors_to_the_python_side():
 
 
 # ------------------------------------------------- what the Python side refuses, the native side leaves to it
-def _on_device(*shape, dtype=torch.bfloat16):
+def _on_device(*shape, dtype=torch.bfloat16, device="cuda"):
     """A tensor of the device in all but its memory: a call that takes it ends before any launch."""
     from torch._subclasses.fake_tensor import FakeTensorMode
 
     with FakeTensorMode():
-        return torch.empty(*shape, dtype=dtype, device="cuda")
+        return torch.empty(*shape, dtype=dtype, device=device)
 
 
 def _backend():
@@ -75,3 +75,27 @@ def test_a_rotary_call_with_the_wrong_group_size_or_table_is_refused():
     if not torch.cuda.is_available():
         with pytest.raises(RuntimeError, match="HIP"):
             be._n.rope_fused(fused, 4, table, False)
+
+
+def _refused():
+    d, f = _on_device, torch.float32
+    a, b, deep = d(16, 64), d(32, 64), lambda n: d(2, 2, n // 4, 64)
+    return {
+        "gemm: B of three dimensions": lambda n: n.gemm(0, a, d(2, 16, 64), 16, 32, 64, None, False, 1, None, None, None, 0),
+        "gemm: A of four": lambda n: n.gemm(0, deep(16), b, 16, 32, 64, None, False, 1, None, None, None, 0),
+        "gemm: residual of four": lambda n: n.gemm(0, a, d(64, 64), 16, 64, 64, None, False, 1, deep(16), None, None, 0),
+        "gemm: output of four": lambda n: n.gemm(0, a, d(64, 64), 16, 64, 64, deep(16), False, 1, None, None, None, 0),
+        "gemm: one row without a row stride": lambda n: n.gemm(0, d(64).expand(1, 64).as_strided((1, 64), (0, 1)), b, 1, 32, 64,
+                                                               None, False, 1, None, None, None, 0),
+        "wgrad: output of three": lambda n: n.wgrad_segments([d(64, 16)], [d(64, 32)], d(1, 16, 32), False, 1, 0),
+        "wgrad: pieces of four": lambda n: n.wgrad_segments([d(2, 2, 16, 16)], [d(64, 32)], None, False, 1, 0),
+        "wgrad: a pair on two devices": lambda n: n.wgrad_segments([d(64, 16)], [d(64, 32, device="cuda:1")], None, False, 1, 0),
+        "rmsnorm: dy of three": lambda n: n.rmsnorm_bwd(d(4, 4, 64), a, d(16, dtype=f), d(64), None, None, None),
+        "rmsnorm: dx of four": lambda n: n.rmsnorm_bwd(a, a, d(16, dtype=f), d(64), None, deep(16), None),
+    }
+
+
+@pytest.mark.parametrize("what", sorted(_refused()))
+def test_operands_the_python_side_refuses_are_left_to_it(what):
+    """(What the Python side copies or views, tensors of more dimensions among it, the native side may take.)"""
+    assert _refused()[what](load_native()) is None
