@@ -641,6 +641,23 @@ class HipBackend:
             raise RuntimeError(f"dropout_add: shapes differ, {tuple(x.shape)} vs {tuple(residual.shape)}")
         if not 0.0 <= p < 1.0:
             raise RuntimeError(f"dropout_add: probability {p} is outside [0, 1)")
+        rows = x.shape[0] if x.dim() > 1 else 1
+        o2 = None
+        if out is None:
+            fits = x.numel() // max(rows, 1) % 8 == 0
+        else:
+            self._dev(out)
+            self._bf16(out)
+            if out.shape != x.shape:
+                raise RuntimeError(f"dropout_add: out has shape {tuple(out.shape)}, operands {tuple(x.shape)}")
+            try:
+                o2 = out.view(rows, -1)
+            except (RuntimeError, ValueError):   # (a tensor without memory words it as the latter)
+                pass
+            fits = o2 is not None and o2.stride(1) == 1 and o2.stride(0) % 8 == 0 and o2.stride(0) >= o2.shape[1]
+        if not fits:
+            raise RuntimeError("dropout_add: out cannot be addressed with a single row stride")
+        # (behind the checks: a call that is refused draws nothing)
         seed = int(torch.randint(0, 1 << 62, (1,), dtype=torch.int64).item())
         done = self._n.dropout_add(x, residual, p, out, seed)
         if done is not None:
@@ -648,17 +665,7 @@ class HipBackend:
         x2, r2 = self._rows(self._leading_rows(x)), self._rows(self._leading_rows(residual))
         if out is None:
             out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        else:
-            self._dev(out)
-            self._bf16(out)
-            if out.shape != x.shape:
-                raise RuntimeError(f"dropout_add: out has shape {tuple(out.shape)}, operands {tuple(x.shape)}")
-        try:
             o2 = out.view(x2.shape)
-        except RuntimeError:
-            o2 = None
-        if o2 is None or o2.stride(1) != 1 or o2.stride(0) % 8 or o2.stride(0) < o2.shape[1]:
-            raise RuntimeError("dropout_add: out cannot be addressed with a single row stride")
         rows, cols = x2.shape
         mask = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
         self._check(self.lib.kr_dropout_add(x2.data_ptr(), x2.stride(0), r2.data_ptr(), r2.stride(0), o2.data_ptr(),

@@ -99,3 +99,20 @@ def _refused():
 def test_operands_the_python_side_refuses_are_left_to_it(what):
     """(What the Python side copies or views, tensors of more dimensions among it, the native side may take.)"""
     assert _refused()[what](load_native()) is None
+
+
+def _bad_outs():
+    d = _on_device
+    return [(d(4, 2, 64), d(4, 2, 32)), (d(4, 2, 64), d(2, 4, 64).transpose(0, 1)), (d(4, 2, 64), d(4, 2, 72)[..., :64]),
+            (d(4, 64), d(4, 68)[:, :64]), (d(3, 4), None), (d(4, 64), torch.empty(4, 64))]
+
+
+@pytest.mark.parametrize("i", range(len(_bad_outs())))
+def test_a_refused_dropout_draws_no_seed(i):
+    """Shapes and strides of ``out`` that cannot be addressed: the CPU generator stays where it was, so the masks of the
+    calls that follow are those of a run without the refused one."""
+    x, out = _bad_outs()[i]
+    before = torch.get_rng_state()
+    with pytest.raises(RuntimeError, match="dropout_add|hip backend"):
+        _backend().dropout_add(x, x, 0.5, out=out)
+    assert torch.equal(torch.get_rng_state(), before)
