@@ -225,7 +225,11 @@ class HipBackend:
     # launch runs beside other streams' kernels (KR_GEMM_BESIDE_OTHER_STREAMS): the workspace is sized with
     # the same weight, so the cuts the dispatcher plans are the cuts the buffer holds
     SHARED_LATENCY_WEIGHT = 0.1
-    _SPLIT_CODE = {None: 0, True: 1, False: 2}   # ``split_k`` as the native side takes it
+
+    @staticmethod
+    def _split_code(split_k) -> int:
+        """``split_k`` as the native side takes it."""
+        return 0 if split_k is None else 1 if split_k else 2
 
     def _workspace(self, nbytes: int, device) -> Tensor:
         """A workspace of at least ``nbytes`` for the current stream.  One buffer per (stream, size
@@ -255,8 +259,8 @@ class HipBackend:
             reserved = reserved_compute_units()
             if reserved:
                 max_cus = max(self._num_cus(a.device) - reserved, 8)
-        done = self._n.gemm(layout, a, b, m, n, k, out, accumulate, self._SPLIT_CODE[split_k], residual, swiglu_out,
-                            swiglu_bwd_x, max_cus)
+        done = self._n.gemm(layout, a, b, m, n, k, out, accumulate, self._split_code(split_k), residual, swiglu_out,
+                            swiglu_bwd_x, int(max_cus))
         if done is not None:
             return done
         self._dev(a, b)
@@ -391,7 +395,7 @@ class HipBackend:
         reserved = reserved_compute_units()
         if reserved:
             max_cus = max(self._num_cus(dys[0].device) - reserved, 8)
-        done = self._n.wgrad_segments(dys, xs, out, accumulate, self._SPLIT_CODE[split_k], max_cus)
+        done = self._n.wgrad_segments(dys, xs, out, accumulate, self._split_code(split_k), max_cus)
         if done is not None:
             return done
         if not self.wgrad_segments_ok(dys, xs):

@@ -45,6 +45,29 @@ PyObject* failed(const std::string& what, int rc) {
   return nullptr;
 }
 
+// numbers: what Python cannot convert ends the call with Python's error, before anything is launched
+struct PythonError : std::exception {};
+int64_t integer(PyObject* o) {
+  const int64_t v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) throw PythonError();
+  return v;
+}
+double real(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw PythonError();
+  return v;
+}
+uint64_t seed_value(PyObject* o) {
+  const uint64_t v = PyLong_AsUnsignedLongLong(o);
+  if (v == (uint64_t)-1 && PyErr_Occurred()) throw PythonError();
+  return v;
+}
+bool truth(PyObject* o) {
+  const int v = PyObject_IsTrue(o);
+  if (v < 0) throw PythonError();
+  return v == 1;
+}
+
 template <typename F>
 PyObject* guarded(F&& f) {
   try {
@@ -119,7 +142,7 @@ PyObject* py_rows_view(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (n_args != 2 || !is_tensor(a[0])) return none();
     PyObject* t = a[0];
     const Tensor& x = tensor(t);
-    const Operand o = operand(x, PyLong_AsLong(a[1]));
+    const Operand o = operand(x, integer(a[1]));
     if (!o.ok) return none();
     if (x.dim() == 2 || o.run_rows > 1) return Py_NewRef(t);
     return wrap(x.as_strided({o.rows, o.cols}, {o.ld, 1}, x.storage_offset()));
@@ -157,11 +180,11 @@ bool fits_int(int64_t v) { return v > 0 && v < ((int64_t)1 << 31); }
 PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
     if (n_args != 13) return none();
-    const int layout = (int)PyLong_AsLong(a[0]);
-    const int64_t m = PyLong_AsLong(a[3]), n = PyLong_AsLong(a[4]), k = PyLong_AsLong(a[5]);
-    const bool accumulate = PyObject_IsTrue(a[7]) == 1;
-    const int split = (int)PyLong_AsLong(a[8]);
-    const int max_cus = (int)PyLong_AsLong(a[12]);
+    const int layout = (int)integer(a[0]);
+    const int64_t m = integer(a[3]), n = integer(a[4]), k = integer(a[5]);
+    const bool accumulate = truth(a[7]);
+    const int split = (int)integer(a[8]);
+    const int max_cus = (int)integer(a[12]);
     PyObject *p_out = a[6], *p_res = a[9], *p_act = a[10], *p_pre = a[11];
     if (!bf16_arg(a[1]) || !bf16_arg(a[2])) return none();
     for (PyObject* p : {p_out, p_res, p_act, p_pre})
@@ -256,8 +279,8 @@ PyObject* py_wgrad_segments(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     const int64_t m = fa.cols, n = fb.cols, k = fa.rows * nseg;
     if (!fits_int(m) || !fits_int(n) || !fits_int(k)) return none();
-    const bool accumulate = PyObject_IsTrue(a[3]) == 1;
-    const int split = (int)PyLong_AsLong(a[4]), max_cus = (int)PyLong_AsLong(a[5]);
+    const bool accumulate = truth(a[3]);
+    const int split = (int)integer(a[4]), max_cus = (int)integer(a[5]);
     const Tensor& like = tensor(PyList_GET_ITEM(a[0], 0));
     if (absent(a[2]) ? accumulate : !bf16_arg(a[2])) return none();
     Tensor out = absent(a[2]) ? matrix(m, n, like) : tensor(a[2]);
@@ -290,7 +313,7 @@ PyObject* py_rmsnorm_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor& x = tensor(a[0]);
     const Operand o = operand(x);
     if (!o.ok || !is_gamma(a[1], o.cols) || !fits_int(o.rows)) return none();
-    const float eps = (float)PyFloat_AsDouble(a[2]);
+    const float eps = (float)real(a[2]);
     Tensor y = matrix(o.rows, o.cols, x);
     Tensor rstd = at::empty({o.rows}, x.options().dtype(at::kFloat));
     const void* g = ptr(tensor(a[1]));
@@ -360,7 +383,8 @@ PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
     if (n_args != 4 || !bf16_arg(a[0]) || !f32_arg(a[2])) return none();
     const Tensor &f = tensor(a[0]), &fr = tensor(a[2]);
-    const int64_t per = PyLong_AsLong(a[1]);
+    const int64_t per = integer(a[1]);
+    const bool backward = truth(a[3]);
     // (the table is one row per position: a dimension between the rows and the channels has to be a 1)
     if (f.dim() != 5 || !f.is_contiguous() || f.size(3) != per + 2 || fr.dim() < 2 || !fr.is_contiguous() ||
         fr.size(-1) != f.size(4) || fr.numel() != fr.size(0) * f.size(4) || fr.size(0) < f.size(0))
@@ -368,7 +392,7 @@ PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t s = f.size(0), b = f.size(1), slots = f.size(3), heads = f.size(2) * slots, hd = f.size(4);
     if (!fits_int(s) || !fits_int(b) || !fits_int(heads)) return none();
     const int rc = kr_rope(ptr(f), ptr(f), (const float*)ptr(fr), (int)s, (int)b, (int)heads, (int)hd, b * heads * hd,
-                           heads * hd, hd, b * heads * hd, heads * hd, hd, PyObject_IsTrue(a[3]) == 1, (int)slots,
+                           heads * hd, hd, b * heads * hd, heads * hd, hd, backward, (int)slots,
                            (int)slots - 1, stream());
     if (rc != KR_OK) return failed("kr_rope", rc);
     Py_RETURN_TRUE;
@@ -381,7 +405,7 @@ PyObject* py_split_qkv(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
     if (n_args != 4 || !is_tensor(a[0])) return none();
     const Tensor& m = tensor(a[0]);
-    const int64_t ng = PyLong_AsLong(a[1]), per = PyLong_AsLong(a[2]), hd = PyLong_AsLong(a[3]);
+    const int64_t ng = integer(a[1]), per = integer(a[2]), hd = integer(a[3]);
     if (m.dim() != 3 || !m.is_contiguous() || m.size(2) != ng * (per + 2) * hd) return none();
     const int64_t s = m.size(0), b = m.size(1), w = m.size(2), g = (per + 2) * hd, off = m.storage_offset();
     PyObject* q = wrap(m.as_strided({s, b, ng, per, hd}, {b * w, w, g, hd, 1}, off));
@@ -429,8 +453,8 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]);
     const AttnShape c = attn_shape(q, k, v);
     if (!c.ok) return none();
-    const float scale = (float)PyFloat_AsDouble(a[3]);
-    const int flags = (int)PyLong_AsLong(a[4]);
+    const float scale = (float)real(a[3]);
+    const int flags = (int)integer(a[4]);
     Tensor o = at::empty({c.s, c.b, c.nq, c.hd}, q.options());
     Tensor lse = at::empty({c.b, c.nq, c.s}, q.options().dtype(at::kFloat));
     Tensor ws;
@@ -461,8 +485,8 @@ PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         dout.numel() != (int64_t)c.s * c.b * c.nq * c.hd || o.numel() != dout.numel() ||
         lse.numel() != (int64_t)c.b * c.nq * c.s)
       return none();
-    const float scale = (float)PyFloat_AsDouble(a[6]);
-    const int flags = (int)PyLong_AsLong(a[7]);
+    const float scale = (float)real(a[6]);
+    const int flags = (int)integer(a[7]);
     const int64_t s = c.s, b = c.b, ng = c.nkv, hd = c.hd, g = (c.per + 2) * hd, w = ng * g;
     Tensor fused = at::empty({s, b, ng, c.per + 2, hd}, q.options());
     Tensor dq = fused.as_strided({s, b, ng, c.per, hd}, {b * w, w, g, hd, 1}, 0);
@@ -494,14 +518,15 @@ PyObject* py_dropout_add(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Operand ox = operand(x), orr = operand(r);
     if (!ox.ok || ox.run_rows > 1 || !orr.ok || orr.run_rows > 1) return none();
     if (!absent(a[3]) && (!bf16_arg(a[3]) || tensor(a[3]).sizes() != x.sizes())) return none();
-    const double p = PyFloat_AsDouble(a[2]);
+    const double p = real(a[2]);
     if (!(p >= 0.0 && p < 1.0)) return none();
+    const uint64_t seed = seed_value(a[4]);
     Tensor out = absent(a[3]) ? at::empty(x.sizes(), x.options()) : tensor(a[3]);
     const Operand oc = operand(out);
     if (!oc.ok || oc.run_rows > 1) return none();
     Tensor mask = at::empty(x.sizes(), x.options().dtype(at::kByte));
     const int rc = kr_dropout_add(ptr(x), ox.ld, ptr(r), orr.ld, ptr(out), oc.ld, ptr(mask), ox.rows, (int)ox.cols, (float)p,
-                                  (uint64_t)PyLong_AsUnsignedLongLong(a[4]), 0, stream());
+                                  seed, 0, stream());
     if (rc != KR_OK) return failed("kr_dropout_add", rc);
     PyObject* po = absent(a[3]) ? wrap(std::move(out)) : Py_NewRef(a[3]);
     PyObject* pm = wrap(std::move(mask));
@@ -516,9 +541,9 @@ PyObject* py_dropout_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor &dy = tensor(a[0]), &mask = tensor(a[1]);
     const Operand o = operand(dy);
     if (!o.ok || o.run_rows > 1 || mask.sizes() != dy.sizes() || !mask.is_contiguous()) return none();
+    const float scale = (float)real(a[2]);
     Tensor dx = at::empty(dy.sizes(), dy.options());
-    const int rc = kr_dropout_bwd(ptr(dy), o.ld, ptr(mask), ptr(dx), o.cols, o.rows, (int)o.cols,
-                                  (float)PyFloat_AsDouble(a[2]), stream());
+    const int rc = kr_dropout_bwd(ptr(dy), o.ld, ptr(mask), ptr(dx), o.cols, o.rows, (int)o.cols, scale, stream());
     if (rc != KR_OK) return failed("kr_dropout_bwd", rc);
     return wrap(std::move(dx));
   });

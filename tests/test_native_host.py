@@ -116,3 +116,24 @@ def test_a_refused_dropout_draws_no_seed(i):
     with pytest.raises(RuntimeError, match="dropout_add|hip backend"):
         _backend().dropout_add(x, x, 0.5, out=out)
     assert torch.equal(torch.get_rng_state(), before)
+
+
+def test_a_number_python_cannot_convert_ends_the_call_with_its_error():
+    n, x = load_native(), torch.zeros(4, 2, 16)
+    for call in (lambda: n.rows_view(x, "16"), lambda: n.split_qkv(x, None, 2, 4),
+                 lambda: n.gemm(0, _on_device(8, 8), _on_device(8, 8), None, 8, 8, None, False, 1, None, None, None, 0)):
+        with pytest.raises(TypeError):
+            call()
+
+
+def test_split_and_budget_may_be_any_truth_value_and_any_number():
+    class Seen:
+        def gemm(self, *args):
+            self.args = args
+            return "done"
+
+    be, x = _backend(), torch.zeros(8, 8)
+    be._n = Seen()
+    for split, code in ((None, 0), (True, 1), (2, 1), (False, 2), (0, 2)):
+        assert be.gemm(0, x, x, 8, 8, 8, split_k=split, max_cus=16.0) == "done"
+        assert be._n.args[8] == code and type(be._n.args[12]) is int
