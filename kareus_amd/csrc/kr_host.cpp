@@ -9,8 +9,9 @@
 // Every function takes the case it was written for — bf16 tensors on the device, operands the kernels
 // address in place, shapes that fit together — and answers None to anything else; the caller then goes
 // through the backend's general Python path, which copies what has to be copied and words the errors.  A
-// code other than KR_OK from the library raises.  Nothing is kept between calls except how much workspace a
-// GEMM shape asks for, which is a pure function of its sizes.
+// code other than KR_OK from the library raises.  From the first allocation to the launch the interpreter is
+// free for other threads.  Nothing is kept between calls except how much workspace a GEMM shape asks for,
+// which is a pure function of its sizes.
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
@@ -67,6 +68,13 @@ bool truth(PyObject* o) {
   if (v < 0) throw PythonError();
   return v == 1;
 }
+
+// From the first allocation to the launch the interpreter is free for other threads: an allocation may have to
+// wait for the device to give cached blocks back, and a launch for room in a full queue.
+struct WithoutInterpreter {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~WithoutInterpreter() { PyEval_RestoreThread(state); }
+};
 
 template <typename F>
 PyObject* guarded(F&& f) {
@@ -224,25 +232,36 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       out_cols = 2 * n;
     }
     if (accumulate && absent(p_out)) return none();
-    Tensor out = absent(p_out) ? matrix(m, out_cols, ta) : tensor(p_out);
-    const Operand oc = operand3(out);
-    if (!oc.ok || oc.rows != m || oc.cols != out_cols) return none();
-    Tensor ws;
-    size_t ws_bytes = 0;
-    if (epi == KR_GEMM_EPI_NONE && split != 0 && oc.run_rows == 1) {
-      ws_bytes = gemm_workspace(layout, (int)m, (int)n, (int)k, split == 1);
-      if (ws_bytes) ws = bytes(ws_bytes, ta);
-    }
-    int rc;
-    void* ws_ptr = ws_bytes ? ptr(ws) : nullptr;
-    const int epilogue = epi | (split == 2 ? KR_GEMM_BESIDE_OTHER_STREAMS : 0);
-    if (oa.run_rows > 1 || oc.run_rows > 1 || ox.run_rows > 1) {
-      rc = kr_gemm_bf16_runs(layout, (int)m, (int)n, (int)k, ptr(ta), oa.ld, oa.run_rows, oa.run_ld, ptr(tb), ob.ld,
-                             ptr(out), oc.ld, oc.run_rows, oc.run_ld, accumulate, epilogue, aux, ox.ld, ox.run_rows,
-                             ox.run_ld, out2, ld_out2, max_cus, ws_ptr, ws_bytes, stream());
+    Tensor out;
+    Operand oc;
+    if (absent(p_out)) {
+      if (out_cols % 8) return none();
+      oc.rows = m, oc.cols = oc.ld = out_cols;
     } else {
-      rc = kr_gemm_bf16_fused(layout, (int)m, (int)n, (int)k, ptr(ta), oa.ld, ptr(tb), ob.ld, ptr(out), oc.ld,
-                              accumulate, epilogue, aux, ox.ld, out2, ld_out2, max_cus, ws_ptr, ws_bytes, stream());
+      out = tensor(p_out);
+      oc = operand3(out);
+      if (!oc.ok || oc.rows != m || oc.cols != out_cols) return none();
+    }
+    const int epilogue = epi | (split == 2 ? KR_GEMM_BESIDE_OTHER_STREAMS : 0);
+    int rc;
+    {
+      WithoutInterpreter free;
+      if (!out.defined()) out = matrix(m, out_cols, ta);
+      Tensor ws;
+      size_t ws_bytes = 0;
+      if (epi == KR_GEMM_EPI_NONE && split != 0 && oc.run_rows == 1) {
+        ws_bytes = gemm_workspace(layout, (int)m, (int)n, (int)k, split == 1);
+        if (ws_bytes) ws = bytes(ws_bytes, ta);
+      }
+      void* ws_ptr = ws_bytes ? ptr(ws) : nullptr;
+      if (oa.run_rows > 1 || oc.run_rows > 1 || ox.run_rows > 1) {
+        rc = kr_gemm_bf16_runs(layout, (int)m, (int)n, (int)k, ptr(ta), oa.ld, oa.run_rows, oa.run_ld, ptr(tb), ob.ld,
+                               ptr(out), oc.ld, oc.run_rows, oc.run_ld, accumulate, epilogue, aux, ox.ld, ox.run_rows,
+                               ox.run_ld, out2, ld_out2, max_cus, ws_ptr, ws_bytes, stream());
+      } else {
+        rc = kr_gemm_bf16_fused(layout, (int)m, (int)n, (int)k, ptr(ta), oa.ld, ptr(tb), ob.ld, ptr(out), oc.ld,
+                                accumulate, epilogue, aux, ox.ld, out2, ld_out2, max_cus, ws_ptr, ws_bytes, stream());
+      }
     }
     if (rc != KR_OK)
       return failed("kr_gemm_bf16(layout=" + std::to_string(layout) + ", M=" + std::to_string(m) + ", N=" +
@@ -260,6 +279,7 @@ PyObject* py_wgrad_segments(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Py_ssize_t nseg = PyList_GET_SIZE(a[0]);
     if (nseg < 1 || nseg > KR_GEMM_MAX_SEGMENTS || PyList_GET_SIZE(a[1]) != nseg) return none();
     const void *pa[KR_GEMM_MAX_SEGMENTS], *pb[KR_GEMM_MAX_SEGMENTS];
+    Tensor held[2 * KR_GEMM_MAX_SEGMENTS];  // the lists may change while the interpreter is free
     Operand fa, fb;
     for (Py_ssize_t i = 0; i < nseg; ++i) {
       PyObject *dy = PyList_GET_ITEM(a[0], i), *x = PyList_GET_ITEM(a[1], i);
@@ -274,25 +294,36 @@ PyObject* py_wgrad_segments(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
                  ob.ld != fb.ld || oa.cols != fa.cols || ob.cols != fb.cols) {
         return none();
       }
-      pa[i] = ptr(tensor(dy));
-      pb[i] = ptr(tensor(x));
+      held[2 * i] = tensor(dy);
+      held[2 * i + 1] = tensor(x);
     }
     const int64_t m = fa.cols, n = fb.cols, k = fa.rows * nseg;
     if (!fits_int(m) || !fits_int(n) || !fits_int(k)) return none();
     const bool accumulate = truth(a[3]);
     const int split = (int)integer(a[4]), max_cus = (int)integer(a[5]);
-    const Tensor& like = tensor(PyList_GET_ITEM(a[0], 0));
     if (absent(a[2]) ? accumulate : !bf16_arg(a[2])) return none();
-    Tensor out = absent(a[2]) ? matrix(m, n, like) : tensor(a[2]);
-    const Operand oc = operand2(out);
-    if (!oc.ok || oc.rows != m || oc.cols != n) return none();
-    Tensor ws;
-    size_t ws_bytes = split ? gemm_workspace(KR_GEMM_NT, (int)m, (int)n, (int)k, split == 1) : 0;
-    if (ws_bytes) ws = bytes(ws_bytes, like);
-    const int rc = kr_gemm_bf16_nt_segments((int)m, (int)n, (int)fa.rows, (int)nseg, pa, fa.ld, fa.run_rows, fa.run_ld, pb,
-                                            fb.ld, ptr(out), oc.ld, accumulate,
-                                            split == 2 ? KR_GEMM_BESIDE_OTHER_STREAMS : 0, max_cus,
-                                            ws_bytes ? ptr(ws) : nullptr, ws_bytes, stream());
+    Tensor out;
+    Operand oc;
+    if (absent(a[2])) {
+      if (n % 8) return none();
+      oc.ld = n;
+    } else {
+      out = tensor(a[2]);
+      oc = operand2(out);
+      if (!oc.ok || oc.rows != m || oc.cols != n) return none();
+    }
+    int rc;
+    {
+      WithoutInterpreter free;
+      if (!out.defined()) out = matrix(m, n, held[0]);
+      const size_t ws_bytes = split ? gemm_workspace(KR_GEMM_NT, (int)m, (int)n, (int)k, split == 1) : 0;
+      Tensor ws;
+      if (ws_bytes) ws = bytes(ws_bytes, held[0]);
+      for (Py_ssize_t i = 0; i < nseg; ++i) pa[i] = ptr(held[2 * i]), pb[i] = ptr(held[2 * i + 1]);
+      rc = kr_gemm_bf16_nt_segments((int)m, (int)n, (int)fa.rows, (int)nseg, pa, fa.ld, fa.run_rows, fa.run_ld, pb, fb.ld,
+                                    ptr(out), oc.ld, accumulate, split == 2 ? KR_GEMM_BESIDE_OTHER_STREAMS : 0, max_cus,
+                                    ws_bytes ? ptr(ws) : nullptr, ws_bytes, stream());
+    }
     if (rc != KR_OK)
       return failed("kr_gemm_bf16_nt_segments(M=" + std::to_string(m) + ", N=" + std::to_string(n) + ", k_seg=" +
                         std::to_string(fa.rows) + ", nseg=" + std::to_string(nseg) + ")",
@@ -314,14 +345,18 @@ PyObject* py_rmsnorm_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Operand o = operand(x);
     if (!o.ok || !is_gamma(a[1], o.cols) || !fits_int(o.rows)) return none();
     const float eps = (float)real(a[2]);
-    Tensor y = matrix(o.rows, o.cols, x);
-    Tensor rstd = at::empty({o.rows}, x.options().dtype(at::kFloat));
-    const void* g = ptr(tensor(a[1]));
-    const int rc = o.run_rows > 1
-                       ? kr_rmsnorm_fwd_runs(ptr(x), g, ptr(y), (float*)ptr(rstd), (int)o.rows, (int)o.cols, o.ld,
-                                             o.run_rows, o.run_ld, eps, stream())
-                       : kr_rmsnorm_fwd(ptr(x), g, ptr(y), (float*)ptr(rstd), (int)o.rows, (int)o.cols, o.ld, eps,
-                                        stream());
+    const Tensor& gamma = tensor(a[1]);
+    Tensor y, rstd;
+    int rc;
+    {
+      WithoutInterpreter free;
+      y = matrix(o.rows, o.cols, x);
+      rstd = at::empty({o.rows}, x.options().dtype(at::kFloat));
+      rc = o.run_rows > 1 ? kr_rmsnorm_fwd_runs(ptr(x), ptr(gamma), ptr(y), (float*)ptr(rstd), (int)o.rows, (int)o.cols, o.ld,
+                                                o.run_rows, o.run_ld, eps, stream())
+                          : kr_rmsnorm_fwd(ptr(x), ptr(gamma), ptr(y), (float*)ptr(rstd), (int)o.rows, (int)o.cols, o.ld, eps,
+                                           stream());
+    }
     if (rc != KR_OK) return failed("kr_rmsnorm_fwd", rc);
     PyObject *py = wrap(std::move(y)), *pr = wrap(std::move(rstd));
     return Py_BuildValue("(NN)", py, pr);
@@ -344,32 +379,42 @@ PyObject* py_rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       if (!orr.ok || orr.rows != ox.rows || orr.cols != ox.cols) return none();
     }
     if (!absent(a[5]) && !bf16_arg(a[5])) return none();
-    Tensor dx = absent(a[5]) ? matrix(ox.rows, ox.cols, x) : tensor(a[5]);
-    oc = operand3(dx);
-    if (!oc.ok || oc.rows != ox.rows || oc.cols != ox.cols) return none();
     const int rows = (int)ox.rows, cols = (int)ox.cols;
-    Tensor dgamma, ws;
-    void* ws_ptr;
-    if (absent(a[6])) {
-      dgamma = at::empty({ox.cols}, x.options());
-      ws = bytes(kr_rmsnorm_bwd_workspace_bytes(rows, cols), x);
-      ws_ptr = ptr(ws);
+    Tensor dx, dgamma, partials;
+    if (absent(a[5])) {
+      if (cols % 8) return none();
+      oc.ld = cols;
     } else {
-      if (!f32_arg(a[6])) return none();
-      const Tensor& p = tensor(a[6]);
-      if (p.dim() != 2 || !p.is_contiguous() || p.size(1) != cols || p.size(0) != kr_rmsnorm_bwd_partial_rows(rows, cols))
-        return none();
-      ws_ptr = ptr(p);
+      dx = tensor(a[5]);
+      oc = operand3(dx);
+      if (!oc.ok || oc.rows != ox.rows || oc.cols != ox.cols) return none();
     }
-    void* dg = dgamma.defined() ? ptr(dgamma) : nullptr;
-    const void *g = ptr(tensor(a[3])), *res = ptr_or_null(a[4]);
-    const int rc =
-        (ox.run_rows > 1 || orr.run_rows > 1 || oc.run_rows > 1)
-            ? kr_rmsnorm_bwd_add_runs(ptr(dy), ptr(x), (const float*)ptr(rstd), g, res, ptr(dx), dg, ws_ptr, rows, cols,
-                                      od.ld, ox.ld, ox.run_rows, ox.run_ld, orr.ld, orr.run_rows, orr.run_ld, oc.ld,
-                                      oc.run_rows, oc.run_ld, stream())
-            : kr_rmsnorm_bwd_add(ptr(dy), ptr(x), (const float*)ptr(rstd), g, res, ptr(dx), dg, ws_ptr, rows, cols, od.ld,
-                                 ox.ld, orr.ld, oc.ld, stream());
+    if (!absent(a[6])) {
+      if (!f32_arg(a[6])) return none();
+      partials = tensor(a[6]);
+      if (partials.dim() != 2 || !partials.is_contiguous() || partials.size(1) != cols ||
+          partials.size(0) != kr_rmsnorm_bwd_partial_rows(rows, cols))
+        return none();
+    }
+    const Tensor& gamma = tensor(a[3]);
+    int rc;
+    {
+      WithoutInterpreter free;
+      if (!dx.defined()) dx = matrix(rows, cols, x);
+      Tensor ws = partials;
+      if (!partials.defined()) {
+        dgamma = at::empty({ox.cols}, x.options());
+        ws = bytes(kr_rmsnorm_bwd_workspace_bytes(rows, cols), x);
+      }
+      void* dg = dgamma.defined() ? ptr(dgamma) : nullptr;
+      const void* res = ptr_or_null(a[4]);
+      rc = (ox.run_rows > 1 || orr.run_rows > 1 || oc.run_rows > 1)
+               ? kr_rmsnorm_bwd_add_runs(ptr(dy), ptr(x), (const float*)ptr(rstd), ptr(gamma), res, ptr(dx), dg, ptr(ws), rows,
+                                         cols, od.ld, ox.ld, ox.run_rows, ox.run_ld, orr.ld, orr.run_rows, orr.run_ld, oc.ld,
+                                         oc.run_rows, oc.run_ld, stream())
+               : kr_rmsnorm_bwd_add(ptr(dy), ptr(x), (const float*)ptr(rstd), ptr(gamma), res, ptr(dx), dg, ptr(ws), rows, cols,
+                                    od.ld, ox.ld, orr.ld, oc.ld, stream());
+    }
     if (rc != KR_OK) return failed("kr_rmsnorm_bwd_add", rc);
     PyObject* pdx = absent(a[5]) ? wrap(std::move(dx)) : Py_NewRef(a[5]);
     PyObject* pdg = dgamma.defined() ? wrap(std::move(dgamma)) : Py_NewRef(Py_None);
@@ -391,9 +436,12 @@ PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       return none();
     const int64_t s = f.size(0), b = f.size(1), slots = f.size(3), heads = f.size(2) * slots, hd = f.size(4);
     if (!fits_int(s) || !fits_int(b) || !fits_int(heads)) return none();
-    const int rc = kr_rope(ptr(f), ptr(f), (const float*)ptr(fr), (int)s, (int)b, (int)heads, (int)hd, b * heads * hd,
-                           heads * hd, hd, b * heads * hd, heads * hd, hd, backward, (int)slots,
-                           (int)slots - 1, stream());
+    int rc;
+    {
+      WithoutInterpreter free;
+      rc = kr_rope(ptr(f), ptr(f), (const float*)ptr(fr), (int)s, (int)b, (int)heads, (int)hd, b * heads * hd, heads * hd, hd,
+                   b * heads * hd, heads * hd, hd, backward, (int)slots, (int)slots - 1, stream());
+    }
     if (rc != KR_OK) return failed("kr_rope", rc);
     Py_RETURN_TRUE;
   });
@@ -455,15 +503,20 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!c.ok) return none();
     const float scale = (float)real(a[3]);
     const int flags = (int)integer(a[4]);
-    Tensor o = at::empty({c.s, c.b, c.nq, c.hd}, q.options());
-    Tensor lse = at::empty({c.b, c.nq, c.s}, q.options().dtype(at::kFloat));
-    Tensor ws;
-    const size_t n = (flags & KR_ATTN_GENERAL_KERNELS) ? 0 : kr_attn_fwd_workspace_bytes(c.s, c.b, c.nq, c.nkv, c.hd);
-    if (n) ws = bytes(n, q);
-    const QStrides sq = q_strides(q, c.per), so = q_strides(o, c.per);
-    const int rc = kr_attn_fwd_ws(ptr(q), ptr(k), ptr(v), ptr(o), (float*)ptr(lse), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s,
-                                  sq.b, sq.g, sq.h, k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1),
-                                  v.stride(2), so.s, so.b, so.g, so.h, flags, n ? ptr(ws) : nullptr, n, stream());
+    Tensor o, lse;
+    int rc;
+    {
+      WithoutInterpreter free;
+      o = at::empty({c.s, c.b, c.nq, c.hd}, q.options());
+      lse = at::empty({c.b, c.nq, c.s}, q.options().dtype(at::kFloat));
+      Tensor ws;
+      const size_t n = (flags & KR_ATTN_GENERAL_KERNELS) ? 0 : kr_attn_fwd_workspace_bytes(c.s, c.b, c.nq, c.nkv, c.hd);
+      if (n) ws = bytes(n, q);
+      const QStrides sq = q_strides(q, c.per), so = q_strides(o, c.per);
+      rc = kr_attn_fwd_ws(ptr(q), ptr(k), ptr(v), ptr(o), (float*)ptr(lse), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b,
+                          sq.g, sq.h, k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), so.s,
+                          so.b, so.g, so.h, flags, n ? ptr(ws) : nullptr, n, stream());
+    }
     if (rc != KR_OK) return failed(attn_name("kr_attn_fwd", c), rc);
     PyObject *po = wrap(std::move(o)), *pl = wrap(std::move(lse));
     return Py_BuildValue("(NN)", po, pl);
@@ -488,21 +541,27 @@ PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const float scale = (float)real(a[6]);
     const int flags = (int)integer(a[7]);
     const int64_t s = c.s, b = c.b, ng = c.nkv, hd = c.hd, g = (c.per + 2) * hd, w = ng * g;
-    Tensor fused = at::empty({s, b, ng, c.per + 2, hd}, q.options());
-    Tensor dq = fused.as_strided({s, b, ng, c.per, hd}, {b * w, w, g, hd, 1}, 0);
-    Tensor dk = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, c.per * hd);
-    Tensor dv = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, (c.per + 1) * hd);
-    const size_t n = kr_attn_bwd_workspace_bytes(c.s, c.b, c.nq, c.nkv, c.hd);
-    Tensor ws = bytes(n < 16 ? 16 : n, q);
-    const QStrides sq = q_strides(q, c.per);
-    const int64_t os = b * c.nq * hd, ob = c.nq * hd, og = c.per * hd;
-    const int rc = kr_attn_bwd_flags(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(o), (const float*)ptr(lse), ptr(dq), ptr(dk),
-                                     ptr(dv), ptr(ws), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b, sq.g, sq.h,
-                                     k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), os, ob,
-                                     og, hd, os, ob, og, hd, b * w, w, g, hd, b * w, w, g, b * w, w, g, flags, stream());
+    Tensor fused, mixed, dq, dk, dv;
+    int rc;
+    {
+      WithoutInterpreter free;
+      fused = at::empty({s, b, ng, c.per + 2, hd}, q.options());
+      mixed = fused.view({s, b, w});
+      dq = fused.as_strided({s, b, ng, c.per, hd}, {b * w, w, g, hd, 1}, 0);
+      dk = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, c.per * hd);
+      dv = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, (c.per + 1) * hd);
+      const size_t n = kr_attn_bwd_workspace_bytes(c.s, c.b, c.nq, c.nkv, c.hd);
+      Tensor ws = bytes(n < 16 ? 16 : n, q);
+      const QStrides sq = q_strides(q, c.per);
+      const int64_t os = b * c.nq * hd, ob = c.nq * hd, og = c.per * hd;
+      rc = kr_attn_bwd_flags(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(o), (const float*)ptr(lse), ptr(dq), ptr(dk), ptr(dv),
+                             ptr(ws), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b, sq.g, sq.h, k.stride(0), k.stride(1),
+                             k.stride(2), v.stride(0), v.stride(1), v.stride(2), os, ob, og, hd, os, ob, og, hd, b * w, w, g, hd,
+                             b * w, w, g, b * w, w, g, flags, stream());
+    }
     if (rc != KR_OK) return failed(attn_name("kr_attn_bwd", c), rc);
     PyObject *pq = wrap(std::move(dq)), *pk = wrap(std::move(dk)), *pv = wrap(std::move(dv));
-    PyObject* pm = wrap(fused.view({s, b, w}));
+    PyObject* pm = wrap(std::move(mixed));
     PyObject* pf = wrap(std::move(fused));
     return Py_BuildValue("(NNNNN)", pq, pk, pv, pm, pf);
   });
@@ -521,12 +580,24 @@ PyObject* py_dropout_add(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const double p = real(a[2]);
     if (!(p >= 0.0 && p < 1.0)) return none();
     const uint64_t seed = seed_value(a[4]);
-    Tensor out = absent(a[3]) ? at::empty(x.sizes(), x.options()) : tensor(a[3]);
-    const Operand oc = operand(out);
-    if (!oc.ok || oc.run_rows > 1) return none();
-    Tensor mask = at::empty(x.sizes(), x.options().dtype(at::kByte));
-    const int rc = kr_dropout_add(ptr(x), ox.ld, ptr(r), orr.ld, ptr(out), oc.ld, ptr(mask), ox.rows, (int)ox.cols, (float)p,
-                                  seed, 0, stream());
+    Tensor out, mask;
+    Operand oc;
+    if (absent(a[3])) {
+      oc.ld = ox.cols;
+      if (oc.ld % 8) return none();
+    } else {
+      out = tensor(a[3]);
+      oc = operand(out);
+      if (!oc.ok || oc.run_rows > 1) return none();
+    }
+    int rc;
+    {
+      WithoutInterpreter free;
+      if (!out.defined()) out = at::empty(x.sizes(), x.options());
+      mask = at::empty(x.sizes(), x.options().dtype(at::kByte));
+      rc = kr_dropout_add(ptr(x), ox.ld, ptr(r), orr.ld, ptr(out), oc.ld, ptr(mask), ox.rows, (int)ox.cols, (float)p, seed, 0,
+                          stream());
+    }
     if (rc != KR_OK) return failed("kr_dropout_add", rc);
     PyObject* po = absent(a[3]) ? wrap(std::move(out)) : Py_NewRef(a[3]);
     PyObject* pm = wrap(std::move(mask));
@@ -542,8 +613,13 @@ PyObject* py_dropout_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Operand o = operand(dy);
     if (!o.ok || o.run_rows > 1 || mask.sizes() != dy.sizes() || !mask.is_contiguous()) return none();
     const float scale = (float)real(a[2]);
-    Tensor dx = at::empty(dy.sizes(), dy.options());
-    const int rc = kr_dropout_bwd(ptr(dy), o.ld, ptr(mask), ptr(dx), o.cols, o.rows, (int)o.cols, scale, stream());
+    Tensor dx;
+    int rc;
+    {
+      WithoutInterpreter free;
+      dx = at::empty(dy.sizes(), dy.options());
+      rc = kr_dropout_bwd(ptr(dy), o.ld, ptr(mask), ptr(dx), o.cols, o.rows, (int)o.cols, scale, stream());
+    }
     if (rc != KR_OK) return failed("kr_dropout_bwd", rc);
     return wrap(std::move(dx));
   });

@@ -1,5 +1,9 @@
 """The native host side of the hip backend (``csrc/kr_host.cpp``) classifies tensors as the Python side does, and
-leaves what it does not take to it.  No GPU needed."""
+leaves what it does not take to it."""
+
+import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -137,3 +141,42 @@ def test_split_and_budget_may_be_any_truth_value_and_any_number():
     for split, code in ((None, 0), (True, 1), (2, 1), (False, 2), (0, 2)):
         assert be.gemm(0, x, x, 8, 8, 8, split_k=split, max_cus=16.0) == "done"
         assert be._n.args[8] == code and type(be._n.args[12]) is int
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+@pytest.mark.parametrize("what", ["gemm", "wgrad", "rotary"])
+def test_other_threads_run_during_a_launch(what):
+    """With a switch interval that never ends, another thread gets the interpreter only where the launching thread lets
+    go of it: inside the native calls.  (Calls into given outputs: the end of a tensor's life lets go of it too.)  The
+    launches go on until the other thread has had three turns, at most for four seconds."""
+    n = load_native()
+    x, out = (torch.ones(256, 256, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    fused, table = torch.ones(128, 1, 1, 3, 128, device="cuda", dtype=torch.bfloat16), torch.zeros(128, 1, 1, 128, device="cuda")
+    call = {"gemm": lambda: n.gemm(0, x, x, 256, 256, 256, out, False, 0, None, None, None, 0),
+            "wgrad": lambda: n.wgrad_segments([x], [x], out, False, 0, 0),
+            "rotary": lambda: n.rope_fused(fused, 1, table, False)}[what]
+    call()
+    torch.cuda.synchronize()
+    turns, stop, old = [0], [False], sys.getswitchinterval()
+
+    def other():
+        while not stop[0]:
+            turns[0] += 1
+            time.sleep(0)
+
+    thread = threading.Thread(target=other)
+    sys.setswitchinterval(1000.0)
+    try:
+        thread.start()
+        seen, end, launched = turns[0], time.perf_counter() + 4.0, 0
+        while turns[0] - seen < 3 and time.perf_counter() < end and launched < 20000:
+            call()
+            launched += 1
+    finally:
+        got = turns[0] - seen
+        stop[0] = True
+        sys.setswitchinterval(old)
+        thread.join()
+    torch.cuda.synchronize()
+    assert got >= 3, f"{launched} launches, {got} turns of the other thread"
