@@ -311,10 +311,11 @@ int kr_dropout_bwd(const void* dy, int64_t lddy, const void* mask, void* dx, int
  * multiple of 128).  Every other shape is padded into them
  * through the workspace (zero channels up to 128, zero rows up to the next multiple of 128: the
  * causal mask keeps the added keys from every real query, and the added queries are given a
- * log-sum-exp that makes them inert in the backward pass): kr_attn_bwd always, the forward when it
- * is called as kr_attn_fwd_ws with a workspace.  Without one (kr_attn_fwd, kr_attn_fwd_flags) such a
- * shape runs on general fp32 kernels that are correct and slow; with KR_ATTN_GENERAL_KERNELS in the
- * flags word any shape does but hd = 128 with s a multiple of 128.  All strides multiples of 8.
+ * log-sum-exp that makes them inert in the backward pass).  That holds for kr_attn_bwd always and for the
+ * forward called as kr_attn_fwd_ws with a workspace.  Without one (kr_attn_fwd, kr_attn_fwd_flags), or
+ * with KR_ATTN_GENERAL_KERNELS in the flags word, any shape but hd = 128 with s a multiple of 128 runs on
+ * general kernels, slow, whose probabilities stay fp32 (the MFMA kernels round them to bf16 in front of
+ * P.V).  All strides multiples of 8.
  * kr_attn_bwd needs a workspace of kr_attn_bwd_workspace_bytes() bytes (16-byte aligned).   */
 int kr_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                 int s, int b, int nq, int nkv, int hd, float scale,
@@ -341,8 +342,8 @@ int kr_attn_fwd_flags(const void* q, const void* k, const void* v, void* o, floa
                       int flags, void* stream);
 /* kr_attn_fwd_flags with a workspace of kr_attn_fwd_workspace_bytes() bytes (0 for hd = 128 and whole
  * 128-row tiles; workspace may then be NULL; one that is too small is KR_EINVAL for any other shape, also
- * for those that run in place and leave it untouched; none at all selects the general kernels for a shape
- * that would be padded): the call the reference's
+ * for those that run in place and leave it untouched; none at all selects the general kernels for any
+ * other shape): the call the reference's
  * flash_attn_gpu.fwd (kareus/flash_attn/flash_attn_interface.py:66-80) maps to for any head
  * dimension and sequence length it accepts.                                                      */
 size_t kr_attn_fwd_workspace_bytes(int s, int b, int nq, int nkv, int hd);

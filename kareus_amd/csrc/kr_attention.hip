@@ -1901,8 +1901,8 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
 
 // =============================================================================================
 // General path: any sequence length, head dimensions that are a multiple of 8 up to 128.
-// The kernels above are built for head dimensions 128 and 64.  With KR_ATTN_GENERAL_KERNELS, or where
-// there is neither an instance nor a workspace to pad into, a shape runs through these plain fp32 kernels:
+// The kernels above are built for head dimensions 128 and 64.  With KR_ATTN_GENERAL_KERNELS, or in the forward without
+// a workspace, any shape but hd = 128 with whole 128-row tiles runs through these plain fp32 kernels:
 // same interface, same tensor layouts, same results to rounding, no MFMA — they exist so that such a
 // shape is computed on the device at all, not to be fast.  A workgroup of 256 threads owns 32
 // query rows (forward, dQ) or 32 keys (dK/dV) and walks 32-row tiles of the other operand through
@@ -2593,11 +2593,14 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
       return KR_EUNSUPPORTED;
   }
   const bool in_place = attn_in_place(s, hd, {q_ss, k_ss, v_ss, o_ss});
+  // Outside the training workloads' shapes a call without a workspace gets the general kernels, whose
+  // probabilities stay fp32, also where the MFMA kernels (bf16 probabilities) would need no workspace.
+  const bool general_kernels = !attn_fast_path(s, hd) && ((flags & KR_ATTN_GENERAL_KERNELS) || workspace == nullptr);
   // (a workspace that is there but too small is a caller's mistake, not a request for the general kernels)
   if (!attn_fast_path(s, hd) && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr &&
       workspace_bytes < kr_attn_fwd_workspace_bytes(s, b, nq, nkv, hd))
     return KR_EINVAL;
-  if (!in_place && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr) {
+  if (!in_place && !general_kernels) {
     // padded into the MFMA kernels
     hipStream_t st = (hipStream_t)stream;
     const int sp = attn_padded_len(s), per = nq / nkv;
@@ -2620,7 +2623,7 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
     if (rc2 == KR_OK) rc2 = launch_resize_rows(lse_p, lse, (int64_t)b * nq, sp, s, 0.f, st);
     return rc2;
   }
-  if (!in_place || (!attn_fast_path(s, hd) && (flags & KR_ATTN_GENERAL_KERNELS))) {
+  if (general_kernels) {
     using namespace general;
     const QLayout ql{q_ss, q_sb, q_sg, q_sh}, ol{o_ss, o_sb, o_sg, o_sh};
     const KLayout kl{k_ss, k_sb, k_sh}, vl{v_ss, v_sb, v_sh};
@@ -2655,7 +2658,8 @@ extern "C" int kr_attn_fwd_flags(const void* q, const void* k, const void* v, vo
 }
 
 // kr_attn_fwd_flags with a workspace of kr_attn_fwd_workspace_bytes(): a shape the MFMA kernels do not take as it
-// lies (attn_in_place) is padded into them through the workspace instead of taking the general kernels.
+// lies (attn_in_place) is padded into them through the workspace; without one the general kernels take every shape but
+// the training workloads'.
 extern "C" int kr_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, int s, int b,
                               int nq, int nkv, int hd, float scale, int64_t q_ss, int64_t q_sb, int64_t q_sg,
                               int64_t q_sh, int64_t k_ss, int64_t k_sb, int64_t k_sh, int64_t v_ss, int64_t v_sb,

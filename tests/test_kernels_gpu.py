@@ -555,6 +555,28 @@ def test_attention_general_shapes(be, s, b, nq, nkv, hd, general):
     assert torch.equal(od, o) and torch.equal(lsed, lse)
 
 
+@pytest.mark.parametrize("s,hd", [(256, 64), (200, 64), (200, 128), (64, 96)])
+@pytest.mark.parametrize("flags", [None, 0, 0x100])
+def test_attention_forward_without_a_workspace_keeps_fp32_probabilities(be, s, hd, flags):
+    """``kr_attn_fwd`` and ``kr_attn_fwd_flags`` have no workspace: shapes other than hd = 128 with whole 128-row tiles run
+    on the general kernels, bit for bit, also those that the MFMA kernels could take as they lie.  Their only rounding is
+    the output's: with V of one sign, so that no sum cancels, o is within half a bf16 step (eight significant bits: at most
+    2^-8 of the value) of the exact result, plus what fp32 sums over at most 256 keys and the fast exponential
+    leave (1e-4)."""
+    _, q, k, v = _grouped(s, 1, 4, 2, hd, seed=130)
+    q, k, v = q.flatten(2, 3).contiguous(), k.contiguous(), v.abs().contiguous()
+    scale = hd ** -0.5
+    o, lse = torch.empty_like(q), torch.empty(1, 4, s, device=DEV)
+    strides = (*be._q_strides(q, 2), *be._k_strides(k), *be._k_strides(v), *be._q_strides(o, 2))
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), s, 1, 4, 2, hd, scale, *strides)
+    rc = be.lib.kr_attn_fwd(*args, be._stream()) if flags is None else be.lib.kr_attn_fwd_flags(*args, flags, be._stream())
+    assert rc == 0
+    want_o, want_lse = be.attn_fwd(q, k, v, scale, general_kernels=True)
+    assert torch.equal(o, want_o) and torch.equal(lse, want_lse)
+    exact = R.causal_gqa_attention(q.double().cpu(), k.double().cpu(), v.double().cpu())
+    assert ((o.double().cpu() - exact).abs() / exact).max() <= 2.0 ** -8 + 1e-4
+
+
 def test_attention_padded_into_the_mfma_kernels_equals_the_whole_tile_call(be):
     """A ragged length is the whole-tile problem with rows taken away: queries below s see the same keys, so the
     padded call must give the bits of the MFMA kernels on the next multiple of 128 restricted to the first s
