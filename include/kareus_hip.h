@@ -333,6 +333,8 @@ int kr_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse
  * (kareus/flash_attn/flash_attn_interface.py:66-80 runs one kernel at a time).                   */
 #define KR_ATTN_BESIDE_OTHER_STREAMS 0x100
 #define KR_ATTN_GENERAL_KERNELS 0x200
+/* forward only: a shape that the MFMA kernels take as it lies runs on them whatever workspace there is */
+#define KR_ATTN_IN_PLACE 0x800
 int kr_attn_fwd_flags(const void* q, const void* k, const void* v, void* o, float* lse,
                       int s, int b, int nq, int nkv, int hd, float scale,
                       int64_t q_stride_s, int64_t q_stride_b, int64_t q_stride_g, int64_t q_stride_h,
@@ -347,6 +349,11 @@ int kr_attn_fwd_flags(const void* q, const void* k, const void* v, void* o, floa
  * flash_attn_gpu.fwd (kareus/flash_attn/flash_attn_interface.py:66-80) maps to for any head
  * dimension and sequence length it accepts.                                                      */
 size_t kr_attn_fwd_workspace_bytes(int s, int b, int nq, int nkv, int hd);
+/* What kr_attn_fwd_ws with KR_ATTN_IN_PLACE, and kr_attn_bwd, need when no sequence stride of their tensors
+ * exceeds max_seq_stride elements: nothing / statistics and partial sums for the shapes that run as they lie,
+ * the sizes of the calls without the suffix (which hold for any strides) for all others.          */
+size_t kr_attn_fwd_workspace_bytes_strided(int s, int b, int nq, int nkv, int hd, int64_t max_seq_stride);
+size_t kr_attn_bwd_workspace_bytes_strided(int s, int b, int nq, int nkv, int hd, int64_t max_seq_stride);
 int kr_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
                    int s, int b, int nq, int nkv, int hd, float scale,
                    int64_t q_stride_s, int64_t q_stride_b, int64_t q_stride_g, int64_t q_stride_h,

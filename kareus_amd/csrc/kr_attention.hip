@@ -2252,6 +2252,18 @@ extern "C" size_t kr_attn_fwd_workspace_bytes(int s, int b, int nq, int nkv, int
   return 2 * attn_padded_bytes(s, b, nq) + 2 * attn_padded_bytes(s, b, nkv) + attn_padded_stat_bytes(s, b, nq);
 }
 
+// The sizes above hold for any strides.  A caller who knows them need not reserve the copies of a shape that is
+// not copied: s 4096, b 2, 32/8 heads of 64 asks for 169 MB forward and 607 MB backward above, for 0 and
+// 136 MB (statistics and fp32 partial sums) here.
+extern "C" size_t kr_attn_fwd_workspace_bytes_strided(int s, int b, int nq, int nkv, int hd, int64_t max_seq_stride) {
+  return attn_in_place(s, hd, {max_seq_stride}) ? 0 : kr_attn_fwd_workspace_bytes(s, b, nq, nkv, hd);
+}
+extern "C" size_t kr_attn_bwd_workspace_bytes_strided(int s, int b, int nq, int nkv, int hd, int64_t max_seq_stride) {
+  if (check_attn_common(s, b, nq, nkv, hd) != KR_OK) return 0;
+  return attn_in_place(s, hd, {max_seq_stride}) ? attn_bwd_fast_bytes(attn_padded_len(s), b, nq, nkv, hd)
+                                                : kr_attn_bwd_workspace_bytes(s, b, nq, nkv, hd);
+}
+
 namespace {
 // dense [s_pad, b, heads, 128] as the kernels' stride quadruple / triple
 QLayout padded_qlayout(int b, int nq, int per) {
@@ -2578,7 +2590,7 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
                            int64_t v_ss, int64_t v_sb, int64_t v_sh, int64_t o_ss, int64_t o_sb,
                            int64_t o_sg, int64_t o_sh, int flags, void* stream, void* workspace = nullptr,
                            size_t workspace_bytes = 0) {
-  if (flags & ~(KR_ATTN_BESIDE_OTHER_STREAMS | KR_ATTN_GENERAL_KERNELS)) return KR_EINVAL;
+  if (flags & ~(KR_ATTN_BESIDE_OTHER_STREAMS | KR_ATTN_GENERAL_KERNELS | KR_ATTN_IN_PLACE)) return KR_EINVAL;
   if (!q || !k || !v || !o || !lse) return KR_EINVAL;
   if (workspace && !kr_aligned16(workspace)) return KR_EINVAL;
   const int rc = check_attn_common(s, b, nq, nkv, hd);
@@ -2595,9 +2607,12 @@ static int attn_fwd_impl(const void* q, const void* k, const void* v, void* o, f
   const bool in_place = attn_in_place(s, hd, {q_ss, k_ss, v_ss, o_ss});
   // Outside the training workloads' shapes a call without a workspace gets the general kernels, whose
   // probabilities stay fp32, also where the MFMA kernels (bf16 probabilities) would need no workspace.
-  const bool general_kernels = !attn_fast_path(s, hd) && ((flags & KR_ATTN_GENERAL_KERNELS) || workspace == nullptr);
+  // (unless it asks for them: KR_ATTN_IN_PLACE)
+  const bool asked_in_place = in_place && (flags & KR_ATTN_IN_PLACE) && !(flags & KR_ATTN_GENERAL_KERNELS);
+  const bool general_kernels = !attn_fast_path(s, hd) && !asked_in_place &&
+                               ((flags & KR_ATTN_GENERAL_KERNELS) || workspace == nullptr);
   // (a workspace that is there but too small is a caller's mistake, not a request for the general kernels)
-  if (!attn_fast_path(s, hd) && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr &&
+  if (!attn_fast_path(s, hd) && !asked_in_place && !(flags & KR_ATTN_GENERAL_KERNELS) && workspace != nullptr &&
       workspace_bytes < kr_attn_fwd_workspace_bytes(s, b, nq, nkv, hd))
     return KR_EINVAL;
   if (!in_place && !general_kernels) {
@@ -2659,7 +2674,7 @@ extern "C" int kr_attn_fwd_flags(const void* q, const void* k, const void* v, vo
 
 // kr_attn_fwd_flags with a workspace of kr_attn_fwd_workspace_bytes(): a shape the MFMA kernels do not take as it
 // lies (attn_in_place) is padded into them through the workspace; without one the general kernels take every shape but
-// the training workloads'.
+// the training workloads', or, with KR_ATTN_IN_PLACE, every shape that would have to be padded.
 extern "C" int kr_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse, int s, int b,
                               int nq, int nkv, int hd, float scale, int64_t q_ss, int64_t q_sb, int64_t q_sg,
                               int64_t q_sh, int64_t k_ss, int64_t k_sb, int64_t k_sh, int64_t v_ss, int64_t v_sb,

@@ -16,6 +16,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -510,12 +511,15 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       o = at::empty({c.s, c.b, c.nq, c.hd}, q.options());
       lse = at::empty({c.b, c.nq, c.s}, q.options().dtype(at::kFloat));
       Tensor ws;
-      const size_t n = (flags & KR_ATTN_GENERAL_KERNELS) ? 0 : kr_attn_fwd_workspace_bytes(c.s, c.b, c.nq, c.nkv, c.hd);
-      if (n) ws = bytes(n, q);
       const QStrides sq = q_strides(q, c.per), so = q_strides(o, c.per);
+      const size_t n = (flags & KR_ATTN_GENERAL_KERNELS)
+                           ? 0
+                           : kr_attn_fwd_workspace_bytes_strided(c.s, c.b, c.nq, c.nkv, c.hd,
+                                                                 std::max({sq.s, so.s, k.stride(0), v.stride(0)}));
+      if (n) ws = bytes(n, q);
       rc = kr_attn_fwd_ws(ptr(q), ptr(k), ptr(v), ptr(o), (float*)ptr(lse), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b,
                           sq.g, sq.h, k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), so.s,
-                          so.b, so.g, so.h, flags, n ? ptr(ws) : nullptr, n, stream());
+                          so.b, so.g, so.h, flags | KR_ATTN_IN_PLACE, n ? ptr(ws) : nullptr, n, stream());
     }
     if (rc != KR_OK) return failed(attn_name("kr_attn_fwd", c), rc);
     PyObject *po = wrap(std::move(o)), *pl = wrap(std::move(lse));
@@ -550,10 +554,11 @@ PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       dq = fused.as_strided({s, b, ng, c.per, hd}, {b * w, w, g, hd, 1}, 0);
       dk = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, c.per * hd);
       dv = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, (c.per + 1) * hd);
-      const size_t n = kr_attn_bwd_workspace_bytes(c.s, c.b, c.nq, c.nkv, c.hd);
-      Tensor ws = bytes(n < 16 ? 16 : n, q);
       const QStrides sq = q_strides(q, c.per);
       const int64_t os = b * c.nq * hd, ob = c.nq * hd, og = c.per * hd;
+      const size_t n = kr_attn_bwd_workspace_bytes_strided(c.s, c.b, c.nq, c.nkv, c.hd,
+                                                           std::max({sq.s, k.stride(0), v.stride(0), os, b * w}));
+      Tensor ws = bytes(n < 16 ? 16 : n, q);
       rc = kr_attn_bwd_flags(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(o), (const float*)ptr(lse), ptr(dq), ptr(dk), ptr(dv),
                              ptr(ws), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b, sq.g, sq.h, k.stride(0), k.stride(1),
                              k.stride(2), v.stride(0), v.stride(1), v.stride(2), os, ob, og, hd, os, ob, og, hd, b * w, w, g, hd,

@@ -178,3 +178,23 @@ def test_swiglu_epilogue_index_model():
     for M, F, WN in [(512, 128, 8), (264, 384, 8), (264, 384, 6), (1000, 1024, 8), (520, 320, 5), (304, 672, 7),
                      (304, 672, 6)]:
         check(M, F, WN)
+
+
+def test_attention_workspaces_by_stride():
+    """What runs as it lies reserves no copies: nothing forward, statistics and partial sums of the rounded-up length
+    backward; what does not (other head dimensions, strides of 2^31 / 127 elements and more) the general sizes."""
+    lib = hip.load_library()
+    for s, hd in ((4096, 64), (1000, 64), (1000, 128), (4096, 128)):
+        sp = (s + 127) // 128 * 128
+        split = 2 if sp // 128 * 32 * 2 <= 512 else 1
+        assert lib.kr_attn_fwd_workspace_bytes_strided(s, 2, 32, 8, hd, 2 * 48 * hd) == 0
+        assert (lib.kr_attn_bwd_workspace_bytes_strided(s, 2, 32, 8, hd, 2 * 48 * hd)
+                == 2 * 2 * 32 * sp * 4 + 2 * 2 * 32 * split * sp * hd * 4)
+        limit = ((1 << 31) - 128) // 127 // 8 * 8
+        assert lib.kr_attn_fwd_workspace_bytes_strided(s, 2, 32, 8, hd, limit) == 0
+        over = limit + 8
+        assert lib.kr_attn_fwd_workspace_bytes_strided(s, 2, 32, 8, hd, over) == lib.kr_attn_fwd_workspace_bytes(s, 2, 32, 8, hd)
+        assert lib.kr_attn_bwd_workspace_bytes_strided(s, 2, 32, 8, hd, over) == lib.kr_attn_bwd_workspace_bytes(s, 2, 32, 8, hd)
+    assert lib.kr_attn_fwd_workspace_bytes_strided(256, 1, 4, 2, 96, 96) == lib.kr_attn_fwd_workspace_bytes(256, 1, 4, 2, 96) > 0
+    assert lib.kr_attn_bwd_workspace_bytes_strided(256, 1, 4, 2, 96, 96) == lib.kr_attn_bwd_workspace_bytes(256, 1, 4, 2, 96) > 0
+    assert lib.kr_attn_bwd_workspace_bytes_strided(256, 1, 4, 2, 136, 136) == 0

@@ -577,6 +577,38 @@ def test_attention_forward_without_a_workspace_keeps_fp32_probabilities(be, s, h
     assert ((o.double().cpu() - exact).abs() / exact).max() <= 2.0 ** -8 + 1e-4
 
 
+@pytest.mark.parametrize("s,b,nq,nkv,hd", [(1024, 2, 8, 2, 64), (1000, 2, 8, 2, 64), (300, 1, 4, 4, 64), (1000, 1, 8, 2, 128)])
+def test_attention_in_place_reserves_and_touches_no_copies(be, s, b, nq, nkv, hd):
+    """Shapes that run as they lie: a call allocates its results and the statistics and partial sums of the backward,
+    no padded copies (2 MiB: the allocator's rounding); and the backward, in a workspace of just that size, leaves
+    what lies behind it alone."""
+    _, q, k, v = _grouped(s, b, nq, nkv, hd, seed=140)
+    do, scale = rnd(s, b, nq, hd, seed=141), hd ** -0.5
+    w = be.lib.kr_attn_bwd_workspace_bytes_strided(s, b, nq, nkv, hd, max(t.stride(0) for t in (q, k, v, do)))
+
+    def peak(fn):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = fn()
+        return got, torch.cuda.max_memory_allocated() - before
+
+    (o, lse), used = peak(lambda: be.attn_fwd(q, k, v, scale))
+    assert used <= o.numel() * 2 + lse.numel() * 4 + (2 << 20)
+    (dq, dk, dv), used = peak(lambda: be.attn_bwd(do, q, k, v, o, lse, scale))
+    assert used <= (dq.numel() + dk.numel() + dv.numel()) * 2 + w + (2 << 20)
+
+    ws = torch.full((w + 4096,), 0xA5, dtype=torch.uint8, device=DEV)
+    got = [torch.empty(t.shape, dtype=t.dtype, device=DEV) for t in (dq, dk, dv)]
+    per = nq // nkv
+    rc = be.lib.kr_attn_bwd(do.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
+                            *(t.data_ptr() for t in got), ws.data_ptr(), s, b, nq, nkv, hd, scale, *be._q_strides(q, per),
+                            *be._k_strides(k), *be._k_strides(v), *be._q_strides(o, per), *be._q_strides(do, per),
+                            *be._q_strides(got[0], per), *be._k_strides(got[1]), *be._k_strides(got[2]), be._stream())
+    assert rc == 0 and bool((ws[w:] == 0xA5).all())
+    assert all(torch.equal(x, y) for x, y in zip(got, (dq, dk, dv)))
+
+
 def test_attention_padded_into_the_mfma_kernels_equals_the_whole_tile_call(be):
     """A ragged length is the whole-tile problem with rows taken away: queries below s see the same keys, so the
     padded call must give the bits of the MFMA kernels on the next multiple of 128 restricted to the first s
