@@ -15,7 +15,7 @@ order inside a layer is kareus/megatron/core/transformer/transformer_layer.py:14
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import Any, List, Optional
+from typing import Any, List, Optional, Tuple
 
 import torch
 
@@ -99,8 +99,10 @@ class LayerConfig:
     kareus_scheduler: Optional[Any] = None
     nanobatch_streams: Optional[List[Any]] = field(default=None, repr=False)
 
-    # the nanobatch streams were made by the block driver (streams that a caller names are always used)
+    # the nanobatch streams were made by the block driver, and which they are (streams that a caller names, in
+    # their place or in a copy of this, are always used)
     streams_are_own: bool = field(default=False, repr=False)
+    made_streams: Optional[Tuple[Any, ...]] = field(default=None, repr=False)
 
     # Nanobatches on streams of their own cost the host 0.9-1.0 ms per nanobatch and layer, forward and backward
     # (launches, and above all the event waits of the schedule points), one after the other on one stream 0.6 ms.
@@ -117,6 +119,9 @@ class LayerConfig:
         is below what its launches cost the host.  Products at 0.75 PFLOP/s, attention at 0.4, forty passes over
         the hidden states at 5 TB/s, the weights read twice at 4.5 TB/s."""
         if not self.streams_are_own or self.backend != "hip":
+            return False
+        made, named = self.made_streams, self.nanobatch_streams
+        if made is not None and (named is None or len(named) != len(made) or any(a is not b for a, b in zip(made, named))):
             return False
         t, h, hd, nq = seq * seqs, self.hidden_size, self.kv_channels, self.num_attention_heads
         weights = h * (self.qkv_width + nq * hd + 3 * self.ffn_hidden_size)
@@ -357,6 +362,7 @@ class LayerStack(torch.nn.Module):
             many = getattr(api, "new_streams", None)
             c.nanobatch_streams = (many(c.num_nanobatches) if many is not None
                                    else [api.new_stream() for _ in range(c.num_nanobatches)])
+            c.made_streams = tuple(c.nanobatch_streams)
         return c.nanobatch_streams
 
     def _get_all_params(self) -> List[torch.nn.Parameter]:

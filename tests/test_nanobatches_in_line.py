@@ -1,9 +1,12 @@
 """Small nanobatches run one after the other on the caller's stream (``LayerConfig.nanobatches_in_line``)."""
 
+import dataclasses
+
 import pytest
 import torch
 
 from kareus_amd import LayerConfig, LayerStack
+from kareus_amd.partitions.streams import use_stream_api
 
 gpu = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")]
 
@@ -19,6 +22,36 @@ def test_the_rule_follows_the_size_of_a_nanobatch():
     assert not own.nanobatches_in_line(4096, 1) and not own.nanobatches_in_line(1024, 4)
     assert not _cfg().nanobatches_in_line(256, 1)                                    # a caller's own streams are used
     assert not _cfg(streams_are_own=True, backend="eager").nanobatches_in_line(256, 1)
+
+
+class _NoDevice:
+    """A stream interface whose streams are mere objects: enough to build a stack."""
+
+    new_stream = new_event = current_stream = staticmethod(object)
+
+    @staticmethod
+    def available():
+        return True
+
+
+def _built(**kw):
+    cfg = _cfg(hidden_size=64, num_attention_heads=2, num_query_groups=1, kv_channels=32, ffn_hidden_size=96, **kw)
+    with use_stream_api(_NoDevice()):
+        LayerStack(cfg)
+    return cfg
+
+
+def test_streams_that_a_caller_names_are_used_whenever_it_names_them():
+    cfg = _built()
+    assert len(cfg.nanobatch_streams) == 2 and cfg.nanobatches_in_line(256, 1)          # the driver's own
+    assert dataclasses.replace(cfg).nanobatches_in_line(256, 1)
+    assert not dataclasses.replace(cfg, nanobatch_streams=[object(), object()]).nanobatches_in_line(256, 1)
+    cfg.nanobatch_streams[1] = object()                                                   # one of them
+    assert not cfg.nanobatches_in_line(256, 1)
+    cfg = _built()
+    cfg.nanobatch_streams = [object(), object()]                                          # all, after the stack was built
+    assert not cfg.nanobatches_in_line(256, 1)
+    assert not _built(nanobatch_streams=[object(), object()]).nanobatches_in_line(256, 1)  # before
 
 
 @pytest.mark.parametrize("nnb,b,s", [(2, 2, 256), (4, 4, 136), (2, 6, 200), (4, 8, 64)])
