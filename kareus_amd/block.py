@@ -111,14 +111,16 @@ class LayerConfig:
     # their latency.  Measured, streams against one stream, two / four nanobatches: small layer (512 hidden) 256-2048
     # tokens 1.5x / 1.5x, 8B shard of four 1024 tokens 1.48x / 1.32x, 2048 tokens 1.13x / 0.98x, 4096 tokens 0.88x / 0.86x,
     # 3B layer 512 tokens 1.41x / 1.31x, 1024 tokens 1.18x / 1.01x, 8B layer 256 tokens 1.20x / 0.84x.
-    IN_LINE_BELOW_MS = 0.65
+    # 0: every pass uses the streams.
+    in_line_below_ms: float = 0.65
 
     def nanobatches_in_line(self, seq: int, seqs: int) -> bool:
         """Whether the nanobatches of a pass ([seq, seqs, hidden] each) run one after the other on the caller's stream
         instead of on their own: where an estimate of one nanobatch's device time per layer, forward and backward,
         is below what its launches cost the host.  Products at 0.75 PFLOP/s, attention at 0.4, forty passes over
-        the hidden states at 5 TB/s, the weights read twice at 4.5 TB/s."""
-        if not self.streams_are_own or self.backend != "hip":
+        the hidden states at 5 TB/s, the weights read twice at 4.5 TB/s.  Not under a plan: its overlap windows and
+        resource shapes are about the streams, and a pass without them would run none of it."""
+        if not self.streams_are_own or self.backend != "hip" or self.kareus_scheduler is not None:
             return False
         made, named = self.made_streams, self.nanobatch_streams
         if made is not None and (named is None or len(named) != len(made) or any(a is not b for a, b in zip(made, named))):
@@ -127,7 +129,7 @@ class LayerConfig:
         weights = h * (self.qkv_width + nq * hd + 3 * self.ffn_hidden_size)
         ms = (6.0 * t * weights / 0.75e12 + 7.0 * seqs * nq * hd * float(seq) ** 2 / 0.4e12
               + 80.0 * t * h / 5e9 + 4.0 * weights / 4.5e9)
-        return ms < self.IN_LINE_BELOW_MS
+        return ms < self.in_line_below_ms
 
     @property
     def qkv_width(self) -> int:

@@ -1,12 +1,16 @@
 """Small nanobatches run one after the other on the caller's stream (``LayerConfig.nanobatches_in_line``)."""
 
 import dataclasses
+import os
 
 import pytest
 import torch
 
 from kareus_amd import LayerConfig, LayerStack
+from kareus_amd.operators.noop_collective import NoOpAllReduce
+from kareus_amd.partitions import partition_base
 from kareus_amd.partitions.streams import use_stream_api
+from kareus_amd.scheduler import PipelineCommScheduler
 
 gpu = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")]
 
@@ -52,6 +56,37 @@ def test_streams_that_a_caller_names_are_used_whenever_it_names_them():
     cfg.nanobatch_streams = [object(), object()]                                          # all, after the stack was built
     assert not cfg.nanobatches_in_line(256, 1)
     assert not _built(nanobatch_streams=[object(), object()]).nanobatches_in_line(256, 1)  # before
+
+
+def test_a_plan_and_the_switch_keep_the_streams():
+    """Under a plan the overlap windows order the streams and the resource shapes leave compute units to them."""
+    cfg = _cfg(streams_are_own=True)
+    assert cfg.nanobatches_in_line(256, 1)
+    cfg.kareus_scheduler = object()
+    assert not cfg.nanobatches_in_line(256, 1)
+    assert not _cfg(streams_are_own=True, in_line_below_ms=0.0).nanobatches_in_line(8, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_plan_reserves_compute_units_on_a_small_pass(fixtures_dir, monkeypatch):
+    """The resource shapes of the shipped plan reach the partitions of a small layer: budgets are entered, as many
+    as without the in-line rule, and the hand-overs record and wait."""
+    budgets, waits = [], []
+    reserve = partition_base.reserve_compute_units
+    monkeypatch.setattr(partition_base, "reserve_compute_units", lambda n: budgets.append(n) or reserve(n))
+    wait = NoOpAllReduce.event_wait
+    monkeypatch.setattr(NoOpAllReduce, "event_wait", lambda self: waits.append(self.batch_idx) or wait(self))
+    cfg = _cfg(hidden_size=1024, num_attention_heads=8, ffn_hidden_size=896, num_layers=2)
+    model = LayerStack(cfg, device="cuda", seed=3)
+    sch = PipelineCommScheduler(os.path.join(fixtures_dir, "scheds_pipeline_02328.py"), pp_rank=0, num_microbatches=8,
+                                use_activation_checkpointing=True)
+    cfg.kareus_scheduler = sch
+    sch.on_step_begin()
+    sch.on_instruction_begin("forward")
+    model(torch.randn(256, 4, 1024, device="cuda", dtype=torch.bfloat16))
+    torch.cuda.synchronize()
+    assert budgets and waits
 
 
 @pytest.mark.parametrize("nnb,b,s", [(2, 2, 256), (4, 4, 136), (2, 6, 200), (4, 8, 64)])
