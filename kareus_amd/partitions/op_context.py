@@ -36,9 +36,6 @@ class OperationContext:
         self.to_save = tensors
 
 
-_EMPTY: Dict[Tuple[torch.device, torch.dtype], torch.Tensor] = {}  # one empty tensor per (device, dtype)
-
-
 def clear_tensor_data(*tensors: Optional[torch.Tensor]) -> None:
     """Drop the storage behind each tensor object now instead of at refcount zero.
 
@@ -49,11 +46,7 @@ def clear_tensor_data(*tensors: Optional[torch.Tensor]) -> None:
     """
     for t in tensors:
         if t is not None:
-            key = (t.device, t.dtype)
-            empty = _EMPTY.get(key)
-            if empty is None:
-                empty = _EMPTY[key] = torch.empty(0, device=t.device, dtype=t.dtype)
-            t.data = empty
+            t.data = t.new_empty(0)  # (a storage of its own: a holder of the object may resize it)
 
 
 def operator_parameters(op: torch.nn.Module):

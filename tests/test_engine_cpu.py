@@ -10,7 +10,7 @@ import torch
 
 from kareus_amd import LayerConfig, LayerStack
 from kareus_amd.operators import NoOpAllReduce, QKVPostProcessOp, RMSNorm
-from kareus_amd.partitions import NanoBatchContext, TensorStore, TransformerBlockAutogradFunction
+from kareus_amd.partitions import NanoBatchContext, TensorStore, TransformerBlockAutogradFunction, clear_tensor_data
 from kareus_amd.partitions.autograd_function import _flatten_grad_params
 from kareus_amd.partitions.partition_base import PartitionBase
 from kareus_amd.partitions.streams import use_stream_api
@@ -556,3 +556,13 @@ def test_resource_shape_reserves_compute_units_for_the_other_streams(monkeypatch
     with torch.no_grad():
         m2(torch.randn(16, 4, 64))
     assert seen == [0] * 8
+
+
+def test_cleared_tensors_share_no_memory():
+    """A holder of a released tensor may grow it again; it must not see another one's data."""
+    a, b, c = torch.ones(3), torch.ones(5), torch.ones(2, 2, dtype=torch.bfloat16)
+    clear_tensor_data(a, None, b, c)
+    assert a.numel() == b.numel() == c.numel() == 0 and c.dtype == torch.bfloat16
+    a.resize_(4).fill_(1.0)
+    b.resize_(4).fill_(2.0)
+    assert a.tolist() == [1.0] * 4 and b.tolist() == [2.0] * 4
