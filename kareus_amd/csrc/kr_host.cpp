@@ -36,6 +36,9 @@ bool bf16_arg(PyObject* o) { return is_tensor(o) && on_device(tensor(o), at::kBF
 bool f32_arg(PyObject* o) { return is_tensor(o) && on_device(tensor(o), at::kFloat); }
 bool absent(PyObject* o) { return o == Py_None; }
 
+// sizes that a tracer keeps as symbols: the Python side's views carry them on
+bool symbolic(const Tensor& t) { return t.unsafeGetTensorImpl()->has_symbolic_sizes_strides(); }
+
 PyObject* none() { Py_RETURN_NONE; }
 PyObject* wrap(Tensor t) { return THPVariable_Wrap(std::move(t)); }
 void* ptr(const Tensor& t) { return t.data_ptr(); }
@@ -148,13 +151,13 @@ Tensor bytes(size_t n, const Tensor& like) { return at::empty({(int64_t)n}, like
 // t itself when its rows come in runs — or None
 PyObject* py_rows_view(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
-    if (n_args != 2 || !is_tensor(a[0])) return none();
+    if (n_args != 2 || !is_tensor(a[0]) || symbolic(tensor(a[0]))) return none();
     PyObject* t = a[0];
     const Tensor& x = tensor(t);
     const Operand o = operand(x, integer(a[1]));
     if (!o.ok) return none();
     if (x.dim() == 2 || o.run_rows > 1) return Py_NewRef(t);
-    return wrap(x.as_strided({o.rows, o.cols}, {o.ld, 1}, x.storage_offset()));
+    return wrap(x.view({o.rows, o.cols}));  // (relative to x: as_strided would bind a trace to x's place in its storage)
   });
 }
 
@@ -452,16 +455,13 @@ PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 // per + 2, hd]): views
 PyObject* py_split_qkv(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
-    if (n_args != 4 || !is_tensor(a[0])) return none();
+    if (n_args != 4 || !is_tensor(a[0]) || symbolic(tensor(a[0]))) return none();
     const Tensor& m = tensor(a[0]);
     const int64_t ng = integer(a[1]), per = integer(a[2]), hd = integer(a[3]);
     if (m.dim() != 3 || !m.is_contiguous() || m.size(2) != ng * (per + 2) * hd) return none();
-    const int64_t s = m.size(0), b = m.size(1), w = m.size(2), g = (per + 2) * hd, off = m.storage_offset();
-    PyObject* q = wrap(m.as_strided({s, b, ng, per, hd}, {b * w, w, g, hd, 1}, off));
-    PyObject* k = wrap(m.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, off + per * hd));
-    PyObject* v = wrap(m.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, off + (per + 1) * hd));
-    PyObject* f = wrap(m.as_strided({s, b, ng, per + 2, hd}, {b * w, w, g, hd, 1}, off));
-    return Py_BuildValue("(NNNN)", q, k, v, f);
+    const Tensor fused = m.view({m.size(0), m.size(1), ng, per + 2, hd});
+    PyObject *q = wrap(fused.narrow(3, 0, per)), *k = wrap(fused.select(3, per)), *v = wrap(fused.select(3, per + 1));
+    return Py_BuildValue("(NNNN)", q, k, v, wrap(fused));
   });
 }
 

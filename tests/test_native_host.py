@@ -53,6 +53,31 @@ def test_calls_leave_other_tensors_to_the_python_side():
     assert n.dropout_bwd(x, x, 1.0) is None and n.wgrad_segments([x], [x], None, False, 1, 0) is None
 
 
+@pytest.mark.parametrize("mode", ["real", "fake", "symbolic"])
+def test_views_can_be_traced(mode):
+    """A trace of the split and of ``rows_view`` holds for tensors that lie elsewhere in their storage."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from kareus_amd.operators import QKVPostProcessOp
+    from kareus_amd.backend import hip
+
+    s, b, ng, per, hd = 6, 2, 3, 4, 16
+    x = torch.randn(4, s, b, ng * (per + 2) * hd)
+    be = HipBackend.__new__(HipBackend)
+    be._n = hip.load_native()
+    op = QKVPostProcessOp(ng, ng * per, hd, grouped_query_view=True, backend="hip")
+
+    def split(m):
+        q, k, v = op.split(m)
+        return q + 0, k + 0, v + 0, be.rows_view(m) + 0
+
+    traced = make_fx(split, tracing_mode=mode)(x[1])
+    for part in (x[0], x[2], x[3].clone()):
+        f = part.view(s, b, ng, per + 2, hd)
+        want = f[..., :per, :], f[..., per, :], f[..., per + 1, :], part.view(s * b, -1)
+        assert all(torch.equal(a, c) for a, c in zip(traced(part), want))
+
+
 # ------------------------------------------------- what the Python side refuses, the native side leaves to it
 def _on_device(*shape, dtype=torch.bfloat16, device="cuda"):
     """A tensor of the device in all but its memory: a call that takes it ends before any launch."""
