@@ -146,9 +146,10 @@ class PartitionBase:
         self._overlap_slots: Dict[str, int] = _build_overlap_slots(self.comp_ops)
 
     def _plans(self) -> List[_OpPlan]:
-        plans = self.__dict__.get("_op_plans")
-        if plans is None or len(plans) != len(self.comp_ops):
-            ops = self.comp_ops
+        plans, ops = self.__dict__.get("_op_plans"), self.comp_ops
+        # (an op of the list, or an op's operator, may have been replaced since the last pass)
+        if plans is None or len(plans) != len(ops) or any(
+                [p.op is not op or p.operator is not op.operator for p, op in zip(plans, ops)]):
             plans = self._op_plans = [_OpPlan(op, ops[i + 1] if i + 1 < len(ops) else None) for i, op in enumerate(ops)]
         return plans
 

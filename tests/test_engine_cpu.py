@@ -566,3 +566,22 @@ def test_cleared_tensors_share_no_memory():
     a.resize_(4).fill_(1.0)
     b.resize_(4).fill_(2.0)
     assert a.tolist() == [1.0] * 4 and b.tolist() == [2.0] * 4
+
+
+def test_an_operator_replaced_between_passes_is_the_one_that_runs():
+    cfg = LayerConfig(**C1, num_layers=1, num_nanobatches=1, params_dtype=torch.float32, backend="eager")
+    model = LayerStack(cfg, seed=1234)
+    x = torch.randn(16, 1, cfg.hidden_size)
+    with torch.no_grad():
+        before = model(x)
+        norm = model.layers[0].pre_mlp_layernorm
+        other = type(norm)(cfg.hidden_size, cfg.layernorm_epsilon, dtype=torch.float32, backend="eager")
+        other.weight.copy_(3 * norm.weight)
+        found = [op for part in model.forward_partitions for op in part.comp_ops if op.operator is norm]
+        assert len(found) == 1
+        found[0].operator = other
+        after = model(x)
+        assert not torch.equal(before, after)
+        found[0].operator = norm
+        norm.weight.mul_(3)
+        assert torch.equal(model(x), after)
