@@ -51,7 +51,7 @@ class BackwardPartition(PartitionBase):
         return nxt
 
     def _execute(self, ctx, pre_ctx, protected: set) -> Dict[int, List]:
-        start, _end, sm_num, block_size = self._setup_comm(ctx.in_line)
+        start, _end, sm_num, block_size = self._setup_comm(ctx)
         store = ctx.tensor_store
         get, put = store.get, store.set
         timed = PartitionBase.timer is not None
@@ -96,7 +96,7 @@ class BackwardPartition(PartitionBase):
                     member_ctx.saved_tensors = None
                 if timed:
                     self._op_done(idx + k)
-            if last == start - 1 and not ctx.in_line:
+            if last == start - 1 and not self._in_order(ctx):
                 self.comm_op.event_record(self._here())
 
             put(group[-1].first_out, dx)

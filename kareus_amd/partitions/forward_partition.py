@@ -28,7 +28,7 @@ class ForwardPartition(PartitionBase):
             self._execute(ctx, pre_ctx)
 
     def _execute(self, ctx: NanoBatchContext, pre_ctx: NanoBatchContext) -> None:
-        start, _end, sm_num, block_size = self._setup_comm(ctx.in_line)
+        start, _end, sm_num, block_size = self._setup_comm(ctx)
         store = ctx.tensor_store
         get, put, needs = store.get, store.set, store.needs_grad
         sinks = ctx.output_sinks
@@ -79,7 +79,7 @@ class ForwardPartition(PartitionBase):
             if timed:
                 for j in range(k):
                     self._op_done(idx + j)
-            if last == start - 1 and not ctx.in_line:
+            if last == start - 1 and not self._in_order(ctx):
                 self.comm_op.event_record(self._here())
 
             tail = group[-1]

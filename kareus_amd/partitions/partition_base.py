@@ -158,6 +158,12 @@ class PartitionBase:
         nanobatch, or nanobatches in line), which ignores it."""
         return None if getattr(self.comm_op.operator, "comm_stream", self) is None else _current_stream()
 
+    def _in_order(self, ctx) -> bool:
+        """Whether the order of one stream already gives every edge of the schedule point: nanobatches in line, and an
+        operator that enqueues nothing anywhere.  One that does (its collective runs on a stream of its own) is told
+        and waited for as ever."""
+        return ctx.in_line and getattr(self.comm_op.operator, "enqueues_nothing", False)
+
     # -- schedule ---------------------------------------------------------------
     def load_schedule(self, schedule) -> None:
         config = getattr(schedule, self.partition_key, None) if self.partition_key else None
@@ -174,7 +180,7 @@ class PartitionBase:
             end = _resolve_slot(self._overlap_slots, end)
         return ((start, end), shape)
 
-    def _setup_comm(self, in_line: bool = False) -> Tuple[int, int, Optional[int], Optional[int]]:
+    def _setup_comm(self, ctx) -> Tuple[int, int, Optional[int], Optional[int]]:
         if self.comm_op is None:
             return -1, -1, None, None
         (start, end), (sm_num, block_size) = self._get_comm_config()
@@ -189,7 +195,7 @@ class PartitionBase:
             )
         if self.force_no_overlap:
             start = -1
-        if start == 0 and not in_line:
+        if start == 0 and not self._in_order(ctx):
             self.comm_op.event_record(self._here())
         return start, end, sm_num, block_size
 
@@ -218,19 +224,19 @@ class PartitionBase:
 
     def _launch_comm(self, pre_ctx, sm_num, block_size, *, backward: bool = False):
         """Release point reached earlier (event already recorded): wait on it, run."""
-        if not pre_ctx.in_line:
+        if not self._in_order(pre_ctx):
             self.comm_op.event_wait()
         return self._run_comm(pre_ctx, sm_num, block_size, backward)
 
     def _launch_comm_no_overlap(self, pre_ctx, sm_num, block_size, *, backward: bool = False):
         """No slot given: release only after all of this partition's compute."""
-        if not pre_ctx.in_line:
+        if not self._in_order(pre_ctx):
             self.comm_op.event_record(self._here())
             self.comm_op.event_wait()
         return self._run_comm(pre_ctx, sm_num, block_size, backward)
 
     def _sync_comm(self, pre_ctx: NanoBatchContext, comm_output, comm_extra_outputs) -> None:
-        if not pre_ctx.in_line:
+        if not self._in_order(pre_ctx):
             self.comm_op.sync(self._here())
         ports = self.comm_op.output_ports
         src = self.comm_op.input_ports

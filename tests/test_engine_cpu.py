@@ -585,3 +585,38 @@ def test_an_operator_replaced_between_passes_is_the_one_that_runs():
         found[0].operator = norm
         norm.weight.mul_(3)
         assert torch.equal(model(x), after)
+
+
+def test_a_collective_with_work_of_its_own_is_waited_for_in_line(monkeypatch):
+    """Nanobatches in line skip the events of the identity hand-over.  An operator that runs its collective on a stream of
+    its own gets every call of the protocol, in order, whether the nanobatches run in line or not."""
+    from kareus_amd.partitions import autograd_function
+    from kareus_amd.partitions.tensor_graph import CommunicationType
+
+    class Collective:
+        def __init__(self, log):
+            self.log, self.comm_stream = log, object()
+
+        def event_record(self, stream):
+            self.log.append("record")
+
+        def event_wait(self):
+            self.log.append("wait")
+
+        def fuser_forward(self, ctxs, x, **kw):
+            self.log.append("run")
+            return x, [()]
+
+        def sync(self, stream=None):
+            self.log.append("sync")
+
+    x, logs = torch.randn(16, 2, C1["hidden_size"]), {}
+    for in_line in (False, True):
+        monkeypatch.setattr(autograd_function, "_nanobatches_in_line", lambda config, hs: in_line)
+        model = LayerStack(LayerConfig(**C1, num_layers=1, num_nanobatches=2, params_dtype=torch.float32, backend="eager"),
+                           seed=1234)
+        logs[in_line] = []
+        model._assign_comm_operators(CommunicationType.ALL_REDUCE, [Collective(logs[in_line])] * 2)
+        model(x.clone().requires_grad_(True)).sum().backward()
+    assert logs[True] == logs[False] and logs[True].count("run") > 0
+    assert logs[True] == ["record", "wait", "run", "sync"] * logs[True].count("run")
