@@ -36,6 +36,16 @@ def _build(dims, layers, nnb, **kw):
     return model
 
 
+def _mode(streams):
+    """Nanobatches of these sizes run in line on the caller's stream unless the rule is switched off."""
+    return dict(in_line_below_ms=0.0) if streams else {}
+
+
+def _is_streamed(model, s, b):
+    c = model.config
+    return len(c.nanobatch_streams) == c.num_nanobatches and not c.nanobatches_in_line(s, b // c.num_nanobatches)
+
+
 def _run(model, x, go):
     for p in model.parameters():
         p.grad = None
@@ -63,10 +73,11 @@ def _rel(got, want):
     (R.LayerDims(3072, 3, 1, 128, 1024), 512, 4, 1),    # config 2 widths (3B TP=8 shard), short sequence
     (R.LayerDims(1024, 8, 2, 128, 896), 384, 4, 2),     # config 4 ratios (8 q / 2 kv heads), two layers
 ])
-@pytest.mark.parametrize("nnb", [1, 2, 4])
-def test_layer_matches_oracle(dims, s, b, layers, nnb):
+@pytest.mark.parametrize("nnb,streams", [(1, False), (2, False), (2, True), (4, False), (4, True)])
+def test_layer_matches_oracle(dims, s, b, layers, nnb, streams):
     x, go = _inputs(s, b, dims.hidden)
-    model = _build(dims, layers, nnb)
+    model = _build(dims, layers, nnb, **_mode(streams))
+    assert nnb == 1 or _is_streamed(model, s, b) is streams
     y, dx, grads = _run(model, x, go)
     ry, rdx, rgrads = _oracle(model, dims, x, go)
     worst = [_rel(y, ry), _rel(dx, rdx)]
@@ -104,12 +115,14 @@ def test_layer_with_hidden_dropout_matches_oracle_given_the_masks(dims, s, b):
     y2, dx2, grads2 = _run(recomputing, x, go)
     assert torch.equal(y, y2) and torch.equal(dx, dx2)
     assert all(torch.equal(a, c) for a, c in zip(grads[0], grads2[0]))
-    two = _build(dims, 1, 2, hidden_dropout=prob)
+    two, on_streams = _build(dims, 1, 2, hidden_dropout=prob), _build(dims, 1, 2, hidden_dropout=prob, **_mode(True))
+    assert not _is_streamed(two, s, b) and _is_streamed(on_streams, s, b)
     torch.manual_seed(22)
     ya, dxa, ga = _run(two, x, go)
-    torch.manual_seed(22)
-    yb, dxb, gb = _run(two, x, go)
-    assert torch.equal(ya, yb) and torch.equal(dxa, dxb) and all(torch.equal(a, c) for a, c in zip(ga[0], gb[0]))
+    for again in (two, on_streams, on_streams):
+        torch.manual_seed(22)
+        yb, dxb, gb = _run(again, x, go)
+        assert torch.equal(ya, yb) and torch.equal(dxa, dxb) and all(torch.equal(a, c) for a, c in zip(ga[0], gb[0]))
     assert not torch.equal(ya, y)
 
 
@@ -125,7 +138,8 @@ def test_layer_with_query_and_key_norms_matches_oracle(dims, s, b, nnb):
     gradient and all gradients, the two head-norm weights' included, against the oracle; recomputation and the
     nanobatch streams change no bit."""
     x, go = _inputs(s, b, dims.hidden)
-    model = _build(dims, 2, nnb, qk_layernorm=True)
+    model = _build(dims, 2, nnb, qk_layernorm=True, **_mode(True))
+    assert nnb == 1 or _is_streamed(model, s, b)
     gen = torch.Generator().manual_seed(9)
     heads = [("q_layernorm", "q_norm"), ("k_layernorm", "k_norm")]
     for layer in model.layers:
@@ -152,15 +166,17 @@ def test_layer_with_query_and_key_norms_matches_oracle(dims, s, b, nnb):
     plain = [{n: t for n, t in p.items() if n not in ("q_norm", "k_norm")} for p in params]
     without = R.stack_forward(x.bfloat16().float(), plain, dims, R.rope_table(s, dims.hd, dims.rope_base))
     assert _rel(without, ry)[0] > 2 * TOL       # the norms matter at this tolerance
-    other = _build(dims, 2, nnb, qk_layernorm=True, checkpoint_activations=True, use_streams=False)
-    other.load_state_dict(model.state_dict())
-    y2, dx2, grads2, extra2 = run(other)
-    assert torch.equal(y, y2) and torch.equal(dx, dx2)
-    for la, lb in zip(grads + extra, grads2 + extra2):
-        assert all(torch.equal(a, c) for a, c in zip(la, lb))
+    for kw in (dict(use_streams=False), {}, _mode(True)):   # one stream by choice, in line, streams
+        other = _build(dims, 2, nnb, qk_layernorm=True, checkpoint_activations=True, **kw)
+        other.load_state_dict(model.state_dict())
+        y2, dx2, grads2, extra2 = run(other)
+        assert torch.equal(y, y2) and torch.equal(dx, dx2)
+        for la, lb in zip(grads + extra, grads2 + extra2):
+            assert all(torch.equal(a, c) for a, c in zip(la, lb))
 
 
-def test_streams_recompute_and_schedule_do_not_change_results(fixtures_dir):
+@pytest.mark.parametrize("streams", [True, False])
+def test_streams_recompute_and_schedule_do_not_change_results(fixtures_dir, streams):
     dims = R.LayerDims(1024, 8, 2, 128, 896)
     x, go = _inputs(256, 4, dims.hidden)
     base = _run(_build(dims, 2, 2, use_streams=False), x, go)
@@ -171,12 +187,18 @@ def test_streams_recompute_and_schedule_do_not_change_results(fixtures_dir):
             for ga, gb in zip(la, lb):
                 assert torch.equal(ga, gb)
 
-    same(_run(_build(dims, 2, 2, use_streams=True), x, go))            # concurrent streams: bit-identical
-    same(_run(_build(dims, 2, 2, checkpoint_activations=True), x, go))  # recompute: bit-identical
+    model = _build(dims, 2, 2, use_streams=True, **_mode(streams))
+    assert _is_streamed(model, 256, 4) is streams
+    same(_run(model, x, go))                                            # concurrent streams, or in line: bit-identical
+    named = _build(dims, 2, 2, nanobatch_streams=[torch.cuda.Stream(), torch.cuda.Stream()])
+    assert _is_streamed(named, 256, 4)
+    same(_run(named, x, go))                                            # streams that the caller names
+    same(_run(_build(dims, 2, 2, checkpoint_activations=True, **_mode(streams)), x, go))  # recompute: bit-identical
     model = _build(dims, 2, 2, checkpoint_activations=True)
     sch = PipelineCommScheduler(os.path.join(fixtures_dir, "scheds_pipeline_02328.py"), pp_rank=0,
                                 num_microbatches=8, use_activation_checkpointing=True)
     model.config.kareus_scheduler = sch
+    assert _is_streamed(model, 256, 4)           # a plan is about the streams
     for p in model.parameters():
         p.grad = None
     xd = x.to("cuda", torch.bfloat16).requires_grad_(True)
@@ -189,7 +211,7 @@ def test_streams_recompute_and_schedule_do_not_change_results(fixtures_dir):
     torch.cuda.synchronize()
     assert torch.equal(y.detach(), base[0]) and torch.equal(xd.grad, base[1])  # any legal schedule: same numbers
     # repeated steps are deterministic
-    m2 = _build(dims, 2, 4)
+    m2 = _build(dims, 2, 4, **_mode(streams))
     r1, r2 = _run(m2, x, go), _run(m2, x, go)
     assert torch.equal(r1[0], r2[0]) and torch.equal(r1[1], r2[1]) and torch.equal(r1[2][1][4], r2[2][1][4])
 

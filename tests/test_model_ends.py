@@ -187,11 +187,13 @@ def test_cross_entropy_kernels(rows, vocab):
 
 
 @gpu
-def test_device_model_matches_oracle():
+@pytest.mark.parametrize("streams", [True, False])
+def test_device_model_matches_oracle(streams):
     global DIMS
     dims = R.LayerDims(hidden=512, nq=4, nkv=2, hd=128, ffn=640)
     cfg = LayerConfig(hidden_size=512, num_attention_heads=4, num_query_groups=2, kv_channels=128,
-                      ffn_hidden_size=640, num_layers=2, num_nanobatches=2, backend="hip")
+                      ffn_hidden_size=640, num_layers=2, num_nanobatches=2, backend="hip",
+                      **(dict(in_line_below_ms=0.0) if streams else {}))   # (in line at this size without it)
     g = torch.Generator().manual_seed(7)
     ids, labels = torch.randint(0, 2048, (4, 256), generator=g), torch.randint(0, 2048, (4, 256), generator=g)
     model = GPTModelShard(cfg, vocab_rows=2048, device="cuda", seed=1234)

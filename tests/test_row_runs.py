@@ -152,7 +152,8 @@ def test_input_gradient_with_swiglu_backward_reads_runs(be, s, b, r, f, h):
 # ---- the whole layer: several sequences per nanobatch, no copy at either end -------------------------------
 @gpu
 @pytest.mark.parametrize("b,nnb", [(8, 2), (4, 2), (16, 2), (8, 4)])
-def test_layer_with_wide_nanobatches_equals_the_copying_run(monkeypatch, b, nnb):
+@pytest.mark.parametrize("streams", [True, False])
+def test_layer_with_wide_nanobatches_equals_the_copying_run(monkeypatch, b, nnb, streams):
     """Configuration 2's widths (3072 hidden, 3 query / 1 KV head, ffn 1024), 4 / 2 / 8 / 2 sequences per
     nanobatch: the run that addresses the nanobatch slices in place gives the bits of the run that copies
     them into dense tensors first (the reference's way), for outputs, input gradients and every weight
@@ -162,10 +163,11 @@ def test_layer_with_wide_nanobatches_equals_the_copying_run(monkeypatch, b, nnb)
 
     s, h = 256, 3072
     cfg = dict(hidden_size=h, num_attention_heads=3, num_query_groups=1, kv_channels=128, ffn_hidden_size=1024,
-               num_layers=2, num_nanobatches=nnb, backend="hip")
+               num_layers=2, num_nanobatches=nnb, backend="hip", **(dict(in_line_below_ms=0.0) if streams else {}))
 
     def run():
         model = LayerStack(LayerConfig(**cfg), device=DEV, seed=1234)
+        assert not (streams and model.config.nanobatches_in_line(s, b // nnb))
         for layer in model.layers:
             for op in (layer.linear_qkv, layer.linear_proj, layer.linear_fc1, layer.linear_fc2):
                 op.split_k = None

@@ -153,14 +153,15 @@ def test_pairs_the_backend_turns_down(be):
         be.linear_wgrad_segments([d[:96] for d in dys], [x[:96] for x in xs])
 
 
-def _layer_grads(whole, nnb, b, s=256, at_end=None, recompute=False):
+def _layer_grads(whole, nnb, b, s=256, at_end=None, recompute=False, streams=True):
     from kareus_amd import LayerConfig, LayerStack
 
     cfg = LayerConfig(hidden_size=1024, num_attention_heads=8, num_query_groups=2, kv_channels=128,
                       ffn_hidden_size=1792, num_layers=2, num_nanobatches=nnb, backend="hip",
                       wgrad_over_all_nanobatches=whole, wgrad_launches_at_end=at_end,
-                      checkpoint_activations=recompute)
+                      checkpoint_activations=recompute, **(dict(in_line_below_ms=0.0) if streams else {}))
     model = LayerStack(cfg, device=DEV, seed=1234)
+    assert len(cfg.nanobatch_streams) == nnb and cfg.nanobatches_in_line(s, b // nnb) is not streams
     g = torch.Generator().manual_seed(7)
     x = torch.randn(s, b, 1024, generator=g).to(DEV, torch.bfloat16).requires_grad_(True)
     go = torch.randn(s, b, 1024, generator=g).to(DEV, torch.bfloat16)
@@ -180,25 +181,28 @@ def _layer_grads(whole, nnb, b, s=256, at_end=None, recompute=False):
 
 @gpu
 @pytest.mark.parametrize("nnb,b", [(4, 4), (2, 4), (2, 2)])
-def test_layer_step_with_one_weight_gradient_per_layer(nnb, b):
-    """Two layers, nanobatches on their own streams: outputs and input gradients do not depend on how the
+@pytest.mark.parametrize("streams", [True, False])
+def test_layer_step_with_one_weight_gradient_per_layer(nnb, b, streams):
+    """Two layers, nanobatches on their own streams or in line: outputs and input gradients do not depend on how the
     weight gradients are summed (bit-equal); the weight gradients agree with the per-nanobatch
     accumulation within bf16 rounding and are the same on every pass."""
-    y_w, dx_w, g_w = _layer_grads(True, nnb, b, at_end=False)
-    y_p, dx_p, g_p = _layer_grads(False, nnb, b)
+    y_w, dx_w, g_w = _layer_grads(True, nnb, b, at_end=False, streams=streams)
+    y_p, dx_p, g_p = _layer_grads(False, nnb, b, streams=streams)
     assert torch.equal(y_w, y_p) and torch.equal(dx_w, dx_p)
     for a, c in zip(g_w, g_p):
         assert (a.float() - c.float()).abs().max() <= TOL * c.float().abs().max()
-    # issued at the end of the backward pass instead of where the last nanobatch delivers: the same launches
-    y_e, dx_e, g_e = _layer_grads(True, nnb, b, at_end=True)
+    # issued at the end of the backward pass instead of where the last nanobatch delivers (in line: there either
+    # way): the same launches
+    y_e, dx_e, g_e = _layer_grads(True, nnb, b, at_end=True, streams=streams)
     assert torch.equal(y_e, y_w) and torch.equal(dx_e, dx_w) and all(torch.equal(a, c) for a, c in zip(g_e, g_w))
 
 
 @gpu
-def test_recomputed_activations_feed_the_same_weight_gradient():
+@pytest.mark.parametrize("streams", [True, False])
+def test_recomputed_activations_feed_the_same_weight_gradient(streams):
     """Activation recompute rebuilds the saved inputs inside the backward pass; the one weight-gradient launch
-    per layer, issued at the end of that pass, must read them as it reads the saved ones."""
-    kept = _layer_grads(True, 4, 4)
-    again = _layer_grads(True, 4, 4, recompute=True)
+    per layer, issued at the end of that pass (on streams), must read them as it reads the saved ones."""
+    kept = _layer_grads(True, 4, 4, streams=streams)
+    again = _layer_grads(True, 4, 4, recompute=True, streams=streams)
     assert torch.equal(kept[0], again[0]) and torch.equal(kept[1], again[1])
     assert all(torch.equal(a, c) for a, c in zip(kept[2], again[2]))
