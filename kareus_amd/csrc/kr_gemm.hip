@@ -1161,6 +1161,33 @@ extern "C" size_t kr_gemm_workspace_bytes_shared(int layout, int M, int N, int K
 }
 
 namespace {
+// The tile and the cuts of a launch: held_bytes is the workspace it may cut into (0: none), beside other streams the
+// compute-unit time of the launch counts, hardly its latency.
+Plan launch_plan(int M, int N, int K, int epi, bool shared, int cus, size_t held_bytes) {
+  int max_splits = 1;
+  if (held_bytes > 0 && epi == KR_GEMM_EPI_NONE) {
+    const size_t held = held_bytes / ((size_t)M * N * sizeof(float));
+    max_splits = held > 16 ? 16 : (int)held;
+    if (max_splits < 1) max_splits = 1;
+  }
+  return choose_plan(M, N, K, shared ? 0.1f : 1.f, cus, max_splits, epi != KR_GEMM_EPI_NONE,
+                     epi != KR_GEMM_EPI_SWIGLU || N % 128 == 0);
+}
+}  // namespace
+
+extern "C" int kr_gemm_plan(int M, int N, int K, int epilogue, int max_cus, size_t workspace_bytes, int* tile_rows,
+                            int* splits) {
+  if (!tile_rows || !splits || M <= 0 || N <= 0 || K <= 0 || max_cus < 0) return KR_EINVAL;
+  const int num_cus = device_compute_units();
+  const Plan plan = launch_plan(M, N, K, epilogue & ~KR_GEMM_BESIDE_OTHER_STREAMS,
+                                (epilogue & KR_GEMM_BESIDE_OTHER_STREAMS) != 0,
+                                max_cus > 0 && max_cus < num_cus ? max_cus : num_cus, workspace_bytes);
+  *tile_rows = plan.small ? 32 * WT_SMALL : 32 * WT_LARGE;
+  *splits = plan.splits;
+  return KR_OK;
+}
+
+namespace {
 int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, const void* B,
                   int64_t ldb, void* C, int64_t ldc, int accumulate, void* workspace,
                   size_t workspace_bytes, void* stream, const Fused& fu) {
@@ -1224,15 +1251,7 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
   // cuts of the contraction the caller's workspace can hold (a caller that wants fewer says so by
   // passing the smaller workspace kr_gemm_workspace_bytes_shared sizes); a fused epilogue works on
   // finished sums and is never cut
-  int max_splits = 1;
-  if (ws != nullptr && fu.epi == KR_GEMM_EPI_NONE && fu.runs.c_sh == 0) {
-    const size_t held = workspace_bytes / ((size_t)M * N * sizeof(float));
-    max_splits = held > 16 ? 16 : (int)held;
-    if (max_splits < 1) max_splits = 1;
-  }
-  // beside other streams the compute-unit time of the launch counts, hardly its latency
-  const Plan plan = choose_plan(M, N, K, fu.shared ? 0.1f : 1.f, cus, max_splits, fu.epi != KR_GEMM_EPI_NONE,
-                                fu.epi != KR_GEMM_EPI_SWIGLU || N % 128 == 0);
+  const Plan plan = launch_plan(M, N, K, fu.epi, fu.shared, cus, ws != nullptr && fu.runs.c_sh == 0 ? workspace_bytes : 0);
   const int wn = fu.epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn;
   const int sp = plan.splits;
   if (fu.epi == KR_GEMM_EPI_SWIGLU_BWD) {

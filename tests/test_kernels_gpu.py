@@ -3,6 +3,7 @@ seeded inputs.  Integer-exact where the arithmetic is exact (residual add, index
 bf16 tolerance: max |err| / max |ref| <= 2e-2 against the fp32 oracle evaluated on the bf16-rounded
 inputs (the stated bf16 tolerance of the benchmark); observed errors are ~3e-3, one bf16 ulp."""
 
+import ctypes
 import math
 
 import pytest
@@ -276,31 +277,85 @@ def test_gemm_plan_does_not_change_the_sums_much(be):
             assert rel(acc, ref + c0.float()) <= TOL
 
 
+def _gemm_plan(be, m, n, k, epilogue=0, workspace=0):
+    rows, splits = ctypes.c_int(), ctypes.c_int()
+    assert be.lib.kr_gemm_plan(m, n, k, epilogue, 0, workspace, ctypes.byref(rows), ctypes.byref(splits)) == 0
+    return rows.value, splits.value
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 8, 8), (128, 128, 64), (136, 264, 72), (120, 128, 128), (520, 1024, 200),
                                    (264, 136, 584), (136, 640, 720), (256, 1000, 1096),   # the deep ring, contraction tails
                                    (512, 3584, 1024),     # one round of small tiles, more than one per compute unit
                                    (2048, 3456, 136)])    # 432 small tiles
 def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
-    """Outputs of few tiles are computed in 128 x 128 tiles.  A launch held to one compute unit takes the large
-    tiles; every element is the same chain of matrix instructions in both, so the bits are the same."""
+    """Outputs of few tiles are computed in 128 x 128 tiles.  The same rows and columns as a corner of an output of 192
+    and more large tiles, which is computed in them: every element is the same chain of matrix instructions in both, so
+    the bits are the same.  (Both plans are asserted.)"""
+    def embed(t, rows=None, cols=None):
+        r, c = max(rows or t.shape[0], t.shape[0]), max(cols or t.shape[1], t.shape[1])
+        big = rnd(r, c, scale=0.05, seed=67)
+        big[:t.shape[0], :t.shape[1]] = t
+        return big
+
+    R_, C_ = 4096, 3072   # 16 x 12 large tiles at the least
     x, w, dy = rnd(m, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(m, n, seed=63)
-    for layout, a, b, shape in ((0, x, w, (m, n, k)), (1, dy, w, (m, k, n)), (2, dy, x, (n, k, m))):
-        one = dict(split_k=None, max_cus=1)
-        got = be.gemm(layout, a, b, *shape, split_k=None)
-        assert torch.equal(got, be.gemm(layout, a, b, *shape, **one))
-        base = rnd(shape[0], shape[1], seed=64)
-        assert torch.equal(be.gemm(layout, a, b, *shape, out=base.clone(), accumulate=True, split_k=None),
-                           be.gemm(layout, a, b, *shape, out=base.clone(), accumulate=True, **one))
-        wide = torch.zeros(shape[0], shape[1] + 8, device=DEV, dtype=torch.bfloat16)
-        be.gemm(layout, a, b, *shape, out=wide[:, :shape[1]], split_k=None)
-        assert torch.equal(wide[:, :shape[1]], got) and not wide[:, shape[1]:].any()
+    for layout, a, b, (p, q, c) in ((0, x, w, (m, n, k)), (1, dy, w, (m, k, n)), (2, dy, x, (n, k, m))):
+        big = (max(p, R_), max(q, C_), c)
+        assert _gemm_plan(be, p, q, c) == (128, 1) and _gemm_plan(be, *big) == (256, 1)
+        big_a = embed(a, cols=R_) if layout == 2 else embed(a, rows=R_)
+        big_b = embed(b, rows=C_) if layout == 0 else embed(b, cols=C_)
+        got = be.gemm(layout, a, b, p, q, c, split_k=None)
+        assert torch.equal(got, be.gemm(layout, big_a, big_b, *big, split_k=None)[:p, :q])
+        base = rnd(p, q, seed=64)
+        assert torch.equal(be.gemm(layout, a, b, p, q, c, out=base.clone(), accumulate=True, split_k=None),
+                           be.gemm(layout, big_a, big_b, *big, out=embed(base, R_, C_), accumulate=True, split_k=None)[:p, :q])
+        wide = torch.zeros(p, q + 8, device=DEV, dtype=torch.bfloat16)
+        be.gemm(layout, a, b, p, q, c, out=wide[:, :q], split_k=None)
+        assert torch.equal(wide[:, :q], got) and not wide[:, q:].any()
     assert rel(be.linear_fwd(x, w), x.float() @ w.float().t()) <= TOL
+    big_x, big_w, big = embed(x, rows=R_), embed(w, rows=C_), (max(m, R_), max(n, C_), k)
     res = rnd(m, n, seed=65)
-    assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(x, w, residual=res, max_cus=1))
-    if be.can_fuse_swiglu(n):
-        y, y1 = (torch.empty(m, n // 2, device=DEV, dtype=torch.bfloat16) for _ in range(2))
-        assert torch.equal(be.linear_fwd(x, w, swiglu_out=y), be.linear_fwd(x, w, swiglu_out=y1, max_cus=1))
-        assert torch.equal(y, y1)
+    assert _gemm_plan(be, m, n, k, 1)[0] == 128 and _gemm_plan(be, *big, 1)[0] == 256
+    assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(big_x, big_w, residual=embed(res, R_, C_))[:m, :n])
+
+
+@pytest.mark.parametrize("m,f,k", [(8, 64, 64), (128, 320, 128), (136, 448, 200), (520, 512, 1096), (512, 1792, 1024)])
+def test_gemm_small_tiles_with_swiglu_have_the_bits_of_the_large_ones(be, m, f, k):
+    """The SwiGLU epilogues, forward (gate and up columns of a tile side by side) and backward, in the same way."""
+    M, F = max(m, 4096), max(3584, f)      # 16 x 28 large tiles: gate and up
+    x, gate, up = rnd(M, k, seed=61), rnd(F, k, scale=0.05, seed=62), rnd(F, k, scale=0.05, seed=63)
+    xs, ws = x[:m].contiguous(), torch.cat([gate[:f], up[:f]])
+    if be.can_fuse_swiglu(2 * f):
+        assert _gemm_plan(be, m, 2 * f, k, 2)[0] == 128 and _gemm_plan(be, M, 2 * F, k, 2)[0] == 256
+        y, big_y = (torch.empty(r, c, device=DEV, dtype=torch.bfloat16) for r, c in ((m, f), (M, F)))
+        got, big = be.linear_fwd(xs, ws, swiglu_out=y), be.linear_fwd(x, torch.cat([gate, up]), swiglu_out=big_y)
+        assert torch.equal(got[:, :f], big[:m, :f]) and torch.equal(got[:, f:], big[:m, F:F + f]) and torch.equal(y, big_y[:m, :f])
+    # backward: the gradient of the activation, [m, f] = dy [m, k] . W [k, f], never stored; out [m, 2 f]
+    dy, w, pre = rnd(M, k, seed=66), rnd(k, F, scale=0.05, seed=67), rnd(M, 2 * F, seed=68)
+    assert _gemm_plan(be, m, f, k, 4)[0] == 128 and _gemm_plan(be, M, F, k, 4)[0] == 256
+    pre_s = torch.cat([pre[:m, :f], pre[:m, F:F + f]], dim=1)
+    got = be.linear_dgrad(dy[:m].contiguous(), w[:, :f].contiguous(), swiglu_bwd_x=pre_s)
+    big = be.linear_dgrad(dy, w, swiglu_bwd_x=pre)
+    assert torch.equal(got[:, :f], big[:m, :f]) and torch.equal(got[:, f:], big[:m, F:F + f])
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("steps,tail", [(151, 64), (151, 8), (152, 40), (153, 64), (153, 24), (154, 8), (155, 64), (159, 56)])
+def test_gemm_deep_ring_cut_into_short_last_ranges(be, layout, steps, tail):
+    """Small tiles alone on their compute units request four K-steps ahead; cut sixteen ways, ``steps`` K-steps leave 1, 2, 3,
+    4, 5 and 9 for the last range (10 for the others), the last one of ``tail`` rows.  Operands of -1, 0 and 1: every
+    sum is a small whole number, exact in fp32 in any order, so the result is the exact product rounded to bf16 once."""
+    m, n, k = 128, 120, (steps - 1) * 64 + tail
+    ws = be.lib.kr_gemm_workspace_bytes(layout, m, n, k)
+    assert ws == 16 * m * n * 4 and _gemm_plan(be, m, n, k, workspace=ws) == (128, 16)
+    assert k // 64 // 16 > 8                                  # the deep ring's condition
+    g = torch.Generator().manual_seed(steps)
+    a, b = (torch.randint(-1, 2, s, generator=g).to(DEV, torch.bfloat16) for s in (((k, m) if layout == 2 else (m, k)),
+                                                                                   ((n, k) if layout == 0 else (k, n))))
+    want = (a.double().t() if layout == 2 else a.double()) @ (b.double().t() if layout == 0 else b.double())
+    assert torch.equal(be.gemm(layout, a, b, m, n, k), want.to(torch.bfloat16))
+    base = torch.randint(-3, 4, (m, n), generator=g).to(DEV, torch.bfloat16)
+    assert torch.equal(be.gemm(layout, a, b, m, n, k, out=base.clone(), accumulate=True), (want + base.double()).to(torch.bfloat16))
 
 
 def test_gemm_is_reproducible(be):
@@ -630,12 +685,18 @@ def test_attention_padded_into_the_mfma_kernels_equals_the_whole_tile_call(be):
 @pytest.mark.parametrize("s,b,nq,nkv,hd", [(8, 1, 2, 1, 64), (127, 1, 2, 2, 64), (128, 1, 2, 1, 64), (129, 2, 4, 1, 64),
                                             (136, 1, 3, 1, 128), (200, 1, 4, 2, 64), (248, 2, 2, 1, 128),
                                             (320, 1, 4, 4, 64), (520, 1, 3, 1, 128), (1000, 2, 32, 8, 64),
-                                            (1000, 8, 8, 2, 128), (1024, 2, 32, 8, 64)])
+                                            (1000, 8, 8, 2, 128), (1024, 2, 32, 8, 64),
+                                            # an odd number of 128-row tiles, more than 1024 of them over all heads: dQ
+                                            # unsplit in 128-query tiles
+                                            (128, 33, 32, 8, 64), (100, 33, 32, 8, 64), (300, 11, 32, 8, 64),
+                                            (100, 33, 32, 8, 128), (300, 11, 32, 8, 128), (128, 33, 32, 8, 128)])
 @pytest.mark.parametrize("beside", [False, True])
 def test_attention_in_place_at_head_dimension_64_and_ragged_lengths(be, s, b, nq, nkv, hd, beside):
     """The MFMA kernels on tensors as they lie: tiles of 128 rows of 64 channels (an odd number of them for the split
-    forms, none at all for a part), last tiles that the sequence ends in, both forms of every kernel
-    (``beside`` takes the unsplit ones; so do the last three shapes).  What lies behind the sequence in memory is
+    forms, none at all for a part), last tiles that the sequence ends in, every form of every kernel: ``beside`` takes
+    the unsplit forward and dK/dV and, at whole 256-query tiles, the dQ kernel of 64 rows per wave, and so do the three
+    shapes of 1000 and 1024 without it; dQ in 128-query tiles is split in two at few workgroups and unsplit in
+    the last six shapes.  What lies behind the sequence in memory is
     infinite: it must not be read into a result.  Tolerances as for every attention shape (bf16 operands, fp32 sums)."""
     base, q, k, v = _grouped(s + 3, b, nq, nkv, hd, seed=120)
     base[s:] = float("inf")
