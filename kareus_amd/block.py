@@ -67,7 +67,7 @@ class LayerConfig:
     num_nanobatches: int = 2
     params_dtype: torch.dtype = torch.bfloat16
     backend: str = "hip"
-    use_streams: bool = True
+    use_streams: bool = True   # (small nanobatches run in line all the same: in_line_below_ms)
     checkpoint_activations: bool = False
     # weight gradients of all nanobatches are summed inside the wgrad GEMM instead of by autograd
     fuse_wgrad_accumulation: bool = True
@@ -107,10 +107,12 @@ class LayerConfig:
     # Nanobatches on streams of their own cost the host 0.9-1.0 ms per nanobatch and layer, forward and backward
     # (launches, and above all the event waits of the schedule points), one after the other on one stream 0.6 ms.
     # Where the device needs less than that for a nanobatch, the streams' overlap hides nothing and the step takes
-    # as long as the host: on one stream it is shorter, and the launches, alone on the device, are planned for
-    # their latency.  Measured, streams against one stream, two / four nanobatches: small layer (512 hidden) 256-2048
+    # as long as the host: on one stream it is shorter, and the GEMMs, alone on the device, are planned for
+    # their latency (the attention keeps the forms the nanobatch count sets, see set_tensor_parallel_group: a run in
+    # line has the bits of a run on one stream by choice).  Measured, streams against one stream, two / four nanobatches: small layer (512 hidden) 256-2048
     # tokens 1.5x / 1.5x, 8B shard of four 1024 tokens 1.48x / 1.32x, 2048 tokens 1.13x / 0.98x, 4096 tokens 0.88x / 0.86x,
-    # 3B layer 512 tokens 1.41x / 1.31x, 1024 tokens 1.18x / 1.01x, 8B layer 256 tokens 1.20x / 0.84x.
+    # 3B layer 512 tokens 1.41x / 1.31x, 1024 tokens 1.18x / 1.01x, 8B layer 256 tokens 1.20x / 0.84x.  The line lies
+    # where four nanobatches stop gaining; it does not look at their number, so two of 1.13x to 1.20x stay on streams.
     # 0: every pass uses the streams.
     in_line_below_ms: float = 0.65
 
