@@ -12,6 +12,7 @@
 // code other than KR_OK from the library raises.  From the first allocation to the launch the interpreter is
 // free for other threads.  Nothing is kept between calls except how much workspace a GEMM shape asks for,
 // which is a pure function of its sizes.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
@@ -80,12 +81,15 @@ struct WithoutInterpreter {
   ~WithoutInterpreter() { PyEval_RestoreThread(state); }
 };
 
+// exceptions leave as PyTorch's own bindings let them out: out of memory as torch.OutOfMemoryError
 template <typename F>
 PyObject* guarded(F&& f) {
   try {
     return f();
-  } catch (const std::exception& e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (const PythonError&) {
+    return nullptr;
+  } catch (...) {
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }

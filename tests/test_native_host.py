@@ -170,6 +170,25 @@ def test_split_and_budget_may_be_any_truth_value_and_any_number():
 
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_running_out_of_memory_is_torchs_own_error():
+    """(A limit on this process's share, so that nothing really runs out.)"""
+    n, x = load_native(), torch.ones(8192, 8192, device="cuda", dtype=torch.bfloat16)
+    gamma = torch.ones(8192, device="cuda", dtype=torch.bfloat16)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (32 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            n.rmsnorm_fwd(x, gamma, 1e-5)                              # a result of 128 MiB
+        with pytest.raises(torch.OutOfMemoryError):
+            n.gemm(0, x, x, 8192, 8192, 8192, None, False, 0, None, None, None, 0)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
 @pytest.mark.parametrize("what", ["gemm", "wgrad", "rotary"])
 def test_other_threads_run_during_a_launch(what):
     """With a switch interval that never ends, another thread gets the interpreter only where the launching thread lets
