@@ -258,7 +258,7 @@ class HipBackend:
         ``max_cus``: compute-unit budget of the launch (0 = the whole device).
         ``swiglu_bwd_x`` ([m, 2n], layout NN): the product is the gradient of a SwiGLU output and
         is not stored; ``out`` ([m, 2n]) receives the gradient of the activation's input instead."""
-        if max_cus == 0:
+        if max_cus == 0 and a.is_cuda:
             reserved = reserved_compute_units()
             if reserved:
                 max_cus = max(self._num_cus(a.device) - reserved, 8)
@@ -396,7 +396,7 @@ class HipBackend:
         microbatch, each pair read where it lies (``wgrad_segments_ok`` says whether the pairs qualify)."""
         max_cus = 0
         reserved = reserved_compute_units()
-        if reserved:
+        if reserved and len(dys) and dys[0].is_cuda:
             max_cus = max(self._num_cus(dys[0].device) - reserved, 8)
         done = self._n.wgrad_segments(dys, xs, out, accumulate, self._split_code(split_k), max_cus)
         if done is not None:

@@ -168,6 +168,18 @@ def test_split_and_budget_may_be_any_truth_value_and_any_number():
         assert be._n.args[8] == code and type(be._n.args[12]) is int
 
 
+def test_a_reservation_does_not_get_in_front_of_the_checks():
+    from kareus_amd.backend import reserve_compute_units
+
+    be, x = _backend(), torch.zeros(64, 64, dtype=torch.bfloat16)
+    with reserve_compute_units(16):
+        with pytest.raises(RuntimeError, match="needs tensors on the HIP device"):
+            be.gemm(0, x, x, 64, 64, 64)
+        for dys, xs in (([x], [x]), ([], [])):
+            with pytest.raises(RuntimeError, match="operand pairs must be"):
+                be.linear_wgrad_segments(dys, xs)
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
 def test_running_out_of_memory_is_torchs_own_error():
