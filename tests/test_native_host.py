@@ -236,3 +236,111 @@ def test_other_threads_run_during_a_launch(what):
         thread.join()
     torch.cuda.synchronize()
     assert got >= 3, f"{launched} launches, {got} turns of the other thread"
+
+
+# ------------------------------------------------- both sides give the same bits
+class _Off:
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _forms(be, dev="cuda"):
+    """(name, function of the native side, call): every form a layer uses, and the odd ones beside them."""
+    g = torch.Generator().manual_seed(3)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(dev, torch.bfloat16)
+    new = lambda *shape: torch.zeros(*shape, device=dev, dtype=torch.bfloat16)
+    m, n, k = 264, 320, 136
+    x, w, dy = rnd(m, k), rnd(n, k), rnd(m, n)
+    wide, runs, deep = rnd(m, 2 * k), rnd(132, 4, k)[:, 1:3], rnd(2, 2, 66, k)
+    res, res_runs, add_runs = rnd(m, n), rnd(132, 4, n)[:, 2:4], rnd(132, 4, k)[:, 0:2]
+    long_dy, long_x = rnd(4096, 128), rnd(4096, 136)   # cut
+    for split in (True, False, None):
+        yield f"forward {split}", "gemm", lambda s=split: be.linear_fwd(x, w, split_k=s)
+        yield f"input gradient {split}", "gemm", lambda s=split: be.linear_dgrad(dy, w, split_k=s)
+        yield f"weight gradient {split}", "gemm", lambda s=split: be.linear_wgrad(dy, x, split_k=s)
+        yield f"cut weight gradient {split}", "gemm", lambda s=split: be.linear_wgrad(long_dy, long_x, split_k=s)
+        yield f"pieces {split}", "wgrad_segments", lambda s=split: be.linear_wgrad_segments(
+            [long_dy[:1024], long_dy[1024:2048]], [long_x[:1024], long_x[1024:2048]], split_k=s)
+    yield "row stride", "gemm", lambda: be.linear_fwd(wide[:, k:], w)
+    yield "budget", "gemm", lambda: be.linear_fwd(x, w, max_cus=9)
+    yield "residual", "gemm", lambda: be.linear_fwd(x, w, residual=res)
+    yield "residual in runs", "gemm", lambda: be.linear_fwd(x, w, residual=res_runs)
+    yield "output in runs", "gemm", lambda: be.linear_fwd(x, w, residual=res, out=new(132, 4, n)[:, 0:2])
+    yield "output with a row stride", "gemm", lambda: be.linear_fwd(x, w, out=new(m, n + 8)[:, :n])
+    yield "accumulated", "gemm", lambda: be.linear_wgrad(dy, x, out=torch.ones(n, k, device=dev, dtype=torch.bfloat16), accumulate=True)
+    yield "gradient in runs", "gemm", lambda: be.linear_dgrad(res_runs, w)
+    yield "weight gradient of runs", "gemm", lambda: be.linear_wgrad(res_runs, x)
+    y1 = new(m, n // 2)
+    yield "swiglu", "gemm", lambda: (be.linear_fwd(x, w, swiglu_out=y1), y1)
+    pre = rnd(m, 2 * k)
+    yield "swiglu backward", "gemm", lambda: be.linear_dgrad(dy, w, swiglu_bwd_x=pre)
+    gamma = rnd(k)
+    for name, t in (("dense", x), ("row stride", wide[:, k:]), ("runs", runs), ("four dimensions", deep)):
+        yield f"norm {name}", "rmsnorm_fwd", lambda t=t: be.rmsnorm_fwd(t, gamma, 1e-5)
+        rstd = be.rmsnorm_fwd(t, gamma, 1e-5)[1]
+        yield f"norm backward {name}", "rmsnorm_bwd", lambda t=t, r=rstd: be.rmsnorm_bwd(x, t, r, gamma)
+    rstd = be.rmsnorm_fwd(runs, gamma, 1e-5)[1]
+    part = torch.zeros(be.rmsnorm_partial_rows(m, k), k, device=dev)
+    yield "norm backward, all in runs", "rmsnorm_bwd", lambda: (
+        be.rmsnorm_bwd(x, runs, rstd, gamma, residual_grad=add_runs, out=new(132, 4, k)[:, 2:4], partials_out=part)[0], part)
+    for hd, s in ((64, 200), (128, 128), (128, 72), (96, 40)):
+        table = torch.randn(s + 8, 1, 1, hd, generator=g).to(dev)
+        buf = rnd(s, 2, 2, 6, hd)
+        q, kk, v = buf[:, :, :, :4], buf[:, :, :, 4], buf[:, :, :, 5]
+        do = rnd(s, 2, 8, hd)
+        for back in (False, True):
+            def rope(buf=buf, table=table, back=back):
+                t = buf.clone()
+                be.rope_fused_inplace(t, 4, table, back)
+                return t
+            yield f"rotary {hd} {s} {back}", "rope_fused", rope
+        for kw in ({}, dict(beside_other_streams=True), dict(general_kernels=True)):
+            yield f"attention {hd} {s} {kw}", "attn_fwd", lambda a=(q, kk, v), kw=kw: be.attn_fwd(*a, 0.1, **kw)
+            dense = (q.flatten(2, 3).contiguous(), kk.contiguous(), v)
+            yield f"attention, dense {hd} {s} {kw}", "attn_fwd", lambda a=dense, kw=kw: be.attn_fwd(*a, 0.1, **kw)
+            o, lse = be.attn_fwd(q, kk, v, 0.1, **kw)
+            yield f"attention backward {hd} {s} {kw}", "attn_bwd", lambda a=(do, q, kk, v, o, lse), kw=kw: be.attn_bwd(*a, 0.1, **kw)
+    x3, r3 = rnd(33, 8, k), rnd(33, 8, k)
+    def dropped(out=None):
+        torch.manual_seed(5)
+        return be.dropout_add(x3, r3, 0.3, out=out)
+    yield "dropout", "dropout_add", dropped
+    yield "dropout into a tensor", "dropout_add", lambda: dropped(new(33, 8, k))
+    mask = dropped()[1]
+    yield "dropout backward", "dropout_bwd", lambda: be.dropout_bwd(x3, mask, 1.5)
+
+
+def _flat(got):
+    return [t for part in got for t in _flat(part)] if isinstance(got, (tuple, list)) else [got] if torch.is_tensor(got) else []
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_the_native_side_gives_the_bits_of_the_python_side():
+    """Every form that the native side takes, against the same call through the Python side: the same kernels on the same
+    operands, so the same bits, shapes and strides."""
+    native, python = HipBackend(), HipBackend()
+    python._n = _Off()
+    taken = []
+
+    class Watch:
+        def __getattr__(self, name):
+            fn = getattr(load_native(), name)
+
+            def call(*args):
+                got = fn(*args)
+                if got is not None:
+                    taken.append(name)
+                return got
+            return call
+
+    native._n = Watch()
+    for (name, fn, a), (_, _, b) in zip(_forms(native), _forms(python)):
+        taken.clear()
+        got = _flat(a())
+        assert fn in taken, f"{name}: left to the Python side"
+        want = _flat(b())
+        assert len(got) == len(want) and got, name
+        for t, u in zip(got, want):
+            assert t.shape == u.shape and t.stride() == u.stride() and t.dtype == u.dtype, name
+            assert torch.equal(t, u), name
