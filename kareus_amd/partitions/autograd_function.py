@@ -71,6 +71,12 @@ def _nanobatches_in_line(config, hs: Sequence[Tensor]) -> bool:
     return len(hs) > 1 and rule is not None and rule(hs[0].shape[0], hs[0].shape[1])
 
 
+def _scheduled(partitions) -> bool:
+    """Whether a plan's item was loaded into any of the partitions (by a scheduler of this pass or an earlier one, or by
+    hand): it is about the nanobatches' streams, so such a pass uses them."""
+    return any([p._schedule_config for p in partitions])
+
+
 def _fork(streams: Sequence[Optional[object]]) -> None:
     """Side streams start after everything already enqueued on the caller's stream."""
     if any(s is not None for s in streams):
@@ -185,7 +191,7 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
             f"got {len(params)} tensors"
         )
 
-        in_line = _nanobatches_in_line(config, hs)
+        in_line = _nanobatches_in_line(config, hs) and not _scheduled(fwd_parts) and not _scheduled(bwd_parts)
         streams = [None] * n if in_line else _nanobatch_streams(config, n)
         ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=in_line) for i in range(n)]
         _seed_forward(ctxs, hs, rotary, mask, seed)

@@ -620,3 +620,27 @@ def test_a_collective_with_work_of_its_own_is_waited_for_in_line(monkeypatch):
         model(x.clone().requires_grad_(True)).sum().backward()
     assert logs[True] == logs[False] and logs[True].count("run") > 0
     assert logs[True] == ["record", "wait", "run", "sync"] * logs[True].count("run")
+
+
+@pytest.mark.parametrize("direction", ["forward", "backward"])
+def test_a_plan_loaded_by_hand_keeps_the_streams(monkeypatch, direction):
+    """``load_schedule`` on a partition, without a scheduler in the configuration: its window and resource shape count."""
+    from kareus_amd.partitions import autograd_function
+
+    monkeypatch.setattr(autograd_function, "_nanobatches_in_line", lambda config, hs: True)
+    seen, real = [], autograd_function.NanoBatchContext
+
+    def context(**kw):
+        seen.append(kw["in_line"])
+        return real(**kw)
+
+    monkeypatch.setattr(autograd_function, "NanoBatchContext", context)
+    model = LayerStack(LayerConfig(**C1, num_layers=1, num_nanobatches=2, params_dtype=torch.float32, backend="eager"), seed=1234)
+    x = torch.randn(16, 2, C1["hidden_size"])
+    model(x)
+    assert seen == [True, True]
+    parts = model.forward_partitions if direction == "forward" else model.backward_partitions
+    config = CommConfig(overlap_window=("none", "none"), resource_shape=(16, 256))
+    parts[1].load_schedule(type("Item", (), {parts[1].partition_key: config}))
+    model(x)
+    assert seen[2:] == [False, False]
