@@ -49,6 +49,8 @@
 //     HBM-bound kernel sums the partials and rounds to bf16.
 #include "kr_common.h"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int BK = 64;
@@ -935,35 +937,48 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
     }
   }
   const double unsplit = best_cost;
-  for (int sp = 2; sp <= 16 && sp <= max_splits && nk / sp >= 8; ++sp)
+  // what a small tile is held against (below): the large tile at its measured rates, in every cut that this one is
+  // chosen in when fewer are allowed, and alone in every width and cut
+  constexpr double kSplitLarge = 5, kLargeRate = 0.8, kFusedLarge = 4;
+  auto large_cost = [&](int wn, int sp) {
+    const int items = tiles_m * ((N + 32 * wn - 1) / (32 * wn)) * sp;
+    const int rounds = (items + num_cus - 1) / num_cus;
+    const double per_item = (double)((nk + sp - 1) / sp) * (wn + 2) / 10.0 * kLargeRate + kItemOverhead + (fused ? kFusedLarge : 0.0);
+    const double reduce = sp > 1 ? sp * reduce_per_split + kSplitLarge : 0.0;
+    return w * rounds * per_item + (1.0 - w) * items * per_item / num_cus + reduce;
+  };
+  const bool alone = w == 1.0;
+  double large = large_cost(best.wn, 1);
+  for (int wn = 8; alone && wn >= min_wn; --wn) large = std::min(large, large_cost(wn, 1));
+  for (int sp = 2; sp <= 16 && sp <= max_splits && nk / sp >= 8; ++sp) {
     for (int wn = 8; wn >= min_wn; --wn) {
       const double c = cost(wn, sp);
       if (c < unsplit * 0.95 && c < best_cost) {  // a split must pay for itself clearly
         best_cost = c;
         best = {wn, sp, false};
       }
+      if (alone) large = std::min(large, large_cost(wn, sp));
     }
+    large = std::min(large, large_cost(best.wn, best.splits));
+  }
   if (!allow_small) return best;
   // 128 x 128 tiles (half the matrix work per byte read, but four times the work items, a quarter of the
   // epilogue in each, and two workgroups per compute unit to hide each other's waits).  Measured K-steps: 0.43 us
   // (0.33 units) with a unit to itself, 0.88 us when every unit holds two, in between when some do; 3 units around
-  // the K loop; a split's extra launch 2 units (5 for a large tile, whose fp32 partials leave in one burst).  Against them the large tiles' measured rates (their
-  // estimate above, which ranks them among themselves, is 20 % high in the K loop; a fused epilogue costs a large
-  // tile 4 units more).  Measured, large -> small tiles, us: 512 tokens of the 8B shard: fc1 with SwiGLU 65.3 ->
+  // the K loop; a split's extra launch 2 units (5 for a large tile, whose fp32 partials leave in one burst).  Against
+  // them the large tiles' measured rates (their estimate above, which ranks them among themselves, is 20 % high in
+  // the K loop; a fused epilogue costs a large tile 4 units more).  Measured, large -> small tiles, us: 512 tokens of the 8B shard: fc1 with SwiGLU 65.3 ->
   // 34.8, out-projection with the residual 22.2 -> 11.1, fc2 49.0 -> 31.3, its input gradient with the SwiGLU
   // backward 62.9 -> 36.1; 256 x 512 x 512 with the residual 17.4 -> 8.2; 4096 x 1024 x 4096 (NN) 44.0 -> 33.8.
   // On the other side of the line: 4096 x 1536 x 4096 45.1 -> 48.7, 1536 x 4096 x 7168 (NN) 80.2 -> 87.8,
   // 1536 tokens of fc1 with SwiGLU 73.0 -> 94.6, 16384 x 512 x 2048 29.2 -> 30.4.
-  constexpr double kAlone = 0.33, kPaired = 0.68, kOverhead = 3, kSplit = 2, kSplitLarge = 5, kLargeRate = 0.8, kFusedLarge = 4;
-  double large;
-  {
-    const int items = tiles_m * ((N + 32 * best.wn - 1) / (32 * best.wn)) * best.splits;
-    const int rounds = (items + num_cus - 1) / num_cus;
-    const double per_item = (double)((nk + best.splits - 1) / best.splits) * (best.wn + 2) / 10.0 * kLargeRate +
-                            kItemOverhead + (fused ? kFusedLarge : 0.0);
-    const double reduce = best.splits > 1 ? best.splits * reduce_per_split + kSplitLarge : 0.0;
-    large = w * rounds * per_item + (1.0 - w) * items * per_item / num_cus + reduce;
-  }
+  // The small tile has to beat, by these rates, whatever the large one would do with any part of the workspace:
+  // measured against the chosen cut alone it could win where sixteen cuts are allowed, be given a workspace for its own
+  // count, and lose there to the large tile uncut, the slowest of the three (us, then -> now: 152 x 4096 x 7168 beside
+  // other streams 70 -> 44, 4096 x 1536 x 6024 118 -> 94).  Alone it has to beat every width and cut besides: a large tile in cuts is faster than its estimate (768 x 7168 x 8192, large in three
+  // cuts 86, small 118; 1000 x 3584 x 8192 65, 68).  Beside other streams the widths hardly differ in
+  // compute-unit time, and the small tile is the shorter one (1024 x 1024 x 512 7.0, 11.6; 768 x 768 x 14336 43, 58).
+  constexpr double kAlone = 0.33, kPaired = 0.68, kOverhead = 3, kSplit = 2;
   const int small_tiles = ((M + 127) / 128) * ((N + 127) / 128);
   auto small_cost = [&](int sp) {
     const int items = small_tiles * sp, steps = (nk + sp - 1) / sp;

@@ -198,3 +198,36 @@ def test_attention_workspaces_by_stride():
     assert lib.kr_attn_fwd_workspace_bytes_strided(256, 1, 4, 2, 96, 96) == lib.kr_attn_fwd_workspace_bytes(256, 1, 4, 2, 96) > 0
     assert lib.kr_attn_bwd_workspace_bytes_strided(256, 1, 4, 2, 96, 96) == lib.kr_attn_bwd_workspace_bytes(256, 1, 4, 2, 96) > 0
     assert lib.kr_attn_bwd_workspace_bytes_strided(256, 1, 4, 2, 136, 136) == 0
+
+
+def test_a_gemm_is_planned_the_same_in_the_workspace_it_asks_for():
+    """``kr_gemm_workspace_bytes`` sizes what the plan with room for sixteen cuts takes.  In a workspace of that size the plan
+    is that one: otherwise a shape whose small tiles beat the large ones in cuts is given no workspace, and runs neither
+    but the large tile uncut."""
+    lib = hip.load_library()
+    widths = (384, 512, 768, 1024, 1376, 1536, 2048, 2752, 3072, 4096, 7168, 14336, 32064)
+    tokens = (96, 152, 304, 520, 768, 1000, 1536, 2008, 4096, 6024, 7008, 8192, 16384)
+
+    def plan(m, n, k, flags, workspace):
+        rows, cuts = ctypes.c_int(), ctypes.c_int()
+        assert lib.kr_gemm_plan(m, n, k, flags, 0, workspace, ctypes.byref(rows), ctypes.byref(cuts)) == 0
+        return rows.value, cuts.value
+
+    seen = set()
+    for t in tokens:
+        for a in widths:
+            for b in widths:
+                for m, n, k in ((t, a, b), (a, b, t)):
+                    for shared in (0, 0x100):
+                        bytes_ = (lib.kr_gemm_workspace_bytes_shared(0, m, n, k, 0.1) if shared
+                                  else lib.kr_gemm_workspace_bytes(0, m, n, k))
+                        free = plan(m, n, k, shared, 16 * m * n * 4)
+                        seen.add((free[0], free[1] > 1))
+                        if shared and bytes_ < free[1] * m * n * 4 and free[1] > 1:
+                            continue                      # (never more cuts than the launch would take alone)
+                        assert plan(m, n, k, shared, bytes_) == free, (m, n, k, shared)
+    assert seen == {(128, False), (128, True), (256, False), (256, True)}
+    # large in cuts, alone and beside other streams, and small where that is the shorter one
+    for shape, flags, rows in (((152, 4096, 7168), 0x100, 256), ((4096, 1536, 6024), 0, 256), ((768, 7168, 8192), 0, 256),
+                               ((1024, 1024, 512), 0x100, 128), ((512, 4096, 3584), 0, 128)):
+        assert plan(*shape, flags, 16 * shape[0] * shape[1] * 4)[0] == rows
