@@ -54,7 +54,8 @@ int kr_device_clock_mhz(void);
 size_t kr_gemm_workspace_bytes(int layout, int M, int N, int K);
 /* Workspace for a GEMM that shares the GPU with kernels of other streams.  The split count of
  * kr_gemm_workspace_bytes() minimises the GEMM's own latency; with latency_weight < 1 the choice
- * leans towards the smallest total CU-time instead, which never asks for more splits.  A launch
+ * leans towards the smallest total CU-time instead, which never asks for more splits than a launch
+ * alone would take in its own output tile or in the large one.  A launch
  * flagged KR_GEMM_BESIDE_OTHER_STREAMS is planned with weight 0.1: size its workspace with that
  * value, so that the cuts the dispatcher plans are the cuts the buffer holds.  kr_gemm_bf16 uses
  * as many splits as the workspace it is handed holds, at most the planned count.              */

@@ -977,28 +977,33 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
   // count, and lose there to the large tile uncut, the slowest of the three (us, then -> now: 152 x 4096 x 7168 beside
   // other streams 70 -> 44, 4096 x 1536 x 6024 118 -> 94).  Alone it has to beat every width and cut besides: a large tile in cuts is faster than its estimate (768 x 7168 x 8192, large in three
   // cuts 86, small 118; 1000 x 3584 x 8192 65, 68).  Beside other streams the widths hardly differ in
-  // compute-unit time, and the small tile is the shorter one (1024 x 1024 x 512 7.0, 11.6; 768 x 768 x 14336 43, 58).
+  // compute-unit time, and the small tile is the shorter one (1024 x 1024 x 512 7.0, 11.6).
   constexpr double kAlone = 0.33, kPaired = 0.68, kOverhead = 3, kSplit = 2;
+  // long contractions: as soon as some units hold two workgroups a K-step takes what it takes when all do (64 K-steps
+  // 0.7 us whether a tenth or half of the units do, 95 of them 1.1), and a cut large tile is the shorter one: 1536 x
+  // 3072 x 6024 107 us small, 74 large in two cuts; 640 x 7168 x 7008 113, 76.  Up to 64 K-steps they are level (3000 x 1536 x
+  // 4096 44.4, 45.5), as is everything fused, where the large tile cannot be cut
+  constexpr int kLong = 80;
   const int small_tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  auto small_cost = [&](int sp) {
+  auto small_cost = [&](int sp, double split) {
     const int items = small_tiles * sp, steps = (nk + sp - 1) / sp;
     const double paired = steps * kPaired + kOverhead;
-    const double reduce = sp > 1 ? sp * reduce_per_split + kSplit : 0.0;
+    const double reduce = sp > 1 ? sp * reduce_per_split + split : 0.0;
     const int full = items / (2 * num_cus), rest = items % (2 * num_cus);
     double latency = full * paired;
-    if (rest > num_cus) latency += steps * (kAlone + (kPaired - kAlone) * (rest - num_cus) / num_cus) + kOverhead;
+    if (rest > num_cus) latency += steps >= kLong && !fused ? paired : steps * (kAlone + (kPaired - kAlone) * (rest - num_cus) / num_cus) + kOverhead;
     else if (rest > 0) latency += steps * kAlone + kOverhead;
     return w * latency + (1.0 - w) * items * paired / (2 * num_cus) + reduce;
   };
-  double small_best = large * 0.93;  // the change must be clear
-  for (int sp = 1; sp == 1 || (sp <= 16 && sp <= max_splits && nk / sp >= 8); ++sp) {
-    const double c = small_cost(sp);
-    if (c < small_best) {
-      small_best = c;
-      best = {4, sp, true};
-    }
-  }
-  return best;
+  auto small_cut = [&](double split) {  // the best cut, a cut's extra launch counted as `split`
+    int at = 1;
+    for (int sp = 2; sp <= 16 && sp <= max_splits && nk / sp >= 8; ++sp)
+      if (small_cost(sp, split) < small_cost(at, split)) at = sp;
+    return at;
+  };
+  if (small_cost(small_cut(kSplit), kSplit) >= large * 0.93) return best;  // the change must be clear
+  // (beside other streams the extra launch is no compute-unit time: 384 x 640 x 4096 in two cuts 21 us, uncut 32)
+  return {4, small_cut(w * kSplit), true};
 }
 
 struct Fused {
@@ -1170,7 +1175,8 @@ extern "C" size_t kr_gemm_workspace_bytes_shared(int layout, int M, int N, int K
   (void)layout;
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   int splits = choose_plan(M, N, K, latency_weight, 256, 16).splits;
-  const int cap = choose_plan(M, N, K, 1.f, 256, 16).splits;
+  // never more than a launch that has the device to itself takes, in its tile or in the large one
+  const int cap = std::max(choose_plan(M, N, K, 1.f, 256, 16).splits, choose_plan(M, N, K, 1.f, 256, 16, false, false).splits);
   if (splits > cap) splits = cap;
   return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
 }

@@ -227,6 +227,12 @@ def test_a_gemm_is_planned_the_same_in_the_workspace_it_asks_for():
                             continue                      # (never more cuts than the launch would take alone)
                         assert plan(m, n, k, shared, bytes_) == free, (m, n, k, shared)
     assert seen == {(128, False), (128, True), (256, False), (256, True)}
+    # long contractions of a few more small tiles than compute units go to the large tile in cuts, short ones do not
+    for shape, rows in (((1536, 3072, 6024), 256), ((640, 7168, 7008), 256), ((1536, 3072, 2048), 128)):
+        assert plan(*shape, 0, 16 * shape[0] * shape[1] * 4)[0] == rows
+    # beside other streams a cut's extra launch is no compute-unit time: small outputs are cut there too
+    for shape, cuts in (((384, 640, 4096), 2), ((304, 640, 7168), 4)):
+        assert plan(*shape, 0x100, 16 * shape[0] * shape[1] * 4) == (128, cuts)
     # large in cuts, alone and beside other streams, and small where that is the shorter one
     for shape, flags, rows in (((152, 4096, 7168), 0x100, 256), ((4096, 1536, 6024), 0, 256), ((768, 7168, 8192), 0, 256),
                                ((1024, 1024, 512), 0x100, 128), ((512, 4096, 3584), 0, 128)):
