@@ -967,22 +967,25 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
   // (0.33 units) with a unit to itself, 0.88 us when every unit holds two, in between when some do; 3 units around
   // the K loop; a split's extra launch 2 units (5 for a large tile, whose fp32 partials leave in one burst).  Against
   // them the large tiles' measured rates (their estimate above, which ranks them among themselves, is 20 % high in
-  // the K loop; a fused epilogue costs a large tile 4 units more).  Measured, large -> small tiles, us: 512 tokens of the 8B shard: fc1 with SwiGLU 65.3 ->
-  // 34.8, out-projection with the residual 22.2 -> 11.1, fc2 49.0 -> 31.3, its input gradient with the SwiGLU
-  // backward 62.9 -> 36.1; 256 x 512 x 512 with the residual 17.4 -> 8.2; 4096 x 1024 x 4096 (NN) 44.0 -> 33.8.
+  // the K loop; a fused epilogue costs a large tile 4 units more).  Measured, large -> small tiles, us: 512 tokens of
+  // the 8B shard: fc1 with SwiGLU 65.3 -> 34.8, out-projection with the residual 22.2 -> 11.1, fc2 49.0 -> 31.3, its
+  // input gradient with the SwiGLU backward 62.9 -> 36.1; 256 x 512 x 512 with the residual 17.4 -> 8.2; 4096 x
+  // 1024 x 4096 (NN) 44.0 -> 33.8.
   // On the other side of the line: 4096 x 1536 x 4096 45.1 -> 48.7, 1536 x 4096 x 7168 (NN) 80.2 -> 87.8,
   // 1536 tokens of fc1 with SwiGLU 73.0 -> 94.6, 16384 x 512 x 2048 29.2 -> 30.4.
   // The small tile has to beat, by these rates, whatever the large one would do with any part of the workspace:
   // measured against the chosen cut alone it could win where sixteen cuts are allowed, be given a workspace for its own
   // count, and lose there to the large tile uncut, the slowest of the three (us, then -> now: 152 x 4096 x 7168 beside
-  // other streams 70 -> 44, 4096 x 1536 x 6024 118 -> 94).  Alone it has to beat every width and cut besides: a large tile in cuts is faster than its estimate (768 x 7168 x 8192, large in three
-  // cuts 86, small 118; 1000 x 3584 x 8192 65, 68).  Beside other streams the widths hardly differ in
-  // compute-unit time, and the small tile is the shorter one (1024 x 1024 x 512 7.0, 11.6).
+  // other streams 70 -> 44, 4096 x 1536 x 6024 118 -> 94).  Alone it has to beat every width and cut besides: a large
+  // tile in cuts is faster than its estimate (768 x 7168 x 8192, large in three cuts 86, small 118; 1000 x 3584 x 8192
+  // 65, 68).  Beside other streams the widths hardly differ in compute-unit time, and the small tile is the
+  // shorter one (1024 x 1024 x 512: small 7.0, large 11.6).
   constexpr double kAlone = 0.33, kPaired = 0.68, kOverhead = 3, kSplit = 2;
   // long contractions: as soon as some units hold two workgroups a K-step takes what it takes when all do (64 K-steps
   // 0.7 us whether a tenth or half of the units do, 95 of them 1.1), and a cut large tile is the shorter one: 1536 x
-  // 3072 x 6024 107 us small, 74 large in two cuts; 640 x 7168 x 7008 113, 76.  Up to 64 K-steps they are level (3000 x 1536 x
-  // 4096 44.4, 45.5), as is everything fused, where the large tile cannot be cut
+  // 3072 x 6024 107 us small, 74 large in two cuts; 640 x 7168 x 7008 113, 76.  Up to 64 K-steps they are level
+  // (3000 x 1536 x 4096 44.4, 45.5); with a fused epilogue the large tile cannot be cut and the small one is as often
+  // the shorter (7168 x 768 x 8192 101, 119; 1376 x 3072 x 6024 113, 97)
   constexpr int kLong = 80;
   const int small_tiles = ((M + 127) / 128) * ((N + 127) / 128);
   auto small_cost = [&](int sp, double split) {
@@ -991,7 +994,8 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
     const double reduce = sp > 1 ? sp * reduce_per_split + split : 0.0;
     const int full = items / (2 * num_cus), rest = items % (2 * num_cus);
     double latency = full * paired;
-    if (rest > num_cus) latency += steps >= kLong && !fused ? paired : steps * (kAlone + (kPaired - kAlone) * (rest - num_cus) / num_cus) + kOverhead;
+    if (rest > num_cus && steps >= kLong && !fused) latency += paired;
+    else if (rest > num_cus) latency += steps * (kAlone + (kPaired - kAlone) * (rest - num_cus) / num_cus) + kOverhead;
     else if (rest > 0) latency += steps * kAlone + kOverhead;
     return w * latency + (1.0 - w) * items * paired / (2 * num_cus) + reduce;
   };
