@@ -51,7 +51,67 @@
 
 #include <algorithm>
 
+// This file is compiled once per operand layout (KR_GEMM_LAYOUT_TU: 0 TN, 1 NN, 2 NT): the instances of a layout are a
+// third of the work, and the three build side by side.  The planner and the C entry points are in the first.
+#ifndef KR_GEMM_LAYOUT_TU
+#error "compile with -DKR_GEMM_LAYOUT_TU=0, 1 and 2"
+#endif
+
+namespace kr_gemm {
+
+// Row runs of A, C and aux (see run_off): shift and distance between run starts; sh = 0 for a
+// plain matrix (the distance is then unused).
+struct RowRuns {
+  int a_sh, a_outer, c_sh, c_outer, x_sh, x_outer;
+};
+
+// The contraction of a weight gradient over the nanobatches of a microbatch: layout NT, operands in up
+// to KR_GEMM_MAX_SEGMENTS pieces (one pair per nanobatch, each `steps` K-steps of 64 rows long, all with
+// the row strides lda / ldb), contracted one after the other into one sum.
+constexpr int MAX_SEGMENTS = KR_GEMM_MAX_SEGMENTS;
+struct Segments {
+  const bf16* a[MAX_SEGMENTS];
+  const bf16* b[MAX_SEGMENTS];
+  int n, steps;
+};
+
+struct Fused {
+  int epi = 0;              // KR_GEMM_EPI_*
+  const bf16* aux = nullptr;
+  int64_t ld_aux = 0;
+  bf16* out2 = nullptr;
+  int64_t ld_out2 = 0;
+  int max_cus = 0;          // > 0: use at most this many compute units
+  bool shared = false;      // other streams' kernels use the units this launch leaves idle
+  RowRuns runs = {0, 0, 0, 0, 0, 0};  // row runs of A, C, aux (all plain by default)
+  const Segments* segs = nullptr;     // layout NT: the operands come in these pieces (A and B are unused)
+};
+
+// One launch as the dispatcher planned it.  wn: 16-column MFMA tiles per wave; small: the 128 x 128 tile; transposed:
+// operands exchanged, C^T stored.
+struct Call {
+  const bf16* a;
+  int64_t lda;
+  const bf16* b;
+  int64_t ldb;
+  bf16* c;
+  int64_t ldc;
+  int m, n, k, accumulate;
+  float* workspace;
+  size_t workspace_bytes;
+  hipStream_t stream;
+  int num_cus, wn, splits;
+  bool small, transposed;
+};
+int launch_tn(const Call& call, const Fused& fu);
+int launch_nn(const Call& call, const Fused& fu);
+int launch_nt(const Call& call, const Fused& fu);
+
+}  // namespace kr_gemm
+
 namespace {
+
+using namespace kr_gemm;
 
 constexpr int BK = 64;
 constexpr int BM = 256, BN = 256;  // the largest tile; a kernel instance covers 32 * WT rows x 32 * WN columns
@@ -68,7 +128,11 @@ constexpr int kDepth = 2, kDepthAlone = 4;
 // s_waitcnt immediate for vmcnt(n); lgkmcnt and expcnt untouched
 constexpr int vm_wait(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int kXcds = 8;
-constexpr int KR_GEMM_EPI_TRANSPOSED_OUT = 100;  // internal: not part of the C ABI's epilogue values
+// internal, not part of the C ABI's epilogue values: the transposed store, and the two kinds of output besides a bf16
+// store of finished sums.  Instances of their own: in one kernel with the plain store the loads of the accumulating one
+// are to the compiler still in flight in the next tile's K loop, where it then waits for every load (4096 x 4096 x 16384
+// 356 -> 443 us), and as whole loops under a branch they spill accumulators.
+constexpr int KR_GEMM_EPI_TRANSPOSED_OUT = 100, KR_GEMM_OUT_PARTIAL = 101, KR_GEMM_OUT_ACCUMULATE = 102;
 constexpr int kGroupM = 4;
 
 // ---- LDS layouts (element offsets inside one operand tile) ----------------------------------
@@ -80,6 +144,15 @@ constexpr int kGroupM = 4;
 // operand re-reads; the same hint on other kernels' stores or on the epilogues' residual loads changed nothing.
 __device__ __forceinline__ void stg8_out(bf16* p, bf16x8 v) {
   __builtin_nontemporal_store(v, reinterpret_cast<bf16x8*>(p));
+}
+
+// An address as a wave-uniform base and this lane's unsigned 32-bit byte offset: one scalar register pair and one
+// vector register, where a 64-bit address per lane costs two vector instructions and two registers per access.
+__device__ __forceinline__ const bf16* at_byte(const bf16* base, uint32_t off) {
+  return reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(base) + off);
+}
+__device__ __forceinline__ bf16* at_byte(bf16* base, uint32_t off) {
+  return reinterpret_cast<bf16*>(reinterpret_cast<char*>(base) + off);
 }
 
 __device__ __forceinline__ int kmajor_off(int row, int chunk) {
@@ -229,21 +302,6 @@ __device__ __forceinline__ void remap_block(int pid, int nblocks, int tiles_m, i
   tn = in_band / band_rows;
 }
 
-// Row runs of A, C and aux (see run_off): shift and distance between run starts; sh = 0 for a
-// plain matrix (the distance is then unused).
-struct RowRuns {
-  int a_sh, a_outer, c_sh, c_outer, x_sh, x_outer;
-};
-
-// The contraction of a weight gradient over the nanobatches of a microbatch: layout NT, operands in up
-// to KR_GEMM_MAX_SEGMENTS pieces (one pair per nanobatch, each `steps` K-steps of 64 rows long, all with
-// the row strides lda / ldb), contracted one after the other into one sum.
-constexpr int MAX_SEGMENTS = KR_GEMM_MAX_SEGMENTS;
-struct Segments {
-  const bf16* a[MAX_SEGMENTS];
-  const bf16* b[MAX_SEGMENTS];
-  int n, steps;
-};
 
 template <int WT, int WN>
 struct Frags {
@@ -302,7 +360,10 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   // columns and stores the gradient of x instead of the product.
   constexpr bool swiglu_bwd = EPI == KR_GEMM_EPI_SWIGLU_BWD;
   static_assert(!swiglu_bwd || (!A_T && B_T), "SwiGLU backward epilogue: layout NN only");
-  static_assert(EPI == KR_GEMM_EPI_NONE || trans_out || swiglu_bwd || (!A_T && !B_T),
+  // PARTIAL: fp32 partial tiles of a cut contraction.  ACCUMULATE: C += product, rounded once.
+  constexpr bool split_k = EPI == KR_GEMM_OUT_PARTIAL, add_old = EPI == KR_GEMM_OUT_ACCUMULATE;
+  constexpr bool narrow = !trans_out && !split_k && !add_old;
+  static_assert(EPI == KR_GEMM_EPI_NONE || trans_out || swiglu_bwd || split_k || add_old || (!A_T && !B_T),
                 "residual / SwiGLU epilogues: K-major layout only");
   static_assert(!trans_out || (A_T && B_T), "transposed store: layout NT only");
   constexpr bool epi_add = EPI == KR_GEMM_EPI_ADD;
@@ -310,7 +371,6 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   const int gate_up_f = swiglu ? N / 2 : 0;
   const int tiles_m = (M + BM_ - 1) / BM_, tiles_n = swiglu ? N / BN_ : (N + BN_ - 1) / BN_;
   const int ntiles = tiles_m * tiles_n;
-  const bool split_k = partial != nullptr;
   const uint32_t smem_b = lds_addr(smem);
   const uint32_t wave_blk = (uint32_t)wave * 1024u;
 
@@ -430,7 +490,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   };
   // After this wave's loads of the last K-step have landed (A in slot sa, B in slot sb): zero
   // the chunks beyond the contraction range.
-  auto fix_tail = [&](uint32_t sa, uint32_t sb) {
+  auto fix_tail = [&](uint32_t sa, uint32_t sb, int k_tail) {
     if (k_tail == BK) return;
     int l2 = lane;
     asm volatile("" : "+v"(l2));
@@ -531,8 +591,12 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
 #pragma unroll
   for (int i = 0; i < WT; ++i)
 #pragma unroll
-    for (int j = 0; j < WN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < WN; ++j) {
+      acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[i][j]));
+    }
 
+  bool carried = false;  // the previous item's K loop has requested this one's first K-steps and read its first fragments
   for (;;) {
     {
       int lf = lane;
@@ -543,7 +607,9 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     // K-step 0 complete in LDS (requested above, or before the previous item's epilogue); the
     // loads of the K-steps behind it may still be in flight (loads retire in order)
     constexpr int STEP_LOADS = NA_LOADS + NB_LOADS;
-    if (nk >= DEPTH) {
+    if (carried) {
+      // (it has landed and been read; what is waited for is every wave's epilogue, whose staging slot K-step DEPTH goes to)
+    } else if (nk >= DEPTH) {
       __builtin_amdgcn_s_waitcnt(vm_wait((DEPTH - 1) * STEP_LOADS));
     } else if (DEPTH > 2 && nk == 3) {
       __builtin_amdgcn_s_waitcnt(vm_wait(2 * STEP_LOADS));
@@ -551,10 +617,10 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       __builtin_amdgcn_s_waitcnt(vm_wait(STEP_LOADS));
     } else {
       __builtin_amdgcn_s_waitcnt(vm_wait(0));
-      fix_tail(ring[0], ring[1]);
+      fix_tail(ring[0], ring[1], k_tail);
     }
     __syncthreads();
-    {
+    if (!carried) {
       uint32_t aa[FragReader<A_T, WT>::NBASE], ba[FragReader<B_T, WT>::NBASE];
       frag_addrs(ring[0], ring[1], 0, aa, ba);
 #pragma unroll
@@ -580,27 +646,56 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       seg_advance();
       rotate();
     }
-    for (; t < nk; ++t) {
+    const int out_m0 = m0, out_n0 = n0;
+    float* const out_partial = split_k ? partial + p_off : nullptr;
+    const int next = item + (int)gridDim.x;
+    const bool more = next < total_items;
+    carried = false;
+    if constexpr (DEPTH == kDepth) {
+      // The last two K-steps request the first two of the next item, where the ones before request their own successors, and
+      // the last half-step reads its first fragments: the operands keep flowing across items.  Requested in one go behind
+      // the K loop (as items of a single K-step still are) they took 1.5 us per tile in layout TN and 2 in the others, the
+      // matrix pipes idle.  With this and the shorter epilogue, us, before -> after at 16384 tokens: 4096 x 1024 plain (TN)
+      // 113 -> 109, 7168 x 4096 plain (TN) 645 -> 634, 4096 x 7168 (NN) 656 -> 643, 3072 x 640 (NN) 65.4 -> 62.6.
+      if (more && nk >= DEPTH) {
+        const int last = nk, tail = k_tail;
+        select_item(next);
+        carried = nk >= DEPTH;
+        if (carried) {
+          set_offsets(BK);
+          for (; t < last; ++t) {
+            const int d = t + DEPTH - last;
+            if (d + 1 == nk && k_tail != BK) set_offsets(k_tail);
+            half(X, Y, ring[0], ring[1], 1, Count<NA_LOADS>{}, a_base(d), la, ring[NSLOTS - 1]);
+            __builtin_amdgcn_s_waitcnt(vm_wait((DEPTH - 2) * STEP_LOADS + NA_LOADS));
+            if (t + 2 == last) fix_tail(ring[2], ring[3], tail);
+            __syncthreads();
+            half(Y, X, ring[2], ring[3], 0, Count<NB_LOADS>{}, b_base(d), lb, ring[0]);
+            seg_advance();
+            rotate();
+          }
+        } else {
+          nk = last;
+          k_tail = tail;
+        }
+      }
+    }
+    for (; t < nk && !carried; ++t) {
       half(X, Y, ring[0], ring[1], 1, Count<0>{}, nullptr, la, 0u);
       // (at most DEPTH - 1 K-steps are left behind this one)
       if (DEPTH > 2 && t + 4 == nk) __builtin_amdgcn_s_waitcnt(vm_wait(2 * STEP_LOADS));
       else if (DEPTH > 2 && t + 3 == nk) __builtin_amdgcn_s_waitcnt(vm_wait(STEP_LOADS));
       else __builtin_amdgcn_s_waitcnt(vm_wait(0));
-      if (t + 2 == nk) fix_tail(ring[2], ring[3]);
+      if (t + 2 == nk) fix_tail(ring[2], ring[3], k_tail);
       __syncthreads();
       // (after the last K-step this reads tiles that do not exist: unused)
       half(Y, X, ring[2], ring[3], 0, Count<0>{}, nullptr, lb, 0u);
       rotate();
     }
 
-    // Every LDS read of this item that matters finished before the last barrier, so all
-    // slots are free: request the first K-steps of the next item now and let them fly
-    // during the epilogue.
-    const int out_m0 = m0, out_n0 = n0;
-    float* const out_partial = split_k ? partial + p_off : nullptr;
-    const int next = item + (int)gridDim.x;
-    const bool more = next < total_items;
-    if (more) {
+    // Every LDS read of this item that matters finished before the last barrier, so all slots but those of requests
+    // already made are free: request the first K-steps of the next item now and let them fly during the epilogue.
+    if (more && !carried) {
       select_item(next);
       request_first();
     }
@@ -637,56 +732,43 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
       };
-      const bool rows_in = m_wave + 16 * WT <= M;  // wave-uniform: no row of the wave tile is cut off
+      const int rows_left = M - m_wave;  // rows of the wave tile that the matrix has (wave-uniform)
       const bool cols_in = 4 * ch < 16 * WN && n_wave + 4 * ch < N;
-      const bool to_partial = out_partial != nullptr;
-      const bool add_old = !to_partial && accumulate;
-      const int ldo = to_partial ? N : ldc;
+      const int ldo = split_k ? N : ldc;
       uint32_t lo[Q32];
 #pragma unroll
       for (int q = 0; q < Q32; ++q) lo[q] = (uint32_t)((64 / L32 * q + hrow) * ldo + 4 * ch);
-      // accumulation into C: the old values of a 16-row block are requested one block ahead of
-      // the pass that uses them (zeros otherwise).  Positions beyond the matrix read a valid
-      // neighbour instead and are never stored back.
-      bf16x4 oldc[2][Q32];
-#pragma unroll
-      for (int q = 0; q < Q32; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) oldc[0][q][e] = oldc[1][q][e] = (bf16)0.f;
-      auto fetch_old = [&](int mt) {
-        const bf16* const cb = C + ((int64_t)(m_wave + mt * 16) * ldc + n_wave);
-#pragma unroll
-        for (int q = 0; q < Q32; ++q) {
-          const bool in = cols_in && (rows_in || m_wave + mt * 16 + 64 / L32 * q + hrow < M);
-          oldc[mt & 1][q] = *reinterpret_cast<const bf16x4*>(in ? cb + lo[q] : C);
-        }
-      };
-      if (add_old) fetch_old(0);
       // bf16 output without accumulation goes through the same place as bf16: 16 rows x 256 bytes
       // per block, two buffers (so one wave-level fence per block), read side row (64 / L16) q + row_r,
       // 16-byte chunk rch = eight consecutive columns, L16 lanes per row
-      const bool narrow = !to_partial && !add_old;
       const int rch = le % L16, row_r = le / L16;
       // first column the wave stores to: n_wave, or with SwiGLU column out_n0 of the gate half
       // (wn = 0) or of the up half (wn = 1) of x
       const int n_store = swiglu ? out_n0 + (wn ? gate_up_f : 0) : n_wave;
       const int ncol = 8 * rch;
       const bool ncols_in = 8 * rch < 16 * WN && (swiglu || n_wave + 8 * rch < N);
-      uint32_t nlo[Q16];
+      uint32_t nlo[Q16];  // bytes from the block's first element: base and offset of a store stay apart (scalar, vector)
 #pragma unroll
       for (int q = 0; q < Q16; ++q)   // (a 16-row block starts at a multiple of the run length: rows map inside it)
-        nlo[q] = (uint32_t)((runs.c_sh ? run_off(64 / L16 * q + row_r, ldc, runs.c_sh, runs.c_outer) : (64 / L16 * q + row_r) * ldc) + ncol);
+        nlo[q] = 2u * (uint32_t)((runs.c_sh ? run_off(64 / L16 * q + row_r, ldc, runs.c_sh, runs.c_outer) : (64 / L16 * q + row_r) * ldc) + ncol);
       // fused residual: the values to add to a 16-row block are requested one block ahead
       // SwiGLU backward: gate and up values of a 16-row block, requested one block ahead
       bf16x8 xg[swiglu_bwd ? 2 : 1][swiglu_bwd ? Q16 : 1], xu[swiglu_bwd ? 2 : 1][swiglu_bwd ? Q16 : 1];
-      auto fetch_x = [&](int mt) {
-        const bf16* const xb = aux + ((int64_t)(m_wave + mt * 16) * ld_aux + n_wave + 8 * rch);
+      uint32_t xlo[epi_add || swiglu_bwd ? Q16 : 1];  // bytes from a block's first element of aux
+      if constexpr (epi_add || swiglu_bwd) {
 #pragma unroll
         for (int q = 0; q < Q16; ++q) {
           const int rr = 64 / L16 * q + row_r;
-          const bool in = ncols_in && (rows_in || m_wave + mt * 16 + rr < M);
-          xg[mt & 1][q] = in ? ldg8(xb + (int64_t)rr * ld_aux) : zero8();
-          xu[mt & 1][q] = in ? ldg8(xb + (int64_t)rr * ld_aux + N) : zero8();
+          xlo[q] = 2u * (uint32_t)((runs.x_sh ? run_off(rr, ld_aux, runs.x_sh, runs.x_outer) : rr * ld_aux) + 8 * rch);
+        }
+      }
+      auto fetch_x = [&](int mt) {
+        const bf16* const xb = aux + ((int64_t)(m_wave + mt * 16) * ld_aux + n_wave);
+#pragma unroll
+        for (int q = 0; q < Q16; ++q) {
+          const bool in = ncols_in && row_r < rows_left - mt * 16 - 64 / L16 * q;
+          xg[mt & 1][q] = in ? ldg8(at_byte(xb, xlo[q])) : zero8();
+          xu[mt & 1][q] = in ? ldg8(at_byte(xb + N, xlo[q])) : zero8();
         }
       };
       if constexpr (swiglu_bwd) fetch_x(0);
@@ -694,16 +776,27 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       auto fetch_res = [&](int mt) {
         const int r0 = m_wave + mt * 16;
         const bf16* const rb =
-            aux + ((runs.x_sh ? (int64_t)(r0 >> runs.x_sh) * runs.x_outer : (int64_t)r0 * ld_aux) + n_wave + 8 * rch);
+            aux + ((runs.x_sh ? (int64_t)(r0 >> runs.x_sh) * runs.x_outer : (int64_t)r0 * ld_aux) + n_wave);
 #pragma unroll
         for (int q = 0; q < Q16; ++q) {
-          const int rr = 64 / L16 * q + row_r;
-          const bool in = ncols_in && (rows_in || m_wave + mt * 16 + rr < M);
-          const int64_t ro = runs.x_sh ? (int64_t)run_off(rr, ld_aux, runs.x_sh, runs.x_outer) : (int64_t)rr * ld_aux;
-          resv[mt & 1][q] = in ? ldg8(rb + ro) : zero8();
+          const bool in = ncols_in && row_r < rows_left - mt * 16 - 64 / L16 * q;
+          resv[mt & 1][q] = in ? ldg8(at_byte(rb, xlo[q])) : zero8();
         }
       };
       if constexpr (epi_add) fetch_res(0);
+      // the accumulators of a 16-row block, left at zero.  Read and written in the order given here (the pins): left
+      // to itself the compiler reads most of the tile into vector registers in front of the first block, and writes the
+      // zeros, which it knows to be zeros, a second time in front of the K loop (256 instructions, 0.5 us a tile).
+      auto take_block = [&](int mt, f32x4 (&vals)[WN]) {
+#pragma unroll
+        for (int nt = 0; nt < WN; ++nt) {
+          asm volatile("" : "+a"(acc[mt][nt]));
+          vals[nt] = acc[mt][nt];
+          asm volatile("" : "+v"(vals[nt]));
+          acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+          asm volatile("" : "+a"(acc[mt][nt]));
+        }
+      };
       if constexpr (trans_out) {
         // C^T leaves in blocks of 16 of its rows (columns nt of the wave tile): the wave's eight
         // 16 x 16 tiles of that column are 16 rows x 128 columns of C^T, staged and stored like a
@@ -713,9 +806,11 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
           f32x4 vals[WT];
 #pragma unroll
           for (int mt = 0; mt < WT; ++mt) {
+            asm volatile("" : "+a"(acc[mt][nt]));
             vals[mt] = acc[mt][nt];
             asm volatile("" : "+v"(vals[mt]));
             acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+a"(acc[mt][nt]));
           }
           const uint32_t buf = stage + (uint32_t)(nt & 1) * 4096u;
 #pragma unroll
@@ -736,27 +831,19 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-      } else {
+      } else if constexpr (narrow) {
 #pragma unroll
-      for (int mt = 0; mt < WT; ++mt) {
-        if (add_old && mt + 1 < WT) fetch_old(mt + 1);
-        if constexpr (epi_add) {
-          if (mt + 1 < WT) fetch_res(mt + 1);
-        }
-        if constexpr (swiglu_bwd) {
-          if (mt + 1 < WT) fetch_x(mt + 1);
-        }
-        f32x4 vals[WN];  // the only place the accumulators are read
-#pragma unroll
-        for (int nt = 0; nt < WN; ++nt) {
-          vals[nt] = acc[mt][nt];
-          asm volatile("" : "+v"(vals[nt]));  // read here, not once in each branch below
-          acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        const int64_t blk = (narrow && runs.c_sh ? (int64_t)((m_wave + mt * 16) >> runs.c_sh) * runs.c_outer
-                                                 : (int64_t)(m_wave + mt * 16) * ldo) +
-                            (narrow ? n_store : n_wave);
-        if (narrow) {
+        for (int mt = 0; mt < WT; ++mt) {
+          if constexpr (epi_add) {
+            if (mt + 1 < WT) fetch_res(mt + 1);
+          }
+          if constexpr (swiglu_bwd) {
+            if (mt + 1 < WT) fetch_x(mt + 1);
+          }
+          f32x4 vals[WN];
+          take_block(mt, vals);
+          const int64_t blk = (runs.c_sh ? (int64_t)((m_wave + mt * 16) >> runs.c_sh) * runs.c_outer
+                                         : (int64_t)(m_wave + mt * 16) * ldc) + n_store;
           const uint32_t buf = stage + (uint32_t)(mt & 1) * SBUF;
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt) {
@@ -770,7 +857,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
           for (int q = 0; q < Q16; ++q) {
             const int rr = 64 / L16 * q + row_r;
             bf16x8 v = *(KR_LDS const bf16x8*)(buf + rr * ROW16 + ((rch ^ (rr & XOR16)) << 4));
-            const bool in = ncols_in && (rows_in || m_wave + mt * 16 + rr < M);
+            const bool in = ncols_in && row_r < rows_left - mt * 16 - 64 / L16 * q;
             if constexpr (epi_add) {
 #pragma unroll
               for (int e = 0; e < 8; ++e) v[e] = (bf16)((float)resv[mt & 1][q][e] + (float)v[e]);
@@ -785,11 +872,11 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
                 d2[e] = (bf16)du;
               }
               if (in) {
-                stg8_out(C + blk + nlo[q], d1);
-                stg8_out(C + blk + nlo[q] + N, d2);
+                stg8_out(at_byte(C + blk, nlo[q]), d1);
+                stg8_out(at_byte(C + blk + N, nlo[q]), d2);
               }
             } else {
-              if (in) stg8_out(C + blk + nlo[q], v);
+              if (in) stg8_out(at_byte(C + blk, nlo[q]), v);
             }
           }
           if constexpr (swiglu) {
@@ -807,33 +894,70 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
               bf16x8 y;
 #pragma unroll
               for (int e = 0; e < 8; ++e) y[e] = (bf16)kr_swiglu_f((float)g[e], (float)u[e]);
-              if (ncols_in && (rows_in || m_wave + mt * 16 + rr < M))
-                stg8_out(out2 + (int64_t)(m_wave + mt * 16 + rr) * ld_out2 + out_n0 + 8 * rch, y);
+              if (ncols_in && rr < rows_left - mt * 16)
+                stg8_out(at_byte(out2 + ((int64_t)(m_wave + mt * 16) * ld_out2 + out_n0), 2u * (uint32_t)(rr * ld_out2 + 8 * rch)), y);
             }
           }
-        } else {
+          __builtin_amdgcn_sched_barrier(0);  // keep the accumulator reads of later blocks below
+        }
+      } else {
+        auto stage_block = [&](int mt) {
+          f32x4 vals[WN];
+          take_block(mt, vals);
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt)
             *(KR_LDS f32x4*)(stage + row16 * ROW32 + (((4 * nt + quad) ^ row16) << 4)) = vals[nt];
           wave_sync();
+        };
+        auto staged = [&](int q) {
+          const int rr = 64 / L32 * q + hrow;
+          return *(KR_LDS const f32x4*)(stage + rr * ROW32 + ((ch ^ rr) << 4));
+        };
+        if constexpr (split_k) {
 #pragma unroll
-          for (int q = 0; q < Q32; ++q) {
-            const int rr = 64 / L32 * q + hrow;
-            const f32x4 v = *(KR_LDS const f32x4*)(stage + rr * ROW32 + ((ch ^ rr) << 4));
-            const bool in = cols_in && (rows_in || m_wave + mt * 16 + rr < M);
-            if (to_partial) {
-              if (in) *reinterpret_cast<f32x4*>(out_partial + blk + lo[q]) = v;
-            } else {
+          for (int mt = 0; mt < WT; ++mt) {
+            stage_block(mt);
+            float* const pb = out_partial + ((int64_t)(m_wave + mt * 16) * N + n_wave);
+#pragma unroll
+            for (int q = 0; q < Q32; ++q) {
+              const f32x4 v = staged(q);
+              if (cols_in && hrow < rows_left - mt * 16 - 64 / L32 * q) *reinterpret_cast<f32x4*>(pb + lo[q]) = v;
+            }
+            wave_sync();
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+          // the old values of a 16-row block are requested one block ahead of the pass that uses them.  Positions
+          // beyond the matrix read a valid neighbour instead and are never stored back.
+          bf16x4 oldc[2][Q32];
+          auto fetch_old = [&](int mt) {
+            const bf16* const cb = C + ((int64_t)(m_wave + mt * 16) * ldc + n_wave);
+#pragma unroll
+            for (int q = 0; q < Q32; ++q) {
+              const bool in = cols_in && hrow < rows_left - mt * 16 - 64 / L32 * q;
+              oldc[mt & 1][q] = *reinterpret_cast<const bf16x4*>(in ? cb + lo[q] : C);
+            }
+          };
+          fetch_old(0);
+#pragma unroll
+          for (int mt = 0; mt < WT; ++mt) {
+            if (mt + 1 < WT) fetch_old(mt + 1);
+            stage_block(mt);
+            bf16* const cb = C + ((int64_t)(m_wave + mt * 16) * ldc + n_wave);
+#pragma unroll
+            for (int q = 0; q < Q32; ++q) {
+              const f32x4 v = staged(q);
               bf16x4 o;
 #pragma unroll
               for (int e = 0; e < 4; ++e) o[e] = (bf16)(v[e] + (float)oldc[mt & 1][q][e]);
-              if (in) __builtin_nontemporal_store(o, reinterpret_cast<bf16x4*>(C + blk + lo[q]));
+              asm volatile("" : "+v"(o));  // used by every lane: a load whose use hangs on a condition stays in flight
+              if (cols_in && hrow < rows_left - mt * 16 - 64 / L32 * q)
+                __builtin_nontemporal_store(o, reinterpret_cast<bf16x4*>(cb + lo[q]));
             }
+            wave_sync();
+            __builtin_amdgcn_sched_barrier(0);
           }
-          wave_sync();
         }
-        __builtin_amdgcn_sched_barrier(0);  // keep the accumulator reads of later blocks below
-      }
       }
     }
     if (!more) break;
@@ -873,6 +997,171 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   for (int e = 0; e < 8; ++e) o[e] = (bf16)acc[e];
   stg8(dst, o);
 }
+
+using GemmKernel = void (*)(const bf16*, int, const bf16*, int, bf16*, int, int, int, int, int, int, int, float*,
+                            const bf16*, int, bf16*, int, RowRuns, Segments);
+
+// raises the dynamic-LDS limit of one kernel instance, once (thread-safe static initialisation)
+template <GemmKernel FN, size_t LDS_BYTES>
+hipError_t raise_lds_limit() {
+  static const hipError_t status = hipFuncSetAttribute((const void*)FN, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)LDS_BYTES);
+  return status;
+}
+
+template <bool A_T, bool B_T, int WN, int EPI = KR_GEMM_EPI_NONE, int WT = WT_LARGE>
+int launch(const Call& call, const Fused& fu) {
+  const bf16 *A = call.a, *B = call.b;
+  bf16* const C = call.c;
+  const int64_t lda = call.lda, ldb = call.ldb, ldc = call.ldc;
+  const int M = call.m, N = call.n, K = call.k, accumulate = call.accumulate;
+  float* const workspace = call.workspace;
+  const size_t workspace_bytes = call.workspace_bytes;
+  const hipStream_t stream = call.stream;
+  int num_cus = call.num_cus;
+  size_t lds_bytes = 0;
+  const int one_per_cu = fu.max_cus > 0 && fu.max_cus < num_cus ? fu.max_cus : num_cus;
+  if (WT == WT_SMALL && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
+  if (fu.max_cus > 0 && fu.max_cus < num_cus) num_cus = fu.max_cus;
+  const int tiles = ((M + 32 * WT - 1) / (32 * WT)) * ((N + 32 * WN - 1) / (32 * WN));
+  // the planned count, which the dispatcher has already capped by what the caller's workspace holds
+  int splits = call.splits;
+  const size_t one = (size_t)M * N * sizeof(float);
+  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE) {
+    splits = 1;  // a fused epilogue works on finished sums
+  } else if ((size_t)splits * one > workspace_bytes) {
+    splits = (int)(workspace_bytes / one);
+  }
+  if (splits < 2 || (int64_t)splits * M * N >= ((int64_t)1 << 31)) splits = 1;
+  // at most one persistent workgroup per compute unit (a workgroup owns a whole CU's LDS; small tiles: half)
+  // Items are spread evenly: with r = ceil(items / CUs) rounds, ceil(items / r) workgroups (rounded
+  // up to a multiple of 8, which keeps item ids and XCDs aligned) finish at the same time as one
+  // workgroup per CU would, and the CUs left over are free for other streams' kernels from the
+  // start of the launch instead of from the end of its first round.
+  auto grid_for = [&](int items) {
+    if (items <= num_cus) return items;
+    const int rounds = (items + num_cus - 1) / num_cus;
+    int g = (items + rounds - 1) / rounds;
+    g = (g + 7) / 8 * 8;
+    return g < num_cus ? g : num_cus;
+  };
+  const bool with_runs = fu.runs.a_sh || fu.runs.c_sh || fu.runs.x_sh;
+  const bool with_segs = fu.segs != nullptr;
+  // instances that honour row runs exist for what the two ends of a layer stack launch: the residual-add
+  // forward (aux or C in runs), the input gradient (plain or with the SwiGLU backward) and the weight
+  // gradient (A in runs); instances that contract operand pieces for the weight gradient (both forms)
+  constexpr bool kRunsInstance = EPI == KR_GEMM_EPI_ADD || EPI == KR_GEMM_EPI_SWIGLU_BWD || (EPI == KR_GEMM_EPI_NONE && B_T);
+  constexpr bool kSegsInstance = A_T && B_T && (EPI == KR_GEMM_EPI_NONE || EPI == KR_GEMM_EPI_TRANSPOSED_OUT);
+  // (pieces in row runs: the direct store form only, A in runs)
+  constexpr bool kSegsRunsInstance = kSegsInstance && EPI == KR_GEMM_EPI_NONE;
+  if ((with_runs && !kRunsInstance) || (with_segs && !kSegsInstance) || (with_segs && with_runs && !kSegsRunsInstance))
+    return KR_EUNSUPPORTED;
+  GemmKernel fn = nullptr;
+  hipError_t attr_status = hipSuccess;
+  auto pick_kind = [&](auto depth_tag, auto kind_tag) {
+    constexpr int DEPTH = decltype(depth_tag)::value;
+    constexpr int KIND = decltype(kind_tag)::value;
+    constexpr size_t LDS = (2 * DEPTH + 1) * kSlotBytes<WT>;
+    lds_bytes = LDS;
+    fn = gemm_kernel<A_T, B_T, WN, KIND, false, false, WT, DEPTH>;
+    attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, KIND, false, false, WT, DEPTH>, LDS>();
+    if constexpr (kRunsInstance) {
+      if (with_runs) {
+        fn = gemm_kernel<A_T, B_T, WN, KIND, true, false, WT, DEPTH>;
+        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, KIND, true, false, WT, DEPTH>, LDS>();
+      }
+    }
+    if constexpr (kSegsInstance) {
+      if (with_segs && !with_runs) {
+        fn = gemm_kernel<A_T, B_T, WN, KIND, false, true, WT, DEPTH>;
+        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, KIND, false, true, WT, DEPTH>, LDS>();
+      }
+    }
+    if constexpr (kSegsRunsInstance) {
+      if (with_segs && with_runs) {
+        fn = gemm_kernel<A_T, B_T, WN, KIND, true, true, WT, DEPTH>;
+        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, KIND, true, true, WT, DEPTH>, LDS>();
+      }
+    }
+  };
+  auto pick = [&](auto depth_tag) {
+    if constexpr (EPI == KR_GEMM_EPI_NONE) {
+      if (splits > 1) return pick_kind(depth_tag, Count<KR_GEMM_OUT_PARTIAL>{});
+      if (accumulate) return pick_kind(depth_tag, Count<KR_GEMM_OUT_ACCUMULATE>{});
+    }
+    pick_kind(depth_tag, Count<EPI>{});
+  };
+  bool deep = false;
+  if constexpr (WT == WT_SMALL) {
+    // A small tile that has its compute unit to itself waits for memory: a K-step lasts 0.5 us there, two of
+    // them are less than a load from HBM takes.  The deep ring asks four ahead.  Operands in HBM, two -> four
+    // ahead, us: 512 tokens of the 8B shard's fc1 51.4 -> 40.2, fc2 46.0 -> 37.9, fc2's input gradient 51.3 ->
+    // 44.3; 4096 x 1024 x 4096 (NT) 49.4 -> 41.1.  Up to 8 K-steps the longer prologue costs more than it
+    // hides (1536 x 512 x 256 6.3 -> 6.9, 4096 x 1024 x 512 8.7 -> 9.0).  Not beside other streams, whose
+    // workgroups can share the unit with a launch that leaves them half of the LDS.
+    deep = tiles * splits <= one_per_cu && !fu.shared && (K / BK) / splits > 8;
+    if (deep) pick(Count<kDepthAlone>{});
+  }
+  if (!deep) pick(Count<kDepth>{});
+  if (attr_status != hipSuccess) return KR_ELAUNCH;
+  const Segments segs = with_segs ? *fu.segs : Segments{};
+  if (splits == 1) {
+    hipLaunchKernelGGL(fn, dim3(grid_for(tiles)), dim3(NTHREADS), lds_bytes, stream, A, (int)lda, B, (int)ldb, C,
+                       (int)ldc, M, N, K, accumulate, 0, 1, (float*)nullptr, fu.aux, (int)fu.ld_aux, fu.out2,
+                       (int)fu.ld_out2, fu.runs, segs);
+    return kr_launch_status();
+  }
+  if constexpr (EPI != KR_GEMM_EPI_NONE) return KR_EINVAL;  // (not reached: a fused launch never splits)
+  int k_per = (K + splits - 1) / splits;
+  k_per = (k_per + BK - 1) / BK * BK;
+  splits = (K + k_per - 1) / k_per;
+  const int items = tiles * splits;
+  // (of the operands only A can be in runs here: an output in runs is never cut)
+  hipLaunchKernelGGL(fn, dim3(grid_for(items)), dim3(NTHREADS), lds_bytes, stream, A, (int)lda, B, (int)ldb, C,
+                     (int)ldc, M, N, K, 0, k_per, splits, workspace, (const bf16*)nullptr, 0, (bf16*)nullptr, 0,
+                     fu.runs, segs);
+  if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
+  const int64_t work = (int64_t)M * (N / 8);
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream,
+                     (const float*)workspace, C, ldc, M, N, splits, accumulate);
+  return kr_launch_status();
+}
+
+// the instances of a layout and epilogue by tile
+template <bool A_T, bool B_T, int EPI, int MIN_WN>
+int launch_tile(const Call& call, const Fused& fu) {
+  if constexpr (EPI != KR_GEMM_EPI_TRANSPOSED_OUT)
+    if (call.small) return launch<A_T, B_T, 4, EPI, WT_SMALL>(call, fu);
+  if constexpr (MIN_WN <= 4)
+    if (call.wn == 4) return launch<A_T, B_T, 4, EPI>(call, fu);
+  switch (call.wn) {
+    case 5: return launch<A_T, B_T, 5, EPI>(call, fu);
+    case 6: return launch<A_T, B_T, 6, EPI>(call, fu);
+    case 7: return launch<A_T, B_T, 7, EPI>(call, fu);
+    default: return launch<A_T, B_T, 8, EPI>(call, fu);
+  }
+}
+
+}  // namespace
+
+#if KR_GEMM_LAYOUT_TU == 1
+int kr_gemm::launch_nn(const Call& call, const Fused& fu) {
+  if (fu.epi == KR_GEMM_EPI_SWIGLU_BWD) return launch_tile<false, true, KR_GEMM_EPI_SWIGLU_BWD, 5>(call, fu);
+  return launch_tile<false, true, KR_GEMM_EPI_NONE, 4>(call, fu);
+}
+#elif KR_GEMM_LAYOUT_TU == 2
+int kr_gemm::launch_nt(const Call& call, const Fused& fu) {
+  if (call.transposed) return launch_tile<true, true, KR_GEMM_EPI_TRANSPOSED_OUT, 5>(call, fu);
+  return launch_tile<true, true, KR_GEMM_EPI_NONE, 4>(call, fu);
+}
+#else
+int kr_gemm::launch_tn(const Call& call, const Fused& fu) {
+  if (fu.epi == KR_GEMM_EPI_SWIGLU) return launch_tile<false, false, KR_GEMM_EPI_SWIGLU, 5>(call, fu);
+  if (fu.epi == KR_GEMM_EPI_ADD) return launch_tile<false, false, KR_GEMM_EPI_ADD, 5>(call, fu);
+  return launch_tile<false, false, KR_GEMM_EPI_NONE, 4>(call, fu);
+}
+
+namespace {
 
 // Tile width for an output with enough tiles to occupy the GPU without a split: 32 * WN columns,
 // WN in 5..8.  The estimate is the launch's own latency — rounds of tiles over the CUs times the
@@ -1010,18 +1299,6 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
   return {4, small_cut(w * kSplit), true};
 }
 
-struct Fused {
-  int epi = 0;              // KR_GEMM_EPI_*
-  const bf16* aux = nullptr;
-  int64_t ld_aux = 0;
-  bf16* out2 = nullptr;
-  int64_t ld_out2 = 0;
-  int max_cus = 0;          // > 0: use at most this many compute units
-  bool shared = false;      // other streams' kernels use the units this launch leaves idle
-  RowRuns runs = {0, 0, 0, 0, 0, 0};  // row runs of A, C, aux (all plain by default)
-  const Segments* segs = nullptr;     // layout NT: the operands come in these pieces (A and B are unused)
-};
-
 // Tile width for a projection with the SwiGLU epilogue: the tiles have to divide the 2F output
 // columns exactly (no partly filled tile column), otherwise as choose_wn.  0: no width fits.
 inline int swiglu_wn(int M, int N, int num_cus) {
@@ -1038,121 +1315,6 @@ inline int swiglu_wn(int M, int N, int num_cus) {
     }
   }
   return best;
-}
-
-using GemmKernel = void (*)(const bf16*, int, const bf16*, int, bf16*, int, int, int, int, int, int, int, float*,
-                            const bf16*, int, bf16*, int, RowRuns, Segments);
-
-// raises the dynamic-LDS limit of one kernel instance, once (thread-safe static initialisation)
-template <GemmKernel FN, size_t LDS_BYTES>
-hipError_t raise_lds_limit() {
-  static const hipError_t status = hipFuncSetAttribute((const void*)FN, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       (int)LDS_BYTES);
-  return status;
-}
-
-template <bool A_T, bool B_T, int WN, int EPI = KR_GEMM_EPI_NONE, int WT = WT_LARGE>
-int launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, bf16* C, int64_t ldc, int M,
-           int N, int K, int accumulate, float* workspace, size_t workspace_bytes,
-           hipStream_t stream, int num_cus, const Fused& fu, int planned_splits = 1) {
-  size_t lds_bytes = 0;
-  const int one_per_cu = fu.max_cus > 0 && fu.max_cus < num_cus ? fu.max_cus : num_cus;
-  if (WT == WT_SMALL && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
-  if (fu.max_cus > 0 && fu.max_cus < num_cus) num_cus = fu.max_cus;
-  const int tiles = ((M + 32 * WT - 1) / (32 * WT)) * ((N + 32 * WN - 1) / (32 * WN));
-  // the planned count, which the dispatcher has already capped by what the caller's workspace holds
-  int splits = planned_splits;
-  const size_t one = (size_t)M * N * sizeof(float);
-  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE) {
-    splits = 1;  // a fused epilogue works on finished sums
-  } else if ((size_t)splits * one > workspace_bytes) {
-    splits = (int)(workspace_bytes / one);
-  }
-  if (splits < 2 || (int64_t)splits * M * N >= ((int64_t)1 << 31)) splits = 1;
-  // at most one persistent workgroup per compute unit (a workgroup owns a whole CU's LDS; small tiles: half)
-  // Items are spread evenly: with r = ceil(items / CUs) rounds, ceil(items / r) workgroups (rounded
-  // up to a multiple of 8, which keeps item ids and XCDs aligned) finish at the same time as one
-  // workgroup per CU would, and the CUs left over are free for other streams' kernels from the
-  // start of the launch instead of from the end of its first round.
-  auto grid_for = [&](int items) {
-    if (items <= num_cus) return items;
-    const int rounds = (items + num_cus - 1) / num_cus;
-    int g = (items + rounds - 1) / rounds;
-    g = (g + 7) / 8 * 8;
-    return g < num_cus ? g : num_cus;
-  };
-  const bool with_runs = fu.runs.a_sh || fu.runs.c_sh || fu.runs.x_sh;
-  const bool with_segs = fu.segs != nullptr;
-  // instances that honour row runs exist for what the two ends of a layer stack launch: the residual-add
-  // forward (aux or C in runs), the input gradient (plain or with the SwiGLU backward) and the weight
-  // gradient (A in runs); instances that contract operand pieces for the weight gradient (both forms)
-  constexpr bool kRunsInstance = EPI == KR_GEMM_EPI_ADD || EPI == KR_GEMM_EPI_SWIGLU_BWD || (EPI == KR_GEMM_EPI_NONE && B_T);
-  constexpr bool kSegsInstance = A_T && B_T && (EPI == KR_GEMM_EPI_NONE || EPI == KR_GEMM_EPI_TRANSPOSED_OUT);
-  // (pieces in row runs: the direct store form only, A in runs)
-  constexpr bool kSegsRunsInstance = kSegsInstance && EPI == KR_GEMM_EPI_NONE;
-  if ((with_runs && !kRunsInstance) || (with_segs && !kSegsInstance) || (with_segs && with_runs && !kSegsRunsInstance))
-    return KR_EUNSUPPORTED;
-  GemmKernel fn = nullptr;
-  hipError_t attr_status = hipSuccess;
-  auto pick = [&](auto depth_tag) {
-    constexpr int DEPTH = decltype(depth_tag)::value;
-    constexpr size_t LDS = (2 * DEPTH + 1) * kSlotBytes<WT>;
-    lds_bytes = LDS;
-    fn = gemm_kernel<A_T, B_T, WN, EPI, false, false, WT, DEPTH>;
-    attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, false, WT, DEPTH>, LDS>();
-    if constexpr (kRunsInstance) {
-      if (with_runs) {
-        fn = gemm_kernel<A_T, B_T, WN, EPI, true, false, WT, DEPTH>;
-        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, false, WT, DEPTH>, LDS>();
-      }
-    }
-    if constexpr (kSegsInstance) {
-      if (with_segs && !with_runs) {
-        fn = gemm_kernel<A_T, B_T, WN, EPI, false, true, WT, DEPTH>;
-        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, false, true, WT, DEPTH>, LDS>();
-      }
-    }
-    if constexpr (kSegsRunsInstance) {
-      if (with_segs && with_runs) {
-        fn = gemm_kernel<A_T, B_T, WN, EPI, true, true, WT, DEPTH>;
-        attr_status = raise_lds_limit<gemm_kernel<A_T, B_T, WN, EPI, true, true, WT, DEPTH>, LDS>();
-      }
-    }
-  };
-  bool deep = false;
-  if constexpr (WT == WT_SMALL) {
-    // A small tile that has its compute unit to itself waits for memory: a K-step lasts 0.5 us there, two of
-    // them are less than a load from HBM takes.  The deep ring asks four ahead.  Operands in HBM, two -> four
-    // ahead, us: 512 tokens of the 8B shard's fc1 51.4 -> 40.2, fc2 46.0 -> 37.9, fc2's input gradient 51.3 ->
-    // 44.3; 4096 x 1024 x 4096 (NT) 49.4 -> 41.1.  Up to 8 K-steps the longer prologue costs more than it
-    // hides (1536 x 512 x 256 6.3 -> 6.9, 4096 x 1024 x 512 8.7 -> 9.0).  Not beside other streams, whose
-    // workgroups can share the unit with a launch that leaves them half of the LDS.
-    deep = tiles * splits <= one_per_cu && !fu.shared && (K / BK) / splits > 8;
-    if (deep) pick(Count<kDepthAlone>{});
-  }
-  if (!deep) pick(Count<kDepth>{});
-  if (attr_status != hipSuccess) return KR_ELAUNCH;
-  const Segments segs = with_segs ? *fu.segs : Segments{};
-  if (splits == 1) {
-    hipLaunchKernelGGL(fn, dim3(grid_for(tiles)), dim3(NTHREADS), lds_bytes, stream, A, (int)lda, B, (int)ldb, C,
-                       (int)ldc, M, N, K, accumulate, 0, 1, (float*)nullptr, fu.aux, (int)fu.ld_aux, fu.out2,
-                       (int)fu.ld_out2, fu.runs, segs);
-    return kr_launch_status();
-  }
-  if constexpr (EPI != KR_GEMM_EPI_NONE) return KR_EINVAL;  // (not reached: a fused launch never splits)
-  int k_per = (K + splits - 1) / splits;
-  k_per = (k_per + BK - 1) / BK * BK;
-  splits = (K + k_per - 1) / k_per;
-  const int items = tiles * splits;
-  // (of the operands only A can be in runs here: an output in runs is never cut)
-  hipLaunchKernelGGL(fn, dim3(grid_for(items)), dim3(NTHREADS), lds_bytes, stream, A, (int)lda, B, (int)ldb, C,
-                     (int)ldc, M, N, K, 0, k_per, splits, workspace, (const bf16*)nullptr, 0, (bf16*)nullptr, 0,
-                     fu.runs, segs);
-  if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
-  const int64_t work = (int64_t)M * (N / 8);
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((work + 255) / 256)), dim3(256), 0, stream,
-                     (const float*)workspace, C, ldc, M, N, splits, accumulate);
-  return kr_launch_status();
 }
 
 int device_compute_units() {
@@ -1278,62 +1440,15 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
   // finished sums and is never cut
   const Plan plan = launch_plan(M, N, K, fu.epi, fu.shared, cus, ws != nullptr && fu.runs.c_sh == 0 ? workspace_bytes : 0);
   const int wn = fu.epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn;
-  const int sp = plan.splits;
-  if (fu.epi == KR_GEMM_EPI_SWIGLU_BWD) {
-    if (lda < K || ldb < N) return KR_EINVAL;
-    if (plan.small)
-      return launch<false, true, 4, KR_GEMM_EPI_SWIGLU_BWD, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu);
-#define KR_GEMM_SWIGLU_BWD(W) \
-  return launch<false, true, W, KR_GEMM_EPI_SWIGLU_BWD>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu)
-    switch (wn) {
-      case 5: KR_GEMM_SWIGLU_BWD(5);
-      case 6: KR_GEMM_SWIGLU_BWD(6);
-      case 7: KR_GEMM_SWIGLU_BWD(7);
-      default: KR_GEMM_SWIGLU_BWD(8);
-    }
-#undef KR_GEMM_SWIGLU_BWD
-  }
-  if (fu.epi != KR_GEMM_EPI_NONE) {
-    if (lda < K || ldb < K || ldc < N) return KR_EINVAL;
-#define KR_GEMM_FUSED(W, E) \
-  return launch<false, false, W, E>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu)
-    if (fu.epi == KR_GEMM_EPI_SWIGLU) {
-      if (plan.small)
-        return launch<false, false, 4, KR_GEMM_EPI_SWIGLU, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu);
-      switch (wn) {
-        case 5: KR_GEMM_FUSED(5, KR_GEMM_EPI_SWIGLU);
-        case 6: KR_GEMM_FUSED(6, KR_GEMM_EPI_SWIGLU);
-        case 7: KR_GEMM_FUSED(7, KR_GEMM_EPI_SWIGLU);
-        default: KR_GEMM_FUSED(8, KR_GEMM_EPI_SWIGLU);
-      }
-    }
-    if (plan.small)
-      return launch<false, false, 4, KR_GEMM_EPI_ADD, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, 0, ws, workspace_bytes, st, num_cus, fu);
-    switch (wn) {
-      case 5: KR_GEMM_FUSED(5, KR_GEMM_EPI_ADD);
-      case 6: KR_GEMM_FUSED(6, KR_GEMM_EPI_ADD);
-      case 7: KR_GEMM_FUSED(7, KR_GEMM_EPI_ADD);
-      default: KR_GEMM_FUSED(8, KR_GEMM_EPI_ADD);
-    }
-#undef KR_GEMM_FUSED
-  }
-#define KR_GEMM_LAUNCH(AT, BT)                                                                           \
-  if (plan.small)                                                                                        \
-    return launch<AT, BT, 4, KR_GEMM_EPI_NONE, WT_SMALL>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
-  switch (wn) {                                                                                          \
-    case 4: return launch<AT, BT, 4>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
-    case 5: return launch<AT, BT, 5>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
-    case 6: return launch<AT, BT, 6>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
-    case 7: return launch<AT, BT, 7>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
-    default: return launch<AT, BT, 8>(a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, fu, sp); \
-  }
+  const Call call{a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, wn,
+                  fu.epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.small, false};
   switch (layout) {
     case KR_GEMM_TN:  // A [M,K], B [N,K]
       if (lda < K || ldb < K || ldc < N) return KR_EINVAL;
-      KR_GEMM_LAUNCH(false, false)
+      return launch_tn(call, fu);
     case KR_GEMM_NN:  // A [M,K], B [K,N]
       if (lda < K || ldb < N || ldc < N) return KR_EINVAL;
-      KR_GEMM_LAUNCH(false, true)
+      return launch_nn(call, fu);
     case KR_GEMM_NT: {  // A [K,M], B [K,N]
       if (lda < M || ldb < N || ldc < N) return KR_EINVAL;
       // Both operands of this layout are read the same way, so C^T = B^T . A is the same kernel
@@ -1363,23 +1478,15 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
             exchanged.steps = fu.segs->steps;
             fut.segs = &exchanged;
           }
-#define KR_GEMM_TRANS(W) \
-  return launch<true, true, W, KR_GEMM_EPI_TRANSPOSED_OUT>(b, ldb, a, lda, c, ldc, N, M, K, 0, nullptr, 0, st, num_cus, fut)
-          switch (wt) {
-            case 5: KR_GEMM_TRANS(5);
-            case 6: KR_GEMM_TRANS(6);
-            case 7: KR_GEMM_TRANS(7);
-            default: KR_GEMM_TRANS(8);
-          }
-#undef KR_GEMM_TRANS
+          const Call exchanged_call{b, ldb, a, lda, c, ldc, N, M, K, 0, nullptr, 0, st, num_cus, wt, 1, false, true};
+          return launch_nt(exchanged_call, fut);
         }
       }
-      KR_GEMM_LAUNCH(true, true)
+      return launch_nt(call, fu);
     }
     default:
       return KR_EINVAL;
   }
-#undef KR_GEMM_LAUNCH
 }
 }  // namespace
 
@@ -1477,3 +1584,4 @@ extern "C" int kr_gemm_bf16_nt_segments(int M, int N, int k_seg, int nseg, const
   return gemm_dispatch(KR_GEMM_NT, M, N, k_seg * nseg, A[0], lda, B[0], ldb, C, ldc, accumulate, workspace,
                        workspace_bytes, stream, fu);
 }
+#endif  // KR_GEMM_LAYOUT_TU == 0

@@ -319,6 +319,33 @@ def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(big_x, big_w, residual=embed(res, R_, C_))[:m, :n])
 
 
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("k", [8, 64, 72, 128, 136, 192, 200, 1096])
+def test_gemm_items_of_one_workgroup_have_the_bits_of_items_of_their_own(be, k, tile):
+    """A workgroup that has further items requests their first K-steps in the last two of the one it is at.  On eight
+    compute units every workgroup has several items, on the whole device one at most: the same bits, in every layout, with
+    every kind of output, at contractions of one K-step, two, three and many, with and without a partial last one."""
+    m, n = (520, 640) if tile == 128 else (4104, 3080)
+    x, w, dy = rnd(m, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(m, n, seed=63)
+    for layout, a, b, (p, q, c) in ((0, x, w, (m, n, k)), (1, x, w.t().contiguous(), (m, n, k)),
+                                    (2, x.t().contiguous(), w.t().contiguous(), (m, n, k))):
+        alone, few = (dict(split_k=None, max_cus=cus) for cus in (0, 8))
+        got = be.gemm(layout, a, b, p, q, c, **few)
+        assert torch.equal(got, be.gemm(layout, a, b, p, q, c, **alone))
+        base = rnd(p, q, seed=64)
+        assert torch.equal(be.gemm(layout, a, b, p, q, c, out=base.clone(), accumulate=True, **few),
+                           be.gemm(layout, a, b, p, q, c, out=base.clone(), accumulate=True, **alone))
+    assert rel(got, x.float() @ w.float().t()) <= TOL
+    pre = rnd(m, 2 * n, seed=65)
+    assert torch.equal(be.gemm(0, x, w, m, n, k, residual=dy, **few), be.gemm(0, x, w, m, n, k, residual=dy, **alone))
+    wt = w.t().contiguous()
+    assert torch.equal(be.gemm(1, x, wt, m, n, k, swiglu_bwd_x=pre, **few), be.gemm(1, x, wt, m, n, k, swiglu_bwd_x=pre, **alone))
+    f = 1280 if tile == 256 else 320
+    ys = [torch.empty(m, f, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+    x2 = [be.gemm(0, x, w[:2 * f].contiguous(), m, 2 * f, k, swiglu_out=y, **how) for y, how in zip(ys, (few, alone))]
+    assert torch.equal(*x2) and torch.equal(*ys)
+
+
 @pytest.mark.parametrize("m,f,k", [(8, 64, 64), (128, 320, 128), (136, 448, 200), (520, 512, 1096), (512, 1792, 1024)])
 def test_gemm_small_tiles_with_swiglu_have_the_bits_of_the_large_ones(be, m, f, k):
     """The SwiGLU epilogues, forward (gate and up columns of a tile side by side) and backward, in the same way."""
