@@ -374,6 +374,8 @@ class HipBackend:
         """Whether ``linear_wgrad_segments`` takes these operand pairs: matrices of one shape and one row
         stride in every pair (the ``dys`` may be nanobatch slices in row runs, all alike), a multiple of 64 rows
         each, at most MAX_WGRAD_SEGMENTS pairs."""
+        if self._n is not None and self.MAX_RUN_ROWS == 16 and self._n.wgrad_segments_ok(dys, xs):
+            return True
         if not 1 <= len(dys) == len(xs) <= self.MAX_WGRAD_SEGMENTS:
             return False
         first = None
@@ -471,6 +473,9 @@ class HipBackend:
 
     def rmsnorm_dgamma(self, partials: Tensor, gamma: Tensor) -> Tensor:
         """Sum of the partial rows ([n, cols] fp32) of all nanobatches -> the weight gradient."""
+        done = self._n.rmsnorm_dgamma(partials, gamma)
+        if done is not None:
+            return done
         dgamma = torch.empty_like(gamma)
         self._check(self.lib.kr_rmsnorm_dgamma(partials.data_ptr(), partials.shape[0], partials.shape[1],
                                                dgamma.data_ptr(), self._stream()), "kr_rmsnorm_dgamma")
@@ -642,6 +647,10 @@ class HipBackend:
         """``residual + dropout(x, p)`` and the byte mask of kept elements (same shape, dense).  The
         mask is keyed by a seed drawn from PyTorch's CPU generator, so ``torch.manual_seed`` fixes it
         and a restored CPU generator state (activation recomputation) reproduces it."""
+        if torch.get_default_device().type == "cpu":
+            done = self._n.dropout_add(x, residual, p, out, None)   # (draws the seed itself, on the default device)
+            if done is not None:
+                return done
         self._dev(x, residual)
         self._bf16(x, residual)
         if x.shape != residual.shape:
@@ -913,3 +922,7 @@ class HipBackend:
                 t._kr_mixed = mixed
                 t._kr_fused5 = fused
         return dq, dk, dv
+
+
+#: the backend's methods as defined here (a caller that goes past them asks whether they still are)
+STOCK = dict(HipBackend.__dict__)

@@ -191,6 +191,41 @@ size_t gemm_workspace(int layout, int m, int n, int k, bool alone) {
 
 bool fits_int(int64_t v) { return v > 0 && v < ((int64_t)1 << 31); }
 
+// What a product's epilogue takes along: the residual, or the activation's input (operand and address), or the
+// activation's output.
+struct Epilogue {
+  int kind = KR_GEMM_EPI_NONE;
+  const void* aux = nullptr;
+  Operand ox;
+  void* out2 = nullptr;
+  int64_t ld_out2 = 0;
+};
+
+// allocates the workspace and launches; the operands have been checked, ``out`` is there
+int run_gemm(int layout, int64_t m, int64_t n, int64_t k, const Tensor& a, const Operand& oa, const Tensor& b,
+             const Operand& ob, const Tensor& out, const Operand& oc, bool accumulate, int split, const Epilogue& e,
+             int max_cus) {
+  const int epilogue = e.kind | (split == 2 ? KR_GEMM_BESIDE_OTHER_STREAMS : 0);
+  Tensor ws;
+  size_t ws_bytes = 0;
+  if (e.kind == KR_GEMM_EPI_NONE && split != 0 && oc.run_rows == 1) {
+    ws_bytes = gemm_workspace(layout, (int)m, (int)n, (int)k, split == 1);
+    if (ws_bytes) ws = bytes(ws_bytes, a);
+  }
+  void* ws_ptr = ws_bytes ? ptr(ws) : nullptr;
+  if (oa.run_rows > 1 || oc.run_rows > 1 || e.ox.run_rows > 1)
+    return kr_gemm_bf16_runs(layout, (int)m, (int)n, (int)k, ptr(a), oa.ld, oa.run_rows, oa.run_ld, ptr(b), ob.ld,
+                             ptr(out), oc.ld, oc.run_rows, oc.run_ld, accumulate, epilogue, e.aux, e.ox.ld, e.ox.run_rows,
+                             e.ox.run_ld, e.out2, e.ld_out2, max_cus, ws_ptr, ws_bytes, stream());
+  return kr_gemm_bf16_fused(layout, (int)m, (int)n, (int)k, ptr(a), oa.ld, ptr(b), ob.ld, ptr(out), oc.ld, accumulate,
+                            epilogue, e.aux, e.ox.ld, e.out2, e.ld_out2, max_cus, ws_ptr, ws_bytes, stream());
+}
+PyObject* gemm_failed(int layout, int64_t m, int64_t n, int64_t k, int epi, int rc) {
+  return failed("kr_gemm_bf16(layout=" + std::to_string(layout) + ", M=" + std::to_string(m) + ", N=" + std::to_string(n) +
+                    ", K=" + std::to_string(k) + ", epilogue=" + std::to_string(epi) + ")",
+                rc);
+}
+
 // gemm(layout, a, b, m, n, k, out, accumulate, split, residual, swiglu_out, swiglu_bwd_x, max_cus); split: 0 never,
 // 1 the GEMM has the device to itself, 2 beside other streams
 PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
@@ -214,29 +249,25 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (layout < KR_GEMM_TN || layout > KR_GEMM_NT || oa.rows != (a_t ? k : m) || oa.cols != (a_t ? m : k) ||
         ob.rows != (b_t ? k : n) || ob.cols != (b_t ? n : k) || !fits_int(m) || !fits_int(n) || !fits_int(k))
       return none();
-    int epi = KR_GEMM_EPI_NONE;
-    const void* aux = nullptr;
-    Operand ox;
-    void* out2 = nullptr;
-    int64_t ld_out2 = 0;
+    Epilogue e;
     int64_t out_cols = n;
     if (!absent(p_res)) {
-      ox = operand3(tensor(p_res));
-      if (!ox.ok || ox.rows != m || ox.cols != n) return none();
-      epi = KR_GEMM_EPI_ADD;
-      aux = ptr(tensor(p_res));
+      e.ox = operand3(tensor(p_res));
+      if (!e.ox.ok || e.ox.rows != m || e.ox.cols != n) return none();
+      e.kind = KR_GEMM_EPI_ADD;
+      e.aux = ptr(tensor(p_res));
     } else if (!absent(p_act)) {
       const Tensor& act = tensor(p_act);
       if (act.dim() != 2 || act.size(0) != m || act.size(1) * 2 != n || act.stride(1) != 1) return none();
-      epi = KR_GEMM_EPI_SWIGLU;
-      out2 = ptr(act);
-      ld_out2 = act.stride(0);
+      e.kind = KR_GEMM_EPI_SWIGLU;
+      e.out2 = ptr(act);
+      e.ld_out2 = act.stride(0);
     } else if (!absent(p_pre)) {
       const Tensor& pre = tensor(p_pre);
       if (accumulate || pre.dim() != 2 || pre.size(0) != m || pre.size(1) != 2 * n || pre.stride(1) != 1) return none();
-      epi = KR_GEMM_EPI_SWIGLU_BWD;
-      ox.ld = pre.stride(0);
-      aux = ptr(pre);
+      e.kind = KR_GEMM_EPI_SWIGLU_BWD;
+      e.ox.ld = pre.stride(0);
+      e.aux = ptr(pre);
       out_cols = 2 * n;
     }
     if (accumulate && absent(p_out)) return none();
@@ -250,32 +281,52 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       oc = operand3(out);
       if (!oc.ok || oc.rows != m || oc.cols != out_cols) return none();
     }
-    const int epilogue = epi | (split == 2 ? KR_GEMM_BESIDE_OTHER_STREAMS : 0);
     int rc;
     {
       WithoutInterpreter free;
       if (!out.defined()) out = matrix(m, out_cols, ta);
-      Tensor ws;
-      size_t ws_bytes = 0;
-      if (epi == KR_GEMM_EPI_NONE && split != 0 && oc.run_rows == 1) {
-        ws_bytes = gemm_workspace(layout, (int)m, (int)n, (int)k, split == 1);
-        if (ws_bytes) ws = bytes(ws_bytes, ta);
-      }
-      void* ws_ptr = ws_bytes ? ptr(ws) : nullptr;
-      if (oa.run_rows > 1 || oc.run_rows > 1 || ox.run_rows > 1) {
-        rc = kr_gemm_bf16_runs(layout, (int)m, (int)n, (int)k, ptr(ta), oa.ld, oa.run_rows, oa.run_ld, ptr(tb), ob.ld,
-                               ptr(out), oc.ld, oc.run_rows, oc.run_ld, accumulate, epilogue, aux, ox.ld, ox.run_rows,
-                               ox.run_ld, out2, ld_out2, max_cus, ws_ptr, ws_bytes, stream());
-      } else {
-        rc = kr_gemm_bf16_fused(layout, (int)m, (int)n, (int)k, ptr(ta), oa.ld, ptr(tb), ob.ld, ptr(out), oc.ld,
-                                accumulate, epilogue, aux, ox.ld, out2, ld_out2, max_cus, ws_ptr, ws_bytes, stream());
-      }
+      rc = run_gemm(layout, m, n, k, ta, oa, tb, ob, out, oc, accumulate, split, e, max_cus);
     }
-    if (rc != KR_OK)
-      return failed("kr_gemm_bf16(layout=" + std::to_string(layout) + ", M=" + std::to_string(m) + ", N=" +
-                        std::to_string(n) + ", K=" + std::to_string(k) + ", epilogue=" + std::to_string(epi) + ")",
-                    rc);
+    if (rc != KR_OK) return gemm_failed(layout, m, n, k, e.kind, rc);
     return absent(p_out) ? wrap(std::move(out)) : Py_NewRef(p_out);
+  });
+}
+
+// operand pairs of a weight gradient over several nanobatches: matrices of one shape and one row stride in every pair (those of
+// ``dys`` may be in row runs, all alike), a multiple of 64 rows each
+struct Pieces {
+  Py_ssize_t n = 0;
+  Tensor held[2 * KR_GEMM_MAX_SEGMENTS];  // the lists may change while the interpreter is free
+  Operand a, b;
+};
+bool pieces(PyObject* dys, PyObject* xs, Pieces& p) {
+  if (!PyList_Check(dys) || !PyList_Check(xs)) return false;
+  p.n = PyList_GET_SIZE(dys);
+  if (p.n < 1 || p.n > KR_GEMM_MAX_SEGMENTS || PyList_GET_SIZE(xs) != p.n) return false;
+  for (Py_ssize_t i = 0; i < p.n; ++i) {
+    PyObject *dy = PyList_GET_ITEM(dys, i), *x = PyList_GET_ITEM(xs, i);
+    if (!bf16_arg(dy) || !bf16_arg(x)) return false;
+    const Operand oa = operand3(tensor(dy)), ob = operand3(tensor(x));
+    if (!oa.ok || !ob.ok || ob.run_rows > 1 || oa.rows != ob.rows || oa.rows % 64 || tensor(x).device() != tensor(dy).device())
+      return false;
+    if (i == 0) {
+      p.a = oa, p.b = ob;
+    } else if (oa.rows != p.a.rows || oa.ld != p.a.ld || oa.run_rows != p.a.run_rows || oa.run_ld != p.a.run_ld ||
+               ob.ld != p.b.ld || oa.cols != p.a.cols || ob.cols != p.b.cols) {
+      return false;
+    }
+    p.held[2 * i] = tensor(dy);
+    p.held[2 * i + 1] = tensor(x);
+  }
+  return true;
+}
+
+// wgrad_segments_ok(dys, xs) -> True, or None where the Python side has to look
+PyObject* py_wgrad_segments_ok(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    Pieces p;
+    if (n_args != 2 || !pieces(a[0], a[1], p)) return none();
+    Py_RETURN_TRUE;
   });
 }
 
@@ -283,28 +334,12 @@ PyObject* py_gemm(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 // are not pieces the kernel takes
 PyObject* py_wgrad_segments(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
-    if (n_args != 6 || !PyList_Check(a[0]) || !PyList_Check(a[1])) return none();
-    const Py_ssize_t nseg = PyList_GET_SIZE(a[0]);
-    if (nseg < 1 || nseg > KR_GEMM_MAX_SEGMENTS || PyList_GET_SIZE(a[1]) != nseg) return none();
+    Pieces p;
+    if (n_args != 6 || !pieces(a[0], a[1], p)) return none();
+    const Py_ssize_t nseg = p.n;
     const void *pa[KR_GEMM_MAX_SEGMENTS], *pb[KR_GEMM_MAX_SEGMENTS];
-    Tensor held[2 * KR_GEMM_MAX_SEGMENTS];  // the lists may change while the interpreter is free
-    Operand fa, fb;
-    for (Py_ssize_t i = 0; i < nseg; ++i) {
-      PyObject *dy = PyList_GET_ITEM(a[0], i), *x = PyList_GET_ITEM(a[1], i);
-      if (!bf16_arg(dy) || !bf16_arg(x)) return none();
-      const Operand oa = operand3(tensor(dy)), ob = operand3(tensor(x));
-      if (!oa.ok || !ob.ok || ob.run_rows > 1 || oa.rows != ob.rows || oa.rows % 64 ||
-          tensor(x).device() != tensor(dy).device())
-        return none();
-      if (i == 0) {
-        fa = oa, fb = ob;
-      } else if (oa.rows != fa.rows || oa.ld != fa.ld || oa.run_rows != fa.run_rows || oa.run_ld != fa.run_ld ||
-                 ob.ld != fb.ld || oa.cols != fa.cols || ob.cols != fb.cols) {
-        return none();
-      }
-      held[2 * i] = tensor(dy);
-      held[2 * i + 1] = tensor(x);
-    }
+    const Operand &fa = p.a, &fb = p.b;
+    Tensor* const held = p.held;
     const int64_t m = fa.cols, n = fb.cols, k = fa.rows * nseg;
     if (!fits_int(m) || !fits_int(n) || !fits_int(k)) return none();
     const bool accumulate = truth(a[3]);
@@ -431,6 +466,16 @@ PyObject* py_rmsnorm_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // ---- rotary embedding on a fused QKV buffer, in place ------------------------------------------------------
+// (the table is one row per position: a dimension between the rows and the channels has to be a 1)
+bool is_rotary_table(const Tensor& fr, int64_t s, int64_t hd) {
+  return fr.dim() >= 2 && fr.is_contiguous() && fr.size(-1) == hd && fr.numel() == fr.size(0) * hd && fr.size(0) >= s;
+}
+int run_rope(const Tensor& f, const Tensor& fr, bool backward) {
+  const int64_t s = f.size(0), b = f.size(1), slots = f.size(3), heads = f.size(2) * slots, hd = f.size(4);
+  return kr_rope(ptr(f), ptr(f), (const float*)ptr(fr), (int)s, (int)b, (int)heads, (int)hd, b * heads * hd, heads * hd, hd,
+                 b * heads * hd, heads * hd, hd, backward, (int)slots, (int)slots - 1, stream());
+}
+
 // rope_fused(fused [s, b, ng, per + 2, hd], per, freqs [rows >= s, 1.., hd] fp32, backward) -> True
 PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
@@ -438,17 +483,12 @@ PyObject* py_rope_fused(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor &f = tensor(a[0]), &fr = tensor(a[2]);
     const int64_t per = integer(a[1]);
     const bool backward = truth(a[3]);
-    // (the table is one row per position: a dimension between the rows and the channels has to be a 1)
-    if (f.dim() != 5 || !f.is_contiguous() || f.size(3) != per + 2 || fr.dim() < 2 || !fr.is_contiguous() ||
-        fr.size(-1) != f.size(4) || fr.numel() != fr.size(0) * f.size(4) || fr.size(0) < f.size(0))
-      return none();
-    const int64_t s = f.size(0), b = f.size(1), slots = f.size(3), heads = f.size(2) * slots, hd = f.size(4);
-    if (!fits_int(s) || !fits_int(b) || !fits_int(heads)) return none();
+    if (f.dim() != 5 || !f.is_contiguous() || f.size(3) != per + 2 || !is_rotary_table(fr, f.size(0), f.size(4))) return none();
+    if (!fits_int(f.size(0)) || !fits_int(f.size(1)) || !fits_int(f.size(2) * f.size(3))) return none();
     int rc;
     {
       WithoutInterpreter free;
-      rc = kr_rope(ptr(f), ptr(f), (const float*)ptr(fr), (int)s, (int)b, (int)heads, (int)hd, b * heads * hd, heads * hd, hd,
-                   b * heads * hd, heads * hd, hd, backward, (int)slots, (int)slots - 1, stream());
+      rc = run_rope(f, fr, backward);
     }
     if (rc != KR_OK) return failed("kr_rope", rc);
     Py_RETURN_TRUE;
@@ -499,6 +539,22 @@ std::string attn_name(const char* what, const AttnShape& c) {
          ", nkv=" + std::to_string(c.nkv) + ", hd=" + std::to_string(c.hd) + ")";
 }
 
+int run_attn_fwd(const AttnShape& c, const Tensor& q, const Tensor& k, const Tensor& v, float scale, int flags, Tensor& o,
+                 Tensor& lse) {
+  o = at::empty({c.s, c.b, c.nq, c.hd}, q.options());
+  lse = at::empty({c.b, c.nq, c.s}, q.options().dtype(at::kFloat));
+  Tensor ws;
+  const QStrides sq = q_strides(q, c.per), so = q_strides(o, c.per);
+  const size_t n = (flags & KR_ATTN_GENERAL_KERNELS)
+                       ? 0
+                       : kr_attn_fwd_workspace_bytes_strided(c.s, c.b, c.nq, c.nkv, c.hd,
+                                                             std::max({sq.s, so.s, k.stride(0), v.stride(0)}));
+  if (n) ws = bytes(n, q);
+  return kr_attn_fwd_ws(ptr(q), ptr(k), ptr(v), ptr(o), (float*)ptr(lse), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b, sq.g,
+                        sq.h, k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), so.s, so.b, so.g,
+                        so.h, flags | KR_ATTN_IN_PLACE, n ? ptr(ws) : nullptr, n, stream());
+}
+
 // attn_fwd(q, k, v, scale, flags) -> (o [s, b, nq, hd], lse [b, nq, s])
 PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
@@ -512,23 +568,40 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     int rc;
     {
       WithoutInterpreter free;
-      o = at::empty({c.s, c.b, c.nq, c.hd}, q.options());
-      lse = at::empty({c.b, c.nq, c.s}, q.options().dtype(at::kFloat));
-      Tensor ws;
-      const QStrides sq = q_strides(q, c.per), so = q_strides(o, c.per);
-      const size_t n = (flags & KR_ATTN_GENERAL_KERNELS)
-                           ? 0
-                           : kr_attn_fwd_workspace_bytes_strided(c.s, c.b, c.nq, c.nkv, c.hd,
-                                                                 std::max({sq.s, so.s, k.stride(0), v.stride(0)}));
-      if (n) ws = bytes(n, q);
-      rc = kr_attn_fwd_ws(ptr(q), ptr(k), ptr(v), ptr(o), (float*)ptr(lse), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b,
-                          sq.g, sq.h, k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), so.s,
-                          so.b, so.g, so.h, flags | KR_ATTN_IN_PLACE, n ? ptr(ws) : nullptr, n, stream());
+      rc = run_attn_fwd(c, q, k, v, scale, flags, o, lse);
     }
     if (rc != KR_OK) return failed(attn_name("kr_attn_fwd", c), rc);
     PyObject *po = wrap(std::move(o)), *pl = wrap(std::move(lse));
     return Py_BuildValue("(NN)", po, pl);
   });
+}
+
+// the gradients of a grouped q, k and v: views of one buffer [s, b, nkv, per + 2, hd]
+struct AttnGrads {
+  Tensor fused, mixed, dq, dk, dv;
+};
+bool attn_bwd_ok(const AttnShape& c, const Tensor& dout, const Tensor& q, const Tensor& o, const Tensor& lse) {
+  return c.ok && q.dim() == 5 && dout.is_contiguous() && o.is_contiguous() && lse.is_contiguous() &&
+         dout.numel() == (int64_t)c.s * c.b * c.nq * c.hd && o.numel() == dout.numel() &&
+         lse.numel() == (int64_t)c.b * c.nq * c.s;
+}
+int run_attn_bwd(const AttnShape& c, const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                 const Tensor& lse, float scale, int flags, AttnGrads& g) {
+  const int64_t s = c.s, b = c.b, ng = c.nkv, hd = c.hd, group = (c.per + 2) * hd, w = ng * group;
+  g.fused = at::empty({s, b, ng, c.per + 2, hd}, q.options());
+  g.mixed = g.fused.view({s, b, w});
+  g.dq = g.fused.as_strided({s, b, ng, c.per, hd}, {b * w, w, group, hd, 1}, 0);
+  g.dk = g.fused.as_strided({s, b, ng, hd}, {b * w, w, group, 1}, c.per * hd);
+  g.dv = g.fused.as_strided({s, b, ng, hd}, {b * w, w, group, 1}, (c.per + 1) * hd);
+  const QStrides sq = q_strides(q, c.per);
+  const int64_t os = b * c.nq * hd, ob = c.nq * hd, og = c.per * hd;
+  const size_t n = kr_attn_bwd_workspace_bytes_strided(c.s, c.b, c.nq, c.nkv, c.hd,
+                                                       std::max({sq.s, k.stride(0), v.stride(0), os, b * w}));
+  const Tensor ws = bytes(n < 16 ? 16 : n, q);
+  return kr_attn_bwd_flags(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(o), (const float*)ptr(lse), ptr(g.dq), ptr(g.dk), ptr(g.dv),
+                           ptr(ws), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b, sq.g, sq.h, k.stride(0), k.stride(1),
+                           k.stride(2), v.stride(0), v.stride(1), v.stride(2), os, ob, og, hd, os, ob, og, hd, b * w, w, group,
+                           hd, b * w, w, group, b * w, w, group, flags, stream());
 }
 
 // attn_bwd(do, q, k, v, o, lse, scale, flags) -> (dq, dk, dv, mixed, fused) for a grouped q: views of one buffer
@@ -542,42 +615,26 @@ PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor &dout = tensor(a[0]), &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &o = tensor(a[4]),
                  &lse = tensor(a[5]);
     const AttnShape c = attn_shape(q, k, v);
-    if (!c.ok || q.dim() != 5 || !dout.is_contiguous() || !o.is_contiguous() || !lse.is_contiguous() ||
-        dout.numel() != (int64_t)c.s * c.b * c.nq * c.hd || o.numel() != dout.numel() ||
-        lse.numel() != (int64_t)c.b * c.nq * c.s)
-      return none();
+    if (!attn_bwd_ok(c, dout, q, o, lse)) return none();
     const float scale = (float)real(a[6]);
     const int flags = (int)integer(a[7]);
-    const int64_t s = c.s, b = c.b, ng = c.nkv, hd = c.hd, g = (c.per + 2) * hd, w = ng * g;
-    Tensor fused, mixed, dq, dk, dv;
+    AttnGrads g;
     int rc;
     {
       WithoutInterpreter free;
-      fused = at::empty({s, b, ng, c.per + 2, hd}, q.options());
-      mixed = fused.view({s, b, w});
-      dq = fused.as_strided({s, b, ng, c.per, hd}, {b * w, w, g, hd, 1}, 0);
-      dk = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, c.per * hd);
-      dv = fused.as_strided({s, b, ng, hd}, {b * w, w, g, 1}, (c.per + 1) * hd);
-      const QStrides sq = q_strides(q, c.per);
-      const int64_t os = b * c.nq * hd, ob = c.nq * hd, og = c.per * hd;
-      const size_t n = kr_attn_bwd_workspace_bytes_strided(c.s, c.b, c.nq, c.nkv, c.hd,
-                                                           std::max({sq.s, k.stride(0), v.stride(0), os, b * w}));
-      Tensor ws = bytes(n < 16 ? 16 : n, q);
-      rc = kr_attn_bwd_flags(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(o), (const float*)ptr(lse), ptr(dq), ptr(dk), ptr(dv),
-                             ptr(ws), c.s, c.b, c.nq, c.nkv, c.hd, scale, sq.s, sq.b, sq.g, sq.h, k.stride(0), k.stride(1),
-                             k.stride(2), v.stride(0), v.stride(1), v.stride(2), os, ob, og, hd, os, ob, og, hd, b * w, w, g, hd,
-                             b * w, w, g, b * w, w, g, flags, stream());
+      rc = run_attn_bwd(c, dout, q, k, v, o, lse, scale, flags, g);
     }
     if (rc != KR_OK) return failed(attn_name("kr_attn_bwd", c), rc);
-    PyObject *pq = wrap(std::move(dq)), *pk = wrap(std::move(dk)), *pv = wrap(std::move(dv));
-    PyObject* pm = wrap(std::move(mixed));
-    PyObject* pf = wrap(std::move(fused));
+    PyObject *pq = wrap(std::move(g.dq)), *pk = wrap(std::move(g.dk)), *pv = wrap(std::move(g.dv));
+    PyObject* pm = wrap(std::move(g.mixed));
+    PyObject* pf = wrap(std::move(g.fused));
     return Py_BuildValue("(NNNNN)", pq, pk, pv, pm, pf);
   });
 }
 
 // ---- hidden dropout ---------------------------------------------------------------------------------------------
-// dropout_add(x, residual, p, out, seed) -> (out, mask)
+// dropout_add(x, residual, p, out, seed) -> (out, mask); without a seed it is drawn from PyTorch's CPU generator, as
+// torch.randint draws it, once the operands have been found to fit
 PyObject* py_dropout_add(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
     if (n_args != 5 || !bf16_arg(a[0]) || !bf16_arg(a[1])) return none();
@@ -588,7 +645,17 @@ PyObject* py_dropout_add(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!absent(a[3]) && (!bf16_arg(a[3]) || tensor(a[3]).sizes() != x.sizes())) return none();
     const double p = real(a[2]);
     if (!(p >= 0.0 && p < 1.0)) return none();
-    const uint64_t seed = seed_value(a[4]);
+    if (absent(a[4]) && !absent(a[3])) {
+      // (the caller has not looked at ``out`` yet: one row per entry of the first dimension, as it takes them)
+      const Tensor& t = tensor(a[3]);
+      int64_t inner = 1;
+      for (int64_t i = t.dim() - 1; i >= 1; --i) {
+        if (t.size(i) != 1 && t.stride(i) != inner) return none();
+        inner *= t.size(i);
+      }
+      if (t.dim() < 2 || t.stride(0) % 8 || t.stride(0) < inner || t.device() != x.device()) return none();
+    }
+    uint64_t seed = absent(a[4]) ? 0 : seed_value(a[4]);
     Tensor out, mask;
     Operand oc;
     if (absent(a[3])) {
@@ -599,6 +666,7 @@ PyObject* py_dropout_add(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       oc = operand(out);
       if (!oc.ok || oc.run_rows > 1) return none();
     }
+    if (absent(a[4])) seed = (uint64_t)at::randint(0, (int64_t)1 << 62, {1}, at::TensorOptions().dtype(at::kLong)).item<int64_t>();
     int rc;
     {
       WithoutInterpreter free;
@@ -634,9 +702,404 @@ PyObject* py_dropout_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   });
 }
 
+// ---- the operators of a partition in one call ----------------------------------------------------------------------
+// What stands between two schedule points of a decoder layer is a fixed chain of operators: norm, QKV projection, split,
+// rotary embedding, attention, out-projection; or norm, fc1, activation, fc2.  The chains below run the launches of such an
+// operator sequence in the same order, with the same plans and results as one call per operator, and hand back what each of
+// them saves; between the launches the interpreter had spent several times what the launches cost.  Whatever a chain does not
+// take is answered with None before anything is launched.
+
+// (no references of a failed chain's tensors are left behind)
+PyObject* pack(std::initializer_list<Tensor*> items) {
+  PyObject* t = PyTuple_New((Py_ssize_t)items.size());
+  if (!t) return nullptr;
+  Py_ssize_t i = 0;
+  for (Tensor* v : items) PyTuple_SET_ITEM(t, i++, v && v->defined() ? wrap(std::move(*v)) : Py_NewRef(Py_None));
+  return t;
+}
+bool is_weight(PyObject* o, int64_t rows, int64_t cols) {
+  if (!bf16_arg(o) || symbolic(tensor(o))) return false;
+  const Operand w = operand2(tensor(o));
+  return w.ok && w.rows == rows && w.cols == cols;
+}
+Operand dense(int64_t rows, int64_t cols) {
+  Operand o;
+  o.rows = rows, o.cols = o.ld = cols, o.ok = true;
+  return o;
+}
+// the output of a product: the caller's tensor, or a new dense one (``given`` stays undefined)
+struct Output {
+  Tensor t;
+  Operand o;
+  bool ok = false;
+};
+Output output(PyObject* given, int64_t rows, int64_t cols) {
+  Output r;
+  if (absent(given)) {
+    r.o = dense(rows, cols);
+    r.ok = cols % 8 == 0;
+  } else if (bf16_arg(given)) {
+    r.t = tensor(given);
+    r.o = operand3(r.t);
+    r.ok = r.o.ok && r.o.rows == rows && r.o.cols == cols;
+  }
+  return r;
+}
+bool residual(PyObject* o, int64_t rows, int64_t cols, Epilogue& e) {
+  if (absent(o)) return true;
+  if (!bf16_arg(o)) return false;
+  e.ox = operand3(tensor(o));
+  e.kind = KR_GEMM_EPI_ADD;
+  e.aux = ptr(tensor(o));
+  return e.ox.ok && e.ox.rows == rows && e.ox.cols == cols;
+}
+// x [s, b, h] of a norm and what it makes: the rows as the kernels address them, y and rstd
+struct Norm {
+  Operand o;
+  Tensor rows, y, rstd;
+};
+int run_norm(const Tensor& x, const Tensor& gamma, float eps, Norm& n) {
+  n.rows = n.o.run_rows > 1 ? x : x.view({n.o.rows, n.o.cols});
+  n.y = matrix(n.o.rows, n.o.cols, x);
+  n.rstd = at::empty({n.o.rows}, x.options().dtype(at::kFloat));
+  return n.o.run_rows > 1 ? kr_rmsnorm_fwd_runs(ptr(x), ptr(gamma), ptr(n.y), (float*)ptr(n.rstd), (int)n.o.rows, (int)n.o.cols,
+                                                n.o.ld, n.o.run_rows, n.o.run_ld, eps, stream())
+                          : kr_rmsnorm_fwd(ptr(x), ptr(gamma), ptr(n.y), (float*)ptr(n.rstd), (int)n.o.rows, (int)n.o.cols,
+                                           n.o.ld, eps, stream());
+}
+bool norm_input(PyObject* x, PyObject* gamma, Norm& n) {
+  if (!bf16_arg(x) || symbolic(tensor(x)) || tensor(x).dim() != 3) return false;
+  n.o = operand(tensor(x));
+  return n.o.ok && is_gamma(gamma, n.o.cols) && fits_int(n.o.rows) && n.o.cols % 8 == 0;
+}
+// what a chain saved is dropped as the engine does it op by op: the tensor object loses its memory
+void release(std::initializer_list<PyObject*> items) {
+  for (PyObject* o : items)
+    if (!absent(o)) tensor(o).set_data(at::empty({0}, tensor(o).options()));
+}
+
+// release(list of tensors): the same from Python
+PyObject* py_release(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    if (n_args != 1 || !PyList_Check(a[0])) return none();
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(a[0]); ++i)
+      if (is_tensor(PyList_GET_ITEM(a[0], i))) release({PyList_GET_ITEM(a[0], i)});
+    return none();
+  });
+}
+
+// attn_chain_fwd(x, gamma, eps, w_qkv, gamma_q, gamma_k, qk_eps, freqs, ng, per, hd, scale, beside other streams, split_qkv, w_proj, split_proj,
+// residual, out, max_cus) -> (y, x rows, rstd, normed, q, k, v, o, lse, o rows, mixed, qk rstd); the last two are None without
+// the per-head norms.  y [s, b, h] has the residual added where one is given, and is None where ``out`` takes it.
+PyObject* py_attn_chain_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    if (n_args != 19) return none();
+    Norm n;
+    if (!norm_input(a[0], a[1], n) || !f32_arg(a[7])) return none();
+    const Tensor &x = tensor(a[0]), &freqs = tensor(a[7]);
+    const float eps = (float)real(a[2]);
+    const int64_t s = x.size(0), b = x.size(1), t = n.o.rows, h = n.o.cols;
+    const int64_t ng = integer(a[8]), per = integer(a[9]), hd = integer(a[10]);
+    const float scale = (float)real(a[11]);
+    const int flags = truth(a[12]) ? KR_ATTN_BESIDE_OTHER_STREAMS : 0;
+    const int split_qkv = (int)integer(a[13]), split_proj = (int)integer(a[15]), max_cus = (int)integer(a[18]);
+    if (ng <= 0 || per <= 0 || hd <= 0) return none();
+    const int64_t w = ng * (per + 2) * hd, wo = ng * per * hd;
+    if (!is_weight(a[3], w, h) || w % 8 || !is_rotary_table(freqs, s, hd) || !fits_int(s) || !fits_int(b) || !fits_int(w))
+      return none();
+    const bool qk = !absent(a[4]);
+    float qk_eps = 0.f;
+    if (qk) {
+      if (!is_gamma(a[4], hd) || !is_gamma(a[5], hd)) return none();
+      qk_eps = (float)real(a[6]);
+    }
+    if (!bf16_arg(a[14]) || symbolic(tensor(a[14])) || tensor(a[14]).dim() != 2) return none();
+    const int64_t out_cols = tensor(a[14]).size(0);
+    Epilogue e;
+    Output y = output(a[17], t, out_cols);
+    if (!is_weight(a[14], out_cols, wo) || !fits_int(out_cols) || wo % 8 || !y.ok || !residual(a[16], t, out_cols, e)) return none();
+    const Tensor &gamma = tensor(a[1]), &wq = tensor(a[3]), &wp = tensor(a[14]);
+    const Operand o_wq = operand2(wq), o_wp = operand2(wp);
+    Tensor mixed, fused, qk_rstd, q, k, v, o, lse, o2d;
+    int rc;
+    const char* what = "kr_rmsnorm_fwd";
+    {
+      WithoutInterpreter free;
+      rc = run_norm(x, gamma, eps, n);
+      if (rc == KR_OK) {
+        what = "kr_gemm_bf16";
+        mixed = matrix(t, w, x);
+        rc = run_gemm(KR_GEMM_TN, t, w, h, n.y, dense(t, h), wq, o_wq, mixed, dense(t, w), false, split_qkv, Epilogue{}, max_cus);
+        mixed = mixed.view({s, b, w});
+        fused = mixed.view({s, b, ng, per + 2, hd});
+      }
+      if (rc == KR_OK && qk) {
+        what = "kr_qk_norm_fwd";
+        fused = at::empty({s, b, ng, per + 2, hd}, x.options());
+        qk_rstd = at::empty({t, 1, ng, per + 1}, x.options().dtype(at::kFloat));
+        rc = kr_qk_norm_fwd(ptr(mixed), ptr(tensor(a[4])), ptr(tensor(a[5])), ptr(fused), (float*)ptr(qk_rstd), t, (int)ng,
+                            (int)per, (int)hd, qk_eps, stream());
+      }
+      if (rc == KR_OK) {
+        what = "kr_rope";
+        rc = run_rope(fused, freqs, false);
+      }
+      if (rc == KR_OK) {
+        what = "kr_attn_fwd";
+        q = fused.narrow(3, 0, per), k = fused.select(3, per), v = fused.select(3, per + 1);
+        rc = run_attn_fwd(attn_shape(q, k, v), q, k, v, scale, flags, o, lse);
+      }
+      if (rc == KR_OK) {
+        what = "kr_gemm_bf16";
+        o2d = o.view({t, wo});
+        if (absent(a[17])) y.t = matrix(t, out_cols, x);
+        rc = run_gemm(KR_GEMM_TN, t, out_cols, wo, o2d, dense(t, wo), wp, o_wp, y.t, y.o, false, split_proj, e, max_cus);
+        if (absent(a[17])) y.t = y.t.view({s, b, out_cols});
+      }
+    }
+    if (rc != KR_OK) return failed(what, rc);
+    if (!qk) mixed = Tensor();
+    if (!absent(a[17])) y.t = Tensor();
+    return pack({&y.t, &n.rows, &n.rstd, &n.y, &q, &k, &v, &o, &lse, &o2d, &mixed, &qk_rstd});
+  });
+}
+
+// mlp_chain_fwd(x, gamma, eps, w1, split1, fuse_activation, w2, split2, residual, out, max_cus) -> (y, x rows, rstd, normed,
+// fc1's output, the activation); y as above
+PyObject* py_mlp_chain_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    if (n_args != 11) return none();
+    Norm n;
+    if (!norm_input(a[0], a[1], n)) return none();
+    const Tensor& x = tensor(a[0]);
+    const float eps = (float)real(a[2]);
+    const int split1 = (int)integer(a[4]), split2 = (int)integer(a[7]), max_cus = (int)integer(a[10]);
+    const bool fuse = truth(a[5]);
+    const int64_t s = x.size(0), b = x.size(1), t = n.o.rows, h = n.o.cols;
+    for (int i : {3, 6})
+      if (!bf16_arg(a[i]) || symbolic(tensor(a[i])) || tensor(a[i]).dim() != 2) return none();
+    const Tensor &w1 = tensor(a[3]), &w2 = tensor(a[6]), &gamma = tensor(a[1]);
+    const int64_t two_f = w1.size(0), f = two_f / 2, out_cols = w2.size(0);
+    Epilogue e;
+    Output y = output(a[9], t, out_cols);
+    if (!is_weight(a[3], two_f, h) || two_f % 16 || !fits_int(two_f) || !is_weight(a[6], out_cols, f) || !fits_int(out_cols) ||
+        !y.ok || !residual(a[8], t, out_cols, e))
+      return none();
+    const Operand o1 = operand2(w1), o2 = operand2(w2);
+    Tensor pre, act;
+    int rc;
+    const char* what = "kr_rmsnorm_fwd";
+    {
+      WithoutInterpreter free;
+      rc = run_norm(x, gamma, eps, n);
+      if (rc == KR_OK) {
+        what = "kr_gemm_bf16";
+        act = matrix(t, f, x);
+        pre = matrix(t, two_f, x);
+        Epilogue swiglu;
+        if (fuse) {
+          swiglu.kind = KR_GEMM_EPI_SWIGLU;
+          swiglu.out2 = ptr(act);
+          swiglu.ld_out2 = f;
+        }
+        rc = run_gemm(KR_GEMM_TN, t, two_f, h, n.y, dense(t, h), w1, o1, pre, dense(t, two_f), false, split1, swiglu, max_cus);
+      }
+      if (rc == KR_OK && !fuse) {
+        what = "kr_swiglu_fwd";
+        rc = kr_swiglu_fwd(ptr(pre), ptr(act), t, (int)f, stream());
+      }
+      if (rc == KR_OK) {
+        what = "kr_gemm_bf16";
+        if (absent(a[9])) y.t = matrix(t, out_cols, x);
+        rc = run_gemm(KR_GEMM_TN, t, out_cols, f, act, dense(t, f), w2, o2, y.t, y.o, false, split2, e, max_cus);
+        if (absent(a[9])) y.t = y.t.view({s, b, out_cols});
+      }
+    }
+    if (rc != KR_OK) return failed(what, rc);
+    if (!absent(a[9])) y.t = Tensor();
+    return pack({&y.t, &n.rows, &n.rstd, &n.y, &pre, &act});
+  });
+}
+
+// dy [.., cols] of a chain's last projection
+bool grad_input(PyObject* o, int64_t rows, int64_t cols, Operand& od) {
+  if (!bf16_arg(o) || symbolic(tensor(o))) return false;
+  od = operand3(tensor(o));
+  return od.ok && od.rows == rows && od.cols == cols;
+}
+bool is_saved(PyObject* o, int64_t rows, int64_t cols) {
+  return bf16_arg(o) && tensor(o).dim() == 2 && tensor(o).is_contiguous() && tensor(o).size(0) == rows && tensor(o).size(1) == cols;
+}
+
+// mlp_chain_bwd(dy, w2, fc1's output, activation, w1, normed, split2, split1, weight gradients, max_cus) -> (dx [rows, h], gradient
+// of fc1's output, dw2, dw1).  With ``weight gradients`` the saved tensors lose their memory once they are used; without, the
+// caller takes the two weight gradients and the last two results are None.
+PyObject* py_mlp_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    if (n_args != 10) return none();
+    for (int i : {1, 4})
+      if (!bf16_arg(a[i]) || tensor(a[i]).dim() != 2) return none();
+    const Tensor &w2 = tensor(a[1]), &w1 = tensor(a[4]);
+    const int64_t cols = w2.size(0), f = w2.size(1), h = w1.size(1);
+    if (!bf16_arg(a[3]) || tensor(a[3]).dim() != 2) return none();
+    const int64_t t = tensor(a[3]).size(0);
+    Operand od;
+    if (!fits_int(t) || !fits_int(cols) || f % 8 || h % 8 || cols % 8 || !is_weight(a[1], cols, f) || !is_weight(a[4], 2 * f, h) ||
+        !is_saved(a[2], t, 2 * f) || !is_saved(a[3], t, f) || !is_saved(a[5], t, h) || !grad_input(a[0], t, cols, od))
+      return none();
+    const int split2 = (int)integer(a[6]), split1 = (int)integer(a[7]), max_cus = (int)integer(a[9]);
+    const bool wgrad = truth(a[8]);
+    const Tensor &dy = tensor(a[0]), &pre = tensor(a[2]), &act = tensor(a[3]), &normed = tensor(a[5]);
+    const Operand o1 = operand2(w1), o2 = operand2(w2);
+    Tensor dpre, dx, dw2, dw1;
+    int rc;
+    {
+      WithoutInterpreter free;
+      dpre = matrix(t, 2 * f, dy);
+      Epilogue e;
+      e.kind = KR_GEMM_EPI_SWIGLU_BWD;
+      e.ox.ld = 2 * f;
+      e.aux = ptr(pre);
+      rc = run_gemm(KR_GEMM_NN, t, f, cols, dy, od, w2, o2, dpre, dense(t, 2 * f), false, split2, e, max_cus);
+      if (rc == KR_OK && wgrad) {
+        dw2 = matrix(cols, f, dy);
+        rc = run_gemm(KR_GEMM_NT, cols, f, t, dy, od, act, dense(t, f), dw2, dense(cols, f), false, split2, Epilogue{}, max_cus);
+      }
+    }
+    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, f, cols, KR_GEMM_EPI_SWIGLU_BWD, rc);
+    if (wgrad) release({a[2], a[3]});
+    {
+      WithoutInterpreter free;
+      dx = matrix(t, h, dy);
+      rc = run_gemm(KR_GEMM_NN, t, h, 2 * f, dpre, dense(t, 2 * f), w1, o1, dx, dense(t, h), false, split1, Epilogue{}, max_cus);
+      if (rc == KR_OK && wgrad) {
+        dw1 = matrix(2 * f, h, dy);
+        rc = run_gemm(KR_GEMM_NT, 2 * f, h, t, dpre, dense(t, 2 * f), normed, dense(t, h), dw1, dense(2 * f, h), false, split1,
+                      Epilogue{}, max_cus);
+      }
+    }
+    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, h, 2 * f, KR_GEMM_EPI_NONE, rc);
+    if (wgrad) release({a[5]});
+    return pack({&dx, &dpre, &dw2, &dw1});
+  });
+}
+
+// attn_chain_bwd(dy, w_proj, q, k, v, o, lse, o rows, freqs, scale, beside other streams, mixed, qk rstd, gamma_q, gamma_k, w_qkv, normed,
+// split_proj, split_qkv, weight gradients, max_cus) -> (dx [rows, h], gradient of the QKV projection's output [rows, w], dw_proj,
+// dw_qkv, dgamma_q, dgamma_k).  Saved tensors and weight gradients as in mlp_chain_bwd.
+PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    if (n_args != 21) return none();
+    for (int i : {2, 3, 4, 5})
+      if (!bf16_arg(a[i])) return none();
+    if (!f32_arg(a[6]) || !f32_arg(a[8])) return none();
+    for (int i : {1, 15})
+      if (!bf16_arg(a[i]) || tensor(a[i]).dim() != 2) return none();
+    const Tensor &q = tensor(a[2]), &k = tensor(a[3]), &v = tensor(a[4]), &o = tensor(a[5]), &lse = tensor(a[6]),
+                 &freqs = tensor(a[8]), &wp = tensor(a[1]), &wq = tensor(a[15]);
+    const AttnShape c = attn_shape(q, k, v);
+    if (!c.ok || q.dim() != 5) return none();
+    const int64_t t = (int64_t)c.s * c.b, wo = (int64_t)c.nq * c.hd, w = (int64_t)c.nkv * (c.per + 2) * c.hd, cols = wp.size(0),
+                  h = wq.size(1);
+    Operand od;
+    if (!fits_int(t) || !fits_int(cols) || wo % 8 || w % 8 || h % 8 || cols % 8 || !is_weight(a[1], cols, wo) ||
+        !is_weight(a[15], w, h) || !is_saved(a[7], t, wo) || !is_saved(a[16], t, h) || !is_rotary_table(freqs, c.s, c.hd) ||
+        !grad_input(a[0], t, cols, od))
+      return none();
+    const bool qk = !absent(a[13]);
+    if (qk) {
+      if (!bf16_arg(a[11]) || !f32_arg(a[12]) || !is_gamma(a[13], c.hd) || !is_gamma(a[14], c.hd)) return none();
+      const Tensor &m = tensor(a[11]), &r = tensor(a[12]);
+      if (!m.is_contiguous() || m.numel() != t * w || !r.is_contiguous() || r.numel() != t * c.nkv * (c.per + 1)) return none();
+    }
+    const float scale = (float)real(a[9]);
+    const int flags = truth(a[10]) ? KR_ATTN_BESIDE_OTHER_STREAMS : 0;
+    const int split_proj = (int)integer(a[17]), split_qkv = (int)integer(a[18]), max_cus = (int)integer(a[20]);
+    const bool wgrad = truth(a[19]);
+    const Tensor &dy = tensor(a[0]), &o2d = tensor(a[7]), &normed = tensor(a[16]);
+    const Operand o_wp = operand2(wp), o_wq = operand2(wq);
+    Tensor dout, dwp, dwq, dx, dgq, dgk, dmixed;
+    AttnGrads g;
+    int rc;
+    {
+      WithoutInterpreter free;
+      dout = matrix(t, wo, dy);
+      rc = run_gemm(KR_GEMM_NN, t, wo, cols, dy, od, wp, o_wp, dout, dense(t, wo), false, split_proj, Epilogue{}, max_cus);
+      if (rc == KR_OK && wgrad) {
+        dwp = matrix(cols, wo, dy);
+        rc = run_gemm(KR_GEMM_NT, cols, wo, t, dy, od, o2d, dense(t, wo), dwp, dense(cols, wo), false, split_proj, Epilogue{},
+                      max_cus);
+      }
+    }
+    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, wo, cols, KR_GEMM_EPI_NONE, rc);
+    if (!attn_bwd_ok(c, dout, q, o, lse)) return failed(attn_name("kr_attn_bwd", c), KR_EINVAL);
+    if (wgrad) release({a[7]});
+    const char* what = "kr_attn_bwd";
+    {
+      WithoutInterpreter free;
+      rc = run_attn_bwd(c, dout, q, k, v, o, lse, scale, flags, g);
+      dout = Tensor();
+      if (rc == KR_OK) {
+        what = "kr_rope";
+        rc = run_rope(g.fused, freqs, true);
+      }
+    }
+    if (rc != KR_OK) return failed(what, rc);
+    if (wgrad) release({a[2], a[3], a[4], a[5], a[6]});
+    {
+      WithoutInterpreter free;
+      if (qk) {
+        const Tensor &gq = tensor(a[13]), &gk = tensor(a[14]);
+        dgq = at::empty({c.hd}, gq.options());
+        dgk = at::empty({c.hd}, gk.options());
+        const size_t n = kr_qk_norm_bwd_workspace_bytes(t, c.nkv, (int)c.per, c.hd);
+        const Tensor ws = bytes(n < 16 ? 16 : n, g.fused);
+        rc = kr_qk_norm_bwd(ptr(g.fused), ptr(tensor(a[11])), (const float*)ptr(tensor(a[12])), ptr(gq), ptr(gk), ptr(dgq), ptr(dgk),
+                            ptr(ws), t, c.nkv, (int)c.per, c.hd, stream());
+      }
+    }
+    if (rc != KR_OK) return failed("kr_qk_norm_bwd", rc);
+    if (wgrad && qk) release({a[11], a[12]});
+    {
+      WithoutInterpreter free;
+      dmixed = g.mixed.view({t, w});
+      dx = matrix(t, h, dmixed);
+      rc = run_gemm(KR_GEMM_NN, t, h, w, dmixed, dense(t, w), wq, o_wq, dx, dense(t, h), false, split_qkv, Epilogue{}, max_cus);
+      if (rc == KR_OK && wgrad) {
+        dwq = matrix(w, h, dmixed);
+        rc = run_gemm(KR_GEMM_NT, w, h, t, dmixed, dense(t, w), normed, dense(t, h), dwq, dense(w, h), false, split_qkv, Epilogue{},
+                      max_cus);
+      }
+    }
+    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, h, w, KR_GEMM_EPI_NONE, rc);
+    if (wgrad) release({a[16]});
+    return pack({&dx, &dmixed, &dwp, &dwq, &dgq, &dgk});
+  });
+}
+
+// rmsnorm_dgamma(partials [n, cols] fp32, gamma) -> the weight gradient
+PyObject* py_rmsnorm_dgamma(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  return guarded([&]() -> PyObject* {
+    if (n_args != 2 || !f32_arg(a[0]) || tensor(a[0]).dim() != 2 || !tensor(a[0]).is_contiguous() ||
+        !is_gamma(a[1], tensor(a[0]).size(1)) || !fits_int(tensor(a[0]).size(0)) || !fits_int(tensor(a[0]).size(1)))
+      return none();
+    const Tensor &p = tensor(a[0]), &gamma = tensor(a[1]);
+    Tensor dgamma;
+    int rc;
+    {
+      WithoutInterpreter free;
+      dgamma = at::empty({p.size(1)}, gamma.options());
+      rc = kr_rmsnorm_dgamma((const float*)ptr(p), (int)p.size(0), (int)p.size(1), ptr(dgamma), stream());
+    }
+    if (rc != KR_OK) return failed("kr_rmsnorm_dgamma", rc);
+    return wrap(std::move(dgamma));
+  });
+}
+
 PyMethodDef kMethods[] = {
     {"rows_view", (PyCFunction)(void*)py_rows_view, METH_FASTCALL, nullptr},
     {"gemm", (PyCFunction)(void*)py_gemm, METH_FASTCALL, nullptr},
+    {"wgrad_segments_ok", (PyCFunction)(void*)py_wgrad_segments_ok, METH_FASTCALL, nullptr},
     {"wgrad_segments", (PyCFunction)(void*)py_wgrad_segments, METH_FASTCALL, nullptr},
     {"rmsnorm_fwd", (PyCFunction)(void*)py_rmsnorm_fwd, METH_FASTCALL, nullptr},
     {"rmsnorm_bwd", (PyCFunction)(void*)py_rmsnorm_bwd, METH_FASTCALL, nullptr},
@@ -646,6 +1109,12 @@ PyMethodDef kMethods[] = {
     {"attn_bwd", (PyCFunction)(void*)py_attn_bwd, METH_FASTCALL, nullptr},
     {"dropout_add", (PyCFunction)(void*)py_dropout_add, METH_FASTCALL, nullptr},
     {"dropout_bwd", (PyCFunction)(void*)py_dropout_bwd, METH_FASTCALL, nullptr},
+    {"release", (PyCFunction)(void*)py_release, METH_FASTCALL, nullptr},
+    {"attn_chain_fwd", (PyCFunction)(void*)py_attn_chain_fwd, METH_FASTCALL, nullptr},
+    {"mlp_chain_fwd", (PyCFunction)(void*)py_mlp_chain_fwd, METH_FASTCALL, nullptr},
+    {"mlp_chain_bwd", (PyCFunction)(void*)py_mlp_chain_bwd, METH_FASTCALL, nullptr},
+    {"attn_chain_bwd", (PyCFunction)(void*)py_attn_chain_bwd, METH_FASTCALL, nullptr},
+    {"rmsnorm_dgamma", (PyCFunction)(void*)py_rmsnorm_dgamma, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

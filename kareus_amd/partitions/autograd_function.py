@@ -71,6 +71,15 @@ def _nanobatches_in_line(config, hs: Sequence[Tensor]) -> bool:
     return len(hs) > 1 and rule is not None and rule(hs[0].shape[0], hs[0].shape[1])
 
 
+def _chains(config) -> bool:
+    """Whether operator sequences may run as one native call in this pass."""
+    if getattr(config, "backend", None) != "hip":
+        return False
+    from ..operators.chains import chains_allowed
+
+    return chains_allowed()
+
+
 def _scheduled(partitions) -> bool:
     """Whether a plan's item was loaded into any of the partitions (by a scheduler of this pass or an earlier one, or by
     hand): it is about the nanobatches' streams, so such a pass uses them."""
@@ -193,7 +202,8 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
 
         in_line = _nanobatches_in_line(config, hs) and not _scheduled(fwd_parts) and not _scheduled(bwd_parts)
         streams = [None] * n if in_line else _nanobatch_streams(config, n)
-        ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=in_line) for i in range(n)]
+        chains = _chains(config)
+        ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=in_line, chains=chains) for i in range(n)]
         _seed_forward(ctxs, hs, rotary, mask, seed)
 
         # The nanobatch outputs are written side by side into one [s, b, h] tensor, so the
@@ -225,6 +235,7 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
         func_ctx.n = n
         func_ctx.streams = streams
         func_ctx.in_line = in_line
+        func_ctx.config = config
         func_ctx.backward_partitions = bwd_parts
         func_ctx.backward_tensor_graph = bwd_graph
         func_ctx.scheduler = scheduler
@@ -270,10 +281,11 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
         scheduler = func_ctx.scheduler
         schedule = scheduler.current_schedule if scheduler is not None else None
 
+        chains = _chains(func_ctx.config)
         _fork(streams)
         if func_ctx.checkpoint_activations:
             hs = func_ctx.saved_tensors
-            ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=func_ctx.in_line) for i in range(n)]
+            ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=func_ctx.in_line, chains=chains) for i in range(n)]
             _seed_forward(ctxs, hs, rotary, mask, seed)
             # with the generators as they were before the forward pass, and put back afterwards
             # (kareus/megatron/core/partitions/autograd_function.py:263-266)
@@ -294,6 +306,7 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
                 lo += cnt
 
         for c, g in zip(ctxs, grad_outs):
+            c.chains = chains
             c.tensor_store = TensorStore()
             c.tensor_store.set(seed.bwd_grad_tid, g)
 
@@ -309,11 +322,14 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
                 at_end = n >= 4
             # ("pending": where such launches are left to be issued behind the last partition of the pass)
             pending = [] if (at_end and func_ctx.wgrad_over_all_nanobatches and not func_ctx.in_line) else None
+            new = {"n": n, "turn": turn, "defer": func_ctx.wgrad_over_all_nanobatches, "pending": pending,
+                   "in_line": func_ctx.in_line}
             for c in ctxs:
                 for op_id, op_ctx in c.op_contexts.items():
-                    op_ctx.wgrad_sink = sinks.setdefault(
-                        op_id, {"n": n, "turn": turn, "defer": func_ctx.wgrad_over_all_nanobatches,
-                                "pending": pending, "in_line": func_ctx.in_line})
+                    sink = sinks.get(op_id)
+                    if sink is None:
+                        sink = sinks[op_id] = new.copy()
+                    op_ctx.wgrad_sink = sink
                     op_ctx.nanobatch_index = c.batch_idx
 
         if func_ctx.join_in_place:

@@ -25,6 +25,11 @@ class BackwardPartition(PartitionBase):
     # as one call; the numbers are those of the separate calls
     fuse_backward_ops: bool = True
 
+    def _chain_at(self, plans, at: int):
+        from ..operators.chains import backward_chain
+
+        return backward_chain(plans, at)
+
     def execute(
         self,
         ctx: NanoBatchContext,
@@ -60,6 +65,8 @@ class BackwardPartition(PartitionBase):
         grad_params: Dict[int, List] = {}
 
         plans = self._plans()
+        chains = self._op_chains if ctx.chains and not timed and self.fuse_backward_ops and not self.profiling_mode else None
+        identity = self.comm_op is not None and len(self.comm_op.output_ports) == 1 and self._is_identity(pre_ctx)
         idx, num_ops = 0, len(plans)
         while idx < num_ops:
             op = plans[idx]
@@ -68,6 +75,18 @@ class BackwardPartition(PartitionBase):
                 break
 
             dy = get(op.first_in)
+            if start == idx and not identity:
+                comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size, backward=True)
+                launched = True
+            chain = chains[idx] if chains is not None else None
+            if chain is not None and not idx < start < idx + chain.length:
+                got = chain.run(ctx, store, dy, protected)
+                if got is not None:
+                    grad_params.update(got)
+                    idx += chain.length
+                    if idx == start and not identity and not self._in_order(ctx):
+                        self.comm_op.event_record(self._here())
+                    continue
             group, group_ctxs = [op], [op_ctx]
             grad_extra_out = [tuple([get(t) for t in op.extra_ids])] if op.extra_ids else []
             follower = self._fusable_follower(plans, idx, start, ctx)
@@ -76,10 +95,6 @@ class BackwardPartition(PartitionBase):
                 group_ctxs.append(ctx.get_op_context(follower.op_id))
                 grad_extra_out = [tuple([get(t) for t in op.extra_ids]), tuple([get(t) for t in follower.extra_ids])]
             last = idx + len(group) - 1
-
-            if start == idx:
-                comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size, backward=True)
-                launched = True
 
             dx, op_param_grads, grad_extra_in = op.operator.fuser_backward(
                 group_ctxs, dy, basic_op_grad_extra_outputs=grad_extra_out
@@ -96,7 +111,7 @@ class BackwardPartition(PartitionBase):
                     member_ctx.saved_tensors = None
                 if timed:
                     self._op_done(idx + k)
-            if last == start - 1 and not self._in_order(ctx):
+            if last == start - 1 and not identity and not self._in_order(ctx):
                 self.comm_op.event_record(self._here())
 
             put(group[-1].first_out, dx)
@@ -110,7 +125,9 @@ class BackwardPartition(PartitionBase):
                         put(tid, g)
             idx = last + 1
 
-        if self.comm_op is not None:
+        if identity:
+            self._hand_on(pre_ctx, sm_num, block_size)
+        elif self.comm_op is not None:
             if not launched:  # no slot given, or the op loop stopped before reaching it
                 comm_out, comm_extra = self._launch_comm_no_overlap(
                     pre_ctx, sm_num, block_size, backward=True

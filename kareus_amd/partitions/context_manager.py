@@ -78,6 +78,8 @@ class NanoBatchContext:
     # the nanobatches of this pass run one after the other on the caller's stream, in the order the
     # partitions are issued: every edge a schedule point would add is already there
     in_line: bool = False
+    # operator sequences may run as one native call in this pass (operators/chains.py)
+    chains: bool = False
     # op_id -> tensor that op's forward output is to be written into (consumed when the op runs)
     output_sinks: Dict[int, torch.Tensor] = field(default_factory=dict)
     _saved_tensors: List[Optional[torch.Tensor]] = field(default_factory=list)

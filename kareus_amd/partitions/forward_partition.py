@@ -23,6 +23,11 @@ class ForwardPartition(PartitionBase):
     # call; the numbers are those of the separate calls
     fuse_forward_ops: bool = True
 
+    def _chain_at(self, plans, at: int):
+        from ..operators.chains import forward_chain
+
+        return forward_chain(plans, at)
+
     def execute(self, ctx: NanoBatchContext, pre_ctx: NanoBatchContext) -> None:
         with self._on_stream(ctx), self._timed():
             self._execute(ctx, pre_ctx)
@@ -36,10 +41,22 @@ class ForwardPartition(PartitionBase):
         comm_out, comm_extra = None, []
 
         plans = self._plans()
+        chains = self._op_chains if ctx.chains and not timed and self.fuse_forward_ops else None
+        identity = self.comm_op is not None and len(self.comm_op.output_ports) == 1 and self._is_identity(pre_ctx)
+        grad = self.is_grad_enabled
         idx, num_ops = 0, len(plans)
         while idx < num_ops:
             plan = plans[idx]
             x = get(plan.first_in)
+            if start == idx and not identity:
+                comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size)
+            chain = chains[idx] if chains is not None else None
+            if (chain is not None and not idx < start < idx + chain.length and (not grad or needs(plan.first_in))
+                    and chain.run(ctx, store, x, grad)):
+                idx += chain.length
+                if idx == start and not identity and not self._in_order(ctx):
+                    self.comm_op.event_record(self._here())
+                continue
             extras = [tuple([get(t) for t in plan.extra_ids])] if plan.extra_ids else []
             # the op behind this one runs in the same call when the two offer a fused forward and the
             # scheduled launch point does not fall between them
@@ -64,9 +81,6 @@ class ForwardPartition(PartitionBase):
             k = len(group)
             last = idx + k - 1
 
-            if start == idx:
-                comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size)
-
             x, extra_out = plan.operator.fuser_forward(
                 group_ctxs,
                 x,
@@ -79,7 +93,7 @@ class ForwardPartition(PartitionBase):
             if timed:
                 for j in range(k):
                     self._op_done(idx + j)
-            if last == start - 1 and not self._in_order(ctx):
+            if last == start - 1 and not identity and not self._in_order(ctx):
                 self.comm_op.event_record(self._here())
 
             tail = group[-1]
@@ -90,7 +104,9 @@ class ForwardPartition(PartitionBase):
                         put(tid, extra, needs_grad)
             idx = last + 1
 
-        if self.comm_op is not None:
+        if identity:
+            self._hand_on(pre_ctx, sm_num, block_size)
+        elif self.comm_op is not None:
             if start == -1:
                 comm_out, comm_extra = self._launch_comm_no_overlap(pre_ctx, sm_num, block_size)
             self._sync_comm(pre_ctx, comm_out, comm_extra)

@@ -151,7 +151,12 @@ class PartitionBase:
         if plans is None or len(plans) != len(ops) or any(
                 [p.op is not op or p.operator is not op.operator for p, op in zip(plans, ops)]):
             plans = self._op_plans = [_OpPlan(op, ops[i + 1] if i + 1 < len(ops) else None) for i, op in enumerate(ops)]
+            # the operator sequences that can run as one native call, by the index they start at (operators/chains.py)
+            self._op_chains = [self._chain_at(plans, i) for i in range(len(plans))]
         return plans
+
+    def _chain_at(self, plans: List[_OpPlan], at: int):
+        return None
 
     def _here(self):
         """The stream the schedule point is told about; None for a slot without a stream of its own (one
@@ -222,6 +227,12 @@ class PartitionBase:
             basic_op_kwargs=[kwargs],
         )
 
+    def _is_identity(self, pre_ctx) -> bool:
+        """Whether the schedule point is nothing but its bookkeeping: the order of one stream gives every edge (or there is
+        no second stream), and the operator is the stock identity."""
+        op = self.comm_op.operator
+        return (pre_ctx.in_line or getattr(op, "comm_stream", self) is None) and getattr(op, "hands_on", None) is not None and op.is_stock()
+
     def _launch_comm(self, pre_ctx, sm_num, block_size, *, backward: bool = False):
         """Release point reached earlier (event already recorded): wait on it, run."""
         if not self._in_order(pre_ctx):
@@ -234,6 +245,14 @@ class PartitionBase:
             self.comm_op.event_record(self._here())
             self.comm_op.event_wait()
         return self._run_comm(pre_ctx, sm_num, block_size, backward)
+
+    def _hand_on(self, pre_ctx: NanoBatchContext, sm_num, block_size) -> None:
+        """The whole schedule point of ``_is_identity``: release, collective and sync in one."""
+        self.comm_op.operator.hands_on(sm_num, block_size)
+        src, dst = self.comm_op.input_ports, self.comm_op.output_ports
+        store = pre_ctx.tensor_store
+        tid = src[0].tensor_id
+        store.set(dst[0].tensor_id, store.get(tid), store.needs_grad(tid))
 
     def _sync_comm(self, pre_ctx: NanoBatchContext, comm_output, comm_extra_outputs) -> None:
         if not self._in_order(pre_ctx):

@@ -1,0 +1,210 @@
+"""Operator sequences that run as one native call (operators/chains.py): found where the graph has them, bit for bit the
+operators one by one, and left alone whenever something looks between the operators or replaced one."""
+
+import gc
+import weakref
+
+import pytest
+import torch
+
+from kareus_amd import LayerConfig, LayerStack
+from kareus_amd.operators import PartitionableRMSNorm, ResidualForkOp, chains
+from kareus_amd.partitions import autograd_function
+from kareus_amd.partitions.partition_base import PartitionBase
+
+
+def config(nnb=1, **kw):
+    base = dict(hidden_size=256, num_attention_heads=4, num_query_groups=2, kv_channels=64, ffn_hidden_size=320, num_layers=2,
+                num_nanobatches=nnb, backend="hip")
+    return LayerConfig(**{**base, **kw})
+
+
+# ---- which sequences are found -------------------------------------------------------------------------------
+@pytest.mark.parametrize("fuse", [True, False])
+def test_every_segment_of_a_layer_is_a_chain(fuse):
+    model = LayerStack(config(fuse_forward_epilogues=fuse), device="cpu")
+    found = []
+    for part in model.forward_partitions + model.backward_partitions:
+        plans = part._plans()
+        for i, chain in enumerate(part._op_chains):
+            if isinstance(chain, (chains._ForwardChain, chains._BackwardChain)):
+                assert [p.op_id for p in chain.plans] == [p.op_id for p in plans[i:i + chain.length]]
+                found.append(type(chain).__name__)
+    assert [found.count(n) for n in ("_ForwardAttention", "_ForwardMlp", "_BackwardMlp", "_BackwardAttention")] == [2, 2, 2, 2]
+
+
+def test_a_model_is_freed_without_the_garbage_collector():
+    """(A chain holds plans, and nothing of a plan or an operator holds the chain.)"""
+    gc.collect()
+    gc.disable()
+    try:
+        model = LayerStack(config(), device="cpu")
+        for part in model.forward_partitions + model.backward_partitions:
+            part._plans()
+        weight = weakref.ref(model.layers[0].linear_qkv)
+        del model, part
+        assert weight() is None
+    finally:
+        gc.enable()
+
+
+def test_a_subclass_or_another_order_is_no_chain():
+    class Mine(PartitionableRMSNorm):
+        pass
+
+    model = LayerStack(config(), device="cpu")
+    part = model.forward_partitions[0]
+    part.comp_ops[1].operator = Mine(256, backend="hip")
+    part._plans()
+    assert not any(isinstance(c, chains._ForwardChain) for c in part._op_chains)
+
+
+def test_replaced_methods_are_noticed(monkeypatch):
+    model = LayerStack(config(), device="cpu")
+    ops = [p.operator for p in model.forward_partitions[0]._plans()]
+    assert chains._untouched(ops)
+    ops[2].fuser_forward = lambda *a, **k: None
+    assert not chains._untouched(ops)
+    del ops[2].fuser_forward
+    ops[0]._backend_name = "eager"
+    assert not chains._untouched(ops)
+    assert chains.chains_allowed()
+    monkeypatch.setattr(ResidualForkOp, "fuser_forward", lambda *a, **k: None)
+    assert not chains.chains_allowed()
+
+
+def test_a_replaced_backend_method_is_noticed(monkeypatch):
+    from kareus_amd.backend import get_backend
+
+    be = get_backend("hip")
+    assert chains.chains_allowed()
+    with monkeypatch.context() as m:
+        m.setattr(type(be), "MAX_RUN_ROWS", 1)
+        assert not chains.chains_allowed()
+    with monkeypatch.context() as m:
+        m.setitem(be.__dict__, "attn_fwd", lambda *a, **k: None)
+        assert not chains.chains_allowed()
+    with monkeypatch.context() as m:
+        m.setattr(be, "_n", object())
+        assert not chains.chains_allowed()
+    assert chains.chains_allowed()
+
+
+# ---- the same bits ---------------------------------------------------------------------------------------------------
+def run(cfg, s, b, *, seed=0, grad=True, before=None, hooks=None):
+    torch.manual_seed(seed)
+    model = LayerStack(cfg, device="cuda", seed=3)
+    if before is not None:
+        before(model)
+    x = torch.randn(s, b, cfg.hidden_size, generator=torch.Generator().manual_seed(1)).to("cuda", torch.bfloat16)
+    go = torch.randn(s, b, cfg.hidden_size, generator=torch.Generator().manual_seed(2)).to("cuda", torch.bfloat16)
+    if not grad:
+        with torch.no_grad():
+            return [model(x)]
+    x.requires_grad_(True)
+    out = []
+    for _ in range(2):   # (the second pass on gradients and plans that are there)
+        with (hooks() if hooks is not None else torch.enable_grad()):
+            y = model(x)
+        y.backward(go)
+        out.append(y.detach())
+    torch.cuda.synchronize()
+    return out + [x.grad] + [p.grad for p in model.parameters()]
+
+
+def both(monkeypatch, *args, **kw):
+    """The pass with chains, which have to have run (``ran``: how many of each), and the pass without."""
+    ran = {}
+    with monkeypatch.context() as m:
+        for cls in (chains._ForwardAttention, chains._ForwardMlp, chains._BackwardMlp, chains._BackwardAttention):
+            def watched(self, *a, _run=cls.run, _name=cls.__name__):
+                got = _run(self, *a)
+                ran[_name] = ran.get(_name, 0) + (got is not None and got is not False)
+                return got
+            m.setattr(cls, "run", watched)
+        got = run(*args, **kw)
+    with monkeypatch.context() as m:
+        m.setattr(autograd_function, "_chains", lambda config: False)
+        want = run(*args, **kw)
+    assert len(got) == len(want)
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+    return ran
+
+
+CASES = {
+    "one nanobatch": (config(), 128, 2),
+    "odd sizes": (config(), 104, 3),
+    "heads of 128, one group, one head": (config(num_attention_heads=1, num_query_groups=1, kv_channels=128), 72, 1),
+    "no epilogue fusion": (config(fuse_forward_epilogues=False), 96, 2),
+    "activation of its own": (config(ffn_hidden_size=344), 96, 2),          # no SwiGLU epilogue for this width
+    "per-head norms and dropout": (config(qk_layernorm=True, hidden_dropout=0.2), 96, 2),
+    "recomputation": (config(checkpoint_activations=True, hidden_dropout=0.1), 96, 2),
+    "nanobatches in line": (config(2), 96, 4),
+    "nanobatches in line, tokens no multiple of 64": (config(2, qk_layernorm=True), 104, 2),
+    "four nanobatches in line, recomputed": (config(4, checkpoint_activations=True), 64, 4),
+    "nanobatches on one stream": (config(2, use_streams=False), 96, 4),
+    "accumulated weight gradients": (config(2, wgrad_over_all_nanobatches=False), 96, 4),
+    "gradients summed by autograd": (config(2, fuse_wgrad_accumulation=False), 96, 4),
+    "nanobatches on streams": (config(2, in_line_below_ms=0.0), 96, 4),
+}
+
+
+@pytest.mark.parametrize("what", sorted(CASES))
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_chain_has_the_bits_of_its_operators(what, monkeypatch):
+    cfg, s, b = CASES[what]
+    ran = both(monkeypatch, cfg, s, b)
+    passes = 2 * cfg.num_layers * cfg.num_nanobatches
+    again = 2 if cfg.checkpoint_activations else 1
+    assert ran["_ForwardAttention"] == ran["_ForwardMlp"] == passes * again
+    whole = what not in ("no epilogue fusion", "nanobatches on streams", "nanobatches on one stream")
+    if whole:
+        assert ran["_BackwardAttention"] == ran["_BackwardMlp"] == passes
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_chains_without_gradients_and_under_saved_tensor_hooks(monkeypatch):
+    ran = both(monkeypatch, config(2), 96, 4, grad=False)
+    assert ran["_ForwardAttention"] == 4
+    both(monkeypatch, config(), 96, 2, hooks=lambda: torch.autograd.graph.save_on_cpu())
+    seen = []
+    both(monkeypatch, config(), 96, 2, hooks=lambda: torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t,
+                                                                                              lambda t: t))
+    half = len(seen) // 2
+    assert half and seen[:half] == seen[half:]     # the same tensors in the same order
+
+
+@pytest.mark.parametrize("part", ["linear_fc1", "linear_proj", "pre_mlp_layernorm"])
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_frozen_weight_gets_no_gradient(part, monkeypatch):
+    both(monkeypatch, config(), 96, 2, before=lambda model: getattr(model.layers[1], part).weight.requires_grad_(False))
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_an_operator_or_a_timer_between_the_operators_is_served(monkeypatch):
+    """A method replaced on one operator runs; a timer sees every operator."""
+    calls, model = [], LayerStack(config(), device="cuda", seed=3)
+    rope = model.layers[0].rotary
+    inner = rope.fuser_forward
+    rope.fuser_forward = lambda *a, **k: calls.append("rope") or inner(*a, **k)
+    x = torch.randn(96, 2, 256, device="cuda").bfloat16()
+    with torch.no_grad():
+        y = model(x)
+        assert calls == ["rope"]
+        del rope.fuser_forward
+        assert torch.equal(model(x), y) and calls == ["rope"]
+
+        class Timer:
+            def begin(self, part): calls.append("begin")
+            def end(self, part): calls.append("end")
+            def op_done(self, part, idx): calls.append(idx)
+        monkeypatch.setattr(PartitionBase, "timer", Timer())
+        calls.clear()
+        assert torch.equal(model(x), y)
+    assert [c for c in calls if not isinstance(c, str)] == list(range(7)) + list(range(6)) + list(range(8)) + list(range(6)) + [0]
+    assert calls.count("begin") == calls.count("end") == 5
