@@ -249,11 +249,11 @@ __device__ __forceinline__ int load_k(int i, int wave, int lane) {
 // v_mfma_f32_16x16x32_bf16 wants from lane l the 8 contraction elements 8 (l / 16) .. + 7 of
 // operand row l % 16.  Fragment (g, h): operand rows row0 + 16 g .., contraction half h (32
 // elements) of the K-step.
-template <bool TRANSPOSED, int WT>
+template <bool TRANSPOSED, int TW>
 struct FragReader {
   // K-major: one base per half (the swizzle XOR depends on the chunk), g is an immediate
   // transposed: one base per g (the XOR depends on the column), the half is an immediate
-  static constexpr int NBASE = TRANSPOSED ? WT : 2;
+  static constexpr int NBASE = TRANSPOSED ? TW / 32 : 2;
   uint32_t base[NBASE];  // byte offsets inside a tile
   __device__ __forceinline__ void init(int row0, int lane) {
     if (!TRANSPOSED) {
@@ -266,7 +266,7 @@ struct FragReader {
       const int p = lane & 15;
       const int krow = 8 * (lane >> 4) + (p >> 2);
 #pragma unroll
-      for (int g = 0; g < WT; ++g) base[g] = 2u * (uint32_t)transp_off<32 * WT>(krow, row0 + 16 * g + (p & 3) * 4);
+      for (int g = 0; g < TW / 32; ++g) base[g] = 2u * (uint32_t)transp_off<TW>(krow, row0 + 16 * g + (p & 3) * 4);
     }
   }
 };
@@ -332,7 +332,12 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   static_assert(!SEG || (A_T && B_T), "operand pieces: layout NT");
   static_assert(DEPTH == kDepth || (DEPTH == kDepthAlone && WT == WT_SMALL), "ring depths");
   static_assert(WT == WT_LARGE || (WT == WT_SMALL && WN == 4 && EPI != KR_GEMM_EPI_TRANSPOSED_OUT), "tile shapes");
-  constexpr int TW = 32 * WT;  // operand rows an LDS tile holds (a B tile may use fewer)
+  // operand rows an LDS tile of A / of B holds.  A K-major B tile may use fewer; a transposed one of 128 columns is laid out
+  // as such: spread over rows of 256, as those of 160 to 224 are, half of what it loads is never read, and a K-step of the
+  // 256 x 128 tile takes 64 KB through the unit's address path instead of 48.  us, before -> after: 3072 x 2048 x 8192 (NT) 128 ->
+  // 106, 1536 x 4096 x 6024 (NT) 99 -> 80, 512 x 2048 x 32768 (NT, cut) 98 -> 81, 6024 x 1024 x 4096 (NN) 67 -> 55, 16384 x 384 x
+  // 3072 (NN) 53 -> 48.
+  constexpr int TW = 32 * WT, TWB = WT == WT_SMALL || (B_T && WN == 4) ? 128 : 256;
   constexpr uint32_t SLOT_BYTES = kSlotBytes<WT>;
   // (without RUNS every run length reads as a compile-time 1: the branches below fold away)
   const RowRuns runs = RUNS ? runs_arg : RowRuns{0, 0, 0, 0, 0, 0};
@@ -340,9 +345,9 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int BN_ = 32 * WN;
-  // loads per wave of a B tile: a K-major tile's unused rows are simply not fetched; in a
-  // transposed tile every load spans all 256 columns
-  constexpr int NB_LOADS = B_T ? WT : WN;
+  // loads per wave of a B tile: a K-major tile's unused rows are simply not fetched; in a transposed tile every load
+  // spans all columns of a tile row
+  constexpr int NB_LOADS = B_T ? TWB / 32 : WN;
   constexpr int NA_LOADS = WT;
   constexpr int BM_ = 32 * WT;
   const int wm = wave >> 1, wn = wave & 1;  // wave tile: rows wm*16*WT.., columns wn*16*WN..
@@ -459,7 +464,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
 #pragma unroll
     for (int i = 0; i < WT; ++i) {
       la[i] = 2u * load_offset<A_T, TW>(i, wave, l2, lda, m0, M, k_left, 0, 0, runs.a_sh, runs.a_outer);
-      lb[i] = 2u * load_offset<B_T, TW>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN);
+      if (i < NB_LOADS) lb[i] = 2u * load_offset<B_T, TWB>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN);
     }
   };
   // the first `count` loads of a tile (NA_LOADS for A, NB_LOADS for B)
@@ -498,17 +503,17 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     for (int i = 0; i < WT; ++i) {
       const uint32_t blk = (uint32_t)(wave + 4 * i) * 1024u + (uint32_t)l2 * 16u;
       if (load_k<A_T, TW>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sa + blk) = zero8();
-      if (load_k<B_T, TW>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sb + blk) = zero8();
+      if (i < NB_LOADS && load_k<B_T, TWB>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sb + blk) = zero8();
     }
   };
 
   // fragment addressing, recomputed per item from an opaque copy of the lane id so that it is
   // not live through the epilogue
-  FragReader<A_T, WT> fa;
-  FragReader<B_T, WT> fb;
+  FragReader<A_T, TW> fa;
+  FragReader<B_T, TWB> fb;
   // addresses for reading half h of the tiles in slots sa / sb
-  auto frag_addrs = [&](uint32_t sa, uint32_t sb, int h, uint32_t (&aa)[FragReader<A_T, WT>::NBASE],
-                        uint32_t (&ba)[FragReader<B_T, WT>::NBASE]) {
+  auto frag_addrs = [&](uint32_t sa, uint32_t sb, int h, uint32_t (&aa)[FragReader<A_T, TW>::NBASE],
+                        uint32_t (&ba)[FragReader<B_T, TWB>::NBASE]) {
     if (!A_T) {
       aa[0] = sa + fa.base[h];
       asm volatile("" : "+v"(aa[0]));
@@ -530,11 +535,11 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       }
     }
   };
-  auto read_a = [&](const uint32_t (&aa)[FragReader<A_T, WT>::NBASE], int g, int h) {
+  auto read_a = [&](const uint32_t (&aa)[FragReader<A_T, TW>::NBASE], int g, int h) {
     if constexpr (!A_T) return frag_kmajor(aa[0], g); else return frag_transp<TW>(aa[g], h);
   };
-  auto read_b = [&](const uint32_t (&ba)[FragReader<B_T, WT>::NBASE], int g, int h) {
-    if constexpr (!B_T) return frag_kmajor(ba[0], g); else return frag_transp<TW>(ba[g], h);
+  auto read_b = [&](const uint32_t (&ba)[FragReader<B_T, TWB>::NBASE], int g, int h) {
+    if constexpr (!B_T) return frag_kmajor(ba[0], g); else return frag_transp<TWB>(ba[g], h);
   };
 
   // One half-step: the 64 MFMAs of one 32-element half of a K-step on `cur`, with the 16
@@ -545,7 +550,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   auto half = [&](Frags<WT, WN>& cur, Frags<WT, WN>& nxt, uint32_t sa, uint32_t sb, int h, auto dma_tag,
                   const bf16* dbase, const uint32_t (&doff)[WT], uint32_t dslot) {
     constexpr int DMA = decltype(dma_tag)::value;  // how many loads to weave in (0: none)
-    uint32_t aa[FragReader<A_T, WT>::NBASE], ba[FragReader<B_T, WT>::NBASE];
+    uint32_t aa[FragReader<A_T, TW>::NBASE], ba[FragReader<B_T, TWB>::NBASE];
     frag_addrs(sa, sb, h, aa, ba);
     const uint32_t dst = dslot + wave_blk;
 #pragma unroll
@@ -621,7 +626,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     }
     __syncthreads();
     if (!carried) {
-      uint32_t aa[FragReader<A_T, WT>::NBASE], ba[FragReader<B_T, WT>::NBASE];
+      uint32_t aa[FragReader<A_T, TW>::NBASE], ba[FragReader<B_T, TWB>::NBASE];
       frag_addrs(ring[0], ring[1], 0, aa, ba);
 #pragma unroll
       for (int g = 0; g < WT; ++g) {

@@ -319,6 +319,20 @@ def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(big_x, big_w, residual=embed(res, R_, C_))[:m, :n])
 
 
+@pytest.mark.parametrize("m,n,k", [(3080, 2008, 2056), (1544, 4072, 2104), (6024, 1000, 1032), (5000, 1160, 4096), (4104, 1032, 1992)])
+def test_gemm_narrow_tiles_have_the_bits_of_wide_ones(be, m, n, k):
+    """Outputs of fewer large tiles than compute units take narrower ones, down to 128 columns, whose transposed operand has a
+    layout of its own: the corner of an output of 192 tiles and more, with remainders in rows, columns and contraction."""
+    M, N = 6144, 4096
+    a, b = rnd(M, k, seed=61), rnd(N, k, scale=0.05, seed=62)
+    for layout, f, g in ((0, lambda t: t, lambda t: t), (1, lambda t: t, lambda t: t.t().contiguous()),
+                         (2, lambda t: t.t().contiguous(), lambda t: t.t().contiguous())):
+        big = be.gemm(layout, f(a), g(b), M, N, k, split_k=None)
+        got = be.gemm(layout, f(a[:m]), g(b[:n]), m, n, k, split_k=None)
+        assert torch.equal(got, big[:m, :n])
+    assert rel(got, a[:m].float() @ b[:n].float().t()) <= TOL
+
+
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("k", [8, 64, 72, 128, 136, 192, 200, 1096])
 def test_gemm_items_of_one_workgroup_have_the_bits_of_items_of_their_own(be, k, tile):
