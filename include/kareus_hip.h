@@ -60,8 +60,8 @@ size_t kr_gemm_workspace_bytes(int layout, int M, int N, int K);
  * value, so that the cuts the dispatcher plans are the cuts the buffer holds.  kr_gemm_bf16 uses
  * as many splits as the workspace it is handed holds, at most the planned count.              */
 size_t kr_gemm_workspace_bytes_shared(int layout, int M, int N, int K, float latency_weight);
-/* What a launch of this size is planned as (for tests and for reading profiles): the rows of an output tile, 256
- * or 128, and the cuts of the contraction.  epilogue, max_cus and workspace_bytes (0: none) as in the
+/* What a launch of this size is planned as (for tests and for reading profiles): the rows of an output tile, 256,
+ * or 128 for the small tiles (128 x 128, 128 x 64 and 64 x 64), and the cuts of the contraction.  epilogue, max_cus and workspace_bytes (0: none) as in the
  * calls below.                                                                                  */
 int kr_gemm_plan(int M, int N, int K, int epilogue, int max_cus, size_t workspace_bytes, int* tile_rows, int* splits);
 int kr_gemm_bf16(int layout, int M, int N, int K,

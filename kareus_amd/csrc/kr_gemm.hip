@@ -38,7 +38,7 @@
 //   * Workgroups are persistent (one per compute unit); ids are remapped so that the tiles
 //     resident on one XCD (ids congruent mod 8) form a compact band of C and share A/B panels
 //     in that XCD's L2.
-//   * Outputs of few tiles (short sequences, thin shards) use 128 x 128 tiles of the same structure:
+//   * Outputs of few tiles (short sequences, thin shards) use 128 x 128 tiles of the same structure, or 128 x 64 and 64 x 64:
 //     4 x 4 MFMA tiles per wave, 16 KB slots, two workgroups per compute unit.  Such a launch is
 //     bound by the number of work items and the latency of a K-step, not by LDS traffic (which a
 //     small tile has twice of per FLOP: 128 KB per 512 MFMA cycles with the loads, so it tops out at
@@ -87,8 +87,8 @@ struct Fused {
   const Segments* segs = nullptr;     // layout NT: the operands come in these pieces (A and B are unused)
 };
 
-// One launch as the dispatcher planned it.  wn: 16-column MFMA tiles per wave; small: the 128 x 128 tile; transposed:
-// operands exchanged, C^T stored.
+// One launch as the dispatcher planned it.  wn: 16-column MFMA tiles per wave; transposed: operands exchanged, C^T stored.
+enum Tile { kLarge, kSmall, kNarrow, kTiny };  // 256 rows (32 wn columns), 128 x 128, 128 x 64, 64 x 64
 struct Call {
   const bf16* a;
   int64_t lda;
@@ -101,7 +101,8 @@ struct Call {
   size_t workspace_bytes;
   hipStream_t stream;
   int num_cus, wn, splits;
-  bool small, transposed;
+  Tile tile;
+  bool transposed;
 };
 int launch_tn(const Call& call, const Fused& fu);
 int launch_nn(const Call& call, const Fused& fu);
@@ -118,7 +119,8 @@ constexpr int BM = 256, BN = 256;  // the largest tile; a kernel instance covers
 // WT: 16x16 MFMA tiles per wave along M; a wave owns 16 * WT rows x 16 * WN columns of C.  WT = 8: 256-row tiles
 // with 32 KB ring slots.  WT = 4 (with WN = 4): 128 x 128 tiles with 16 KB slots, two workgroups per compute unit
 // (see choose_plan for when they are taken).
-constexpr int WT_LARGE = 8, WT_SMALL = 4;
+// WT = 4 or 2 with WN = 2: 128 x 64 and 64 x 64 tiles, for outputs that would leave units without a small tile (see choose_plan).
+constexpr int WT_LARGE = 8, WT_SMALL = 4, WT_TINY = 2;
 constexpr int NTHREADS = 256;
 template <int WT>
 constexpr uint32_t kSlotBytes = 32 * WT * BK * sizeof(bf16);  // one operand tile (either layout)
@@ -161,12 +163,16 @@ __device__ __forceinline__ int kmajor_off(int row, int chunk) {
 // transposed tile [64 k-rows][256]: 512-byte rows, 16-byte chunk index XORed with a value made of
 // k-row bits 0, 1 (the four k-rows one 16-lane group reads together) and bit 3 (the two groups
 // of a 32-lane half read k-rows 8 apart).
-__device__ __forceinline__ int transp_swz(int krow) { return ((krow & 3) << 2) | (((krow >> 3) & 1) << 1); }
+// (tile rows of 64 elements are half as long as all banks: the low bit of the k-row picks the half by itself)
+template <int TW>
+__device__ __forceinline__ int transp_swz(int krow) {
+  return (TW == 64 ? ((krow >> 1) & 1) << 2 : (krow & 3) << 2) | (((krow >> 3) & 1) << 1);
+}
 // A small tile has rows of 128 elements, 256 bytes: as many as there are banks, so what a row and the
 // swizzle do to the banks is the same.
 template <int TW>
 __device__ __forceinline__ int transp_off(int krow, int col) {
-  return krow * TW + (((col >> 3) ^ transp_swz(krow)) << 3) + (col & 7);
+  return krow * TW + (((col >> 3) ^ transp_swz<TW>(krow)) << 3) + (col & 7);
 }
 
 // ---- direct global -> LDS loads ---------------------------------------------------------------
@@ -212,7 +218,7 @@ __device__ __forceinline__ int run_off(int r, int ld, int sh, int outer) {
 }
 template <int TW>
 __device__ __forceinline__ int load_krow(int i, int wave, int lane) {
-  return TW == 256 ? 2 * wave + (lane >> 5) + 8 * i : 4 * wave + (lane >> 4) + 16 * i;
+  return TW == 256 ? 2 * wave + (lane >> 5) + 8 * i : TW == 128 ? 4 * wave + (lane >> 4) + 16 * i : 8 * wave + (lane >> 3) + 32 * i;
 }
 template <bool TRANSPOSED, int TW>
 __device__ __forceinline__ uint32_t load_offset(int i, int wave, int lane, int ld, int row0,
@@ -230,7 +236,7 @@ __device__ __forceinline__ uint32_t load_offset(int i, int wave, int lane, int l
   // (the contraction rows of a K-step start at a multiple of 64, hence of the run length: the
   // position inside the K-step maps like a row of its own)
   int krow = load_krow<TW>(i, wave, lane);
-  int c = row0 + ((lane & (TW / 8 - 1)) ^ transp_swz(krow)) * 8;
+  int c = row0 + ((lane & (TW / 8 - 1)) ^ transp_swz<TW>(krow)) * 8;
   c = c + 8 <= rows_total ? c : rows_total - 8;
   krow = krow < k_left ? krow : k_left - 1;
   return (uint32_t)((sh ? run_off(krow, ld, sh, outer) : krow * ld) + c);
@@ -330,14 +336,15 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
                                                         bf16* __restrict__ out2, int ld_out2,
                                                         RowRuns runs_arg, Segments segs) {
   static_assert(!SEG || (A_T && B_T), "operand pieces: layout NT");
-  static_assert(DEPTH == kDepth || (DEPTH == kDepthAlone && WT == WT_SMALL), "ring depths");
-  static_assert(WT == WT_LARGE || (WT == WT_SMALL && WN == 4 && EPI != KR_GEMM_EPI_TRANSPOSED_OUT), "tile shapes");
+  static_assert(DEPTH == kDepth || (DEPTH == kDepthAlone && WT != WT_LARGE), "ring depths");
+  static_assert(WT == WT_LARGE || (((WT == WT_SMALL && (WN == 4 || WN == 2)) || (WT == WT_TINY && WN == 2)) &&
+                                   EPI != KR_GEMM_EPI_TRANSPOSED_OUT), "tile shapes");
   // operand rows an LDS tile of A / of B holds.  A K-major B tile may use fewer; a transposed one of 128 columns is laid out
   // as such: spread over rows of 256, as those of 160 to 224 are, half of what it loads is never read, and a K-step of the
   // 256 x 128 tile takes 64 KB through the unit's address path instead of 48.  us, before -> after: 3072 x 2048 x 8192 (NT) 128 ->
   // 106, 1536 x 4096 x 6024 (NT) 99 -> 80, 512 x 2048 x 32768 (NT, cut) 98 -> 81, 6024 x 1024 x 4096 (NN) 67 -> 55, 16384 x 384 x
   // 3072 (NN) 53 -> 48.
-  constexpr int TW = 32 * WT, TWB = WT == WT_SMALL || (B_T && WN == 4) ? 128 : 256;
+  constexpr int TW = 32 * WT, TWB = WN == 2 ? 64 : WT == WT_SMALL || (B_T && WN == 4) ? 128 : 256;
   constexpr uint32_t SLOT_BYTES = kSlotBytes<WT>;
   // (without RUNS every run length reads as a compile-time 1: the branches below fold away)
   const RowRuns runs = RUNS ? runs_arg : RowRuns{0, 0, 0, 0, 0, 0};
@@ -473,8 +480,8 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     const uint32_t dst = slot + wave_blk;
     dma_b128<0 * 4096>(base, off[0], dst);
     dma_b128<1 * 4096>(base, off[1], dst);
-    dma_b128<2 * 4096>(base, off[2], dst);
-    dma_b128<3 * 4096>(base, off[3], dst);
+    if constexpr (COUNT > 2) dma_b128<2 * 4096>(base, off[2], dst);
+    if constexpr (COUNT > 3) dma_b128<3 * 4096>(base, off[3], dst);
     if constexpr (COUNT > 4) dma_b128<4 * 4096>(base, off[4], dst);
     if constexpr (COUNT > 5) dma_b128<5 * 4096>(base, off[5], dst);
     if constexpr (COUNT > 6) dma_b128<6 * 4096>(base, off[6], dst);
@@ -569,13 +576,13 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
                        : "v"(cur.b[nt]), "v"(cur.a[g]));
         }
         if (nt == 0) nxt.a[g] = read_a(aa, g, h);
-        if (nt == 2 && g < WN) nxt.b[g] = read_b(ba, g, h);
+        if (nt == (WN > 2 ? 2 : 1) && g < WN) nxt.b[g] = read_b(ba, g, h);
         if constexpr (DMA > 0) {
-          if (nt == (WN > 4 ? 4 : 3) && g < DMA) {
+          if (nt == (WN > 4 ? 4 : WN > 2 ? 3 : 1) && g < DMA) {
             if (g == 0) dma_b128<0 * 4096>(dbase, doff[0], dst);
             if (g == 1) dma_b128<1 * 4096>(dbase, doff[1], dst);
-            if (g == 2) dma_b128<2 * 4096>(dbase, doff[2], dst);
-            if (g == 3) dma_b128<3 * 4096>(dbase, doff[3], dst);
+            if constexpr (DMA > 2) if (g == 2) dma_b128<2 * 4096>(dbase, doff[2], dst);
+            if constexpr (DMA > 3) if (g == 3) dma_b128<3 * 4096>(dbase, doff[3], dst);
             if constexpr (DMA > 4) if (g == 4) dma_b128<4 * 4096>(dbase, doff[4], dst);
             if constexpr (DMA > 5) if (g == 5) dma_b128<5 * 4096>(dbase, doff[5], dst);
             if constexpr (DMA > 6) if (g == 6) dma_b128<6 * 4096>(dbase, doff[6], dst);
@@ -719,13 +726,12 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     // data: program order of its LDS instructions is all the ordering needed.  The accumulators
     // are read in one place for all three kinds of output.
     {
-      // staged rows: 256 bytes of bf16 (two buffers of 16 rows) or 512 of fp32 (one buffer), half of that for
-      // a small tile, whose waves are 64 columns wide
-      constexpr bool small = WT == WT_SMALL;
-      constexpr uint32_t STAGE = SLOT_BYTES / 4, SBUF = STAGE / 2, ROW16 = SBUF / 16, ROW32 = STAGE / 16;
-      constexpr int XOR16 = small ? 7 : 15;         // a bf16 row has 8 or 16 chunks
-      constexpr int L16 = small ? 8 : 16, Q16 = L16 / 4;   // lanes per stored row, passes per 16-row block: bf16
-      constexpr int L32 = small ? 16 : 32, Q32 = L32 / 4;  // ... and fp32
+      // staged rows are as wide as the wave's tile, 128, 64 or 32 columns: bf16 in two buffers of 16 rows, fp32 in one
+      constexpr int PW = WN > 4 ? 128 : WN > 2 ? 64 : 32;
+      constexpr uint32_t ROW16 = 2 * PW, SBUF = 16 * ROW16, STAGE = 2 * SBUF, ROW32 = 4 * PW;
+      constexpr int L16 = PW / 8, Q16 = L16 > 4 ? L16 / 4 : 1;   // lanes per stored row, passes per 16-row block: bf16
+      constexpr int L32 = PW / 4, Q32 = L32 / 4;                 // ... and fp32
+      constexpr int XOR16 = L16 - 1, XOR32 = L32 > 16 ? 15 : L32 - 1;
       const uint32_t stage = ring[NSLOTS - 1] + (uint32_t)wave * STAGE;
       int le = lane;  // opaque copy: nothing derived from it is kept alive through the K loop
       asm volatile("" : "+v"(le));
@@ -892,14 +898,15 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
             const uint32_t gbuf = ring[NSLOTS - 1] + (uint32_t)(2 * wm) * STAGE + (uint32_t)(mt & 1) * SBUF;
             const uint32_t ubuf = gbuf + STAGE;
 #pragma unroll
-            for (int qq = 0; qq < Q16 / 2; ++qq) {
-              const int rr = 64 / L16 * (Q16 / 2 * wn + qq) + row_r;
+            for (int qq = 0; qq < (Q16 > 1 ? Q16 / 2 : 1); ++qq) {
+              // (one pass covers all 16 rows of a 32-column block: half the lanes take the wave's eight)
+              const int rr = Q16 > 1 ? 64 / L16 * (Q16 / 2 * wn + qq) + row_r : 8 * wn + (row_r & 7);
               const bf16x8 g = *(KR_LDS const bf16x8*)(gbuf + rr * ROW16 + ((rch ^ (rr & XOR16)) << 4));
               const bf16x8 u = *(KR_LDS const bf16x8*)(ubuf + rr * ROW16 + ((rch ^ (rr & XOR16)) << 4));
               bf16x8 y;
 #pragma unroll
               for (int e = 0; e < 8; ++e) y[e] = (bf16)kr_swiglu_f((float)g[e], (float)u[e]);
-              if (ncols_in && rr < rows_left - mt * 16)
+              if (ncols_in && rr < rows_left - mt * 16 && (Q16 > 1 || row_r < 8))
                 stg8_out(at_byte(out2 + ((int64_t)(m_wave + mt * 16) * ld_out2 + out_n0), 2u * (uint32_t)(rr * ld_out2 + 8 * rch)), y);
             }
           }
@@ -911,12 +918,12 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
           take_block(mt, vals);
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt)
-            *(KR_LDS f32x4*)(stage + row16 * ROW32 + (((4 * nt + quad) ^ row16) << 4)) = vals[nt];
+            *(KR_LDS f32x4*)(stage + row16 * ROW32 + (((4 * nt + quad) ^ (row16 & XOR32)) << 4)) = vals[nt];
           wave_sync();
         };
         auto staged = [&](int q) {
           const int rr = 64 / L32 * q + hrow;
-          return *(KR_LDS const f32x4*)(stage + rr * ROW32 + ((ch ^ rr) << 4));
+          return *(KR_LDS const f32x4*)(stage + rr * ROW32 + ((ch ^ (rr & XOR32)) << 4));
         };
         if constexpr (split_k) {
 #pragma unroll
@@ -1026,13 +1033,14 @@ int launch(const Call& call, const Fused& fu) {
   int num_cus = call.num_cus;
   size_t lds_bytes = 0;
   const int one_per_cu = fu.max_cus > 0 && fu.max_cus < num_cus ? fu.max_cus : num_cus;
-  if (WT == WT_SMALL && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
+  constexpr bool kOneRound = WT != WT_LARGE && WN == 2;  // (planned for outputs that have a unit for every tile)
+  if (WT == WT_SMALL && !kOneRound && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
   if (fu.max_cus > 0 && fu.max_cus < num_cus) num_cus = fu.max_cus;
   const int tiles = ((M + 32 * WT - 1) / (32 * WT)) * ((N + 32 * WN - 1) / (32 * WN));
   // the planned count, which the dispatcher has already capped by what the caller's workspace holds
   int splits = call.splits;
   const size_t one = (size_t)M * N * sizeof(float);
-  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE) {
+  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE || kOneRound) {
     splits = 1;  // a fused epilogue works on finished sums
   } else if ((size_t)splits * one > workspace_bytes) {
     splits = (int)(workspace_bytes / one);
@@ -1091,13 +1099,16 @@ int launch(const Call& call, const Fused& fu) {
   };
   auto pick = [&](auto depth_tag) {
     if constexpr (EPI == KR_GEMM_EPI_NONE) {
-      if (splits > 1) return pick_kind(depth_tag, Count<KR_GEMM_OUT_PARTIAL>{});
+      if constexpr (!kOneRound)
+        if (splits > 1) return pick_kind(depth_tag, Count<KR_GEMM_OUT_PARTIAL>{});
       if (accumulate) return pick_kind(depth_tag, Count<KR_GEMM_OUT_ACCUMULATE>{});
     }
     pick_kind(depth_tag, Count<EPI>{});
   };
-  bool deep = false;
-  if constexpr (WT == WT_SMALL) {
+  bool deep = kOneRound;
+  if constexpr (kOneRound) {
+    pick(Count<kDepthAlone>{});
+  } else if constexpr (WT == WT_SMALL) {
     // A small tile that has its compute unit to itself waits for memory: a K-step lasts 0.5 us there, two of
     // them are less than a load from HBM takes.  The deep ring asks four ahead.  Operands in HBM, two -> four
     // ahead, us: 512 tokens of the 8B shard's fc1 51.4 -> 40.2, fc2 46.0 -> 37.9, fc2's input gradient 51.3 ->
@@ -1107,7 +1118,8 @@ int launch(const Call& call, const Fused& fu) {
     deep = tiles * splits <= one_per_cu && !fu.shared && (K / BK) / splits > 8;
     if (deep) pick(Count<kDepthAlone>{});
   }
-  if (!deep) pick(Count<kDepth>{});
+  if constexpr (!kOneRound)
+    if (!deep) pick(Count<kDepth>{});
   if (attr_status != hipSuccess) return KR_ELAUNCH;
   const Segments segs = with_segs ? *fu.segs : Segments{};
   if (splits == 1) {
@@ -1136,7 +1148,12 @@ int launch(const Call& call, const Fused& fu) {
 template <bool A_T, bool B_T, int EPI, int MIN_WN>
 int launch_tile(const Call& call, const Fused& fu) {
   if constexpr (EPI != KR_GEMM_EPI_TRANSPOSED_OUT)
-    if (call.small) return launch<A_T, B_T, 4, EPI, WT_SMALL>(call, fu);
+    switch (call.tile) {
+      case kSmall: return launch<A_T, B_T, 4, EPI, WT_SMALL>(call, fu);
+      case kNarrow: return launch<A_T, B_T, 2, EPI, WT_SMALL>(call, fu);
+      case kTiny: return launch<A_T, B_T, 2, EPI, WT_TINY>(call, fu);
+      default: break;
+    }
   if constexpr (MIN_WN <= 4)
     if (call.wn == 4) return launch<A_T, B_T, 4, EPI>(call, fu);
   switch (call.wn) {
@@ -1201,14 +1218,14 @@ inline int choose_wn(int M, int N, int num_cus) {
 // keep its CU-time small (the dispatcher uses latency_weight 0.1).  `max_splits` is what the caller's workspace holds.
 struct Plan {
   int wn, splits;
-  bool small;  // 128 x 128 tiles (wn is 4)
+  Tile tile = kLarge;  // (wn is 4 for the small tile, 2 for the two below it)
 };
 inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, int max_splits,
                         bool fused = false, bool allow_small = true) {
   constexpr int kItemOverhead = 4;
   const int min_wn = fused ? 5 : 4;
   const int tiles_m = (M + BM - 1) / BM;
-  if (tiles_m * ((N + BN - 1) / BN) >= 192) return {choose_wn(M, N, num_cus), 1, false};
+  if (tiles_m * ((N + BN - 1) / BN) >= 192) return {choose_wn(M, N, num_cus), 1};
   const double w = latency_weight < 0.f ? 0.0 : (latency_weight > 1.f ? 1.0 : (double)latency_weight);
   const int nk = (K + BK - 1) / BK;
   const double reduce_per_split = (double)M * N * 8.0 / 5.0e12 / 1.3e-6;
@@ -1221,13 +1238,13 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
     const double cu_time = items * per_item / num_cus + reduce;
     return w * latency + (1.0 - w) * cu_time;
   };
-  Plan best{8, 1, false};
+  Plan best{8, 1};
   double best_cost = cost(8, 1);
   for (int wn = 7; wn >= min_wn; --wn) {
     const double c = cost(wn, 1);
     if (c < best_cost) {
       best_cost = c;
-      best = {wn, 1, false};
+      best = {wn, 1};
     }
   }
   const double unsplit = best_cost;
@@ -1249,7 +1266,7 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
       const double c = cost(wn, sp);
       if (c < unsplit * 0.95 && c < best_cost) {  // a split must pay for itself clearly
         best_cost = c;
-        best = {wn, sp, false};
+        best = {wn, sp};
       }
       if (alone) large = std::min(large, large_cost(wn, sp));
     }
@@ -1299,9 +1316,32 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
       if (small_cost(sp, split) < small_cost(at, split)) at = sp;
     return at;
   };
-  if (small_cost(small_cut(kSplit), kSplit) >= large * 0.93) return best;  // the change must be clear
+  // Fewer small tiles than units, alone on the device: a unit takes in about 32 KB per 0.35 us (operands in the L2s or the
+  // memory-side cache) to 0.75 (in HBM) whatever its ring holds, and a K-step of a small tile is 32 KB.  128 x 64 and 64 x 64 tiles, 24 and 16 KB a
+  // K-step, use the units that would have none, as long as every tile has a unit.
+  // Measured, small -> these, us: 512 x 4096 x 3584 with the residual 35 -> 26 (128 x 64), 512 x 3584 x 4096 (NN) with the SwiGLU
+  // backward 42 -> 35, 128 x 4096 x 3584 31 -> 14 (64 x 64), 256 x 512 x 1376 16 -> 9, 384 x 1024 x 3072 (NN) with the SwiGLU backward 25 ->
+  // 13, 1024 x 512 x 2048 (two cuts) 17 -> 9; of 130 sizes none is slower.  In units as above: 0.21-0.42 us a K-step.
+  constexpr double kStepNarrow = 0.26, kStepTiny = 0.20, kOverheadNarrow = 2.5;
+  Tile under = kSmall;
+  double under_cost = 1e30;
+  if (alone) {
+    auto try_tile = [&](Tile tile, int rows, double step) {
+      const int items = ((M + rows - 1) / rows) * ((N + 63) / 64);
+      const double c = nk * step + kOverheadNarrow;
+      if (items <= num_cus && c < under_cost) {
+        under = tile;
+        under_cost = c;
+      }
+    };
+    try_tile(kNarrow, 128, kStepNarrow);
+    try_tile(kTiny, 64, kStepTiny);
+  }
+  const double small = small_cost(small_cut(kSplit), kSplit);
+  if (std::min(small, under_cost) >= large * 0.93) return best;  // the change must be clear
+  if (under_cost < small) return {2, 1, under};
   // (beside other streams the extra launch is no compute-unit time: 384 x 640 x 4096 in two cuts 21 us, uncut 32)
-  return {4, small_cut(w * kSplit), true};
+  return {4, small_cut(w * kSplit), kSmall};
 }
 
 // Tile width for a projection with the SwiGLU epilogue: the tiles have to divide the 2F output
@@ -1374,7 +1414,7 @@ extern "C" int kr_gemm_plan(int M, int N, int K, int epilogue, int max_cus, size
   const Plan plan = launch_plan(M, N, K, epilogue & ~KR_GEMM_BESIDE_OTHER_STREAMS,
                                 (epilogue & KR_GEMM_BESIDE_OTHER_STREAMS) != 0,
                                 max_cus > 0 && max_cus < num_cus ? max_cus : num_cus, workspace_bytes);
-  *tile_rows = plan.small ? 32 * WT_SMALL : 32 * WT_LARGE;
+  *tile_rows = plan.tile != kLarge ? 32 * WT_SMALL : 32 * WT_LARGE;
   *splits = plan.splits;
   return KR_OK;
 }
@@ -1446,7 +1486,7 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
   const Plan plan = launch_plan(M, N, K, fu.epi, fu.shared, cus, ws != nullptr && fu.runs.c_sh == 0 ? workspace_bytes : 0);
   const int wn = fu.epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn;
   const Call call{a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, wn,
-                  fu.epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.small, false};
+                  fu.epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.tile, false};
   switch (layout) {
     case KR_GEMM_TN:  // A [M,K], B [N,K]
       if (lda < K || ldb < K || ldc < N) return KR_EINVAL;
@@ -1483,7 +1523,7 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
             exchanged.steps = fu.segs->steps;
             fut.segs = &exchanged;
           }
-          const Call exchanged_call{b, ldb, a, lda, c, ldc, N, M, K, 0, nullptr, 0, st, num_cus, wt, 1, false, true};
+          const Call exchanged_call{b, ldb, a, lda, c, ldc, N, M, K, 0, nullptr, 0, st, num_cus, wt, 1, kLarge, true};
           return launch_nt(exchanged_call, fut);
         }
       }

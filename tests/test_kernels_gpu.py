@@ -319,6 +319,28 @@ def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(big_x, big_w, residual=embed(res, R_, C_))[:m, :n])
 
 
+@pytest.mark.parametrize("m,n,k", [(8, 8, 8), (64, 64, 64), (72, 136, 1096), (200, 328, 264), (128, 4096, 200), (520, 3208, 584), (1000, 512, 2752),
+                                   (264, 1376, 256)])
+def test_gemm_smallest_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
+    """Outputs that would leave compute units without a tile of 128 x 128 are computed in 128 x 64 or 64 x 64 tiles: every layout
+    and kind of output against a corner of an output of 192 large tiles, at contractions shorter than the ring and longer."""
+    M, N = 4096, 3072 if n <= 3072 else 4096
+    a, b, old, res = rnd(M, k, seed=61), rnd(N, k, scale=0.05, seed=62), rnd(M, N, seed=63), rnd(M, N, seed=64)
+    for layout, f, g in ((0, lambda t: t, lambda t: t), (1, lambda t: t, lambda t: t.t().contiguous()),
+                         (2, lambda t: t.t().contiguous(), lambda t: t.t().contiguous())):
+        big, few = (layout, f(a), g(b), M, N, k), (layout, f(a[:m]), g(b[:n]), m, n, k)
+        assert torch.equal(be.gemm(*few, split_k=None), be.gemm(*big, split_k=None)[:m, :n])
+        acc = [be.gemm(*c, out=o.clone(), accumulate=True, split_k=None) for c, o in ((few, old[:m, :n]), (big, old))]
+        assert torch.equal(acc[0], acc[1][:m, :n])
+    assert rel(be.linear_fwd(a[:m], b[:n]), a[:m].float() @ b[:n].float().t()) <= TOL
+    assert torch.equal(be.linear_fwd(a[:m], b[:n], residual=res[:m, :n]), be.linear_fwd(a, b, residual=res)[:m, :n])
+    wt = b.t().contiguous()
+    pre = rnd(M, 2 * N, seed=65)
+    few_pre = torch.cat([pre[:m, :n], pre[:m, N:N + n]], dim=1)
+    dx, big_dx = (be.linear_dgrad(x, w, swiglu_bwd_x=p) for x, w, p in ((a[:m], wt[:, :n].contiguous(), few_pre), (a, wt, pre)))
+    assert torch.equal(dx[:, :n], big_dx[:m, :n]) and torch.equal(dx[:, n:], big_dx[:m, N:N + n])
+
+
 @pytest.mark.parametrize("m,n,k", [(3080, 2008, 2056), (1544, 4072, 2104), (6024, 1000, 1032), (5000, 1160, 4096), (4104, 1032, 1992)])
 def test_gemm_narrow_tiles_have_the_bits_of_wide_ones(be, m, n, k):
     """Outputs of fewer large tiles than compute units take narrower ones, down to 128 columns, whose transposed operand has a
