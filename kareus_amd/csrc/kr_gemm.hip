@@ -88,7 +88,8 @@ struct Fused {
 };
 
 // One launch as the dispatcher planned it.  wn: 16-column MFMA tiles per wave; transposed: operands exchanged, C^T stored.
-enum Tile { kLarge, kSmall, kNarrow, kTiny };  // 256 rows (32 wn columns), 128 x 128, 128 x 64, 64 x 64
+// 256 rows (32 wn columns), 128 x 128, 128 x 64, 64 x 64, 224 or 192 rows of 256 columns
+enum Tile { kLarge, kSmall, kNarrow, kTiny, kRows224, kRows192 };
 struct Call {
   const bf16* a;
   int64_t lda;
@@ -119,11 +120,12 @@ constexpr int BM = 256, BN = 256;  // the largest tile; a kernel instance covers
 // WT: 16x16 MFMA tiles per wave along M; a wave owns 16 * WT rows x 16 * WN columns of C.  WT = 8: 256-row tiles
 // with 32 KB ring slots.  WT = 4 (with WN = 4): 128 x 128 tiles with 16 KB slots, two workgroups per compute unit
 // (see choose_plan for when they are taken).
+// WT = 7 or 6 (K-major A, WN = 8): 224- and 192-row tiles, for outputs whose rows or rounds they divide better.
 // WT = 4 or 2 with WN = 2: 128 x 64 and 64 x 64 tiles, for outputs that would leave units without a small tile (see choose_plan).
 constexpr int WT_LARGE = 8, WT_SMALL = 4, WT_TINY = 2;
 constexpr int NTHREADS = 256;
 template <int WT>
-constexpr uint32_t kSlotBytes = 32 * WT * BK * sizeof(bf16);  // one operand tile (either layout)
+constexpr uint32_t kSlotBytes = 32 * (WT > 4 ? 8 : WT) * BK * sizeof(bf16);  // one operand tile (either layout)
 // DEPTH: how many K-steps ahead a tile is requested; the ring has 2 * DEPTH + 1 slots.  2: 5 x 32 KB = the whole
 // 160 KB of LDS (5 x 16 KB: half of it).  4, for small tiles that have a compute unit to themselves: 9 x 16 KB.
 constexpr int kDepth = 2, kDepthAlone = 4;
@@ -336,8 +338,9 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
                                                         bf16* __restrict__ out2, int ld_out2,
                                                         RowRuns runs_arg, Segments segs) {
   static_assert(!SEG || (A_T && B_T), "operand pieces: layout NT");
-  static_assert(DEPTH == kDepth || (DEPTH == kDepthAlone && WT != WT_LARGE), "ring depths");
-  static_assert(WT == WT_LARGE || (((WT == WT_SMALL && (WN == 4 || WN == 2)) || (WT == WT_TINY && WN == 2)) &&
+  static_assert(DEPTH == kDepth || (DEPTH == kDepthAlone && WT <= WT_SMALL), "ring depths");
+  static_assert(WT == WT_LARGE || ((WT == 7 || WT == 6) && !A_T && WN == 8 && !RUNS && !SEG) ||
+                    (((WT == WT_SMALL && (WN == 4 || WN == 2)) || (WT == WT_TINY && WN == 2)) &&
                                    EPI != KR_GEMM_EPI_TRANSPOSED_OUT), "tile shapes");
   // operand rows an LDS tile of A / of B holds.  A K-major B tile may use fewer; a transposed one of 128 columns is laid out
   // as such: spread over rows of 256, as those of 160 to 224 are, half of what it loads is never read, and a K-step of the
@@ -356,6 +359,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   // spans all columns of a tile row
   constexpr int NB_LOADS = B_T ? TWB / 32 : WN;
   constexpr int NA_LOADS = WT;
+  constexpr int NL = NA_LOADS > NB_LOADS ? NA_LOADS : NB_LOADS;
   constexpr int BM_ = 32 * WT;
   const int wm = wave >> 1, wn = wave & 1;  // wave tile: rows wm*16*WT.., columns wn*16*WN..
   // fused epilogues: ADD: C = bf16(bf16(A.B) + aux), aux [M,N] with row stride ld_aux.
@@ -463,19 +467,19 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   // with that register class, see mfma() below); fragments in ordinary vector registers
   f32x4 acc[WT][WN];
   Frags<WT, WN> X, Y;
-  uint32_t la[WT], lb[WT];  // byte offsets of this lane's chunk in the loads of an A / a B tile
+  uint32_t la[NL], lb[NL];  // byte offsets of this lane's chunk in the loads of an A / a B tile
 
   auto set_offsets = [&](int k_left) {
     int l2 = lane;
     asm volatile("" : "+v"(l2));
 #pragma unroll
-    for (int i = 0; i < WT; ++i) {
-      la[i] = 2u * load_offset<A_T, TW>(i, wave, l2, lda, m0, M, k_left, 0, 0, runs.a_sh, runs.a_outer);
+    for (int i = 0; i < NL; ++i) {
+      if (i < NA_LOADS) la[i] = 2u * load_offset<A_T, TW>(i, wave, l2, lda, m0, M, k_left, 0, 0, runs.a_sh, runs.a_outer);
       if (i < NB_LOADS) lb[i] = 2u * load_offset<B_T, TWB>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN);
     }
   };
   // the first `count` loads of a tile (NA_LOADS for A, NB_LOADS for B)
-  auto request = [&](const bf16* base, const uint32_t (&off)[WT], uint32_t slot, auto count_tag) {
+  auto request = [&](const bf16* base, const uint32_t (&off)[NL], uint32_t slot, auto count_tag) {
     constexpr int COUNT = decltype(count_tag)::value;
     const uint32_t dst = slot + wave_blk;
     dma_b128<0 * 4096>(base, off[0], dst);
@@ -507,9 +511,9 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     int l2 = lane;
     asm volatile("" : "+v"(l2));
 #pragma unroll
-    for (int i = 0; i < WT; ++i) {
+    for (int i = 0; i < NL; ++i) {
       const uint32_t blk = (uint32_t)(wave + 4 * i) * 1024u + (uint32_t)l2 * 16u;
-      if (load_k<A_T, TW>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sa + blk) = zero8();
+      if (i < NA_LOADS && load_k<A_T, TW>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sa + blk) = zero8();
       if (i < NB_LOADS && load_k<B_T, TWB>(i, wave, l2) >= k_tail) *(KR_LDS bf16x8*)(sb + blk) = zero8();
     }
   };
@@ -555,7 +559,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   // operands are swapped (the B fragment feeds the instruction's A port), so a lane ends up
   // with four consecutive columns of one row of C.
   auto half = [&](Frags<WT, WN>& cur, Frags<WT, WN>& nxt, uint32_t sa, uint32_t sb, int h, auto dma_tag,
-                  const bf16* dbase, const uint32_t (&doff)[WT], uint32_t dslot) {
+                  const bf16* dbase, const uint32_t (&doff)[NL], uint32_t dslot) {
     constexpr int DMA = decltype(dma_tag)::value;  // how many loads to weave in (0: none)
     uint32_t aa[FragReader<A_T, TW>::NBASE], ba[FragReader<B_T, TWB>::NBASE];
     frag_addrs(sa, sb, h, aa, ba);
@@ -577,6 +581,8 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
         }
         if (nt == 0) nxt.a[g] = read_a(aa, g, h);
         if (nt == (WN > 2 ? 2 : 1) && g < WN) nxt.b[g] = read_b(ba, g, h);
+        // (fewer rows of MFMA tiles than columns: the fragments and loads left over ride in rows 2 and 3)
+        if (WN > WT && nt == 6 && g >= 2 && g - 2 + WT < WN) nxt.b[g - 2 + WT] = read_b(ba, g - 2 + WT, h);
         if constexpr (DMA > 0) {
           if (nt == (WN > 4 ? 4 : WN > 2 ? 3 : 1) && g < DMA) {
             if (g == 0) dma_b128<0 * 4096>(dbase, doff[0], dst);
@@ -585,8 +591,13 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
             if constexpr (DMA > 3) if (g == 3) dma_b128<3 * 4096>(dbase, doff[3], dst);
             if constexpr (DMA > 4) if (g == 4) dma_b128<4 * 4096>(dbase, doff[4], dst);
             if constexpr (DMA > 5) if (g == 5) dma_b128<5 * 4096>(dbase, doff[5], dst);
-            if constexpr (DMA > 6) if (g == 6) dma_b128<6 * 4096>(dbase, doff[6], dst);
-            if constexpr (DMA > 7) if (g == 7) dma_b128<7 * 4096>(dbase, doff[7], dst);
+            if constexpr (DMA > 6 && WT > 6) if (g == 6) dma_b128<6 * 4096>(dbase, doff[6], dst);
+            if constexpr (DMA > 7 && WT > 7) if (g == 7) dma_b128<7 * 4096>(dbase, doff[7], dst);
+          }
+          if constexpr (DMA > WT && WT > 4) {
+            if (nt == 7 && g == 2) dma_b128<WT * 4096>(dbase, doff[WT], dst);
+            if constexpr (DMA > WT + 1)
+              if (nt == 7 && g == 3) dma_b128<(WT + 1) * 4096>(dbase, doff[WT + 1], dst);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -636,8 +647,8 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       uint32_t aa[FragReader<A_T, TW>::NBASE], ba[FragReader<B_T, TWB>::NBASE];
       frag_addrs(ring[0], ring[1], 0, aa, ba);
 #pragma unroll
-      for (int g = 0; g < WT; ++g) {
-        X.a[g] = read_a(aa, g, 0);
+      for (int g = 0; g < (WT > WN ? WT : WN); ++g) {
+        if (g < WT) X.a[g] = read_a(aa, g, 0);
         if (g < WN) X.b[g] = read_b(ba, g, 0);
       }
     }
@@ -1033,6 +1044,7 @@ int launch(const Call& call, const Fused& fu) {
   int num_cus = call.num_cus;
   size_t lds_bytes = 0;
   const int one_per_cu = fu.max_cus > 0 && fu.max_cus < num_cus ? fu.max_cus : num_cus;
+  constexpr bool kFewRows = WT == 7 || WT == 6;   // plain operands and outputs only (see fewer_rows)
   constexpr bool kOneRound = WT != WT_LARGE && WN == 2;  // (planned for outputs that have a unit for every tile)
   if (WT == WT_SMALL && !kOneRound && fu.max_cus <= 0) num_cus *= 2;  // two workgroups per unit, where the caller names no limit
   if (fu.max_cus > 0 && fu.max_cus < num_cus) num_cus = fu.max_cus;
@@ -1040,7 +1052,7 @@ int launch(const Call& call, const Fused& fu) {
   // the planned count, which the dispatcher has already capped by what the caller's workspace holds
   int splits = call.splits;
   const size_t one = (size_t)M * N * sizeof(float);
-  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE || kOneRound) {
+  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE || kOneRound || kFewRows) {
     splits = 1;  // a fused epilogue works on finished sums
   } else if ((size_t)splits * one > workspace_bytes) {
     splits = (int)(workspace_bytes / one);
@@ -1063,7 +1075,7 @@ int launch(const Call& call, const Fused& fu) {
   // instances that honour row runs exist for what the two ends of a layer stack launch: the residual-add
   // forward (aux or C in runs), the input gradient (plain or with the SwiGLU backward) and the weight
   // gradient (A in runs); instances that contract operand pieces for the weight gradient (both forms)
-  constexpr bool kRunsInstance = EPI == KR_GEMM_EPI_ADD || EPI == KR_GEMM_EPI_SWIGLU_BWD || (EPI == KR_GEMM_EPI_NONE && B_T);
+  constexpr bool kRunsInstance = !kFewRows && (EPI == KR_GEMM_EPI_ADD || EPI == KR_GEMM_EPI_SWIGLU_BWD || (EPI == KR_GEMM_EPI_NONE && B_T));
   constexpr bool kSegsInstance = A_T && B_T && (EPI == KR_GEMM_EPI_NONE || EPI == KR_GEMM_EPI_TRANSPOSED_OUT);
   // (pieces in row runs: the direct store form only, A in runs)
   constexpr bool kSegsRunsInstance = kSegsInstance && EPI == KR_GEMM_EPI_NONE;
@@ -1098,7 +1110,7 @@ int launch(const Call& call, const Fused& fu) {
     }
   };
   auto pick = [&](auto depth_tag) {
-    if constexpr (EPI == KR_GEMM_EPI_NONE) {
+    if constexpr (EPI == KR_GEMM_EPI_NONE && !kFewRows) {
       if constexpr (!kOneRound)
         if (splits > 1) return pick_kind(depth_tag, Count<KR_GEMM_OUT_PARTIAL>{});
       if (accumulate) return pick_kind(depth_tag, Count<KR_GEMM_OUT_ACCUMULATE>{});
@@ -1154,6 +1166,10 @@ int launch_tile(const Call& call, const Fused& fu) {
       case kTiny: return launch<A_T, B_T, 2, EPI, WT_TINY>(call, fu);
       default: break;
     }
+  if constexpr (!A_T && (EPI == KR_GEMM_EPI_NONE || EPI == KR_GEMM_EPI_ADD)) {
+    if (call.tile == kRows224) return launch<A_T, B_T, 8, EPI, 7>(call, fu);
+    if (call.tile == kRows192) return launch<A_T, B_T, 8, EPI, 6>(call, fu);
+  }
   if constexpr (MIN_WN <= 4)
     if (call.wn == 4) return launch<A_T, B_T, 4, EPI>(call, fu);
   switch (call.wn) {
@@ -1216,6 +1232,28 @@ inline int choose_wn(int M, int N, int num_cus) {
 // A GEMM that has the GPU to itself wants the smallest latency (latency_weight 1); one that
 // runs beside kernels of other streams, which can use the CUs it leaves idle, should mostly
 // keep its CU-time small (the dispatcher uses latency_weight 0.1).  `max_splits` is what the caller's workspace holds.
+// 224 or 192 rows of 256 columns in place of 256 rows of `wn` units, by the same estimate (rounds of tiles times their larger
+// side's units and one): where it is at least a ninth smaller and the last round is at least 5/8 full.  us before -> after:
+// TN 776 x 32064 x 4096 196 -> 178, 1152 x 32064 x 4096 246 -> 229, 6024 x 4096 x 3584 (residual) 151 -> 138; NN 6024 x 4096 x
+// 7168 280 -> 257, 12240 x 2048 x 16384 660 -> 575.  Outside the rule nothing is won: the workgroups of a round that is a third
+// full run faster than those of a full one (NN 6440 x 3072 x 16384 551 -> 557, 1504 x 12288 x 4096 142 -> 143), and a saving
+// of 1 in 36 is eaten by the operands that smaller tiles load more often (NN 20000 x 3072 x 2048 194 -> 194).
+inline Tile fewer_rows(int M, int N, int wn, int num_cus) {
+  auto tiles = [&](int rows, int cols) { return ((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
+  auto rounds = [&](int t) { return (long)((t + num_cus - 1) / num_cus); };
+  long best = rounds(tiles(BM, 32 * wn)) * (wn + 1) * 8;
+  Tile tile = kLarge;
+  for (int wt = 7; wt >= 6; --wt) {
+    const int t = tiles(32 * wt, BN), last = t - (int)(rounds(t) - 1) * num_cus;
+    const long cost = rounds(t) * (wt + 1);
+    if (cost * 9 <= best && last * 8 >= num_cus * 5) {
+      best = cost * 8;
+      tile = wt == 7 ? kRows224 : kRows192;
+    }
+  }
+  return tile;
+}
+
 struct Plan {
   int wn, splits;
   Tile tile = kLarge;  // (wn is 4 for the small tile, 2 for the two below it)
@@ -1485,8 +1523,13 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
   // finished sums and is never cut
   const Plan plan = launch_plan(M, N, K, fu.epi, fu.shared, cus, ws != nullptr && fu.runs.c_sh == 0 ? workspace_bytes : 0);
   const int wn = fu.epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn;
+  Tile tile = plan.tile;
+  const bool plain = fu.runs.a_sh == 0 && fu.runs.c_sh == 0 && fu.runs.x_sh == 0 && !accumulate;
+  if (tile == kLarge && plain && layout != KR_GEMM_NT && (fu.epi == KR_GEMM_EPI_NONE || fu.epi == KR_GEMM_EPI_ADD) && plan.splits == 1 &&
+      ((M + BM - 1) / BM) * ((N + BN - 1) / BN) >= 192)
+    tile = fewer_rows(M, N, wn, cus);
   const Call call{a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, wn,
-                  fu.epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.tile, false};
+                  fu.epi == KR_GEMM_EPI_NONE ? plan.splits : 1, tile, false};
   switch (layout) {
     case KR_GEMM_TN:  // A [M,K], B [N,K]
       if (lda < K || ldb < K || ldc < N) return KR_EINVAL;

@@ -341,6 +341,19 @@ def test_gemm_smallest_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     assert torch.equal(dx[:, :n], big_dx[:m, :n]) and torch.equal(dx[:, n:], big_dx[:m, N:N + n])
 
 
+@pytest.mark.parametrize("m,n,k", [(776, 16384, 200), (1144, 32056, 72), (6024, 4096, 136), (6072, 4088, 64), (5200, 4360, 1096)])
+def test_gemm_tiles_of_fewer_rows_have_the_bits_of_the_large_ones(be, m, n, k):
+    """Outputs whose rows or rounds 224 or 192 rows divide better than 256: the first rows of an output of 8192, plain and with
+    a residual, with one K-step, two, three and many of them, the last one whole or partial."""
+    M = 8192
+    a, b, res = rnd(M, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(M, n, seed=64)
+    wt, few = b.t().contiguous(), a[:m]
+    got = be.linear_fwd(few, b)
+    assert torch.equal(got, be.linear_fwd(a, b)[:m]) and rel(got, few.float() @ b.float().t()) <= TOL
+    assert torch.equal(be.linear_dgrad(few, wt), be.linear_dgrad(a, wt)[:m])
+    assert torch.equal(be.linear_fwd(few, b, residual=res[:m]), be.linear_fwd(a, b, residual=res)[:m])
+
+
 @pytest.mark.parametrize("m,n,k", [(3080, 2008, 2056), (1544, 4072, 2104), (6024, 1000, 1032), (5000, 1160, 4096), (4104, 1032, 1992)])
 def test_gemm_narrow_tiles_have_the_bits_of_wide_ones(be, m, n, k):
     """Outputs of fewer large tiles than compute units take narrower ones, down to 128 columns, whose transposed operand has a
