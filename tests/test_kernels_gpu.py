@@ -341,11 +341,11 @@ def test_gemm_smallest_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     assert torch.equal(dx[:, :n], big_dx[:m, :n]) and torch.equal(dx[:, n:], big_dx[:m, N:N + n])
 
 
-@pytest.mark.parametrize("m,n,k", [(776, 16384, 200), (1144, 32056, 72), (6024, 4096, 136), (6072, 4088, 64), (5200, 4360, 1096)])
-def test_gemm_tiles_of_fewer_rows_have_the_bits_of_the_large_ones(be, m, n, k):
-    """Outputs whose rows or rounds 224 or 192 rows divide better than 256: the first rows of an output of 8192, plain and with
-    a residual, with one K-step, two, three and many of them, the last one whole or partial."""
-    M = 8192
+@pytest.mark.parametrize("m,M,n,k", [(536, 1024, 16384, 72), (776, 1024, 16384, 200), (1600, 2048, 8192, 64), (3000, 4096, 4096, 136),
+                                     (3304, 4096, 4088, 1096), (6024, 7424, 4096, 136)])
+def test_gemm_tiles_of_fewer_rows_have_the_bits_of_the_large_ones(be, m, M, n, k):
+    """Outputs whose rows or rounds 224 or 192 rows divide better than 256: the first rows of an output of M, which takes 256,
+    plain and with a residual, with one K-step, two, three and many of them, the last one whole or partial."""
     a, b, res = rnd(M, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(M, n, seed=64)
     wt, few = b.t().contiguous(), a[:m]
     got = be.linear_fwd(few, b)
