@@ -105,7 +105,8 @@ class LayerConfig:
     made_streams: Optional[Tuple[Any, ...]] = field(default=None, repr=False)
 
     # Nanobatches on streams of their own cost the host 0.9-1.0 ms per nanobatch and layer, forward and backward
-    # (launches, and above all the event waits of the schedule points), one after the other on one stream 0.6 ms.
+    # (launches, and above all the event waits of the schedule points), one after the other on one stream 0.6 ms when this
+    # was measured (0.3-0.4 since the operators between two schedule points are one native call).
     # Where the device needs less than that for a nanobatch, the streams' overlap hides nothing and the step takes
     # as long as the host: on one stream it is shorter, and the GEMMs, alone on the device, are planned for
     # their latency (the attention keeps the forms the nanobatch count sets, see set_tensor_parallel_group: a run in
