@@ -580,10 +580,9 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 struct AttnGrads {
   Tensor fused, mixed, dq, dk, dv;
 };
-bool attn_bwd_ok(const AttnShape& c, const Tensor& dout, const Tensor& q, const Tensor& o, const Tensor& lse) {
-  return c.ok && q.dim() == 5 && dout.is_contiguous() && o.is_contiguous() && lse.is_contiguous() &&
-         dout.numel() == (int64_t)c.s * c.b * c.nq * c.hd && o.numel() == dout.numel() &&
-         lse.numel() == (int64_t)c.b * c.nq * c.s;
+bool attn_bwd_ok(const AttnShape& c, const Tensor& q, const Tensor& o, const Tensor& lse) {
+  return c.ok && q.dim() == 5 && o.is_contiguous() && lse.is_contiguous() &&
+         o.numel() == (int64_t)c.s * c.b * c.nq * c.hd && lse.numel() == (int64_t)c.b * c.nq * c.s;
 }
 int run_attn_bwd(const AttnShape& c, const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
                  const Tensor& lse, float scale, int flags, AttnGrads& g) {
@@ -615,7 +614,7 @@ PyObject* py_attn_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor &dout = tensor(a[0]), &q = tensor(a[1]), &k = tensor(a[2]), &v = tensor(a[3]), &o = tensor(a[4]),
                  &lse = tensor(a[5]);
     const AttnShape c = attn_shape(q, k, v);
-    if (!attn_bwd_ok(c, dout, q, o, lse)) return none();
+    if (!attn_bwd_ok(c, q, o, lse) || !dout.is_contiguous() || dout.numel() != o.numel()) return none();
     const float scale = (float)real(a[6]);
     const int flags = (int)integer(a[7]);
     AttnGrads g;
@@ -998,7 +997,7 @@ PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Tensor &q = tensor(a[2]), &k = tensor(a[3]), &v = tensor(a[4]), &o = tensor(a[5]), &lse = tensor(a[6]),
                  &freqs = tensor(a[8]), &wp = tensor(a[1]), &wq = tensor(a[15]);
     const AttnShape c = attn_shape(q, k, v);
-    if (!c.ok || q.dim() != 5) return none();
+    if (!attn_bwd_ok(c, q, o, lse)) return none();
     const int64_t t = (int64_t)c.s * c.b, wo = (int64_t)c.nq * c.hd, w = (int64_t)c.nkv * (c.per + 2) * c.hd, cols = wp.size(0),
                   h = wq.size(1);
     Operand od;
@@ -1032,7 +1031,6 @@ PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       }
     }
     if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, wo, cols, KR_GEMM_EPI_NONE, rc);
-    if (!attn_bwd_ok(c, dout, q, o, lse)) return failed(attn_name("kr_attn_bwd", c), KR_EINVAL);
     if (wgrad) release({a[7]});
     const char* what = "kr_attn_bwd";
     {

@@ -177,6 +177,21 @@ def test_chains_without_gradients_and_under_saved_tensor_hooks(monkeypatch):
     assert half and seen[:half] == seen[half:]     # the same tensors in the same order
 
 
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_saved_attention_output_with_gaps_runs_operator_by_operator(monkeypatch):
+    """(The native backward reads it dense; the answer comes before anything is launched.)"""
+    def with_gaps(t):
+        if t.shape != (96, 2, 4, 64):
+            return t
+        gaps.append(torch.empty(96, 2, 4, 128, dtype=t.dtype, device=t.device)[..., :64].copy_(t))
+        return gaps[-1]
+
+    gaps = []
+    ran = both(monkeypatch, config(), 96, 2, hooks=lambda: torch.autograd.graph.saved_tensors_hooks(lambda t: t, with_gaps))
+    assert gaps and ran.get("_BackwardAttention", 0) == 0 and ran["_BackwardMlp"] == 4
+
+
 @pytest.mark.parametrize("part", ["linear_fc1", "linear_proj", "pre_mlp_layernorm"])
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
