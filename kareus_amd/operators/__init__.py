@@ -10,6 +10,7 @@ from .qkv_postprocess import QKVPostProcessOp
 from .residual_fork import ResidualForkOp
 from .rmsnorm import PartitionableRMSNorm, RMSNorm
 from .rotary_embedding import RotaryEmbeddingOp, rotary_frequencies
+from . import chains  # noqa: F401  (loaded with the package: the engine asks for it inside a pass)
 
 __all__ = [
     "BiasDropoutAddOp",

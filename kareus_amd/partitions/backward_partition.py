@@ -25,10 +25,10 @@ class BackwardPartition(PartitionBase):
     # as one call; the numbers are those of the separate calls
     fuse_backward_ops: bool = True
 
-    def _chain_at(self, plans, at: int):
-        from ..operators.chains import backward_chain
+    def _find_chains(self, plans):
+        from ..operators.chains import backward_chains
 
-        return backward_chain(plans, at)
+        return backward_chains(plans)
 
     def execute(
         self,

@@ -23,10 +23,10 @@ class ForwardPartition(PartitionBase):
     # call; the numbers are those of the separate calls
     fuse_forward_ops: bool = True
 
-    def _chain_at(self, plans, at: int):
-        from ..operators.chains import forward_chain
+    def _find_chains(self, plans):
+        from ..operators.chains import forward_chains
 
-        return forward_chain(plans, at)
+        return forward_chains(plans)
 
     def execute(self, ctx: NanoBatchContext, pre_ctx: NanoBatchContext) -> None:
         with self._on_stream(ctx), self._timed():

@@ -97,7 +97,7 @@ class _OpPlan:
     __slots__ = ("op", "operator", "op_id", "in_ids", "first_in", "extra_ids", "out_ids", "first_out", "extra_out_ids",
                  "forward_pair", "backward_pair")
 
-    def __init__(self, op: ComputeOp, nxt: Optional[ComputeOp]) -> None:
+    def __init__(self, op: ComputeOp, nxt: Optional["_OpPlan"]) -> None:
         self.op, self.operator, self.op_id = op, op.operator, op.op_id
         self.in_ids = tuple(op.get_input_tensor_ids())
         self.out_ids = tuple(op.get_output_tensor_ids())
@@ -105,7 +105,7 @@ class _OpPlan:
         self.first_out, self.extra_out_ids = self.out_ids[0] if self.out_ids else None, self.out_ids[1:]
         self.forward_pair = self.backward_pair = False
         if nxt is not None:
-            nxt_ins, nxt_outs = nxt.get_input_tensor_ids(), nxt.get_output_tensor_ids()
+            nxt_ins, nxt_outs = nxt.in_ids, nxt.out_ids
             meets = bool(self.out_ids) and bool(nxt_ins) and nxt_ins[0] == self.out_ids[0]
             self.forward_pair = (meets and len(self.out_ids) == 1 and len(nxt_ins) == 1 and len(nxt_outs) == 1
                                  and hasattr(op.operator, "can_fuse_forward_with"))
@@ -150,13 +150,18 @@ class PartitionBase:
         # (an op of the list, or an op's operator, may have been replaced since the last pass)
         if plans is None or len(plans) != len(ops) or any(
                 [p.op is not op or p.operator is not op.operator for p, op in zip(plans, ops)]):
-            plans = self._op_plans = [_OpPlan(op, ops[i + 1] if i + 1 < len(ops) else None) for i, op in enumerate(ops)]
+            plans, nxt = [], None
+            for op in reversed(ops):   # (each looks at the one behind it)
+                nxt = _OpPlan(op, nxt)
+                plans.append(nxt)
+            plans.reverse()
+            self._op_plans = plans
             # the operator sequences that can run as one native call, by the index they start at (operators/chains.py)
-            self._op_chains = [self._chain_at(plans, i) for i in range(len(plans))]
+            self._op_chains = self._find_chains(plans)
         return plans
 
-    def _chain_at(self, plans: List[_OpPlan], at: int):
-        return None
+    def _find_chains(self, plans: List[_OpPlan]) -> List[Any]:
+        return [None] * len(plans)
 
     def _here(self):
         """The stream the schedule point is told about; None for a slot without a stream of its own (one
