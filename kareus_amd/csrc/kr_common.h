@@ -70,10 +70,10 @@ __device__ __forceinline__ float kr_swiglu_f(float gate, float up) { return gate
 // SwiGLU backward on one element: upstream gradient gy, forward inputs (gate, up) -> gradients.
 __device__ __forceinline__ void kr_swiglu_bwd_f(float gy, float gate, float up, float& d_gate, float& d_up) {
   const float sg = kr_sigmoidf(gate);
-  // (gy sg and gy sg gate serve both gradients: nine instructions, where the products written out are eleven)
-  const float t = gy * sg;
-  d_up = t * gate;
-  d_gate = (t + d_up * (1.0f - sg)) * up;
+  // (written out: with gy sg gate shared by both, d_gate is inf (1 - sg) = NaN, or inf, where gy sg gate overflows and it
+  // does not; the two instructions less were within the scatter of whole steps, 0.997-1.003)
+  d_gate = gy * sg * (1.0f + gate * (1.0f - sg)) * up;
+  d_up = gy * gate * sg;
 }
 
 static inline bool kr_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -133,6 +133,23 @@ def test_swiglu(be, rows, f):
     assert torch.isfinite(be.swiglu_fwd(big)).all() and be.swiglu_fwd(big).abs().max() < 1e-8
 
 
+def test_swiglu_gradient_of_a_gate_is_finite_where_that_of_its_up_value_is_not(be):
+    """gy gate sigmoid(gate) above the largest float, gy sigmoid(gate) (1 + ..) up below it: on its own and in the epilogue of the
+    input gradient (one row of the weight holds gy, so the product is gy exactly)."""
+    gy, f = 3.0e38, 64
+    gate = torch.tensor([4.0, 16.0, 20.0, 88.0]).repeat(f // 4)
+    x = torch.cat([gate, torch.full((f,), 0.5)]).repeat(8, 1).to(DEV, torch.bfloat16)
+    dy = torch.full((8, f), gy, device=DEV, dtype=torch.bfloat16)
+    g, top = gate.double(), dy[0].double().cpu()
+    want = top * torch.sigmoid(g) * (1.0 + g * (1.0 - torch.sigmoid(g))) * 0.5
+    one, w = torch.zeros(8, 8, device=DEV, dtype=torch.bfloat16), torch.zeros(8, f, device=DEV, dtype=torch.bfloat16)
+    one[:, 0], w[0] = 1.0, gy
+    for dx in (be.swiglu_bwd(dy, x), be.linear_dgrad(one, w, swiglu_bwd_x=x)):
+        d_gate, d_up = dx[:, :f].double().cpu(), dx[:, f:].double().cpu()
+        assert ((d_gate - want).abs() <= 2.0 ** -8 * want).all()   # one rounding to bf16, and fp32's
+        assert (d_up == math.inf).all()
+
+
 @pytest.mark.parametrize("s,b,heads,hd", [(256, 2, 8, 128), (64, 1, 3, 64), (4096, 1, 2, 128)])
 def test_rope(be, s, b, heads, hd):
     t = rnd(s, b, heads, hd, seed=5)
