@@ -60,9 +60,13 @@ size_t kr_gemm_workspace_bytes(int layout, int M, int N, int K);
  * value, so that the cuts the dispatcher plans are the cuts the buffer holds.  kr_gemm_bf16 uses
  * as many splits as the workspace it is handed holds, at most the planned count.              */
 size_t kr_gemm_workspace_bytes_shared(int layout, int M, int N, int K, float latency_weight);
-/* What a launch of this size is planned as (for tests and for reading profiles): the rows of an output tile, 256,
- * or 128 for the small tiles (128 x 128, 128 x 64 and 64 x 64), and the cuts of the contraction.  epilogue, max_cus and workspace_bytes (0: none) as in the
- * calls below.                                                                                  */
+/* What a launch of this size is planned as (for tests and for reading profiles): the rows and columns of C that a
+ * workgroup computes at a time (256 x 128 to 256 in steps of 32, either way round in layout NT; 224 or 192 x 256; 128 x 128;
+ * 128 x 64; 64 x 64) and the pieces that the contraction is summed in.  Dense operands of the layout; epilogue, accumulate,
+ * max_cus and workspace_bytes (0: none) as in the calls below.  kr_gemm_plan: the rows and pieces of a product that is stored,
+ * in layout TN (NN with KR_GEMM_EPI_SWIGLU_BWD).                                                  */
+int kr_gemm_plan_tile(int layout, int M, int N, int K, int epilogue, int accumulate, int max_cus, size_t workspace_bytes,
+                      int* tile_rows, int* tile_cols, int* splits);
 int kr_gemm_plan(int M, int N, int K, int epilogue, int max_cus, size_t workspace_bytes, int* tile_rows, int* splits);
 int kr_gemm_bf16(int layout, int M, int N, int K,
                  const void* A, int64_t lda, const void* B, int64_t ldb,

@@ -1443,17 +1443,63 @@ Plan launch_plan(int M, int N, int K, int epi, bool shared, int cus, size_t held
   return choose_plan(M, N, K, shared ? 0.1f : 1.f, cus, max_splits, epi != KR_GEMM_EPI_NONE,
                      epi != KR_GEMM_EPI_SWIGLU || N % 128 == 0);
 }
+// What a call is launched as: the plan, the tile that the layout and the output leave of it, operands exchanged or not.
+struct Choice {
+  int wn, splits;
+  Tile tile;
+  bool transposed;
+};
+// plain: no row runs and no accumulation; may_exchange: layout NT, a plain store and an operand A that can stand in B's place
+Choice choose_launch(int layout, int M, int N, int K, int epi, bool shared, int cus, size_t held_bytes, bool plain, bool may_exchange) {
+  const Plan plan = launch_plan(M, N, K, epi, shared, cus, held_bytes);
+  Choice c{epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn, epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.tile, false};
+  const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  if (c.tile == kLarge && plain && layout != KR_GEMM_NT && (epi == KR_GEMM_EPI_NONE || epi == KR_GEMM_EPI_ADD) && plan.splits == 1 && tiles >= 192)
+    c.tile = fewer_rows(M, N, c.wn, cus);
+  // Both operands of layout NT are read the same way, so C^T = B^T . A is the same kernel
+  // with the operands exchanged and a transposing store.  Take that form when its tile grid
+  // needs fewer rounds of workgroups (fc1's weight gradient, 7168 x 4096: 448 tiles of
+  // 256 x 256 are two rounds on 224 units; transposed, 512 tiles of 256 x 224 are two full
+  // rounds of smaller tiles).  Only for a plain store: accumulation and split-K keep the
+  // direct form.
+  if (may_exchange && tiles >= 192 && ((N + BM - 1) / BM) * ((M + BN - 1) / BN) >= 192) {
+    auto cost = [&](int rows, int cols, int w) {
+      const int t = ((rows + BM - 1) / BM) * ((cols + 32 * w - 1) / (32 * w));
+      return (long)((t + cus - 1) / cus) * (w + 1);
+    };
+    const int wt = choose_wn(N, M, cus);
+    if (cost(N, M, wt) < cost(M, N, c.wn)) return {wt, 1, kLarge, true};
+  }
+  return c;
+}
+// the same for dense operands, and the rows and columns of C that a workgroup computes at a time
+Choice planned(int layout, int M, int N, int K, int epilogue, int accumulate, int max_cus, size_t workspace_bytes, int* rows, int* cols) {
+  const int num_cus = device_compute_units();
+  const Choice c = choose_launch(layout, M, N, K, epilogue & ~KR_GEMM_BESIDE_OTHER_STREAMS, (epilogue & KR_GEMM_BESIDE_OTHER_STREAMS) != 0,
+                                 max_cus > 0 && max_cus < num_cus ? max_cus : num_cus, workspace_bytes, !accumulate,
+                                 layout == KR_GEMM_NT && !accumulate && (int64_t)M * M < ((int64_t)1 << 31) && M <= (1 << 26));
+  constexpr int rows_of[] = {BM, 128, 128, 64, 224, 192}, cols_of[] = {0, 128, 64, 64, BN, BN};  // (by Tile)
+  *rows = c.transposed ? 32 * c.wn : rows_of[c.tile];
+  *cols = c.transposed ? BM : c.tile == kLarge ? 32 * c.wn : cols_of[c.tile];
+  return c;
+}
 }  // namespace
+
+extern "C" int kr_gemm_plan_tile(int layout, int M, int N, int K, int epilogue, int accumulate, int max_cus, size_t workspace_bytes,
+                                 int* tile_rows, int* tile_cols, int* splits) {
+  if (!tile_rows || !tile_cols || !splits || M <= 0 || N <= 0 || K <= 0 || max_cus < 0 || layout < KR_GEMM_TN || layout > KR_GEMM_NT)
+    return KR_EINVAL;
+  if ((epilogue & ~KR_GEMM_BESIDE_OTHER_STREAMS) == KR_GEMM_EPI_SWIGLU && swiglu_wn(M, N, 256) == 0) return KR_EUNSUPPORTED;
+  *splits = planned(layout, M, N, K, epilogue, accumulate, max_cus, workspace_bytes, tile_rows, tile_cols).splits;
+  return KR_OK;
+}
 
 extern "C" int kr_gemm_plan(int M, int N, int K, int epilogue, int max_cus, size_t workspace_bytes, int* tile_rows,
                             int* splits) {
   if (!tile_rows || !splits || M <= 0 || N <= 0 || K <= 0 || max_cus < 0) return KR_EINVAL;
-  const int num_cus = device_compute_units();
-  const Plan plan = launch_plan(M, N, K, epilogue & ~KR_GEMM_BESIDE_OTHER_STREAMS,
-                                (epilogue & KR_GEMM_BESIDE_OTHER_STREAMS) != 0,
-                                max_cus > 0 && max_cus < num_cus ? max_cus : num_cus, workspace_bytes);
-  *tile_rows = plan.tile != kLarge ? 32 * WT_SMALL : 32 * WT_LARGE;
-  *splits = plan.splits;
+  const bool backward = (epilogue & ~KR_GEMM_BESIDE_OTHER_STREAMS) == KR_GEMM_EPI_SWIGLU_BWD;
+  int cols = 0;
+  *splits = planned(backward ? KR_GEMM_NN : KR_GEMM_TN, M, N, K, epilogue, 0, max_cus, workspace_bytes, tile_rows, &cols).splits;
   return KR_OK;
 }
 
@@ -1521,15 +1567,11 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
   // cuts of the contraction the caller's workspace can hold (a caller that wants fewer says so by
   // passing the smaller workspace kr_gemm_workspace_bytes_shared sizes); a fused epilogue works on
   // finished sums and is never cut
-  const Plan plan = launch_plan(M, N, K, fu.epi, fu.shared, cus, ws != nullptr && fu.runs.c_sh == 0 ? workspace_bytes : 0);
-  const int wn = fu.epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn;
-  Tile tile = plan.tile;
-  const bool plain = fu.runs.a_sh == 0 && fu.runs.c_sh == 0 && fu.runs.x_sh == 0 && !accumulate;
-  if (tile == kLarge && plain && layout != KR_GEMM_NT && (fu.epi == KR_GEMM_EPI_NONE || fu.epi == KR_GEMM_EPI_ADD) && plan.splits == 1 &&
-      ((M + BM - 1) / BM) * ((N + BN - 1) / BN) >= 192)
-    tile = fewer_rows(M, N, wn, cus);
-  const Call call{a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, wn,
-                  fu.epi == KR_GEMM_EPI_NONE ? plan.splits : 1, tile, false};
+  const bool stored = !accumulate && fu.runs.a_sh == 0 && fu.runs.c_sh == 0;
+  const Choice c_of = choose_launch(layout, M, N, K, fu.epi, fu.shared, cus, ws != nullptr && fu.runs.c_sh == 0 ? workspace_bytes : 0,
+                                    stored && fu.runs.x_sh == 0,
+                                    layout == KR_GEMM_NT && stored && (int64_t)M * lda < ((int64_t)1 << 31) && M <= (1 << 26));
+  const Call call{a, lda, b, ldb, c, ldc, M, N, K, accumulate, ws, workspace_bytes, st, num_cus, c_of.wn, c_of.splits, c_of.tile, false};
   switch (layout) {
     case KR_GEMM_TN:  // A [M,K], B [N,K]
       if (lda < K || ldb < K || ldc < N) return KR_EINVAL;
@@ -1539,36 +1581,20 @@ int gemm_dispatch(int layout, int M, int N, int K, const void* A, int64_t lda, c
       return launch_nn(call, fu);
     case KR_GEMM_NT: {  // A [K,M], B [K,N]
       if (lda < M || ldb < N || ldc < N) return KR_EINVAL;
-      // Both operands of this layout are read the same way, so C^T = B^T . A is the same kernel
-      // with the operands exchanged and a transposing store.  Take that form when its tile grid
-      // needs fewer rounds of workgroups (fc1's weight gradient, 7168 x 4096: 448 tiles of
-      // 256 x 256 are two rounds on 224 units; transposed, 512 tiles of 256 x 224 are two full
-      // rounds of smaller tiles).  Only for a plain store: accumulation and split-K keep the
-      // direct form.
-      if (!accumulate && fu.runs.a_sh == 0 && fu.runs.c_sh == 0 && ((int64_t)M * lda < ((int64_t)1 << 31)) && M <= (1 << 26)) {
-        auto cost = [&](int rows, int cols, int w) {
-          const int tiles = ((rows + BM - 1) / BM) * ((cols + 32 * w - 1) / (32 * w));
-          return (long)((tiles + cus - 1) / cus) * (w + 1);
-        };
-        const int wt = choose_wn(N, M, cus);
-        const int tiles_direct = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-        const int tiles_trans = ((N + BM - 1) / BM) * ((M + BN - 1) / BN);
-        if (tiles_direct >= 192 && tiles_trans >= 192 && cost(N, M, wt) < cost(M, N, wn)) {
-          // (operand pieces change places with the operands)
-          Segments exchanged{};
-          Fused fut = fu;
-          if (fu.segs != nullptr) {
-            for (int i = 0; i < MAX_SEGMENTS; ++i) {
-              exchanged.a[i] = fu.segs->b[i];
-              exchanged.b[i] = fu.segs->a[i];
-            }
-            exchanged.n = fu.segs->n;
-            exchanged.steps = fu.segs->steps;
-            fut.segs = &exchanged;
+      if (c_of.transposed) {  // (operand pieces change places with the operands)
+        Segments exchanged{};
+        Fused fut = fu;
+        if (fu.segs != nullptr) {
+          for (int i = 0; i < MAX_SEGMENTS; ++i) {
+            exchanged.a[i] = fu.segs->b[i];
+            exchanged.b[i] = fu.segs->a[i];
           }
-          const Call exchanged_call{b, ldb, a, lda, c, ldc, N, M, K, 0, nullptr, 0, st, num_cus, wt, 1, kLarge, true};
-          return launch_nt(exchanged_call, fut);
+          exchanged.n = fu.segs->n;
+          exchanged.steps = fu.segs->steps;
+          fut.segs = &exchanged;
         }
+        const Call exchanged_call{b, ldb, a, lda, c, ldc, N, M, K, 0, nullptr, 0, st, num_cus, c_of.wn, 1, kLarge, true};
+        return launch_nt(exchanged_call, fut);
       }
       return launch_nt(call, fu);
     }

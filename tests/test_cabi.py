@@ -222,11 +222,11 @@ def test_a_gemm_is_planned_the_same_in_the_workspace_it_asks_for():
                         bytes_ = (lib.kr_gemm_workspace_bytes_shared(0, m, n, k, 0.1) if shared
                                   else lib.kr_gemm_workspace_bytes(0, m, n, k))
                         free = plan(m, n, k, shared, 16 * m * n * 4)
-                        seen.add((free[0], free[1] > 1))
+                        seen.add((free[0] <= 128, free[1] > 1))
                         if shared and bytes_ < free[1] * m * n * 4 and free[1] > 1:
                             continue                      # (never more cuts than the launch would take alone)
                         assert plan(m, n, k, shared, bytes_) == free, (m, n, k, shared)
-    assert seen == {(128, False), (128, True), (256, False), (256, True)}
+    assert seen == {(True, False), (True, True), (False, False), (False, True)}
     # long contractions of a few more small tiles than compute units go to the large tile in cuts, short ones do not
     for shape, rows in (((1536, 3072, 6024), 256), ((640, 7168, 7008), 256), ((1536, 3072, 2048), 128)):
         assert plan(*shape, 0, 16 * shape[0] * shape[1] * 4)[0] == rows
@@ -237,3 +237,29 @@ def test_a_gemm_is_planned_the_same_in_the_workspace_it_asks_for():
     for shape, flags, rows in (((152, 4096, 7168), 0x100, 256), ((4096, 1536, 6024), 0, 256), ((768, 7168, 8192), 0, 256),
                                ((1024, 1024, 512), 0x100, 128), ((512, 4096, 3584), 0, 128)):
         assert plan(*shape, flags, 16 * shape[0] * shape[1] * 4)[0] == rows
+
+
+def test_the_plan_names_the_tile_that_runs():
+    """Rows and columns of a workgroup's part of C, by layout and kind of output (device of 256 compute units)."""
+    lib = hip.load_library()
+
+    def tile(layout, m, n, k, epilogue=0, accumulate=0, max_cus=0, workspace=0):
+        got = [ctypes.c_int() for _ in range(3)]
+        assert lib.kr_gemm_plan_tile(layout, m, n, k, epilogue, accumulate, max_cus, workspace, *[ctypes.byref(v) for v in got]) == 0
+        rows, cuts = ctypes.c_int(), ctypes.c_int()
+        if layout == (1 if epilogue == 4 else 0) and not accumulate:
+            assert lib.kr_gemm_plan(m, n, k, epilogue, max_cus, workspace, ctypes.byref(rows), ctypes.byref(cuts)) == 0
+            assert (rows.value, cuts.value) == (got[0].value, got[2].value)
+        return got[0].value, got[1].value
+
+    assert tile(0, 16384, 4096, 4096) == (256, 256)
+    assert tile(0, 776, 32064, 4096) == (224, 256) and tile(0, 776, 32064, 4096, accumulate=1) != (224, 256)
+    assert tile(0, 6024, 4096, 3584, 1) == tile(1, 6024, 4096, 7168) == (192, 256)
+    assert tile(0, 6024, 4096, 3584, accumulate=1)[0] == tile(2, 6024, 4096, 7168, accumulate=1)[0] == 256
+    assert tile(0, 776, 4096, 3584, 1) == (128, 128) and tile(0, 512, 4096, 3584, 1) == (128, 64) and tile(0, 128, 4096, 3584, 1) == (64, 64)
+    assert tile(1, 512, 3584, 4096, 4) == (128, 64) and tile(0, 1024, 1024, 512, 0x100) == (128, 128)
+    assert tile(2, 7168, 4096, 16384) == (224, 256)           # operands exchanged: rows of C are the narrow side
+    out = [ctypes.byref(ctypes.c_int()) for _ in range(3)]
+    assert lib.kr_gemm_plan_tile(3, 64, 64, 64, 0, 0, 0, 0, *out) == lib.kr_gemm_plan_tile(0, 0, 64, 64, 0, 0, 0, 0, *out) == -1
+    assert lib.kr_gemm_plan_tile(0, 64, 64, 64, 0, 0, 0, 0, None, None, None) == -1
+    assert lib.kr_gemm_plan_tile(0, 64, 2 * 64, 64, 2, 0, 0, 0, *out) == -2      # no tile of the SwiGLU epilogue divides this width

@@ -300,12 +300,19 @@ def _gemm_plan(be, m, n, k, epilogue=0, workspace=0):
     return rows.value, splits.value
 
 
+def _gemm_tile(be, layout, m, n, k, epilogue=0, accumulate=0, max_cus=0, workspace=0):
+    rows, cols, pieces = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert be.lib.kr_gemm_plan_tile(layout, m, n, k, epilogue, accumulate, max_cus, workspace, ctypes.byref(rows), ctypes.byref(cols),
+                                    ctypes.byref(pieces)) == 0
+    return rows.value, cols.value, pieces.value
+
+
 @pytest.mark.parametrize("m,n,k", [(8, 8, 8), (128, 128, 64), (136, 264, 72), (120, 128, 128), (520, 1024, 200),
                                    (264, 136, 584), (136, 640, 720), (256, 1000, 1096),   # the deep ring, contraction tails
                                    (512, 3584, 1024),     # one round of small tiles, more than one per compute unit
                                    (2048, 3456, 136)])    # 432 small tiles
 def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
-    """Outputs of few tiles are computed in 128 x 128 tiles.  The same rows and columns as a corner of an output of 192
+    """Outputs of few tiles are computed in tiles of 128 rows or 64.  The same rows and columns as a corner of an output of 192
     and more large tiles, which is computed in them: every element is the same chain of matrix instructions in both, so
     the bits are the same.  (Both plans are asserted.)"""
     def embed(t, rows=None, cols=None):
@@ -318,7 +325,8 @@ def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     x, w, dy = rnd(m, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(m, n, seed=63)
     for layout, a, b, (p, q, c) in ((0, x, w, (m, n, k)), (1, dy, w, (m, k, n)), (2, dy, x, (n, k, m))):
         big = (max(p, R_), max(q, C_), c)
-        assert _gemm_plan(be, p, q, c) == (128, 1) and _gemm_plan(be, *big) == (256, 1)
+        rows, cols, pieces = _gemm_tile(be, layout, p, q, c)
+        assert rows <= 128 and cols <= 128 and pieces == 1 and max(_gemm_tile(be, layout, *big)[:2]) == 256
         big_a = embed(a, cols=R_) if layout == 2 else embed(a, rows=R_)
         big_b = embed(b, rows=C_) if layout == 0 else embed(b, cols=C_)
         got = be.gemm(layout, a, b, p, q, c, split_k=None)
@@ -332,43 +340,75 @@ def test_gemm_small_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
     assert rel(be.linear_fwd(x, w), x.float() @ w.float().t()) <= TOL
     big_x, big_w, big = embed(x, rows=R_), embed(w, rows=C_), (max(m, R_), max(n, C_), k)
     res = rnd(m, n, seed=65)
-    assert _gemm_plan(be, m, n, k, 1)[0] == 128 and _gemm_plan(be, *big, 1)[0] == 256
+    assert _gemm_plan(be, m, n, k, 1)[0] <= 128 and _gemm_plan(be, *big, 1)[0] == 256
     assert torch.equal(be.linear_fwd(x, w, residual=res), be.linear_fwd(big_x, big_w, residual=embed(res, R_, C_))[:m, :n])
 
 
-@pytest.mark.parametrize("m,n,k", [(8, 8, 8), (64, 64, 64), (72, 136, 1096), (200, 328, 264), (128, 4096, 200), (520, 3208, 584), (1000, 512, 2752),
-                                   (264, 1376, 256)])
-def test_gemm_smallest_tiles_have_the_bits_of_the_large_ones(be, m, n, k):
-    """Outputs that would leave compute units without a tile of 128 x 128 are computed in 128 x 64 or 64 x 64 tiles: every layout
-    and kind of output against a corner of an output of 192 large tiles, at contractions shorter than the ring and longer."""
-    M, N = 4096, 3072 if n <= 3072 else 4096
+@pytest.mark.parametrize("m,n,k,tile", [(8, 8, 8, (64, 64)), (64, 64, 64, (64, 64)), (72, 136, 1096, (64, 64)), (200, 328, 264, (64, 64)),
+                                        (128, 4096, 200, (64, 64)), (520, 3208, 584, (128, 64)), (1000, 512, 2752, (64, 64)),
+                                        (264, 1376, 256, (64, 64)),
+                                        # more tiles than compute units, or one per unit and short or deep rings of K-steps
+                                        (2008, 3456, 200, (128, 128)), (1000, 5000, 1096, (128, 128)), (520, 5000, 72, (128, 128)),
+                                        (776, 4096, 584, (128, 128)), (776, 2952, 1096, (128, 128)), (904, 4096, 2056, (128, 128))])
+def test_gemm_smallest_tiles_have_the_bits_of_the_large_ones(be, m, n, k, tile):
+    """Outputs of few tiles are computed in 128 x 128 tiles, those that would leave compute units without one in 128 x 64 or
+    64 x 64: every layout and kind of output against a corner of an output of 192 large tiles, at contractions shorter than the
+    ring and longer.  (What runs is asserted.)"""
+    M, N = 4096, 3072 if n <= 3072 else 4096 if n <= 4096 else 5120
     a, b, old, res = rnd(M, k, seed=61), rnd(N, k, scale=0.05, seed=62), rnd(M, N, seed=63), rnd(M, N, seed=64)
+
+    def asserted(layout, epilogue=0, accumulate=0):
+        assert _gemm_tile(be, layout, m, n, k, epilogue, accumulate) == (*tile, 1)
+        assert max(_gemm_tile(be, layout, M, N, k, epilogue, accumulate)[:2]) == 256
+
     for layout, f, g in ((0, lambda t: t, lambda t: t), (1, lambda t: t, lambda t: t.t().contiguous()),
                          (2, lambda t: t.t().contiguous(), lambda t: t.t().contiguous())):
         big, few = (layout, f(a), g(b), M, N, k), (layout, f(a[:m]), g(b[:n]), m, n, k)
+        asserted(layout)
         assert torch.equal(be.gemm(*few, split_k=None), be.gemm(*big, split_k=None)[:m, :n])
+        asserted(layout, accumulate=1)
         acc = [be.gemm(*c, out=o.clone(), accumulate=True, split_k=None) for c, o in ((few, old[:m, :n]), (big, old))]
         assert torch.equal(acc[0], acc[1][:m, :n])
     assert rel(be.linear_fwd(a[:m], b[:n]), a[:m].float() @ b[:n].float().t()) <= TOL
+    asserted(0, 1)
     assert torch.equal(be.linear_fwd(a[:m], b[:n], residual=res[:m, :n]), be.linear_fwd(a, b, residual=res)[:m, :n])
     wt = b.t().contiguous()
     pre = rnd(M, 2 * N, seed=65)
     few_pre = torch.cat([pre[:m, :n], pre[:m, N:N + n]], dim=1)
+    asserted(1, 4)
     dx, big_dx = (be.linear_dgrad(x, w, swiglu_bwd_x=p) for x, w, p in ((a[:m], wt[:, :n].contiguous(), few_pre), (a, wt, pre)))
     assert torch.equal(dx[:, :n], big_dx[:m, :n]) and torch.equal(dx[:, n:], big_dx[:m, N:N + n])
 
 
-@pytest.mark.parametrize("m,M,n,k", [(536, 1024, 16384, 72), (776, 1024, 16384, 200), (1600, 2048, 8192, 64), (3000, 4096, 4096, 136),
-                                     (3304, 4096, 4088, 1096), (6024, 7424, 4096, 136)])
-def test_gemm_tiles_of_fewer_rows_have_the_bits_of_the_large_ones(be, m, M, n, k):
+@pytest.mark.parametrize("m,M,n,k,rows", [(536, 1024, 16384, 72, 192), (776, 1024, 16384, 200, 224), (1600, 2048, 8192, 64, 224),
+                                          (3000, 4096, 4096, 136, 192), (6024, 7424, 4096, 136, 192),
+                                          # a partial last column of tiles, many K-steps with a partial last one
+                                          (776, 1024, 16360, 1096, 224), (1600, 2048, 8136, 1096, 224), (536, 1024, 16328, 1096, 192),
+                                          (3000, 4096, 4088, 1096, 192)])
+def test_gemm_tiles_of_fewer_rows_have_the_bits_of_the_large_ones(be, m, M, n, k, rows):
     """Outputs whose rows or rounds 224 or 192 rows divide better than 256: the first rows of an output of M, which takes 256,
-    plain and with a residual, with one K-step, two, three and many of them, the last one whole or partial."""
+    plain and with a residual, with one K-step, two, three and many of them, the last one whole or partial.  (What runs is
+    asserted.)"""
+    for layout, epilogue in ((0, 0), (1, 0), (0, 1)):
+        assert _gemm_tile(be, layout, m, n, k, epilogue) == (rows, 256, 1) and _gemm_tile(be, layout, M, n, k, epilogue) == (256, 256, 1)
     a, b, res = rnd(M, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(M, n, seed=64)
     wt, few = b.t().contiguous(), a[:m]
     got = be.linear_fwd(few, b)
     assert torch.equal(got, be.linear_fwd(a, b)[:m]) and rel(got, few.float() @ b.float().t()) <= TOL
     assert torch.equal(be.linear_dgrad(few, wt), be.linear_dgrad(a, wt)[:m])
     assert torch.equal(be.linear_fwd(few, b, residual=res[:m]), be.linear_fwd(a, b, residual=res)[:m])
+
+
+@pytest.mark.parametrize("m,n,k,rows", [(3000, 4088, 1096, 192), (3000, 4088, 136, 192), (1600, 8136, 1096, 224), (1600, 8136, 72, 224)])
+def test_gemm_tiles_of_fewer_rows_several_to_a_workgroup(be, m, n, k, rows):
+    """On half the compute units a workgroup has two such tiles, on all of them one: the same bits."""
+    a, b, res = rnd(m, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(m, n, seed=64)
+    for layout, w, what in ((0, b, {}), (1, b.t().contiguous(), {}), (0, b, dict(residual=res))):
+        got = []
+        for cus in (0, 128):
+            assert _gemm_tile(be, layout, m, n, k, 1 if what else 0, max_cus=cus) == (rows, 256, 1)
+            got.append(be.gemm(layout, a, w, m, n, k, split_k=None, max_cus=cus, **what))
+        assert torch.equal(*got)
 
 
 @pytest.mark.parametrize("m,n,k", [(3080, 2008, 2056), (1544, 4072, 2104), (6024, 1000, 1032), (5000, 1160, 4096), (4104, 1032, 1992)])
@@ -412,20 +452,24 @@ def test_gemm_items_of_one_workgroup_have_the_bits_of_items_of_their_own(be, k, 
     assert torch.equal(*x2) and torch.equal(*ys)
 
 
-@pytest.mark.parametrize("m,f,k", [(8, 64, 64), (128, 320, 128), (136, 448, 200), (520, 512, 1096), (512, 1792, 1024)])
-def test_gemm_small_tiles_with_swiglu_have_the_bits_of_the_large_ones(be, m, f, k):
+@pytest.mark.parametrize("m,f,k,forward,backward", [(8, 64, 64, (64, 64), (64, 64)), (128, 320, 128, (64, 64), (64, 64)),
+                                                    (136, 448, 200, (64, 64), (64, 64)), (520, 512, 1096, (64, 64), (64, 64)),
+                                                    (512, 1792, 1024, (128, 64), (64, 64)), (776, 2048, 584, (128, 128), (128, 64)),
+                                                    (1000, 1728, 1096, (128, 128), (128, 64)), (520, 2048, 2056, (128, 128), (128, 64)),
+                                                    (2008, 1536, 72, (128, 128), (128, 128))])
+def test_gemm_small_tiles_with_swiglu_have_the_bits_of_the_large_ones(be, m, f, k, forward, backward):
     """The SwiGLU epilogues, forward (gate and up columns of a tile side by side) and backward, in the same way."""
     M, F = max(m, 4096), max(3584, f)      # 16 x 28 large tiles: gate and up
     x, gate, up = rnd(M, k, seed=61), rnd(F, k, scale=0.05, seed=62), rnd(F, k, scale=0.05, seed=63)
     xs, ws = x[:m].contiguous(), torch.cat([gate[:f], up[:f]])
     if be.can_fuse_swiglu(2 * f):
-        assert _gemm_plan(be, m, 2 * f, k, 2)[0] == 128 and _gemm_plan(be, M, 2 * F, k, 2)[0] == 256
+        assert _gemm_tile(be, 0, m, 2 * f, k, 2) == (*forward, 1) and _gemm_plan(be, M, 2 * F, k, 2)[0] == 256
         y, big_y = (torch.empty(r, c, device=DEV, dtype=torch.bfloat16) for r, c in ((m, f), (M, F)))
         got, big = be.linear_fwd(xs, ws, swiglu_out=y), be.linear_fwd(x, torch.cat([gate, up]), swiglu_out=big_y)
         assert torch.equal(got[:, :f], big[:m, :f]) and torch.equal(got[:, f:], big[:m, F:F + f]) and torch.equal(y, big_y[:m, :f])
     # backward: the gradient of the activation, [m, f] = dy [m, k] . W [k, f], never stored; out [m, 2 f]
     dy, w, pre = rnd(M, k, seed=66), rnd(k, F, scale=0.05, seed=67), rnd(M, 2 * F, seed=68)
-    assert _gemm_plan(be, m, f, k, 4)[0] == 128 and _gemm_plan(be, M, F, k, 4)[0] == 256
+    assert _gemm_tile(be, 1, m, f, k, 4) == (*backward, 1) and _gemm_plan(be, M, F, k, 4)[0] == 256
     pre_s = torch.cat([pre[:m, :f], pre[:m, F:F + f]], dim=1)
     got = be.linear_dgrad(dy[:m].contiguous(), w[:, :f].contiguous(), swiglu_bwd_x=pre_s)
     big = be.linear_dgrad(dy, w, swiglu_bwd_x=pre)
