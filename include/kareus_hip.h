@@ -58,7 +58,8 @@ size_t kr_gemm_workspace_bytes(int layout, int M, int N, int K);
  * alone would take in its own output tile or in the large one.  A launch
  * flagged KR_GEMM_BESIDE_OTHER_STREAMS is planned with weight 0.1: size its workspace with that
  * value, so that the cuts the dispatcher plans are the cuts the buffer holds.  kr_gemm_bf16 uses
- * as many splits as the workspace it is handed holds, at most the planned count.              */
+ * as many splits as the workspace it is handed holds, at most the planned count.  (The smallest tiles
+ * write nothing there: they add up the same number of pieces in registers.)                     */
 size_t kr_gemm_workspace_bytes_shared(int layout, int M, int N, int K, float latency_weight);
 /* What a launch of this size is planned as (for tests and for reading profiles): the rows and columns of C that a
  * workgroup computes at a time (256 x 128 to 256 in steps of 32, either way round in layout NT; 224 or 192 x 256; 128 x 128;

@@ -379,6 +379,11 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
   // PARTIAL: fp32 partial tiles of a cut contraction.  ACCUMULATE: C += product, rounded once.
   constexpr bool split_k = EPI == KR_GEMM_OUT_PARTIAL, add_old = EPI == KR_GEMM_OUT_ACCUMULATE;
   constexpr bool narrow = !trans_out && !split_k && !add_old;
+  // 128 x 64 and 64 x 64 tiles take the whole contraction in one workgroup, but add it up in the pieces of k_per that larger
+  // tiles would be cut into (0: one piece): a product has the same bits whichever tile is taken.  16 or 32 registers more of
+  // the few hundred that such a tile leaves, and an addition per piece: 1024 x 512 x 2048 whole 9.1 us, in four pieces 9.8,
+  // cut into four ranges of 128 x 128 tiles 17.
+  constexpr bool in_pieces = WN == 2 && (EPI == KR_GEMM_EPI_NONE || add_old);
   static_assert(EPI == KR_GEMM_EPI_NONE || trans_out || swiglu_bwd || split_k || add_old || (!A_T && !B_T),
                 "residual / SwiGLU epilogues: K-major layout only");
   static_assert(!trans_out || (A_T && B_T), "transposed store: layout NT only");
@@ -660,6 +665,32 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     // half-step computes on Y while X is read from the tiles of t+1 and B(t+DEPTH) is requested
     // where A(t) was.
     int t = 0;
+    f32x4 done[in_pieces ? WT : 1][in_pieces ? WN : 1];  // the sum of the pieces behind the current one
+    int steps_left = in_pieces && k_per > 0 ? k_per / BK : nk + 1;
+    if constexpr (in_pieces) {
+#pragma unroll
+      for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) done[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto end_of_step = [&]() {
+      if constexpr (in_pieces) {
+        if (--steps_left == 0) {
+          steps_left = k_per / BK;
+          asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // (the MFMAs' results, as behind the K loop)
+#pragma unroll
+          for (int i = 0; i < WT; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+              asm volatile("" : "+a"(acc[i][j]));
+              done[i][j] += acc[i][j];
+              acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+              asm volatile("" : "+a"(acc[i][j]));
+            }
+          asm volatile("s_nop 7" ::: "memory");  // (written before the next MFMA reads them)
+        }
+      }
+    };
     for (; t + DEPTH < nk; ++t) {
       if (t + DEPTH + 1 == nk && k_tail != BK) set_offsets(k_tail);
       half(X, Y, ring[0], ring[1], 1, Count<NA_LOADS>{}, a_base(t + DEPTH), la, ring[NSLOTS - 1]);
@@ -668,6 +699,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       half(Y, X, ring[2], ring[3], 0, Count<NB_LOADS>{}, b_base(t + DEPTH), lb, ring[0]);
       seg_advance();
       rotate();
+      end_of_step();
     }
     const int out_m0 = m0, out_n0 = n0;
     float* const out_partial = split_k ? partial + p_off : nullptr;
@@ -714,6 +746,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       // (after the last K-step this reads tiles that do not exist: unused)
       half(Y, X, ring[2], ring[3], 0, Count<0>{}, nullptr, lb, 0u);
       rotate();
+      end_of_step();
     }
 
     // Every LDS read of this item that matters finished before the last barrier, so all slots but those of requests
@@ -725,6 +758,18 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
     // the compiler does not know the MFMAs' latency: let the last ones finish before their
     // results are read
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    if constexpr (in_pieces) {
+      if (k_per > 0) {
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+#pragma unroll
+          for (int j = 0; j < WN; ++j) {
+            asm volatile("" : "+a"(acc[i][j]));
+            acc[i][j] = done[i][j] + acc[i][j];
+            asm volatile("" : "+a"(acc[i][j]));
+          }
+      }
+    }
 
     // Epilogue.  A lane holds C[m][n..n+3] for m = 16 mt + lane%16, n = 16 nt + 4 (lane/16):
     // stored from there, every instruction would scatter 64 small pieces over 16 rows.  Instead
@@ -1052,7 +1097,7 @@ int launch(const Call& call, const Fused& fu) {
   // the planned count, which the dispatcher has already capped by what the caller's workspace holds
   int splits = call.splits;
   const size_t one = (size_t)M * N * sizeof(float);
-  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE || kOneRound || kFewRows) {
+  if (workspace == nullptr || EPI != KR_GEMM_EPI_NONE || kFewRows) {
     splits = 1;  // a fused epilogue works on finished sums
   } else if ((size_t)splits * one > workspace_bytes) {
     splits = (int)(workspace_bytes / one);
@@ -1134,15 +1179,15 @@ int launch(const Call& call, const Fused& fu) {
     if (!deep) pick(Count<kDepth>{});
   if (attr_status != hipSuccess) return KR_ELAUNCH;
   const Segments segs = with_segs ? *fu.segs : Segments{};
-  if (splits == 1) {
+  int k_per = (K + splits - 1) / splits;
+  k_per = (k_per + BK - 1) / BK * BK;
+  if (splits == 1 || kOneRound) {  // (one workgroup adds up all pieces of its tile)
     hipLaunchKernelGGL(fn, dim3(grid_for(tiles)), dim3(NTHREADS), lds_bytes, stream, A, (int)lda, B, (int)ldb, C,
-                       (int)ldc, M, N, K, accumulate, 0, 1, (float*)nullptr, fu.aux, (int)fu.ld_aux, fu.out2,
+                       (int)ldc, M, N, K, accumulate, splits == 1 ? 0 : k_per, 1, (float*)nullptr, fu.aux, (int)fu.ld_aux, fu.out2,
                        (int)fu.ld_out2, fu.runs, segs);
     return kr_launch_status();
   }
   if constexpr (EPI != KR_GEMM_EPI_NONE) return KR_EINVAL;  // (not reached: a fused launch never splits)
-  int k_per = (K + splits - 1) / splits;
-  k_per = (k_per + BK - 1) / BK * BK;
   splits = (K + k_per - 1) / k_per;
   const int items = tiles * splits;
   // (of the operands only A can be in runs here: an output in runs is never cut)
@@ -1359,7 +1404,7 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
   // K-step, use the units that would have none, as long as every tile has a unit.
   // Measured, small -> these, us: 512 x 4096 x 3584 with the residual 35 -> 26 (128 x 64), 512 x 3584 x 4096 (NN) with the SwiGLU
   // backward 42 -> 35, 128 x 4096 x 3584 31 -> 14 (64 x 64), 256 x 512 x 1376 16 -> 9, 384 x 1024 x 3072 (NN) with the SwiGLU backward 25 ->
-  // 13, 1024 x 512 x 2048 (two cuts) 17 -> 9; of 130 sizes none is slower.  In units as above: 0.21-0.42 us a K-step.
+  // 13, 1024 x 512 x 2048 (four cuts) 17 -> 10; of 130 sizes none is slower.  In units as above: 0.21-0.42 us a K-step.
   constexpr double kStepNarrow = 0.26, kStepTiny = 0.20, kOverheadNarrow = 2.5;
   Tile under = kSmall;
   double under_cost = 1e30;
@@ -1376,10 +1421,10 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
     try_tile(kTiny, 64, kStepTiny);
   }
   const double small = small_cost(small_cut(kSplit), kSplit);
-  if (std::min(small, under_cost) >= large * 0.93) return best;  // the change must be clear
-  if (under_cost < small) return {2, 1, under};
   // (beside other streams the extra launch is no compute-unit time: 384 x 640 x 4096 in two cuts 21 us, uncut 32)
-  return {4, small_cut(w * kSplit), kSmall};
+  const Plan in_tiles = small >= large * 0.93 ? best : Plan{4, small_cut(w * kSplit), kSmall};  // the change must be clear
+  if (under_cost >= small || under_cost >= large * 0.93) return in_tiles;
+  return {2, in_tiles.splits, under};  // (its sums in the pieces that they would be cut into)
 }
 
 // Tile width for a projection with the SwiGLU epilogue: the tiles have to divide the 2F output

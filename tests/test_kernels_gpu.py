@@ -380,6 +380,28 @@ def test_gemm_smallest_tiles_have_the_bits_of_the_large_ones(be, m, n, k, tile):
     assert torch.equal(dx[:, :n], big_dx[:m, :n]) and torch.equal(dx[:, n:], big_dx[:m, N:N + n])
 
 
+@pytest.mark.parametrize("m,n,k,cus", [(1024, 512, 2048, 120), (1000, 504, 1992, 116), (1000, 1000, 2056, 196), (256, 512, 1376, 12), (256, 512, 1376, 28), (504, 2040, 4104, 88),
+                                       (512, 2048, 4104, 248)])
+def test_gemm_smallest_tiles_add_up_the_pieces_that_larger_ones_are_cut_into(be, m, n, k, cus):
+    """A contraction that larger tiles would be cut into: the 128 x 64 and 64 x 64 tiles walk it whole and add it up in the same
+    pieces, in the same order.  Against the cut launch on fewer compute units (both plans are asserted), in every layout, stored,
+    accumulated and with the operands in pieces of their own."""
+    a, b, old = rnd(m, k, seed=61), rnd(n, k, scale=0.05, seed=62), rnd(m, n, seed=64)
+    ws = be.lib.kr_gemm_workspace_bytes(0, m, n, k)
+    for layout, x, w in ((0, a, b), (1, a, b.t().contiguous()), (2, a.t().contiguous(), b.t().contiguous())):
+        for acc in (False, True):
+            whole, cut = (_gemm_tile(be, layout, m, n, k, 0, acc, c, ws) for c in (0, cus))
+            assert whole[:2] == (64, 64) and cut[0] * cut[1] > 64 * 64 and whole[2] == cut[2] > 1
+            got = [be.gemm(layout, x, w, m, n, k, max_cus=c, **(dict(out=old.clone(), accumulate=True) if acc else {})) for c in (0, cus)]
+            assert torch.equal(*got)
+            assert rel(got[0], a.float() @ b.float().t() + (old.float() if acc else 0.0)) <= TOL
+    if k % 64 == 0:
+        x, w = a.t().contiguous(), b.t().contiguous()
+        half = k // 128 * 64
+        if 2 * half == k:
+            assert torch.equal(be.linear_wgrad_segments([x[:half], x[half:]], [w[:half], w[half:]]), be.gemm(2, x, w, m, n, k))
+
+
 @pytest.mark.parametrize("m,M,n,k,rows", [(536, 1024, 16384, 72, 192), (776, 1024, 16384, 200, 224), (1600, 2048, 8192, 64, 224),
                                           (3000, 4096, 4096, 136, 192), (6024, 7424, 4096, 136, 192),
                                           # a partial last column of tiles, many K-steps with a partial last one
