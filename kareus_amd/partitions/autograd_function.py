@@ -203,7 +203,8 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
         in_line = _nanobatches_in_line(config, hs) and not _scheduled(fwd_parts) and not _scheduled(bwd_parts)
         streams = [None] * n if in_line else _nanobatch_streams(config, n)
         chains = _chains(config)
-        ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=in_line, chains=chains) for i in range(n)]
+        out_tid = fwd_graph.get_output_channel(seed.fwd_output_channel)
+        ctxs = [NanoBatchContext(batch_idx=i, stream=streams[i], in_line=in_line, chains=chains, output_id=out_tid) for i in range(n)]
         _seed_forward(ctxs, hs, rotary, mask, seed)
 
         # The nanobatch outputs are written side by side into one [s, b, h] tensor, so the
@@ -229,7 +230,6 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
         _run_forward(fwd_parts, ctxs, schedule, is_grad_enabled)
         _join(streams)
 
-        out_tid = fwd_graph.get_output_channel(seed.fwd_output_channel)
         outs = [c.tensor_store.get(out_tid) for c in ctxs]
 
         func_ctx.n = n
@@ -305,8 +305,9 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
                 c.restore_saved_tensors(saved[lo : lo + cnt])
                 lo += cnt
 
+        grad_tid = func_ctx.backward_tensor_graph.get_output_channel(seed.bwd_output_channel)
         for c, g in zip(ctxs, grad_outs):
-            c.chains = chains
+            c.chains, c.output_id = chains, grad_tid
             c.tensor_store = TensorStore()
             c.tensor_store.set(seed.bwd_grad_tid, g)
 
@@ -352,7 +353,6 @@ class TransformerBlockAutogradFunction(torch.autograd.Function):
             launch()
         _join(streams)
 
-        grad_tid = func_ctx.backward_tensor_graph.get_output_channel(seed.bwd_output_channel)
         dhs = [c.tensor_store.get(grad_tid) if grad_tid is not None else None for c in ctxs]
 
         grads: List[Optional[Tensor]] = []

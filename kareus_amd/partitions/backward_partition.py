@@ -28,7 +28,7 @@ class BackwardPartition(PartitionBase):
     def _find_chains(self, plans):
         from ..operators.chains import backward_chains
 
-        return backward_chains(plans)
+        return backward_chains(plans, self.graph_reads)
 
     def execute(
         self,
@@ -79,7 +79,7 @@ class BackwardPartition(PartitionBase):
                 comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size, backward=True)
                 launched = True
             chain = chains[idx] if chains is not None else None
-            if chain is not None and not idx < start < idx + chain.length:
+            if chain is not None and not idx < start < idx + chain.length and ctx.output_id not in chain.inside:
                 got = chain.run(ctx, store, dy, protected)
                 if got is not None:
                     grad_params.update(got)

@@ -80,6 +80,8 @@ class NanoBatchContext:
     in_line: bool = False
     # operator sequences may run as one native call in this pass (operators/chains.py)
     chains: bool = False
+    # the tensor that the pass takes out of the store when it is through (None: no other than the graph's own readers)
+    output_id: Optional[str] = None
     # op_id -> tensor that op's forward output is to be written into (consumed when the op runs)
     output_sinks: Dict[int, torch.Tensor] = field(default_factory=dict)
     _saved_tensors: List[Optional[torch.Tensor]] = field(default_factory=list)

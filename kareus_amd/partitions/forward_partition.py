@@ -26,7 +26,7 @@ class ForwardPartition(PartitionBase):
     def _find_chains(self, plans):
         from ..operators.chains import forward_chains
 
-        return forward_chains(plans)
+        return forward_chains(plans, self.graph_reads)
 
     def execute(self, ctx: NanoBatchContext, pre_ctx: NanoBatchContext) -> None:
         with self._on_stream(ctx), self._timed():
@@ -51,7 +51,8 @@ class ForwardPartition(PartitionBase):
             if start == idx and not identity:
                 comm_out, comm_extra = self._launch_comm(pre_ctx, sm_num, block_size)
             chain = chains[idx] if chains is not None else None
-            if (chain is not None and not idx < start < idx + chain.length and (not grad or needs(plan.first_in))
+            if (chain is not None and not idx < start < idx + chain.length and ctx.output_id not in chain.inside
+                    and (not grad or needs(plan.first_in))
                     and chain.run(ctx, store, x, grad)):
                 idx += chain.length
                 if idx == start and not identity and not self._in_order(ctx):

@@ -18,6 +18,7 @@ after its compute.
 
 from __future__ import annotations
 
+from collections import Counter
 from typing import List, Optional, Sequence, Tuple, Type, Union
 
 from .backward_partition import BackwardPartition
@@ -72,6 +73,7 @@ class PartitionBuilder:
                 f"({nnb} x {len(segments)} segments), got {len(partition_keys)}."
             )
 
+        reads = Counter(tid for node in ops for tid in node.get_input_tensor_ids())
         partitions: list = []
         prev_comm: Optional[CommunicationOp] = None
         for seg_idx, (comp_ops, comm_after) in enumerate(segments):
@@ -88,6 +90,7 @@ class PartitionBuilder:
                         comp_ops=comp_ops,
                         comm_op=_clone_comm(carried) if carried is not None else None,
                         force_no_overlap=(nnb == 1),
+                        graph_reads=reads,
                     )
                 )
             prev_comm = comm_after

@@ -1,15 +1,16 @@
 """Operator sequences that run as one native call (operators/chains.py): found where the graph has them, bit for bit the
 operators one by one, and left alone whenever something looks between the operators or replaced one."""
 
+import dataclasses
 import gc
 import weakref
 
 import pytest
 import torch
 
-from kareus_amd import LayerConfig, LayerStack
+from kareus_amd import LayerConfig, LayerStack, operators
 from kareus_amd.operators import PartitionableRMSNorm, ResidualForkOp, chains
-from kareus_amd.partitions import autograd_function
+from kareus_amd.partitions import Channel, ComputeOp, TensorPort, autograd_function
 from kareus_amd.partitions.partition_base import PartitionBase
 
 
@@ -57,6 +58,68 @@ def test_a_subclass_or_another_order_is_no_chain():
     part.comp_ops[1].operator = Mine(256, backend="hip")
     part._plans()
     assert not any(isinstance(c, chains._ForwardChain) for c in part._op_chains)
+
+
+def with_a_reader(model, channels, layer=0):
+    """The model's partitions built again with one more operator behind a layer's, which adds up two of the layer's channels."""
+    class BiasDropoutAddOp(operators.BiasDropoutAddOp):   # (its name is what the overlap slots know)
+        def get_input_channels(self):
+            return [Channel(i, name) for i, name in enumerate(channels)]
+
+        def get_output_channels(self):
+            return [Channel(0, "sum")]
+
+        def get_backward_ops(self):
+            return []
+
+        def fuser_forward(self, *a, **kw):
+            got = super().fuser_forward(*a, **kw)
+            self.sums.append(got[0])
+            return got
+
+    reader = BiasDropoutAddOp()
+    reader.sums = []
+    ops = model.layers[layer].get_all_operators() + [reader]
+    model.layers[layer].get_all_operators = lambda: ops
+    model._build_partitions()
+    model.set_tensor_parallel_group(None)
+    return reader
+
+
+def found_in(partitions):
+    names = []
+    for part in partitions:
+        part._plans()
+        names += [type(c).__name__ for c in part._op_chains if isinstance(c, chains._Chain)]
+    return names
+
+
+@pytest.mark.parametrize("channels,left", [(("key", "value"), ["_ForwardMlp", "_ForwardAttention", "_ForwardMlp"]),
+                                           (("residual", "main"), ["_ForwardAttention", "_ForwardMlp"] * 2),
+                                           (("residual", "value"), ["_ForwardMlp", "_ForwardAttention", "_ForwardMlp"])])
+def test_a_sequence_with_another_reader_inside_is_no_chain(channels, left):
+    """The reader is in another partition than the tensors that it reads: key and value are made inside the attention sequence,
+    the residual beside it."""
+    model = LayerStack(config(), device="cpu")
+    with_a_reader(model, channels)
+    assert found_in(model.forward_partitions) == left
+
+
+def test_a_reader_that_replaces_an_operator_or_reads_a_gradient_is_noticed():
+    model = LayerStack(config(), device="cpu")
+    part = model.forward_partitions[0]
+    inside = part.comp_ops[3].get_output_tensor_ids()[1]       # the key in front of the rotary embedding
+    assert found_in([part]) == ["_ForwardAttention"]
+    part.comp_ops.append(ComputeOp(operators.BiasDropoutAddOp(), [TensorPort(0, inside), TensorPort(1, inside)],
+                                   [TensorPort(0, "t_sum")], op_id=999))
+    assert found_in([part]) == []
+    back = model.backward_partitions[0]
+    assert found_in([back]) == ["_BackwardMlp"]
+    back.graph_reads = {**back.graph_reads, back.comp_ops[1].get_output_tensor_ids()[0]: 2}
+    back._op_plans = None
+    assert found_in([back]) == []
+    back.graph_reads = back._op_plans = None                  # nothing is known of the graph
+    assert found_in([back]) == []
 
 
 def test_replaced_methods_are_noticed(monkeypatch):
@@ -190,6 +253,17 @@ def test_a_saved_attention_output_with_gaps_runs_operator_by_operator(monkeypatc
     gaps = []
     ran = both(monkeypatch, config(), 96, 2, hooks=lambda: torch.autograd.graph.saved_tensors_hooks(lambda t: t, with_gaps))
     assert gaps and ran.get("_BackwardAttention", 0) == 0 and ran["_BackwardMlp"] == 4
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_tensor_inside_a_sequence_is_there_for_its_other_reader(monkeypatch):
+    """An operator behind the layer reads the first layer's key and value; the block's output may be any channel."""
+    sums = []
+    both(monkeypatch, config(2), 96, 4, before=lambda model: sums.append(with_a_reader(model, ("key", "value")).sums))
+    assert len(sums[0]) == len(sums[1]) == 4 and all(torch.equal(a, b) for a, b in zip(*sums))
+    both(monkeypatch, config(num_layers=1), 96, 2, grad=False,
+         before=lambda model: setattr(model, "seed_config", dataclasses.replace(model.seed_config, fwd_output_channel="value")))
 
 
 @pytest.mark.parametrize("part", ["linear_fc1", "linear_proj", "pre_mlp_layernorm"])
