@@ -96,12 +96,12 @@ def _matches(plans, at: int, classes) -> bool:
 
 
 def _untouched(ops) -> bool:
-    """No method of these operators was replaced on the instance, and they run on the hip backend."""
+    """No method of these operators was replaced on the instance, nor its class since the plans were made (parametrizations do
+    that), and they run on the hip backend."""
     for op in ops:
         d = op.__dict__
-        if d["_backend_name"] != "hip":
-            return False
-        if not _METHODS[type(op)].isdisjoint(d):
+        methods = _METHODS.get(type(op))
+        if methods is None or d.get("_backend_name") != "hip" or not methods.isdisjoint(d):
             return False
     return True
 

@@ -131,9 +131,28 @@ def test_replaced_methods_are_noticed(monkeypatch):
     del ops[2].fuser_forward
     ops[0]._backend_name = "eager"
     assert not chains._untouched(ops)
+    del ops[0]._backend_name
+    assert not chains._untouched(ops)
+    ops[0]._backend_name = "hip"
+    assert chains._untouched(ops)
     assert chains.chains_allowed()
     monkeypatch.setattr(ResidualForkOp, "fuser_forward", lambda *a, **k: None)
     assert not chains.chains_allowed()
+
+
+class Halved(torch.nn.Module):
+    def forward(self, w):
+        return 0.5 * w
+
+
+def test_an_operator_whose_class_changed_is_noticed():
+    """(register_parametrization gives the module a class of its own, behind plans that are there.)"""
+    model = LayerStack(config(), device="cpu")
+    part = model.forward_partitions[0]
+    ops = [p.operator for p in part._plans()]
+    assert chains._untouched(ops)
+    torch.nn.utils.parametrize.register_parametrization(model.layers[0].linear_qkv, "weight", Halved(), unsafe=True)
+    assert not chains._untouched(ops) and found_in([part]) == ["_ForwardAttention"]
 
 
 def test_a_replaced_backend_method_is_noticed(monkeypatch):
@@ -264,6 +283,20 @@ def test_a_tensor_inside_a_sequence_is_there_for_its_other_reader(monkeypatch):
     assert len(sums[0]) == len(sums[1]) == 4 and all(torch.equal(a, b) for a, b in zip(*sums))
     both(monkeypatch, config(num_layers=1), 96, 2, grad=False,
          before=lambda model: setattr(model, "seed_config", dataclasses.replace(model.seed_config, fwd_output_channel="value")))
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_parametrized_weight_runs_operator_by_operator(monkeypatch):
+    """Registered on a model that has run: its layer leaves the chains, and the product is that of the weight it now has."""
+    x = torch.randn(96, 2, 256, generator=torch.Generator().manual_seed(1)).to("cuda", torch.bfloat16)
+    model, plain = (LayerStack(config(), device="cuda", seed=3) for _ in range(2))
+    with torch.no_grad():
+        first = model(x)
+        torch.nn.utils.parametrize.register_parametrization(model.layers[0].linear_qkv, "weight", Halved(), unsafe=True)
+        plain.layers[0].linear_qkv.weight.mul_(0.5)
+        got, want = model(x), plain(x)
+    assert torch.equal(got, want) and not torch.equal(got, first)
 
 
 @pytest.mark.parametrize("part", ["linear_fc1", "linear_proj", "pre_mlp_layernorm"])
