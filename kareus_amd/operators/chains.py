@@ -307,8 +307,9 @@ def _add_pair(be, linear, ctx, dy, x):
     pairs = sink.get("pairs")
     if pairs is None:
         pairs = sink["pairs"] = []
-    # (aliases: the storage behind the saved tensor objects is dropped)
-    pairs.append((ctx.nanobatch_index, dy.detach(), x.detach()))
+    # (aliases: the storage behind the saved tensor objects is dropped; the record is the one that _weight_grad leaves without
+    # events: another nanobatch of the pass may get here operator by operator)
+    pairs.append((ctx.nanobatch_index, dy.detach(), x.detach(), None, None))
     if len(pairs) < n:
         return None
     pairs.sort(key=lambda p: p[0])

@@ -3,6 +3,7 @@ operators one by one, and left alone whenever something looks between the operat
 
 import dataclasses
 import gc
+import itertools
 import weakref
 
 import pytest
@@ -11,6 +12,7 @@ import torch
 from kareus_amd import LayerConfig, LayerStack, operators
 from kareus_amd.operators import PartitionableRMSNorm, ResidualForkOp, chains
 from kareus_amd.partitions import Channel, ComputeOp, TensorPort, autograd_function
+from kareus_amd.partitions.op_context import OperationContext
 from kareus_amd.partitions.partition_base import PartitionBase
 
 
@@ -172,6 +174,39 @@ def test_a_replaced_backend_method_is_noticed(monkeypatch):
     assert chains.chains_allowed()
 
 
+class HostBackend:
+    """The two products that the weight gradient's sink needs, on the host."""
+    class _n:
+        wgrad_segments = staticmethod(lambda *a: None)
+
+    linear_wgrad_segments = None
+    _split_code = staticmethod(lambda split_k: 1)
+    wgrad_segments_ok = staticmethod(lambda dys, xs: False)
+
+    @staticmethod
+    def linear_wgrad(dy, x, out=None, accumulate=False, split_k=True):
+        dw = dy.t() @ x
+        return dw if out is None else out.copy_(out + dw if accumulate else dw)
+
+
+@pytest.mark.parametrize("order", [(0, 1, 2), (2, 0, 1)])
+@pytest.mark.parametrize("ways", [way for way in itertools.product("co", repeat=3)])
+def test_nanobatches_meet_in_the_sink_whichever_way_they_ran(ways, order):
+    """One weight gradient over three nanobatches in line, each of which left its pair as a chain (c) or operator by operator (o)."""
+    linear, be = operators.TERowParallelLinearOp(8, 16), HostBackend()
+    sink = {"n": 3, "turn": [0], "defer": True, "pending": None, "in_line": True}
+    pairs = [(torch.randn(4, 16), torch.randn(4, 8)) for _ in range(3)]
+    got = []
+    for i, way in zip(order, ways):
+        ctx = OperationContext()
+        ctx.wgrad_sink, ctx.nanobatch_index, ctx.alone = sink, i, True
+        got.append(chains._add_pair(be, linear, ctx, *pairs[i]) if way == "c" else linear._weight_grad(be, ctx, *pairs[i]))
+    want = pairs[0][0].t() @ pairs[0][1]
+    for dy, x in pairs[1:]:
+        want = want + dy.t() @ x
+    assert got[0] is None and got[1] is None and torch.equal(got[2], want) and sink["turn"] == [1] and sink["pairs"] is None
+
+
 # ---- the same bits ---------------------------------------------------------------------------------------------------
 def run(cfg, s, b, *, seed=0, grad=True, before=None, hooks=None):
     torch.manual_seed(seed)
@@ -283,6 +318,26 @@ def test_a_tensor_inside_a_sequence_is_there_for_its_other_reader(monkeypatch):
     assert len(sums[0]) == len(sums[1]) == 4 and all(torch.equal(a, b) for a, b in zip(*sums))
     both(monkeypatch, config(num_layers=1), 96, 2, grad=False,
          before=lambda model: setattr(model, "seed_config", dataclasses.replace(model.seed_config, fwd_output_channel="value")))
+
+
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_one_of_two_nanobatches_in_line_runs_operator_by_operator(which, monkeypatch):
+    """The saved attention outputs of one nanobatch come back with gaps: its attention runs one by one, the other's as a chain, and
+    the two meet in the projections' weight gradients."""
+    def hooks():
+        seen = []
+
+        def pack(t):
+            if t.shape != (96, 2, 4, 64):
+                return t
+            seen.append(t)
+            return t if (len(seen) - 1) // 2 != which else torch.empty(96, 2, 4, 128, dtype=t.dtype, device=t.device)[..., :64].copy_(t)
+        return torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t)
+
+    ran = both(monkeypatch, config(2), 96, 4, hooks=hooks)
+    assert ran["_BackwardAttention"] == 4 and ran["_BackwardMlp"] == 8
 
 
 @pytest.mark.gpu
