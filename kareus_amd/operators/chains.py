@@ -54,7 +54,8 @@ _METHODS = {
     BiasDropoutAddOp: frozenset(("fuser_forward", "fuser_backward")),
 }
 _STOCK = tuple((cls, n, getattr(cls, n)) for cls, names in _METHODS.items() for n in sorted(names))
-_BACKEND_METHODS = ("gemm", "linear_fwd", "linear_dgrad", "linear_wgrad", "rows_view", "rows_in_place", "_operand", "rmsnorm_fwd",
+_BACKEND_METHODS = ("gemm", "linear_fwd", "linear_dgrad", "linear_wgrad", "linear_wgrad_segments", "wgrad_segments_ok",
+                    "MAX_WGRAD_SEGMENTS", "rows_view", "rows_in_place", "_operand", "rmsnorm_fwd",
                     "split_qkv", "qk_norm_fwd", "qk_norm_bwd", "rope_fused_inplace", "attn_fwd", "attn_bwd", "swiglu_fwd",
                     "can_fuse_swiglu", "can_fuse_swiglu_bwd", "MAX_RUN_ROWS", "_split_code", "_num_cus")
 _BACKEND_STOCK: list = []

@@ -168,6 +168,16 @@ def test_a_replaced_backend_method_is_noticed(monkeypatch):
     with monkeypatch.context() as m:
         m.setitem(be.__dict__, "attn_fwd", lambda *a, **k: None)
         assert not chains.chains_allowed()
+    for name in ("linear_wgrad_segments", "wgrad_segments_ok", "linear_wgrad"):   # (the sum over nanobatches in line)
+        with monkeypatch.context() as m:
+            m.setattr(type(be), name, lambda *a, **k: None)
+            assert not chains.chains_allowed()
+        with monkeypatch.context() as m:
+            m.setitem(be.__dict__, name, lambda *a, **k: None)
+            assert not chains.chains_allowed()
+    with monkeypatch.context() as m:
+        m.setattr(type(be), "MAX_WGRAD_SEGMENTS", 1)
+        assert not chains.chains_allowed()
     with monkeypatch.context() as m:
         m.setattr(be, "_n", object())
         assert not chains.chains_allowed()
