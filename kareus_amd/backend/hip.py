@@ -375,10 +375,10 @@ class HipBackend:
         """Whether ``linear_wgrad_segments`` takes these operand pairs: matrices of one shape and one row
         stride in every pair (the ``dys`` may be nanobatch slices in row runs, all alike), a multiple of 64 rows
         each, at most MAX_WGRAD_SEGMENTS pairs."""
-        if self._n is not None and self.MAX_RUN_ROWS == 16 and self._n.wgrad_segments_ok(dys, xs):
-            return True
         if not 1 <= len(dys) == len(xs) <= self.MAX_WGRAD_SEGMENTS:
             return False
+        if self._n is not None and self.MAX_RUN_ROWS == 16 and self._n.wgrad_segments_ok(dys, xs):
+            return True
         first = None
         for dy, x in zip(dys, xs):
             a, b = self._operand(dy), self._operand(x)

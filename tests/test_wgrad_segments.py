@@ -54,6 +54,21 @@ def test_operand_pairs_on_the_host_are_turned_down():
     assert not be.wgrad_segments_ok(dys, xs[:1]) and not be.wgrad_segments_ok([], [])
 
 
+def test_a_backend_that_takes_fewer_pairs_turns_more_down():
+    """(An instance with a limit of its own: the native check knows the library's.)"""
+    from kareus_amd.backend.hip import HipBackend
+
+    class Takes:
+        wgrad_segments_ok = staticmethod(lambda dys, xs: True)
+
+    be = HipBackend.__new__(HipBackend)
+    be._n = Takes
+    pairs = [torch.empty(64, 8, dtype=torch.bfloat16) for _ in range(3)]
+    assert be.wgrad_segments_ok(pairs, pairs)
+    be.MAX_WGRAD_SEGMENTS = 2
+    assert be.wgrad_segments_ok(pairs[:2], pairs[:2]) and not be.wgrad_segments_ok(pairs, pairs)
+
+
 # ---- kernels ------------------------------------------------------------------------------------------
 def _rnd(*shape, seed=0):
     g = torch.Generator().manual_seed(seed)
