@@ -708,6 +708,26 @@ PyObject* py_dropout_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 // them saves; between the launches the interpreter had spent several times what the launches cost.  Whatever a chain does not
 // take is answered with None before anything is launched.
 
+// The call that a chain is at, for the error that its operator's own call would raise.
+struct Step {
+  const char* name = "";
+  AttnShape attention{};   // (ok: one of the attention's calls)
+  bool product = false;
+  int layout = 0, epi = 0;
+  int64_t m = 0, n = 0, k = 0;
+  void call(const char* what, const AttnShape& c = AttnShape{}) { name = what, attention = c, product = false; }
+};
+PyObject* failed(const Step& at, int rc) {
+  if (at.product) return gemm_failed(at.layout, at.m, at.n, at.k, at.epi, rc);
+  return failed(at.attention.ok ? attn_name(at.name, at.attention) : at.name, rc);
+}
+int run_gemm(Step& at, int layout, int64_t m, int64_t n, int64_t k, const Tensor& a, const Operand& oa, const Tensor& b, const Operand& ob,
+             const Tensor& out, const Operand& oc, int split, const Epilogue& e, int max_cus) {
+  at.product = true;
+  at.layout = layout, at.epi = e.kind, at.m = m, at.n = n, at.k = k;
+  return run_gemm(layout, m, n, k, a, oa, b, ob, out, oc, false, split, e, max_cus);
+}
+
 // (no references of a failed chain's tensors are left behind)
 PyObject* pack(std::initializer_list<Tensor*> items) {
   PyObject* t = PyTuple_New((Py_ssize_t)items.size());
@@ -821,42 +841,42 @@ PyObject* py_attn_chain_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Operand o_wq = operand2(wq), o_wp = operand2(wp);
     Tensor mixed, fused, qk_rstd, q, k, v, o, lse, o2d;
     int rc;
-    const char* what = "kr_rmsnorm_fwd";
+    Step at;
+    at.call("kr_rmsnorm_fwd");
     {
       WithoutInterpreter free;
       rc = run_norm(x, gamma, eps, n);
       if (rc == KR_OK) {
-        what = "kr_gemm_bf16";
         mixed = matrix(t, w, x);
-        rc = run_gemm(KR_GEMM_TN, t, w, h, n.y, dense(t, h), wq, o_wq, mixed, dense(t, w), false, split_qkv, Epilogue{}, max_cus);
+        rc = run_gemm(at, KR_GEMM_TN, t, w, h, n.y, dense(t, h), wq, o_wq, mixed, dense(t, w), split_qkv, Epilogue{}, max_cus);
         mixed = mixed.view({s, b, w});
         fused = mixed.view({s, b, ng, per + 2, hd});
       }
       if (rc == KR_OK && qk) {
-        what = "kr_qk_norm_fwd";
+        at.call("kr_qk_norm_fwd");
         fused = at::empty({s, b, ng, per + 2, hd}, x.options());
         qk_rstd = at::empty({t, 1, ng, per + 1}, x.options().dtype(at::kFloat));
         rc = kr_qk_norm_fwd(ptr(mixed), ptr(tensor(a[4])), ptr(tensor(a[5])), ptr(fused), (float*)ptr(qk_rstd), t, (int)ng,
                             (int)per, (int)hd, qk_eps, stream());
       }
       if (rc == KR_OK) {
-        what = "kr_rope";
+        at.call("kr_rope");
         rc = run_rope(fused, freqs, false);
       }
       if (rc == KR_OK) {
-        what = "kr_attn_fwd";
         q = fused.narrow(3, 0, per), k = fused.select(3, per), v = fused.select(3, per + 1);
-        rc = run_attn_fwd(attn_shape(q, k, v), q, k, v, scale, flags, o, lse);
+        const AttnShape c = attn_shape(q, k, v);
+        at.call("kr_attn_fwd", c);
+        rc = run_attn_fwd(c, q, k, v, scale, flags, o, lse);
       }
       if (rc == KR_OK) {
-        what = "kr_gemm_bf16";
         o2d = o.view({t, wo});
         if (absent(a[17])) y.t = matrix(t, out_cols, x);
-        rc = run_gemm(KR_GEMM_TN, t, out_cols, wo, o2d, dense(t, wo), wp, o_wp, y.t, y.o, false, split_proj, e, max_cus);
+        rc = run_gemm(at, KR_GEMM_TN, t, out_cols, wo, o2d, dense(t, wo), wp, o_wp, y.t, y.o, split_proj, e, max_cus);
         if (absent(a[17])) y.t = y.t.view({s, b, out_cols});
       }
     }
-    if (rc != KR_OK) return failed(what, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (!qk) mixed = Tensor();
     if (!absent(a[17])) y.t = Tensor();
     return pack({&y.t, &n.rows, &n.rstd, &n.y, &q, &k, &v, &o, &lse, &o2d, &mixed, &qk_rstd});
@@ -887,12 +907,12 @@ PyObject* py_mlp_chain_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Operand o1 = operand2(w1), o2 = operand2(w2);
     Tensor pre, act;
     int rc;
-    const char* what = "kr_rmsnorm_fwd";
+    Step at;
+    at.call("kr_rmsnorm_fwd");
     {
       WithoutInterpreter free;
       rc = run_norm(x, gamma, eps, n);
       if (rc == KR_OK) {
-        what = "kr_gemm_bf16";
         act = matrix(t, f, x);
         pre = matrix(t, two_f, x);
         Epilogue swiglu;
@@ -901,20 +921,19 @@ PyObject* py_mlp_chain_fwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
           swiglu.out2 = ptr(act);
           swiglu.ld_out2 = f;
         }
-        rc = run_gemm(KR_GEMM_TN, t, two_f, h, n.y, dense(t, h), w1, o1, pre, dense(t, two_f), false, split1, swiglu, max_cus);
+        rc = run_gemm(at, KR_GEMM_TN, t, two_f, h, n.y, dense(t, h), w1, o1, pre, dense(t, two_f), split1, swiglu, max_cus);
       }
       if (rc == KR_OK && !fuse) {
-        what = "kr_swiglu_fwd";
+        at.call("kr_swiglu_fwd");
         rc = kr_swiglu_fwd(ptr(pre), ptr(act), t, (int)f, stream());
       }
       if (rc == KR_OK) {
-        what = "kr_gemm_bf16";
         if (absent(a[9])) y.t = matrix(t, out_cols, x);
-        rc = run_gemm(KR_GEMM_TN, t, out_cols, f, act, dense(t, f), w2, o2, y.t, y.o, false, split2, e, max_cus);
+        rc = run_gemm(at, KR_GEMM_TN, t, out_cols, f, act, dense(t, f), w2, o2, y.t, y.o, split2, e, max_cus);
         if (absent(a[9])) y.t = y.t.view({s, b, out_cols});
       }
     }
-    if (rc != KR_OK) return failed(what, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (!absent(a[9])) y.t = Tensor();
     return pack({&y.t, &n.rows, &n.rstd, &n.y, &pre, &act});
   });
@@ -952,6 +971,7 @@ PyObject* py_mlp_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const Operand o1 = operand2(w1), o2 = operand2(w2);
     Tensor dpre, dx, dw2, dw1;
     int rc;
+    Step at;
     {
       WithoutInterpreter free;
       dpre = matrix(t, 2 * f, dy);
@@ -959,25 +979,25 @@ PyObject* py_mlp_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       e.kind = KR_GEMM_EPI_SWIGLU_BWD;
       e.ox.ld = 2 * f;
       e.aux = ptr(pre);
-      rc = run_gemm(KR_GEMM_NN, t, f, cols, dy, od, w2, o2, dpre, dense(t, 2 * f), false, split2, e, max_cus);
+      rc = run_gemm(at, KR_GEMM_NN, t, f, cols, dy, od, w2, o2, dpre, dense(t, 2 * f), split2, e, max_cus);
       if (rc == KR_OK && wgrad) {
         dw2 = matrix(cols, f, dy);
-        rc = run_gemm(KR_GEMM_NT, cols, f, t, dy, od, act, dense(t, f), dw2, dense(cols, f), false, split2, Epilogue{}, max_cus);
+        rc = run_gemm(at, KR_GEMM_NT, cols, f, t, dy, od, act, dense(t, f), dw2, dense(cols, f), split2, Epilogue{}, max_cus);
       }
     }
-    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, f, cols, KR_GEMM_EPI_SWIGLU_BWD, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (wgrad) release({a[2], a[3]});
     {
       WithoutInterpreter free;
       dx = matrix(t, h, dy);
-      rc = run_gemm(KR_GEMM_NN, t, h, 2 * f, dpre, dense(t, 2 * f), w1, o1, dx, dense(t, h), false, split1, Epilogue{}, max_cus);
+      rc = run_gemm(at, KR_GEMM_NN, t, h, 2 * f, dpre, dense(t, 2 * f), w1, o1, dx, dense(t, h), split1, Epilogue{}, max_cus);
       if (rc == KR_OK && wgrad) {
         dw1 = matrix(2 * f, h, dy);
-        rc = run_gemm(KR_GEMM_NT, 2 * f, h, t, dpre, dense(t, 2 * f), normed, dense(t, h), dw1, dense(2 * f, h), false, split1,
+        rc = run_gemm(at, KR_GEMM_NT, 2 * f, h, t, dpre, dense(t, 2 * f), normed, dense(t, h), dw1, dense(2 * f, h), split1,
                       Epilogue{}, max_cus);
       }
     }
-    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, h, 2 * f, KR_GEMM_EPI_NONE, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (wgrad) release({a[5]});
     return pack({&dx, &dpre, &dw2, &dw1});
   });
@@ -1020,30 +1040,32 @@ PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     Tensor dout, dwp, dwq, dx, dgq, dgk, dmixed;
     AttnGrads g;
     int rc;
+    Step at;
     {
       WithoutInterpreter free;
       dout = matrix(t, wo, dy);
-      rc = run_gemm(KR_GEMM_NN, t, wo, cols, dy, od, wp, o_wp, dout, dense(t, wo), false, split_proj, Epilogue{}, max_cus);
+      rc = run_gemm(at, KR_GEMM_NN, t, wo, cols, dy, od, wp, o_wp, dout, dense(t, wo), split_proj, Epilogue{}, max_cus);
       if (rc == KR_OK && wgrad) {
         dwp = matrix(cols, wo, dy);
-        rc = run_gemm(KR_GEMM_NT, cols, wo, t, dy, od, o2d, dense(t, wo), dwp, dense(cols, wo), false, split_proj, Epilogue{},
+        rc = run_gemm(at, KR_GEMM_NT, cols, wo, t, dy, od, o2d, dense(t, wo), dwp, dense(cols, wo), split_proj, Epilogue{},
                       max_cus);
       }
     }
-    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, wo, cols, KR_GEMM_EPI_NONE, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (wgrad) release({a[7]});
-    const char* what = "kr_attn_bwd";
+    at.call("kr_attn_bwd", c);
     {
       WithoutInterpreter free;
       rc = run_attn_bwd(c, dout, q, k, v, o, lse, scale, flags, g);
       dout = Tensor();
       if (rc == KR_OK) {
-        what = "kr_rope";
+        at.call("kr_rope");
         rc = run_rope(g.fused, freqs, true);
       }
     }
-    if (rc != KR_OK) return failed(what, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (wgrad) release({a[2], a[3], a[4], a[5], a[6]});
+    at.call("kr_qk_norm_bwd");
     {
       WithoutInterpreter free;
       if (qk) {
@@ -1056,20 +1078,20 @@ PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
                             ptr(ws), t, c.nkv, (int)c.per, c.hd, stream());
       }
     }
-    if (rc != KR_OK) return failed("kr_qk_norm_bwd", rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (wgrad && qk) release({a[11], a[12]});
     {
       WithoutInterpreter free;
       dmixed = g.mixed.view({t, w});
       dx = matrix(t, h, dmixed);
-      rc = run_gemm(KR_GEMM_NN, t, h, w, dmixed, dense(t, w), wq, o_wq, dx, dense(t, h), false, split_qkv, Epilogue{}, max_cus);
+      rc = run_gemm(at, KR_GEMM_NN, t, h, w, dmixed, dense(t, w), wq, o_wq, dx, dense(t, h), split_qkv, Epilogue{}, max_cus);
       if (rc == KR_OK && wgrad) {
         dwq = matrix(w, h, dmixed);
-        rc = run_gemm(KR_GEMM_NT, w, h, t, dmixed, dense(t, w), normed, dense(t, h), dwq, dense(w, h), false, split_qkv, Epilogue{},
+        rc = run_gemm(at, KR_GEMM_NT, w, h, t, dmixed, dense(t, w), normed, dense(t, h), dwq, dense(w, h), split_qkv, Epilogue{},
                       max_cus);
       }
     }
-    if (rc != KR_OK) return gemm_failed(KR_GEMM_NN, t, h, w, KR_GEMM_EPI_NONE, rc);
+    if (rc != KR_OK) return failed(at, rc);
     if (wgrad) release({a[16]});
     return pack({&dx, &dmixed, &dwp, &dwq, &dgq, &dgk});
   });

@@ -350,6 +350,46 @@ def test_one_of_two_nanobatches_in_line_runs_operator_by_operator(which, monkeyp
     assert ran["_BackwardAttention"] == 4 and ran["_BackwardMlp"] == 8
 
 
+def misaligned(t):
+    """A dense copy two bytes beyond a boundary of 16: the library turns it down before it launches anything."""
+    return torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)[1:t.numel() + 1].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("where", ["linear_qkv", "linear_proj", "linear_fc1", "linear_fc2", "q_layernorm", "dgrad linear_qkv",
+                                   "dgrad linear_proj", "dgrad linear_fc1", "dgrad linear_fc2", "wgrad (192, 320)", "wgrad (192, 256)",
+                                   "head dimension"])
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_a_call_that_fails_is_named_as_by_its_operator(where, monkeypatch):
+    """The same error, with the call's sizes, from a sequence and from its operators."""
+    def broken():
+        cfg = config(num_layers=1, qk_layernorm=True, kv_channels=136 if where == "head dimension" else 64)
+        model = LayerStack(cfg, device="cuda", seed=3)
+        layer = model.layers[0]
+        x = torch.randn(96, 2, 256, device="cuda").bfloat16().requires_grad_(True)
+        weight = {"q_layernorm": lambda: layer.qkv_postprocess.q_layernorm}.get(where, lambda: getattr(layer, where.split()[-1], None))()
+        hooks = torch.autograd.graph.saved_tensors_hooks(
+            lambda t: t, lambda t: misaligned(t) if where == f"wgrad {tuple(t.shape)}" else t)
+        with pytest.raises(RuntimeError) as failure:
+            if weight is not None and not where.startswith("dgrad"):
+                weight.weight.data = misaligned(weight.weight.data)
+            with hooks:
+                y = model(x)
+            if weight is not None:
+                weight.weight.data = misaligned(weight.weight.data)
+            y.sum().backward()
+        torch.cuda.synchronize()
+        return str(failure.value)
+
+    chained = broken()
+    with monkeypatch.context() as m:
+        m.setattr(autograd_function, "_chains", lambda config: False)
+        assert chained == broken()
+    assert "(code -" in chained
+    if "grad" in where or where.startswith("linear"):
+        assert "M=" in chained and f"layout={2 if 'wgrad' in where else 1 if 'dgrad' in where else 0}" in chained
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
 def test_a_parametrized_weight_runs_operator_by_operator(monkeypatch):
