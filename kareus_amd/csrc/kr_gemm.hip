@@ -1265,20 +1265,9 @@ inline int choose_wn(int M, int N, int num_cus) {
   return best;
 }
 
-// Tile width and number of cuts of the contraction.  An output of at least 192 full-width tiles is
-// never cut and takes the width of choose_wn.  A smaller one has too few tiles to occupy the GPU:
-// narrower tiles (down to 128 columns; 160 with a fused epilogue) and cuts of the contraction both
-// make more work items, and the pair with the least estimated cost wins.  Two estimates, in units of one K-step of a full-width tile (~1.3 us;
-// a tile of WN columns takes (WN + 2) / 10 of it):
-//   latency  rounds of work items over the CUs, each item paying its K-steps plus a fixed
-//            prologue/epilogue, plus the traffic of the fp32 partial tiles (written once, read
-//            once by the reduce kernel at ~5 TB/s);
-//   CU-time  the same work summed over the CUs it occupies, per CU of the device.
-// A GEMM that has the GPU to itself wants the smallest latency (latency_weight 1); one that
-// runs beside kernels of other streams, which can use the CUs it leaves idle, should mostly
-// keep its CU-time small (the dispatcher uses latency_weight 0.1).  `max_splits` is what the caller's workspace holds.
-// 224 or 192 rows of 256 columns in place of 256 rows of `wn` units, by the same estimate (rounds of tiles times their larger
-// side's units and one): where it is at least a ninth smaller and the last round is at least 5/8 full.  us before -> after:
+// 224 or 192 rows of 256 columns in place of 256 rows and 32 * wn columns, by choose_wn's estimate (rounds of tiles times the units
+// of 32 of the side that is not 256, and one): where it is at least a ninth smaller and the last round is at least 5/8 full.  us
+// before -> after:
 // TN 776 x 32064 x 4096 196 -> 178, 1152 x 32064 x 4096 246 -> 229, 6024 x 4096 x 3584 (residual) 151 -> 138; NN 6024 x 4096 x
 // 7168 280 -> 257, 12240 x 2048 x 16384 660 -> 575.  Outside the rule nothing is won: the workgroups of a round that is a third
 // full run faster than those of a full one (NN 6440 x 3072 x 16384 551 -> 557, 1504 x 12288 x 4096 142 -> 143), and a saving
@@ -1299,6 +1288,18 @@ inline Tile fewer_rows(int M, int N, int wn, int num_cus) {
   return tile;
 }
 
+// Tile width and number of cuts of the contraction.  An output of at least 192 full-width tiles is
+// never cut and takes the width of choose_wn.  A smaller one has too few tiles to occupy the GPU:
+// narrower tiles (down to 128 columns; 160 with a fused epilogue) and cuts of the contraction both
+// make more work items, and the pair with the least estimated cost wins.  Two estimates, in units of one K-step of a full-width tile (~1.3 us;
+// a tile of WN columns takes (WN + 2) / 10 of it):
+//   latency  rounds of work items over the CUs, each item paying its K-steps plus a fixed
+//            prologue/epilogue, plus the traffic of the fp32 partial tiles (written once, read
+//            once by the reduce kernel at ~5 TB/s);
+//   CU-time  the same work summed over the CUs it occupies, per CU of the device.
+// A GEMM that has the GPU to itself wants the smallest latency (latency_weight 1); one that
+// runs beside kernels of other streams, which can use the CUs it leaves idle, should mostly
+// keep its CU-time small (the dispatcher uses latency_weight 0.1).  `max_splits` is what the caller's workspace holds.
 struct Plan {
   int wn, splits;
   Tile tile = kLarge;  // (wn is 4 for the small tile, 2 for the two below it)
