@@ -17,7 +17,6 @@ kareus/megatron/core/transformer/transformer_layer.py:148-174 and the files each
 from __future__ import annotations
 
 import math
-from collections import Counter
 from typing import List, Optional
 
 import torch
@@ -124,8 +123,11 @@ class _Chain:
         self.plans = list(plans)
         self.length = len(self.plans)
         self.ops = [p.operator for p in self.plans]
-        first, last = self.plans[0], self.plans[-1]
-        self.inside = frozenset([t for p in plans for t in p.out_ids]).difference(first.extra_out_ids, (last.first_out,))
+        inside = self.inside = set()
+        for p in plans:
+            inside.update(p.out_ids)
+        inside.difference_update(plans[0].extra_out_ids)
+        inside.discard(plans[-1].first_out)
 
 
 class _ForwardChain(_Chain):
@@ -388,35 +390,36 @@ class _BackwardAttention(_BackwardChain):
         return {po.op_id: [dwo], pa.op_id: [], pr.op_id: [], pp.op_id: [] if gq is None else [dgq, dgk], pq.op_id: [dwq]}
 
 
-def _chains(plans, reads, find, behind_add) -> List:
-    """By index, the chain that starts there, if one does: a chain, or a residual add and the chain behind it.  Only where every
-    read that the graph has (``reads``: by tensor id, how many ports) of a tensor between the operators is the chain's own, and,
-    should an operator of the partition have been replaced by one with other ports, every read of the partition's is too.  (Part
-    of a new model's first pass: 65 us for a layer with two nanobatches.)"""
-    if reads is None:
+def _chains(plans, read_twice, find, behind_add) -> List:
+    """By index, the chain that starts there, if one does: a chain, or a residual add and the chain behind it.  A chain reads each
+    tensor between its operators once, so one that the graph reads twice (``read_twice``), or this partition, should one of its
+    operators have been replaced by one with other ports, has another reader: no chain.  (Part of a new model's first pass: 100 us
+    for a layer with two nanobatches.)"""
+    if read_twice is None:
         return [None] * len(plans)
     found = [find(plans, at) for at in range(len(plans))]
-    for at, chain in enumerate(found[1:]):
-        if chain is not None and type(plans[at].operator) is BiasDropoutAddOp and plans[at].first_out == plans[at + 1].first_in:
-            found[at] = behind_add(plans[at], chain)
-    if any(found):
-        here = Counter([t for p in plans for t in p.in_ids])
-        for at, chain in enumerate(found):
-            if chain is not None:
-                own = Counter([t for p in plans[at:at + chain.length] for t in p.in_ids])
-                if any([max(reads.get(t, 0), here[t]) > own[t] for t in chain.inside]):
-                    found[at] = None
+    ids = [t for p in plans for t in p.in_ids]
+    if len(set(ids)) != len(ids):
+        read_twice = read_twice.union([t for t in ids if ids.count(t) > 1])
+    for at, chain in enumerate(found):
+        if chain is None:
+            continue
+        if not chain.inside.isdisjoint(read_twice):
+            found[at] = None
+        elif (at and type(plans[at - 1].operator) is BiasDropoutAddOp and plans[at - 1].first_out == plans[at].first_in
+              and plans[at].first_in not in read_twice):
+            found[at - 1] = behind_add(plans[at - 1], chain)
     return found
 
 
-def forward_chains(plans, reads) -> List:
+def forward_chains(plans, read_twice) -> List:
     """The chains of operators of a forward partition."""
-    return _chains(plans, reads, _forward_chain, _ForwardBehindAdd)
+    return _chains(plans, read_twice, _forward_chain, _ForwardBehindAdd)
 
 
-def backward_chains(plans, reads) -> List:
+def backward_chains(plans, read_twice) -> List:
     """The same for a backward partition."""
-    return _chains(plans, reads, _backward_chain, _BackwardBehindAdd)
+    return _chains(plans, read_twice, _backward_chain, _BackwardBehindAdd)
 
 
 def _forward_chain(plans, at: int) -> Optional[_ForwardChain]:

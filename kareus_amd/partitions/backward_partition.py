@@ -28,7 +28,7 @@ class BackwardPartition(PartitionBase):
     def _find_chains(self, plans):
         from ..operators.chains import backward_chains
 
-        return backward_chains(plans, self.graph_reads)
+        return backward_chains(plans, self.read_twice)
 
     def execute(
         self,

@@ -26,7 +26,7 @@ class ForwardPartition(PartitionBase):
     def _find_chains(self, plans):
         from ..operators.chains import forward_chains
 
-        return forward_chains(plans, self.graph_reads)
+        return forward_chains(plans, self.read_twice)
 
     def execute(self, ctx: NanoBatchContext, pre_ctx: NanoBatchContext) -> None:
         with self._on_stream(ctx), self._timed():

@@ -19,7 +19,7 @@ from __future__ import annotations
 
 import contextlib
 from dataclasses import dataclass, field
-from typing import Any, Dict, List, Mapping, Optional, Tuple, Union
+from typing import Any, Dict, FrozenSet, List, Optional, Tuple, Union
 
 from ..backend import reserve_compute_units
 from ..utils.debug import roctx_enabled, roctx_range
@@ -141,8 +141,8 @@ class PartitionBase:
     force_no_overlap: bool = False
     # the schedule's resource shape sets a compute-unit budget for this partition's GEMM launches
     apply_resource_shape: bool = True
-    # by tensor id, how many ports of the whole graph read it (None: not known, and no operators are run as one call)
-    graph_reads: Optional[Mapping[str, int]] = None
+    # the tensors that more than one port of the whole graph reads (None: not known, and no operators are run as one call)
+    read_twice: Optional[FrozenSet[Optional[str]]] = None
 
     def __post_init__(self) -> None:
         self._overlap_slots: Dict[str, int] = _build_overlap_slots(self.comp_ops)

@@ -18,7 +18,6 @@ after its compute.
 
 from __future__ import annotations
 
-from collections import Counter
 from typing import List, Optional, Sequence, Tuple, Type, Union
 
 from .backward_partition import BackwardPartition
@@ -73,7 +72,11 @@ class PartitionBuilder:
                 f"({nnb} x {len(segments)} segments), got {len(partition_keys)}."
             )
 
-        reads = Counter(tid for node in ops for tid in node.get_input_tensor_ids())
+        seen, read_twice = set(), set()
+        for node in ops:
+            for port in node.input_ports:
+                (read_twice if port.tensor_id in seen else seen).add(port.tensor_id)
+        read_twice = frozenset(read_twice)
         partitions: list = []
         prev_comm: Optional[CommunicationOp] = None
         for seg_idx, (comp_ops, comm_after) in enumerate(segments):
@@ -90,7 +93,7 @@ class PartitionBuilder:
                         comp_ops=comp_ops,
                         comm_op=_clone_comm(carried) if carried is not None else None,
                         force_no_overlap=(nnb == 1),
-                        graph_reads=reads,
+                        read_twice=read_twice,
                     )
                 )
             prev_comm = comm_after

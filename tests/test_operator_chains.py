@@ -115,12 +115,20 @@ def test_a_reader_that_replaces_an_operator_or_reads_a_gradient_is_noticed():
     part.comp_ops.append(ComputeOp(operators.BiasDropoutAddOp(), [TensorPort(0, inside), TensorPort(1, inside)],
                                    [TensorPort(0, "t_sum")], op_id=999))
     assert found_in([part]) == []
+    behind = model.forward_partitions[1]                       # [residual add, fork, norm, ..]
+    assert found_in([behind]) == ["_ForwardMlp"] and isinstance(behind._op_chains[0], chains._ForwardBehindAdd)
+    handed_on = behind.comp_ops[0].get_output_tensor_ids()[0]
+    behind.comp_ops.append(ComputeOp(operators.BiasDropoutAddOp(), [TensorPort(0, handed_on), TensorPort(1, "ext_main")],
+                                     [TensorPort(0, "t_sum")], op_id=998))
+    assert found_in([behind]) == ["_ForwardMlp"] and behind._op_chains[0] is None
     back = model.backward_partitions[0]
     assert found_in([back]) == ["_BackwardMlp"]
-    back.graph_reads = {**back.graph_reads, back.comp_ops[1].get_output_tensor_ids()[0]: 2}
-    back._op_plans = None
+    known = back.read_twice
+    back.read_twice, back._op_plans = known | {back.comp_ops[1].get_output_tensor_ids()[0]}, None
     assert found_in([back]) == []
-    back.graph_reads = back._op_plans = None                  # nothing is known of the graph
+    back.read_twice, back._op_plans = known, None
+    assert found_in([back]) == ["_BackwardMlp"]
+    back.read_twice = back._op_plans = None                   # nothing is known of the graph
     assert found_in([back]) == []
 
 
