@@ -157,9 +157,10 @@ class PartitionBase:
                 nxt = _OpPlan(op, nxt)
                 plans.append(nxt)
             plans.reverse()
-            self._op_plans = plans
-            # the operator sequences that can run as one native call, by the index they start at (operators/chains.py)
+            # the operator sequences that can run as one native call, by the index they start at (operators/chains.py); the plans
+            # last: another thread that finds them finds the chains too
             self._op_chains = self._find_chains(plans)
+            self._op_plans = plans
         return plans
 
     def _find_chains(self, plans: List[_OpPlan]) -> List[Any]:

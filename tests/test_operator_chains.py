@@ -4,6 +4,7 @@ operators one by one, and left alone whenever something looks between the operat
 import dataclasses
 import gc
 import itertools
+import threading
 import weakref
 
 import pytest
@@ -130,6 +131,25 @@ def test_a_reader_that_replaces_an_operator_or_reads_a_gradient_is_noticed():
     assert found_in([back]) == ["_BackwardMlp"]
     back.read_twice = back._op_plans = None                   # nothing is known of the graph
     assert found_in([back]) == []
+
+
+def test_a_second_thread_finds_no_plans_without_their_chains():
+    """Two threads' first passes of one model: while one looks for chains, the other has to look for itself."""
+    model = LayerStack(config(), device="cpu")
+    part = model.forward_partitions[0]
+    find, got = part._find_chains, []
+
+    def first(plans):
+        del part._find_chains
+        other = threading.Thread(target=lambda: got.append((part._plans(), part._op_chains)))
+        other.start()
+        other.join()
+        return find(plans)
+
+    part._find_chains = first
+    part._plans()
+    (plans, chained), = got
+    assert len(plans) == len(chained) and isinstance(chained[0], chains._ForwardAttention)
 
 
 def test_replaced_methods_are_noticed(monkeypatch):
