@@ -17,7 +17,7 @@ kareus/megatron/core/transformer/transformer_layer.py:148-174 and the files each
 from __future__ import annotations
 
 import math
-from typing import List, Optional
+from typing import List, Optional, Tuple
 
 import torch
 
@@ -57,11 +57,12 @@ _BACKEND_METHODS = ("gemm", "linear_fwd", "linear_dgrad", "linear_wgrad", "linea
                     "MAX_WGRAD_SEGMENTS", "rows_view", "rows_in_place", "_operand", "rmsnorm_fwd",
                     "split_qkv", "qk_norm_fwd", "qk_norm_bwd", "rope_fused_inplace", "attn_fwd", "attn_bwd", "swiglu_fwd",
                     "can_fuse_swiglu", "can_fuse_swiglu_bwd", "MAX_RUN_ROWS", "_split_code", "_num_cus")
-_BACKEND_STOCK: list = []
+_BACKEND_STOCK: Tuple = ()   # (filled by the first pass, whole: other threads' first passes may be at it too)
 
 
 def chains_allowed() -> bool:
     """Whether the operators' and the hip backend's methods are the package's own and nothing traces: asked once per pass."""
+    global _BACKEND_STOCK
     if torch._C._get_tracing_state() is not None:
         return False
     for cls, name, fn in _STOCK:
@@ -72,8 +73,7 @@ def chains_allowed() -> bool:
     if not _BACKEND_STOCK:
         from ..backend import hip
 
-        _BACKEND_STOCK.extend((n, hip.STOCK[n]) for n in _BACKEND_METHODS)
-        _BACKEND_STOCK.append(("_n", hip.load_native()))
+        _BACKEND_STOCK = (*[(n, hip.STOCK[n]) for n in _BACKEND_METHODS], ("_n", hip.load_native()))
     own = be.__dict__
     for name, fn in _BACKEND_STOCK:
         if name in own:

@@ -152,6 +152,17 @@ def test_a_second_thread_finds_no_plans_without_their_chains():
     assert len(plans) == len(chained) and isinstance(chained[0], chains._ForwardAttention)
 
 
+def test_a_second_thread_asks_for_every_backend_method(monkeypatch):
+    """While one thread's first pass gathers what the backend's methods are, another's has to see all of them or none."""
+    from kareus_amd.backend import hip
+
+    seen, load = [], hip.load_native
+    monkeypatch.setattr(chains, "_BACKEND_STOCK", type(chains._BACKEND_STOCK)())
+    monkeypatch.setattr(hip, "load_native", lambda: seen.append(len(chains._BACKEND_STOCK)) or load())
+    assert chains.chains_allowed()
+    assert set(seen) == {0} and len(chains._BACKEND_STOCK) == len(chains._BACKEND_METHODS) + 1
+
+
 def test_replaced_methods_are_noticed(monkeypatch):
     model = LayerStack(config(), device="cpu")
     ops = [p.operator for p in model.forward_partitions[0]._plans()]
