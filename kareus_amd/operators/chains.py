@@ -8,9 +8,9 @@ operators one by one, every operator's context holds what the operator itself wo
 way and backward the other), and saved activations are dropped at the same points.  One operator at a time the interpreter
 spent 6-10 us per operator around launches of 3-5 us.
 
-A sequence runs operator by operator whenever something looks inside it or is not the stock case: a timer or a schedule's
-launch point between its operators, an operator, an operator method or a backend method that was replaced, another backend,
-frozen weights, operands that the kernels do not address in place, a trace.  (Reference for what the operators do:
+A sequence runs operator by operator whenever something looks inside it or is not the stock case: another reader of a tensor
+between its operators, a timer or a schedule's launch point there, an operator, its class, an operator method or a backend
+method that was replaced, another backend, frozen weights, operands that the kernels do not address in place, a trace.  (Reference for what the operators do:
 kareus/megatron/core/transformer/transformer_layer.py:148-174 and the files each operator names.)
 """
 
