@@ -970,7 +970,7 @@ template <int D>
 __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* __restrict__ dout,
                                                          const bf16* __restrict__ o,
                                                          const float* __restrict__ lse,
-                                                         float* __restrict__ delta,
+                                                         float* __restrict__ neg_delta,
                                                          float* __restrict__ neg_lse2, int s, int sp, int nq,
                                                          int per, int64_t total_rows, QLayout dol,
                                                          QLayout ol) {
@@ -983,7 +983,7 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* __restrict_
   const int bi = (int)(row / ((int64_t)sp * nq));
   if (si >= s) {
     if (sub == 0) {
-      delta[row] = 0.f;
+      neg_delta[row] = 0.f;
       neg_lse2[row] = -kPadLse * kLog2e;
     }
     return;
@@ -996,7 +996,7 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* __restrict_
 #pragma unroll
   for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, KR_WAVE);
   if (sub == 0) {
-    delta[row] = acc;
+    neg_delta[row] = -acc;
     // -lse in the log2 domain, so that the dK/dV kernel's exponent is one multiply-add and its
     // row statistics can go straight from global memory into LDS
     neg_lse2[row] = -lse[((int64_t)bi * nq + head) * s + si] * kLog2e;
@@ -1023,19 +1023,19 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16* __restrict_
 // land (it must be complete by the first barrier of iteration it+2: the score waves start on a
 // tile one block ahead).
 // PARTIAL = true: fp32 results for this query head go to part_k / part_v [b, nq, qsplit, sp, D].
-// D = 64: a tile is 128 queries, walked as four 32-query blocks with a hand-over each.
-template <int D, bool RAGGED, bool PARTIAL>
+// (Head dimension 128; attn_bwd_dkdv64_kernel below takes 64.)
+template <bool RAGGED, bool PARTIAL>
 __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
-    const bf16* __restrict__ dout, const float* __restrict__ neg_lse2, const float* __restrict__ delta,
+    const bf16* __restrict__ dout, const float* __restrict__ neg_lse2, const float* __restrict__ neg_delta,
     bf16* __restrict__ dk, bf16* __restrict__ dv, float* __restrict__ part_k,
     float* __restrict__ part_v, int s, int nq, int nkv, int qsplit, int hpw, float scale, float scale_log2,
     QLayout ql, KLayout kl, KLayout vl, QLayout dol, KLayout dkl, KLayout dvl) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
-  constexpr int TQ = tile_rows<D>, NSUB = TQ / 32;  // queries of a tile, its 32-query blocks
+  constexpr int D = HD, TQ = tile_rows<D>;  // queries of a tile: two blocks of 32
   constexpr int DT = D / 32, KK = D / 16;
   constexpr int NF = 4 * DT;                        // transposed fragments of a block, two channel operands
-  // stage layout: Q tile | dO tile (blocked tiles) | lse[TQ] fp32 | delta[TQ] fp32
+  // stage layout: Q tile | dO tile (blocked tiles) | -lse[TQ] fp32 | -delta[TQ] fp32
   constexpr uint32_t STAGE = 2 * BT_BYTES + 8 * TQ;  // bytes
   constexpr int NS = 3;
   // hand-over area behind the stages: [block parity][key block][slot 0..3][lane] 16 bytes each
@@ -1064,7 +1064,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const int kw0 = key0 + wave * 32;
   const int krow = kw0 + (lane & 31);
   const int qt_first = key0 / TQ;
-  // this part's query tiles, per head (with tiles of 128 the second part of the last key tile has none)
+  // this part's query tiles, per head
   const int niter = (sp / TQ - qt_first - part + qsplit - 1) / qsplit;
   const int nit_all = niter * hpw;                                       // ... over all heads of the workgroup
   const uint32_t lds0 = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem;
@@ -1153,7 +1153,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[g * 4 + e], scale_log2, l4[e]));
-          const float ds = p * (dpacc[g * 4 + e] - d4[e]);
+          const float ds = p * (dpacc[g * 4 + e] + d4[e]);
           pb[g >> 1][(g & 1) * 4 + e] = (bf16)p;
           dsb[g >> 1][(g & 1) * 4 + e] = (bf16)ds;
         }
@@ -1176,14 +1176,10 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       const int stage = it % NS;
       const int q0 = (qt_first + itl * qsplit + part) * TQ;
       itl = itl + 1 == niter ? 0 : itl + 1;  // the next head starts over at the diagonal
-#pragma unroll
-      for (int sub = 0; sub < NSUB; sub += 2) {
-        step(stage, sub, q0 + 32 * sub, s0, dp0, stage, sub + 1, s1, dp1);
-        __syncthreads();  // hand-over of block `sub`
-        const bool more = sub + 2 < NSUB;
-        step(stage, sub + 1, q0 + 32 * sub + 32, s1, dp1, more ? stage : (it + 1) % NS, more ? sub + 2 : 0, s0, dp0);
-        __syncthreads();  // hand-over of block `sub` + 1
-      }
+      step(stage, 0, q0, s0, dp0, stage, 1, s1, dp1);
+      __syncthreads();  // hand-over of block 0
+      step(stage, 1, q0 + 32, s1, dp1, (it + 1) % NS, 0, s0, dp0);
+      __syncthreads();  // hand-over of block 1
     }
     return;
   }
@@ -1192,7 +1188,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const bf16* qb = q + ql.at(bi, head, per);
   const bf16* dob = dout + dol.at(bi, head, per);
   const int64_t stat0 = ((int64_t)bi * nq + head) * sp;
-  // A tile is brought in by nine requests per wave (with D = 128 eight for waves 2 and 3): the TQ + TQ row
+  // A tile is brought in by nine requests per wave (eight for waves 2 and 3): the TQ + TQ row
   // statistics, 4 bytes per lane, 64 of them per wave, then four consecutive rows (+ 16, 32, 48
   // through the lanes) of the Q tile and four of the dO tile.  request_begin names the tile,
   // request_piece(i) issues piece i = 0..8, in this order (requests retire in order).
@@ -1201,7 +1197,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const bf16 *req_q = qb, *req_do = dob;
   int64_t req_stat = stat0;
   int req_qt = 0;
-  const bool has_stat = D == 64 || wave < 2;
+  const bool has_stat = wave < 2;
   auto request_begin = [&](int it) {
     const int hh = it / niter, itl = it - hh * niter;  // head of the workgroup, query tile of that head
     req_qt = qt_first + itl * qsplit + part;
@@ -1215,10 +1211,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       if (has_stat) {
         int l2 = lane;
         asm volatile("" : "+v"(l2));
-        // D = 128: one wave per statistic; D = 64: two, 64 rows each
-        const bool first = D == 128 ? wave == 0 : wave < 2;
-        const int row = D == 128 ? 0 : (wave & 1) * 64;
-        dma_b32((first ? neg_lse2 : delta) + req_stat + req_qt * TQ + row, (uint32_t)l2 * 4u,
+        dma_b32((wave == 0 ? neg_lse2 : neg_delta) + req_stat + req_qt * TQ, (uint32_t)l2 * 4u,
                 req_tile + 2 * BT_BYTES + wave * 256);
       }
       return;
@@ -1272,7 +1265,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       dkacc[dt][e] = 0.f;
       dvacc[dt][e] = 0.f;
     }
-  if (D == 128 || nit_all > 0) request_tile(0);
+  request_tile(0);
   if (nit_all > 1) request_tile(1);
   if (nit_all > 2) {
     request_tile(2);
@@ -1304,7 +1297,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   for (int it = 0; it < nit_all; ++it) {
     const int stage = it % NS;
 #pragma unroll
-    for (int sub = 0; sub < NSUB; ++sub) {
+    for (int sub = 0; sub < 2; ++sub) {
       // tile it+1 (requested an iteration and a half ago) must have landed before this
       // iteration's first barrier: the score waves start on it right after.  Tile it+2 may still
       // be on its way.
@@ -1326,7 +1319,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       // tile it+3 goes into its stage, one request behind each of the first MFMAs — pieces 0-4
       // in this block, pieces 5-8 in the first block of the next iteration, so that neither
       // block of the accumulate waves outlasts the score waves' step beside it.
-      const bool first_pieces = sub == NSUB - 1 && it + 3 < nit_all;
+      const bool first_pieces = sub == 1 && it + 3 < nit_all;
       const bool last_pieces = sub == 0 && it > 0 && it + 2 < nit_all;
       if (first_pieces) request_begin(it + 3);
       const uint32_t xa = xch_lane + (sub & 1) * 16384;
@@ -1335,7 +1328,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       for (int c = 0; c < 4; ++c) hand[c] = *(KR_LDS const bf16x8*)(xa + c * 1024);
       // next block: the next of this tile, or the first of the next tile (complete since this
       // iteration's first barrier; behind the last tile a stale stage, unused)
-      uint32_t next_base = lds0 + (sub < NSUB - 1 ? stage : (it + 1) % NS) * STAGE + cols_lane;
+      uint32_t next_base = lds0 + (sub == 0 ? stage : (it + 1) % NS) * STAGE + cols_lane;
       asm volatile("" : "+v"(next_base));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1345,12 +1338,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
           dkacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], hand[2 + f / (2 * DT)], dkacc[dt], 0, 0, 0);
         else
           dvacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], hand[f / (2 * DT)], dvacc[dt], 0, 0, 0);
-        if (f > 0) fr[f - 1] = frag(next_base, (sub + 1) % NSUB, f - 1);
+        if (f > 0) fr[f - 1] = frag(next_base, sub ^ 1, f - 1);
         if (first_pieces && f < 5) request_piece(f);
         if (last_pieces && f < 4) request_piece(5 + f);
         __builtin_amdgcn_sched_barrier(0);
       }
-      fr[NF - 1] = frag(next_base, (sub + 1) % NSUB, NF - 1);
+      fr[NF - 1] = frag(next_base, sub ^ 1, NF - 1);
     }
   }
 
@@ -1365,6 +1358,343 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   } else {
     store_rows_bf16<D, RAGGED>(rs, dkacc, scale, dk + dkl.at(bi, kvh) + (int64_t)kw0 * dkl.s_, dkl.s_, s - kw0);
     store_rows_bf16<D, RAGGED>(rs, dvacc, 1.0f, dv + dvl.at(bi, kvh) + (int64_t)kw0 * dvl.s_, dvl.s_, s - kw0);
+  }
+}
+// dK/dV at head dimension 64.  A wave's K and V fragments and both accumulators are half of what 128 channels take
+// (96 registers instead of 192), so a wave does all the work of its 32 keys — scores, exponentials, both accumulating
+// products — and no hand-over is needed.  Eight waves, two per SIMD: waves w and w + 4 have the same 32 of the
+// workgroup's 128 keys and take the first and the second 64 queries of every 128-query tile; at the end one of them
+// gets the sum of dK, the other of dV.  Four stages of a Q and a dO tile, one barrier per tile.
+// The loop is one pipeline of sixteen slots per 32-query block b, each slot one MFMA (32 cycles of the matrix pipe) and
+// the vector work of one score (multiply-add, exponential, multiplication, conversions: 27 cycles), so that one
+// wave alone already keeps the pipe nearly full:
+//   slots 0-7    S and dP of block b + 1
+//   slots 8-11   dV and dK, first 16 queries of block b
+//   slots 12-15  ... last 16 queries
+// A score's multiply-add, its exponential and its remaining work are in consecutive slots (in one slot a wave would wait for
+// each of them); score 0 of block b + 1 starts in slot 10 of block b.
+// What bounds it: between the matrix pipe and the instructions around it (without its LDS reads, requests and barriers,
+// MFMAs and exponentials alone, it takes 203 us where it takes 274).  The kernel that specialised its waves, as the one above does,
+// waited for hand-overs: b 2 x 32/8 x s 4096 404 -> 274 us (0.70 -> 1.03 PFLOP/s of the four products), b 1 beside other streams 199
+// -> 143, s 2048, b 1 60 -> 46, 4 x 1000 tokens, 8 heads 38 (with the sum of its partial results) -> 22, s 256 9.1 -> 9.8.
+// Two independent workgroups of four waves per compute unit took 309 (each a barrier fewer, but the first key tiles
+// run on alone); row statistics through one lane each and lane broadcasts, instead of 8 KB of LDS reads a block, the same.
+// Everything read from LDS is requested about four slots before it is used.  dP starts from -delta, read straight into
+// the accumulator, which takes the subtraction out of every score.
+// PARTIAL = true: fp32 results for this group of heads go to part_k / part_v [b, nq / hpw, qsplit, sp, 64].
+template <bool RAGGED, bool PARTIAL>
+__global__ __launch_bounds__(512, 1) void attn_bwd_dkdv64_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
+    const bf16* __restrict__ dout, const float* __restrict__ neg_lse2, const float* __restrict__ neg_delta,
+    bf16* __restrict__ dk, bf16* __restrict__ dv, float* __restrict__ part_k,
+    float* __restrict__ part_v, int s, int nq, int nkv, int qsplit, int hpw, float scale, float scale_log2,
+    QLayout ql, KLayout kl, KLayout vl, QLayout dol, KLayout dkl, KLayout dvl) {
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  constexpr int D = 64, TQ = tile_rows<D>, DT = D / 32, KK = D / 16;
+  constexpr uint32_t STAGE = 2 * BT_BYTES + 8 * TQ;  // Q tile | dO tile | -lse[TQ] fp32 | -delta[TQ] fp32
+  constexpr int NS = 4;
+
+  const int lane = threadIdx.x & 63, h = lane >> 5;
+  const int wave8 = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave = wave8 & 3, half = wave8 >> 2;  // key block of the tile; which 64 queries of a tile
+  const int sp = RAGGED ? (s + 127) / 128 * 128 : s;  // rows of the statistics and of the partial results
+  const int nkt = sp / 128;
+  const int lid_all = xcd_contiguous_id(blockIdx.x, gridDim.x);
+  const int part = lid_all % qsplit;
+  int kt_rev, hg;
+  longest_first(lid_all / qsplit, nkt, gridDim.x / (nkt * qsplit), kt_rev, hg);
+  const int kt = nkt - 1 - kt_rev;  // low key tiles see the most queries
+  const int nhg = nq / hpw;
+  const int hgroup = hg % nhg;
+  const int head = hgroup * hpw;  // `hpw` consecutive query heads of one KV group, one after the other
+  const int bi = hg / nhg;
+  const int per = nq / nkv;
+  const int kvh = head / per;
+  const int kw0 = kt * 128 + wave * 32;
+  const int krow = kw0 + (lane & 31);
+  const int kld = RAGGED && krow >= s ? s - 1 : krow;
+  const int niter = (nkt - kt - part + qsplit - 1) / qsplit;  // this part's query tiles, per head
+  const int nit_all = niter * hpw;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(KR_LDS const bf16*)smem;
+
+  const bf16* kp = k + kl.at(bi, kvh) + (int64_t)kld * kl.s_;
+  const bf16* vp = v + vl.at(bi, kvh) + (int64_t)kld * vl.s_;
+  bf16x8 kf[KK], vf[KK];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk) {
+    kf[kk] = ldg8(kp + kk * 16 + h * 8);
+    vf[kk] = ldg8(vp + kk * 16 + h * 8);
+  }
+
+  // A tile is brought in by the eight waves together: waves 0-3 request 64 of its row statistics each (0, 1: -lse, 2, 3:
+  // -delta), then every wave two blocks of the Q tile and two of the dO tile (block B of a tile holds its rows r, r + 16, r +
+  // 32, r + 48, r = 4 (B % 4) + B / 4, and + 64): blocks wave8 and wave8 + 8, rows r0 and r0 + 2.  Pointers to row r0 of
+  // the next tile are kept, so that a request is a handful of scalar instructions.
+  const int r0 = 4 * wave + half;
+  const bf16* qb = q + ql.at(bi, head, per);
+  const bf16* dob = dout + dol.at(bi, head, per);
+  const float* statb = (wave < 2 ? neg_lse2 : neg_delta) + ((int64_t)bi * nq + head) * sp + (wave & 1) * 64;
+  const uint32_t q_lane = tile_lane_off<D>(lane, (int)ql.s_), do_lane = tile_lane_off<D>(lane, (int)dol.s_);
+  const uint32_t stat_lane4 = (uint32_t)lane * 4u;
+  const int64_t q_step = (int64_t)(qsplit * TQ) * ql.s_, do_step = (int64_t)(qsplit * TQ) * dol.s_;
+  int req_it = 0, req_head = 0, req_qt = kt + part;  // the next tile to ask for
+  const bf16 *q_next = nullptr, *do_next = nullptr;
+  const float* stat_next = nullptr;
+  auto seek = [&]() {
+    q_next = qb + req_head * ql.h_ + (int64_t)(req_qt * TQ + r0) * ql.s_;
+    do_next = dob + req_head * dol.h_ + (int64_t)(req_qt * TQ + r0) * dol.s_;
+    stat_next = statb + (int64_t)req_head * sp + req_qt * TQ;
+  };
+  seek();
+  // One piece of the next tile (0: statistics, which both halves ask for, 1, 2: Q, 3, 4: dO).  Behind the last tile that one
+  // is asked for again, into a free stage: no branch, so that the pipeline below stays one block of code.
+  auto request_piece = [&](uint32_t stage, int i) {
+    const int j = (i - 1) & 1;
+    const bool second = i > 2;
+    const uint32_t dst = stage + (second ? BT_BYTES : 0) + (wave8 + 8 * j) * BT_BLK;
+    if (i == 0)
+      dma_b32(stat_next, stat_lane4, stage + 2 * BT_BYTES + wave * 256);
+    else if (RAGGED)
+      request_clamped<D>(second ? dob + req_head * dol.h_ : qb + req_head * ql.h_, second ? dol.s_ : ql.s_, req_qt * TQ,
+                         r0 + 2 * j, s, lane, dst);
+    else if (second)
+      dma_b128(do_next + 2 * j * dol.s_, do_lane, dst);
+    else
+      dma_b128(q_next + 2 * j * ql.s_, q_lane, dst);
+  };
+  auto requested = [&]() {  // on to the next tile; the next head starts over at the diagonal
+    if (++req_it >= nit_all) return;
+    req_qt += qsplit;
+    if (req_qt >= nkt) {
+      req_qt = kt + part;
+      ++req_head;
+      seek();
+    } else {
+      q_next += q_step;
+      do_next += do_step;
+      stat_next += qsplit * TQ;
+    }
+  };
+  // rows of query tile qt beyond the sequence: zeros once they have landed (their probabilities are zero, see kPadLse)
+  auto zero_tail = [&](uint32_t stage, int qt) {
+    if (RAGGED && (qt + 1) * TQ > s) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        zero_block_tail<D>(qt * TQ, r0 + 2 * j, s, lane, stage + (wave8 + 8 * j) * BT_BLK);
+        zero_block_tail<D>(qt * TQ, r0 + 2 * j, s, lane, stage + BT_BYTES + (wave8 + 8 * j) * BT_BLK);
+      }
+    }
+  };
+  f32x16 dkacc[DT], dvacc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      dkacc[dt][e] = 0.f;
+      dvacc[dt][e] = 0.f;
+    }
+  const uint32_t rows_lane = bt_rows_lane(lane), cols_lane = bt_cols_lane(lane) + half * 128;
+  const uint32_t rows_half = rows_lane + half * 128;  // 32-row blocks 2 and 3 are column half 1 of the tile's image
+  const uint32_t stat_lane = 2 * BT_BYTES + 16 * h + half * 256;
+
+  struct Scores { f32x16 s, dp; };
+  bf16x8 qfr[3], dofr[3];      // row fragments, contraction step kk in place kk % 3
+  bf16x8 fr[2 * DT];           // transposed fragments: dO^T, Q^T of each channel block
+  f32x4 l4[2];                 // -lse of four scores, group g in place g % 2
+  u32x4 pb[2], dsb[2];         // P and dS of the block, rounded to bf16, two to a register
+  float x_at = 0.f, p_at = 0.f, p_even = 0.f, ds_even = 0.f;  // scores under way
+  auto row_frag = [&](uint32_t rows, int sub, int kk) {
+    qfr[kk % 3] = bt_rows<D>(rows, sub, kk);
+    dofr[kk % 3] = bt_rows<D>(rows + BT_BYTES, sub, kk);
+  };
+  auto begin_dp = [&](Scores& x, uint32_t stats, int sub, int g) {
+    const f32x4 d4 = *(KR_LDS const f32x4*)(stats + 4 * (TQ + sub * 32 + 8 * g));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.dp[4 * g + e] = d4[e];
+  };
+  auto lse_of = [&](uint32_t stats, int sub, int g) { l4[g & 1] = *(KR_LDS const f32x4*)(stats + 4 * (sub * 32 + 8 * g)); };
+  auto s_mfma = [&](Scores& x, int kk) {
+    if (kk == 0)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) x.s[e] = 0.f;
+    x.s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfr[kk % 3], kf[kk], x.s, 0, 0, 0);
+  };
+  auto dp_mfma = [&](Scores& x, int kk) {
+    x.dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dofr[kk % 3], vf[kk], x.dp, 0, 0, 0);
+  };
+  auto mask = [&](Scores& x, int qs0) {  // queries qs0 .. + 31; only blocks that reach the diagonal pay for it
+    if (qs0 < kw0 + 31) {
+      const int lim = krow - qs0 - 4 * h;  // element offsets below it are queries before the key
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        float v = 8 * (e >> 2) + (e & 3) < lim ? -INFINITY : x.s[e];
+        asm volatile("" : "+v"(v));  // keeps this a branch: off the diagonal no mask code runs
+        x.s[e] = v;
+      }
+    }
+  };
+  // The three steps of a score.  Each result passes through an (empty) volatile asm: left alone the compiler moves the
+  // work of several slots behind the next branch, away from the MFMAs that should cover it.
+  auto score_a = [&](const Scores& x, int i) {
+    x_at = __builtin_fmaf(x.s[i], scale_log2, l4[(i >> 2) & 1][i & 3]);
+    asm volatile("" : "+v"(x_at));
+  };
+  auto score_b = [&]() {
+    p_at = __builtin_amdgcn_exp2f(x_at);
+    asm volatile("" : "+v"(p_at));
+  };
+  auto pack = [&](float lo, float hi) {
+    bf16x2 v;
+    v[0] = (bf16)lo;
+    v[1] = (bf16)hi;
+    uint32_t w = __builtin_bit_cast(uint32_t, v);
+    asm volatile("" : "+v"(w));
+    return w;
+  };
+  auto score_c = [&](const Scores& x, int i) {
+    float ds = p_at * x.dp[i];
+    asm volatile("" : "+v"(ds));
+    if (i & 1) {
+      pb[i >> 3][(i >> 1) & 3] = pack(p_even, p_at);
+      dsb[i >> 3][(i >> 1) & 3] = pack(ds_even, ds);
+    } else {
+      p_even = p_at;
+      ds_even = ds;
+    }
+  };
+  // transposed fragment f of 16-query group k2: 2 dt: dO^T, 2 dt + 1: Q^T of channel block dt
+  auto col_frag = [&](uint32_t cols, int sub, int k2, int f) {
+    fr[f] = bt_cols<D>((f & 1) ? cols : cols + BT_BYTES, 2 * sub + k2, f >> 1);
+  };
+  // Block `sub` at (cols, stats); the block after it is n1 at (rows1, stats1), the one after that n2 at (rows2, stats2).
+  auto block = [&](Scores& cur, Scores& nxt, uint32_t cols, uint32_t stats, int sub, uint32_t rows1, uint32_t stats1,
+                   int n1, uint32_t rows2, uint32_t stats2, int n2, int qs1, auto&& behind_mfma, auto&& between) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (i == 10) {
+        between();
+        mask(nxt, qs1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (i < 8) {
+        if (i & 1) dp_mfma(nxt, i >> 1);
+        else s_mfma(nxt, i >> 1);
+      } else {
+        const int f = i & 3, k2 = (i - 8) >> 2, dt = f >> 1;
+        const bf16x8 p8 = __builtin_bit_cast(bf16x8, (f & 1) ? dsb[k2] : pb[k2]);
+        if (f & 1) dkacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], p8, dkacc[dt], 0, 0, 0);
+        else dvacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], p8, dvacc[dt], 0, 0, 0);
+      }
+      behind_mfma(i);
+      if (i == 0) row_frag(rows1, n1, 2);
+      if (i == 2) row_frag(rows1, n1, 3);
+      if (i >= 4 && i < 8) col_frag(cols, sub, 0, i - 4);
+      if (i >= 8 && i < 12) col_frag(cols, sub, 1, i - 8);
+      if (i == 2) lse_of(stats, sub, 3);
+      if (i == 6 || i == 10 || i == 14) lse_of(stats1, n1, (i - 6) / 4);
+      if (i < 12) score_c(cur, i + 4);
+      else score_c(nxt, i - 12);
+      score_b();
+      if (i < 10) score_a(cur, i + 6);
+      else score_a(nxt, i - 10);
+      if (i == 12) row_frag(rows2, n2, 0);
+      if (i == 14) row_frag(rows2, n2, 1);
+      if (i >= 12) begin_dp(cur, stats2, n2, i - 12);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  if (nit_all > 0) {
+    auto stage_of = [&](int it) { return lds0 + (it & (NS - 1)) * STAGE; };
+    for (int t = 0; t < NS - 1 && t < nit_all; ++t) {
+#pragma unroll
+      for (int i = 0; i < 5; ++i) request_piece(stage_of(t), i);
+      requested();
+    }
+    if (nit_all >= NS - 1)
+      __builtin_amdgcn_s_waitcnt(0x0f75);  // vmcnt(5): all but the newest tile
+    else
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    int qt = kt + part;  // query tile at hand
+    const int qt_next = niter > 1 ? qt + qsplit : qt;
+    zero_tail(lds0, qt);
+    if (nit_all > 1) zero_tail(stage_of(1), qt_next);
+    __syncthreads();
+    settle_scalar_loads();
+    const int qoff = 64 * half;  // this wave's queries of a tile
+    Scores a, b;
+    {
+      const uint32_t rows = lds0 + rows_half, stats = lds0 + stat_lane;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) begin_dp(a, stats, 0, g);
+      lse_of(stats, 0, 0);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        row_frag(rows, 0, kk);
+        s_mfma(a, kk);
+        dp_mfma(a, kk);
+      }
+      mask(a, qt * TQ + qoff);
+      lse_of(stats, 0, 1);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        if (i >= 2) score_c(a, i - 2);
+        if (i >= 1) score_b();
+        score_a(a, i);
+      }
+      lse_of(stats, 0, 2);
+      row_frag(rows, 1, 0);
+      row_frag(rows, 1, 1);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) begin_dp(b, stats, 1, g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int it = 0; it < nit_all; ++it) {
+      const uint32_t here = stage_of(it), there = stage_of(it + 1);
+      uint32_t rows = here + rows_half, cols = here + cols_lane, stats = here + stat_lane;
+      uint32_t rows_n = there + rows_half, stats_n = there + stat_lane;
+      asm volatile("" : "+v"(rows), "+v"(cols), "+v"(stats), "+v"(rows_n), "+v"(stats_n));
+      const int q0 = qt * TQ + qoff;
+      qt = qt + qsplit >= nkt ? kt + part : qt + qsplit;  // of the next tile
+      // from the last slots of block 0 on the next tile is read (behind the last one a stale stage, unused)
+      block(a, b, cols, stats, 0, rows, stats, 1, rows_n, stats_n, 0, q0 + 32, [](int) {}, [&] {
+        __builtin_amdgcn_s_waitcnt(0x0f75);  // vmcnt(5): of this wave's requests only those of tile it + 2 may be on their way
+        if (it > 0 && it + 1 < nit_all) zero_tail(there, qt);  // (tiles 0 and 1 were settled before the loop)
+        __syncthreads();  // everyone's share of tile it + 1 has landed, and nobody reads tile it - 1 any more
+      });
+      const uint32_t free = stage_of(it + NS - 1);
+      block(b, a, cols, stats, 1, rows_n, stats_n, 0, rows_n, stats_n, 1, qt * TQ + qoff,
+            [&](int i) { if (i < 5) request_piece(free, i); }, [] {});
+      requested();
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the requests behind the last tile
+  // The stages are free.  Wave w of the first half gives its dV to wave w of the second and gets its dK ([value][wave]
+  // [lane] layout, 32 KB each); the first half stores dK, the second dV, through 4 KB per wave behind them.
+  __syncthreads();
+  float* xch = reinterpret_cast<float*>(smem) + wave * 64 + lane;
+  float* mine = xch + half * (32 * 256);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mine[(dt * 16 + e) * 256] = half == 0 ? dvacc[dt][e] : dkacc[dt][e];
+  __syncthreads();
+  const float* other = xch + (1 - half) * (32 * 256);
+  f32x16 acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[dt][e] = (half == 0 ? dkacc[dt][e] : dvacc[dt][e]) + other[(dt * 16 + e) * 256];
+  RowStage rs;
+  rs.init(reinterpret_cast<char*>(smem) + 65536 + wave8 * 4096, lane);
+  const float mul = half == 0 ? scale : 1.0f;
+  if (PARTIAL) {
+    const int64_t prow = (((int64_t)bi * nhg + hgroup) * qsplit + part) * sp + kw0;
+    store_rows_f32<D>(rs, acc, mul, (half == 0 ? part_k : part_v) + prow * D, D);
+  } else if (half == 0) {
+    store_rows_bf16<D, RAGGED>(rs, acc, mul, dk + dkl.at(bi, kvh) + (int64_t)kw0 * dkl.s_, dkl.s_, s - kw0);
+  } else {
+    store_rows_bf16<D, RAGGED>(rs, acc, mul, dv + dvl.at(bi, kvh) + (int64_t)kw0 * dvl.s_, dvl.s_, s - kw0);
   }
 }
 
@@ -1417,7 +1747,7 @@ __global__ __launch_bounds__(256) void attn_group_reduce_kernel(
 template <int D, bool RAGGED, int HALVES>
 __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
-    const bf16* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta,
+    const bf16* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ neg_delta,
     bf16* __restrict__ dq, int s, int nq, int nkv, float scale, float scale_log2, QLayout ql,
     KLayout kl, KLayout vl, QLayout dol, QLayout dql) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
@@ -1454,7 +1784,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
   }
   const int64_t stat = (int64_t)bi * nq + head;
   const float neg_lse = -lse[stat * s + qld] * kLog2e;
-  const float my_delta = delta[stat * sp + qld];
+  const float my_neg_delta = neg_delta[stat * sp + qld];
 
   f32x16 dqacc[DT];
 #pragma unroll
@@ -1534,7 +1864,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[e], scale_log2, neg_lse));
-          dsb[e >> 3][e & 7] = (bf16)(p * (dpacc[e] - my_delta));
+          dsb[e >> 3][e & 7] = (bf16)(p * (dpacc[e] + my_neg_delta));
         }
 #pragma unroll
         for (int k2 = 0; k2 < 2; ++k2)
@@ -1715,7 +2045,7 @@ template <int D, bool RAGGED>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const bf16* __restrict__ dout, const bf16* __restrict__ o, const float* __restrict__ lse,
-    float* __restrict__ delta_out, float* __restrict__ neg_lse2_out, bf16* __restrict__ dq, int s, int nq,
+    float* __restrict__ neg_delta_out, float* __restrict__ neg_lse2_out, bf16* __restrict__ dq, int s, int nq,
     int nkv, float scale, float scale_log2, QLayout ql, KLayout kl, KLayout vl, QLayout dol, QLayout ol,
     QLayout dql) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
@@ -1773,7 +2103,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
       neg_lse[qb] = -kPadLse * kLog2e;
     }
     if (h == 0) {
-      delta_out[stat] = dsum;
+      neg_delta_out[stat] = -dsum;
       neg_lse2_out[stat] = neg_lse[qb];
     }
 #pragma unroll
@@ -2214,9 +2544,16 @@ __global__ __launch_bounds__(256) void attn_resize_rows_kernel(const float* __re
 #ifndef KR_DKDV_HPW_MAX
 #define KR_DKDV_HPW_MAX 4
 #endif
-// The dK/dV kernel runs one workgroup per CU.  With at most two rounds of workgroups its time is
-// set by the first key tiles (they see every query): two workgroups then share each key tile.
-static int dkdv_query_split(int s, int b, int nq) { return (s / 128) * nq * b <= 2 * 256 ? 2 : 1; }
+// The dK/dV kernels run one workgroup per CU.  With few of them their time is set by the first key tiles (they see every
+// query): two workgroups then share each key tile, which costs fp32 partial sums and a launch that adds them.  At head
+// dimension 64 the halves of a workgroup share a key tile's queries already, so that pays only for long rows (whole -> split,
+// with the launch that adds, us): 8 heads at s 200, b 2 10.2 -> 13.5, at s 1000 19.3 -> 18.9, at s 1000, b 4 21.8 -> 33.7;
+// at s 1536 23.1 -> 24.9; one head at s 4096 47.0 -> 32.6, 4 heads 50.2 -> 38.4; 4/2 heads at s 2048 32.5 -> 23.7.
+static int dkdv_query_split(int s, int b, int nq, int hd) {
+  const int key_tiles = (s / 128) * nq * b;
+  if (hd == 64) return key_tiles <= 128 && s >= 2048 ? 2 : 1;
+  return key_tiles <= 2 * 256 ? 2 : 1;
+}
 
 static int attn_padded_len(int s) { return (s + BQ - 1) / BQ * BQ; }
 // bytes of one padded [s_pad, b, heads, 128] bf16 tensor / of the padded statistics [b, nq, s_pad]
@@ -2230,7 +2567,7 @@ static size_t attn_padded_stat_bytes(int s, int b, int nq) {
 // workspace of the MFMA backward kernels for a shape they take as it is
 static size_t attn_bwd_fast_bytes(int s, int b, int nq, int nkv, int hd) {
   size_t bytes = 2 * (size_t)b * nq * s * sizeof(float);  // delta, and -lse in the log2 domain
-  const int qsplit = dkdv_query_split(s, b, nq);
+  const int qsplit = dkdv_query_split(s, b, nq, hd);
   if (nq != nkv || qsplit > 1)  // fp32 dK, dV partials per (query head, query-tile part)
     bytes += 2 * (size_t)b * nq * qsplit * s * hd * sizeof(float);
   return bytes;
@@ -2303,13 +2640,13 @@ struct AttnForms {
   bool shared_fwd, shared_dq;
   int qsplit;
 };
-static AttnForms attn_forms(int s, int b, int nq, int flags) {  // s: rounded up to whole 128-row tiles
+static AttnForms attn_forms(int s, int b, int nq, int hd, int flags) {  // s: rounded up to whole 128-row tiles
   const bool beside = (flags & KR_ATTN_BESIDE_OTHER_STREAMS) != 0;
   const int tiles256 = (s / 256) * nq * b;
   AttnForms f;
   f.shared_fwd = s % 256 == 0 && (beside || tiles256 >= kr_compute_units());
   f.shared_dq = s % 256 == 0 && (beside || tiles256 >= kr_compute_units());
-  f.qsplit = beside ? 1 : dkdv_query_split(s, b, nq);
+  f.qsplit = beside ? 1 : dkdv_query_split(s, b, nq, hd);
   return f;
 }
 
@@ -2339,11 +2676,11 @@ int attn_bwd_mfma(const BwdCall& c) {
   const QLayout ql = c.ql, ol = c.ol, dol = c.dol, dql = c.dql;
   const KLayout kl = c.kl, vl = c.vl, dkl = c.dkl, dvl = c.dvl;
   hipStream_t st = c.st;
-  float* delta = c.workspace;
+  float* neg_delta = c.workspace;
   const int64_t rows = (int64_t)b * nq * sp;
-  float* neg_lse2 = delta + rows;
+  float* neg_lse2 = neg_delta + rows;
   float* part_k = neg_lse2 + rows;
-  const AttnForms forms = attn_forms(sp, b, nq, c.flags);
+  const AttnForms forms = attn_forms(sp, b, nq, D, c.flags);
   const int qsplit = forms.qsplit;
   float* part_v = part_k + rows * qsplit * D;
   // query heads of a KV group per dK/dV workgroup: as many as leave two workgroups per compute
@@ -2359,15 +2696,21 @@ int attn_bwd_mfma(const BwdCall& c) {
       }
   }
   const bool partial = nq / hpw != nkv || qsplit > 1;
-  constexpr size_t lds_dkdv = 3 * (2 * BT_BYTES + 8 * tile_rows<D>) + 32768;  // three stages + the hand-over area
+  // D = 128: three stages and the hand-over area; D = 64: four stages
+  constexpr size_t lds_dkdv = D == 64 ? 4 * (2 * BT_BYTES + 8 * tile_rows<D>) : 3 * (2 * BT_BYTES + 8 * tile_rows<D>) + 32768;
+  const auto dkdv_kernel = [](bool partial) {
+    if constexpr (D == 64)
+      return partial ? attn_bwd_dkdv64_kernel<RAGGED, true> : attn_bwd_dkdv64_kernel<RAGGED, false>;
+    else
+      return partial ? attn_bwd_dkdv_kernel<RAGGED, true> : attn_bwd_dkdv_kernel<RAGGED, false>;
+  };
   constexpr size_t lds_dq = 2 * (2 * BT_BYTES);  // two stages of a K and a V tile
   constexpr size_t lds_dq_w64 = 3 * (2 * BT_BYTES) + 4 * 4096;  // three stages + a 4 KB output stage per wave
-  static const hipError_t attr_status = [] {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<D, RAGGED, false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
+  static const hipError_t attr_status = [&] {
+    hipError_t e = hipFuncSetAttribute((const void*)dkdv_kernel(false), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds_dkdv);
     if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)attn_bwd_dkdv_kernel<D, RAGGED, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
+      e = hipFuncSetAttribute((const void*)dkdv_kernel(true), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dkdv);
     if (e == hipSuccess)
       e = hipFuncSetAttribute((const void*)attn_bwd_dq_kernel<D, RAGGED, 1>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_dq);
@@ -2389,40 +2732,34 @@ int attn_bwd_mfma(const BwdCall& c) {
     // It comes first: it also computes delta and the log2-domain copy of lse that the dK/dV kernel reads.
     hipLaunchKernelGGL((attn_bwd_dq_w64_kernel<D, RAGGED>), dim3(dq_blocks / 2), dim3(256), lds_dq_w64, st,
                        q, k, v, dout, o, lse,
-                       delta, neg_lse2, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol, ol, dql);
+                       neg_delta, neg_lse2, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol, ol, dql);
   } else {
     hipLaunchKernelGGL((attn_delta_kernel<D>), dim3((unsigned)((rows * (D / 8) + 255) / 256)), dim3(256), 0, st,
-                       dout, o, lse, delta, neg_lse2, s, sp, nq, per, rows, dol, ol);
+                       dout, o, lse, neg_delta, neg_lse2, s, sp, nq, per, rows, dol, ol);
   }
   if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
   const dim3 grid_kv((sp / 128) * (nq / hpw) * b * qsplit);
-#define KR_DKDV_LAUNCH(P)                                                                           \
-  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, RAGGED, P>), grid_kv, dim3(512), lds_dkdv, st, q,   \
-                     k, v, dout, neg_lse2,     \
-                     delta, dk, dv, part_k, part_v, s, nq, nkv,         \
-                     partial ? qsplit : 1, hpw, scale, scale_log2, ql, kl, vl, dol, dkl, dvl)
+  hipLaunchKernelGGL(dkdv_kernel(partial), grid_kv, dim3(512), lds_dkdv, st, q, k, v, dout, neg_lse2,
+                     neg_delta, dk, dv, part_k, part_v, s, nq, nkv, partial ? qsplit : 1, hpw, scale, scale_log2, ql, kl,
+                     vl, dol, dkl, dvl);
   if (partial) {
-    KR_DKDV_LAUNCH(true);
     if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
     const int64_t total = (int64_t)b * nkv * s * (D / 8);
     hipLaunchKernelGGL((attn_group_reduce_kernel<D>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
                        st, part_k, part_v, dk, dv, s, sp,
                        nq / hpw, nkv, qsplit, total, dkl, dvl);
-  } else {
-    KR_DKDV_LAUNCH(false);
   }
-#undef KR_DKDV_LAUNCH
   if (hipGetLastError() != hipSuccess) return KR_ELAUNCH;
   if (forms.shared_dq) return kr_launch_status();  // its dQ kernel ran in front of the dK/dV kernel
   if (dq_blocks <= 4 * 256) {  // few workgroups: the longest causal rows set the time
     hipLaunchKernelGGL((attn_bwd_dq_kernel<D, RAGGED, 2>), dim3(dq_blocks), dim3(512), 2 * lds_dq, st,
                        q, k, v, dout, lse,
-                       delta, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
+                       neg_delta, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
                        dql);
   } else {
     hipLaunchKernelGGL((attn_bwd_dq_kernel<D, RAGGED, 1>), dim3(dq_blocks), dim3(256), lds_dq, st,
                        q, k, v, dout, lse,
-                       delta, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
+                       neg_delta, dq, s, nq, nkv, scale, scale_log2, ql, kl, vl, dol,
                        dql);
   }
   return kr_launch_status();
@@ -2559,7 +2896,7 @@ struct FwdCall {
 template <int D, bool RAGGED>
 int attn_fwd_mfma(const FwdCall& c) {
   const int s = c.s, b = c.b, nq = c.nq, sp = attn_padded_len(s);
-  if (attn_forms(sp, b, nq, c.flags).shared_fwd) {
+  if (attn_forms(sp, b, nq, D, c.flags).shared_fwd) {
     // 256-query tiles (one for every compute unit, or other streams beside): the halves share their K / V tiles
     constexpr size_t lds_sh = 3 * 16 * ((1024 + 16) + (1024 + 64));  // 100 KiB
     static const hipError_t attr_sh = hipFuncSetAttribute(

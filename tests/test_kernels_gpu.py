@@ -874,6 +874,25 @@ def test_attention_in_place_at_head_dimension_64_and_ragged_lengths(be, s, b, nq
     assert rel(dq.flatten(2, 3), qf.grad) <= TOL and rel(dk, kf.grad) <= TOL and rel(dv, vf.grad) <= TOL
 
 
+@pytest.mark.parametrize("s,b,nq,nkv", [(256, 1, 2, 1), (384, 1, 2, 2),          # two and three query tiles: the ring of four stages starts
+                                        (640, 2, 4, 2), (2048, 8, 2, 1),         # ... and turns over
+                                        (2056, 1, 4, 2), (2304, 1, 2, 2),        # few key tiles, long rows: two workgroups a key tile
+                                        (512, 64, 8, 2), (500, 64, 8, 2),        # four heads of a group in one workgroup, whole and ragged
+                                        (256, 128, 6, 2)])                       # three
+def test_key_value_gradients_at_head_dimension_64(be, s, b, nq, nkv):
+    """Each half of a workgroup takes 64 of every 128 queries and the halves' sums are exchanged at the end: every length of the
+    loop, several heads per workgroup, partial results and direct ones, against fp32 autograd; the same bits again."""
+    _, q, k, v = _grouped(s, b, nq, nkv, 64, seed=130)
+    do = rnd(s, b, nq, 64, seed=131)
+    o, lse = be.attn_fwd(q, k, v, 0.125)
+    qf, kf, vf = (t.float().cpu().clone().requires_grad_(True) for t in (q.flatten(2, 3), k, v))
+    R.causal_gqa_attention(qf, kf, vf).backward(do.float().cpu())
+    _, dk, dv = be.attn_bwd(do, q, k, v, o, lse, 0.125)
+    assert rel(dk, kf.grad) <= TOL and rel(dv, vf.grad) <= TOL
+    _, dk2, dv2 = be.attn_bwd(do, q, k, v, o, lse, 0.125)
+    assert torch.equal(dk, dk2) and torch.equal(dv, dv2)
+
+
 # ------------------------------------------------------------------ fused GEMM epilogues
 @pytest.mark.parametrize("m,n,k", [(512, 768, 512), (264, 520, 200), (4096, 4096, 1024), (1000, 3072, 640),
                                    (16384, 640, 72)])
