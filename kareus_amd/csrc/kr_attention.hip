@@ -2554,6 +2554,8 @@ static int dkdv_query_split(int s, int b, int nq, int hd) {
   if (hd == 64) return key_tiles <= 128 && s >= 2048 ? 2 : 1;
   return key_tiles <= 2 * 256 ? 2 : 1;
 }
+// ... and how many the workspace has room for, at any head dimension
+static int dkdv_query_split_reserved(int s, int b, int nq) { return dkdv_query_split(s, b, nq, HD); }
 
 static int attn_padded_len(int s) { return (s + BQ - 1) / BQ * BQ; }
 // bytes of one padded [s_pad, b, heads, 128] bf16 tensor / of the padded statistics [b, nq, s_pad]
@@ -2567,7 +2569,7 @@ static size_t attn_padded_stat_bytes(int s, int b, int nq) {
 // workspace of the MFMA backward kernels for a shape they take as it is
 static size_t attn_bwd_fast_bytes(int s, int b, int nq, int nkv, int hd) {
   size_t bytes = 2 * (size_t)b * nq * s * sizeof(float);  // delta, and -lse in the log2 domain
-  const int qsplit = dkdv_query_split(s, b, nq, hd);
+  const int qsplit = dkdv_query_split_reserved(s, b, nq);
   if (nq != nkv || qsplit > 1)  // fp32 dK, dV partials per (query head, query-tile part)
     bytes += 2 * (size_t)b * nq * qsplit * s * hd * sizeof(float);
   return bytes;
