@@ -1229,7 +1229,7 @@ int launch_tile(const Call& call, const Fused& fu) {
 
 #if KR_GEMM_LAYOUT_TU == 1
 int kr_gemm::launch_nn(const Call& call, const Fused& fu) {
-  if (fu.epi == KR_GEMM_EPI_SWIGLU_BWD) return launch_tile<false, true, KR_GEMM_EPI_SWIGLU_BWD, 5>(call, fu);
+  if (fu.epi == KR_GEMM_EPI_SWIGLU_BWD) return launch_tile<false, true, KR_GEMM_EPI_SWIGLU_BWD, 4>(call, fu);
   return launch_tile<false, true, KR_GEMM_EPI_NONE, 4>(call, fu);
 }
 #elif KR_GEMM_LAYOUT_TU == 2
@@ -1239,8 +1239,8 @@ int kr_gemm::launch_nt(const Call& call, const Fused& fu) {
 }
 #else
 int kr_gemm::launch_tn(const Call& call, const Fused& fu) {
-  if (fu.epi == KR_GEMM_EPI_SWIGLU) return launch_tile<false, false, KR_GEMM_EPI_SWIGLU, 5>(call, fu);
-  if (fu.epi == KR_GEMM_EPI_ADD) return launch_tile<false, false, KR_GEMM_EPI_ADD, 5>(call, fu);
+  if (fu.epi == KR_GEMM_EPI_SWIGLU) return launch_tile<false, false, KR_GEMM_EPI_SWIGLU, 4>(call, fu);
+  if (fu.epi == KR_GEMM_EPI_ADD) return launch_tile<false, false, KR_GEMM_EPI_ADD, 4>(call, fu);
   return launch_tile<false, false, KR_GEMM_EPI_NONE, 4>(call, fu);
 }
 
@@ -1423,7 +1423,21 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
   }
   const double small = small_cost(small_cut(kSplit), kSplit);
   // (beside other streams the extra launch is no compute-unit time: 384 x 640 x 4096 in two cuts 21 us, uncut 32)
-  const Plan in_tiles = small >= large * 0.93 ? best : Plan{4, small_cut(w * kSplit), kSmall};  // the change must be clear
+  Plan in_tiles = small >= large * 0.93 ? best : Plan{4, small_cut(w * kSplit), kSmall};  // the change must be clear
+  // More small tiles than units, uncut, whose 256 x 128 tiles are one round: half the workgroups, one a unit, and 48 instead of
+  // 64 KB per K-step for the same products.  us, small -> 256 x 128, operands in HBM (tiles, K-steps): with SwiGLU 776 x 7168 x
+  // 4096 (224, 64) 62.0 -> 55.6, 1024 x 7168 x 4096 72.0 -> 56.1, 512 x 16384 x 2048 (256, 32) 46.2 -> 34.2, 256 x 28672 x 4096
+  // (224, 64) 82.8 -> 72.7; its backward 2048 x 3584 x 4096 (224, 64) 80.4 -> 57.9, 1024 x 8192 x 3072 (256, 48) 66.3 -> 52.9,
+  // 1280 x 3584 x 4096 (140, 64) 58.1 -> 54.9; residual 2048 x 3072 x 3072 (192, 48) 48.2 -> 41.2, 2048 x 4096 x 3584 (256, 56)
+  // 56.2 -> 51.1; plain 1280 x 4096 x 4096 (160, 64) 59.5 -> 51.3, 1024 x 5120 x 3072 (160, 48) 49.7 -> 40.6, 640 x 8192 x 3072 (NN,
+  // 192, 48) 48.9 -> 38.4, 1152 x 4096 x 1536 (160, 24) 21.5 -> 19.7.
+  // Outside the rule: fewer tiles, when most small ones have a unit to themselves (residual 1536 x 3072 x 8192 (144, 128) 95.6 ->
+  // 101.8, SwiGLU backward 6024 x 768 x 2048 (144, 32) 28.1 -> 30.4), and short contractions, where the longer prologue and epilogue
+  // count (plain 1280 x 4096 x 1024 (160, 16) 14.4 -> 14.8, residual 3072 x 2048 x 2048 (192, 32) 27.6 -> 28.2).
+  if (alone && in_tiles.tile == kSmall && in_tiles.splits == 1 && small_tiles > num_cus) {
+    const int tiles = tiles_m * ((N + 127) / 128);
+    if (tiles <= num_cus && tiles * 8 >= num_cus * 5 && nk >= (fused && tiles * 4 <= num_cus * 3 ? 40 : 24)) in_tiles = {4, 1};
+  }
   if (under_cost >= small || under_cost >= large * 0.93) return in_tiles;
   return {2, in_tiles.splits, under};  // (its sums in the pieces that they would be cut into)
 }
@@ -1498,7 +1512,9 @@ struct Choice {
 // plain: no row runs and no accumulation; may_exchange: layout NT, a plain store and an operand A that can stand in B's place
 Choice choose_launch(int layout, int M, int N, int K, int epi, bool shared, int cus, size_t held_bytes, bool plain, bool may_exchange) {
   const Plan plan = launch_plan(M, N, K, epi, shared, cus, held_bytes);
-  Choice c{epi == KR_GEMM_EPI_SWIGLU ? swiglu_wn(M, N, cus) : plan.wn, epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.tile, false};
+  // (128-column tiles divide an output that the plan gives them to: it is one that small tiles may compute)
+  const bool any_width = epi != KR_GEMM_EPI_SWIGLU || (plan.tile == kLarge && plan.wn == 4);
+  Choice c{any_width ? plan.wn : swiglu_wn(M, N, cus), epi == KR_GEMM_EPI_NONE ? plan.splits : 1, plan.tile, false};
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   if (c.tile == kLarge && plain && layout != KR_GEMM_NT && (epi == KR_GEMM_EPI_NONE || epi == KR_GEMM_EPI_ADD) && plan.splits == 1 && tiles >= 192)
     c.tile = fewer_rows(M, N, c.wn, cus);

@@ -498,6 +498,35 @@ def test_gemm_small_tiles_with_swiglu_have_the_bits_of_the_large_ones(be, m, f, 
     assert torch.equal(got[:, :f], big[:m, :f]) and torch.equal(got[:, f:], big[:m, F:F + f])
 
 
+@pytest.mark.parametrize("m,n,k", [(776, 7168, 2560), (1000, 5120, 2568), (2040, 4096, 1544), (1160, 4352, 2632)])
+def test_gemm_one_round_of_narrow_tiles_with_an_epilogue_has_the_bits_of_wide_ones(be, m, n, k):
+    """More 128 x 128 tiles than compute units, whose 256 x 128 tiles are one round: the residual and both SwiGLU epilogues against
+    a corner of an output of 192 tiles and more, with remainders in rows, columns (backward) and contraction, and with the
+    residual in row runs."""
+    M, f = 4096, n // 2
+    F = max(3584, f)
+    x, gate, up = rnd(M, k, seed=61), rnd(F, k, scale=0.05, seed=62), rnd(F, k, scale=0.05, seed=63)
+    xs, ws = x[:m].contiguous(), torch.cat([gate[:f], up[:f]])
+    assert _gemm_tile(be, 0, m, n, k, 2) == (256, 128, 1)
+    y, big_y = (torch.empty(r, c, device=DEV, dtype=torch.bfloat16) for r, c in ((m, f), (M, F)))
+    got, big = be.linear_fwd(xs, ws, swiglu_out=y), be.linear_fwd(x, torch.cat([gate, up]), swiglu_out=big_y)
+    assert torch.equal(got[:, :f], big[:m, :f]) and torch.equal(got[:, f:], big[:m, F:F + f]) and torch.equal(y, big_y[:m, :f])
+    c = n - 8  # a remainder in columns
+    res, w = rnd(M, 2 * F, seed=65), torch.cat([gate, up])
+    assert _gemm_tile(be, 0, m, c, k, 1)[:2] == (256, 128) and max(_gemm_tile(be, 0, M, 2 * F, k, 1)[:2]) == 256
+    want = be.linear_fwd(x, w, residual=res)[:m, :c]
+    assert torch.equal(be.linear_fwd(xs, w[:c].contiguous(), residual=res[:m, :c].contiguous()), want)
+    runs = torch.zeros(m // 4, 8, c, device=DEV, dtype=torch.bfloat16)[:, 2:6]
+    runs.copy_(res[:m, :c].reshape(m // 4, 4, c))
+    assert torch.equal(be.linear_fwd(xs, w[:c].contiguous(), residual=runs), want)
+    dy, wb, pre = rnd(M, k, seed=66), rnd(k, 2 * F, scale=0.05, seed=67), rnd(M, 4 * F, seed=68)
+    assert _gemm_tile(be, 1, m, c, k, 4) == (256, 128, 1) and _gemm_plan(be, M, 2 * F, k, 4)[0] == 256
+    pre_s = torch.cat([pre[:m, :c], pre[:m, 2 * F:2 * F + c]], dim=1)
+    got = be.linear_dgrad(dy[:m].contiguous(), wb[:, :c].contiguous(), swiglu_bwd_x=pre_s)
+    big = be.linear_dgrad(dy, wb, swiglu_bwd_x=pre)
+    assert torch.equal(got[:, :c], big[:m, :c]) and torch.equal(got[:, c:], big[:m, 2 * F:2 * F + c])
+
+
 @pytest.mark.parametrize("layout", [0, 1, 2])
 @pytest.mark.parametrize("steps,tail", [(151, 64), (151, 8), (152, 40), (153, 64), (153, 24), (154, 8), (155, 64), (159, 56)])
 def test_gemm_deep_ring_cut_into_short_last_ranges(be, layout, steps, tail):
