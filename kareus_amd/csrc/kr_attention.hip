@@ -36,24 +36,50 @@ constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kRescaleSlack = 8.0f;
 constexpr int kXcds = 8;
 
-__device__ __forceinline__ int xcd_contiguous_id(int pid, int nblocks) {
-  const int q = nblocks / kXcds, r = nblocks % kXcds;
-  const int xcd = pid % kXcds;
-  return xcd * q + (xcd < r ? xcd : r) + pid / kXcds;
-}
-
-// Workgroup -> (query tile, (batch, head) pair), longest causal rows first.  With fewer than 32
-// tiles per pair an XCD starts its 32 compute units on the longest tiles of `grp` pairs at once,
-// and the short tiles that follow land on the units that finish first.
-__device__ __forceinline__ void longest_first(int lid, int nqt, int total_pairs, int& qt, int& pair) {
-  const int grp = (nqt < 32 && 32 % nqt == 0) ? 32 / nqt : 1;
-  const int span = grp * nqt, base = lid / span, i = lid % span;
+// Workgroup -> (rank of its tile by the length of its causal rows or columns, 0 the longest; (batch, head) pair).  An XCD has a
+// contiguous range of the pairs' tiles, so that what pairs share stays in its L2, and starts with the longest of all its pairs:
+// short ones fill up the units that finish first.  With more than sixteen pairs (and more than two workgroups for each of its 32
+// units) what the pairs read no longer fits the L2: 32 / ntiles of them start at once, and the others follow.
+// Rows of each pair in sequence -> this order, us, dQ, forward and dK/dV at head dimension 128: 3 x 2008 tokens of 8/2 heads 67
+// -> 54, 58 -> 45, 92 -> 84; dK/dV 6 x 4096 of 3/1 heads 249 -> 180, 4 x 4096 of 24/8 heads 867 -> 843; two pairs at once -> this
+// order, 2 x 8192 of 32/8 heads forward 1016 -> 978, dQ 1363 -> 1330.  All pairs at once beyond sixteen: 64 x 512 tokens of 32/8
+// heads forward 276 -> 300, dK/dV 366 -> 411.
+__device__ __forceinline__ void longest_first(int pid, int nblocks, int ntiles, int& rank, int& pair) {
+  const int q = nblocks / kXcds, r = nblocks % kXcds, xcd = pid % kXcds;
+  const int first = xcd * q + (xcd < r ? xcd : r), count = q + (xcd < r ? 1 : 0), i = pid / kXcds;
+  if (count <= 64 || count <= 16 * ntiles) {
+    // ids first .. first + count - 1, id = pair * ntiles + rank: every rank `full` times, `extra` ranks from that of the
+    // first id on (cyclically) once more.  Ranks [0, a) occur na times, [a, b) nb times, the others na times again.
+    const int start = first % ntiles, full = count / ntiles, extra = count - full * ntiles;
+    const bool wraps = start + extra > ntiles;
+    const int a = wraps ? start + extra - ntiles : start, b = wraps ? start : start + extra;
+    const int na = wraps ? full + 1 : full, nb = wraps ? full : full + 1;
+    int at = i, from = 0, n = na;
+    if (at >= a * na) {
+      at -= a * na;
+      from = a;
+      n = nb;
+      if (at >= (b - a) * nb) {
+        at -= (b - a) * nb;
+        from = b;
+        n = na;
+      }
+    }
+    const int row = at / n;
+    rank = from + row;
+    const int ahead = rank - start;
+    pair = (first + (ahead < 0 ? ahead + ntiles : ahead)) / ntiles + (at - row * n);
+    return;
+  }
+  const int lid = first + i, total_pairs = nblocks / ntiles;
+  const int grp = (ntiles < 32 && 32 % ntiles == 0) ? 32 / ntiles : 1;
+  const int span = grp * ntiles, base = lid / span, at = lid % span;
   if ((base + 1) * grp <= total_pairs) {
-    qt = nqt - 1 - i / grp;
-    pair = base * grp + i % grp;
+    rank = at / grp;
+    pair = base * grp + at % grp;
   } else {  // a last, incomplete group keeps the plain order
-    qt = nqt - 1 - (lid % nqt);
-    pair = lid / nqt;
+    rank = lid % ntiles;
+    pair = lid / ntiles;
   }
 }
 
@@ -399,10 +425,11 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nqt = (s + BQ - 1) / BQ;
-  const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int qt = nqt - 1 - (lid % nqt);  // longest rows first inside each (batch, head)
-  const int head = (lid / nqt) % nq;
-  const int bi = lid / (nqt * nq);
+  int rank, pair;
+  longest_first(blockIdx.x, gridDim.x, nqt, rank, pair);
+  const int qt = nqt - 1 - rank;
+  const int head = pair % nq;
+  const int bi = pair / nq;
   const int per = nq / nkv;
   const int kvh = head / per, hj = head % per;
 
@@ -726,8 +753,9 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
   const int lane = tid & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nqt = (s + BQ2 - 1) / BQ2;
-  int qt, pair;
-  longest_first(xcd_contiguous_id(blockIdx.x, gridDim.x), nqt, gridDim.x / nqt, qt, pair);
+  int rank, pair;
+  longest_first(blockIdx.x, gridDim.x, nqt, rank, pair);
+  const int qt = nqt - 1 - rank;
   const int head = pair % nq;
   const int bi = pair / nq;
   const int per = nq / nkv;
@@ -1047,17 +1075,18 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   const int wave = wave8 & 3;   // key block of the tile
   const int sp = RAGGED ? (s + 127) / 128 * 128 : s;  // rows of the statistics and of the partial results
   const int nkt = sp / 128;
-  const int lid_all = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int part = lid_all % qsplit, lid = lid_all / qsplit;
+  // (a key tile's parts count as tiles of half its length; low key tiles see the most queries)
+  int rank, hg;
+  longest_first(blockIdx.x, gridDim.x, nkt * qsplit, rank, hg);
+  const int part = rank % qsplit, kt = rank / qsplit;
   // A workgroup takes `hpw` consecutive query heads of one KV group, one after the other: its K / V
   // fragments and its dK / dV accumulators serve them all, so a group leaves per / hpw partial
   // results instead of per (none at all when hpw = per), and the workgroup's start and end are
   // paid once for hpw heads.  The host picks hpw so that enough workgroups remain.
-  const int kt = lid % nkt;  // low key tiles see the most queries: they come first
   const int nhg = nq / hpw;
-  const int hgroup = (lid / nkt) % nhg;
+  const int hgroup = hg % nhg;
   const int head = hgroup * hpw;  // the first of this workgroup's heads
-  const int bi = lid / (nkt * nhg);
+  const int bi = hg / nhg;
   const int per = nq / nkv;
   const int kvh = head / per;
   const int key0 = kt * 128;
@@ -1399,11 +1428,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv64_kernel(
   const int wave = wave8 & 3, half = wave8 >> 2;  // key block of the tile; which 64 queries of a tile
   const int sp = RAGGED ? (s + 127) / 128 * 128 : s;  // rows of the statistics and of the partial results
   const int nkt = sp / 128;
-  const int lid_all = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int part = lid_all % qsplit;
-  int kt_rev, hg;
-  longest_first(lid_all / qsplit, nkt, gridDim.x / (nkt * qsplit), kt_rev, hg);
-  const int kt = nkt - 1 - kt_rev;  // low key tiles see the most queries
+  int rank, hg;
+  longest_first(blockIdx.x, gridDim.x, nkt * qsplit, rank, hg);
+  const int part = rank % qsplit, kt = rank / qsplit;  // low key tiles see the most queries
   const int nhg = nq / hpw;
   const int hgroup = hg % nhg;
   const int head = hgroup * hpw;  // `hpw` consecutive query heads of one KV group, one after the other
@@ -1760,9 +1787,9 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
   constexpr int ROWS = BQ;  // queries per workgroup
   const int sp = RAGGED ? (s + 127) / 128 * 128 : s;
   const int nqt = sp / ROWS;
-  const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int qt = nqt - 1 - (lid % nqt);
-  const int pair = lid / nqt;
+  int rank, pair;
+  longest_first(blockIdx.x, gridDim.x, nqt, rank, pair);
+  const int qt = nqt - 1 - rank;
   const int head = pair % nq;
   const int bi = pair / nq;
   const int per = nq / nkv;
@@ -2058,9 +2085,9 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int sp = RAGGED ? (s + 127) / 128 * 128 : s;  // rows of the statistics (whole 256-query tiles here)
   const int nqt = sp / ROWS;
-  const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  int qt, pair;
-  longest_first(lid, nqt, gridDim.x / nqt, qt, pair);
+  int rank, pair;
+  longest_first(blockIdx.x, gridDim.x, nqt, rank, pair);
+  const int qt = nqt - 1 - rank;
   const int head = pair % nq;
   const int bi = pair / nq;
   const int per = nq / nkv;
@@ -2549,13 +2576,20 @@ __global__ __launch_bounds__(256) void attn_resize_rows_kernel(const float* __re
 // dimension 64 the halves of a workgroup share a key tile's queries already, so that pays only for long rows (whole -> split,
 // with the launch that adds, us): 8 heads at s 200, b 2 10.2 -> 13.5, at s 1000 19.3 -> 18.9, at s 1000, b 4 21.8 -> 33.7;
 // at s 1536 23.1 -> 24.9; one head at s 4096 47.0 -> 32.6, 4 heads 50.2 -> 38.4; 4/2 heads at s 2048 32.5 -> 23.7.
-static int dkdv_query_split(int s, int b, int nq, int hd) {
-  const int key_tiles = (s / 128) * nq * b;
-  if (hd == 64) return key_tiles <= 128 && s >= 2048 ? 2 : 1;
-  return key_tiles <= 2 * 256 ? 2 : 1;
+// At head dimension 128, by the number of (key tile, head) pairs against the units (us with the launch that adds; whole and split,
+// 2h: with two heads of a group to a workgroup).  Fewer pairs than units: split (64 64, 44; 128 119, 88; 192 at s 1504 63, 45),
+// but not short rows that leave few units idle (192 at s 512 28, 32).  One each: long rows (s 2048 69, 60; s 1024 45, 49).  More:
+// whole (384 at s 2048 81 and 92, 102 and 113; at s 4096 149, 160).  Two each: 2h (s 2048 99, 92; s 4096 158, 150), where the XCDs get
+// equal shares of it (4 head groups at s 8192 270, 348).
+static int dkdv_query_split(int s, int b, int nq, int nkv, int hd) {
+  const int key_tiles = s / 128, pairs = key_tiles * nq * b, cus = kr_compute_units();
+  if (hd == 64) return pairs <= 128 && s >= 2048 ? 2 : 1;
+  if (pairs < cus) return 2 * pairs <= cus || key_tiles >= 8 ? 2 : 1;
+  if (4 * pairs < 5 * cus) return key_tiles >= 16 ? 2 : 1;
+  return pairs == 2 * cus && (nq / nkv) % 2 == 0 && (nq / 2 * b) % kXcds == 0 ? 2 : 1;
 }
-// ... and how many the workspace has room for, at any head dimension
-static int dkdv_query_split_reserved(int s, int b, int nq) { return dkdv_query_split(s, b, nq, HD); }
+// how many the workspace has room for
+static int dkdv_query_split_reserved(int s, int b, int nq) { return (s / 128) * nq * b <= 2 * 256 ? 2 : 1; }
 
 static int attn_padded_len(int s) { return (s + BQ - 1) / BQ * BQ; }
 // bytes of one padded [s_pad, b, heads, 128] bf16 tensor / of the padded statistics [b, nq, s_pad]
@@ -2642,13 +2676,17 @@ struct AttnForms {
   bool shared_fwd, shared_dq;
   int qsplit;
 };
-static AttnForms attn_forms(int s, int b, int nq, int hd, int flags) {  // s: rounded up to whole 128-row tiles
+// One 256-query tile for every unit is not enough for the unsplit forms unless the rows are short: the longest row is then the
+// launch (split forms -> unsplit, us: 8 pairs at s 8192 forward 134 -> 183, dQ 199 -> 247; 32 pairs at s 2048 47 -> 54, 68 -> 88;
+// 64 at s 1024 30 -> 31, 44 -> 45; 128 at s 512 24 -> 20, 30 -> 32; at nine eighths of that, 32 pairs at s 2304, 67 -> 65, 104 -> 91).
+static AttnForms attn_forms(int s, int b, int nq, int nkv, int hd, int flags) {  // s: rounded up to whole 128-row tiles
   const bool beside = (flags & KR_ATTN_BESIDE_OTHER_STREAMS) != 0;
-  const int tiles256 = (s / 256) * nq * b;
+  const int tiles256 = (s / 256) * nq * b, cus = kr_compute_units();
+  const bool unsplit = s % 256 == 0 && (beside || tiles256 > cus || (tiles256 == cus && s <= 1024));
   AttnForms f;
-  f.shared_fwd = s % 256 == 0 && (beside || tiles256 >= kr_compute_units());
-  f.shared_dq = s % 256 == 0 && (beside || tiles256 >= kr_compute_units());
-  f.qsplit = beside ? 1 : dkdv_query_split(s, b, nq, hd);
+  f.shared_fwd = f.shared_dq = unsplit;
+  const int split = beside ? 1 : dkdv_query_split(s, b, nq, nkv, hd), room = dkdv_query_split_reserved(s, b, nq);
+  f.qsplit = split < room ? split : room;
   return f;
 }
 
@@ -2682,7 +2720,7 @@ int attn_bwd_mfma(const BwdCall& c) {
   const int64_t rows = (int64_t)b * nq * sp;
   float* neg_lse2 = neg_delta + rows;
   float* part_k = neg_lse2 + rows;
-  const AttnForms forms = attn_forms(sp, b, nq, D, c.flags);
+  const AttnForms forms = attn_forms(sp, b, nq, c.nkv, D, c.flags);
   const int qsplit = forms.qsplit;
   float* part_v = part_k + rows * qsplit * D;
   // query heads of a KV group per dK/dV workgroup: as many as leave two workgroups per compute
@@ -2898,7 +2936,7 @@ struct FwdCall {
 template <int D, bool RAGGED>
 int attn_fwd_mfma(const FwdCall& c) {
   const int s = c.s, b = c.b, nq = c.nq, sp = attn_padded_len(s);
-  if (attn_forms(sp, b, nq, D, c.flags).shared_fwd) {
+  if (attn_forms(sp, b, nq, c.nkv, D, c.flags).shared_fwd) {
     // 256-query tiles (one for every compute unit, or other streams beside): the halves share their K / V tiles
     constexpr size_t lds_sh = 3 * 16 * ((1024 + 16) + (1024 + 64));  // 100 KiB
     static const hipError_t attr_sh = hipFuncSetAttribute(

@@ -903,6 +903,29 @@ def test_attention_in_place_at_head_dimension_64_and_ragged_lengths(be, s, b, nq
     assert rel(dq.flatten(2, 3), qf.grad) <= TOL and rel(dk, kf.grad) <= TOL and rel(dv, vf.grad) <= TOL
 
 
+@pytest.mark.parametrize("s,b,nq,nkv,hd", [(1152, 5, 3, 1, 128),     # 15 pairs of 9 tiles: an XCD's range starts and ends inside a pair
+                                           (1152, 5, 3, 1, 64), (904, 7, 2, 2, 128), (136, 1, 2, 1, 128),
+                                           (2048, 5, 8, 2, 128),     # more than 64 workgroups per XCD, of at most 16 pairs
+                                           (256, 70, 8, 2, 128),     # ... of more pairs
+                                           (2048, 4, 8, 2, 128)])    # a 256-query tile for every unit: split forms, two heads per workgroup
+def test_attention_over_orders_of_workgroups(be, s, b, nq, nkv, hd):
+    """Every tile of every (batch, head) pair is computed once, whatever part of the pairs an XCD has: a tile left out or taken
+    twice for another is far outside the tolerance (every tensor is filled before it is written)."""
+    _, q, k, v = _grouped(s, b, nq, nkv, hd, seed=140)
+    do = rnd(s, b, nq, hd, seed=141)
+    scale = hd ** -0.5
+    qf, kf, vf = (t.float().cpu().clone().requires_grad_(True) for t in (q.flatten(2, 3), k, v))
+    ro, rlse = R.causal_gqa_attention(qf, kf, vf, return_lse=True)
+    ro.backward(do.float().cpu())
+    for beside in (False, True):
+        trash = [torch.full((s * b * nq * hd * 4,), float("nan"), device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+        del trash     # (what the allocator hands out next held NaN)
+        o, lse = be.attn_fwd(q, k, v, scale, beside_other_streams=beside)
+        assert rel(o, ro) <= TOL and rel(lse, rlse) <= 1e-4
+        dq, dk, dv = be.attn_bwd(do, q, k, v, o, lse, scale, beside_other_streams=beside)
+        assert rel(dq.flatten(2, 3), qf.grad) <= TOL and rel(dk, kf.grad) <= TOL and rel(dv, vf.grad) <= TOL
+
+
 @pytest.mark.parametrize("s,b,nq,nkv", [(256, 1, 2, 1), (384, 1, 2, 2),          # two and three query tiles: the ring of four stages starts
                                         (640, 2, 4, 2), (2048, 8, 2, 1),         # ... and turns over
                                         (2056, 1, 4, 2), (2304, 1, 2, 2),        # few key tiles, long rows: two workgroups a key tile
