@@ -32,7 +32,7 @@ __global__ __launch_bounds__(kThreads) void embedding_fwd_kernel(const int64_t* 
 
 // ---- embedding backward ------------------------------------------------------------------------
 // dweight[r, :] = sum over tokens t with ids[t] - vocab_start == r of dout[t, :], rows without a
-// token are written as zeros.  No atomics on the result: a workgroup owns kRowsPerBlock
+// token are written as zeros.  No atomics on the result: a workgroup owns rows_per_block
 // consecutive vocabulary rows.  It scans all ids once (memory order, [b, s]) and collects the
 // tokens that fall into its rows as (row, position) keys in LDS, sorts the keys (bitonic), then
 // walks them row by row, adding each row's tokens in position order with fp32 accumulators and
@@ -41,28 +41,42 @@ __global__ __launch_bounds__(kThreads) void embedding_fwd_kernel(const int64_t* 
 // re-scanning the ids once per row, still in position order.
 // Bytes: dout read once in total (each token belongs to one row) + dweight written once + the id
 // array re-read by every workgroup out of L2.
-constexpr int kRowsPerBlock = 64;
+// A workgroup is a chain of waits: the scan, its tokens' rows one after the other, its stores.  Few rows per workgroup keep
+// eight of them on every compute unit, and the scan asks for eight ids per thread at once.  us, 64 rows and one id at a time
+// -> now (floor: bytes at the rate of a copy): 32064 x 4096, 4096 tokens 78 -> 54 (58), 16384 tokens 141 -> 67 (78); 32064 x
+// 2048, 4096 tokens 31 -> 24 (29); 16384 x 3072, 8192 tokens 64 -> 31 (30), 32768 tokens 232 -> 75 (59); 4096 x 512, 512 tokens
+// 20 -> 7.5.
+constexpr int kIdsAtOnce = 8;
 constexpr int kListCap = 4096;   // keys held in LDS (a power of two, for the bitonic sort)
 constexpr int kPosBits = 26;     // key = row_in_block << 26 | position; positions < 2^26
-template <int VECS>              // hidden / 8 <= 256 * VECS
+template <int VECS, bool STREAM>  // hidden / 8 <= 256 * VECS; non-temporal stores (a run-time choice is merged into plain ones)
 __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* __restrict__ ids,
                                                                 const bf16* __restrict__ dout,
                                                                 bf16* __restrict__ dweight, int s,
                                                                 int b, int hidden, int64_t vocab_start,
-                                                                int64_t vocab_rows) {
+                                                                int64_t vocab_rows, int rows_per_block) {
   __shared__ unsigned keys[kListCap];
   __shared__ int count;
   const int tid = threadIdx.x;
-  const int64_t row0 = (int64_t)blockIdx.x * kRowsPerBlock;
+  const int64_t row0 = (int64_t)blockIdx.x * rows_per_block;
   const int64_t tokens = (int64_t)s * b;
   const int nvec = hidden / 8;
   if (tid == 0) count = 0;
   __syncthreads();
-  for (int64_t t = tid; t < tokens; t += kThreads) {
-    const int64_t d = ids[t] - vocab_start - row0;
-    if (d >= 0 && d < kRowsPerBlock) {
-      const int slot = atomicAdd(&count, 1);
-      if (slot < kListCap) keys[slot] = ((unsigned)d << kPosBits) | (unsigned)t;
+  for (int64_t t0 = tid; t0 < tokens; t0 += kIdsAtOnce * kThreads) {
+    int64_t id[kIdsAtOnce];
+#pragma unroll
+    for (int c = 0; c < kIdsAtOnce; ++c) {
+      const int64_t t = t0 + c * kThreads;
+      id[c] = ids[t < tokens ? t : tokens - 1];
+    }
+#pragma unroll
+    for (int c = 0; c < kIdsAtOnce; ++c) {
+      const int64_t t = t0 + c * kThreads, d = id[c] - vocab_start - row0;
+      if (t < tokens && d >= 0 && d < rows_per_block) {
+        const int slot = atomicAdd(&count, 1);
+        if (slot < kListCap) keys[slot] = ((unsigned)d << kPosBits) | (unsigned)t;
+      }
     }
   }
   __syncthreads();
@@ -104,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
     }
   };
   int next = 0;
-  for (int r = 0; r < kRowsPerBlock && row0 + r < vocab_rows; ++r) {
+  for (int r = 0; r < rows_per_block && row0 + r < vocab_rows; ++r) {
 #pragma unroll
     for (int c = 0; c < VECS; ++c)
 #pragma unroll
@@ -144,7 +158,10 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
         bf16x8 o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = (bf16)acc[c][e];
-        stg8(dst + v * 8, o);
+        if constexpr (STREAM)
+          stg8_stream(dst + v * 8, o);
+        else
+          stg8(dst + v * 8, o);
       }
     }
   }
@@ -249,15 +266,26 @@ extern "C" int kr_embedding_fwd(const int64_t* ids, const void* weight, void* ou
   return kr_launch_status();
 }
 
+// Eight rows: every workgroup scans all ids, which costs more than it gains beyond 8192 tokens (8 and 16 rows, us: 16384 x 3072,
+// 8192 tokens 31, 32; 32064 x 2048, 16384 tokens 48, 40, 32768 tokens 83, 61).
+static int embedding_rows_per_block(int64_t tokens) { return tokens <= 8192 ? 8 : 16; }
+// Whether the launch's rows are stored with the non-temporal hint: where what it reads and writes is more than the 256 MB
+// memory-side cache holds (plain and hinted stores, us: 32064 x 4096, 776 tokens, 269 MB 39, 52; 4096 tokens, 296 MB 65, 54;
+// 16384 x 3072, 16384 tokens, 201 MB 46, 50, 32768 tokens, 302 MB 96, 75).
+static bool embedding_streams(int64_t rows, int hidden) { return 2 * rows * hidden > (int64_t)280 << 20; }
+
 extern "C" int kr_embedding_bwd(const int64_t* ids, const void* dout, void* dweight, int s, int b,
                                 int hidden, int64_t vocab_start, int64_t vocab_rows, void* stream) {
   if (!ids || !dout || !dweight || s <= 0 || b <= 0 || hidden <= 0 || vocab_rows <= 0) return KR_EINVAL;
   if (hidden % 8 || hidden > 8192 || (int64_t)s * b >= ((int64_t)1 << kPosBits)) return KR_EUNSUPPORTED;
   if (!kr_aligned16(dout) || !kr_aligned16(dweight)) return KR_EINVAL;
-  const unsigned blocks = (unsigned)((vocab_rows + kRowsPerBlock - 1) / kRowsPerBlock);
+  const int rows_per_block = embedding_rows_per_block((int64_t)s * b);
+  const bool stream_out = embedding_streams(vocab_rows + (int64_t)s * b, hidden);
+  const unsigned blocks = (unsigned)((vocab_rows + rows_per_block - 1) / rows_per_block);
 #define KR_EMB_BWD(C)                                                                               \
-  hipLaunchKernelGGL(embedding_bwd_kernel<C>, dim3(blocks), dim3(kThreads), 0, (hipStream_t)stream, \
-                     ids, (const bf16*)dout, (bf16*)dweight, s, b, hidden, vocab_start, vocab_rows)
+  hipLaunchKernelGGL((stream_out ? embedding_bwd_kernel<C, true> : embedding_bwd_kernel<C, false>), dim3(blocks),           \
+                     dim3(kThreads), 0, (hipStream_t)stream, ids, (const bf16*)dout, (bf16*)dweight, s, b, hidden,         \
+                     vocab_start, vocab_rows, rows_per_block)
   if (hidden <= 2048) KR_EMB_BWD(1);
   else if (hidden <= 4096) KR_EMB_BWD(2);
   else KR_EMB_BWD(4);

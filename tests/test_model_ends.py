@@ -138,6 +138,22 @@ def test_embedding_kernels(b, s, hidden, rows, start):
 
 
 @gpu
+@pytest.mark.parametrize("b,s,hidden,rows,start", [(1, 1, 64, 9, 0), (1, 2049, 64, 23, 8), (3, 2731, 128, 41, 8),  # 8193 tokens: 16 rows per workgroup
+                                                   (2, 2048, 4096, 32064, 0)])  # more than the memory-side cache: non-temporal stores
+def test_embedding_gradient_over_rows_per_workgroup(b, s, hidden, rows, start):
+    """Sums in position order, whatever the split of the rows: the bits of an in-order sum in fp32, rounded once."""
+    be = get_backend("hip")
+    g = torch.Generator().manual_seed(6)
+    ids = torch.randint(0, rows + 2 * start, (b, s), generator=g)
+    dout = torch.randn(s, b, hidden, generator=g).bfloat16()
+    want = torch.zeros(rows, hidden)
+    for t, i in enumerate((ids.reshape(-1) - start).tolist()):
+        if 0 <= i < rows:
+            want[i] += dout[t % s, t // s].float()
+    assert torch.equal(be.embedding_bwd(ids.cuda(), dout.cuda(), rows, start).cpu(), want.bfloat16())
+
+
+@gpu
 def test_embedding_backward_with_heavily_repeated_ids():
     """A block of 64 vocabulary rows that attracts more tokens than its LDS key list holds (4096) falls
     back to one in-order scan per row; a sparse block in the same launch takes the sorted-list path."""
