@@ -207,6 +207,10 @@ __device__ __forceinline__ uint32_t lds_addr(const bf16* p) {
 // clamped to the last valid row; a chunk that would start beyond the contraction range
 // (k_left = elements from the K-step's base to the end, >= 8) is redirected to a valid address —
 // it is zeroed in LDS afterwards, so what it fetches does not matter.
+// A transposed tile of 160 to 224 columns (`cols`) lies in rows of 256, and its loads span them: a lane whose columns the tile does
+// not use fetches some that another lane of its row fetches, so that a row of 160 columns takes three cache lines instead of four.
+// us: 3072 x 3072 x 16384 (NT, 160 columns) 294 -> 262, 2048 x 768 x 32768 (192, cut) 111 -> 107, 1536 x 4096 x 16384 (224, cut)
+// 187 -> 182; where the matrix pipes or the epilogue bound it the same (16384 x 3584 x 4096 with the SwiGLU backward 431 -> 431).
 // gate_up_f > 0 (K-major B of a fused SwiGLU projection, weight rows [gate: 0..F) | up: F..2F)):
 // the first `half_rows` rows of the tile hold the gate rows row0 .., the next `half_rows` the up rows
 // of the same output columns, so that the waves of the tile's left half end up with gate values
@@ -225,7 +229,7 @@ __device__ __forceinline__ int load_krow(int i, int wave, int lane) {
 template <bool TRANSPOSED, int TW>
 __device__ __forceinline__ uint32_t load_offset(int i, int wave, int lane, int ld, int row0,
                                                 int rows_total, int k_left, int gate_up_f = 0,
-                                                int half_rows = 0, int sh = 0, int outer = 0) {
+                                                int half_rows = 0, int sh = 0, int outer = 0, int cols = TW) {
   if (!TRANSPOSED) {
     const int row = 8 * wave + (lane >> 3) + 32 * i;
     int chunk = ((lane & 7) ^ ((row >> 1) & 7)) * 8;
@@ -238,7 +242,9 @@ __device__ __forceinline__ uint32_t load_offset(int i, int wave, int lane, int l
   // (the contraction rows of a K-step start at a multiple of 64, hence of the run length: the
   // position inside the K-step maps like a row of its own)
   int krow = load_krow<TW>(i, wave, lane);
-  int c = row0 + ((lane & (TW / 8 - 1)) ^ transp_swz<TW>(krow)) * 8;
+  int chunk = (lane & (TW / 8 - 1)) ^ transp_swz<TW>(krow);
+  if (cols < TW && chunk * 8 >= cols) chunk -= 16;
+  int c = row0 + chunk * 8;
   c = c + 8 <= rows_total ? c : rows_total - 8;
   krow = krow < k_left ? krow : k_left - 1;
   return (uint32_t)((sh ? run_off(krow, ld, sh, outer) : krow * ld) + c);
@@ -480,7 +486,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       if (i < NA_LOADS) la[i] = 2u * load_offset<A_T, TW>(i, wave, l2, lda, m0, M, k_left, 0, 0, runs.a_sh, runs.a_outer);
-      if (i < NB_LOADS) lb[i] = 2u * load_offset<B_T, TWB>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN);
+      if (i < NB_LOADS) lb[i] = 2u * load_offset<B_T, TWB>(i, wave, l2, ldb, n0, N, k_left, gate_up_f, 16 * WN, 0, 0, B_T && TWB == 256 ? 32 * WN : TWB);
     }
   };
   // the first `count` loads of a tile (NA_LOADS for A, NB_LOADS for B)
