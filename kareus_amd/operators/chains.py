@@ -251,15 +251,11 @@ class _BackwardChain(_Chain):
     """``run`` returns the parameter gradients by op id, or None where the chain did not run."""
 
     def _contexts(self, ctx) -> Optional[List]:
-        """The operators' contexts, if every one needs a gradient and the weight gradients are summed, where several
-        nanobatches are, on one stream."""
+        """The operators' contexts, if every one needs a gradient."""
         ctxs = [ctx.op_contexts[p.op_id] for p in self.plans]
         for c in ctxs:
             if not c.requires_grad:
                 return None
-        sink = getattr(ctxs[0], "wgrad_sink", None)
-        if sink is not None and sink["n"] > 1 and not sink.get("in_line"):
-            return None
         return ctxs
 
     def _finish(self, store, ctxs, dy, dx, protected, released: bool) -> None:
@@ -300,12 +296,12 @@ class _BackwardBehindAdd:
 
 
 def _add_pair(be, linear, ctx, dy, x):
-    """The weight gradient of a projection over nanobatches that run one after the other on one stream
-    (PartitionableLinear._weight_grad without the events): the pair is left in the layer's sink, and the last nanobatch
-    contracts all of them in nanobatch order."""
+    """The weight gradient of a projection over nanobatches.  On streams of their own it is PartitionableLinear._weight_grad, whose
+    event then lies behind the chain's input gradients.  On one stream the pair is left in the layer's sink without events, and
+    the last nanobatch contracts all of them in nanobatch order."""
     sink = ctx.wgrad_sink
     n = sink["n"]
-    if not sink["defer"] or sink["pending"] is not None:
+    if not sink.get("in_line") or not sink["defer"] or sink["pending"] is not None:
         return PartitionableLinear._weight_grad(be, ctx, dy, x, linear._split(ctx))
     pairs = sink.get("pairs")
     if pairs is None:

@@ -330,6 +330,29 @@ def test_a_chain_has_the_bits_of_its_operators(what, monkeypatch):
         assert ran["_BackwardAttention"] == ran["_BackwardMlp"] == passes
 
 
+ON_STREAMS = {
+    "two": (config(2), 96, 4),
+    "two, tokens no multiple of 64, per-head norms, dropout": (config(2, qk_layernorm=True, hidden_dropout=0.2), 104, 2),
+    "four, weight gradients at the end": (config(4), 64, 4),                # (their launches are left to the end of the pass)
+    "four, weight gradients at once": (config(4, wgrad_launches_at_end=False), 64, 4),
+    "accumulated weight gradients": (config(2, wgrad_over_all_nanobatches=False), 96, 4),
+    "gradients summed by autograd": (config(2, fuse_wgrad_accumulation=False), 96, 4),
+    "recomputation": (config(2, checkpoint_activations=True), 96, 4),
+}
+
+
+@pytest.mark.parametrize("what", sorted(ON_STREAMS))
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_backward_chains_of_nanobatches_on_streams(what, monkeypatch):
+    """Every nanobatch's backward chains run on its own stream; the operands of the weight gradients meet in the layer's sink with
+    the events behind them."""
+    cfg, s, b = ON_STREAMS[what]
+    cfg = dataclasses.replace(cfg, in_line_below_ms=0.0)
+    ran = both(monkeypatch, cfg, s, b)
+    assert ran["_BackwardAttention"] == ran["_BackwardMlp"] == 2 * cfg.num_layers * cfg.num_nanobatches
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
 def test_chains_without_gradients_and_under_saved_tensor_hooks(monkeypatch):
