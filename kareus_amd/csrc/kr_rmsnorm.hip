@@ -28,7 +28,8 @@ __device__ __forceinline__ int64_t row_at(int64_t row, int64_t ld, Runs r) {
   return r.sh ? (row >> r.sh) * r.outer + (row & ((1 << r.sh) - 1)) * ld : row * ld;
 }
 
-template <int NCHUNK>
+// KEEP: plain stores for small results, which the next launch finds in the memory-side cache (see rmsnorm_fwd_impl).
+template <int NCHUNK, bool KEEP>
 __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_kernel(const bf16* __restrict__ x,
                                                                const bf16* __restrict__ gamma,
                                                                bf16* __restrict__ y,
@@ -71,7 +72,10 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_kernel(const bf16* __res
         bf16x8 o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = (bf16)(((float)xv[c][e] * rs) * (float)g[c][e]);
-        stg8_stream(yr + v * 8, o);
+        if constexpr (KEEP)
+          stg8(yr + v * 8, o);
+        else
+          stg8_stream(yr + v * 8, o);
       }
     }
   }
@@ -309,8 +313,11 @@ int rmsnorm_fwd_impl(const void* x, const void* gamma, void* y, float* rstd, int
   int blocks = (rows + kWaves - 1) / kWaves;
   if (blocks > 256 * 8) blocks = 256 * 8;
   const int nc = chunks_for(cols);
-  KR_DISPATCH_CHUNKS(nc, hipLaunchKernelGGL(rmsnorm_fwd_kernel<C_>, dim3(blocks), dim3(kThreads), 0,
-                                           (hipStream_t)stream, (const bf16*)x, (const bf16*)gamma,
+  // up to 16 MB of result stay in the caches for the projection behind the norm (figures at stg8_out in kr_gemm.hip; at 64 MB
+  // and more the hint is what is faster: see kr_common.h)
+  const bool keep = (int64_t)rows * cols <= (int64_t)8 << 20;
+  KR_DISPATCH_CHUNKS(nc, hipLaunchKernelGGL((keep ? rmsnorm_fwd_kernel<C_, true> : rmsnorm_fwd_kernel<C_, false>), dim3(blocks),
+                                           dim3(kThreads), 0, (hipStream_t)stream, (const bf16*)x, (const bf16*)gamma,
                                            (bf16*)y, rstd, rows, cols, x_ld, eps, x_runs));
   return kr_launch_status();
 }
