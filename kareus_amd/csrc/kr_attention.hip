@@ -194,8 +194,8 @@ static bool attn_fast_path(int s, int hd) { return hd == HD && s % BQ == 0; }
 // copy into padded buffers of 128 channels and whole tiles and back (nine to eleven small launches, and half
 // of the matrix work on zeros where D = 64).  Measured, padded -> in place, forward / backward in us:
 //   s 256, b 1, 8/8 heads of 64       28 / 57     ->   9 / 22     (launches)
-//   s 2048, b 1, 32/8 heads of 64     75 / 190    ->  37 / 106
-//   s 4096, b 2, 32/8 heads of 64    282 / 909    -> 171 / 556    (0.80 / 0.62 PFLOP/s)
+//   s 2048, b 1, 32/8 heads of 64     75 / 190    ->  35 / 100
+//   s 4096, b 2, 32/8 heads of 64    282 / 909    -> 171 / 495    (0.80 / 0.69 PFLOP/s)
 //   s 776, b 1, 8/2 heads of 128      31 / 78     ->  20 / 53
 //   s 4000, b 4, 8/2 heads of 128    167 / 532    -> 145 / 485    (whole tiles, s 4096: 133 / 470)
 //   s 8184, b 2, 32/8 heads of 128  1121 / 3744   -> 1092 / 3623
@@ -234,7 +234,7 @@ inline bool attn_strides_ok(const int64_t (&seq)[N], std::initializer_list<int64
 // Backward.  Launches: delta pre-pass, dK/dV pass, (group reduction), dQ pass — or, with 256-query
 // tiles, the one-wave dQ kernel first (it computes delta itself), then dK/dV and the group
 // reduction.  No atomics, deterministic.
-//   1. delta[b, h, i] = sum_d dO[i, d] * O[i, d]                      (HBM-bound pre-pass)
+//   1. delta[b, h, i] = sum_d dO[i, d] * O[i, d]                      (HBM-bound pre-pass; kept negated)
 //   2. dK, dV: a workgroup owns 128 keys of one (batch, QUERY head) — 32 per pair of waves,
 //      their K and V fragments in the registers of the pair's score wave, dK and dV in those of
 //      its accumulate wave — and streams every query tile at or below the diagonal through LDS.
