@@ -180,6 +180,45 @@ def test_swiglu_epilogue_index_model():
         check(M, F, WN)
 
 
+def test_the_order_of_attention_workgroups_is_a_permutation():
+    """The kernels' map from workgroups to tiles (longest_first), as a model: every (rank, pair) once, an XCD's pairs a contiguous
+    range of ids, and, where all of its pairs start together, its ranks in order of length."""
+    def longest_first(pid, nblocks, ntiles):
+        q, r, xcd, i = nblocks // 8, nblocks % 8, pid % 8, pid // 8
+        first, count = xcd * q + min(xcd, r), q + (xcd < r)
+        if count <= 64 or count <= 16 * ntiles:
+            start, full = first % ntiles, count // ntiles
+            extra = count - full * ntiles
+            wraps = start + extra > ntiles
+            a, b = (start + extra - ntiles, start) if wraps else (start, start + extra)
+            na, nb = (full + 1, full) if wraps else (full, full + 1)
+            at, begin, n = i, 0, na
+            if at >= a * na:
+                at, begin, n = at - a * na, a, nb
+                if at >= (b - a) * nb:
+                    at, begin, n = at - (b - a) * nb, b, na
+            assert n > 0
+            row = at // n
+            rank = begin + row
+            return rank, (first + (rank - start) % ntiles) // ntiles + at - row * n
+        lid, total = first + i, nblocks // ntiles
+        grp = 32 // ntiles if ntiles < 32 and 32 % ntiles == 0 else 1
+        base, at = divmod(lid, grp * ntiles)
+        return (at // grp, base * grp + at % grp) if (base + 1) * grp <= total else (lid % ntiles, lid // ntiles)
+
+    for ntiles in (1, 2, 3, 4, 5, 8, 9, 16, 17, 31, 32, 33, 64, 65):
+        for pairs in (1, 2, 3, 7, 8, 9, 12, 15, 16, 24, 31, 64, 129, 200):
+            nblocks = ntiles * pairs
+            got = [longest_first(p, nblocks, ntiles) for p in range(nblocks)]
+            assert sorted(got) == [(r, p) for r in range(ntiles) for p in range(pairs)]
+            for xcd in range(min(8, nblocks)):
+                mine = got[xcd::8]
+                ids = sorted(p * ntiles + r for r, p in mine)
+                assert ids[-1] - ids[0] == len(ids) - 1 or len(mine) > max(64, 16 * ntiles)
+                if len(mine) <= max(64, 16 * ntiles):
+                    assert [r for r, _ in mine] == sorted(r for r, _ in mine)
+
+
 def test_attention_workspaces_by_stride():
     """What runs as it lies reserves no copies: nothing forward, statistics and partial sums of the rounded-up length
     backward; what does not (other head dimensions, strides of 2^31 / 127 elements and more) the general sizes."""
