@@ -44,10 +44,13 @@ constexpr int kXcds = 8;
 // -> 54, 58 -> 45, 92 -> 84; dK/dV 6 x 4096 of 3/1 heads 249 -> 180, 4 x 4096 of 24/8 heads 867 -> 843; two pairs at once -> this
 // order, 2 x 8192 of 32/8 heads forward 1016 -> 978, dQ 1363 -> 1330.  All pairs at once beyond sixteen: 64 x 512 tokens of 32/8
 // heads forward 276 -> 300, dK/dV 366 -> 411.
+// The choice is the launch's: the first order permutes the ids of one XCD, the second those of groups that cross from one XCD's
+// range into the next, so that only all of them together take every tile once.  (The XCDs' shares differ by one workgroup.)
 __device__ __forceinline__ void longest_first(int pid, int nblocks, int ntiles, int& rank, int& pair) {
   const int q = nblocks / kXcds, r = nblocks % kXcds, xcd = pid % kXcds;
   const int first = xcd * q + (xcd < r ? xcd : r), count = q + (xcd < r ? 1 : 0), i = pid / kXcds;
-  if (count <= 64 || count <= 16 * ntiles) {
+  const int most = q + (r > 0 ? 1 : 0);  // workgroups of the XCD with the most
+  if (most <= 64 || most <= 16 * ntiles) {
     // ids first .. first + count - 1, id = pair * ntiles + rank: every rank `full` times, `extra` ranks from that of the
     // first id on (cyclically) once more.  Ranks [0, a) occur na times, [a, b) nb times, the others na times again.
     const int start = first % ntiles, full = count / ntiles, extra = count - full * ntiles;

@@ -4,6 +4,9 @@ import ctypes
 import glob
 import os
 import re
+import subprocess
+
+import numpy as np
 
 from kareus_amd.backend import hip
 
@@ -180,43 +183,35 @@ def test_swiglu_epilogue_index_model():
         check(M, F, WN)
 
 
-def test_the_order_of_attention_workgroups_is_a_permutation():
-    """The kernels' map from workgroups to tiles (longest_first), as a model: every (rank, pair) once, an XCD's pairs a contiguous
-    range of ids, and, where all of its pairs start together, its ranks in order of length."""
-    def longest_first(pid, nblocks, ntiles):
-        q, r, xcd, i = nblocks // 8, nblocks % 8, pid % 8, pid // 8
-        first, count = xcd * q + min(xcd, r), q + (xcd < r)
-        if count <= 64 or count <= 16 * ntiles:
-            start, full = first % ntiles, count // ntiles
-            extra = count - full * ntiles
-            wraps = start + extra > ntiles
-            a, b = (start + extra - ntiles, start) if wraps else (start, start + extra)
-            na, nb = (full + 1, full) if wraps else (full, full + 1)
-            at, begin, n = i, 0, na
-            if at >= a * na:
-                at, begin, n = at - a * na, a, nb
-                if at >= (b - a) * nb:
-                    at, begin, n = at - (b - a) * nb, b, na
-            assert n > 0
-            row = at // n
-            rank = begin + row
-            return rank, (first + (rank - start) % ntiles) // ntiles + at - row * n
-        lid, total = first + i, nblocks // ntiles
-        grp = 32 // ntiles if ntiles < 32 and 32 % ntiles == 0 else 1
-        base, at = divmod(lid, grp * ntiles)
-        return (at // grp, base * grp + at % grp) if (base + 1) * grp <= total else (lid % ntiles, lid // ntiles)
+def test_the_order_of_attention_workgroups_is_a_permutation(tmp_path):
+    """The kernels' map from workgroups to tiles (longest_first, compiled for the host from the kernels' source): every (rank,
+    pair) once, and, where an XCD starts with the longest tiles of all its pairs, its ids a contiguous range and its ranks in
+    order of length.  The pair counts are small ones and those around which the order changes."""
+    source = open(os.path.join(ROOT, "kareus_amd", "csrc", "kr_attention.hip")).read()
+    begin = source.index("__device__ __forceinline__ void longest_first(")
+    body = source[begin:source.index("\n}\n", begin) + 3].replace("__device__ __forceinline__", "static")
+    xcds = re.search(r"^constexpr int kXcds = \d+;$", source, re.M).group(0)
+    (tmp_path / "order.cpp").write_text(
+        f"{xcds}\n{body}\nextern \"C\" void order(int nblocks, int ntiles, int* rank, int* pair) {{\n"
+        "  for (int i = 0; i < nblocks; ++i) longest_first(i, nblocks, ntiles, rank[i], pair[i]);\n}\n")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "order.cpp", "-o", "order.so"], cwd=tmp_path, check=True)
+    lib = ctypes.CDLL(str(tmp_path / "order.so"))
 
-    for ntiles in (1, 2, 3, 4, 5, 8, 9, 16, 17, 31, 32, 33, 64, 65):
-        for pairs in (1, 2, 3, 7, 8, 9, 12, 15, 16, 24, 31, 64, 129, 200):
-            nblocks = ntiles * pairs
-            got = [longest_first(p, nblocks, ntiles) for p in range(nblocks)]
-            assert sorted(got) == [(r, p) for r in range(ntiles) for p in range(pairs)]
-            for xcd in range(min(8, nblocks)):
-                mine = got[xcd::8]
-                ids = sorted(p * ntiles + r for r, p in mine)
-                assert ids[-1] - ids[0] == len(ids) - 1 or len(mine) > max(64, 16 * ntiles)
-                if len(mine) <= max(64, 16 * ntiles):
-                    assert [r for r, _ in mine] == sorted(r for r, _ in mine)
+    for ntiles in (*range(1, 66), 128, 130):
+        edge = 8 * max(64, 16 * ntiles) // ntiles
+        counts = {*range(1, 33), 64, 127, 128, 129, 200, 255, 256, 257, 258, 259, *range(edge - 4, edge + 5), 2 * edge + 1}
+        for pairs in sorted(p for p in counts if p * ntiles <= 1 << 15):
+            n = ntiles * pairs
+            rank, pair = np.full(n, -1, np.int32), np.full(n, -1, np.int32)
+            lib.order(n, ntiles, rank.ctypes.data_as(ctypes.c_void_p), pair.ctypes.data_as(ctypes.c_void_p))
+            assert rank.min() >= 0 and rank.max() < ntiles and pair.min() >= 0 and pair.max() < pairs, (ntiles, pairs)
+            ids = pair * ntiles + rank
+            assert np.unique(ids).size == n, (ntiles, pairs)
+            if -(-n // 8) <= max(64, 16 * ntiles):
+                for xcd in range(min(8, n)):
+                    mine = ids[xcd::8]
+                    assert mine.max() - mine.min() == mine.size - 1, (ntiles, pairs)
+                    assert (np.diff(rank[xcd::8]) >= 0).all(), (ntiles, pairs)
 
 
 def test_attention_workspaces_by_stride():

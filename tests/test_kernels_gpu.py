@@ -907,6 +907,8 @@ def test_attention_in_place_at_head_dimension_64_and_ragged_lengths(be, s, b, nq
                                            (1152, 5, 3, 1, 64), (904, 7, 2, 2, 128), (136, 1, 2, 1, 128),
                                            (2048, 5, 8, 2, 128),     # more than 64 workgroups per XCD, of at most 16 pairs
                                            (256, 70, 8, 2, 128),     # ... of more pairs
+                                           (1024, 43, 3, 1, 128),    # 516 workgroups: 65 on four XCDs, 64 on the others, one order on all
+                                           (512, 129, 2, 1, 128), (256, 129, 8, 2, 128), (256, 129, 8, 2, 64),
                                            (2048, 4, 8, 2, 128)])    # a 256-query tile for every unit: split forms, two heads per workgroup
 def test_attention_over_orders_of_workgroups(be, s, b, nq, nkv, hd):
     """Every tile of every (batch, head) pair is computed once, whatever part of the pairs an XCD has: a tile left out or taken
