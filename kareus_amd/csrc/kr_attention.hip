@@ -538,8 +538,8 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
   }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   if (D == 128 || nmine > 0) zero_v_tail(0);
-  __syncthreads();
-  if (half == 1) __syncthreads();  // half 1 starts one period late
+  kr_barrier();
+  if (half == 1) kr_barrier();  // half 1 starts one period late
 
   bf16x8 pb[NB][2];
 
@@ -615,7 +615,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    __syncthreads();
+    kr_barrier();
 
     // ---- vector period of tile j: the softmax, and between its eight groups of exponentials
     // the eight requests for K(j+2) and V(j+1) (their buffers were last read in the matrix period
@@ -684,14 +684,14 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
     else
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): nothing was requested
     if (RAGGED && j > 0 && mine) zero_v_tail(j);  // (tile 0 was settled before the loop)
-    __syncthreads();
+    kr_barrier();
   }
   // last matrix period: the product of the final tile
   __builtin_amdgcn_s_setprio(1);
   if (D == 128 || nsteps - 1 < nmine) pv_step(nsteps - 1);
   __builtin_amdgcn_s_setprio(0);
-  __syncthreads();
-  if (half == 0) __syncthreads();  // the period half 1 is behind by
+  kr_barrier();
+  if (half == 0) kr_barrier();  // the period half 1 is behind by
 
   // merge the two halves' partial softmax: half 1 -> LDS -> half 0 (every buffer is idle: the
   // loop ended with a barrier and no request is in flight).  [value][wave][lane] layout.
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pp_kernel(
 #pragma unroll
       for (int e = 0; e < 16; ++e) xch[(2 + dt * 16 + e) * 256 + slot] = oacc[dt][e];
   }
-  __syncthreads();
+  kr_barrier();
   if (half == 1) return;
   {
     const float m_b = xch[slot], l_b = xch[256 + slot];
@@ -831,8 +831,8 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   zero_v_tail(0, 0);
   zero_v_tail(1, 1);
-  __syncthreads();
-  if (half == 1) __syncthreads();  // half 1 starts one period late
+  kr_barrier();
+  if (half == 1) kr_barrier();  // half 1 starts one period late
 
   bf16x8 pb[NB][2];
 
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    __syncthreads();
+    kr_barrier();
 
     // ---- vector period of tile j: the softmax, and between its four groups of exponentials
     // this wave's four requests for tile j+2 of its operand (the ring slot was last read two
@@ -970,7 +970,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
     else
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     if (RAGGED && j > 0 && j + 1 < ntiles) zero_v_tail(j + 1, slot == 2 ? 0 : slot + 1);
-    __syncthreads();
+    kr_barrier();
     slot_prev = slot;
     slot = slot == 2 ? 0 : slot + 1;
     slot_req = slot_req == 2 ? 0 : slot_req + 1;
@@ -981,7 +981,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_sh_kernel(
     pv_step(slot_prev);
     __builtin_amdgcn_s_setprio(0);
   }
-  if (half == 0) __syncthreads();  // the barrier half 1 spent on starting late
+  if (half == 0) kr_barrier();  // the barrier half 1 spent on starting late
 
   // No tile is requested any more and K tiles are no longer read: each wave stages its output
   // rows through 4 KiB of the K ring.
@@ -1119,7 +1119,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       kf[kk] = ldg8(kp + kk * 16 + h * 8);
       vf[kk] = ldg8(vp + kk * 16 + h * 8);
     }
-    __syncthreads();  // tile 0 (and 1) requested by the accumulate waves have landed
+    kr_barrier();  // tile 0 (and 1) requested by the accumulate waves have landed
     // S = Q.K^T and dP = dO.V^T of one 32-query block: sixteen fragments, then sixteen MFMAs
     auto issue_scores = [&](int stage, int sub, f32x16& sacc, f32x16& dpacc) {
       uint32_t q_rows = lds0 + stage * STAGE + bt_rows_lane(lane);
@@ -1216,9 +1216,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
       const int q0 = (qt_first + itl * qsplit + part) * TQ;
       itl = itl + 1 == niter ? 0 : itl + 1;  // the next head starts over at the diagonal
       step(stage, 0, q0, s0, dp0, stage, 1, s1, dp1);
-      __syncthreads();  // hand-over of block 0
+      kr_barrier();  // hand-over of block 0
       step(stage, 1, q0 + 32, s1, dp1, (it + 1) % NS, 0, s0, dp0);
-      __syncthreads();  // hand-over of block 1
+      kr_barrier();  // hand-over of block 1
     }
     return;
   }
@@ -1314,7 +1314,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
   }
   zero_tail(0);
   zero_tail(1);
-  __syncthreads();
+  kr_barrier();
   // The transposed fragments of a block (fr[2 DT k2 + 2 dt]: dO^T, fr[2 DT k2 + 2 dt + 1]: Q^T,
   // queries 16 k2 .. of the block, channels 32 dt ..) live in registers across blocks: each is
   // refilled for the next block right behind the MFMA that consumed it (one MFMA later), so the
@@ -1352,7 +1352,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
         }
         zero_tail(it + 1);
       }
-      __syncthreads();
+      kr_barrier();
       // After the last barrier nobody reads tile it any more (this wave fetched its last
       // fragments of it during the block before, the score waves before the barrier in front of this):
       // tile it+3 goes into its stage, one request behind each of the first MFMAs — pieces 0-4
@@ -1656,7 +1656,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv64_kernel(
     const int qt_next = niter > 1 ? qt + qsplit : qt;
     zero_tail(lds0, qt);
     if (nit_all > 1) zero_tail(stage_of(1), qt_next);
-    __syncthreads();
+    kr_barrier();
     settle_scalar_loads();
     const int qoff = 64 * half;  // this wave's queries of a tile
     Scores a, b;
@@ -1697,7 +1697,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv64_kernel(
       block(a, b, cols, stats, 0, rows, stats, 1, rows_n, stats_n, 0, q0 + 32, [](int) {}, [&] {
         __builtin_amdgcn_s_waitcnt(0x0f75);  // vmcnt(5): of this wave's requests only those of tile it + 2 may be on their way
         if (it > 0 && it + 1 < nit_all) zero_tail(there, qt);  // (tiles 0 and 1 were settled before the loop)
-        __syncthreads();  // everyone's share of tile it + 1 has landed, and nobody reads tile it - 1 any more
+        kr_barrier();  // everyone's share of tile it + 1 has landed, and nobody reads tile it - 1 any more
       });
       const uint32_t free = stage_of(it + NS - 1);
       block(b, a, cols, stats, 1, rows_n, stats_n, 0, rows_n, stats_n, 1, qt * TQ + qoff,
@@ -1708,14 +1708,14 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv64_kernel(
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the requests behind the last tile
   // The stages are free.  Wave w of the first half gives its dV to wave w of the second and gets its dK ([value][wave]
   // [lane] layout, 32 KB each); the first half stores dK, the second dV, through 4 KB per wave behind them.
-  __syncthreads();
+  kr_barrier();
   float* xch = reinterpret_cast<float*>(smem) + wave * 64 + lane;
   float* mine = xch + half * (32 * 256);
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) mine[(dt * 16 + e) * 256] = half == 0 ? dvacc[dt][e] : dkacc[dt][e];
-  __syncthreads();
+  kr_barrier();
   const float* other = xch + (1 - half) * (32 * 256);
   f32x16 acc[DT];
 #pragma unroll
@@ -1856,7 +1856,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
   stage_request(0, 0);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   zero_tail(0, 0);
-  __syncthreads();
+  kr_barrier();
 
   settle_scalar_loads();
   for (int j = 0; j < ntiles; ++j) {
@@ -1914,7 +1914,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's share of the next tiles has landed
     if (RAGGED && j + 1 < ntiles) zero_tail(j + 1, cur ^ 1);
-    __syncthreads();
+    kr_barrier();
   }
 
   if (HALVES == 2) {  // half 1 -> LDS -> half 0 ([value][wave][lane]; the staging areas are free)
@@ -1926,7 +1926,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq
 #pragma unroll
         for (int e = 0; e < 16; ++e) xch[(dt * 16 + e) * 256 + slot] = dqacc[dt][e];
     }
-    __syncthreads();
+    kr_barrier();
     if (half == 1) return;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -2177,7 +2177,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
   stage_request(1, 1);  // ntiles >= 2
   __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): everything but the second tile's requests has landed
   zero_tail(0, 0);
-  __syncthreads();
+  kr_barrier();
   settle_scalar_loads();
 
   const uint32_t rows_lane = bt_rows_lane(lane), cols_lane = bt_cols_lane(lane);
@@ -2201,7 +2201,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_w64_kernel(
   auto arrive = [&](int j) {  // between the two steps of tile j
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's share of tile j + 1 has landed
     if (RAGGED && j + 1 < ntiles) zero_tail(j + 1, buf == NSTAGE - 1 ? 0 : buf + 1);
-    __syncthreads();                     // ... and everyone's; nobody reads tile j - 1 any more
+    kr_barrier();                     // ... and everyone's; nobody reads tile j - 1 any more
   };
   auto turn = [&](int j) {
     arrive(j);
@@ -2342,10 +2342,10 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_fwd_kernel(
   const int qrow = q0 + r;
   const int last_key = (q0 + GT - 1 < s ? q0 + GT - 1 : s - 1);
   for (int k0 = 0; k0 <= last_key; k0 += GT) {
-    __syncthreads();  // the previous tile's K, V and probabilities are no longer read
+    kr_barrier();  // the previous tile's K, V and probabilities are no longer read
     load_tile(sk, kb, kl.s_, k0, s, hd, tid);
     load_tile(sv, vb, vl.s_, k0, s, hd, tid);
-    __syncthreads();
+    kr_barrier();
     float sc[4];
     dot4(sq, sk, r, p, hd, sc);
     float mx = -INFINITY;
@@ -2368,7 +2368,7 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_fwd_kernel(
     const float alpha = m == -INFINITY ? 0.f : __expf(m - m_new);
     l = l * alpha + ps;
     m = m_new;
-    __syncthreads();
+    kr_barrier();
     for (int i = 0; i < c; ++i) acc[i] *= alpha;
     for (int kj = 0; kj < GT; ++kj) {
       const float pv = sp[r][kj];
@@ -2440,7 +2440,7 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_dkdv_kernel(
     const bf16* dob = dout + dol.at(bi, head, per);
     const int64_t stat = ((int64_t)bi * nq + head) * s;
     for (int q0 = k0; q0 < s; q0 += GT) {  // query tiles at or below the diagonal (k0 is a multiple of 32)
-      __syncthreads();
+      kr_barrier();
       load_tile(sq, qb, ql.s_, q0, s, hd, tid);
       load_tile(sdo, dob, dol.s_, q0, s, hd, tid);
       if (tid < GT) {
@@ -2448,7 +2448,7 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_dkdv_kernel(
         slse[tid] = in ? lse[stat + q0 + tid] : 0.f;
         sdelta[tid] = in ? delta[stat + q0 + tid] : 0.f;
       }
-      __syncthreads();
+      kr_barrier();
       float pr[4], ds[4];
       block_p_ds(sq, sk, sv, sdo, slse, sdelta, r, p, hd, q0, k0, s, scale, pr, ds);
 #pragma unroll
@@ -2456,7 +2456,7 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_dkdv_kernel(
         sp[r][4 * p + j] = pr[j];
         sds[r][4 * p + j] = ds[j];
       }
-      __syncthreads();
+      kr_barrier();
       // this thread now is (key r, channels p c ..): dV += P^T dO, dK += dS^T Q
       for (int qi = 0; qi < GT; ++qi) {
         const float pv = sp[qi][r], dsv = sds[qi][r];
@@ -2504,15 +2504,15 @@ __global__ __launch_bounds__(GTHREADS) void attn_general_dq_kernel(
   for (int i = 0; i < GHD_MAX / 8; ++i) adq[i] = 0.f;
   const int last_key = (q0 + GT - 1 < s ? q0 + GT - 1 : s - 1);
   for (int k0 = 0; k0 <= last_key; k0 += GT) {
-    __syncthreads();
+    kr_barrier();
     load_tile(sk, kb, kl.s_, k0, s, hd, tid);
     load_tile(sv, vb, vl.s_, k0, s, hd, tid);
-    __syncthreads();
+    kr_barrier();
     float pr[4], ds[4];
     block_p_ds(sq, sk, sv, sdo, slse, sdelta, r, p, hd, q0, k0, s, scale, pr, ds);
 #pragma unroll
     for (int j = 0; j < 4; ++j) sds[r][4 * p + j] = ds[j];
-    __syncthreads();
+    kr_barrier();
     for (int kj = 0; kj < GT; ++kj) {
       const float dsv = sds[r][kj];
       const bf16* kr = sk + kj * GLD + p * c;

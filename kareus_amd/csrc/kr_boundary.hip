@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
   const int64_t tokens = (int64_t)s * b;
   const int nvec = hidden / 8;
   if (tid == 0) count = 0;
-  __syncthreads();
+  kr_barrier();
   for (int64_t t0 = tid; t0 < tokens; t0 += kIdsAtOnce * kThreads) {
     int64_t id[kIdsAtOnce];
 #pragma unroll
@@ -79,14 +79,14 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
       }
     }
   }
-  __syncthreads();
+  kr_barrier();
   const int n = count;
   const bool listed = n <= kListCap;
   if (listed && n > 1) {  // bitonic sort of the smallest power of two >= n keys, padded with ~0
     int m = 2;
     while (m < n) m <<= 1;
     for (int i = n + tid; i < m; i += kThreads) keys[i] = 0xffffffffu;
-    __syncthreads();
+    kr_barrier();
     for (int k = 2; k <= m; k <<= 1)
       for (int j = k >> 1; j > 0; j >>= 1) {
         for (int i = tid; i < m; i += kThreads) {
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
             }
           }
         }
-        __syncthreads();
+        kr_barrier();
       }
   }
 
@@ -138,10 +138,10 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
         unsigned long long* ballots = reinterpret_cast<unsigned long long*>(keys);
         const unsigned long long bal = __ballot(hit);
         if ((tid & 63) == 0) ballots[tid >> 6] = bal;
-        __syncthreads();
+        kr_barrier();
 #pragma unroll
         for (int w = 0; w < 4; ++w) mask[w] = ballots[w];
-        __syncthreads();
+        kr_barrier();
         for (int w = 0; w < 4; ++w)
           while (mask[w]) {
             const int bit = __builtin_ctzll(mask[w]);
@@ -171,17 +171,17 @@ __global__ __launch_bounds__(kThreads) void embedding_bwd_kernel(const int64_t* 
 __device__ __forceinline__ float block_max(float v, float* red) {
   v = wave_max(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
+  kr_barrier();
   if (lane == 0) red[wave] = v;
-  __syncthreads();
+  kr_barrier();
   return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
+  kr_barrier();
   if (lane == 0) red[wave] = v;
-  __syncthreads();
+  kr_barrier();
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 

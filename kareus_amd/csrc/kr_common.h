@@ -76,6 +76,16 @@ __device__ __forceinline__ void kr_swiglu_bwd_f(float gy, float gate, float up, 
   d_up = gy * gate * sg;
 }
 
+// Workgroup barrier.  To the compiler's machine code neither s_barrier nor the fences around it store anything, so a load from
+// LDS whose value is first used behind a later branch may be moved there, past the barrier that lets other waves overwrite
+// what it reads.  (A dK/dV kernel of attention read 15 of its first tile's fragments behind the barrier that gave the tile's
+// stage to the loads of the fourth: wrong dK about once in a thousand launches, where an instruction cache miss delayed the
+// reads.)  An assembly statement that may write memory holds the loads in front of it.
+__device__ __forceinline__ void kr_barrier() {
+  asm volatile("" ::: "memory");
+  __syncthreads();
+}
+
 static inline bool kr_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 static inline int kr_launch_status() {

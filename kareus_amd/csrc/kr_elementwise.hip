@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(
     cs[i] = c_;
     sn[i] = s_ * sin_sign;
   }
-  __syncthreads();
+  kr_barrier();
   const int vec_per_row = half / 8;
   const int rows = b * heads;
   const int total = rows * vec_per_row;

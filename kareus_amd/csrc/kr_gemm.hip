@@ -662,7 +662,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       __builtin_amdgcn_s_waitcnt(vm_wait(0));
       fix_tail(ring[0], ring[1], k_tail);
     }
-    __syncthreads();
+    kr_barrier();
     if (!carried) {
       uint32_t aa[FragReader<A_T, TW>::NBASE], ba[FragReader<B_T, TWB>::NBASE];
       frag_addrs(ring[0], ring[1], 0, aa, ba);
@@ -710,7 +710,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       if (t + DEPTH + 1 == nk && k_tail != BK) set_offsets(k_tail);
       half(X, Y, ring[0], ring[1], 1, Count<NA_LOADS>{}, a_base(t + DEPTH), la, ring[NSLOTS - 1]);
       __builtin_amdgcn_s_waitcnt(vm_wait((DEPTH - 2) * STEP_LOADS + NA_LOADS));
-      __syncthreads();
+      kr_barrier();
       half(Y, X, ring[2], ring[3], 0, Count<NB_LOADS>{}, b_base(t + DEPTH), lb, ring[0]);
       seg_advance();
       rotate();
@@ -739,7 +739,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
             half(X, Y, ring[0], ring[1], 1, Count<NA_LOADS>{}, a_base(d), la, ring[NSLOTS - 1]);
             __builtin_amdgcn_s_waitcnt(vm_wait((DEPTH - 2) * STEP_LOADS + NA_LOADS));
             if (t + 2 == last) fix_tail(ring[2], ring[3], tail);
-            __syncthreads();
+            kr_barrier();
             half(Y, X, ring[2], ring[3], 0, Count<NB_LOADS>{}, b_base(d), lb, ring[0]);
             seg_advance();
             rotate();
@@ -757,7 +757,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
       else if (DEPTH > 2 && t + 3 == nk) __builtin_amdgcn_s_waitcnt(vm_wait(STEP_LOADS));
       else __builtin_amdgcn_s_waitcnt(vm_wait(0));
       if (t + 2 == nk) fix_tail(ring[2], ring[3], k_tail);
-      __syncthreads();
+      kr_barrier();
       // (after the last K-step this reads tiles that do not exist: unused)
       half(Y, X, ring[2], ring[3], 0, Count<0>{}, nullptr, lb, 0u);
       rotate();
@@ -934,7 +934,7 @@ __global__ __launch_bounds__(NTHREADS, WT == WT_SMALL && DEPTH == kDepth ? 2 : 1
             for (int e = 0; e < 4; ++e) o[e] = (bf16)vals[nt][e];
             *(KR_LDS bf16x4*)(buf + row16 * ROW16 + (((2 * nt + (quad >> 1)) ^ (row16 & XOR16)) << 4) + (quad & 1) * 8) = o;
           }
-          if constexpr (swiglu) __syncthreads(); else wave_sync();  // SwiGLU reads the neighbour wave's block too
+          if constexpr (swiglu) kr_barrier(); else wave_sync();  // SwiGLU reads the neighbour wave's block too
 #pragma unroll
           for (int q = 0; q < Q16; ++q) {
             const int rr = 64 / L16 * q + row_r;

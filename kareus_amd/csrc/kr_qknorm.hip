@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void qk_norm_bwd_kernel(bf16* dmixed, con
     red[0][slot][sub * 8 + e] = dgq[e];
     red[1][slot][sub * 8 + e] = dgk[e];
   }
-  __syncthreads();
+  kr_barrier();
   for (int i = threadIdx.x; i < 2 * HD; i += kThreads) {
     const int which = i / HD, c = i % HD;
     float acc = 0.f;
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(16 * kWalkers) void qk_norm_dgamma_kernel(const flo
 #pragma unroll 8
   for (int b = walker; b < nblocks; b += kWalkers) acc += part[(int64_t)b * 2 * hd + col];
   red[walker][c] = acc;
-  __syncthreads();
+  kr_barrier();
   if (walker == 0) {
     float sum = 0.f;
 #pragma unroll 8

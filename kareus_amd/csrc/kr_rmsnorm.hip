@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_bwd_kernel(
     dot = wave_sum(dot);
     if (SPLIT == 2) {
       if (lane == 0) halves[parity][slot][part] = dot;
-      __syncthreads();
+      kr_barrier();
       dot = halves[parity][slot][0] + halves[parity][slot][1];
       parity ^= 1;  // the next row uses the other buffer: one barrier per row is enough
     }
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_bwd_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) red[(slot - 1) * SPLIT + part][e * 64 + lane] = dg[c][e];
     }
-    __syncthreads();
+    kr_barrier();
     if (slot == 0) {
       const int v = v0 + c * 64;
       if (v < nvec) {
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_bwd_kernel(
         }
       }
     }
-    __syncthreads();
+    kr_barrier();
   }
 }
 
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(kDgammaThreads) void rmsnorm_dgamma_kernel(const fl
     for (; p < nparts; p += 32) a0 += src[(int64_t)p * cols];
   }
   red[rl][c] = (a0 + a1) + (a2 + a3);
-  __syncthreads();
+  kr_barrier();
   if (rl == 0 && col < cols) {
     float sum = 0.f;
 #pragma unroll

@@ -136,3 +136,23 @@ def test_every_instance_of_the_kernel_keeps_the_distance(tmp_path):
         assert n_asm == 128 and not bad, (name, n_asm, bad[:5])
         meta = text[text.index(name, text.index("amdhsa.kernels")):]
         assert int(re.search(r"\.vgpr_spill_count:\s*(\d+)", meta).group(1)) == 0
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc is not installed")
+def test_fragments_of_a_stage_are_read_in_front_of_the_barrier_that_frees_it(tmp_path):
+    """The accumulating waves of the dK/dV kernel fetch the next block's fragments (32 transposing reads) during a block's sixteen
+    MFMAs, and other waves may load over that stage behind the barrier after them: no read may have been moved there."""
+    out = tmp_path / "kr_attention.s"
+    subprocess.run(["make", "-C", CSRC, f"HIPCC={HIPCC}", f"ASMDIR={tmp_path}", str(out)], check=True,
+                   stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL, timeout=600)
+    text = out.read_text()
+    names = re.findall(r"^_Z\w*(attn_bwd_dkdv_kernel\w*):", text, re.M)
+    assert len(set(names)) == 4   # whole and ragged lengths, partial sums and results
+    for name in names:
+        blocks = []
+        for piece in re.split(r"^\s+s_barrier\b", "\n".join(_kernel_body(text, name)), flags=re.M):
+            mfmas, hand_over, fragments = (len(re.findall(rf"^\s+{op}", piece, re.M))
+                                           for op in ("v_mfma", "ds_read_b128", "ds_read_b64_tr"))
+            if mfmas == 16 and hand_over == 4:
+                blocks.append(fragments)
+        assert len(blocks) >= 2 and set(blocks) == {32}, (name, blocks)
