@@ -2583,18 +2583,23 @@ __global__ __launch_bounds__(256) void attn_resize_rows_kernel(const float* __re
 #endif
 // The dK/dV kernels run one workgroup per CU.  With few of them their time is set by the first key tiles (they see every
 // query): two workgroups then share each key tile, which costs fp32 partial sums and a launch that adds them.  At head
-// dimension 64 the halves of a workgroup share a key tile's queries already, so that pays only for long rows (whole -> split,
-// with the launch that adds, us): 8 heads at s 200, b 2 10.2 -> 13.5, at s 1000 19.3 -> 18.9, at s 1000, b 4 21.8 -> 33.7;
-// at s 1536 23.1 -> 24.9; one head at s 4096 47.0 -> 32.6, 4 heads 50.2 -> 38.4; 4/2 heads at s 2048 32.5 -> 23.7.
+// dimension 64 the halves of a workgroup share a key tile's queries already, so that pays only for long rows and, where the heads
+// of a group leave partial sums anyway, for few workgroups (whole -> split, with the launch that adds, us): 8 heads at s 200, b 2
+// 10.2 -> 13.5, at s 1000 19.3 -> 18.9, at s 1000, b 4 21.8 -> 33.7; at s 1536 23.1 -> 24.9; one head at s 4096 47.0 -> 32.6, 4 heads
+// 50.2 -> 38.4; in groups 6 heads at s 3072 45.6 -> 34.7, 8 heads at s 1024 23.0 -> 20.8, s 512 16.9 -> 16.0, s 256 13.8 -> 13.6, 16 heads
+// 17.8 -> 18.2 and 14.2 -> 14.6 at the last two, one tile 12.3 -> 12.8.
 // At head dimension 128, by the number of (key tile, head) pairs against the units (us with the launch that adds; whole and split,
 // 2h: with two heads of a group to a workgroup).  Fewer pairs than units: split (64 64, 44; 128 119, 88; 192 at s 1504 63, 45),
-// but not short rows that leave few units idle (192 at s 512 28, 32).  One each: long rows (s 2048 69, 60; s 1024 45, 49).  More:
-// whole (384 at s 2048 81 and 92, 102 and 113; at s 4096 149, 160).  Two each: 2h (s 2048 99, 92; s 4096 158, 150), where the XCDs get
-// equal shares of it (4 head groups at s 8192 270, 348).
+// but not short rows that leave few units idle (192 at s 512 28, 32; in groups, by key tiles: 4 144 28, 26, 160 28, 29; 5 160 31.4, 29.9,
+// 180 32.4, 33.4; 6 168 34.6, 33.0, 192 35.5, 34.9, 240 37.8, 41.7; 7 168 38.0, 33.8, 224 40.4, 40.6; without groups whole stores no
+// partial sums: 5 160 24.1, 30.3, 6 168 28.0, 34.3, 7 168 31.5, 34.3).  One each: long rows (s 2048 69, 60; s 1024 45, 49).  More:
+// whole (384 at s 2048 81 and 92, 102 and 113; at s 4096 149, 160; 480 at s 2048 97, 116; 496 at s 3968 156, 175).  Two each is the
+// one count that has room for two parts (below) and leaves two workgroups a unit when each takes two heads: 2h (s 512 52.6, 51.4;
+// s 1024 65.4, 64.1; s 2048 98.5, 97.1; s 4096 164.8, 163.3), where the XCDs get equal shares of it (4 head groups at s 8192 301, 403).
 static int dkdv_query_split(int s, int b, int nq, int nkv, int hd) {
   const int key_tiles = s / 128, pairs = key_tiles * nq * b, cus = kr_compute_units();
-  if (hd == 64) return pairs <= 128 && s >= 2048 ? 2 : 1;
-  if (pairs < cus) return 2 * pairs <= cus || key_tiles >= 8 ? 2 : 1;
+  if (hd == 64) return (2 * pairs <= cus && key_tiles >= 16) || (nq != nkv && key_tiles >= 2 && pairs <= 8 * key_tiles && pairs <= cus) ? 2 : 1;
+  if (pairs < cus) return 2 * pairs <= cus || (nq != nkv ? 8 * pairs <= cus * key_tiles : key_tiles >= 8) ? 2 : 1;
   if (4 * pairs < 5 * cus) return key_tiles >= 16 ? 2 : 1;
   return pairs == 2 * cus && (nq / nkv) % 2 == 0 && (nq / 2 * b) % kXcds == 0 ? 2 : 1;
 }

@@ -907,6 +907,7 @@ def test_attention_in_place_at_head_dimension_64_and_ragged_lengths(be, s, b, nq
                                            (1152, 5, 3, 1, 64), (904, 7, 2, 2, 128), (136, 1, 2, 1, 128),
                                            (2048, 5, 8, 2, 128),     # more than 64 workgroups per XCD, of at most 16 pairs
                                            (256, 70, 8, 2, 128),     # ... of more pairs
+                                           (768, 5, 6, 2, 128), (640, 5, 6, 6, 128),  # few short rows: two workgroups a key tile in groups, one without
                                            (1024, 43, 3, 1, 128),    # 516 workgroups: 65 on four XCDs, 64 on the others, one order on all
                                            (512, 129, 2, 1, 128), (256, 129, 8, 2, 128), (256, 129, 8, 2, 64),
                                            (2048, 4, 8, 2, 128)])    # a 256-query tile for every unit: split forms, two heads per workgroup
@@ -930,6 +931,7 @@ def test_attention_over_orders_of_workgroups(be, s, b, nq, nkv, hd):
 
 @pytest.mark.parametrize("s,b,nq,nkv", [(256, 1, 2, 1), (384, 1, 2, 2),          # two and three query tiles: the ring of four stages starts
                                         (640, 2, 4, 2), (2048, 8, 2, 1),         # ... and turns over
+                                        (1536, 1, 6, 2), (1536, 1, 6, 6),        # few workgroups: two a key tile in groups, one without
                                         (2056, 1, 4, 2), (2304, 1, 2, 2),        # few key tiles, long rows: two workgroups a key tile
                                         (512, 64, 8, 2), (500, 64, 8, 2),        # four heads of a group in one workgroup, whole and ragged
                                         (256, 128, 6, 2)])                       # three
