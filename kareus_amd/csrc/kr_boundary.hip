@@ -267,8 +267,17 @@ extern "C" int kr_embedding_fwd(const int64_t* ids, const void* weight, void* ou
 }
 
 // Eight rows: every workgroup scans all ids, which costs more than it gains beyond 8192 tokens (8 and 16 rows, us: 16384 x 3072,
-// 8192 tokens 31, 32; 32064 x 2048, 16384 tokens 48, 40, 32768 tokens 83, 61).
-static int embedding_rows_per_block(int64_t tokens) { return tokens <= 8192 ? 8 : 16; }
+// 8192 tokens 31, 32; 32064 x 2048, 16384 tokens 48, 40, 32768 tokens 83, 61).  With a large vocabulary the scans are what many
+// tokens of few channels take: 16 rows sooner (8 and 16, us: 64128 x 1024, 8192 tokens 42, 33; 128256 x 2048, 8192 tokens 83, 105) and
+// then 32, where those still are five workgroups a unit and more (16 and 32, us: 128256 x 512, 12288 tokens 58, 46; 64128 x 1024, 16384
+// tokens 49, 40, 131072 tokens 278, 185; 151936 x 1024, 49152 tokens 228, 137; 128256 x 2048, 131072 tokens 636, 441; 64128 x 4096,
+// 49152 tokens 260, 243; but 128256 x 2048, 16384 tokens 94, 113; 128256 x 4096, 32768 tokens 202, 226; 16384 x 3072, 65536 tokens 168,
+// 242).  Not 64: a row that fills the key list has its workgroup scan the ids once for each of its rows.
+static int embedding_rows_per_block(int64_t tokens, int64_t vocab_rows, int hidden) {
+  const bool scans_count = vocab_rows >= 40960;
+  if (scans_count && tokens > 10 * hidden) return 32;
+  return tokens > 8192 || (scans_count && tokens > 6 * hidden) ? 16 : 8;
+}
 // Whether the launch's rows are stored with the non-temporal hint: where what it reads and writes is more than the 256 MB
 // memory-side cache holds (plain and hinted stores, us: 32064 x 4096, 776 tokens, 269 MB 39, 52; 4096 tokens, 296 MB 65, 54;
 // 16384 x 3072, 16384 tokens, 201 MB 46, 50, 32768 tokens, 302 MB 96, 75).
@@ -279,7 +288,7 @@ extern "C" int kr_embedding_bwd(const int64_t* ids, const void* dout, void* dwei
   if (!ids || !dout || !dweight || s <= 0 || b <= 0 || hidden <= 0 || vocab_rows <= 0) return KR_EINVAL;
   if (hidden % 8 || hidden > 8192 || (int64_t)s * b >= ((int64_t)1 << kPosBits)) return KR_EUNSUPPORTED;
   if (!kr_aligned16(dout) || !kr_aligned16(dweight)) return KR_EINVAL;
-  const int rows_per_block = embedding_rows_per_block((int64_t)s * b);
+  const int rows_per_block = embedding_rows_per_block((int64_t)s * b, vocab_rows, hidden);
   const bool stream_out = embedding_streams(vocab_rows + (int64_t)s * b, hidden);
   const unsigned blocks = (unsigned)((vocab_rows + rows_per_block - 1) / rows_per_block);
 #define KR_EMB_BWD(C)                                                                               \

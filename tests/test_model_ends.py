@@ -139,6 +139,7 @@ def test_embedding_kernels(b, s, hidden, rows, start):
 
 @gpu
 @pytest.mark.parametrize("b,s,hidden,rows,start", [(1, 1, 64, 9, 0), (1, 2049, 64, 23, 8), (3, 2731, 128, 41, 8),  # 8193 tokens: 16 rows per workgroup
+                                                   (2, 256, 64, 40963, 8), (1, 800, 64, 40963, 8),  # a large vocabulary, few channels: 16 and 32
                                                    (2, 2048, 4096, 32064, 0)])  # more than the memory-side cache: non-temporal stores
 def test_embedding_gradient_over_rows_per_workgroup(b, s, hidden, rows, start):
     """Sums in position order, whatever the split of the rows: the bits of an in-order sum in fp32, rounded once."""
