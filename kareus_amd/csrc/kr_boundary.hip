@@ -278,10 +278,10 @@ static int embedding_rows_per_block(int64_t tokens, int64_t vocab_rows, int hidd
   if (scans_count && tokens > 10 * hidden) return 32;
   return tokens > 8192 || (scans_count && tokens > 6 * hidden) ? 16 : 8;
 }
-// Whether the launch's rows are stored with the non-temporal hint: where what it reads and writes is more than the 256 MB
-// memory-side cache holds (plain and hinted stores, us: 32064 x 4096, 776 tokens, 269 MB 39, 52; 4096 tokens, 296 MB 65, 54;
-// 16384 x 3072, 16384 tokens, 201 MB 46, 50, 32768 tokens, 302 MB 96, 75).
-static bool embedding_streams(int64_t rows, int hidden) { return 2 * rows * hidden > (int64_t)280 << 20; }
+// Whether the launch's rows are stored with the non-temporal hint: where what it reads and writes is more than the 256 MiB
+// memory-side cache keeps of it, with 18 MiB for what else lies there (plain and hinted stores, us, by MiB read and written: 192 46, 45;
+// 222 51, 50; 253 65, 61; 257 39, 52; 266 45, 51; 282 65, 54; 288 95, 76; 317 118, 83).
+static bool embedding_streams(int64_t rows, int hidden) { return 2 * rows * hidden > (int64_t)274 << 20; }
 
 extern "C" int kr_embedding_bwd(const int64_t* ids, const void* dout, void* dweight, int s, int b,
                                 int hidden, int64_t vocab_start, int64_t vocab_rows, void* stream) {
