@@ -1305,7 +1305,7 @@ inline Tile fewer_rows(int M, int N, int wn, int num_cus) {
 
 // Tile width and number of cuts of the contraction.  An output of at least 192 full-width tiles is
 // never cut and takes the width of choose_wn.  A smaller one has too few tiles to occupy the GPU:
-// narrower tiles (down to 128 columns; 160 with a fused epilogue) and cuts of the contraction both
+// narrower tiles (down to 128 columns; 160 with a fused epilogue, 128 where that is one round) and cuts of the contraction both
 // make more work items, and the pair with the least estimated cost wins.  Two estimates, in units of one K-step of a full-width tile (~1.3 us;
 // a tile of WN columns takes (WN + 2) / 10 of it):
 //   latency  rounds of work items over the CUs, each item paying its K-steps plus a fixed
@@ -1320,8 +1320,9 @@ struct Plan {
   Tile tile = kLarge;  // (wn is 4 for the small tile, 2 for the two below it)
 };
 inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, int max_splits,
-                        bool fused = false, bool allow_small = true) {
+                        int epi = KR_GEMM_EPI_NONE, bool allow_small = true) {
   constexpr int kItemOverhead = 4;
+  const bool fused = epi != KR_GEMM_EPI_NONE;
   const int min_wn = fused ? 5 : 4;
   const int tiles_m = (M + BM - 1) / BM;
   if (tiles_m * ((N + BN - 1) / BN) >= 192) return {choose_wn(M, N, num_cus), 1};
@@ -1448,10 +1449,15 @@ inline Plan choose_plan(int M, int N, int K, float latency_weight, int num_cus, 
   // 192, 48) 48.9 -> 38.4, 1152 x 4096 x 1536 (160, 24) 21.5 -> 19.7.
   // Outside the rule: fewer tiles, when most small ones have a unit to themselves (residual 1536 x 3072 x 8192 (144, 128) 95.6 ->
   // 101.8, SwiGLU backward 6024 x 768 x 2048 (144, 32) 28.1 -> 30.4), and short contractions, where the longer prologue and epilogue
-  // count (plain 1280 x 4096 x 1024 (160, 16) 14.4 -> 14.8, residual 3072 x 2048 x 2048 (192, 32) 27.6 -> 28.2).
+  // count (plain 1280 x 4096 x 1024 (160, 16) 14.4 -> 14.8, residual 3072 x 2048 x 2048 (192, 32) 27.6 -> 28.2).  An epilogue that
+  // reads the output's place (residual, backward) makes a short contraction one of 40 K-steps, but for wide outputs, whose weights come
+  // from memory (residual 3928 x 2048 x 2048 (256, 32) 31.3 -> 32.2, x 1536 25.4 -> 26.4; backward 37.3 -> 39.6, 9872 x 768 x 2048 (234, 32)
+  // 35.0 -> 36.7, 4800 x 1536 x 2048 (228, 32) 34.6 -> 34.8, 1024 x 8192 x 2048 (256, 32) 50.7 -> 48.2).
   if (alone && in_tiles.tile == kSmall && in_tiles.splits == 1 && small_tiles > num_cus) {
     const int tiles = tiles_m * ((N + 127) / 128);
-    if (tiles <= num_cus && tiles * 8 >= num_cus * 5 && nk >= (fused && tiles * 4 <= num_cus * 3 ? 40 : 24)) in_tiles = {4, 1};
+    const bool nearly_all = tiles * 4 > num_cus * 3;  // ... of the units have a tile
+    const bool short_pays = !fused || (nearly_all && (epi == KR_GEMM_EPI_SWIGLU || N >= 2 * M));
+    if (tiles <= num_cus && tiles * 8 >= num_cus * 5 && nk >= (short_pays ? 24 : 40)) in_tiles = {4, 1};
   }
   if (under_cost >= small || under_cost >= large * 0.93) return in_tiles;
   return {2, in_tiles.splits, under};  // (its sums in the pieces that they would be cut into)
@@ -1500,7 +1506,7 @@ extern "C" size_t kr_gemm_workspace_bytes_shared(int layout, int M, int N, int K
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   int splits = choose_plan(M, N, K, latency_weight, 256, 16).splits;
   // never more than a launch that has the device to itself takes, in its tile or in the large one
-  const int cap = std::max(choose_plan(M, N, K, 1.f, 256, 16).splits, choose_plan(M, N, K, 1.f, 256, 16, false, false).splits);
+  const int cap = std::max(choose_plan(M, N, K, 1.f, 256, 16).splits, choose_plan(M, N, K, 1.f, 256, 16, KR_GEMM_EPI_NONE, false).splits);
   if (splits > cap) splits = cap;
   return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
 }
@@ -1515,7 +1521,7 @@ Plan launch_plan(int M, int N, int K, int epi, bool shared, int cus, size_t held
     max_splits = held > 16 ? 16 : (int)held;
     if (max_splits < 1) max_splits = 1;
   }
-  return choose_plan(M, N, K, shared ? 0.1f : 1.f, cus, max_splits, epi != KR_GEMM_EPI_NONE,
+  return choose_plan(M, N, K, shared ? 0.1f : 1.f, cus, max_splits, epi,
                      epi != KR_GEMM_EPI_SWIGLU || N % 128 == 0);
 }
 // What a call is launched as: the plan, the tile that the layout and the output leave of it, operands exchanged or not.
