@@ -949,12 +949,21 @@ bool is_saved(PyObject* o, int64_t rows, int64_t cols) {
   return bf16_arg(o) && tensor(o).dim() == 2 && tensor(o).is_contiguous() && tensor(o).size(0) == rows && tensor(o).size(1) == cols;
 }
 
-// mlp_chain_bwd(dy, w2, fc1's output, activation, w1, normed, split2, split1, weight gradients, max_cus) -> (dx [rows, h], gradient
-// of fc1's output, dw2, dw1).  With ``weight gradients`` the saved tensors lose their memory once they are used; without, the
-// caller takes the two weight gradients and the last two results are None.
+// Calls the caller's function between two steps of a chain, if there is one; false: it raised.
+bool called(PyObject* function) {
+  if (absent(function)) return true;
+  PyObject* got = PyObject_CallNoArgs(function);
+  Py_XDECREF(got);
+  return got != nullptr;
+}
+
+// mlp_chain_bwd(dy, w2, fc1's output, activation, w1, normed, split2, split1, weight gradients, max_cus, between) -> (dx [rows, h],
+// gradient of fc1's output, dw2, dw1).  With ``weight gradients`` the saved tensors lose their memory once they are used; without,
+// the caller takes the two weight gradients and the last two results are None.  ``between`` (None or a function without arguments) is
+// called where fc2's weight gradient may be taken: behind fc2's input gradient.
 PyObject* py_mlp_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
-    if (n_args != 10) return none();
+    if (n_args != 11) return none();
     for (int i : {1, 4})
       if (!bf16_arg(a[i]) || tensor(a[i]).dim() != 2) return none();
     const Tensor &w2 = tensor(a[1]), &w1 = tensor(a[4]);
@@ -986,6 +995,7 @@ PyObject* py_mlp_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       }
     }
     if (rc != KR_OK) return failed(at, rc);
+    if (!called(a[10])) return nullptr;
     if (wgrad) release({a[2], a[3]});
     {
       WithoutInterpreter free;
@@ -1004,11 +1014,11 @@ PyObject* py_mlp_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // attn_chain_bwd(dy, w_proj, q, k, v, o, lse, o rows, freqs, scale, beside other streams, mixed, qk rstd, gamma_q, gamma_k, w_qkv, normed,
-// split_proj, split_qkv, weight gradients, max_cus) -> (dx [rows, h], gradient of the QKV projection's output [rows, w], dw_proj,
-// dw_qkv, dgamma_q, dgamma_k).  Saved tensors and weight gradients as in mlp_chain_bwd.
+// split_proj, split_qkv, weight gradients, max_cus, between) -> (dx [rows, h], gradient of the QKV projection's output [rows, w],
+// dw_proj, dw_qkv, dgamma_q, dgamma_k).  Saved tensors, weight gradients and ``between`` as in mlp_chain_bwd.
 PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   return guarded([&]() -> PyObject* {
-    if (n_args != 21) return none();
+    if (n_args != 22) return none();
     for (int i : {2, 3, 4, 5})
       if (!bf16_arg(a[i])) return none();
     if (!f32_arg(a[6]) || !f32_arg(a[8])) return none();
@@ -1052,6 +1062,7 @@ PyObject* py_attn_chain_bwd(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
       }
     }
     if (rc != KR_OK) return failed(at, rc);
+    if (!called(a[21])) return nullptr;
     if (wgrad) release({a[7]});
     at.call("kr_attn_bwd", c);
     {

@@ -295,13 +295,32 @@ class _BackwardBehindAdd:
         return got
 
 
+class _BetweenProjections:
+    """A chain's first projection leaves the operands of its weight gradient over nanobatches on streams where the operators would:
+    behind its own input gradient, so that the event is there, and the launch over all nanobatches, before the chain's others are
+    enqueued.  (Behind the whole chain, two nanobatches of 4 x 4096 tokens of a 3/1-head shard took 1.3 % longer.)"""
+
+    __slots__ = ("be", "linear", "ctx", "dy", "x", "dw")
+
+    def __init__(self, be, linear, ctx, dy, x) -> None:
+        self.be, self.linear, self.ctx, self.dy, self.x, self.dw = be, linear, ctx, dy, x, None
+
+    def __call__(self) -> None:
+        self.dw = PartitionableLinear._weight_grad(self.be, self.ctx, self.be.rows_in_place(self.dy), self.x,
+                                                   self.linear._split(self.ctx))
+
+
+def _between(be, linear, ctx, dy, x) -> Optional[_BetweenProjections]:
+    sink = getattr(ctx, "wgrad_sink", None)
+    return None if sink is None or sink.get("in_line") else _BetweenProjections(be, linear, ctx, dy, x)
+
+
 def _add_pair(be, linear, ctx, dy, x):
-    """The weight gradient of a projection over nanobatches.  On streams of their own it is PartitionableLinear._weight_grad, whose
-    event then lies behind the chain's input gradients.  On one stream the pair is left in the layer's sink without events, and
-    the last nanobatch contracts all of them in nanobatch order."""
+    """The weight gradient of a projection over nanobatches.  On streams of their own it is PartitionableLinear._weight_grad.  On
+    one stream the pair is left in the layer's sink without events, and the last nanobatch contracts all of them in nanobatch order."""
     sink = ctx.wgrad_sink
     n = sink["n"]
-    if not sink.get("in_line") or not sink["defer"] or sink["pending"] is not None:
+    if not sink.get("in_line") or not sink["defer"]:
         return PartitionableLinear._weight_grad(be, ctx, dy, x, linear._split(ctx))
     pairs = sink.get("pairs")
     if pairs is None:
@@ -339,13 +358,14 @@ class _BackwardMlp(_BackwardChain):
         be = get_backend("hip")
         alone = c2.alone
         here = getattr(c2, "wgrad_sink", None) is None
+        between = _between(be, fc2, c2, dy, activated)
         done = be._n.mlp_chain_bwd(dy, w2, pre, activated, w1, normed, _split(be, fc2, alone), _split(be, fc1, alone), here,
-                                   _max_cus(be, dy.device))
+                                   _max_cus(be, dy.device), between)
         if done is None:
             return None
         dx, dpre, dw2, dw1 = done
         if not here:
-            dw2 = _add_pair(be, fc2, c2, be.rows_in_place(dy), activated)
+            dw2 = between.dw if between is not None else _add_pair(be, fc2, c2, be.rows_in_place(dy), activated)
             dw1 = _add_pair(be, fc1, c1, dpre, normed)
         self._finish(store, ctxs, dy, dx.view(*dy.shape[:-1], dx.shape[1]), protected, here)
         p2, pa, p1 = self.plans
@@ -370,14 +390,15 @@ class _BackwardAttention(_BackwardChain):
         be = get_backend("hip")
         alone = co.alone
         here = getattr(co, "wgrad_sink", None) is None
+        between = _between(be, proj, co, dy, o2d)
         done = be._n.attn_chain_bwd(dy, wo, q, k, v, o, lse, o2d, freqs, ca.scale, attn.beside_other_streams, mixed, qk_rstd,
                                     gq, gk, wq, normed, _split(be, proj, alone), _split(be, qkv, alone), here,
-                                    _max_cus(be, dy.device))
+                                    _max_cus(be, dy.device), between)
         if done is None:
             return None
         dx, dmixed, dwo, dwq, dgq, dgk = done
         if not here:
-            dwo = _add_pair(be, proj, co, be.rows_in_place(dy), o2d)
+            dwo = between.dw if between is not None else _add_pair(be, proj, co, be.rows_in_place(dy), o2d)
             dwq = _add_pair(be, qkv, cq, dmixed, normed)
         elif id(freqs) not in protected:
             clear_tensor_data(freqs)

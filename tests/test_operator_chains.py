@@ -11,10 +11,12 @@ import pytest
 import torch
 
 from kareus_amd import LayerConfig, LayerStack, operators
+from kareus_amd.backend import get_backend
 from kareus_amd.operators import PartitionableRMSNorm, ResidualForkOp, chains
 from kareus_amd.partitions import Channel, ComputeOp, TensorPort, autograd_function
 from kareus_amd.partitions.op_context import OperationContext
 from kareus_amd.partitions.partition_base import PartitionBase
+from kareus_amd.partitions.streams import stream_api
 
 
 def config(nnb=1, **kw):
@@ -325,8 +327,7 @@ def test_a_chain_has_the_bits_of_its_operators(what, monkeypatch):
     passes = 2 * cfg.num_layers * cfg.num_nanobatches
     again = 2 if cfg.checkpoint_activations else 1
     assert ran["_ForwardAttention"] == ran["_ForwardMlp"] == passes * again
-    whole = what not in ("no epilogue fusion", "nanobatches on streams", "nanobatches on one stream")
-    if whole:
+    if what != "no epilogue fusion":
         assert ran["_BackwardAttention"] == ran["_BackwardMlp"] == passes
 
 
@@ -351,6 +352,43 @@ def test_backward_chains_of_nanobatches_on_streams(what, monkeypatch):
     cfg = dataclasses.replace(cfg, in_line_below_ms=0.0)
     ran = both(monkeypatch, cfg, s, b)
     assert ran["_BackwardAttention"] == ran["_BackwardMlp"] == 2 * cfg.num_layers * cfg.num_nanobatches
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+def test_the_first_projection_of_a_chain_leaves_its_event_before_the_other_steps(monkeypatch):
+    """Nanobatches on streams: the operands of the out-projection's and of fc2's weight gradient are left, with their event, inside
+    the native call, as the operators would leave them; an error there leaves the call."""
+    log, api, native = [], stream_api(), get_backend("hip")._n
+    new_event = api.new_event
+
+    def event(*a):
+        log.append("event")
+        return new_event(*a)
+
+    monkeypatch.setattr(api, "new_event", event)
+    for name in ("mlp_chain_bwd", "attn_chain_bwd"):
+        def call(*a, _call=getattr(native, name)):
+            log.append("in")
+            got = _call(*a)
+            log.append("out")
+            return got
+        monkeypatch.setattr(native, name, call)
+    cfg = dataclasses.replace(config(2), in_line_below_ms=0.0)
+    run(cfg, 96, 4)
+    starts = [i for i, what in enumerate(log) if what == "in"]
+    assert len(starts) == 2 * 2 * cfg.num_layers * cfg.num_nanobatches
+    assert all(log[i + 1:i + 3] == ["event", "out"] for i in starts)
+
+    def no_event(*a):
+        if log[-1] == "in":
+            raise RuntimeError("no event")
+        return event(*a)
+
+    monkeypatch.setattr(api, "new_event", no_event)
+    with pytest.raises(RuntimeError, match="no event"):
+        run(cfg, 96, 4)
+    torch.cuda.synchronize()
 
 
 @pytest.mark.gpu
