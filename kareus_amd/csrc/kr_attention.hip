@@ -44,8 +44,8 @@ constexpr int kXcds = 8;
 // -> 54, 58 -> 45, 92 -> 84; dK/dV 6 x 4096 of 3/1 heads 249 -> 180, 4 x 4096 of 24/8 heads 867 -> 843; two pairs at once -> this
 // order, 2 x 8192 of 32/8 heads forward 1016 -> 978, dQ 1363 -> 1330.  All pairs at once beyond sixteen: 64 x 512 tokens of 32/8
 // heads forward 276 -> 300, dK/dV 366 -> 411.  Where every workgroup has a unit to itself all start at once, and where pairs are
-// one tile there is nothing to order; the divisions only delay them: one pair after the other (256 tokens of 8/8 heads of 64 forward 9.6 -> 9.3, dQ 8.0 -> 7.7; 512 tokens
-// of 8/2 heads 11.9 -> 11.6, 10.5 -> 10.3).
+// one tile there is nothing to order; the divisions only delay them: one pair after the other (256 tokens of 8/8 heads of 64 forward
+// 9.6 -> 9.3, dQ 8.0 -> 7.7; 512 tokens of 8/2 heads 11.9 -> 11.6, 10.5 -> 10.3).
 // The choice is the launch's: the first order permutes the ids of one XCD, the second those of groups that cross from one XCD's
 // range into the next, so that only all of them together take every tile once.  (The XCDs' shares differ by one workgroup.)
 __device__ __forceinline__ void longest_first(int pid, int nblocks, int ntiles, int& rank, int& pair) {
