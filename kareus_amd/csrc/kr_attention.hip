@@ -1412,10 +1412,11 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
 //   slots 12-15  ... last 16 queries
 // A score's multiply-add, its exponential and its remaining work are in consecutive slots (in one slot a wave would wait for
 // each of them); score 0 of block b + 1 starts in slot 10 of block b.
-// What bounds it: between the matrix pipe and the instructions around it (without its LDS reads, requests and barriers,
-// MFMAs and exponentials alone, it takes 203 us where it takes 274).  The kernel that specialised its waves, as the one above does,
+// What bounds it: no unit alone.  The matrix pipes are busy 58 % of the cycles, the vector ALUs 47, the LDS pipes 59, a wave waits a quarter of
+// its time, and the power limit leaves 1.8 of 2.4 GHz; without LDS reads, requests and barriers it takes 203 us where it takes 274.  The kernel that specialised its waves, as the one above does,
 // waited for hand-overs: b 2 x 32/8 x s 4096 404 -> 274 us (0.70 -> 1.03 PFLOP/s of the four products), b 1 beside other streams 199
-// -> 143, s 2048, b 1 60 -> 46, 4 x 1000 tokens, 8 heads 38 (with the sum of its partial results) -> 22, s 256 9.1 -> 9.8.
+// -> 143, s 2048, b 1 60 -> 46, 4 x 1000 tokens, 8 heads 38 (with the sum of its partial results) -> 22.  Short rows
+// pay for the exchange at the end: s 256, 8/8 heads 11.8 (with that sum) -> 9.2, 8/2 heads 12.4 -> 13.5.
 // Two independent workgroups of four waves per compute unit took 309 (each a barrier fewer, but the first key tiles
 // run on alone); row statistics through one lane each and lane broadcasts, instead of 8 KB of LDS reads a block, the same.
 // Everything read from LDS is requested about four slots before it is used.  dP starts from -delta, read straight into
@@ -1779,7 +1780,7 @@ __global__ __launch_bounds__(256) void attn_group_reduce_kernel(
 // HALVES = 2: as in the forward kernel, two halves of an 8-wave workgroup own the same 128
 // queries and walk the even / odd key tiles; half 1's dQ partial is added to half 0's through
 // LDS at the end.  Chosen by the host when there are few workgroups.
-// When there is a 256-query tile for every compute unit (or other streams run beside the launch)
+// When there are more 256-query tiles than compute units (or other streams run beside the launch; see attn_forms)
 // the host takes attn_bwd_dq_w64_kernel below instead.
 template <int D, bool RAGGED, int HALVES>
 __global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void attn_bwd_dq_kernel(
@@ -2783,7 +2784,7 @@ int attn_bwd_mfma(const BwdCall& c) {
   const float scale_log2 = scale * kLog2e;
   const int dq_blocks = (sp / BQ) * nq * b;
   if (forms.shared_dq) {
-    // 256-query tiles (one for every compute unit, or other streams beside): one wave per SIMD, 64 rows each.
+    // 256-query tiles (see attn_forms): one wave per SIMD, 64 rows each.
     // It comes first: it also computes delta and the log2-domain copy of lse that the dK/dV kernel reads.
     hipLaunchKernelGGL((attn_bwd_dq_w64_kernel<D, RAGGED>), dim3(dq_blocks / 2), dim3(256), lds_dq_w64, st,
                        q, k, v, dout, o, lse,
@@ -2952,7 +2953,7 @@ template <int D, bool RAGGED>
 int attn_fwd_mfma(const FwdCall& c) {
   const int s = c.s, b = c.b, nq = c.nq, sp = attn_padded_len(s);
   if (attn_forms(sp, b, nq, c.nkv, D, c.flags).shared_fwd) {
-    // 256-query tiles (one for every compute unit, or other streams beside): the halves share their K / V tiles
+    // 256-query tiles (see attn_forms): the halves share their K / V tiles
     constexpr size_t lds_sh = 3 * 16 * ((1024 + 16) + (1024 + 64));  // 100 KiB
     static const hipError_t attr_sh = hipFuncSetAttribute(
         (const void*)attn_fwd_sh_kernel<D, RAGGED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_sh);
