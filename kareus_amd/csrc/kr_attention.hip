@@ -1412,11 +1412,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(
 //   slots 12-15  ... last 16 queries
 // A score's multiply-add, its exponential and its remaining work are in consecutive slots (in one slot a wave would wait for
 // each of them); score 0 of block b + 1 starts in slot 10 of block b.
-// What bounds it: no unit alone.  The matrix pipes are busy 58 % of the cycles, the vector ALUs 47, the LDS pipes 59, a wave waits a quarter of
-// its time, and the power limit leaves 1.8 of 2.4 GHz; without LDS reads, requests and barriers it takes 203 us where it takes 274.  The kernel that specialised its waves, as the one above does,
-// waited for hand-overs: b 2 x 32/8 x s 4096 404 -> 274 us (0.70 -> 1.03 PFLOP/s of the four products), b 1 beside other streams 199
-// -> 143, s 2048, b 1 60 -> 46, 4 x 1000 tokens, 8 heads 38 (with the sum of its partial results) -> 22.  Short rows
-// pay for the exchange at the end: s 256, 8/8 heads 11.8 (with that sum) -> 9.2, 8/2 heads 12.4 -> 13.5.
+// What bounds it: no unit alone.  The matrix pipes are busy 58 % of the cycles, the vector ALUs 47, the LDS pipes 59, a wave waits a
+// quarter of its time, and the power limit leaves 1.8 of 2.4 GHz; without LDS reads, requests and barriers it takes 203 us where it
+// takes 274.  The kernel that specialised its waves, as the one above does, waited for hand-overs: b 2 x 32/8 x s 4096 404 -> 274 us
+// (0.70 -> 1.03 PFLOP/s of the four products), b 1 beside other streams 199 -> 143, s 2048, b 1 60 -> 46, 4 x 1000 tokens, 8 heads 38
+// (with the sum of its partial results) -> 22.  Short rows pay for the exchange at the end: s 256, 8/8 heads 11.8 (with that sum) ->
+// 9.2, 8/2 heads 12.4 -> 13.5.
 // Two independent workgroups of four waves per compute unit took 309 (each a barrier fewer, but the first key tiles
 // run on alone); row statistics through one lane each and lane broadcasts, instead of 8 KB of LDS reads a block, the same.
 // Everything read from LDS is requested about four slots before it is used.  dP starts from -delta, read straight into

@@ -148,7 +148,8 @@ constexpr int kGroupM = 4;
 // operand re-reads; the same hint on other kernels' stores or on the epilogues' residual loads changed nothing.
 // KEEP: plain stores in the tiles that small activations and gradients are made of (128 columns and less), which the next launch
 // then finds in a cache.  With those of the norm's forward (kr_rmsnorm.hip), us: logits of a prompt of 776 tokens, two layers 493
-// -> 480, four nanobatches of 512 tokens of the 3B layer 1981 -> 1935; larger steps the same.  Weight gradients are read by no
+// -> 480, four nanobatches of 512 tokens of the 3B layer 1981 -> 1935; larger steps the same (alone, a launch takes 2-6 % longer:
+// its results leave the L2 at its end).  Weight gradients are read by no
 // launch of the pass: with plain stores three sequences of 2008 tokens took 0.3 % more.
 template <bool KEEP>
 __device__ __forceinline__ void stg8_out(bf16* p, bf16x8 v) {

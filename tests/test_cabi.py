@@ -186,7 +186,8 @@ def test_swiglu_epilogue_index_model():
 def test_the_order_of_attention_workgroups_is_a_permutation(tmp_path):
     """The kernels' map from workgroups to tiles (longest_first, compiled for the host from the kernels' source): every (rank,
     pair) once, and, where an XCD starts with the longest tiles of all its pairs, its ids a contiguous range and its ranks in
-    order of length (with a unit for every workgroup, its ids in sequence).  The pair counts are small ones and those around which the order changes."""
+    order of length (with a unit for every workgroup, or tiles of one length, its ids in sequence).  The pair counts are small ones
+    and those around which the order changes."""
     source = open(os.path.join(ROOT, "kareus_amd", "csrc", "kr_attention.hip")).read()
     begin = source.index("__device__ __forceinline__ void longest_first(")
     body = source[begin:source.index("\n}\n", begin) + 3].replace("__device__ __forceinline__", "static")
@@ -199,7 +200,8 @@ def test_the_order_of_attention_workgroups_is_a_permutation(tmp_path):
 
     for ntiles in (*range(1, 66), 128, 130):
         edge = 8 * max(64, 16 * ntiles) // ntiles
-        counts = {*range(1, 33), 256 // ntiles, 256 // ntiles + 1, 64, 127, 128, 129, 200, 255, 256, 257, 258, 259, *range(edge - 4, edge + 5), 2 * edge + 1}
+        counts = {*range(1, 33), 256 // ntiles, 256 // ntiles + 1, 64, 127, 128, 129, 200, 255, 256, 257, 258, 259,
+                  *range(edge - 4, edge + 5), 2 * edge + 1}
         for pairs in sorted(p for p in counts if 0 < p * ntiles <= 1 << 15):
             n = ntiles * pairs
             rank, pair = np.full(n, -1, np.int32), np.full(n, -1, np.int32)
